@@ -33,7 +33,7 @@ drtc::DeltaArgs delta_args(const py::dict& d) {
   VAL(ld_decay); PTR(gate); VAL(ld_gate); PTR(a_exp); PTR(dt_bias); PTR(norm_w); VAL(eps);
   VAL(H); VAL(Hk); VAL(dim); VAL(vdim); VAL(taps); VAL(C); PTR(out);
   PTR(seg_row); PTR(seg_len); PTR(seg_pos); PTR(seg_state); PTR(positions); PTR(row_state);
-  VAL(nseg); VAL(rows);
+  VAL(nseg); VAL(rows); PTR(ws); VAL(ws_floats); PTR(ws_o); VAL(vdim16);
   return a;
 }
 

@@ -12,6 +12,8 @@
 //                        of a portion come from the sequence's ring of the last `taps` inputs
 //   delta_chunk_kernel   one workgroup per (portion, head): 8 tokens at a time in matrix form on
 //                        the fp32 MFMA (derivation at the kernel)
+//   delta_prep / chain / read_kernel  the same in three launches with chunks of 16 tokens, for a few
+//                        long portions (ops/delta.py _chain_ok)
 //   delta_scan_kernel    the same token by token, for sizes the chunk form does not take
 //   delta_decode_kernel  one workgroup per (sequence, head): all of it for one token; the
 //                        state streams through registers once
@@ -715,6 +717,423 @@ __global__ __launch_bounds__(NTHR, 2) void delta_chunk_kernel(DeltaArgs a) {
   keep_ring<T>(a, slot, h, n, row0, pos0);
 }
 
+// The same in three launches, for a few long portions: what a chunk needs besides the state does not
+// wait for it.  Chunks of 16 tokens:
+//   delta_prep   a workgroup per (chunk, head): unit keys and queries, decays, A, B, [M_U; M_O] -
+//                written as MFMA operands, 16 bytes per lane (ChainEntry)
+//   delta_chain  a workgroup per (portion, head, 16 CT value columns): its waves divide the key
+//                channels of S, kept as accumulator tiles; the partial products meet in LDS, wave ct
+//                forms R, U and O of column tile ct.  R and U of 16 tokens are one tile each, whose
+//                layout is also a B operand
+//   delta_read   output norm and gate, rings
+// The chain is bound by the fp32 MFMA (32 cycles each, 64 + 32 of them per chunk and column tile, over
+// NW waves) and by two exchanges through LDS, about 700 cycles a chunk: 1.5 us per 16 tokens at CT = 2
+// against 10.3 us of delta_chunk, whose five barriers also wait for the staging.  Heads of 128,
+// 4 x 3,500 tokens, 16 heads: 664 us (prep 197, chain 397, read 65), delta_chunk 2,244; one portion of
+// 4,000: 457 against 2,492.  With portions and heads enough for every CU delta_chunk keeps the fp32
+// units as busy without operands in memory (64 x 250, 32 heads: 959 against 1,249).
+// Chunks are numbered through the portions in their order: at most rows / 16 + nseg of them.
+// Waits for this wave's LDS traffic only: loads for the next chunk stay in flight.
+DRTC_DEVICE void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+template <int DT>
+struct ChainEntry {  // floats of a (chunk, head)
+  static constexpr int ek = 0, eq = 256 * DT, kd = 512 * DT;  // [DT][64 lanes][4]
+  static constexpr int gt = 768 * DT;                         // [16 DT] decay over the chunk
+  static constexpr int mu = gt + 16 * DT, mo = mu + 256;      // [64 lanes][4]
+  static constexpr int N = mo + 256;
+};
+struct ChunkAt {
+  int seg, slot, n, row0, pos0, t0;  // portion, its state, tokens, first row and position; first token
+};
+
+// The portion of chunk blockIdx.x, by a scan of the portions' chunk counts in every wave (no
+// barrier, no LDS); false: none.
+DRTC_DEVICE bool find_chunk(const DeltaArgs& a, ChunkAt& at) {
+  const int e = blockIdx.x, lane = threadIdx.x & 63;
+  int base = 0;  // chunks of the portions ahead of s0
+  for (int s0 = 0; s0 < a.nseg; s0 += 64) {
+    const int s = s0 + lane, c = s < a.nseg ? (a.seg_len[s] + 15) / 16 : 0;
+    int x = c;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(x, o, 64);
+      x += lane >= o ? y : 0;
+    }
+    const int first = base + x - c;
+    const uint64_t hit = __ballot(e >= first && e < first + c);
+    if (hit) {
+      const int l = __builtin_ctzll(hit), f = __builtin_amdgcn_readlane(first, l), i = s0 + l;
+      at = {i, a.seg_state[i], a.seg_len[i], a.seg_row[i], a.seg_pos[i], 16 * (e - f)};
+      return true;
+    }
+    base += __builtin_amdgcn_readlane(x, 63);
+  }
+  return false;
+}
+
+template <class T, int DT>
+__global__ __launch_bounds__(256, 5) void delta_prep_kernel(DeltaArgs a, int h0) {
+  using E = ChainEntry<DT>;
+  constexpr int DP = 16 * DT, DS = DP + 4;
+  __shared__ __attribute__((aligned(16))) float ks[16 * DS], qs[16 * DS], cs[16 * DS];
+  __shared__ float am[16][17], bm[16][17], mu[16][17], mo[16][17], be[16];
+  ChunkAt at;
+  if (!find_chunk(a, at) || at.slot < 0) return;
+  const int tid = threadIdx.x, h = h0 + blockIdx.y;
+  float* w = a.ws + ((int64_t)blockIdx.x * gridDim.y + blockIdx.y) * E::N;
+  const int hk = h / (a.H / a.Hk), cq = hk * a.dim, ck = (a.Hk + hk) * a.dim;
+  {
+    const int tok = tid >> 4, e8 = (tid & 15) * 8;
+    const bool live = at.t0 + tok < at.n && e8 < a.dim;
+    float q[8], k[8], l[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) q[j] = k[j] = l[j] = 0.f;
+    const int64_t row = at.row0 + at.t0 + tok;
+    if (live) {
+      const float decay_scale = -a.a_exp[h] * kLog2e;
+      load8(q, (const T*)a.conv + row * a.C + cq + e8);
+      load8(k, (const T*)a.conv + row * a.C + ck + e8);
+      load8(l, (const T*)a.decay + row * a.ld_decay + h * a.dim + e8);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) l[j] = decay_scale * softplus_hw(l[j] + a.dt_bias[h * a.dim + e8 + j]);
+    }
+    float sq = 0.f, sk = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      sq += q[j] * q[j];
+      sk += k[j] * k[j];
+    }
+    const float rq = rsqrtf((float)a.dim) / sqrtf(sum16(sq) + 1e-6f), rk = 1.f / sqrtf(sum16(sk) + 1e-6f);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      q[j] *= rq;
+      k[j] *= rk;
+    }
+    if (e8 < DP) {
+      store8(qs + tok * DS + e8, q);
+      store8(ks + tok * DS + e8, k);
+      store8(cs + tok * DS + e8, l);
+    }
+    if ((tid & 15) == 0)
+      be[tok] = at.t0 + tok < at.n ? sigmoid_hw(to_f32(((const T*)a.proj)[row * a.ldp + a.off_b + h])) : 0.f;
+  }
+  __syncthreads();
+  if (tid < DP) {  // running decays; keys decayed to the chunk's end
+    float run[16], acc = 0.f;
+#pragma unroll
+    for (int t = 0; t < 16; ++t) run[t] = acc += cs[t * DS + tid];
+    w[E::gt + tid] = fast_exp2(acc);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      f32x4 x;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        cs[(4 * g + r) * DS + tid] = run[4 * g + r];
+        x[r] = ks[(4 * g + r) * DS + tid] * fast_exp2(acc - run[4 * g + r]);
+      }
+      *(f32x4*)(w + E::kd + ((tid >> 4) * 64 + 16 * g + (tid & 15)) * 4) = x;
+    }
+  }
+  __syncthreads();
+  // A and B: 16 lanes to a block of 4 x 4 pairs, every lane its channels; ten blocks of the lower
+  // triangle (a pair per lane read five vectors of LDS for every product, and took 130 us of 190)
+  if (tid < 160) {
+    const int blk = tid >> 4, l16 = tid & 15;
+    const int bi = blk < 1 ? 0 : blk < 3 ? 1 : blk < 6 ? 2 : 3, bj = blk - bi * (bi + 1) / 2;
+    float A[4][4], B[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) A[i][j] = B[i][j] = 0.f;
+#pragma unroll 1
+    for (int d = 4 * l16; d < DP; d += 64) {
+      f32x4 xj[4], zj[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        xj[j] = *(const f32x4*)(ks + (4 * bj + j) * DS + d);
+        zj[j] = *(const f32x4*)(cs + (4 * bj + j) * DS + d);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const f32x4 k4 = *(const f32x4*)(ks + (4 * bi + i) * DS + d);
+        const f32x4 q4 = *(const f32x4*)(qs + (4 * bi + i) * DS + d);
+        const f32x4 c4 = *(const f32x4*)(cs + (4 * bi + i) * DS + d);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int m = 0; m < 4; ++m) {
+            const float y = xj[j][m] * fast_exp2(fminf(c4[m] - zj[j][m], 0.f));
+            A[i][j] += k4[m] * y;
+            B[i][j] += q4[m] * y;
+          }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        A[i][j] = sum_lanes<16>(A[i][j]);
+        B[i][j] = sum_lanes<16>(B[i][j]);
+        if (l16 == 4 * i + j) {
+          am[4 * bi + i][4 * bj + j] = A[i][j];
+          bm[4 * bi + i][4 * bj + j] = B[i][j];
+        }
+      }
+  }
+  __syncthreads();
+  if (tid < 64) {  // column tid & 15 of M_U by forward substitution; four rows of it of M_O = B M_U
+    const int c = tid & 15, g = tid >> 4;
+    float m[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float x = 0.f;
+#pragma unroll
+      for (int j = 0; j < i; ++j) x += am[i][j] * m[j];
+      m[i] = (i == c ? be[i] : 0.f) - be[i] * x;
+      if (g == 0) mu[i][c] = m[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float x = 0.f;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) x += j <= 4 * g + i ? bm[4 * g + i][j] * m[j] : 0.f;
+      mo[4 * g + i][c] = x;
+    }
+  }
+  // keys and queries decayed from the chunk's start, in lane order
+#pragma unroll
+  for (int i = 0; i < DT / 4 + (DT < 4); ++i) {
+    const int v = 256 * i + tid, d = 16 * (v >> 6) + 4 * ((v >> 4) & 3), t = v & 15;
+    if (DT >= 4 || v < 64 * DT) {
+      const f32x4 c4 = *(const f32x4*)(cs + t * DS + d);
+      f32x4 k4 = *(const f32x4*)(ks + t * DS + d), q4 = *(const f32x4*)(qs + t * DS + d);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float e = fast_exp2(c4[r]);
+        k4[r] *= e;
+        q4[r] *= e;
+      }
+      *(f32x4*)(w + E::ek + v * 4) = k4;
+      *(f32x4*)(w + E::eq + v * 4) = q4;
+    }
+  }
+  __syncthreads();
+  if (tid < 64) {
+    f32x4 x, y;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      x[r] = mu[tid & 15][4 * (tid >> 4) + r];
+      y[r] = mo[tid & 15][4 * (tid >> 4) + r];
+    }
+    *(f32x4*)(w + E::mu + tid * 4) = x;
+    *(f32x4*)(w + E::mo + tid * 4) = y;
+  }
+}
+
+// Waves of a workgroup divide the key channels; all of them hold the same CT column tiles of S.
+constexpr int chain_waves(int dt) { return dt < 4 ? dt : 4; }
+template <class T, int DT, int CT>
+__global__ __launch_bounds__(64 * chain_waves(DT), 2) void delta_chain_kernel(DeltaArgs a, int h0, int nh) {
+  using E = ChainEntry<DT>;
+  constexpr int NW = chain_waves(DT), TW = DT / NW;
+  static_assert(CT <= NW, "a wave to a column tile");
+  __shared__ __attribute__((aligned(16))) float part[NW * 2 * CT * 256], us[CT * 256];
+  const int seg = blockIdx.x / nh, hh = blockIdx.x % nh, h = h0 + hh;
+  const int slot = a.seg_state[seg];
+  if (slot < 0) return;
+  const int n = a.seg_len[seg], row0 = a.seg_row[seg], pos0 = a.seg_pos[seg], nch = (n + 15) / 16;
+  const int w = wave_id_uniform(), lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
+  const int x0 = 16 * CT * blockIdx.y;
+  int entry = 0;
+  for (int s = lane; s < seg; s += 64) entry += (a.seg_len[s] + 15) / 16;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) entry += __shfl_xor(entry, o, 64);
+  float* S = a.state + ((int64_t)slot * a.H + h) * a.dim * a.vdim;
+  auto state = [&](auto&& f) {
+#pragma unroll
+    for (int t = 0; t < TW; ++t)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int d = 16 * (TW * w + t) + 4 * g + r, x = x0 + 16 * ct + col;
+          f(t, ct, r, d < a.dim && x < a.vdim, S + (int64_t)d * a.vdim + x);
+        }
+  };
+  f32x4 st[TW][CT];
+  state([&](int t, int ct, int r, bool in, float* at) { st[t][ct][r] = pos0 > 0 && in ? *at : 0.f; });
+  const float* p = a.ws + ((int64_t)entry * nh + hh) * E::N;
+  // wave w < CT: R, U and O of column tile w
+  const int xo = x0 + 16 * min(w, CT - 1) + col;
+  const T* v = (const T*)a.conv + (int64_t)row0 * a.C + 2 * a.Hk * a.dim + h * a.vdim + min(xo, a.vdim - 1);
+  const int64_t ldo = (int64_t)a.H * a.vdim16;
+  float* o = a.ws_o + ((int64_t)entry * 16 + 4 * g) * ldo + h * a.vdim16 + xo;
+  const bool mine = w < CT && xo < a.vdim16;
+  // operands of two chunks: each part is loaded again, two chunks ahead, where it has been read
+  // (one chunk is shorter than a load from HBM takes)
+  struct Ops {
+    f32x4 ek[TW], eq[TW], kd[TW], gt[TW], mu, mo;
+    T v[4];
+  };
+  auto load_k = [&](Ops& x, const float* p) {
+#pragma unroll
+    for (int t = 0; t < TW; ++t) {
+      x.ek[t] = *(const f32x4*)(p + E::ek + 256 * (TW * w + t) + 4 * lane);
+      x.eq[t] = *(const f32x4*)(p + E::eq + 256 * (TW * w + t) + 4 * lane);
+    }
+  };
+  auto load_u = [&](Ops& x, const float* p) {
+#pragma unroll
+    for (int t = 0; t < TW; ++t) {
+      x.kd[t] = *(const f32x4*)(p + E::kd + 256 * (TW * w + t) + 4 * lane);
+      x.gt[t] = *(const f32x4*)(p + E::gt + 16 * (TW * w + t) + 4 * g);
+    }
+  };
+  auto load_m = [&](Ops& x, const float* p, int t0) {  // rows behind the portion's end: its last one
+    x.mu = *(const f32x4*)(p + E::mu + 4 * lane);
+    x.mo = *(const f32x4*)(p + E::mo + 4 * lane);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) x.v[r] = v[(int64_t)min(t0 + 4 * g + r, n - 1) * a.C];
+  };
+  Ops even, odd;
+  auto chunk = [&](int c) { return p + (int64_t)min(c, nch - 1) * nh * E::N; };
+  if (nch > 0) {
+    load_k(even, chunk(0));
+    load_m(even, chunk(0), 0);
+    load_u(even, chunk(0));
+    load_k(odd, chunk(1));
+    load_m(odd, chunk(1), 16);
+    load_u(odd, chunk(1));
+  }
+  float* mypart = part + w * 2 * CT * 256 + 4 * lane;
+  const float* sums = part + 256 * min(w, CT - 1) + 4 * lane;
+  auto compute = [&](int c, Ops& x) {
+    const float* ahead = chunk(c + 2);
+    f32x4 rk[CT], ok[CT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) rk[ct] = ok[ct] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < TW; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+          rk[ct] = mfma_f32(x.ek[t][r], st[t][ct][r], rk[ct]);
+          ok[ct] = mfma_f32(x.eq[t][r], st[t][ct][r], ok[ct]);
+        }
+    load_k(x, ahead);
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      *(f32x4*)(mypart + 256 * ct) = rk[ct];
+      *(f32x4*)(mypart + 256 * (CT + ct)) = ok[ct];
+    }
+    lds_barrier();
+    f32x4 res, y;
+    if (w < CT) {
+      f32x4 rs = *(const f32x4*)sums;
+      y = *(const f32x4*)(sums + 256 * CT);
+#pragma unroll
+      for (int i = 1; i < NW; ++i) {
+        rs += *(const f32x4*)(sums + i * 2 * CT * 256);
+        y += *(const f32x4*)(sums + i * 2 * CT * 256 + 256 * CT);
+      }
+      f32x4 u = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int r = 0; r < 4; ++r) res[r] = 16 * c + 4 * g + r < n ? to_f32(x.v[r]) - rs[r] : 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) u = mfma_f32(x.mu[r], res[r], u);
+      *(f32x4*)(us + 256 * w + 4 * lane) = u;
+    }
+    lds_barrier();
+    f32x4 u[CT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) u[ct] = *(const f32x4*)(us + 256 * ct + 4 * lane);
+#pragma unroll
+    for (int t = 0; t < TW; ++t)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) st[t][ct] *= x.gt[t];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int t = 0; t < TW; ++t)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) st[t][ct] = mfma_f32(x.kd[t][r], u[ct][r], st[t][ct]);
+    load_u(x, ahead);
+    if (w < CT) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) y = mfma_f32(x.mo[r], res[r], y);
+      if (mine)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[(int64_t)(16 * c + r) * ldo] = y[r];
+    }
+    load_m(x, ahead, 16 * (c + 2));
+  };
+  for (int c = 0; c < nch; c += 2) {
+    compute(c, even);
+    if (c + 1 < nch) compute(c + 1, odd);
+  }
+  state([&](int t, int ct, int r, bool in, float* at) {
+    if (in) *at = st[t][ct][r];
+  });
+}
+
+// Four heads of a chunk, NV times 8 columns per lane.
+template <class T, int NV>
+__global__ __launch_bounds__(256) void delta_read_kernel(DeltaArgs a) {
+  constexpr int NH = 4;
+  ChunkAt at;
+  if (!find_chunk(a, at)) return;
+  const int tok = threadIdx.x >> 4, l16 = threadIdx.x & 15, h0 = NH * blockIdx.y;
+  const int64_t row = at.row0 + at.t0 + tok;
+  const bool live = at.t0 + tok < at.n;
+  if (live && at.slot < 0) {  // padding row of a decode bucket
+    T* out = (T*)a.out + (row * a.H + h0) * a.vdim;
+    for (int i = l16; i < min(NH, a.H - h0) * a.vdim; i += 16) out[i] = from_f32<T>(0.f);
+  } else if (live) {
+    const float* o = a.ws_o + (((int64_t)blockIdx.x * 16 + tok) * a.H + h0) * a.vdim16;
+    const T* gate = (const T*)a.gate + row * a.ld_gate + h0 * a.vdim;
+    T* out = (T*)a.out + (row * a.H + h0) * a.vdim;
+    float x[NH][NV][8], z[NH][NV][8];
+#pragma unroll
+    for (int k = 0; k < NH; ++k)
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const int e = 128 * i + 8 * l16;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[k][i][j] = 0.f;
+        if (h0 + k < a.H && e < a.vdim) {
+          load8(x[k][i], o + k * a.vdim16 + e);
+          load8(z[k][i], gate + k * a.vdim + e);
+        }
+      }
+    float w[NV][8];
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) w[i][j] = 128 * i + 8 * l16 < a.vdim ? a.norm_w[128 * i + 8 * l16 + j] : 0.f;
+#pragma unroll
+    for (int k = 0; k < NH; ++k) {
+      float so = 0.f;
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) so += x[k][i][j] * x[k][i][j];
+      const float r = 1.f / sqrtf(sum_lanes<16>(so) / (float)a.vdim + a.eps);
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const int e = 128 * i + 8 * l16;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[k][i][j] *= r * w[i][j] * sigmoid_hw(z[k][i][j]);
+        if (h0 + k < a.H && e < a.vdim) store8(out + k * a.vdim + e, x[k][i]);
+      }
+    }
+  }
+  if (at.slot >= 0 && at.t0 + 16 >= at.n)
+    for (int h = h0; h < min(a.H, h0 + NH); ++h) keep_ring<T>(a, at.slot, h, at.n, at.row0, at.pos0);
+}
+
 template <class T, int DPL, int CPL>
 __global__ __launch_bounds__(512) void delta_decode_kernel(DeltaArgs a) {
   constexpr int DP = 8 * DPL;
@@ -849,10 +1268,43 @@ static int chunk_t(const DeltaArgs& a, hipStream_t st) {
   return chunk_go<T, 8>(a, st);
 }
 
+template <class T, int DT>
+static int chain_go(const DeltaArgs& a, hipStream_t st) {
+  const int64_t entries = a.rows / 16 + a.nseg;
+  const int nh = (int)std::min<int64_t>(a.H, a.ws_floats / (entries * ChainEntry<DT>::N));
+  if (nh < 1) return -1;
+  for (int h0 = 0; h0 < a.H; h0 += nh) {
+    const int m = std::min(nh, a.H - h0);
+    delta_prep_kernel<T, DT><<<dim3(entries, m), dim3(256), 0, st>>>(a, h0);
+    // 64 columns to a workgroup read the operands half as often; 32 where that would leave CUs idle
+    constexpr int NW = chain_waves(DT);
+    if (NW == 4 && (int64_t)a.nseg * m * ((a.vdim16 + 63) / 64) >= 512)
+      delta_chain_kernel<T, DT, NW><<<dim3(a.nseg * m, (a.vdim16 + 16 * NW - 1) / (16 * NW)), dim3(64 * NW), 0, st>>>(a, h0, m);
+    else
+      delta_chain_kernel<T, DT, 2><<<dim3(a.nseg * m, (a.vdim16 + 31) / 32), dim3(64 * NW), 0, st>>>(a, h0, m);
+  }
+  if (a.vdim <= 128) delta_read_kernel<T, 1><<<dim3(entries, (a.H + 3) / 4), dim3(256), 0, st>>>(a);
+  else delta_read_kernel<T, 2><<<dim3(entries, (a.H + 3) / 4), dim3(256), 0, st>>>(a);
+  return 0;
+}
+template <class T>
+static int chain_t(const DeltaArgs& a, hipStream_t st) {
+  if (a.dim <= 32) return chain_go<T, 2>(a, st);
+  if (a.dim <= 64) return chain_go<T, 4>(a, st);
+  return chain_go<T, 8>(a, st);
+}
+
 // cpl 0: the chunk form where the sizes allow it
 int launch_delta_scan(int f32, const DeltaArgs& a, int cpl, hipStream_t st) {
   if (a.nseg == 0) return 0;
   if (a.Hk < 1 || a.H % a.Hk) return -1;
+  if (cpl == 0 && a.ws) {
+    if (a.dim % 8 || a.vdim % 8 || a.dim > 128 || a.vdim > 256 || a.ld_decay % 8 || a.ld_gate % 8 ||
+        a.vdim16 % 16 || a.vdim16 < a.vdim || !a.ws_o)
+      return -1;
+    const int rc = f32 ? chain_t<float>(a, st) : chain_t<bf16_t>(a, st);
+    return rc ? rc : (int)hipGetLastError();
+  }
   if (cpl == 0) {
     if (a.dim % 8 == 0 && a.vdim % 8 == 0 && a.dim <= 128 && a.vdim <= 256 &&
         a.ld_decay % 8 == 0 && a.ld_gate % 8 == 0) {

@@ -103,6 +103,12 @@ struct DeltaArgs {
   const int* positions;
   const int* row_state;
   int rows;
+  // prefill in chains: operands of (rows / 16 + nseg) chunks of as many heads as fit, outputs ahead
+  // of the norm [(rows / 16 + nseg) * 16, H, vdim16] (value columns padded to 16)
+  float* ws;
+  int64_t ws_floats;
+  float* ws_o;
+  int vdim16;
 };
 int launch_short_conv(int f32, void* out, const void* proj, int ldp, const float* w,
                       const void* ring, const int* positions, const int* row_off,

@@ -102,7 +102,7 @@ def _args(proj, off_b, w: DeltaWeights, ring, state, decay, gate, out) -> dict:
                 ld_decay=decay.stride(0), gate=gate.data_ptr(), ld_gate=gate.stride(0),
                 a_exp=w.a_exp.data_ptr(), dt_bias=w.dt_bias.data_ptr(),
                 norm_w=w.norm.data_ptr(), eps=float(w.eps), H=w.heads, Hk=w.kv_heads, dim=w.dim,
-                vdim=w.vdim, taps=w.taps, C=w.channels, out=out.data_ptr(), nseg=0, rows=0)
+                vdim=w.vdim, taps=w.taps, C=w.channels, out=out.data_ptr(), nseg=0, rows=0, ws_floats=0, vdim16=0)
 
 
 def _token_ref(w: DeltaWeights, x, beta_in, decay, gate, S):
@@ -129,7 +129,7 @@ def delta_scan(proj: torch.Tensor, off_b: int, conv: torch.Tensor, w: DeltaWeigh
     """The recurrence over packed portions, each continuing its slot's state (from zero at
     position 0), then output norm and gate -> [rows, heads * vdim].  Leaves the state and the
     ring as of each portion's last token.  Rows in no portion are not written.  ``columns`` 0:
-    chunks of 8 tokens on the fp32 MFMA where the sizes allow it; 2 / 4: token by token, with
+    chunks of 8 or 16 tokens on the fp32 MFMA where the sizes allow it; 2 / 4: token by token, with
     that many state columns to a lane."""
     rows = p.row_state.numel()
     out = torch.empty((rows, w.heads * w.vdim), dtype=proj.dtype, device=proj.device)
@@ -154,10 +154,37 @@ def delta_scan(proj: torch.Tensor, off_b: int, conv: torch.Tensor, w: DeltaWeigh
         assert t.dtype == torch.int32 and t.is_cuda and t.numel() == n
     assert conv.is_contiguous() and conv.shape[1] == w.channels and conv.dtype == proj.dtype
     a.update(conv=conv.data_ptr(), seg_row=p.seg_row.data_ptr(), seg_len=p.seg_len.data_ptr(),
-             seg_pos=p.seg_pos.data_ptr(), seg_state=p.seg_state.data_ptr(), nseg=n)
+             seg_pos=p.seg_pos.data_ptr(), seg_state=p.seg_state.data_ptr(), nseg=n, rows=rows)
+    ws = _chain_workspace(w, rows, n, proj.device) if columns == 0 and _chain_ok(w, decay, gate, p) else None
+    if ws is not None:
+        a.update(ws=ws[0].data_ptr(), ws_floats=ws[0].numel(), ws_o=ws[1].data_ptr(), vdim16=-(-w.vdim // 16) * 16)
     check(hipk().delta_scan(int(proj.dtype == torch.float32), a,
                             columns, stream_ptr(proj)), "delta_scan")
     return out
+
+
+CHAIN_BYTES = 1 << 30  # operands of the chunks prepared ahead: as many heads at a time
+
+
+def _chain_ok(w: DeltaWeights, decay: torch.Tensor, gate: torch.Tensor, p: Portions) -> bool:
+    """Whether the recurrence runs as delta_prep / chain / read: where the longest portion, and not the
+    work of all, sets the time of the one-launch form.  That form has a workgroup per (portion, head),
+    the chains need operands prepared in memory; with about one workgroup per CU they are equal (16
+    heads of 128: 16 x 1,000 tokens 603 against 681 us, 20 x 150 149 against 151, 64 x 24 124 against
+    84).  Portions of a few chunks do not repay three launches (16 heads: 8 x 16 tokens 35 against
+    26 us; 32 heads: one of 48 tokens 34 against 44)."""
+    return (w.dim % 8 == w.vdim % 8 == 0 and w.dim <= 128 and w.vdim <= 256
+            and decay.stride(0) % 8 == gate.stride(0) % 8 == 0
+            and p.max_len > 32 and p.row_state.numel() * w.heads <= 256 * p.max_len)
+
+
+def _chain_workspace(w: DeltaWeights, rows: int, n: int, dev) -> tuple[torch.Tensor, torch.Tensor]:
+    """(operands, outputs ahead of the norm) of delta_chain (delta_rule.hip: ChainEntry)."""
+    chunks, tiles = rows // 16 + n, 2 if w.dim <= 32 else 4 if w.dim <= 64 else 8
+    head = chunks * (768 * tiles + 16 * tiles + 512)
+    heads = min(w.heads, max(1, CHAIN_BYTES // (4 * head)))
+    return (torch.empty(heads * head, dtype=torch.float32, device=dev),
+            torch.empty(chunks * 16 * w.heads * (-(-w.vdim // 16) * 16), dtype=torch.float32, device=dev))
 
 
 def delta_decode(proj: torch.Tensor, off_b: int, w: DeltaWeights, ring: torch.Tensor,

@@ -324,6 +324,53 @@ def test_delta_rule(target, shape, columns):
     close(state[2], states[0], t)
 
 
+CHAIN_CASES = [  # heads, key heads, dim, vdim, lengths in the order of the portions, chunk bytes
+    (2, 1, 128, 128, [33, 16, 49], 1 << 30), (3, 3, 40, 24, [64, 1, 17, 15], 1 << 30),
+    (2, 2, 24, 8, [47], 1 << 30), (4, 2, 128, 72, [40, 34], 40000 * 4),  # one head at a time
+    (16, 4, 128, 256, [34, 33, 35, 17, 32, 31, 20, 34], 1 << 30), (4, 4, 64, 136, [80, 2], 1 << 30)]
+
+
+@on
+@pytest.mark.parametrize("case", CHAIN_CASES, ids=str)
+def test_delta_chains(target, case, monkeypatch):
+    """A few long portions (chunks prepared ahead): lengths around the chunks of 16, head sizes that
+    pad, heads in several passes, 64 columns to a workgroup; portions not in the order of their rows,
+    a padding portion, and the second half of every sequence continuing the first's state."""
+    dev, dt = target
+    *shape, lens, most = case
+    H, Hk, d, dv = shape
+    monkeypatch.setattr(ops.delta, "CHAIN_BYTES", most)
+    proj, off_b, w, decay, gate, want, states = _delta_case(dev, dt, *shape, 3, lens)
+    assert ops.delta._chain_ok(w, decay, gate, _portions(dev, lens, [0] * len(lens), range(len(lens)))[0])
+    t, n = tol(dt, 5e-5, 3e-2), len(lens)
+    ring = torch.full((n, 3, w.channels), 9.0, dtype=dt, device=dev)
+    state = torch.full((n, H, d, dv), 9.0, device=dev)
+    slots = list(range(n))[::-1]
+    p, pos = _portions(dev, lens, [0] * n, slots)
+    conv = ops.short_conv(proj, w, ring, pos, p)
+    back = ops.Portions(*(x.flip(0).contiguous() for x in (p.seg_row, p.seg_len, p.seg_pos, p.seg_state)),
+                        p.row_off, p.row_state, p.max_len)
+    out = ops.delta_scan(proj, off_b, conv, w, ring, state, decay, gate, back)
+    close(out, want, t)
+    for s, S in zip(slots, states):
+        close(state[s], S, t)
+    # the longest sequence in two portions, a padding portion ahead of the second
+    m, row = max(lens), sum(lens[:lens.index(max(lens))])
+    ring.fill_(9.0), state.fill_(9.0)
+    parts, cut = [], m - m // 2 - 3
+    for a, b in ((0, cut), (cut, m)):
+        s = slice(row + a, row + b)
+        p, pos = _portions(dev, [2, b - a], [0, a], [-1, 0])
+        x, dec, g = (torch.cat([z[:2], z[s]]) for z in (proj, decay, gate))
+        conv = ops.short_conv(x, w, ring, pos, p)
+        o = ops.delta_scan(x, off_b, conv, w, ring, state, dec, g, p)
+        if dev != "cpu":
+            assert (o[:2] == 0).all()
+        parts.append(o[2:])
+    close(torch.cat(parts), want[row:row + m], t)
+    close(state[0], states[lens.index(m)], t)
+
+
 @on
 def test_delta_remembers_far_tokens(target):
     """Channels that hardly decay: a loud write hundreds of tokens back still shows."""
