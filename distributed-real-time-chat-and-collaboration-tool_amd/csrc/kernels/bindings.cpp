@@ -194,6 +194,11 @@ PYBIND11_MODULE(_hipk, m) {
   });
   m.def("ar_ipc_close", [](u64 p) { return drtc::ar_ipc_close(P<void>(p)); });
   m.def("ar_error", [](u64 base) { return drtc::ar_error(P<void>(base)); });
+  m.def("stream_gemm", [](u64 y, u64 x, u64 w, int M, int N, int K, int ldx, int ldy, int glu, int act, float limit,
+                          int slices, u64 slab, int64_t slab_bytes, u64 tickets, int n_tickets, u64 st) {
+    return drtc::launch_stream_gemm(P<void>(y), P<const void>(x), P<const void>(w), M, N, K, ldx, ldy, glu, act, limit,
+                                    slices, P<void>(slab), slab_bytes, P<void>(tickets), n_tickets, S(st));
+  });
   m.def("midm_gemm", [](u64 y, u64 x, u64 w, u64 res, int M, int N, int K, int ldx, int ldy,
                         int ldr, int epi, int splits, u64 slab, int64_t slab_bytes, u64 st) {
     return drtc::launch_midm_gemm(P<void>(y), P<const void>(x), P<const void>(w),

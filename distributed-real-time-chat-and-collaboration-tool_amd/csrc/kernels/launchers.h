@@ -190,6 +190,9 @@ void set_splitk_spin_limit(int limit);
 int configure_kernels();
 int configure_decode();
 int configure_prefill();
+// weight-streaming decode GEMM, M <= 64 (gemm_stream.hip)
+int launch_stream_gemm(void* y, const void* x, const void* w, int M, int N, int K, int ldx, int ldy, int glu, int act,
+                       float limit, int slices, void* slab, int64_t slab_bytes, void* tickets, int n_tickets, hipStream_t st);
 // medium-M decode GEMM (gemm_midm.hip)
 int64_t midm_slab_bytes(int M, int N, int S);
 int launch_midm_gemm(void* y, const void* x, const void* w, const void* res, int M, int N,

@@ -8,6 +8,7 @@ shape (M, N, K, row stride of x) ONCE to a route, cached per shape (``route``):
             persistent, 256 x 256 tiles (``mfma_gemm``)     K <= W4_MAX_K)
   "skinny"  gemv.hip weight-streaming kernels (M <= 16)     decode buckets where the table (or
                                                             ``skinny_variant`` untuned) says so
+            gemm_stream.hip (variant STREAM, M <= 64)       where ``stream_ok`` says so
   "midm"    gemm_midm.hip medium-M kernel (M <= 256)        decode buckets where the table says so
   "xd"      gemm_xd.hip: 128-row tiles, full K, tile order  decode buckets where the table says so
             partitioned by XCD (``xd_gemm``)                (full-batch qkv / o / down)
@@ -222,6 +223,8 @@ def _resolve(M: int, N: int, K: int, ldx: int) -> tuple[str, int]:
             return ("w4", 0)
         a = _prefill_algo(M, N, K, ldx, 0)
         return ("lt", a) if a >= 0 else ("torch", 0)
+    if ldx % 8 == 0 and stream_ok(M, N, K):
+        return ("skinny", STREAM)
     found = _decode_entry(M, N, K, ldx)
     if found is None:
         v = skinny_variant(M, N, K, ldx)
@@ -281,7 +284,7 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         check(hipk().lt_gemm(y.data_ptr(), x.data_ptr(), w.data_ptr(), M, N, K, x.stride(0), N,
                              0.0, stream_ptr(x)), "lt_gemm")
         return y
-    if kind == "skinny":
+    if kind == "skinny" and (arg != STREAM or _aligned(x, w)):
         return skinny_linear(x, w, arg)
     if kind == "midm":
         return midm_gemm(x, w, "store", splits=arg)
@@ -320,7 +323,9 @@ def skinny_ok(M: int, N: int, K: int, ldx: int) -> bool:
 
 
 def skinny_linear(x: torch.Tensor, w: torch.Tensor, variant: int = 0) -> torch.Tensor:
-    """y = x @ w.T on the skinny decode kernel (M <= 16 rows of x)."""
+    """y = x @ w.T on a skinny decode kernel (M <= 16 rows of x; STREAM: up to 64)."""
+    if variant == STREAM:
+        return stream_gemm(x, w)
     M, K = x.shape
     N = w.shape[0]
     variant = variant or skinny_variant(M, N, K, x.stride(0))
@@ -428,6 +433,73 @@ def glu_linear(gu: torch.Tensor, w: torch.Tensor, act: str = "silu") -> torch.Te
                                          stream_ptr(gu)), "skinny_glu_gemm")
             return y
     return linear(act_glu(gu, act), w)
+
+
+# ------------------------------------------------------------------ weight-streaming decode GEMM
+STREAM_MAX_M = 64
+# K steps of 32 that a wave's registers hold of 16, 32 or 64 rows of x (gemm_stream.hip instances)
+STREAM_KS = {1: (16, 14, 8), 2: (16, 14, 8), 4: (8,)}
+STREAM = 10  # as a variant of the skinny kernels in the router
+STREAM_ACT = {"store": (0, 0), "relu2": (0, 1), "silu": (1, 0), "gelu_tanh": (1, 1), "clamped": (1, 2)}
+
+
+def stream_slices(M: int, N: int, K: int, epi: str = "store") -> int:
+    """K slices of ``stream_gemm`` for the shape (N output columns), 0 where it does not take it."""
+    if not (1 <= M <= STREAM_MAX_M and N % 16 == 0 and N >= 16 and epi in STREAM_ACT):
+        return 0
+    mt = 1 if M <= 16 else 2 if M <= 32 else 4
+    for ks in STREAM_KS[mt]:
+        s = K // (256 * ks)
+        parts = N // 16 * mt * (1 + STREAM_ACT[epi][0])
+        if K % (256 * ks) == 0 and 1 <= s <= 16 and \
+                (s == 1 or (s * parts * 1024 <= WS_SLAB_BYTES and parts < WS_COUNTERS - 1)):
+            return s
+    return 0
+
+
+def stream_ok(M: int, N: int, K: int, epi: str = "store") -> bool:
+    """Whether a decode batch of M rows takes ``stream_gemm``, N output columns.  us against what the
+    table picks, activation pass included, both without the norm ahead (it costs the same):
+      one slice, up to 16 rows: from 24 M weights on, where the stream outlasts the first loads
+        (6144 x 4096 14.0 / 15.5, 14336 x 2048 gated 16.2 / 18.4, 32000 x 4096 46 / 65; 8192 x 2048 11.7 /
+        10.3); two rows and one stay with the dot2 form (6144 x 4096 12.0 / 11.5)
+      17 .. 32 rows: 2048 columns take what the other kernels need for 64 rows (2560 x 2048 8.1 / 11.4);
+        4096 columns leave the registers for one workgroup per CU, which pays for long W (16384 rows 29 /
+        33, 32000 51 / 65; 12800 27 / 26)
+      33 .. 64 rows: 2048 columns and long W (32768 gated 34 / 39, 64000 59 / 71; 8192 15.7 / 12.6)
+      slices: adding the parts up costs about 3 us, and more for more rows: plain products of few
+        slices (4096 x 14336 25.4 / 27.8, 2048 x 16384 17.3 / 23.2, 2048 x 7168 also at 32 rows 15.4 / 18.4;
+        4096 x 14336 at 32 rows 30.3 / 29.1, 8192 x 28672 91 / 89)"""
+    s = stream_slices(M, N, K, epi)
+    if not s or M < 3 or SKINNY_MAX_M <= 0:
+        return False
+    rows = N * (1 + STREAM_ACT[epi][0])
+    if s > 1:
+        return epi == "store" and s <= 4 and (M <= 16 or M <= 32 and s == 2 and N <= 2048)
+    if M <= 16:
+        return rows * K >= 24_000_000
+    if M <= 32:
+        return rows >= (16384 if K > 2048 else 2048)
+    return rows >= 14336
+
+
+def stream_gemm(x: torch.Tensor, w: torch.Tensor, epi: str = "store", out: torch.Tensor | None = None,
+                limit: float = 0.0) -> torch.Tensor:
+    """y = epi(x @ w.T) for at most 64 rows, csrc/kernels/gemm_stream.hip: one pass over W with x in
+    registers.  epi as ``xd_gemm``, without "residual"."""
+    M, K = x.shape
+    glu, act = STREAM_ACT[epi]
+    N = w.shape[0] // 2 if glu else w.shape[0]
+    s = stream_slices(M, N, K, epi)
+    assert s and x.dtype == w.dtype == torch.bfloat16 and x.stride(1) == 1 and w.is_contiguous() and w.shape[1] == K
+    if out is None:
+        out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    assert out.shape == (M, N) and out.stride(1) == 1 and out.dtype == x.dtype
+    slab, cnt = gemm_workspace(x.device) if s > 1 else (None, None)
+    check(hipk().stream_gemm(out.data_ptr(), x.data_ptr(), w.data_ptr(), M, N, K, x.stride(0), out.stride(0), glu, act,
+                             limit, s, ptr(slab), slab.numel() * 4 if slab is not None else 0, ptr(cnt),
+                             cnt.numel() if cnt is not None else 0, stream_ptr(x)), "stream_gemm")
+    return out
 
 
 # ------------------------------------------------------------ hand-written MFMA GEMM
@@ -784,10 +856,16 @@ def glu_form(M: int, N2: int, K: int, ldx: int, act: str = "silu") -> int:
     return form if form and xd_supported(M, N2 // 2, K, form, glu=True) else 0
 
 
+def _stream_glu_ok(x: torch.Tensor, w: torch.Tensor, act: str) -> bool:
+    return (act in GATED and _gpu_bf16(x, w) and w.shape[1] == x.shape[1] and w.shape[0] % 2 == 0
+            and stream_ok(x.shape[0], w.shape[0] // 2, x.shape[1], act))
+
+
 def fused_glu_ok(x: torch.Tensor, w: torch.Tensor, act: str) -> bool:
     """Whether ``norm_glu`` computes x [M, K] @ [gate; up]^T with the GLU inside a GEMM
-    epilogue (gemm_w4 at prefill-sized / full decode batches, or a tuned gated gemm_xd form)."""
-    if w4_glu_ok(x, w, act):
+    epilogue (gemm_w4 at prefill-sized / full decode batches, the weight-streaming GEMM at small
+    ones, or a tuned gated gemm_xd form)."""
+    if w4_glu_ok(x, w, act) or _stream_glu_ok(x, w, act) and _aligned(x, w):
         return True
     return (act in GATED and _gpu_bf16(x, w) and w.shape[1] == x.shape[1] and _aligned(x, w)
             and glu_form(x.shape[0], w.shape[0], x.shape[1], x.shape[1], act) != 0)
@@ -802,6 +880,10 @@ def norm_glu(p, w: torch.Tensor, act: str = "silu") -> torch.Tensor:
     from .activation import act_glu
 
     x = p.x
+    if act in ("silu", "gelu_tanh") and isinstance(x, torch.Tensor) and _stream_glu_ok(x, w, act):
+        xm = p.materialize()
+        if _aligned(xm, w):
+            return stream_gemm(xm, w, act)
     if (act in ("silu", "gelu_tanh") and isinstance(x, torch.Tensor) and _gpu_bf16(x, w)
             and w.shape[1] == x.shape[1] and _aligned(x, w)):
         form = glu_form(x.shape[0], w.shape[0], x.shape[1], x.shape[1])  # normed x: dense
@@ -821,6 +903,8 @@ def gated(x: torch.Tensor, w: torch.Tensor, act: str = "silu", limit: float = 0.
     the same choice of kernels as ``norm_glu``; ``limit``: bound of the clamped activation."""
     from .activation import act_glu
 
+    if _stream_glu_ok(x, w, act) and _aligned(x, w):
+        return stream_gemm(x, w, act, limit=limit)
     if fused_glu_ok(x, w, act):
         M, K = x.shape
         form = glu_form(M, w.shape[0], K, x.stride(0), act)
@@ -833,8 +917,8 @@ def gated(x: torch.Tensor, w: torch.Tensor, act: str = "silu", limit: float = 0.
 
 def squared_relu(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
     """out = relu(x @ w.T)^2, into rows of any stride (columns of a wider operand): in the
-    epilogue of gemm_w4 at prefill size and of gemm_xd where ``linear`` takes that, else a pass
-    behind ``linear``."""
+    epilogue of gemm_w4 at prefill size and of gemm_xd or the weight-streaming GEMM where ``linear``
+    takes those, else a pass behind ``linear``."""
     M, K = x.shape
     assert out.shape == (M, w.shape[0]) and out.stride(1) == 1
     if not on_gpu(x):
@@ -845,6 +929,8 @@ def squared_relu(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.T
                          group_m=w4_group_m(M, w.shape[0], K))
     if _gpu_bf16(x, w) and _aligned(x, w) and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0:
         kind, form = route(M, w.shape[0], K, x.stride(0))
+        if (kind, form) == ("skinny", STREAM):
+            return stream_gemm(x, w, "relu2", out=out)
         if kind == "xd":
             return xd_gemm(x, w, "relu2", out=out, form=form)
     y = linear(x, w)
@@ -1015,4 +1101,4 @@ __all__ = ["linear", "route", "norm_linear", "glu_linear", "norm_glu", "fused_gl
            "gemm_workspace", "new_gemm_workspace", "private_workspace", "check_splitk_fault", "SplitKFault", "SplitKWatch",
            "set_splitk_spin_limit", "skinny_linear", "skinny_ok",
            "skinny_variant", "skinny_supports", "midm_gemm", "midm_supported", "midm_splits",
-           "xd_gemm", "xd_supported", "xd_default_form", "tune", "save_entries", "load_table", "reset", "set_enabled", "table_path"]
+           "stream_gemm", "stream_ok", "stream_slices", "xd_gemm", "xd_supported", "xd_default_form", "tune", "save_entries", "load_table", "reset", "set_enabled", "table_path"]

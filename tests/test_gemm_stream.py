@@ -1,0 +1,101 @@
+"""The weight-streaming decode GEMM (csrc/kernels/gemm_stream.hip) against fp64, and its rule."""
+import pytest
+import torch
+
+from drtc_amd import ops
+from drtc_amd.ops import gemm as G
+
+
+def test_rule_takes_only_what_the_kernel_takes():
+    """Every shape that the rule accepts has a slice count whose K steps the kernel is built for, whole
+    tiles of rows and a workspace that holds the parts; others keep their routes."""
+    seen = set()
+    for M in range(0, 70):
+        for N in (8, 16, 48, 2048, 2560, 6144, 16384, 32000, 256000):
+            for K in (256, 512, 2048, 3584, 4096, 5632, 7168, 8192, 14336, 16384, 28672):
+                for epi in G.STREAM_ACT:
+                    s = G.stream_slices(M, N, K, epi)
+                    if G.stream_ok(M, N, K, epi):
+                        assert s
+                    if not s:
+                        continue
+                    mt = 1 if M <= 16 else 2 if M <= 32 else 4
+                    assert 1 <= M <= 64 and N % 16 == 0 and K % (256 * s) == 0 and K // (256 * s) in G.STREAM_KS[mt]
+                    parts = N // 16 * mt * (1 + G.STREAM_ACT[epi][0])
+                    assert s == 1 or s * parts * 1024 <= G.WS_SLAB_BYTES and parts < G.WS_COUNTERS - 1
+                    seen.add((mt, K // (256 * s), s > 1))
+    assert {(m, k) for m, k, _ in seen} == {(m, k) for m in G.STREAM_KS for k in G.STREAM_KS[m]}
+
+
+def _want(x, w, epi, N, limit):
+    r = x.double() @ w.double().t()
+    if epi == "relu2":
+        return torch.relu(r).square()
+    if epi == "store":
+        return r
+    g, u = r[:, :N], r[:, N:]
+    if epi == "clamped":
+        g = g.clamp(max=limit)
+        return g * torch.sigmoid(1.702 * g) * (u.clamp(-limit, limit) + 1)
+    f = torch.nn.functional
+    return (f.silu(g) if epi == "silu" else f.gelu(g, approximate="tanh")) * u
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 3, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N,K,epi", [(16, 2048, "store"), (4112, 4096, "store"), (8208, 2048, "silu"),
+                                     (48, 7168, "relu2"), (4096, 14336, "store"), (80, 16384, "store"),
+                                     (2064, 4096, "gelu_tanh"), (112, 8192, "clamped")])
+def test_stream_gemm(hipk, M, N, K, epi):
+    """One tile and many, more tiles than workgroups, one slice and several, rows in strides; the same
+    bits twice, tickets left at zero, and in replays of a graph on new inputs between other work."""
+    if not G.stream_slices(M, N, K, epi):
+        pytest.skip("not an instance")
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    buf = torch.randn(M, K + 24, device="cuda", generator=g).to(torch.bfloat16)
+    x = buf[:, 8:K + 8]
+    w = (torch.randn(N * (1 + G.STREAM_ACT[epi][0]), K, device="cuda", generator=g) * 0.03).to(torch.bfloat16)
+    out = torch.full((M + 1, N + 8), 7.0, device="cuda", dtype=torch.bfloat16)
+
+    def check(y):
+        # fp32 sums of K products: far below the rounding of the result to bf16 (2^-9 of each value)
+        r = _want(x, w, epi, N, 0.8)
+        assert (y.double() - r).norm() <= 2 ** -9 * 1.1 * r.norm() + 1e-5 * K ** 0.5
+
+    G.stream_gemm(x, w, epi, out=out[:M, :N], limit=0.8)
+    check(out[:M, :N])
+    assert (out[M] == 7).all() and (out[:, N:] == 7).all()
+    assert torch.equal(G.stream_gemm(x, w, epi, limit=0.8), out[:M, :N])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = G.stream_gemm(x, w, epi, limit=0.8)
+    for _ in range(3):
+        buf.normal_(generator=g)
+        graph.replay()
+        check(y)
+        assert torch.equal(G.stream_gemm(x, w, epi, limit=0.8), y)
+    assert int(G.gemm_workspace(x.device)[1].abs().sum()) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [3, 16, 32])
+def test_routes_to_the_stream(hipk, M):
+    """linear, norm_glu, gated and squared_relu at a shape of the rule: the same numbers as the kernel
+    itself, unaligned rows through another route."""
+    K, N = 4096, 16384
+    g = torch.Generator(device="cuda").manual_seed(M)
+    buf = torch.randn(M * K + 8, device="cuda", generator=g).to(torch.bfloat16)
+    x, nw = buf[:M * K].view(M, K), torch.ones(K, device="cuda", dtype=torch.bfloat16)
+    w = (torch.randn(N, K, device="cuda", generator=g) * 0.03).to(torch.bfloat16)
+    G.reset()
+    assert G.route(M, N, K, K) == ("skinny", G.STREAM)
+    assert torch.equal(ops.linear(x, w), G.stream_gemm(x, w))
+    odd = buf[1:M * K + 1].view(M, K)
+    assert (ops.linear(odd, w).double() - odd.double() @ w.double().t()).norm() < 0.01 * (K ** 0.5) * (M * N) ** 0.5
+    assert ops.gemm.fused_glu_ok(x, w, "silu")
+    xn = ops.rmsnorm(x, nw, 1e-5)
+    assert torch.equal(ops.norm_glu(ops.PendingNorm(x, None, nw, 1e-5, False), w, "silu"), G.stream_gemm(xn, w, "silu"))
+    assert torch.equal(ops.gated(x, w, "clamped", 0.9), G.stream_gemm(x, w, "clamped", limit=0.9))
+    out = torch.zeros(M, N + 8, device="cuda", dtype=torch.bfloat16)
+    ops.squared_relu(x, w, out[:, 8:])
+    assert torch.equal(out[:, 8:], G.stream_gemm(x, w, "relu2")) and (out[:, :8] == 0).all()
