@@ -152,6 +152,7 @@ __global__ __launch_bounds__(512, KS * (1 + MT) <= 16 ? 4 : 2) void stream_gemm_
   // slices: a wave's sum waits here for the end (one at most, see go): publishing drains its loads
   f32x4 held[TP];
   int held_t = -1, held_mt = 0, buf = 0;
+#pragma unroll 1
   for (int u = 0;; ++u) {  // gated: u counts gate and up tiles
     const int i = u / TP, t = b + i * G, p = u % TP, p1 = (u + 1) % TP, t1 = b + (u + 1) / TP * G;
     if (t >= tiles) break;
@@ -191,6 +192,138 @@ __global__ __launch_bounds__(512, KS * (1 + MT) <= 16 ? 4 : 2) void stream_gemm_
   if (held_t >= 0) publish(held_t, held_mt, held);
 }
 
+// The same over the experts of a mixture: entry i of the device's table is up to 16 MT rows of x for one
+// expert's matrix.  The (entry, tile) pairs in order are dealt to the workgroups in equal runs, so a run
+// seldom changes its expert; the stream of W goes on while x is read again.  GATHER: rows of x by token.
+struct StreamMoe {
+  bf16_t* y;
+  const bf16_t* x;
+  const bf16_t* w;
+  int N, K, ldx, ldy, act;  // N: rows of an expert's matrix, gated: half of them
+  float limit;
+  int64_t w_stride;         // elements of an expert's matrix
+  const int *tok, *expert, *row0, *rows, *n;
+};
+template <int KS, int MT, bool GLU, bool GATHER, int NW>
+__global__ __launch_bounds__(64 * NW, KS * (1 + MT) <= 16 && !GLU ? 4 : 2) void stream_moe_kernel(StreamMoe a) {
+  static_assert(KS % 2 == 0, "loads come in pairs");
+  constexpr int TP = GLU ? 2 : 1;
+  __shared__ __attribute__((aligned(16))) f32x4 red[2][NW][TP][MT][64];
+  const int wv = wave_id_uniform(), lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int tiles = a.N / 16, units = a.n[0] * tiles, k0 = wv * (32 * KS);
+  const int q0 = (int)((int64_t)blockIdx.x * units / gridDim.x), q1 = (int)((int64_t)(blockIdx.x + 1) * units / gridDim.x);
+  if (q0 >= q1) return;
+  const bool low = r < 8;
+  const bf16_t* wa = a.w + (int64_t)(r & 7) * a.K + k0 + (low ? 8 * g : 32 + 8 * g);
+  const bf16_t* wb = a.w + (int64_t)(8 + (r & 7)) * a.K + k0 + (low ? 32 + 8 * g : 8 * g);
+  int ei = q0 / tiles, t = q0 - ei * tiles;
+  auto rows = [&](int64_t base, int t, int p) { return base + ((int64_t)p * a.N + 16 * t) * a.K; };
+  int64_t base = a.expert[ei] * a.w_stride;  // this entry's matrix
+  bf16x8 wr[KS], xb[MT][KS];
+  {
+    const int64_t at = rows(base, t, 0);
+#pragma unroll
+    for (int s = 0; s < KS; s += 2) {
+      wr[s] = load_once(wa + at + 32 * s);
+      wr[s + 1] = load_once(wb + at + 32 * s);
+    }
+  }
+  const bf16x8 zero = {};
+  int row0 = 0, nr = 0, buf = 0, first = 0;
+  bool fresh = true;
+#pragma unroll 1
+  for (int u = q0 * TP; u < q1 * TP; ++u) {
+    const int p = u % TP;
+    if (fresh) {  // x of this entry
+      row0 = a.row0[ei];
+      nr = a.rows[ei];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        const int m = min(16 * mt + r, nr - 1);
+        const bf16_t* xp = a.x + (int64_t)(GATHER ? a.tok[row0 + m] : row0 + m) * a.ldx + k0 + 8 * g;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) xb[mt][s] = load_bf16x8(xp + 32 * s);
+      }
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+          if (16 * mt + r >= nr) xb[mt][s] = zero;
+      fresh = false;
+    }
+    // the tile after this one
+    const int e0 = ei, t0 = t;
+    const int64_t b0 = base;
+    if (p == TP - 1 && ++t == tiles) {
+      t = 0;
+      ++ei;
+      if (u + 1 < q1 * TP) base = a.expert[ei] * a.w_stride;
+      fresh = true;
+    }
+    const bool more = u + 1 < q1 * TP;
+    const int64_t next = p == TP - 1 ? rows(base, t, 0) : rows(b0, t0, 1);
+    const bf16_t* na = more ? wa + next : a.w;
+    const bf16_t* nb = more ? wb + next : a.w;
+    f32x4 acc[MT][2];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[mt][0] = acc[mt][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < KS; s += 2) {
+      const u32x4 x = *(const u32x4*)&wr[s], z = *(const u32x4*)&wr[s + 1];
+      u32x4 f0, f1;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        f0[i] = low ? x[i] : z[i];
+        f1[i] = low ? z[i] : x[i];
+      }
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        acc[mt][0] = mfma16(*(const bf16x8*)&f0, xb[mt][s], acc[mt][0]);
+        acc[mt][1] = mfma16(*(const bf16x8*)&f1, xb[mt][s + 1], acc[mt][1]);
+      }
+      wr[s] = load_once(na + 32 * s);
+      wr[s + 1] = load_once(nb + 32 * s);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      f32x4 v = acc[mt][0];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] += __shfl_xor(acc[mt][1][j], 32, 64);
+      red[buf][wv][p][mt][lane] = v;
+    }
+    if (p != TP - 1) continue;
+    lds_barrier();
+    int mt = wv - first;  // MT of the waves from ``first`` on, the next ones for the next tile
+    mt += mt < 0 ? NW : 0;
+    first = (first + MT) % NW;
+    if (mt < MT) {
+      f32x4 v[TP];
+#pragma unroll
+      for (int q = 0; q < TP; ++q) {
+        v[q] = red[buf][0][q][mt][lane];
+#pragma unroll
+        for (int j = 1; j < NW; ++j) v[q] += red[buf][j][q][mt][lane];
+      }
+      if (16 * mt + r < nr) {
+        bf16x4 o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float f;
+          if constexpr (GLU)
+            f = a.act == 0 ? glu_value<0>(v[0][i], v[1][i], 0.f) : a.act == 1 ? glu_value<1>(v[0][i], v[1][i], 0.f)
+                                                                 : glu_value<2>(v[0][i], v[1][i], a.limit);
+          else
+            f = a.act == 3 ? fmaxf(v[0][i], 0.f) * fmaxf(v[0][i], 0.f) : v[0][i];
+          o[i] = f2bf(f);
+        }
+        *reinterpret_cast<bf16x4*>(a.y + (int64_t)(row0 + 16 * mt + r) * a.ldy + 16 * t0 + 4 * g) = o;
+      }
+    }
+    buf ^= 1;
+  }
+}
+
 template <int KS, int MT, bool GLU>
 int go(const StreamArgs& a, hipStream_t st) {
   // one round of workgroups, two to a CU where the registers allow it
@@ -204,6 +337,37 @@ int go(const StreamArgs& a, hipStream_t st) {
 template <int KS, int MT>
 int form(const StreamArgs& a, bool glu, hipStream_t st) {
   return glu ? go<KS, MT, true>(a, st) : go<KS, MT, false>(a, st);
+}
+
+// K steps and waves of stream_moe for K columns, {0, 0}: none
+struct MoeCut { int ks, nw; };
+MoeCut moe_cut(int K, int mt) {
+  for (const MoeCut c : {MoeCut{8, 8}, MoeCut{8, 7}, MoeCut{16, 8}, MoeCut{14, 8}})
+    if (K == 32 * c.ks * c.nw && (mt <= 2 || c.ks == 8)) return c;
+  return {0, 0};
+}
+template <int MT, bool GLU, bool GATHER>
+int moe_go(const StreamMoe& a, hipStream_t st) {
+  const MoeCut c = moe_cut(a.K, MT);
+#define DRTC_MOE_CUT(KS, NW)                                                                                        \
+  if (c.ks == KS && c.nw == NW) {                                                                                   \
+    stream_moe_kernel<KS, MT, GLU, GATHER, NW>                                                                      \
+        <<<dim3(KS * (1 + MT) <= 16 && !GLU ? 512 : 256), dim3(64 * NW), 0, st>>>(a);                               \
+    return (int)hipGetLastError();                                                                                  \
+  }
+  DRTC_MOE_CUT(8, 8)
+  DRTC_MOE_CUT(8, 7)
+  if constexpr (MT <= 2) {
+    DRTC_MOE_CUT(16, 8)
+    DRTC_MOE_CUT(14, 8)
+  }
+#undef DRTC_MOE_CUT
+  return -1;
+}
+template <int MT>
+int moe_form(const StreamMoe& a, bool glu, bool gather, hipStream_t st) {
+  if (glu) return gather ? moe_go<MT, true, true>(a, st) : -1;
+  return gather ? moe_go<MT, false, true>(a, st) : moe_go<MT, false, false>(a, st);
 }
 
 }  // namespace
@@ -229,6 +393,34 @@ int launch_stream_gemm(void* y, const void* x, const void* w, int M, int N, int 
   DRTC_STREAM(8, 2) DRTC_STREAM(14, 2) DRTC_STREAM(16, 2)
   DRTC_STREAM(8, 4)
 #undef DRTC_STREAM
+  return -1;
+}
+
+// Tiles of 16 rows that a table entry of the streamed experts holds where they hold ``rows_e`` rows on
+// average (1, 2, 4), 0: not taken.  H and I: the columns of the experts' matrices.  An expert with more
+// rows than an entry is streamed again, so entries hold half as many more than the average.  us of a whole
+// layer against variants 1 and 3, rows: 2048 x 1792, 16 gated experts, 3: 75 / 97, 103; 24: 83 / 100, 105;
+// 40: 88 / 101, 106; 50: 105 / 104, 108.  20 squared-relu ones, 40: 89 / 112, 112; 60: 104 / 118, 118.
+// 4096 x 3584, gated, 3: 226 / 283, 244; 12: 266 / 296, 259; squared relu, 2: 209 / 293, 255; 19: 221 / 290,
+// 259.
+int stream_moe_tiles(int rows_e, int H, int I, bool glu) {
+  if (H % 16 || I % 16 || H > 16384 || I > 16384) return 0;
+  const bool wide = H > 2048 || I > 2048;  // registers for 32 rows at most
+  const int mt = rows_e <= 10 ? 1 : rows_e <= 22 && !(wide && glu) ? 2 : rows_e <= (glu ? 44 : 60) && !wide ? 4 : 0;
+  return mt && moe_cut(H, mt).ks && moe_cut(I, mt).ks ? mt : 0;
+}
+
+// act: of launch_moe (3: squared relu without a gate, 4: none); tok: rows of x by token, or null.
+int launch_stream_moe(void* y, const void* x, const void* w, int N, int K, int ldx, int ldy, int mt, int act,
+                      float limit, int64_t w_stride, const int* tok, const int* expert, const int* row0,
+                      const int* rows, const int* n, hipStream_t st) {
+  const bool glu = act < 3;
+  if (N % 16 || ldx % 8 || ldy % 4 || act < 0 || act > 4 || (glu && !tok)) return -1;
+  const StreamMoe a{(bf16_t*)y, (const bf16_t*)x, (const bf16_t*)w, N, K, ldx, ldy, act, limit, w_stride, tok,
+                    expert, row0, rows, n};
+  if (mt == 1) return moe_form<1>(a, glu, tok != nullptr, st);
+  if (mt == 2) return moe_form<2>(a, glu, tok != nullptr, st);
+  if (mt == 4) return moe_form<4>(a, glu, tok != nullptr, st);
   return -1;
 }
 

@@ -193,6 +193,11 @@ int configure_prefill();
 // weight-streaming decode GEMM, M <= 64 (gemm_stream.hip)
 int launch_stream_gemm(void* y, const void* x, const void* w, int M, int N, int K, int ldx, int ldy, int glu, int act,
                        float limit, int slices, void* slab, int64_t slab_bytes, void* tickets, int n_tickets, hipStream_t st);
+// ... over the experts of a mixture (moe.hip variant 5)
+int stream_moe_tiles(int rows_e, int H, int I, bool glu);
+int launch_stream_moe(void* y, const void* x, const void* w, int N, int K, int ldx, int ldy, int mt, int act,
+                      float limit, int64_t w_stride, const int* tok, const int* expert, const int* row0,
+                      const int* rows, const int* n, hipStream_t st);
 // medium-M decode GEMM (gemm_midm.hip)
 int64_t midm_slab_bytes(int M, int N, int S);
 int launch_midm_gemm(void* y, const void* x, const void* w, const void* res, int M, int N,

@@ -3,6 +3,7 @@
 // hipGraph-capturable - the decode step of Mixtral replays with no host sync.
 //
 //   moe_router_kernel     router logits in fp32, [E, T] (routing that must not round them)
+//   moe_plan_kernel       the next three in one workgroup, for decode batches
 //   moe_route / offsets / scatter   top-k over the router logits (+ softmax over the
 //                         selected logits), within the best groups of neighbouring experts
 //                         where a design limits a token to some; stable counting sort of the
@@ -57,9 +58,77 @@ constexpr int kMoeRouteWG = 256;
 DRTC_DEVICE float logit_f32(float x) { return fmaxf(x, -3.0e38f); }
 DRTC_DEVICE float logit_f32(bf16_t x) { return logit_f32(bf2f(x)); }
 
-// L: type of the logits; KM: bound of k (the sorted list in registers).  groups > 1: experts form
-// that many equal groups of neighbours, and only those of the ``keep`` groups with the largest
-// logits can be chosen (ties: the lower group).
+// The choice of token t: experts id[0 .. k), best first, and their weights w; all in registers.  L: type
+// of the logits; KM: bound of k.  groups > 1: experts form that many equal groups of neighbours, and only
+// those of the ``keep`` groups with the largest logits can be chosen (ties: the lower group); gmax: one
+// float per group and thread of a workgroup of NT.
+template <class L, int KM, int NT>
+DRTC_DEVICE void moe_choose(const L* logits, int t, int E, int k, int lts, int les, int groups, int keep, float* gmax,
+                            int (&id)[KM], float (&w)[KM]) {
+  const int tid = threadIdx.x;
+  // logit (t, e) at t * lts + e * les: [T, E] rows, or the router GEMM's [E, T] output read
+  // in place (lts = 1: consecutive threads read consecutive tokens of one expert row)
+  const L* lr = logits + (int64_t)t * lts;
+  const int per = E / groups;
+  uint64_t open = ~0ull;
+  if (groups > 1) {
+    for (int g = 0; g < groups; ++g) {
+      float m = -INFINITY;
+      for (int e = g * per; e < (g + 1) * per; ++e) m = fmaxf(m, logit_f32(lr[(int64_t)e * les]));
+      gmax[g * NT + tid] = m;
+    }
+    open = 0;
+    for (int g = 0; g < groups; ++g) {
+      const float m = gmax[g * NT + tid];
+      int ahead = 0;
+      for (int o = 0; o < groups; ++o) {
+        const float mo = gmax[o * NT + tid];
+        ahead += mo > m || (mo == m && o < g);
+      }
+      if (ahead < keep) open |= 1ull << g;
+    }
+  }
+  // sorted top list kept in registers (fully unrolled: no scratch), as one integer each - the logit's
+  // bits in an order that compares as the logits do, then the complement of the expert's number: one
+  // comparison settles value and tie, also for entries carried down the list
+  uint64_t top[KM];
+#pragma unroll
+  for (int j = 0; j < KM; ++j) top[j] = 0;
+  for (int g = 0; g < groups; ++g) {
+    if (!(open >> g & 1)) continue;
+    for (int e0 = g * per; e0 < (g + 1) * per; e0 += 8) {
+      const int ne = min(8, (g + 1) * per - e0);
+      float xs[8];  // loads in flight together
+#pragma unroll
+      for (int i = 0; i < 8; ++i) xs[i] = logit_f32(lr[(int64_t)(e0 + min(i, ne - 1)) * les]);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint32_t u = __float_as_uint(xs[i] + 0.f);  // -0 is 0
+        const uint32_t key = u ^ (u >> 31 ? 0xffffffffu : 0x80000000u);
+        uint64_t x = i < ne ? (uint64_t)key << 32 | (uint32_t)~(e0 + i) : 0;  // behind the last: never in
+#pragma unroll
+        for (int j = 0; j < KM; ++j) {
+          const uint64_t hi = x > top[j] ? x : top[j];
+          x = x > top[j] ? top[j] : x;
+          top[j] = hi;
+        }
+      }
+    }
+  }
+  float v[KM];
+#pragma unroll
+  for (int j = 0; j < KM; ++j) {
+    const uint32_t key = top[j] >> 32;
+    v[j] = __uint_as_float(key ^ (key >> 31 ? 0x80000000u : 0xffffffffu));
+    id[j] = (int)~(uint32_t)top[j];
+  }
+  float s = 0.f;
+#pragma unroll
+  for (int j = 0; j < KM; ++j) s += (j < k) ? __expf(v[j] - v[0]) : 0.f;
+#pragma unroll
+  for (int j = 0; j < KM; ++j) w[j] = __expf(v[j] - v[0]) / s;
+}
+
 template <class L, int KM>
 __global__ __launch_bounds__(kMoeRouteWG) void moe_route_kernel(
     const L* __restrict__ logits, int T, int E, int k, int lts, int les, int groups, int keep,
@@ -71,63 +140,13 @@ __global__ __launch_bounds__(kMoeRouteWG) void moe_route_kernel(
   __syncthreads();
   const int t = blockIdx.x * kMoeRouteWG + tid;
   if (t < T) {
-    // logit (t, e) at t * lts + e * les: [T, E] rows, or the router GEMM's [E, T] output read
-    // in place (lts = 1: consecutive threads read consecutive tokens of one expert row)
-    const L* lr = logits + (int64_t)t * lts;
-    const int per = E / groups;
-    uint64_t open = ~0ull;
-    if (groups > 1) {
-      for (int g = 0; g < groups; ++g) {
-        float m = -INFINITY;
-        for (int e = g * per; e < (g + 1) * per; ++e) m = fmaxf(m, logit_f32(lr[(int64_t)e * les]));
-        gmax[g * kMoeRouteWG + tid] = m;
-      }
-      open = 0;
-      for (int g = 0; g < groups; ++g) {
-        const float m = gmax[g * kMoeRouteWG + tid];
-        int ahead = 0;
-        for (int o = 0; o < groups; ++o) {
-          const float mo = gmax[o * kMoeRouteWG + tid];
-          ahead += mo > m || (mo == m && o < g);
-        }
-        if (ahead < keep) open |= 1ull << g;
-      }
-    }
-    // sorted top list kept in registers (fully unrolled: no scratch)
-    float v[KM];
     int id[KM];
-#pragma unroll
-    for (int j = 0; j < KM; ++j) { v[j] = -INFINITY; id[j] = 0x7fffffff; }
-    for (int g = 0; g < groups; ++g) {
-      if (!(open >> g & 1)) continue;
-      for (int e0 = g * per; e0 < (g + 1) * per; e0 += 8) {
-        const int ne = min(8, (g + 1) * per - e0);
-        float xs[8];  // loads in flight together
-#pragma unroll
-        for (int i = 0; i < 8; ++i) xs[i] = logit_f32(lr[(int64_t)(e0 + min(i, ne - 1)) * les]);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          float x = i < ne ? xs[i] : -INFINITY;  // behind the last: never in the list
-          int xi = i < ne ? e0 + i : 0x7fffffff;
-#pragma unroll
-          for (int j = 0; j < KM; ++j) {
-            // order (value desc, id asc): a displaced entry carried down the list
-            // must not overtake an equal-valued entry with a higher id
-            if (x > v[j] || (x == v[j] && xi < id[j])) {
-              const float tv = v[j]; const int ti = id[j];
-              v[j] = x; id[j] = xi; x = tv; xi = ti;
-            }
-          }
-        }
-      }
-    }
-    float s = 0.f;
-#pragma unroll
-    for (int j = 0; j < KM; ++j) s += (j < k) ? __expf(v[j] - v[0]) : 0.f;
+    float w[KM];
+    moe_choose<L, KM, kMoeRouteWG>(logits, t, E, k, lts, les, groups, keep, gmax, id, w);
 #pragma unroll
     for (int j = 0; j < KM; ++j) {
       if (j < k) {
-        topk_w[t * k + j] = __expf(v[j] - v[0]) / s;
+        topk_w[t * k + j] = w[j];
         topi[t * k + j] = id[j];
         atomicAdd(&hist[id[j]], 1);  // a count: its order does not matter
       }
@@ -135,6 +154,110 @@ __global__ __launch_bounds__(kMoeRouteWG) void moe_route_kernel(
   }
   __syncthreads();
   for (int e = tid; e < E; e += kMoeRouteWG) wg_cnt[blockIdx.x * E + e] = hist[e];
+}
+
+// The three passes in one workgroup for decode batches: nothing crosses memory between them.  224
+// tokens, 16 experts, 4 per token: 9 us against 11 + 5 + 7.  NT 256 or 1024 threads, one per token; the
+// order of an expert's pairs is (slot, token).
+struct MoePlan {
+  int* sorted_tok;
+  float* sorted_w;
+  int* inv_pos;
+  float* topk_w;
+  int *tile_expert, *tile_row0, *tile_rows, *n_tiles, *local_range, *grp_off;
+  int max_tiles, e_off, e_local, bm;
+};
+template <class L, int KM, int NT>
+__global__ __launch_bounds__(NT) void moe_plan_kernel(const L* __restrict__ logits, int T, int E, int k, int lts,
+                                                      int les, int groups, int keep, MoePlan p) {
+  extern __shared__ float gmax[];  // [groups][NT] (groups > 1)
+  __shared__ int run[256], off[257], toff[257], wcnt[NT / 64][256];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  for (int e = t; e < E; e += NT) run[e] = 0;
+  __syncthreads();
+  int id[KM];
+  float w[KM];
+#pragma unroll
+  for (int j = 0; j < KM; ++j) id[j] = -1;
+  if (t < T) {
+    moe_choose<L, KM, NT>(logits, t, E, k, lts, les, groups, keep, gmax, id, w);
+#pragma unroll
+    for (int j = 0; j < KM; ++j)
+      if (j < k) {
+        p.topk_w[t * k + j] = w[j];
+        atomicAdd(&run[id[j]], 1);  // a count: its order does not matter
+      }
+  }
+  __syncthreads();
+  if (wv == 0) {  // offsets of pairs and row tiles, 64 experts at a time
+    int o = 0, to = 0;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      const int e = e0 + lane, c = e < E ? run[e] : 0;
+      const bool loc = e >= p.e_off && e < p.e_off + p.e_local;  // tiles only for this rank's experts (EP)
+      const int n = loc ? (c + p.bm - 1) / p.bm : 0;
+      int x = c, y = n;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int a = __shfl_up(x, d, 64), b = __shfl_up(y, d, 64);
+        x += lane >= d ? a : 0;
+        y += lane >= d ? b : 0;
+      }
+      if (e < E) {
+        off[e] = o + x - c;
+        toff[e] = to + y - n;
+      }
+      o += __builtin_amdgcn_readlane(x, 63);
+      to += __builtin_amdgcn_readlane(y, 63);
+    }
+    if (lane == 0) {
+      off[E] = o;
+      toff[E] = to;
+    }
+  }
+  __syncthreads();
+  if (t == 0) {
+    p.n_tiles[0] = min(toff[E], p.max_tiles);
+    p.local_range[0] = off[p.e_off];
+    p.local_range[1] = off[p.e_off + p.e_local];
+  }
+  if (p.grp_off != nullptr && t <= p.e_local) p.grp_off[t] = off[p.e_off + t];
+  for (int e = t; e < E; e += NT) {
+    const int c = off[e + 1] - off[e], nt = toff[e + 1] - toff[e];
+    for (int i = 0; i < nt && toff[e] + i < p.max_tiles; ++i) {
+      const int ti = toff[e] + i;
+      p.tile_expert[ti] = e - p.e_off;  // local weight index
+      p.tile_row0[ti] = off[e] + i * p.bm;
+      p.tile_rows[ti] = min(p.bm, c - i * p.bm);
+    }
+    run[e] = off[e];
+  }
+  const uint64_t below = (1ull << lane) - 1;
+#pragma unroll
+  for (int j = 0; j < KM; ++j) {
+    if (j >= k) break;
+    const int e = id[j];
+    int rank = 0;
+    for (int x = 0; x < E; ++x) {  // this wave's pairs of expert x, in lane order
+      const uint64_t m = __ballot(e == x);
+      if (e == x) rank = __popcll(m & below);
+      if (lane == 0) wcnt[wv][x] = __popcll(m);
+    }
+    __syncthreads();
+    if (e >= 0) {
+      int r = run[e] + rank;
+      for (int v = 0; v < wv; ++v) r += wcnt[v][e];
+      p.sorted_tok[r] = t;
+      p.sorted_w[r] = w[j];
+      p.inv_pos[t * k + j] = r;
+    }
+    __syncthreads();
+    for (int x = t; x < E; x += NT) {
+      int c = 0;
+      for (int v = 0; v < NT / 64; ++v) c += wcnt[v][x];
+      run[x] += c;
+    }
+    __syncthreads();
+  }
 }
 
 // Router logits in fp32, transposed: out[e * T + t] = w[e] . x[t].  Workgroup: 32 tokens, every
@@ -892,7 +1015,8 @@ int launch_moe(void* out, const void* x, const void* router_logits, const void* 
   if (opt.f32) variant = 0;
   const int P = T * k;
   // GEMM structure: 0 = 128-row 2-barrier (small tiles, decode), 1 = 128-row
-  // 3-stage pipeline, 2 = 256-row 3-stage pipeline, 3 = gemm_xd grouped mode (gate_up with
+  // 3-stage pipeline, 2 = 256-row 3-stage pipeline, 5 = gemm_stream's form for a few rows per expert
+  // (weights straight to registers), 3 = gemm_xd grouped mode (gate_up with
   // the GLU in its epilogue and down, forms gu_form / dn_form; 0 = by rows per expert);
   // -1 = pick by rows per expert (scripts/moe_bench.py, Mixtral shapes)
   const int rows_e = P / e_local;
@@ -901,8 +1025,12 @@ int launch_moe(void* out, const void* x, const void* router_logits, const void* 
   // expert-ordered rows; Mixtral shapes, profiles/r6j: 770 / 917 / 1061 TF/s at T = 1024 /
   // 2048 / 4096 against 703 / 841 / 1019 on variant 3), gemm_xd's grouped forms from ~a
   // 96-row tile
-  if (auto_v) variant = rows_e >= kMoeW4Rows ? 4 : (rows_e >= 96 ? 3 : 1);
-  if (variant > 4) return -1;
+  const int stream_mt = opt.f32 ? 0 : stream_moe_tiles(rows_e, H, I, glu);
+  // ... below it where an expert's matrix is large (us of a layer, variants 1 / 3: 8 x 4096 x 14336, 16
+  // tokens 526 / 475, 256 tokens 561 / 535; 20 x 2048 x 3584 178 / 159; 16 x 2048 x 1792 102 / 107)
+  if (auto_v)
+    variant = rows_e >= kMoeW4Rows ? 4 : rows_e >= 96 ? 3 : stream_mt ? 5 : (int64_t)H * I >= 6 << 20 ? 3 : 1;
+  if (variant > 5 || (variant == 5 && !stream_mt)) return -1;
   // variant 4: the persistent GEMM's prologue stages two K tiles; the down reduction is I
   if (variant == 4 && (H / 64 < 2 || I % (glu ? 128 : 256) || I / 64 < 2 || H % 256)) {
     if (!auto_v) return -1;
@@ -949,7 +1077,7 @@ int launch_moe(void* out, const void* x, const void* router_logits, const void* 
     }
   }
   const int bm = variant == 3 ? 128 * ((gu_form % 1000) / 100)
-                              : (variant == 2 || variant == 4 ? 256 : 128);
+                              : (variant == 2 || variant == 4 ? 256 : variant == 5 ? 16 * stream_mt : 128);
   const int max_tiles = (P + bm - 1) / bm + e_local;
   // workspace carve (all 256-B aligned)
   auto align = [](int64_t v) { return (v + 255) & ~int64_t(255); };
@@ -978,23 +1106,45 @@ int launch_moe(void* out, const void* x, const void* router_logits, const void* 
   const bool dn_split = variant == 4 && dn_form == 0 && dn_tiles < kMoeW4SplitTiles &&
                         (I / 64) % 2 == 0 && I / 128 >= 2;
   const int route_lds = opt.groups > 1 ? opt.groups * kMoeRouteWG * 4 : 0;
+  if (T <= kMoeRouteWG || (T <= 1024 && opt.groups == 1)) {
+    const MoePlan plan{sorted_tok, sorted_w, inv_pos, topk_w, t_e, t_r0, t_n, n_tiles, local_range,
+                       variant == 4 ? grp_off : nullptr, max_tiles, e_off, e_local, bm};
+#define DRTC_PLAN_T(L, KM, NT) \
+  moe_plan_kernel<L, KM, NT><<<dim3(1), dim3(NT), route_lds, st>>>((const L*)router_logits, T, E, k, logit_ts, logit_es, opt.groups, opt.keep, plan)
+#define DRTC_PLAN(L)                                        \
+  if (T <= kMoeRouteWG) {                                   \
+    if (k <= 4) DRTC_PLAN_T(L, 4, kMoeRouteWG);             \
+    else if (k <= 8) DRTC_PLAN_T(L, 8, kMoeRouteWG);        \
+    else DRTC_PLAN_T(L, 16, kMoeRouteWG);                   \
+  } else {                                                  \
+    if (k <= 4) DRTC_PLAN_T(L, 4, 1024);                    \
+    else if (k <= 8) DRTC_PLAN_T(L, 8, 1024);               \
+    else DRTC_PLAN_T(L, 16, 1024);                          \
+  }
+    if (opt.logits_f32) { DRTC_PLAN(float) } else { DRTC_PLAN(bf16_t) }
+#undef DRTC_PLAN
+#undef DRTC_PLAN_T
+  } else {
 #define DRTC_ROUTE(L, KM)                                                                       \
   moe_route_kernel<L, KM><<<dim3(G), dim3(kMoeRouteWG), route_lds, st>>>(                       \
       (const L*)router_logits, T, E, k, logit_ts, logit_es, opt.groups, opt.keep, inv_pos,      \
       topk_w, wg_cnt)
-  if (opt.logits_f32) {
-    if (k <= 8) DRTC_ROUTE(float, 8);
-    else DRTC_ROUTE(float, 16);
-  } else {
-    if (k <= 8) DRTC_ROUTE(bf16_t, 8);
-    else DRTC_ROUTE(bf16_t, 16);
-  }
+    if (opt.logits_f32) {
+      if (k <= 4) DRTC_ROUTE(float, 4);
+      else if (k <= 8) DRTC_ROUTE(float, 8);
+      else DRTC_ROUTE(float, 16);
+    } else {
+      if (k <= 4) DRTC_ROUTE(bf16_t, 4);
+      else if (k <= 8) DRTC_ROUTE(bf16_t, 8);
+      else DRTC_ROUTE(bf16_t, 16);
+    }
 #undef DRTC_ROUTE
-  hipLaunchKernelGGL(moe_offsets_kernel, dim3(1), dim3(1024), 0, st, (const int*)wg_cnt, G, E,
-                     wg_base, t_e, t_r0, t_n, n_tiles, local_range, max_tiles, e_off, e_local, bm,
-                     variant == 4 ? grp_off : (int*)nullptr);
-  hipLaunchKernelGGL(moe_scatter_kernel, dim3(G), dim3(kMoeRouteWG), 0, st, (const float*)topk_w,
-                     (const int*)wg_base, T, E, k, sorted_tok, sorted_w, inv_pos);
+    hipLaunchKernelGGL(moe_offsets_kernel, dim3(1), dim3(1024), 0, st, (const int*)wg_cnt, G, E,
+                       wg_base, t_e, t_r0, t_n, n_tiles, local_range, max_tiles, e_off, e_local, bm,
+                       variant == 4 ? grp_off : (int*)nullptr);
+    hipLaunchKernelGGL(moe_scatter_kernel, dim3(G), dim3(kMoeRouteWG), 0, st, (const float*)topk_w,
+                       (const int*)wg_base, T, E, k, sorted_tok, sorted_w, inv_pos);
+  }
   const dim3 g_gu((I / (glu ? 64 : 128)) * max_tiles), g_dn((H / 128) * max_tiles);
   if (opt.f32) {
     const dim3 g_up(glu ? (I + 31) / 32 : (I + 63) / 64, max_tiles);
@@ -1049,6 +1199,13 @@ int launch_moe(void* out, const void* x, const void* router_logits, const void* 
                                t_r0, t_n, t_e, n_tiles, nullptr, (int64_t)H * I, slab,
                                slab_bytes, counters, n_counters, 0.f, st);
     if (e) return e;
+  } else if (variant == 5) {
+    int e = launch_stream_moe(hbuf, x, w_gu, I, H, H, I, stream_mt, act, opt.limit, (int64_t)up_rows * H, sorted_tok,
+                              t_e, t_r0, t_n, n_tiles, st);
+    if (!e)
+      e = launch_stream_moe(zbuf, hbuf, w_dn, H, I, I, H, stream_mt, 4, 0.f, (int64_t)H * I, nullptr, t_e, t_r0, t_n,
+                            n_tiles, st);
+    if (e) return e;
   } else if (variant == 0) {
     hipLaunchKernelGGL((glu ? moe_gemm_kernel<0> : moe_gemm_kernel<2>), g_gu, dim3(256), 0, st, hbuf,
                        (const bf16_t*)x, (const bf16_t*)w_gu, sorted_tok, t_e, t_r0, t_n, n_tiles, H,
@@ -1089,9 +1246,13 @@ int launch_moe(void* out, const void* x, const void* router_logits, const void* 
 
 int configure_moe() {
   int e = 0;
-  for (const void* f : {(const void*)moe_route_kernel<float, 8>, (const void*)moe_route_kernel<float, 16>,
-                        (const void*)moe_route_kernel<bf16_t, 8>,
-                        (const void*)moe_route_kernel<bf16_t, 16>})
+  for (const void* f :
+       {(const void*)moe_route_kernel<float, 4>, (const void*)moe_route_kernel<float, 8>,
+        (const void*)moe_route_kernel<float, 16>, (const void*)moe_route_kernel<bf16_t, 4>,
+        (const void*)moe_route_kernel<bf16_t, 8>, (const void*)moe_route_kernel<bf16_t, 16>,
+        (const void*)moe_plan_kernel<float, 4, kMoeRouteWG>, (const void*)moe_plan_kernel<float, 8, kMoeRouteWG>,
+        (const void*)moe_plan_kernel<float, 16, kMoeRouteWG>, (const void*)moe_plan_kernel<bf16_t, 4, kMoeRouteWG>,
+        (const void*)moe_plan_kernel<bf16_t, 8, kMoeRouteWG>, (const void*)moe_plan_kernel<bf16_t, 16, kMoeRouteWG>})
     e |= (int)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
                                   kMoeMaxGroups * kMoeRouteWG * 4);
   e |= (int)hipFuncSetAttribute((const void*)moe_gemm_pipe_kernel<128, 0>,
@@ -1112,8 +1273,8 @@ int configure_moe() {
 int64_t moe_workspace_bytes(int T, int H, int I, int e_local, int k, int f32) {
   auto align = [](int64_t v) { return (v + 255) & ~int64_t(255); };
   const int64_t P = (int64_t)T * k;
-  const int64_t mt = (P + kMoeBM - 1) / kMoeBM + e_local;
-  // (tile tables sized for the 128-row tiles: the largest count of any variant)
+  const int64_t mt = (P + 15) / 16 + e_local;
+  // (tile tables sized for tiles of 16 rows: the largest count of any variant)
   // (routing: per-workgroup counts and bases for up to 256 experts)
   const int64_t G = (T + kMoeRouteWG - 1) / kMoeRouteWG;
   const int64_t es = f32 ? 4 : 2;

@@ -99,3 +99,66 @@ def test_routes_to_the_stream(hipk, M):
     out = torch.zeros(M, N + 8, device="cuda", dtype=torch.bfloat16)
     ops.squared_relu(x, w, out[:, 8:])
     assert torch.equal(out[:, 8:], G.stream_gemm(x, w, "relu2")) and (out[:, :8] == 0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 5, 16, 37, 80, 150])
+@pytest.mark.parametrize("H,I,E,k,act,e_off", [(2048, 1792, 16, 4, "silu", 0), (4096, 3584, 20, 4, "relu2", 0),
+                                              (2048, 4096, 8, 2, "gelu_tanh", 0), (1792, 2048, 24, 6, "clamped", 0),
+                                              (2048, 2048, 12, 3, "silu", 4)])
+def test_streamed_experts(hipk, T, H, I, E, k, act, e_off):
+    """Experts with no row, one, a tile and more than an entry holds (every third token goes to the first
+    expert first), a part of the experts on this rank; against the fp32 oracle, and the same bits in
+    replays of a graph."""
+    e_local = E // 2 if e_off else E
+    g = torch.Generator(device="cuda").manual_seed(T + E)
+    x = torch.randn(T, H, device="cuda", generator=g).to(torch.bfloat16)
+    lg = torch.randn(T, E, device="cuda", generator=g)
+    lg[::3, e_off] = 9.0
+    n_in = I if act == "relu2" else 2 * I
+    w_in = (torch.randn(e_local, n_in, H, device="cuda", generator=g) * 0.02).to(torch.bfloat16)
+    w_out = (torch.randn(e_local, H, I, device="cuda", generator=g) * 0.02).to(torch.bfloat16)
+    ws = ops.moe.make_workspace(T, H, I, e_local, k, "cuda")
+    G.gemm_workspace(x.device)
+
+    def run(v=5):
+        return ops.fused_moe(x, lg, w_in, w_out, k, act, E, e_off, ws, variant=v, limit=0.9)
+
+    try:
+        y = run()
+    except RuntimeError:
+        assert T * k // e_local > 10  # entries of more rows than the registers hold
+        y = run(-1)
+    want = ops.fused_moe_ref(x, lg, w_in, w_out, k, act, e_off, limit=0.9).double()
+    # both round the hidden rows and the experts' outputs to bf16: a few of them differ by one unit
+    assert (y.double() - want).norm() <= 2e-3 * want.norm() + 1e-6
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        z = run(-1)
+    for _ in range(3):
+        x.normal_(generator=g)
+        lg.normal_(generator=g)
+        graph.replay()
+        assert torch.equal(z, run(-1))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 255, 256, 257, 1000, 1024, 1025])
+@pytest.mark.parametrize("E,k,groups,keep", [(16, 4, 1, 1), (250, 16, 1, 1), (24, 5, 4, 2)])
+def test_routing_plan(hipk, T, E, k, groups, keep):
+    """Logits on a coarse grid, so that most choices are ties, with both zeros and infinities among them,
+    in one workgroup (T <= 1024) and in three passes: identical experts must come out of a model whose
+    experts return their number (the weighted sum tells which were chosen)."""
+    g = torch.Generator(device="cuda").manual_seed(T + E)
+    lg = (torch.randn(T, E, device="cuda", generator=g) * 2).round() / 2
+    lg[::5] *= -0.0
+    lg[1::7, 3] = float("-inf")
+    x = torch.ones(T, 128, device="cuda")
+    w_in = torch.ones(E, 8, 128, device="cuda") / 128  # hidden 1 for all
+    w_out = (torch.arange(E, device="cuda").float() + 1).view(E, 1, 1).expand(E, 128, 8).contiguous() / 8
+    for logits in (lg, lg.t().contiguous().t(), lg.to(torch.bfloat16)):
+        y = ops.fused_moe(x, logits, w_in, w_out, k, "relu2", E, groups=groups, keep=keep)
+        ids, w = ops.moe.route_ref(logits, k, groups, keep)
+        want = (w * (ids + 1)).sum(-1)
+        # a wrong expert moves the sum by a weight times a whole number; the fp32 sums by 1e-5 of it
+        assert (y[:, 0] - want).abs().max() <= 1e-4 * E
