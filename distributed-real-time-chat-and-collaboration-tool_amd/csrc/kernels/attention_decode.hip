@@ -43,6 +43,9 @@ __device__ __forceinline__ void vm_wait_all() {
 namespace drtc {
 
 constexpr int kBS = 32;  // tokens per KV-cache block (fixed by the layout)
+// partitions that the merge inside paged_decode_kernel takes: two floats for each of them and of 16
+// heads lie in the LDS of the waves' merge (4 x 64 x 16 floats at the smallest head)
+constexpr int kFusedMergeParts = 128;
 
 template <int D>
 struct KVRegs {
@@ -69,14 +72,107 @@ DRTC_DEVICE void load_kv_block(KVRegs<D>& r, const bf16_t* kb, const bf16_t* vb,
   }
 }
 
+// Block loads that skip the tokens of a partial last block (nvalid < 32):
+// a K row (256 B at D = 128) or a 4-token V group is not fetched when all of
+// its tokens are past the context; the registers are zeroed instead (their
+// probabilities are exactly 0, zeros keep 0 * V finite).
 template <int D>
+DRTC_DEVICE void load_kv_block_n(KVRegs<D>& r, const bf16_t* kb, const bf16_t* vb, int lane,
+                                 int nvalid) {
+  if (nvalid >= kBS) {
+    load_kv_block<D>(r, kb, vb, lane);
+    return;
+  }
+  const int t = lane & 15, g = lane >> 4;
+  bf16x8 z8;
+  bf16x4 z4;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) z8[j] = f2bf(0.f);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) z4[j] = f2bf(0.f);
+#pragma unroll
+  for (int s = 0; s < D / 32; ++s) {
+    r.k0[s] = z8;
+    r.k1[s] = z8;
+  }
+#pragma unroll
+  for (int i = 0; i < D / 16; ++i) {
+    r.vlo[i] = z4;
+    r.vhi[i] = z4;
+  }
+  if (t < nvalid) {
+#pragma unroll
+    for (int s = 0; s < D / 32; ++s) r.k0[s] = load_bf16x8(kb + t * D + 32 * s + 8 * g);
+  }
+  if (16 + t < nvalid) {
+#pragma unroll
+    for (int s = 0; s < D / 32; ++s) r.k1[s] = load_bf16x8(kb + (16 + t) * D + 32 * s + 8 * g);
+  }
+  if (4 * g < nvalid) {
+#pragma unroll
+    for (int i = 0; i < D / 16; ++i) r.vlo[i] = load_bf16x4(vb + g * (4 * D) + (16 * i + t) * 4);
+  }
+  if (16 + 4 * g < nvalid) {
+#pragma unroll
+    for (int i = 0; i < D / 16; ++i)
+      r.vhi[i] = load_bf16x4(vb + (4 + g) * (4 * D) + (16 * i + t) * 4);
+  }
+}
+
+// The step's token for kernels that rotate and write it themselves (see the persistent kernel)
+struct DecodeRope {
+  const int* positions;
+  const int64_t* slots;
+  const float* cos_sin;   // [max_pos][D]: cos | sin
+  bf16_t* k_cache;        // the caches the kernel reads (written for the step's token)
+  bf16_t* v_cache;
+};
+
+// rotate the lane's fragments f[0..KS) of one head (position pos), rounding as rope_kv
+template <int D>
+DRTC_DEVICE void rope_frags(bf16x8* f, const float* __restrict__ cos_sin, int pos, int g) {
+  constexpr int KS = D / 32;
+  const float* cs = cos_sin + (int64_t)pos * D + 8 * g;
+#pragma unroll
+  for (int s = 0; s < KS / 2; ++s) {
+    const f32x4 ca = *reinterpret_cast<const f32x4*>(cs + 32 * s);
+    const f32x4 cb = *reinterpret_cast<const f32x4*>(cs + 32 * s + 4);
+    const f32x4 sa = *reinterpret_cast<const f32x4*>(cs + D / 2 + 32 * s);
+    const f32x4 sb = *reinterpret_cast<const f32x4*>(cs + D / 2 + 32 * s + 4);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float c = j < 4 ? ca[j] : cb[j - 4];
+      const float sn = j < 4 ? sa[j] : sb[j - 4];
+      const float a = bf2f(f[s][j]), b = bf2f(f[s + KS / 2][j]);
+      f[s][j] = f2bf(a * c - b * sn);
+      f[s + KS / 2][j] = f2bf(b * c + a * sn);
+    }
+    // one fragment pair's cos / sin (16 VGPRs) live at a time: this runs beside a whole
+    // prefetched K/V block in the persistent kernel, at its register ceiling
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+DRTC_DEVICE void store_part(float* p, float v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+DRTC_DEVICE float load_part(const float* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// ROPE (decode batches too small for the persistent kernel): q, k and v of the step's token come
+// unrotated, as there; wave 0 of the last partition opens its softmax with that token and writes its
+// rows, the cache is read up to the token ahead of it.  Bound by its chain of round trips (table,
+// K / V, partials, count, merge), not by bytes, until a batch fills the chip: one sequence of 266 tokens
+// 9.9 us, 16 of 1000 20.6 us for 65 MB (rope_kv + a wave per partition + reduce: 19.1 and 26.4), 128 of
+// 1000 98 us (5.4 TB/s; rope_kv + this without ROPE 105).
+template <int D, bool ROPE>
 __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_kernel(
     bf16_t* __restrict__ out, float* __restrict__ part_o,
     float* __restrict__ part_ml, int* __restrict__ counters, const bf16_t* __restrict__ q,
     int q_stride, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     const int* __restrict__ block_tables, int bt_stride,
     const int* __restrict__ context_lens, int Hq, int Hkv, float scale_log2e,
-    int max_parts, int blocks_per_part) {
+    int max_parts, int blocks_per_part, DecodeRope rope) {
   constexpr int NT = D / 16;  // output d-tiles
   constexpr int KS = D / 32;  // k-steps of the QK product
   const int b = blockIdx.x / Hkv;
@@ -102,6 +198,9 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_kernel(
     else for (int j = 0; j < 8; ++j) qf[s][j] = f2bf(0.f);
   }
   const int ctx = context_lens[b];
+  const int nc = ROPE ? ctx - 1 : ctx;  // tokens read from the cache
+  const int pos = ROPE ? rope.positions[b] : 0;
+  const int64_t slot = ROPE ? rope.slots[b] : 0;
   const int nblk = (ctx + kBS - 1) / kBS;
   const int nparts = (nblk + blocks_per_part - 1) / blocks_per_part;
 
@@ -121,21 +220,62 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_kernel(
   float m = kNegBig, lsum = 0.f;
 
   const int64_t blk_elems = (int64_t)kBS * D;
+  auto load_block = [&](KVRegs<D>& r, int64_t phys, int blk) {
+    const bf16_t* kb = k_cache + (phys * Hkv + h) * blk_elems;
+    const bf16_t* vb = v_cache + (phys * Hkv + h) * blk_elems;
+    if constexpr (ROPE) load_kv_block_n<D>(r, kb, vb, lane, nc - blk * kBS);
+    else load_kv_block<D>(r, kb, vb, lane);
+  };
   KVRegs<D> cur, nxt;
   int blk = blk_begin + w;
   int ph_next = ph_b;  // table entry of block blk + 4, loaded one step ahead
   if (blk < blk_end) {
     const int64_t phys = ph_a;
-    load_kv_block<D>(cur, k_cache + (phys * Hkv + h) * blk_elems,
-                     v_cache + (phys * Hkv + h) * blk_elems, lane);
+    load_block(cur, phys, blk);
+  }
+  if constexpr (ROPE) {
+    rope_frags<D>(qf, rope.cos_sin, pos, g);
+    if (w == 0 && p == nparts - 1) {
+      const bf16_t* kn = q + (int64_t)b * q_stride + (int64_t)(Hq + h) * D;
+      const bf16_t* vn = kn + (int64_t)Hkv * D;
+      bf16x8 kf[KS];
+#pragma unroll
+      for (int s = 0; s < KS; ++s) kf[s] = load_bf16x8(kn + 32 * s + 8 * g);
+      rope_frags<D>(kf, rope.cos_sin, pos, g);
+      float dot = 0.f;
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) dot += bf2f(qf[s][j]) * bf2f(kf[s][j]);
+      dot += __shfl_xor(dot, 16, 64);
+      dot += __shfl_xor(dot, 32, 64);
+      m = dot * scale_log2e;
+      lsum = g == 0 ? 1.f : 0.f;  // p = 1, counted once
+      const int64_t cblk = slot / kBS, off = slot - cblk * kBS;
+      if (col == 0 && slot >= 0) {
+        bf16_t* kd = rope.k_cache + ((cblk * Hkv + h) * kBS + off) * D + 8 * g;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) store_bf16x8(kd + 32 * s, kf[s]);
+      }
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        const bf16x4 v = load_bf16x4(vn + 16 * i + 4 * g);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[i][r] = bf2f(v[r]);
+      }
+      if (slot >= 0) {  // V block [8 groups of 4 tokens][D][4]
+        bf16_t* vd = rope.v_cache + (cblk * Hkv + h) * blk_elems + (off >> 2) * (4 * D) + (off & 3);
+#pragma unroll
+        for (int d = lane; d < D; d += 64) vd[d * 4] = vn[d];
+      }
+    }
   }
   vm_wait_all();  // the first block lands before the loop (vm_wait_all)
   for (; blk < blk_end; blk += 4) {
     const int nb = blk + 4;
     if (nb < blk_end) {  // register double-buffer: next block in flight
       const int64_t phys = ph_next;
-      load_kv_block<D>(nxt, k_cache + (phys * Hkv + h) * blk_elems,
-                       v_cache + (phys * Hkv + h) * blk_elems, lane);
+      load_block(nxt, phys, nb);
       ph_next = bt[min(nb + 4, bt_stride - 1)];
     }
     f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
@@ -148,8 +288,8 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_kernel(
     float bmax = kNegBig;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      s0[r] = (tok0 + r < ctx) ? s0[r] * scale_log2e : kNegBig;
-      s1[r] = (tok0 + 16 + r < ctx) ? s1[r] * scale_log2e : kNegBig;
+      s0[r] = (tok0 + r < nc) ? s0[r] * scale_log2e : kNegBig;
+      s1[r] = (tok0 + 16 + r < nc) ? s1[r] * scale_log2e : kNegBig;
       bmax = fmaxf(bmax, fmaxf(s0[r], s1[r]));
     }
     bmax = fmaxf(bmax, __shfl_xor(bmax, 16, 64));
@@ -161,8 +301,12 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_kernel(
     float psum = 0.f;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const float p0 = fast_exp2(s0[r] - m_new);
-      const float p1 = fast_exp2(s1[r] - m_new);
+      float p0 = fast_exp2(s0[r] - m_new);
+      float p1 = fast_exp2(s1[r] - m_new);
+      if constexpr (ROPE) {  // a block may hold no cached token at all (m_new = kNegBig)
+        p0 = (tok0 + r < nc) ? p0 : 0.f;
+        p1 = (tok0 + 16 + r < nc) ? p1 : 0.f;
+      }
       psum += p0 + p1;
       pf[r] = f2bf(p0);
       pf[4 + r] = f2bf(p1);
@@ -219,38 +363,46 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_kernel(
       out[((int64_t)b * Hq + hq) * D + d] = f2bf(O / L);
     } else {
       const int64_t pi = ((int64_t)b * Hq + hq) * max_parts + p;
-      part_o[pi * D + d] = O;
+      store_part(part_o + pi * D + d, O);
       if (d == 0) {
-        part_ml[pi * 2 + 0] = M;
-        part_ml[pi * 2 + 1] = L;
+        store_part(part_ml + pi * 2, M);
+        store_part(part_ml + pi * 2 + 1, L);
       }
     }
   }
   if (single || counters == nullptr) return;
-  // Split-K merge without a second launch: the last partition of this
-  // (sequence, kv head) to finish - counted with an agent-scope atomic after
-  // a release fence over the partial stores - merges all partitions in fixed
-  // order (deterministic) and re-arms the counter for the next launch.
+  // Split-K merge without a second launch: the last partition of this (sequence, kv head) to finish
+  // merges all partitions in fixed order (deterministic) and re-arms the counter for the next launch.
+  // Partials are written through to where every XCD reads them and have arrived before the count, so
+  // neither side needs a fence over its caches.
   __shared__ int is_last;
-  __shared__ float mh[16], ilh[16];
-  __threadfence();
+  __shared__ float ilh[16];
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (threadIdx.x == 0) {
-    const int prev = __hip_atomic_fetch_add(counters + blockIdx.x, 1, __ATOMIC_ACQ_REL,
+    const int prev = __hip_atomic_fetch_add(counters + blockIdx.x, 1, __ATOMIC_RELAXED,
                                             __HIP_MEMORY_SCOPE_AGENT);
     is_last = (prev == nparts - 1);
     if (is_last) __hip_atomic_store(counters + blockIdx.x, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
   if (!is_last) return;
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  if (threadIdx.x < G) {
-    const float* ml = part_ml + ((int64_t)b * Hq + h * G + threadIdx.x) * max_parts * 2;
+  // the partitions' weights and sums, a wave per head, over the LDS of the waves' merge
+  float* const lds_l = smem + G * nparts;
+  for (int hh = w; hh < G; hh += 4) {
+    const float* ml = part_ml + ((int64_t)b * Hq + h * G + hh) * max_parts * 2;
     float M = kNegBig;
-    for (int pp = 0; pp < nparts; ++pp) M = fmaxf(M, ml[2 * pp]);
+    for (int pp = lane; pp < nparts; pp += 64) M = fmaxf(M, load_part(ml + 2 * pp));
+    M = wave_max(M);
+    for (int pp = lane; pp < nparts; pp += 64) {
+      smem[hh * nparts + pp] = fast_exp2(load_part(ml + 2 * pp) - M);
+      lds_l[hh * nparts + pp] = load_part(ml + 2 * pp + 1);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < G) {
     float L = 0.f;
-    for (int pp = 0; pp < nparts; ++pp) L += ml[2 * pp + 1] * fast_exp2(ml[2 * pp] - M);
-    mh[threadIdx.x] = M;
+    for (int pp = 0; pp < nparts; ++pp) L += lds_l[threadIdx.x * nparts + pp] * smem[threadIdx.x * nparts + pp];
     ilh[threadIdx.x] = 1.f / L;
   }
   __syncthreads();
@@ -258,11 +410,16 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_kernel(
     const int hh = item / D;
     const int d = item - hh * D;
     const int64_t bh = (int64_t)b * Hq + h * G + hh;
-    const float* ml = part_ml + bh * max_parts * 2;
-    const float M = mh[hh];
+    const float* po = part_o + bh * max_parts * D + d;
+    const float* f = smem + hh * nparts;
     float O = 0.f;
-    for (int pp = 0; pp < nparts; ++pp)
-      O += part_o[(bh * max_parts + pp) * D + d] * fast_exp2(ml[2 * pp] - M);
+    for (int pp = 0; pp < nparts; pp += 8) {  // eight partials in flight
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = load_part(po + (int64_t)min(pp + j, nparts - 1) * D);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) O += (pp + j < nparts ? v[j] : 0.f) * f[min(pp + j, nparts - 1)];
+    }
     out[bh * D + d] = f2bf(O * ilh[hh]);
   }
 }
@@ -418,53 +575,6 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_wave_kerne
   }
 }
 
-// Block loads that skip the tokens of a partial last block (nvalid < 32):
-// a K row (256 B at D = 128) or a 4-token V group is not fetched when all of
-// its tokens are past the context; the registers are zeroed instead (their
-// probabilities are exactly 0, zeros keep 0 * V finite).
-template <int D>
-DRTC_DEVICE void load_kv_block_n(KVRegs<D>& r, const bf16_t* kb, const bf16_t* vb, int lane,
-                                 int nvalid) {
-  if (nvalid >= kBS) {
-    load_kv_block<D>(r, kb, vb, lane);
-    return;
-  }
-  const int t = lane & 15, g = lane >> 4;
-  bf16x8 z8;
-  bf16x4 z4;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) z8[j] = f2bf(0.f);
-#pragma unroll
-  for (int j = 0; j < 4; ++j) z4[j] = f2bf(0.f);
-#pragma unroll
-  for (int s = 0; s < D / 32; ++s) {
-    r.k0[s] = z8;
-    r.k1[s] = z8;
-  }
-#pragma unroll
-  for (int i = 0; i < D / 16; ++i) {
-    r.vlo[i] = z4;
-    r.vhi[i] = z4;
-  }
-  if (t < nvalid) {
-#pragma unroll
-    for (int s = 0; s < D / 32; ++s) r.k0[s] = load_bf16x8(kb + t * D + 32 * s + 8 * g);
-  }
-  if (16 + t < nvalid) {
-#pragma unroll
-    for (int s = 0; s < D / 32; ++s) r.k1[s] = load_bf16x8(kb + (16 + t) * D + 32 * s + 8 * g);
-  }
-  if (4 * g < nvalid) {
-#pragma unroll
-    for (int i = 0; i < D / 16; ++i) r.vlo[i] = load_bf16x4(vb + g * (4 * D) + (16 * i + t) * 4);
-  }
-  if (16 + 4 * g < nvalid) {
-#pragma unroll
-    for (int i = 0; i < D / 16; ++i)
-      r.vhi[i] = load_bf16x4(vb + (4 + g) * (4 * D) + (16 * i + t) * 4);
-  }
-}
-
 // Variant 3: persistent waves.  The grid holds ~2 workgroups per CU; wave w
 // of the grid takes work items w, w + W, w + 2W, ... (item = (partition,
 // sequence, kv head), partition slowest) and streams their cache blocks back
@@ -487,39 +597,6 @@ DRTC_DEVICE void load_kv_block_n(KVRegs<D>& r, const bf16_t* kb, const bf16_t* v
 //     m = that score, p = 1, o = its v row;
 //   * that item also writes the rotated k row and the v row into the paged cache (slot from
 //     `slots`) for the next steps - the same bytes rope_kv_kernel_v2 writes.
-struct DecodeRope {
-  const int* positions;
-  const int64_t* slots;
-  const float* cos_sin;   // [max_pos][D]: cos | sin
-  bf16_t* k_cache;        // the caches the kernel reads (written for the step's token)
-  bf16_t* v_cache;
-};
-
-// rotate the lane's fragments f[0..KS) of one head (position pos), rounding as rope_kv
-template <int D>
-DRTC_DEVICE void rope_frags(bf16x8* f, const float* __restrict__ cos_sin, int pos, int g) {
-  constexpr int KS = D / 32;
-  const float* cs = cos_sin + (int64_t)pos * D + 8 * g;
-#pragma unroll
-  for (int s = 0; s < KS / 2; ++s) {
-    const f32x4 ca = *reinterpret_cast<const f32x4*>(cs + 32 * s);
-    const f32x4 cb = *reinterpret_cast<const f32x4*>(cs + 32 * s + 4);
-    const f32x4 sa = *reinterpret_cast<const f32x4*>(cs + D / 2 + 32 * s);
-    const f32x4 sb = *reinterpret_cast<const f32x4*>(cs + D / 2 + 32 * s + 4);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float c = j < 4 ? ca[j] : cb[j - 4];
-      const float sn = j < 4 ? sa[j] : sb[j - 4];
-      const float a = bf2f(f[s][j]), b = bf2f(f[s + KS / 2][j]);
-      f[s][j] = f2bf(a * c - b * sn);
-      f[s + KS / 2][j] = f2bf(b * c + a * sn);
-    }
-    // one fragment pair's cos / sin (16 VGPRs) live at a time: this runs beside a whole
-    // prefetched K/V block in the persistent kernel, at its register ceiling
-    __builtin_amdgcn_sched_barrier(0);
-  }
-}
-
 // One LDS-DMA wave-instruction of one dword per lane: 256 contiguous bytes land at the LDS byte
 // address `dst` (M0 saved and restored).  Counts in vmcnt like any vector load.
 DRTC_DEVICE void dma_dword_lds(unsigned dst, unsigned voff, __amdgpu_buffer_rsrc_t rsrc) {
@@ -938,17 +1015,18 @@ int launch_paged_decode(void* out, float* part_o, float* part_ml, int* counters,
     return (int)hipGetLastError();
   }
   if (variant != 1) return -3;
+  if (max_parts > kFusedMergeParts) counters = nullptr;
   dim3 grid(B * Hkv, max_parts), block(256);
   const size_t lds = (128 + 4 * (size_t)D * 16) * sizeof(float);
   switch (D) {
     case 64:
-      hipLaunchKernelGGL(paged_decode_kernel<64>, grid, block, lds, st, (bf16_t*)out, part_o, part_ml, counters, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, bt_stride, context_lens, Hq, Hkv, sl2, max_parts, blocks_per_part);
+      hipLaunchKernelGGL((paged_decode_kernel<64, false>), grid, block, lds, st, (bf16_t*)out, part_o, part_ml, counters, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, bt_stride, context_lens, Hq, Hkv, sl2, max_parts, blocks_per_part, DecodeRope{});
       break;
     case 128:
-      hipLaunchKernelGGL(paged_decode_kernel<128>, grid, block, lds, st, (bf16_t*)out, part_o, part_ml, counters, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, bt_stride, context_lens, Hq, Hkv, sl2, max_parts, blocks_per_part);
+      hipLaunchKernelGGL((paged_decode_kernel<128, false>), grid, block, lds, st, (bf16_t*)out, part_o, part_ml, counters, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, bt_stride, context_lens, Hq, Hkv, sl2, max_parts, blocks_per_part, DecodeRope{});
       break;
     case 256:
-      hipLaunchKernelGGL(paged_decode_kernel<256>, grid, block, lds, st, (bf16_t*)out, part_o, part_ml, counters, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, bt_stride, context_lens, Hq, Hkv, sl2, max_parts, blocks_per_part);
+      hipLaunchKernelGGL((paged_decode_kernel<256, false>), grid, block, lds, st, (bf16_t*)out, part_o, part_ml, counters, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, bt_stride, context_lens, Hq, Hkv, sl2, max_parts, blocks_per_part, DecodeRope{});
       break;
     default:
       return -1;
@@ -960,7 +1038,8 @@ int launch_paged_decode(void* out, float* part_o, float* part_ml, int* counters,
   return (int)hipGetLastError();
 }
 
-// Persistent decode attention with the step's RoPE + KV write fused (DecodeRope above).
+// Decode attention with the step's RoPE + KV write fused (DecodeRope above): variant 3, or 1 for batches
+// that leave the persistent waves without items.
 // q = row 0 of the QKV GEMM output [B][q_stride] (q | k | v heads, unrotated); D <= 128
 // (the persistent form at D = 256 spills; the caller runs rope_kv + the plain form there).
 int launch_paged_decode_rope(void* out, float* part_o, float* part_ml, const void* q,
@@ -968,9 +1047,9 @@ int launch_paged_decode_rope(void* out, float* part_o, float* part_ml, const voi
                              const int* block_tables, int bt_stride, const int* context_lens,
                              int B, int Hq, int Hkv, int D, float scale, int max_parts,
                              int blocks_per_part, const int* positions, const int64_t* slots,
-                             const float* cos_sin, int max_wgs, hipStream_t st) {
+                             const float* cos_sin, int max_wgs, int* counters, int variant, hipStream_t st) {
   if (B == 0) return 0;
-  if (Hkv <= 0 || Hq % Hkv != 0 || Hq / Hkv > 16 || D > 128) return -1;
+  if (Hkv <= 0 || Hq % Hkv != 0 || Hq / Hkv > 16 || (D != 64 && D != 128)) return -1;
   if (!positions || !slots || !cos_sin || q_stride < (Hq + 2 * Hkv) * D) return -1;
   if (max_parts > 1 && (!part_o || !part_ml)) return -2;
   static int n_cu = 0;
@@ -989,6 +1068,16 @@ int launch_paged_decode_rope(void* out, float* part_o, float* part_ml, const voi
   if (max_wgs > 0) wgs = std::min(wgs, max_wgs);
   const dim3 pgrid(std::max(1, wgs)), pblock(256);
   const DecodeRope r{positions, slots, cos_sin, (bf16_t*)k_cache, (bf16_t*)v_cache};
+  if (variant == 1) {  // a workgroup per (sequence, kv head, partition)
+    if (max_parts > 1 && !counters) return -2;
+    if (max_parts > kFusedMergeParts) return -1;
+    const dim3 grid(B * Hkv, max_parts);
+    const size_t lds = (128 + 4 * (size_t)D * 16) * sizeof(float);
+    (D == 64 ? paged_decode_kernel<64, true> : paged_decode_kernel<128, true>)<<<grid, pblock, lds, st>>>(
+        (bf16_t*)out, part_o, part_ml, counters, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache,
+        (const bf16_t*)v_cache, block_tables, bt_stride, context_lens, Hq, Hkv, sl2, max_parts, blocks_per_part, r);
+    return (int)hipGetLastError();
+  }
   switch (D) {
     case 64:
       hipLaunchKernelGGL((paged_decode_persist_kernel<64, true>), pgrid, pblock, 0, st, (bf16_t*)out, part_o, part_ml, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, bt_stride, context_lens, B, Hq, Hkv, sl2, max_parts, blocks_per_part, r);
@@ -1008,7 +1097,7 @@ int launch_paged_decode_rope(void* out, float* part_o, float* part_ml, const voi
 
 int configure_decode() {
   const int lds = (128 + 4 * 256 * 16) * sizeof(float);
-  return (int)hipFuncSetAttribute((const void*)paged_decode_kernel<256>,
+  return (int)hipFuncSetAttribute((const void*)paged_decode_kernel<256, false>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds);
 }
 

@@ -126,9 +126,9 @@ def decode_variant(batch: int, Hkv: int, D: int, max_blocks: int) -> int:
     3 (persistent waves, next item prefetched) when there are >= 4096
     (sequence, kv head) items and D <= 128 - the serving batches (B 1024 x 8
     kv heads: 141 vs 150 us); 2 (wave per item) when the context must be
-    split over partitions to fill the chip (B 8 x 4k tokens: 30 vs 53 us for
-    variant 1, whose in-kernel merge pays an agent-scope fence per workgroup
-    across the 8 XCD L2s); 1 otherwise (B 256 x ~1k tokens: 196 vs 206 us).
+    split over partitions to fill the chip; 1 otherwise (B 256 x ~1k tokens:
+    196 vs 206 us).  Where the step's RoPE runs in the same launch
+    (``fused_rope_variant``) 1 also takes the shapes of 2.
     r2l (profiles/r2l_decode_geometries.md): from 2048 items v3 also wins at
     chat lengths (Mixtral / 70B heads at B 256: 38.4 vs 40.1 / 38.9 vs 41.2 us);
     at D = 256 (Gemma-2B, one kv head) v2 wins from 1024 items (B 1024: 34.2 vs
@@ -245,10 +245,23 @@ def paged_decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
     return out
 
 
-# RoPE + KV write fused into the persistent decode attention (attention_decode.hip
+# RoPE + KV write fused into the decode attention (attention_decode.hip
 # DecodeRope): the step's q / k / v come unrotated from the QKV GEMM output; one launch
-# per layer instead of rope_kv + attention.  DRTC_DECODE_FUSED_ROPE=0 keeps the two launches.
+# per layer instead of rope_kv + attention (+ reduce).  DRTC_DECODE_FUSED_ROPE=0 keeps the launches apart.
 FUSED_ROPE = os.environ.get("DRTC_DECODE_FUSED_ROPE", "1") != "0"
+
+
+def fused_rope_variant(variant: int, D: int, max_parts: int) -> int:
+    """The kernel that takes RoPE, the KV write and the merge of the partitions into the attention
+    launch, or 0.  3 stays itself; 1 runs the shapes of 1 and 2: a workgroup per partition, so 8
+    blocks are 2 per wave, and one launch instead of rope_kv, attention and decode_reduce.  Its merge
+    holds up to 128 partitions.  32 heads of 128 over 8 kv heads, three launches against one:
+    1 x 266 tokens 19.1 -> 9.9 us, 1 x 16000 43.7 -> 27.0, 1 x 64000 95 -> 68, 8 x 4000 42.7 -> 31.8,
+    16 x 1000 26.4 -> 20.6; two launches (one partition) against one: 40 x 1000 47.2 -> 42.6,
+    64 x 300 23.2 -> 21.1, 128 x 1000 105 -> 98, 200 x 400 74.0 -> 74.5."""
+    if D not in (64, 128) or DECODE_VARIANT == 2:
+        return 0
+    return 3 if variant == 3 else 1 if max_parts <= (128 if FUSED_SPLIT_MERGE else 1) else 0
 
 
 def paged_decode_attention_rope(qkv: torch.Tensor, positions: torch.Tensor, slots: torch.Tensor,
@@ -262,8 +275,8 @@ def paged_decode_attention_rope(qkv: torch.Tensor, positions: torch.Tensor, slot
     """Decode-step attention from the raw QKV rows [B, (Hq + 2 Hkv) D]: rotate q / k of
     the step's token (position ``positions[b]`` = context_lens[b] - 1), write its k / v
     into the paged cache at ``slots[b]`` and attend over the whole context - the result
-    of ``rope_kv_`` followed by ``paged_decode_attention``.  On the GPU the persistent
-    kernel (variant 3, D <= 128) does it in one launch; other shapes run the two ops.
+    of ``rope_kv_`` followed by ``paged_decode_attention``.  On the GPU one launch does it at
+    head sizes 64 and 128 (``fused_rope_variant``); other shapes run the two ops.
     ``max_wgs`` > 0 caps the persistent grid at that many 4-wave workgroups (attention on
     part of the chip, beside another stream's GEMMs; 0: two per CU)."""
     from .rope import rope_kv_
@@ -271,7 +284,12 @@ def paged_decode_attention_rope(qkv: torch.Tensor, positions: torch.Tensor, slot
     B = qkv.shape[0]
     q = qkv.as_strided((B, Hq, D), (qkv.stride(0), D, 1))
     variant = decode_variant(B, Hkv, D, block_tables.shape[1]) if on_gpu(qkv) else 0
-    if not (on_gpu(qkv) and FUSED_ROPE and variant == 3 and D <= 128):
+    fused = 0
+    if on_gpu(qkv) and FUSED_ROPE:
+        max_parts = (workspace.max_parts if blocks_per_part is not None and workspace is not None
+                     else decode_partitioning(B, Hkv, block_tables.shape[1], variant=variant, D=D)[1])
+        fused = fused_rope_variant(variant, D, max_parts)
+    if not fused:
         rope_kv_(qkv, positions, slots, cos_sin, Hq, Hkv, D, k_cache, v_cache, KV_BLOCK)
         return paged_decode_attention(q, k_cache, v_cache, block_tables, context_lens, scale,
                                       out=out, blocks_per_part=blocks_per_part,
@@ -299,5 +317,6 @@ def paged_decode_attention_rope(qkv: torch.Tensor, positions: torch.Tensor, slot
                                    block_tables.stride(0), context_lens.data_ptr(), B, Hq, Hkv, D,
                                    float(scale), workspace.max_parts, blocks_per_part,
                                    positions.data_ptr(), slots.data_ptr(), cos_sin.data_ptr(),
-                                   int(max_wgs), stream_ptr(qkv)), "paged_decode_rope")
+                                   int(max_wgs), ptr(workspace.counters), fused,
+                                   stream_ptr(qkv)), "paged_decode_rope")
     return out

@@ -268,6 +268,47 @@ def test_paged_decode_fused_rope(hipk, monkeypatch, D, Hq, Hkv, ctx_lens, bpp):
         if c == 0:
             assert out[b].abs().max().item() == 0.0
 
+@pytest.mark.parametrize("D,Hq,Hkv,parts", [(128, 32, 8, 1), (128, 8, 8, 3), (64, 16, 1, 7), (128, 16, 1, 9)])
+@pytest.mark.parametrize("ctx_lens", [[1, 2, 32, 33, 0, 65, 129, 257], [1000, 1025, 2049, 0, 513]])
+def test_paged_decode_rope_workgroups(hipk, D, Hq, Hkv, parts, ctx_lens):
+    """RoPE, the KV write and the merge of the partitions in one launch of the workgroup-per-partition
+    kernel: against the references of the ops it fuses (tolerance of the tests above), a step's token
+    alone in its block or partition, padded rows zero, counters back at zero, graph replays equal."""
+    from drtc_amd.ops import attention as attn_ops
+
+    B = len(ctx_lens)
+    assert attn_ops.fused_rope_variant(attn_ops.decode_variant(B, Hkv, D, 65), D, parts) == 1
+    _, kc, vc, bt, _ = _paged_setup(B, Hq, Hkv, D, [max(c, 1) for c in ctx_lens], seed=21)
+    cl = torch.tensor(ctx_lens, dtype=torch.int32, device=DEV)
+    g = torch.Generator().manual_seed(22)
+    qkv = torch.randn(B, (Hq + 2 * Hkv) * D + 8, generator=g).to(torch.bfloat16).to(DEV)[:, :(Hq + 2 * Hkv) * D]
+    pos = (cl - 1).clamp(min=0)
+    slots = torch.tensor([int(bt[b, p // 32]) * 32 + p % 32 if c else -1
+                          for b, (c, p) in enumerate(zip(ctx_lens, pos.tolist()))], device=DEV)
+    cs = ops.build_rope_cache(4096, D, 5e5, device=DEV)
+    bpp = math.ceil(bt.shape[1] / parts)
+    ws = ops.DecodeWorkspace(B, Hq, D, parts, DEV)
+    want_k, want_v, rot = kc.clone(), vc.clone(), qkv.clone()
+    ops.rope_kv_ref(rot, pos, slots, cs, Hq, Hkv, D, want_k, want_v, ops.KV_BLOCK)
+    q = rot.as_strided((B, Hq, D), (rot.stride(0), D, 1))
+    want = ops.paged_decode_ref(q.float(), want_k.float(), want_v.float(), bt, cl, D ** -0.5)
+    out = torch.empty(B, Hq, D, dtype=torch.bfloat16, device=DEV)
+    run = lambda: ops.paged_decode_attention_rope(qkv, pos, slots, cs, Hq, Hkv, D, kc, vc, bt, cl, D ** -0.5,
+                                                  out=out, blocks_per_part=bpp, workspace=ws)
+    run()
+    first = out.clone()
+    _close(first, want, 2e-2, 2e-2, "output")
+    _close(kc, want_k, 1e-2, 1e-2, "k cache")
+    assert torch.equal(vc, want_v)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run()
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        assert torch.equal(out, first)
+    assert parts == 1 or not ws.counters.any()
+
 
 @pytest.mark.parametrize("variant", [1, 2, 3])
 def test_paged_decode_strided_q_and_padding(hipk, variant):
