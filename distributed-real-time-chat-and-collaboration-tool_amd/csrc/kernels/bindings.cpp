@@ -237,6 +237,13 @@ PYBIND11_MODULE(_hipk, m) {
     return drtc::lt_tune(P<void>(y), P<const void>(x), P<const void>(w), M, N, K, ldx, ldy,
                          iters, max_candidates, S(st));
   });
+  m.def("embed", [](u64 out, u64 ids, int wide, u64 table, int rows, int V, int H, u64 st) {
+    return drtc::launch_embed(P<void>(out), P<const void>(ids), wide, P<const void>(table), rows, V, H, S(st));
+  });
+  m.def("step_begin", [](u64 ids, u64 src, u64 sampled, u64 host, int B, u64 counter, u64 position, u64 st) {
+    return drtc::launch_step_begin(P<int>(ids), P<const int64_t>(src), P<const int>(sampled), P<const int>(host), B,
+                                   P<int64_t>(counter), P<int64_t>(position), S(st));
+  });
   m.def("sample", [](u64 out_tokens, u64 logits, int B, int V, int ld,
                      u64 temperature, u64 top_k, u64 top_p, uint64_t seed,
                      u64 step, u64 st) {

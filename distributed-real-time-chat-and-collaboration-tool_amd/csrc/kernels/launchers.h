@@ -48,6 +48,9 @@ int launch_prefill_attn(void* out, int out_stride, const void* qkv,
                         const int* tile_q0, int ntiles, float scale, int causal, int persist,
                         hipStream_t st);
 
+int launch_embed(void* out, const void* ids, int wide, const void* table, int rows, int V, int H, hipStream_t st);
+int launch_step_begin(int* ids, const int64_t* src, const int* sampled, const int* host, int B, int64_t* counter,
+                      int64_t* position, hipStream_t st);
 int launch_sample(int* out_tokens, const void* logits, int B, int V, int ld,
                   const float* temperature, const int* top_k, const float* top_p,
                   uint64_t seed, const int64_t* step, hipStream_t st);

@@ -535,6 +535,33 @@ __global__ __launch_bounds__(kSampThreads, 4 * OCC) void sample_kernel(
   }
 }
 
+// The start of a decode step: each row's token, from the last step's samples (src >= 0) or from the host,
+// and the step's position in the random stream, which the next step's start finds advanced.  One launch
+// in place of compare, clamp, index_select, where and add, 3 to 5 us each between two kernels of a graph.
+__global__ __launch_bounds__(256) void step_begin_kernel(int* __restrict__ ids, const int64_t* __restrict__ src,
+                                                         const int* __restrict__ sampled,
+                                                         const int* __restrict__ host, int B,
+                                                         int64_t* __restrict__ counter,
+                                                         int64_t* __restrict__ position) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < B) {
+    const int64_t s = src[i];
+    ids[i] = s >= 0 && s < B ? sampled[s] : host[i];
+  }
+  if (i == 0) {
+    const int64_t c = *counter;
+    *position = c;
+    *counter = c + 1;
+  }
+}
+
+int launch_step_begin(int* ids, const int64_t* src, const int* sampled, const int* host, int B, int64_t* counter,
+                      int64_t* position, hipStream_t st) {
+  if (B <= 0) return B == 0 ? 0 : -1;
+  step_begin_kernel<<<(B + 255) / 256, 256, 0, st>>>(ids, src, sampled, host, B, counter, position);
+  return (int)hipGetLastError();
+}
+
 int launch_sample(int* out_tokens, const void* logits, int B, int V, int ld,
                   const float* temperature, const int* top_k, const float* top_p,
                   uint64_t seed, const int64_t* step, hipStream_t st) {

@@ -4,7 +4,7 @@ The whole decode step - embedding, 32 x (QKV GEMM, RoPE+KV write, paged MFMA
 attention, o_proj, add+norm, gate|up GEMM, act, down, add+norm), LM head and
 the sampler, plus the RNG-step increment - is captured once per batch bucket
 and replayed with a single ``hipGraphLaunch``.  Per step the host only
-uploads three packed staging buffers (int32 / int64 / fp32) and reads back
+uploads one packed staging buffer (int64 | int32 | fp32) and reads back
 the sampled token ids.  Steps can be pipelined: the next step's input tokens
 are gathered from the previous step's samples on the device, so the engine
 enqueues step t+1 before it reads step t's tokens and the host bookkeeping of
@@ -48,7 +48,9 @@ class DecodeRunner:
         B, MB = max_batch, max_blocks
         # ---- device buffers (persistent: graphs capture these addresses)
         n_i32 = 3 * B + B * MB + B + B
-        self.i32 = torch.zeros(n_i32, dtype=torch.int32, device=dev)
+        # one allocation, so that a step's staging is one copy
+        self.stage = torch.zeros(16 * B + 4 * n_i32 + 8 * B, dtype=torch.uint8, device=dev)
+        self.i64, self.i32, self.f32 = self._parts(self.stage, B)
         self.ids = self.i32[0:B]
         self.positions = self.i32[B:2 * B]
         self.ctx = self.i32[2 * B:3 * B]
@@ -58,13 +60,13 @@ class DecodeRunner:
         self.has_state = getattr(kv_cache, "states", None) is not None
         # int64 staging: KV slot per sequence | source row of the input token
         # in the previous step's sampled tokens (-1: take ``ids`` from the host)
-        self.i64 = torch.full((2 * B,), -1, dtype=torch.int64, device=dev)
+        self.i64.fill_(-1)
         self.slots = self.i64[0:B]
         self.src = self.i64[B:2 * B]
-        self.f32 = torch.zeros(2 * B, dtype=torch.float32, device=dev)
         self.temp = self.f32[0:B]
         self.topp = self.f32[B:2 * B]
         self.step_ctr = torch.zeros(1, dtype=torch.int64, device=dev)
+        self.step_at = torch.zeros(1, dtype=torch.int64, device=dev)  # its value for the step under way
         self.out = torch.zeros(B, dtype=torch.int32, device=dev)
         self.attn_out = model.decode_buffer(B)
         # the step's logits per bucket, for callers that read them instead of the samples
@@ -73,9 +75,10 @@ class DecodeRunner:
         # ---- pinned host staging, double-buffered: step t+1 is staged while
         # step t's copies may still be pending (pipelined decode)
         pin = dev.type == "cuda"
-        self.h_i32 = [torch.zeros(n_i32, dtype=torch.int32, pin_memory=pin) for _ in range(2)]
-        self.h_i64 = [torch.full((2 * B,), -1, dtype=torch.int64, pin_memory=pin) for _ in range(2)]
-        self.h_f32 = [torch.zeros(2 * B, dtype=torch.float32, pin_memory=pin) for _ in range(2)]
+        self.h_stage = [torch.zeros(self.stage.shape, dtype=torch.uint8, pin_memory=pin) for _ in range(2)]
+        self.h_i64, self.h_i32, self.h_f32 = zip(*(self._parts(h, B) for h in self.h_stage))
+        for h in self.h_i64:
+            h.fill_(-1)
         self.h_out = [torch.zeros(B, dtype=torch.int32, pin_memory=pin) for _ in range(2)]
         self.events = [torch.cuda.Event() if pin else None for _ in range(2)]
         self._k = 0
@@ -104,6 +107,12 @@ class DecodeRunner:
         # given exactly the counter value its first run sampled with
         self._ctr = 0
 
+    @staticmethod
+    def _parts(stage: torch.Tensor, B: int) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+        """The int64, int32 and fp32 parts of a staging buffer (views)."""
+        return (stage[:16 * B].view(torch.int64), stage[16 * B:-8 * B].view(torch.int32),
+                stage[-8 * B:].view(torch.float32))
+
     # ------------------------------------------------------------------
     def bucket(self, n: int) -> int:
         i = bisect.bisect_left(self.buckets, n)
@@ -125,20 +134,16 @@ class DecodeRunner:
         meta = self._meta(Bb)
         # input tokens: the previous step's samples still on the device
         # (pipelined steps, src >= 0) or host-provided ids (src = -1)
-        src = self.src[:Bb]
-        ids = torch.where(src >= 0, self.out[:Bb].index_select(0, src.clamp(min=0)),
-                          self.ids[:Bb])
-        if self.ep:
-            self.ids_used[:Bb].copy_(ids)
+        ids = self.ids_used[:Bb]
+        ops.step_begin(ids, self.src[:Bb], self.out[:Bb], self.ids[:Bb], self.step_ctr, self.step_at)
+        if not (self.device.type == "cuda" and torch.cuda.is_current_stream_capturing()):
+            self._ctr += 1
         logits = self.model.forward_decode(ids, meta, self.kv,
                                            None if self.attn_out is None else self.attn_out[:Bb])
         if self.keep_logits:
             self.logits[Bb] = logits
         ops.sample(logits.to(torch.bfloat16), self.temp[:Bb], self.topk[:Bb], self.topp[:Bb], seed=self.seed,
-                   step=self.step_ctr, out=self.out[:Bb])
-        self.step_ctr.add_(1)
-        if not (self.device.type == "cuda" and torch.cuda.is_current_stream_capturing()):
-            self._ctr += 1
+                   step=self.step_at, out=self.out[:Bb])
 
     def capture(self, Bb: int) -> None:
         if not self.use_graphs or Bb in self._graphs:
@@ -216,9 +221,7 @@ class DecodeRunner:
         hf[B:B + n] = topp
         hf[B + n:B + Bb] = 1.0
         nb = self.device.type == "cuda"
-        self.i32.copy_(self.h_i32[k], non_blocking=nb)
-        self.i64.copy_(self.h_i64[k], non_blocking=nb)
-        self.f32.copy_(self.h_f32[k], non_blocking=nb)
+        self.stage.copy_(self.h_stage[k], non_blocking=nb)
         g = self._graphs.get(Bb)
         timing = nb and self.time_gpu
         if timing:
@@ -266,9 +269,7 @@ class DecodeRunner:
             if j == 0:
                 self.h_i32[k].numpy()[0:n] = self.h_in[k].numpy()[:n]
                 self.h_i64[k].numpy()[B:B + n] = -1
-            self.i32.copy_(self.h_i32[k])
-            self.i64.copy_(self.h_i64[k])
-            self.f32.copy_(self.h_f32[k])
+            self.stage.copy_(self.h_stage[k])
             # the counter value of the step's first run: the redo samples the same RNG
             # stream, so the tokens never depend on the capacity
             self.step_ctr.fill_(p["ctr"])

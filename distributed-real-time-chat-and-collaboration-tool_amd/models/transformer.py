@@ -277,7 +277,7 @@ class TransformerLM:
 
     # ------------------------------------------------------------ forward
     def _embed(self, ids: torch.Tensor) -> torch.Tensor:
-        h = F.embedding(ids, self.embed)
+        h = ops.embed(ids, self.embed)
         if self.cfg.embed_scale:
             # Gemma: x * sqrt(H) with the normaliser rounded to the activation
             # dtype; a python scalar keeps the op graph-capturable (no H2D copy)

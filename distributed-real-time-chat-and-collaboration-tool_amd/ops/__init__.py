@@ -27,12 +27,12 @@ from .latent import (LatentDecodeWorkspace, PortionKeys, build_interleaved_rope,
                      latent_prep, latent_qtile, latent_width, portion_tiles, window_reach)
 from .memory import MemoryWeights, memory_decode, memory_scan, memory_slices
 from .moe import fused_moe, fused_moe_ref, router_logits, router_logits_f32
-from .norm import PendingNorm, dyt, dyt_ref, group_rms, rmsnorm, rmsnorm_ref
+from .norm import PendingNorm, dyt, dyt_ref, embed, group_rms, rmsnorm, rmsnorm_ref
 from .norm_conv import (MAX_TAPS, ConvTiles, LayerNorm, conv_tile_rows, norm_conv, sinusoid_turns,
                         softcap_)
 from .norm_side import side_gate, side_input, side_norm, stream_add
 from .rope import build_rope_cache, kv_write_v, kv_write_v_ref, rope_kv_, rope_kv_ref
-from .sampling import sample, sample_ref
+from .sampling import sample, sample_ref, step_begin
 from .talking import (MIX_TILE, STATS_TILE, TalkDecodeWorkspace, TalkPortions, TalkWeights,
                       head_prep, pad8, talk_cache_shapes, talk_decode, talk_prefill)
 
@@ -44,7 +44,8 @@ __all__ = [
     "decode_partitioning", "paged_decode_attention", "paged_decode_attention_rope",
     "paged_decode_ref", "prefill_attention", "prefill_attention_ref", "prefill_tiles",
     "set_prefill_persist", "rmsnorm", "rmsnorm_ref", "build_rope_cache", "rope_kv_",
-    "rope_kv_ref", "kv_write_v", "kv_write_v_ref", "sample", "sample_ref", "dyt", "dyt_ref",
+    "rope_kv_ref", "kv_write_v", "kv_write_v_ref", "sample", "sample_ref", "step_begin", "dyt", "dyt_ref",
+    "embed",
     "gated", "DeltaWeights", "Portions", "delta_decode", "delta_scan", "short_conv",
     "LatentDecodeWorkspace", "PortionKeys", "build_interleaved_rope", "head_linear",
     "latent_decode_attention", "latent_gather", "latent_prefill_attention", "latent_prep",

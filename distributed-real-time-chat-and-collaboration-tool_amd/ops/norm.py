@@ -50,6 +50,19 @@ def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, gemma: bool = False,
     return out
 
 
+def embed(ids: torch.Tensor, table: torch.Tensor) -> torch.Tensor:
+    """table[ids] of token ids [rows] (int32 or int64)."""
+    if not (on_gpu(table) and ids.device == table.device and ids.dim() == 1 and ids.is_contiguous()
+            and ids.dtype in (torch.int32, torch.int64) and table.dtype == torch.bfloat16
+            and table.is_contiguous() and table.shape[1] % 8 == 0
+            and not (table.requires_grad and torch.is_grad_enabled())):
+        return torch.nn.functional.embedding(ids, table)
+    out = table.new_empty(ids.shape[0], table.shape[1])
+    check(hipk().embed(out.data_ptr(), ids.data_ptr(), int(ids.dtype == torch.int64), table.data_ptr(),
+                       ids.shape[0], *table.shape, stream_ptr(table)), "embed")
+    return out
+
+
 def dyt_ref(h, w, b, alpha, y=None, ids=None, embed=None, dtype=torch.bfloat16):
     if ids is not None:
         h.copy_(embed[ids.long()])

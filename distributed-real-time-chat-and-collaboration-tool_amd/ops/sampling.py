@@ -96,3 +96,20 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor | None = None,
                         ptr(temperature), ptr(top_k), ptr(top_p), int(seed) & ((1 << 64) - 1),
                         ptr(step), stream_ptr(logits)), "sample")
     return out
+
+
+def step_begin(ids: torch.Tensor, src: torch.Tensor, sampled: torch.Tensor, host: torch.Tensor,
+               counter: torch.Tensor, position: torch.Tensor) -> None:
+    """The tokens a decode step starts from, into ``ids``: ``sampled[src]``, or ``host`` where src is
+    negative (all int32 [B], src int64); then position = counter, counter += 1 (int64 [1])."""
+    if not on_gpu(ids):
+        ids.copy_(torch.where(src >= 0, sampled.index_select(0, src.clamp(min=0)), host))
+        position.copy_(counter)
+        counter.add_(1)
+        return
+    B = ids.numel()
+    for t, dt, n in ((ids, torch.int32, B), (src, torch.int64, B), (sampled, torch.int32, B),
+                     (host, torch.int32, B), (counter, torch.int64, 1), (position, torch.int64, 1)):
+        assert t.dtype == dt and t.is_contiguous() and t.numel() == n and t.is_cuda
+    check(hipk().step_begin(ids.data_ptr(), src.data_ptr(), sampled.data_ptr(), host.data_ptr(), B,
+                            counter.data_ptr(), position.data_ptr(), stream_ptr(ids)), "step_begin")

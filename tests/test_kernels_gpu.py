@@ -974,3 +974,34 @@ def test_router_logits_on_skinny_kernel_match_fp32(hipk, T):
     assert torch.equal(sub, got[: max(1, T // 3)])
     view = M.router_logits(x, wr, contiguous=False)
     assert view.shape == (T, 8) and view.stride(0) == 1 and torch.equal(view, got)
+
+
+@pytest.mark.parametrize("rows,V,H", [(1, 3, 8), (5, 1000, 2048), (300, 77, 2056), (7, 128, 12288)])
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+def test_embed(hipk, rows, V, H, dtype):
+    """Rows of the table bit for bit, first and last token, rows past one trip of the workgroup; NaN for
+    tokens that the table does not have."""
+    g = torch.Generator().manual_seed(rows)
+    table = torch.randn(V, H, generator=g).to(torch.bfloat16).to(DEV)
+    ids = torch.randint(0, V, (rows,), generator=g)
+    ids[0], ids[-1] = 0, V - 1
+    ids = ids.to(dtype).to(DEV)
+    assert torch.equal(ops.embed(ids, table), table[ids.long()])
+    odd = ops.embed(torch.tensor([-1, V, 0], dtype=dtype, device=DEV), table)
+    assert odd[:2].isnan().all() and torch.equal(odd[2], table[0])
+
+
+@pytest.mark.parametrize("B", [1, 255, 257])
+def test_step_begin(hipk, B):
+    """Against the torch form on the CPU: tokens of the host and of the last samples in any order."""
+    g = torch.Generator().manual_seed(B)
+    src = torch.randint(-1, B, (B,), generator=g)
+    sampled, host = (torch.randint(0, 1 << 20, (B,), generator=g, dtype=torch.int32) for _ in range(2))
+    want, at, ctr = torch.empty(B, dtype=torch.int32), torch.zeros(1).long(), torch.tensor([1 << 40])
+    args = [x.to(DEV) for x in (want, src, sampled, host, ctr, at)]
+    for _ in range(2):
+        ops.step_begin(want, src, sampled, host, ctr, at)
+        ops.step_begin(*args)
+        for a, b in zip(args, (want, src, sampled, host, ctr, at)):
+            assert torch.equal(a.cpu(), b)
+    assert int(at) == (1 << 40) + 1
