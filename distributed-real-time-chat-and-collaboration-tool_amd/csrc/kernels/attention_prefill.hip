@@ -4,13 +4,10 @@
 // in-place RoPE kernel), so no Q/K/V copies are made: sequence s occupies
 // rows cu_seqlens[s] .. cu_seqlens[s+1] of the packed [T, qkv_stride] buffer.
 //
-// Work decomposition: grid = (n_q_tiles, Hq / GH); a workgroup owns a
-// 64-row query tile of GH query heads sharing one KV head (details below).
-// Measured on MI355X (scripts/prefill_attn_bench.py, vs the previous
-// one-head-per-workgroup kernel with synchronous staging and a scattered
-// V^T LDS image): Llama-3-8B smart-reply batch (1024 x ~148 tokens)
-// 1.67 -> 1.13 ms, summarize batch (512 x ~432) 3.62 -> 2.09 ms,
-// 16 x 4096 tokens 7.0 -> 3.3 ms (708 TFLOP/s), Gemma-2B 1.12 -> 0.61 ms.
+// Work decomposition: a workgroup owns a 64-row query tile of GH query heads
+// sharing one KV head.  Head sizes 64 and 128 run prefill_attn32_kernel (32
+// rows per wave, at the end), 256 and single heads of 128 the two kernels of
+// 16 rows per wave.
 //
 // MFMA formulation (16x16x32 bf16): the scores are computed transposed,
 //   S^T[key, q] = K[key, :] . Q[q, :]   (A = K from LDS, B = Q^T in registers)
@@ -409,6 +406,230 @@ __global__ __launch_bounds__(256 * GH) void prefill_attn_persist_kernel(
   }
 }
 
+// Head sizes 64 and 128: 32 query rows per wave.  What bounds a wave of 16 rows is the LDS: it reads each
+// tile's K and V (32 KiB at D = 128) for 512 cycles of MFMA, and 16 waves of a CU take 4096 LDS cycles
+// for 2048 of the matrix cores.  Two 32-row column blocks halve that: S^T[key, q] and O^T[d, q] are 32x32x16 MFMAs
+// (A = K rows / V columns, B = Q^T / P^T), lane l holds query l % 32 and, of 32 keys, those of its
+// half h = l / 32: accumulator word i is key 8 (i / 4) + 4 h + i % 4, so words 8t..8t+7 are the P^T operand of
+// the t-th 16 keys as they stand and the V operand is read in the same order of keys.
+// A workgroup is the 64-row query tile of GH heads as above, 2 waves per head.  The mask runs on tiles
+// that reach past the first query row or the sequence only, the rescaling of O where a maximum grew.
+// V rows are padded to 16 banks more than whole turns (the four rows and two column halves of a tr read).
+// PERSIST: resident workgroups loop over the items (see prefill_attn_persist_kernel).
+// 16 rows per wave -> this, us (TF/s of the causal half): 4 x 4000 tokens of 16 heads over 4 444 -> 331
+// (773), 4 x 4096 of 32 over 8 880 -> 636 (865), 15 x 1000 persistent 228 -> 188, 300 x 148 301 -> 292,
+// 8 x 2000 of 16 heads of 64 138 -> 101.  What bounds it now is each wave's own chain of scores, softmax
+// and output with only two waves to a SIMD (matrix cores busy for about 36 %).
+// One head of 128 per workgroup (2 waves, 64 staging registers each) stays with the 16-row waves above:
+// 16 x 1000 tokens 172 us there, 173 here, 64 x 150 45 and 53.
+template <int D, int GH>
+constexpr bool prefill32 = D == 64 || (D == 128 && GH >= 2);
+
+template <int D, int GH>
+struct Prefill32 {
+  static constexpr int KROW = D + 8;
+  static constexpr int VROW = D == 64 ? 96 : D + 32;
+  static constexpr int K_ELEMS = kKT * KROW;
+  static constexpr int BUF = K_ELEMS + kKT * VROW;
+  static constexpr size_t BYTES = (size_t)2 * BUF * 2;
+  static constexpr int NTHR = 128 * GH;
+};
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+DRTC_DEVICE f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+
+// the other half's value: lanes l and l ^ 32
+DRTC_DEVICE float half_max(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+template <int D, int GH, bool PERSIST>
+__global__ __launch_bounds__(128 * GH, 2) void prefill_attn32_kernel(
+    bf16_t* __restrict__ out, int out_stride, const bf16_t* __restrict__ qkv, int qkv_stride, int Hq, int Hkv,
+    const int* __restrict__ cu_seqlens, const int* __restrict__ tile_seq, const int* __restrict__ tile_q0, int n_tiles,
+    float scale_log2e, int causal) {
+  using L = Prefill32<D, GH>;
+  constexpr int KS = D / 16, NT = D / 32, VPR = D / 8, NV = kKT * VPR / L::NTHR;
+  static_assert(NV >= 1 && (kKT * VPR) % L::NTHR == 0, "staging split");
+  extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
+  const int G = Hq / Hkv, groups = G / GH, n_hg = Hq / GH, n_work = n_tiles * n_hg;
+  const int w = wave_id_uniform(), lane = threadIdx.x & 63;
+  const int col = lane & 31, h = lane >> 5;
+  const float scale = fabsf(scale_log2e);
+  const unsigned flip = scale_log2e < 0.f ? 0x80008000u : 0u;  // the sign goes to Q: the largest score stays that
+
+  struct Item {
+    int s_begin, seqlen, q0, hq, hk, ntiles;
+  };
+  auto info = [&](int item) -> Item {
+    const int tile = item / n_hg, hg = item - tile * n_hg, hk = hg / groups;
+    const int seq = tile_seq[tile], q0 = tile_q0[tile], s_begin = cu_seqlens[seq];
+    const int seqlen = cu_seqlens[seq + 1] - s_begin;
+    const int kv_end = causal ? min(seqlen, q0 + kQT) : seqlen;
+    return Item{s_begin, seqlen, q0, hk * G + (hg - hk * groups) * GH + (w >> 1), hk, (kv_end + kKT - 1) / kKT};
+  };
+  bf16x8 kr[NV], vr[NV];
+  auto issue = [&](const Item& it, int k0) {
+    const bf16_t* base = qkv + (int64_t)(it.s_begin + k0) * qkv_stride + (Hq + it.hk) * D;
+#pragma unroll
+    for (int n = 0; n < NV; ++n) {
+      const int v = threadIdx.x + n * L::NTHR, key = v / VPR, c = (v - key * VPR) * 8;
+      if (k0 + key < it.seqlen) {
+        const bf16_t* rp = base + key * qkv_stride + c;
+        kr[n] = load_bf16x8(rp);
+        vr[n] = load_bf16x8(rp + Hkv * D);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) kr[n][j] = vr[n][j] = f2bf(0.f);
+      }
+    }
+  };
+  auto commit = [&](bf16_t* kb) {
+#pragma unroll
+    for (int n = 0; n < NV; ++n) {
+      const int v = threadIdx.x + n * L::NTHR, key = v / VPR, c = (v - key * VPR) * 8;
+      store_bf16x8(kb + key * L::KROW + c, kr[n]);
+      store_bf16x8(kb + L::K_ELEMS + key * L::VROW + c, vr[n]);
+    }
+  };
+  auto load_q = [&](bf16x8* qf, const Item& it) {
+    const int qrow = it.q0 + 32 * (w & 1) + col;
+    const bf16_t* qp = qkv + (int64_t)(it.s_begin + qrow) * qkv_stride + it.hq * D + 8 * h;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      if (qrow < it.seqlen) qf[s] = load_bf16x8(qp + 16 * s);
+      else for (int j = 0; j < 8; ++j) qf[s][j] = f2bf(0.f);
+    }
+  };
+  auto turn = [&](bf16x8* qf) {
+    if (flip == 0) return;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      u32x4 t = __builtin_bit_cast(u32x4, qf[s]);
+      t ^= flip;
+      qf[s] = __builtin_bit_cast(bf16x8, t);
+    }
+  };
+  const int k_at = col * L::KROW + 8 * h;
+  const int v_at = (4 * h + ((lane & 15) >> 2)) * L::VROW + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+
+  const int nwg = gridDim.x;
+  auto item_of = [&](int round) -> int {
+    const int slot = (round & 1) ? nwg - 1 - (int)blockIdx.x : (int)blockIdx.x;
+    return round * nwg + slot;
+  };
+  int round = 0, buf = 0;
+  if (item_of(0) >= n_work) return;
+  Item cur = info(item_of(0));
+  issue(cur, 0);
+  bf16x8 qf[KS], qn[PERSIST ? KS : 1];
+  load_q(qf, cur);
+  while (true) {
+    turn(qf);
+    const int qrow = cur.q0 + 32 * (w & 1) + col;
+    // keys below `open` need no mask for any row of the workgroup
+    const int open = causal ? min(cur.seqlen, cur.q0 + 1) : cur.seqlen;
+    const int last = causal ? min(cur.seqlen - 1, qrow) : cur.seqlen - 1;  // last key of this row
+    f32x16 o[NT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
+    float m = kNegBig, lsum = 0.f;
+    const bool have_next = PERSIST && item_of(round + 1) < n_work;
+    Item nxt = cur;
+    for (int kt = 0; kt < cur.ntiles; ++kt) {
+      bf16_t* kb = lds + buf * L::BUF;
+      const bf16_t* vb = kb + L::K_ELEMS + v_at;
+      buf ^= 1;
+      commit(kb);
+      __syncthreads();
+      if (kt + 1 < cur.ntiles) {
+        issue(cur, (kt + 1) * kKT);
+      } else if (have_next) {
+        nxt = info(item_of(round + 1));
+        issue(nxt, 0);
+        if constexpr (PERSIST) load_q(qn, nxt);
+      }
+      f32x16 sc[2];
+#pragma unroll
+      for (int st = 0; st < 2; ++st) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sc[st][r] = 0.f;
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+          sc[st] = mfma32(load_bf16x8(kb + 32 * st * L::KROW + k_at + 16 * s), qf[s], sc[st]);
+      }
+      const int k0 = kt * kKT;
+      if (k0 + kKT > open) {
+        const int past = last - k0 - 4 * h;
+#pragma unroll
+        for (int st = 0; st < 2; ++st)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) sc[st][r] = 32 * st + 8 * (r / 4) + r % 4 <= past ? sc[st][r] : kNegBig;
+      }
+      float top = kNegBig;
+#pragma unroll
+      for (int st = 0; st < 2; ++st)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) top = fmaxf(top, sc[st][r]);
+      const float m_new = fmaxf(m, half_max(top) * scale);
+      const float alpha = fast_exp2(m - m_new);
+      if (__any(m != m_new)) {
+        lsum *= alpha;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) o[i] *= alpha;
+      }
+      m = m_new;
+      float psum[4] = {0.f, 0.f, 0.f, 0.f};
+      bf16x8 pf[4];
+#pragma unroll
+      for (int st = 0; st < 2; ++st)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float p = fast_exp2(__builtin_fmaf(sc[st][r], scale, -m));
+          psum[r & 3] += p;
+          pf[2 * st + r / 8][r % 8] = f2bf(p);
+        }
+      lsum += (psum[0] + psum[1]) + (psum[2] + psum[3]);
+#pragma unroll
+      for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const bf16x4 lo = lds_read_tr16(vb + 16 * t * L::VROW + 32 * i);
+          const bf16x4 hi = lds_read_tr16(vb + (16 * t + 8) * L::VROW + 32 * i);
+          bf16x8 a;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) { a[j] = lo[j]; a[4 + j] = hi[j]; }
+          o[i] = mfma32(a, pf[t], o[i]);
+        }
+    }
+    lsum += __shfl_xor(lsum, 32, 64);
+    if (qrow < cur.seqlen) {
+      const float inv = 1.f / lsum;
+      bf16_t* op = out + (int64_t)(cur.s_begin + qrow) * out_stride + cur.hq * D + 4 * h;
+#pragma unroll
+      for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          bf16x4 v;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = f2bf(o[i][4 * q + r] * inv);
+          *reinterpret_cast<bf16x4*>(op + 32 * i + 8 * q) = v;
+        }
+    }
+    if (!have_next) break;
+    if constexpr (PERSIST) {
+      cur = nxt;
+      ++round;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) qf[s] = qn[s];
+    }
+  }
+}
+
 static int prefill_persist_grid(int n_work) {
   static int n_cu = 0;
   if (n_cu == 0) {
@@ -425,27 +646,45 @@ template <int D, int GH>
 static void launch_tile(dim3 grid, hipStream_t st, bf16_t* out, int out_stride, const bf16_t* qkv,
                       int qkv_stride, int Hq, int Hkv, const int* cu, const int* ts,
                       const int* tq, float sl2, int causal, int persist) {
-  constexpr size_t lds_bytes = PrefillLds<D, GH>::BYTES;
-  if (persist) {
-    // resident workgroups per CU for this instantiation (VGPRs / LDS / waves)
-    static int per_cu = 0;
-    if (per_cu == 0) {
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-              &per_cu, prefill_attn_persist_kernel<D, GH>, 256 * GH, lds_bytes) != hipSuccess ||
-          per_cu <= 0)
-        per_cu = 1;
+  const int n_work = (int)(grid.x * grid.y);
+  if constexpr (prefill32<D, GH>) {
+    using L = Prefill32<D, GH>;
+    if constexpr (GH == 4) {  // with fewer waves to a workgroup the others of its CU fill its gaps
+      if (persist) {
+        static int per_cu = 0;
+        if (per_cu == 0 && (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                                &per_cu, prefill_attn32_kernel<D, GH, true>, L::NTHR, L::BYTES) != hipSuccess ||
+                            per_cu <= 0))
+          per_cu = 1;
+        const int n_wg = std::min(n_work, prefill_persist_grid(n_work * per_cu) * per_cu);
+        prefill_attn32_kernel<D, GH, true><<<std::max(1, n_wg), L::NTHR, L::BYTES, st>>>(
+            out, out_stride, qkv, qkv_stride, Hq, Hkv, cu, ts, tq, (int)grid.x, sl2, causal);
+        return;
+      }
     }
-    const int n_work = (int)(grid.x * grid.y);
-    const int n_wg = std::min(n_work, prefill_persist_grid(n_work * per_cu) * per_cu);
-    prefill_attn_persist_kernel<D, GH><<<dim3(std::max(1, n_wg)), dim3(256 * GH),
-                                          lds_bytes, st>>>(
+    prefill_attn32_kernel<D, GH, false><<<n_work, L::NTHR, L::BYTES, st>>>(
         out, out_stride, qkv, qkv_stride, Hq, Hkv, cu, ts, tq, (int)grid.x, sl2, causal);
-    return;
+  } else {
+    constexpr size_t lds_bytes = PrefillLds<D, GH>::BYTES;
+    if (persist) {
+      // resident workgroups per CU for this instantiation (VGPRs / LDS / waves)
+      static int per_cu = 0;
+      if (per_cu == 0) {
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &per_cu, prefill_attn_persist_kernel<D, GH>, 256 * GH, lds_bytes) != hipSuccess ||
+            per_cu <= 0)
+          per_cu = 1;
+      }
+      const int n_wg = std::min(n_work, prefill_persist_grid(n_work * per_cu) * per_cu);
+      prefill_attn_persist_kernel<D, GH><<<dim3(std::max(1, n_wg)), dim3(256 * GH),
+                                            lds_bytes, st>>>(
+          out, out_stride, qkv, qkv_stride, Hq, Hkv, cu, ts, tq, (int)grid.x, sl2, causal);
+      return;
+    }
+    prefill_attn_kernel<D, GH><<<grid, dim3(256 * GH), lds_bytes, st>>>(
+        out, out_stride, qkv, qkv_stride, Hq, Hkv, cu, ts, tq, sl2, causal);
   }
-  prefill_attn_kernel<D, GH><<<grid, dim3(256 * GH), lds_bytes, st>>>(
-      out, out_stride, qkv, qkv_stride, Hq, Hkv, cu, ts, tq, sl2, causal);
 }
-
 
 template <int D>
 static int launch_gh(int GH, int ntiles, int Hq, int Hkv, hipStream_t st, bf16_t* out,
@@ -495,13 +734,18 @@ int launch_prefill_attn(void* out, int out_stride, const void* qkv,
 
 template <int D, int GH>
 static int set_lds() {
-  int e = (int)hipFuncSetAttribute((const void*)prefill_attn_kernel<D, GH>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)PrefillLds<D, GH>::BYTES);
-  if (!e)
-    e = (int)hipFuncSetAttribute((const void*)prefill_attn_persist_kernel<D, GH>,
-                                 hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 (int)PrefillLds<D, GH>::BYTES);
+  auto set = [](auto* kernel, size_t bytes) {
+    return (int)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  };
+  int e;
+  if constexpr (prefill32<D, GH>) {
+    e = set(prefill_attn32_kernel<D, GH, false>, Prefill32<D, GH>::BYTES);
+    if constexpr (GH == 4)
+      if (!e) e = set(prefill_attn32_kernel<D, GH, true>, Prefill32<D, GH>::BYTES);
+  } else {
+    e = set(prefill_attn_kernel<D, GH>, PrefillLds<D, GH>::BYTES);
+    if (!e) e = set(prefill_attn_persist_kernel<D, GH>, PrefillLds<D, GH>::BYTES);
+  }
   return e;
 }
 

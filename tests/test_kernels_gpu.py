@@ -356,6 +356,25 @@ def test_prefill_attention(hipk, D, Hq, Hkv, lens, persist):
     _close(out, ref, 2e-2, 2e-2, "prefill")
 
 
+@pytest.mark.parametrize("D,Hq,Hkv", [(128, 16, 8), (128, 8, 2), (64, 2, 2), (64, 8, 4)])
+@pytest.mark.parametrize("causal,sign", [(True, 1), (False, 1), (True, -1)])
+@pytest.mark.parametrize("persist", [True, False])
+def test_prefill_rows32(hipk, D, Hq, Hkv, causal, sign, persist):
+    """32 query rows per wave: lengths around its rows and key tiles, all keys, a negative scale (the sign
+    goes to Q), rows with spare columns.  Scores of a standard deviation of 1, tolerance as above."""
+    lens = [1, 31, 33, 64, 65, 96, 129, 300]
+    cu = [sum(lens[:i]) for i in range(len(lens) + 1)]
+    g = torch.Generator().manual_seed(3)
+    W = (Hq + 2 * Hkv) * D
+    qkv = torch.randn(cu[-1], W + 24, generator=g).to(torch.bfloat16).to(DEV)[:, :W]
+    ops.set_prefill_persist(persist)
+    out = ops.prefill_attention(qkv, torch.tensor(cu, dtype=torch.int32, device=DEV), Hq, Hkv, D,
+                                sign * D ** -0.5, causal, cu_host=cu)
+    ops.set_prefill_persist(None)
+    ref = ops.prefill_attention_ref(qkv.float(), cu, Hq, Hkv, D, sign * D ** -0.5, causal)
+    _close(out, ref, 2e-2, 2e-2, "prefill")
+
+
 @pytest.mark.parametrize("persist", [True, False])
 def test_prefill_attention_shape_padding_rows_zero(hipk, persist):
     """A shape-padded chunk (T > cu[-1]): the op allocates its output, only the
