@@ -644,19 +644,23 @@ class LLMEngine:
                 lens_a, starts, blk_tab,
                 np.fromiter((r.state_slot for r in batch), np.int64, count=nseq), Tp, d_state,
                 d_start)
-        h_i32 = torch.from_numpy(np.concatenate([
+        h_i32 = np.concatenate([
             ids, pos, np.asarray(cu, np.int32), np.asarray(ts, np.int32),
             np.asarray(tq, np.int32), seg_tok, seg_len, seg_blk,
             params[:, 2].astype(np.int32)] + dec_i32
-            + [v.astype(np.int32) for v in x32.values()]))
-        h_i64 = torch.from_numpy(np.concatenate([
-            slots, last_idx, np.array([step + (1 << 40)], dtype=np.int64), *x64.values()]))
-        h_f32 = torch.from_numpy(params[:, :2].T.astype(np.float32).reshape(-1))
-        if cuda:  # pinned staging: the copies stay asynchronous to the host
-            h_i32, h_i64, h_f32 = h_i32.pin_memory(), h_i64.pin_memory(), h_f32.pin_memory()
-        t_i32 = h_i32.to(dev, non_blocking=True)
-        t_i64 = h_i64.to(dev, non_blocking=True)
-        t_f32 = h_f32.to(dev, non_blocking=True)
+            + [v.astype(np.int32) for v in x32.values()])
+        h_i64 = np.concatenate([
+            slots, last_idx, np.array([step + (1 << 40)], dtype=np.int64), *x64.values()])
+        h_f32 = params[:, :2].T.astype(np.float32).reshape(-1)
+        # one buffer, one copy
+        stage = torch.from_numpy(np.concatenate([v.view(np.uint8) for v in (h_i64, h_i32, h_f32)]))
+        if cuda:  # pinned staging: the copy stays asynchronous to the host
+            stage = stage.pin_memory()
+        stage = stage.to(dev, non_blocking=True)
+        b64, b32 = h_i64.nbytes, h_i64.nbytes + h_i32.nbytes
+        t_i64 = stage[:b64].view(torch.int64)
+        t_i32 = stage[b64:b32].view(torch.int32)
+        t_f32 = stage[b32:].view(torch.float32)
         nt, ns = len(ts), len(seg_tok)
         o = 0
         d_ids = t_i32[o:o + R]; o += R
@@ -779,17 +783,14 @@ class LLMEngine:
         dids = np.array([entries[e][1][0] for e, _, _ in dec], dtype=np.int32)
         out: list = [None] * len(entries)
         if segs:
-            rows, owner = [], []
-            for q, (e, r, _) in enumerate(segs):
-                rows += [(q, t) for t in entries[e][2]]
-                owner += [e] * len(entries[e][2])
-            for q, (e, _, _) in enumerate(dec):
-                rows += [(-1, q) for _ in entries[e][2]]
-                owner += [e] * len(entries[e][2])
+            rows = [(q, t) for q, (e, _, _) in enumerate(segs) for t in entries[e][2]]
+            rows += [(-1, q) for q, (e, _, _) in enumerate(dec) for _ in entries[e][2]]
             st = self._stage_prefill([(r, entries[e][1], a) for e, r, a in segs], dslots, dids, rows)
             logits = self.model.forward_prefill(st["ids"], st["meta"], self.kv)
-            for e in range(len(entries)):
-                out[e] = logits[[i for i, o in enumerate(owner) if o == e]]
+            at = 0
+            for e, _, _ in segs + dec:  # an entry's rows lie together
+                out[e] = logits[at:at + len(entries[e][2])]
+                at += len(entries[e][2])
         else:
             pos = self.ctx[dslots]
             n = len(dec)
@@ -802,7 +803,7 @@ class LLMEngine:
             self.runner.wait(h)
             logits = self.runner.logits[self.runner.bucket(n)]
             for q, (e, _, _) in enumerate(dec):
-                out[e] = logits[[q] * len(entries[e][2])]
+                out[e] = logits[q:q + 1].repeat(len(entries[e][2]), 1)
         for r, toks, _ in entries:
             self.ctx[r.slot] += len(toks)
             r.prompt_ids = list(r.prompt_ids) + list(toks)

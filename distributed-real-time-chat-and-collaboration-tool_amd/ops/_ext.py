@@ -51,7 +51,8 @@ def hipk():
 
 
 def stream_ptr(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # the handle without a Stream object: a third of the host time of a small kernel's launch
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def check(rc: int, name: str) -> None:
