@@ -466,7 +466,8 @@ def stream_ok(M: int, N: int, K: int, epi: str = "store") -> bool:
       17 .. 32 rows: 2048 columns take what the other kernels need for 64 rows (2560 x 2048 8.1 / 11.4);
         4096 columns leave the registers for one workgroup per CU, which pays for long W (16384 rows 29 /
         33, 32000 51 / 65; 12800 27 / 26)
-      33 .. 64 rows: 2048 columns and long W (32768 gated 34 / 39, 64000 59 / 71; 8192 15.7 / 12.6)
+      33 .. 64 rows: 2048 columns and long W (64000 rows 59 / 71; 8192 15.7 / 12.6); gated where gemm_xd's
+        form does not fill the chip (32768 rows 34.7, gemm_xd 32.5)
       slices: adding the parts up costs about 3 us, and more for more rows: plain products of few
         slices (4096 x 14336 25.4 / 27.8, 2048 x 16384 17.3 / 23.2, 2048 x 7168 also at 32 rows 15.4 / 18.4;
         4096 x 14336 at 32 rows 30.3 / 29.1, 8192 x 28672 91 / 89)"""
@@ -480,7 +481,7 @@ def stream_ok(M: int, N: int, K: int, epi: str = "store") -> bool:
         return rows * K >= 24_000_000
     if M <= 32:
         return rows >= (16384 if K > 2048 else 2048)
-    return rows >= 14336
+    return rows >= 14336 and not (STREAM_ACT[epi][0] and _glu_default(M, N, K))
 
 
 def stream_gemm(x: torch.Tensor, w: torch.Tensor, epi: str = "store", out: torch.Tensor | None = None,
@@ -845,15 +846,42 @@ def w4_glu_ok(x: torch.Tensor, w: torch.Tensor, act: str) -> bool:
 
 
 def glu_form(M: int, N2: int, K: int, ldx: int, act: str = "silu") -> int:
-    """gemm_xd gated form the tuning table measured fastest for a decode batch M through the
-    [gate; up] weight [N2, K] (bucket-above for an off-bucket M), 0 if none."""
+    """gemm_xd gated form for a decode batch M through the [gate; up] weight [N2, K]: the one the
+    tuning table measured fastest (bucket-above for an off-bucket M), else ``_glu_default``; 0:
+    none."""
     if not (_xd_enabled and _enabled) or M > DECODE_MAX_M:
         return 0
     found = _decode_entry(M, N2, K, ldx)
-    form = found[1][4] if found is not None else 0
+    form = found[1][4] if found is not None and found[1][4] else _glu_default(M, N2 // 2, K)
     if act == "clamped" and form // 10 % 10 not in XD_CLAMP_NF:
         return 0
     return form if form and xd_supported(M, N2 // 2, K, form, glu=True) else 0
+
+
+def _glu_default(M: int, I: int, K: int) -> int:
+    """gemm_xd gated form of a shape without a measured one, 0 where the library's product and an
+    activation pass, or above 640 rows gemm_w4, are as fast.  One launch and no [M, 2 I] intermediate
+    win where ``xd_default_form``'s tiles fill the chip: 160 of them, 112 where K is short.  us,
+    library + pass / gemm_xd: 7168 x 2048 rows of W a half, 64 rows of x 22.8 / 16.6, 160 28.6 / 20.2, 512
+    38.5 / 32.4; 14336 x 4096, 64 rows 56.0 / 48.7; 11008 x 4096, 224 rows 64.9 / 56.6; too few tiles:
+    3584 x 4096, 64 rows 21.4 / 24.8.  Tiles of 128 columns a half lose to narrower ones up to 128 rows
+    (28672 x 8192 188 / 199, narrow 179) and to the library above 256 (14336 x 4096, 320 rows 82 / 97).
+    Above 512 rows for the shapes that leave gemm_w4 fewer than three quarters of the CUs: 3584 x 2048, 768 rows
+    90 / 29.6, 1024 49 / 30.7; 7168 x 2048, 1024 rows (224 tiles) 53.0 / 53.4."""
+    if not 17 <= M <= DECODE_MAX_M or M > 512 and -(-M // 256) * (I // 128) > 176:
+        return 0
+    form = xd_default_form(M, I, K, True)
+    if form // 10 % 10 == 8 and M <= 512:
+        if M > 256:
+            return 0
+        if M <= 128:
+            form = 141
+    if not form or not xd_supported(M, I, K, form, True):
+        return 0
+    mt, nf, _ = xd_form(form)
+    if -(-M // (128 * mt)) * (I // (16 * nf)) < (112 if K <= 2048 else 160):
+        return 0
+    return form + 1000 if xd_nt_ok(M, form) else form
 
 
 def _stream_glu_ok(x: torch.Tensor, w: torch.Tensor, act: str) -> bool:

@@ -162,3 +162,25 @@ def test_routing_plan(hipk, T, E, k, groups, keep):
         want = (w * (ids + 1)).sum(-1)
         # a wrong expert moves the sum by a weight times a whole number; the fp32 sums by 1e-5 of it
         assert (y[:, 0] - want).abs().max() <= 1e-4 * E
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,I,K,act", [(17, 8192, 2048, "silu"), (33, 14336, 1024, "gelu_tanh"), (127, 10240, 4096, "silu"),
+                                       (129, 3584, 4096, "silu"), (257, 7168, 1024, "clamped"), (511, 5632, 512, "silu"),
+                                       (700, 1792, 2048, "silu"), (130, 28672, 512, "gelu_tanh")])
+def test_gated_default_form(hipk, M, I, K, act):
+    """Shapes that no table measured, through the rule that sends them to gemm_xd: rows of x apart, M
+    around its tiles, against 64 bits (bf16 rounding of the result, 2^-9 of it, and of nothing else)."""
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K + 16, generator=g).bfloat16().to("cuda")[:, :K]
+    w = (torch.randn(2 * I, K, generator=g) / K ** 0.5).bfloat16().to("cuda")
+    form = ops.gemm.glu_form(M, 2 * I, K, x.stride(0), act)
+    assert form == ops.gemm._glu_default(M, I, K) != 0 and ops.gemm.fused_glu_ok(x, w, act)
+    got = ops.gemm.gated(x, w, act, limit=1.0).double()
+    a, b = (x.double() @ w.double().t()).chunk(2, -1)
+    if act == "clamped":
+        a, b = a.clamp(max=1.0), b.clamp(-1.0, 1.0)
+        want = a * torch.sigmoid(1.702 * a) * (b + 1)
+    else:
+        want = (torch.nn.functional.silu(a) if act == "silu" else torch.nn.functional.gelu(a, approximate="tanh")) * b
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all()
