@@ -70,6 +70,8 @@ DRTC_DEVICE void moe_choose(const L* logits, int t, int E, int k, int lts, int l
   // in place (lts = 1: consecutive threads read consecutive tokens of one expert row)
   const L* lr = logits + (int64_t)t * lts;
   const int per = E / groups;
+  // rows of 16-bit logits that lie in whole 16-byte pieces
+  const bool rows8 = les == 1 && lts % 8 == 0 && per % 8 == 0 && ((uintptr_t)logits & 15) == 0;
   uint64_t open = ~0ull;
   if (groups > 1) {
     for (int g = 0; g < groups; ++g) {
@@ -96,23 +98,43 @@ DRTC_DEVICE void moe_choose(const L* logits, int t, int E, int k, int lts, int l
   for (int j = 0; j < KM; ++j) top[j] = 0;
   for (int g = 0; g < groups; ++g) {
     if (!(open >> g & 1)) continue;
-    for (int e0 = g * per; e0 < (g + 1) * per; e0 += 8) {
-      const int ne = min(8, (g + 1) * per - e0);
-      float xs[8];  // loads in flight together
+    const int end = (g + 1) * per;
+    L xs[2][16];  // loads in flight together: these logits and the next
+    auto fetch = [&](L (&d)[16], int e0) {
+      if constexpr (sizeof(L) == 2) {
+        if (rows8) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) xs[i] = logit_f32(lr[(int64_t)(e0 + min(i, ne - 1)) * les]);
+          for (int i = 0; i < 16; i += 8) {
+            const bf16x8 v = load_bf16x8(lr + min(e0 + i, end - 8));
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const uint32_t u = __float_as_uint(xs[i] + 0.f);  // -0 is 0
-        const uint32_t key = u ^ (u >> 31 ? 0xffffffffu : 0x80000000u);
-        uint64_t x = i < ne ? (uint64_t)key << 32 | (uint32_t)~(e0 + i) : 0;  // behind the last: never in
-#pragma unroll
-        for (int j = 0; j < KM; ++j) {
-          const uint64_t hi = x > top[j] ? x : top[j];
-          x = x > top[j] ? top[j] : x;
-          top[j] = hi;
+            for (int j = 0; j < 8; ++j) d[i + j] = v[j];
+          }
+          return;
         }
       }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) d[i] = lr[(int64_t)min(e0 + i, end - 1) * les];
+    };
+    fetch(xs[0], g * per);
+    for (int e0 = g * per; e0 < end; e0 += 16) {
+      const int ne = min(16, end - e0);
+      if (e0 + 16 < end) fetch(xs[1], e0 + 16);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        if (i < ne) {  // (a break would leave the logits indexed at run time)
+          const uint32_t u = __float_as_uint(logit_f32(xs[0][i]) + 0.f);  // -0 is 0
+          const uint32_t key = u ^ (u >> 31 ? 0xffffffffu : 0x80000000u);
+          uint64_t x = (uint64_t)key << 32 | (uint32_t)~(e0 + i);
+#pragma unroll
+          for (int j = 0; j < KM; ++j) {
+            const uint64_t hi = x > top[j] ? x : top[j];
+            x = x > top[j] ? top[j] : x;
+            top[j] = hi;
+          }
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) xs[0][i] = xs[1][i];
     }
   }
   float v[KM];
@@ -157,8 +179,8 @@ __global__ __launch_bounds__(kMoeRouteWG) void moe_route_kernel(
 }
 
 // The three passes in one workgroup for decode batches: nothing crosses memory between them.  224
-// tokens, 16 experts, 4 per token: 9 us against 11 + 5 + 7.  NT 256 or 1024 threads, one per token; the
-// order of an expert's pairs is (slot, token).
+// tokens, 16 experts, 4 per token: 7 us against 11 + 5 + 7 (13 with a count per slot and expert).  NT 256 or 1024 threads, one per token.
+// A wave's tokens of an expert are a bit mask, so an expert's pairs lie in token order.
 struct MoePlan {
   int* sorted_tok;
   float* sorted_w;
@@ -171,28 +193,34 @@ template <class L, int KM, int NT>
 __global__ __launch_bounds__(NT) void moe_plan_kernel(const L* __restrict__ logits, int T, int E, int k, int lts,
                                                       int les, int groups, int keep, MoePlan p) {
   extern __shared__ float gmax[];  // [groups][NT] (groups > 1)
-  __shared__ int run[256], off[257], toff[257], wcnt[NT / 64][256];
+  constexpr int NW = NT / 64;
+  __shared__ unsigned has[NW][256][2];  // tokens of a wave that chose an expert
+  __shared__ int off[257], toff[257], pre[NW][256];
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  for (int e = t; e < E; e += NT) run[e] = 0;
+  for (int i = t; i < NW * E; i += NT) has[i / E][i % E][0] = has[i / E][i % E][1] = 0;
   __syncthreads();
   int id[KM];
   float w[KM];
-#pragma unroll
-  for (int j = 0; j < KM; ++j) id[j] = -1;
   if (t < T) {
     moe_choose<L, KM, NT>(logits, t, E, k, lts, les, groups, keep, gmax, id, w);
 #pragma unroll
     for (int j = 0; j < KM; ++j)
       if (j < k) {
         p.topk_w[t * k + j] = w[j];
-        atomicAdd(&run[id[j]], 1);  // a count: its order does not matter
+        atomicOr(&has[wv][id[j]][lane >> 5], 1u << (lane & 31));
       }
   }
   __syncthreads();
   if (wv == 0) {  // offsets of pairs and row tiles, 64 experts at a time
     int o = 0, to = 0;
     for (int e0 = 0; e0 < E; e0 += 64) {
-      const int e = e0 + lane, c = e < E ? run[e] : 0;
+      const int e = e0 + lane;
+      int c = 0;
+      if (e < E)
+        for (int v = 0; v < NW; ++v) {
+          pre[v][e] = c;
+          c += __popc(has[v][e][0]) + __popc(has[v][e][1]);
+        }
       const bool loc = e >= p.e_off && e < p.e_off + p.e_local;  // tiles only for this rank's experts (EP)
       const int n = loc ? (c + p.bm - 1) / p.bm : 0;
       int x = c, y = n;
@@ -229,34 +257,17 @@ __global__ __launch_bounds__(NT) void moe_plan_kernel(const L* __restrict__ logi
       p.tile_row0[ti] = off[e] + i * p.bm;
       p.tile_rows[ti] = min(p.bm, c - i * p.bm);
     }
-    run[e] = off[e];
   }
-  const uint64_t below = (1ull << lane) - 1;
+  if (t >= T) return;
 #pragma unroll
   for (int j = 0; j < KM; ++j) {
     if (j >= k) break;
     const int e = id[j];
-    int rank = 0;
-    for (int x = 0; x < E; ++x) {  // this wave's pairs of expert x, in lane order
-      const uint64_t m = __ballot(e == x);
-      if (e == x) rank = __popcll(m & below);
-      if (lane == 0) wcnt[wv][x] = __popcll(m);
-    }
-    __syncthreads();
-    if (e >= 0) {
-      int r = run[e] + rank;
-      for (int v = 0; v < wv; ++v) r += wcnt[v][e];
-      p.sorted_tok[r] = t;
-      p.sorted_w[r] = w[j];
-      p.inv_pos[t * k + j] = r;
-    }
-    __syncthreads();
-    for (int x = t; x < E; x += NT) {
-      int c = 0;
-      for (int v = 0; v < NT / 64; ++v) c += wcnt[v][x];
-      run[x] += c;
-    }
-    __syncthreads();
+    const uint64_t m = (uint64_t)has[wv][e][1] << 32 | has[wv][e][0];
+    const int r = off[e] + pre[wv][e] + __popcll(m & ((1ull << lane) - 1));
+    p.sorted_tok[r] = t;
+    p.sorted_w[r] = w[j];
+    p.inv_pos[t * k + j] = r;
   }
 }
 
@@ -326,8 +337,8 @@ __global__ __launch_bounds__(64 * kRouterWaves) void moe_router_kernel(float* __
 }
 
 // The same sums in the same order for decode-sized batches: 16 tokens to a workgroup, twice the steps
-// in flight, one barrier.
-template <int ET>
+// in flight, one barrier.  U: steps of a wave in flight (a step behind the end costs its loads all the same).
+template <int ET, int U>
 __global__ __launch_bounds__(64 * kRouterWaves) void moe_router_few_kernel(
     float* __restrict__ out, const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict__ w, int T,
     int E, int K) {
@@ -340,7 +351,6 @@ __global__ __launch_bounds__(64 * kRouterWaves) void moe_router_few_kernel(
   bf16x8 zero;
 #pragma unroll
   for (int j = 0; j < 8; ++j) zero[j] = f2bf(0.f);
-  constexpr int U = 16;
   for (int c0 = 32 * wv; c0 < K; c0 += 32 * kRouterWaves * U) {
     bf16x8 b[U], a[U][ET];
 #pragma unroll
@@ -380,8 +390,10 @@ int launch_moe_router(float* out, const void* x, int ldx, const void* w, int T, 
   const bf16_t *xx = (const bf16_t*)x, *ww = (const bf16_t*)w;
 #define DRTC_ROUTER(N) moe_router_kernel<N><<<grid, dim3(64 * kRouterWaves), 0, st>>>(out, xx, ldx, ww, T, E, K)
   if (T <= 1024 && E <= 32) {
-    if (E <= 16) moe_router_few_kernel<1><<<few, dim3(64 * kRouterWaves), 0, st>>>(out, xx, ldx, ww, T, E, K);
-    else moe_router_few_kernel<2><<<few, dim3(64 * kRouterWaves), 0, st>>>(out, xx, ldx, ww, T, E, K);
+    const bool u8 = K <= 32 * kRouterWaves * 8;
+    (E <= 16 ? u8 ? moe_router_few_kernel<1, 8> : moe_router_few_kernel<1, 16>
+             : u8 ? moe_router_few_kernel<2, 8> : moe_router_few_kernel<2, 16>)
+        <<<few, dim3(64 * kRouterWaves), 0, st>>>(out, xx, ldx, ww, T, E, K);
   } else if (E <= 16) DRTC_ROUTER(1);
   else if (E <= 32) DRTC_ROUTER(2);
   else if (E <= 64) DRTC_ROUTER(4);
