@@ -190,6 +190,30 @@ struct StateTile {
         s[i][c] = r < dim && col + c < vdim ? S[(int64_t)r * vdim + col + c] : 0.f;
     }
   }
+  // of a state that fills the tiles: one register of addresses
+  template <bool STORE>
+  DRTC_DEVICE void move_all(float* S, int col, int p, int vdim) {
+    static_assert(CPL % 4 == 0, "16-byte pieces");
+    const __amdgpu_buffer_rsrc_t at =
+        __builtin_amdgcn_make_buffer_rsrc((void*)S, (short)0, 8 * DPL * vdim * 4, 0x00020000);
+    const int off = (4 * p * vdim + col) * 4;
+#pragma unroll
+    for (int i = 0; i < DPL; ++i)
+#pragma unroll
+      for (int c = 0; c < CPL; c += 4) {
+        const int so = row_of(i, 0) * vdim * 4;
+        f32x4 v;
+        if constexpr (STORE) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] = s[i][c + j];
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), at, off + 4 * c, so, 0);
+        } else {
+          v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(at, off + 4 * c, so, 0));
+#pragma unroll
+          for (int j = 0; j < 4; ++j) s[i][c + j] = v[j];
+        }
+      }
+  }
   DRTC_DEVICE void store(float* S, int col, int p, int dim, int vdim) const {
     if constexpr (CPL % 4 == 0) {
       if ((vdim & 3) == 0) {
@@ -1134,7 +1158,11 @@ __global__ __launch_bounds__(256) void delta_read_kernel(DeltaArgs a) {
     for (int h = h0; h < min(a.H, h0 + NH); ++h) keep_ring<T>(a, at.slot, h, at.n, at.row0, at.pos0);
 }
 
-template <class T, int DPL, int CPL>
+// Bound by the state, read and written once; everything a token needs besides it is asked for ahead of
+// it, so that the token is prepared while it arrives (memory answers in order).  EXACT: the state fills
+// the lanes' tiles, so no load of it stands behind a condition and the waits can count them.
+constexpr int kDecodeTaps = 4;  // taps whose inputs are fetched ahead; more are read where they are used
+template <class T, int DPL, int CPL, bool EXACT>
 __global__ __launch_bounds__(512) void delta_decode_kernel(DeltaArgs a) {
   constexpr int DP = 8 * DPL;
   extern __shared__ __attribute__((aligned(16))) float sm[];
@@ -1157,32 +1185,62 @@ __global__ __launch_bounds__(512) void delta_decode_kernel(DeltaArgs a) {
   const int grp = a.H / a.Hk, hk = h / grp;
   const int cq = hk * a.dim, ck = (a.Hk + hk) * a.dim, cv = 2 * a.Hk * a.dim + h * a.vdim;
   float* S = a.state + ((int64_t)slot * a.H + h) * a.dim * a.vdim;
-  StateTile<DPL, CPL> st;  // in flight while the token's inputs are prepared
-  if (pos > 0) st.load(S, col, p, a.dim, a.vdim);
-  else st.zero();
-
   const T* pr = (const T*)a.proj + (int64_t)row * a.ldp;
   T* ring = (T*)a.ring + (int64_t)slot * a.taps * a.C;
   const bool own = h % grp == 0;
-  auto conv = [&](int c, bool keep) {
-    const T x0 = pr[c];
-    float acc = to_f32(x0) * a.conv_w[(int64_t)(a.taps - 1) * a.C + c];
-    const int back = min(pos, a.taps - 1);
-    for (int j = 1; j <= back; ++j)
+  const int back = min(pos, a.taps - 1);
+  struct Taps {
+    T x[kDecodeTaps];
+    float w[kDecodeTaps];
+  };
+  auto fetch = [&](Taps& t, int c) {
+#pragma unroll
+    for (int j = 0; j < kDecodeTaps; ++j) {
+      t.x[j] = from_f32<T>(0.f);
+      t.w[j] = 0.f;
+      if (j <= back) {
+        t.x[j] = j ? ring[(int64_t)((pos - j) % a.taps) * a.C + c] : pr[c];
+        t.w[j] = a.conv_w[(int64_t)(a.taps - 1 - j) * a.C + c];
+      }
+    }
+  };
+  auto conv = [&](const Taps& t, int c, bool keep) {
+    float acc = to_f32(t.x[0]) * t.w[0];
+#pragma unroll
+    for (int j = 1; j < kDecodeTaps; ++j) acc += to_f32(t.x[j]) * t.w[j];
+    for (int j = kDecodeTaps; j <= back; ++j)
       acc += to_f32(ring[(int64_t)((pos - j) % a.taps) * a.C + c]) *
              a.conv_w[(int64_t)(a.taps - 1 - j) * a.C + c];
-    if (keep) ring[(int64_t)(pos % a.taps) * a.C + c] = x0;
+    if (keep) ring[(int64_t)(pos % a.taps) * a.C + c] = t.x[0];
     return to_f32(from_f32<T>(silu_as<T>(acc)));
   };
+  // this thread's first channels: q, k, the decay, v; threads past them take the last
+  const T* dec = (const T*)a.decay + (int64_t)row * a.ld_decay + h * a.dim;
+  const int i0 = min(tid, a.dim - 1), e0 = min(tid, a.vdim - 1);
+  Taps tq, tk, tv;
+  fetch(tq, cq + i0);
+  fetch(tk, ck + i0);
+  fetch(tv, cv + e0);
+  T d0 = dec[i0];
+  const float dt0 = a.dt_bias[h * a.dim + i0];
+  __builtin_amdgcn_sched_barrier(0);
+  StateTile<DPL, CPL> st;
+  if constexpr (EXACT) st.template move_all<false>(S, col, p, a.vdim);
+  else if (pos > 0) st.load(S, col, p, a.dim, a.vdim);
+  __builtin_amdgcn_sched_barrier(0);
   float sq = 0.f, sk = 0.f, dot = 0.f;
   const float aexp = a.a_exp[h];
-  const T* dec = (const T*)a.decay + (int64_t)row * a.ld_decay + h * a.dim;
   for (int i = tid; i < DP; i += nthr) {
     float q = 0.f, k = 0.f, g = 1.f;
     if (i < a.dim) {
-      q = conv(cq + i, own);
-      k = conv(ck + i, own);
-      g = expf(-aexp * softplus_f(to_f32(dec[i]) + a.dt_bias[h * a.dim + i]));
+      if (i != tid) {
+        fetch(tq, cq + i);
+        fetch(tk, ck + i);
+        d0 = dec[i];
+      }
+      q = conv(tq, cq + i, own);
+      k = conv(tk, ck + i, own);
+      g = expf(-aexp * softplus_f(to_f32(d0) + (i == tid ? dt0 : a.dt_bias[h * a.dim + i])));
     }
     qs[i] = q;
     ks[i] = k;
@@ -1191,7 +1249,10 @@ __global__ __launch_bounds__(512) void delta_decode_kernel(DeltaArgs a) {
     sk += k * k;
     dot += q * k;
   }
-  for (int i = tid; i < a.vdim; i += nthr) vs[i] = conv(cv + i, true);
+  for (int i = tid; i < a.vdim; i += nthr) {
+    if (i != tid) fetch(tv, cv + i);
+    vs[i] = conv(tv, cv + i, true);
+  }
   const float beta = sigmoid_f(to_f32(pr[a.off_b + h]));
   const float rq = rsqrtf((float)a.dim) / sqrtf(block_sum(sq, red) + 1e-6f);
   const float rk = 1.f / sqrtf(block_sum(sk, red) + 1e-6f);
@@ -1201,6 +1262,7 @@ __global__ __launch_bounds__(512) void delta_decode_kernel(DeltaArgs a) {
     ks[i] *= rk;
   }
   __syncthreads();
+  if (pos == 0) st.zero();
   float o[CPL], so = 0.f;
 #pragma unroll
   for (int c = 0; c < CPL; ++c) o[c] = 0.f;
@@ -1209,7 +1271,8 @@ __global__ __launch_bounds__(512) void delta_decode_kernel(DeltaArgs a) {
 #pragma unroll
     for (int c = 0; c < CPL; ++c) v[c] = col + c < a.vdim ? vs[col + c] : 0.f;
     st.token(ks, qs, gs, p, beta, qk, v, o);
-    st.store(S, col, p, a.dim, a.vdim);
+    if constexpr (EXACT) st.template move_all<true>(S, col, p, a.vdim);
+    else st.store(S, col, p, a.dim, a.vdim);
 #pragma unroll
     for (int c = 0; c < CPL; ++c)
       if (col + c < a.vdim && p == 0) so += o[c] * o[c];
@@ -1322,7 +1385,13 @@ static int decode_go(const DeltaArgs& a, hipStream_t st) {
   const int waves = (a.vdim + 8 * CPL - 1) / (8 * CPL);
   const size_t lds = sizeof(float) * (size_t)(3 * 8 * DPL + a.vdim);
   if (waves > 8) return -1;
-  delta_decode_kernel<T, DPL, CPL><<<dim3(a.rows, a.H), dim3(64 * waves), lds, st>>>(a);
+  if constexpr (DPL <= 16) {
+    if (a.dim == 8 * DPL && a.vdim == 8 * CPL * waves) {
+      delta_decode_kernel<T, DPL, CPL, true><<<dim3(a.rows, a.H), dim3(64 * waves), lds, st>>>(a);
+      return 0;
+    }
+  }
+  delta_decode_kernel<T, DPL, CPL, false><<<dim3(a.rows, a.H), dim3(64 * waves), lds, st>>>(a);
   return 0;
 }
 template <class T, int DPL>

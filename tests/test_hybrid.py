@@ -330,6 +330,35 @@ CHAIN_CASES = [  # heads, key heads, dim, vdim, lengths in the order of the port
     (16, 4, 128, 256, [34, 33, 35, 17, 32, 31, 20, 34], 1 << 30), (4, 4, 64, 136, [80, 2], 1 << 30)]
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,Hk,d,dv,taps", [(4, 2, 128, 128, 4), (2, 2, 128, 256, 6), (3, 1, 64, 96, 4), (2, 2, 32, 320, 2),
+                                           (2, 1, 72, 72, 5)])
+def test_delta_decode_state_ahead(hipk, dt, H, Hk, d, dv, taps):
+    """States that fill the lanes' tiles and one that does not, more and fewer taps than are fetched ahead,
+    first tokens over a state of NaN, a row without a state; against the plain form on the CPU.  Sums of
+    at most 128 products of about 1: 1e-4 in fp32; in bf16 the output and the inputs' convolutions are rounded."""
+    g = torch.Generator().manual_seed(d + dv)
+    r = lambda *s, std=1.0: torch.randn(*s, generator=g) * std
+    pos = torch.tensor([0, 1, 3, 9, 4, 700], dtype=torch.int32)
+    slot = torch.tensor([2, 0, 5, -1, 1, 3], dtype=torch.int32)
+    B, C = 6, 2 * Hk * d + H * dv
+    proj, decay, gate = r(B, C + 8).to(dt), r(B, H * d).to(dt), r(B, H * dv).to(dt)
+    w = ops.DeltaWeights(r(taps, C, std=0.5), torch.linspace(-1, 1, H).exp(), r(H * d) - 2, 1 + 0.1 * r(dv), 1e-5, H,
+                         Hk, d, dv)
+    ring, state = r(B, taps, C).to(dt), r(B, H, d, dv)
+    state[2] = float("nan")
+    dev = lambda x: x.to("cuda") if torch.is_tensor(x) else x
+    wg = ops.DeltaWeights(*(dev(x) for x in (w.conv, w.a_exp, w.dt_bias, w.norm)), 1e-5, H, Hk, d, dv)
+    rg, sg = dev(ring), dev(state)
+    got = ops.delta_decode(dev(proj), C, wg, rg, sg, dev(decay), dev(gate), dev(pos), dev(slot))
+    want = ops.delta_decode(proj, C, w, ring, state, decay, gate, pos, slot)
+    tol = 1e-4 if dt == torch.float32 else 2e-2
+    assert torch.equal(rg.cpu(), ring)
+    assert ((got.cpu().float() - want.float()).abs() <= tol * (1 + want.float().abs())).all()
+    assert ((sg.cpu() - state).abs() <= tol * (1 + state.abs()))[state.isfinite()].all() and sg.isfinite().all()
+
+
 @on
 @pytest.mark.parametrize("case", CHAIN_CASES, ids=str)
 def test_delta_chains(target, case, monkeypatch):
