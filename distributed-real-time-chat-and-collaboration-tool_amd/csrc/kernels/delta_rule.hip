@@ -1160,7 +1160,8 @@ __global__ __launch_bounds__(256) void delta_read_kernel(DeltaArgs a) {
 
 // Bound by the state, read and written once; everything a token needs besides it is asked for ahead of
 // it, so that the token is prepared while it arrives (memory answers in order).  EXACT: the state fills
-// the lanes' tiles, so no load of it stands behind a condition and the waits can count them.
+// the lanes' tiles, so no load of it stands behind a condition and the waits can count them.  64 sequences x 32 heads of
+// 128 x 128 58.7 -> 53.7 us (5.0 TB/s), 256 x 32 284 -> 223 (4.8).
 constexpr int kDecodeTaps = 4;  // taps whose inputs are fetched ahead; more are read where they are used
 template <class T, int DPL, int CPL, bool EXACT>
 __global__ __launch_bounds__(512) void delta_decode_kernel(DeltaArgs a) {

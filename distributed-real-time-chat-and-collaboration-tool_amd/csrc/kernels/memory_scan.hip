@@ -35,15 +35,25 @@ DRTC_DEVICE float mem_gate(float g, int silu) {
 }
 
 // log gates of a head's token
+struct MemGateIn {  // fixed decay: its logarithm in f
+  float f, i, f_bias, i_bias;
+};
+template <class T>
+DRTC_DEVICE MemGateIn mem_gate_in(const MemoryArgs& a, const T* row, int h) {
+  if (a.log_decay) return MemGateIn{a.log_decay[h], 0.f, 0.f, 0.f};
+  return MemGateIn{to_f32(row[a.off_f + h]), to_f32(row[a.off_i + h]), a.f_bias[h], a.i_bias[h]};
+}
+DRTC_DEVICE void mem_gates(const MemoryArgs& a, const MemGateIn& in, float& f, float& i) {
+  f = in.f;
+  i = 0.f;
+  if (!a.log_decay) {
+    i = a.cap * tanhf((in.i + in.i_bias) / a.cap);
+    f = mem_logsig(a.cap * tanhf((in.f + in.f_bias) / a.cap));
+  }
+}
 template <class T>
 DRTC_DEVICE void mem_gates(const MemoryArgs& a, const T* row, int h, float& f, float& i) {
-  if (a.log_decay) {
-    f = a.log_decay[h];
-    i = 0.f;
-  } else {
-    i = a.cap * tanhf((to_f32(row[a.off_i + h]) + a.i_bias[h]) / a.cap);
-    f = mem_logsig(a.cap * tanhf((to_f32(row[a.off_f + h]) + a.f_bias[h]) / a.cap));
-  }
+  mem_gates(a, mem_gate_in(a, row, h), f, i);
 }
 
 // Element c of a head's query or key, rotated and scaled.
@@ -690,8 +700,10 @@ __global__ __launch_bounds__(64 * NW, 2) void memory_chunk_kernel(MemoryArgs a) 
 
 // ------------------------------------------------------------------ decode
 // V columns to a thread, rows spread over the threads that share them; the first rows' loads are in
-// flight while queries and keys are prepared.
-template <class T, int V>
+// flight while queries and keys are prepared.  Bound by the state, read and written once: 200 sequences x
+// 16 heads of 128 x 128 66 us (6.3 TB/s), 256 x 32 213 (5.0); with the token's inputs asked for behind the
+// state and loads behind conditions 74 and 231.
+template <class T, int V, bool EXACT>
 __global__ __launch_bounds__(256) void memory_decode_kernel(MemoryArgs a) {
   constexpr int U = 16;
   __shared__ float ks[256], qs[256], part[256 * V], os[1024], red[16];
@@ -709,6 +721,33 @@ __global__ __launch_bounds__(256) void memory_decode_kernel(MemoryArgs a) {
   const int cg = (a.vdim + V - 1) / V, nc = min(cg, 256), RG = 256 / nc;
   const int rg = tid / nc, c = tid - rg * nc;
   const bool live = rg < RG;
+  // memory answers in order: what the token needs besides the state is asked for ahead of it, and
+  // prepared while the state arrives
+  const int64_t head = (int64_t)slot * a.H + h;
+  const int i0 = min(tid, a.dim - 1), half = a.rot_dims >> 1;
+  const bool turn = i0 < a.rot_dims;
+  const int pair = !turn ? i0 : i0 < half ? i0 + half : i0 - half, at = min(i0, pair);
+  const T *qp = pr + h * a.dim, *kp = pr + a.off_k + h * a.dim;
+  const T q0 = qp[i0], q1 = qp[pair], k0 = kp[i0], k1 = kp[pair];
+  float cos = 1.f, sin = 0.f;
+  if (a.rot_dims) {
+    const float* cs = a.cos_sin + (int64_t)pos * a.rot_dims;
+    cos = cs[min(at, half - 1)];
+    sin = cs[half + min(at, half - 1)];
+  }
+  const MemGateIn gates = mem_gate_in(a, pr, h);
+  float nv = 0.f, m = 0.f, f, i;
+  if (gated) {
+    m = a.top[head * a.slices];
+    nv = a.nrm[head * a.slices * a.dim + i0];
+  }
+  T v0[V], g0;
+  float w0 = 1.f;
+#pragma unroll
+  for (int v = 0; v < V; ++v) v0[v] = pr[a.off_v + h * a.vdim + min(c * V + v, a.vdim - 1)];
+  g0 = pr[a.off_g + h * a.vdim + min(tid, a.vdim - 1)];
+  if (a.norm_w) w0 = a.norm_w[h * a.vdim + min(tid, a.vdim - 1)];
+  __builtin_amdgcn_sched_barrier(0);
   float s[U][V];
   auto load = [&](int r0, int x) {
 #pragma unroll
@@ -728,20 +767,34 @@ __global__ __launch_bounds__(256) void memory_decode_kernel(MemoryArgs a) {
       }
     }
   };
-  load(rg, c * V);
-  const int64_t head = (int64_t)slot * a.H + h;
-  float nv = 0.f, m = 0.f, f, i;
-  if (gated && pos > 0) {
-    m = a.top[head * a.slices];
-    if (tid < a.dim) nv = a.nrm[head * a.slices * a.dim + tid];
+  // EXACT: the threads' U rows of V columns are the state; one register of addresses, no condition
+  [[maybe_unused]] const __amdgpu_buffer_rsrc_t buf =
+      __builtin_amdgcn_make_buffer_rsrc((void*)S, (short)0, a.dim * a.vdim * 4, 0x00020000);
+  [[maybe_unused]] const int mine = (rg * a.vdim + c * V) * 4, step = RG * a.vdim * 4;
+  if constexpr (EXACT) {
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const f32x4 y = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(buf, mine, i * step, 0));
+#pragma unroll
+      for (int v = 0; v < V; ++v) s[i][v] = y[v];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  } else {
+    load(rg, c * V);
   }
-  mem_gates(a, pr, h, f, i);
+  if (pos == 0) m = nv = 0.f;
+  mem_gates(a, gates, f, i);
   const float mn = fmaxf(f + m, i), da = expf(f + m - mn), db = expf(i - mn);
-  const float* cs = a.rot_dims ? a.cos_sin + (int64_t)pos * a.rot_dims : nullptr;
   float nq = 0.f;
   if (tid < a.dim) {
-    const float q = mem_turned(pr + h * a.dim, tid, cs, a.rot_dims, a.q_scale);
-    const float k = mem_turned(pr + a.off_k + h * a.dim, tid, cs, a.rot_dims, a.k_scale);
+    float q = to_f32(q0), k = to_f32(k0);
+    if (turn) {
+      const float sn = i0 < half ? -sin : sin;
+      q = q * cos + to_f32(q1) * sn;
+      k = k * cos + to_f32(k1) * sn;
+    }
+    q *= a.q_scale;
+    k *= a.k_scale;
     qs[tid] = q;
     ks[tid] = k;
     nv = da * nv + db * k;
@@ -756,15 +809,34 @@ __global__ __launch_bounds__(256) void memory_decode_kernel(MemoryArgs a) {
     if (tid < a.slices) a.top[head * a.slices + tid] = mn;
   }
   __syncthreads();
-  for (int cb = 0; cb < cg; cb += nc) {
+  for (int cb = 0; cb < (EXACT ? 1 : cg); cb += nc) {
     const int x = (cb + c) * V;
     float u[V], o[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) {
       o[v] = 0.f;
-      u[v] = x + v < a.vdim ? db * to_f32(pr[a.off_v + h * a.vdim + x + v]) : 0.f;
+      u[v] = x + v < a.vdim ? db * to_f32(cb == 0 ? v0[v] : pr[a.off_v + h * a.vdim + x + v]) : 0.f;
     }
-    for (int r0 = rg; r0 < a.dim; r0 += RG * U) {
+    if constexpr (EXACT) {
+      if (pos == 0) {
+#pragma unroll
+        for (int j = 0; j < U; ++j)
+#pragma unroll
+          for (int v = 0; v < V; ++v) s[j][v] = 0.f;
+      }
+#pragma unroll
+      for (int j = 0; j < U; ++j) {
+        const float k = ks[rg + j * RG], q = qs[rg + j * RG];
+        f32x4 y;
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          y[v] = s[j][v] * da + k * u[v];
+          o[v] += q * y[v];
+        }
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, y), buf, mine, j * step, 0);
+        __builtin_amdgcn_sched_barrier(0);  // a row at a time: few registers
+      }
+    } else for (int r0 = rg; r0 < a.dim; r0 += RG * U) {
       if (cb > 0 || r0 > rg) load(r0, x);
 #pragma unroll
       for (int j = 0; j < U; ++j) {
@@ -798,9 +870,11 @@ __global__ __launch_bounds__(256) void memory_decode_kernel(MemoryArgs a) {
   float so = 0.f;
   for (int x = tid; x < a.vdim; x += 256) so += os[x] * os[x];
   const float r = 1.f / sqrtf(block_sum(so, red) / (float)a.vdim + a.eps);
-  for (int x = tid; x < a.vdim; x += 256)
-    out[x] = from_f32<T>(os[x] * r * (a.norm_w ? a.norm_w[h * a.vdim + x] : 1.f) *
-                         mem_gate<T>(to_f32(pr[a.off_g + h * a.vdim + x]), a.silu));
+  for (int x = tid; x < a.vdim; x += 256) {
+    const bool first = x == tid;  // its gate and weight are here
+    out[x] = from_f32<T>(os[x] * r * (first ? w0 : a.norm_w ? a.norm_w[h * a.vdim + x] : 1.f) *
+                         mem_gate<T>(to_f32(first ? g0 : pr[a.off_g + h * a.vdim + x]), a.silu));
+  }
 }
 
 // Norm and gate of read-outs that several workgroups left in `out`: one (portion, head) each.
@@ -895,12 +969,16 @@ int launch_memory_decode(int f32, const MemoryArgs& a, hipStream_t st) {
   if (mem_check(a)) return -1;
   const dim3 grid(a.rows, a.H), blk(256);
   const bool vec = a.vdim % 4 == 0;
+  // 16 rows of 4 columns to a thread are the whole state
+  const bool exact = vec && a.vdim <= 256 && 256 % (a.vdim / 4) == 0 && a.dim == 16 * (256 / (a.vdim / 4));
   if (f32) {
-    if (vec) memory_decode_kernel<float, 4><<<grid, blk, 0, st>>>(a);
-    else memory_decode_kernel<float, 1><<<grid, blk, 0, st>>>(a);
+    if (exact) memory_decode_kernel<float, 4, true><<<grid, blk, 0, st>>>(a);
+    else if (vec) memory_decode_kernel<float, 4, false><<<grid, blk, 0, st>>>(a);
+    else memory_decode_kernel<float, 1, false><<<grid, blk, 0, st>>>(a);
   } else {
-    if (vec) memory_decode_kernel<bf16_t, 4><<<grid, blk, 0, st>>>(a);
-    else memory_decode_kernel<bf16_t, 1><<<grid, blk, 0, st>>>(a);
+    if (exact) memory_decode_kernel<bf16_t, 4, true><<<grid, blk, 0, st>>>(a);
+    else if (vec) memory_decode_kernel<bf16_t, 4, false><<<grid, blk, 0, st>>>(a);
+    else memory_decode_kernel<bf16_t, 1, false><<<grid, blk, 0, st>>>(a);
   }
   return (int)hipGetLastError();
 }

@@ -2,6 +2,8 @@
 (portions, decoded tokens, reused slots, far keys), the layer norm behind a token's side input, head
 gates and shared latents of latent attention, squared-relu experts added to the stream.  On the CPU
 (fp32 op references) and, marked gpu, on the HIP kernels in fp32 and bf16."""
+import dataclasses
+
 import numpy as np
 import pytest
 import torch
@@ -166,6 +168,34 @@ def same_state(states, slot, want, t):
         for c in range(states[1].shape[2]):
             close(states[1][slot, :, c], want[1], t)
             close(states[2][slot, :, c], want[2], min(t, 1e-3))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("kind", ["retention", "memory"])
+@pytest.mark.parametrize("shape", [(2, 128, 128, 128), (2, 64, 256, 32), (1, 256, 64, 0), (2, 128, 124, 64)], ids=str)
+def test_memory_decode_state_ahead(kind, shape, dt):
+    """States that are exactly the threads' rows, and one that is not: first tokens over a state of NaN,
+    later ones, a row without a state; against the plain form on the CPU (fp32 sums; in bf16 the output
+    is rounded)."""
+    proj, w, _, fresh = memory("cpu", dt, kind, shape, 6)
+    dev = lambda x: None if x is None else x.to("cuda")
+    wg = dataclasses.replace(w, **{f.name: dev(getattr(w, f.name)) for f in dataclasses.fields(w)
+                                   if torch.is_tensor(getattr(w, f.name))})
+    states = fresh(6, 0.5)
+    for s in states:
+        if s is not None:
+            s[2] = float("nan")
+    on_gpu = [dev(s) for s in states]
+    pos, slot = i32([0, 1, 3, 9, 4, 300], "cpu"), i32([2, 0, 5, -1, 1, 3], "cpu")
+    H, _, dv, _ = shape
+    want, got = (torch.full((6, H * dv), 7.0, dtype=dt, device=d) for d in ("cpu", "cuda"))
+    ops.memory_decode(proj, w, states, pos, slot, want)
+    ops.memory_decode(dev(proj), wg, on_gpu, dev(pos), dev(slot), got)
+    close(got, want.double(), tol(dt, 1e-4, 3e-2))
+    for a, b in zip(on_gpu, states):
+        if b is not None:
+            close(a, b.double(), 1e-4)
 
 
 @on
