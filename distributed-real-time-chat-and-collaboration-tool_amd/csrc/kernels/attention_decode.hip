@@ -153,6 +153,32 @@ DRTC_DEVICE void rope_frags(bf16x8* f, const float* __restrict__ cos_sin, int po
   }
 }
 
+// the same from cos | sin held in registers
+template <int D>
+struct RopeRegs {
+  f32x4 c[D / 64][2], s[D / 64][2];
+  DRTC_DEVICE void load(const float* __restrict__ cos_sin, int pos, int g) {
+    const float* cs = cos_sin + (int64_t)pos * D + 8 * g;
+#pragma unroll
+    for (int i = 0; i < D / 64; ++i)
+#pragma unroll
+      for (int z = 0; z < 2; ++z) {
+        c[i][z] = *reinterpret_cast<const f32x4*>(cs + 32 * i + 4 * z);
+        s[i][z] = *reinterpret_cast<const f32x4*>(cs + D / 2 + 32 * i + 4 * z);
+      }
+  }
+  DRTC_DEVICE void turn(bf16x8* f) const {
+#pragma unroll
+    for (int i = 0; i < D / 64; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float a = bf2f(f[i][j]), b = bf2f(f[i + D / 64][j]), cc = c[i][j >> 2][j & 3], sn = s[i][j >> 2][j & 3];
+        f[i][j] = f2bf(a * cc - b * sn);
+        f[i + D / 64][j] = f2bf(b * cc + a * sn);
+      }
+  }
+};
+
 DRTC_DEVICE void store_part(float* p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -162,9 +188,10 @@ DRTC_DEVICE float load_part(const float* p) {
 // ROPE (decode batches too small for the persistent kernel): q, k and v of the step's token come
 // unrotated, as there; wave 0 of the last partition opens its softmax with that token and writes its
 // rows, the cache is read up to the token ahead of it.  Bound by its chain of round trips (table,
-// K / V, partials, count, merge), not by bytes, until a batch fills the chip: one sequence of 266 tokens
-// 9.9 us, 16 of 1000 20.6 us for 65 MB (rope_kv + a wave per partition + reduce: 19.1 and 26.4), 128 of
-// 1000 98 us (5.4 TB/s; rope_kv + this without ROPE 105).
+// K / V, partials, count, merge), not by bytes, until a batch fills the chip: one sequence of 2000 tokens
+// 11.3 us, 16 of 1000 19.9 us for 65 MB (rope_kv + a wave per partition + reduce: 21.9 and 26.4), 128 of
+// 1000 100 us (5.2 TB/s; rope_kv + this without ROPE 105).  cos | sin and the token's rows asked for
+// behind the first block: 200 of 400 75.8 us, now 71.5.
 template <int D, bool ROPE>
 __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_kernel(
     bf16_t* __restrict__ out, float* __restrict__ part_o,
@@ -197,6 +224,21 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_kernel(
     if (col < G) qf[s] = load_bf16x8(qrow + 32 * s + 8 * g);
     else for (int j = 0; j < 8; ++j) qf[s][j] = f2bf(0.f);
   }
+  // the step's own k and v rows (wave 0: it takes the token, if this is the last partition)
+  [[maybe_unused]] bf16x8 kf[ROPE ? KS : 1];
+  [[maybe_unused]] bf16x4 vf[ROPE ? NT : 1];
+  [[maybe_unused]] bf16_t vw[ROPE ? D / 64 : 1];
+  if constexpr (ROPE) {
+    if (w == 0) {
+      const bf16_t* kn = q + (int64_t)b * q_stride + (int64_t)(Hq + h) * D;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) kf[s] = load_bf16x8(kn + 32 * s + 8 * g);
+#pragma unroll
+      for (int i = 0; i < NT; ++i) vf[i] = load_bf16x4(kn + (int64_t)Hkv * D + 16 * i + 4 * g);
+#pragma unroll
+      for (int i = 0; i < D / 64; ++i) vw[i] = kn[(int64_t)Hkv * D + 64 * i + lane];
+    }
+  }
   const int ctx = context_lens[b];
   const int nc = ROPE ? ctx - 1 : ctx;  // tokens read from the cache
   const int pos = ROPE ? rope.positions[b] : 0;
@@ -226,6 +268,12 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_kernel(
     if constexpr (ROPE) load_kv_block_n<D>(r, kb, vb, lane, nc - blk * kBS);
     else load_kv_block<D>(r, kb, vb, lane);
   };
+  // cos | sin ahead of the cache: memory answers in order, q and k turn while the block arrives
+  [[maybe_unused]] RopeRegs<D> cs;
+  if constexpr (ROPE) {
+    cs.load(rope.cos_sin, pos, g);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   KVRegs<D> cur, nxt;
   int blk = blk_begin + w;
   int ph_next = ph_b;  // table entry of block blk + 4, loaded one step ahead
@@ -234,14 +282,9 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_kernel(
     load_block(cur, phys, blk);
   }
   if constexpr (ROPE) {
-    rope_frags<D>(qf, rope.cos_sin, pos, g);
+    cs.turn(qf);
     if (w == 0 && p == nparts - 1) {
-      const bf16_t* kn = q + (int64_t)b * q_stride + (int64_t)(Hq + h) * D;
-      const bf16_t* vn = kn + (int64_t)Hkv * D;
-      bf16x8 kf[KS];
-#pragma unroll
-      for (int s = 0; s < KS; ++s) kf[s] = load_bf16x8(kn + 32 * s + 8 * g);
-      rope_frags<D>(kf, rope.cos_sin, pos, g);
+      cs.turn(kf);
       float dot = 0.f;
 #pragma unroll
       for (int s = 0; s < KS; ++s)
@@ -258,15 +301,13 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_kernel(
         for (int s = 0; s < KS; ++s) store_bf16x8(kd + 32 * s, kf[s]);
       }
 #pragma unroll
-      for (int i = 0; i < NT; ++i) {
-        const bf16x4 v = load_bf16x4(vn + 16 * i + 4 * g);
+      for (int i = 0; i < NT; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[i][r] = bf2f(v[r]);
-      }
+        for (int r = 0; r < 4; ++r) o[i][r] = bf2f(vf[i][r]);
       if (slot >= 0) {  // V block [8 groups of 4 tokens][D][4]
         bf16_t* vd = rope.v_cache + (cblk * Hkv + h) * blk_elems + (off >> 2) * (4 * D) + (off & 3);
 #pragma unroll
-        for (int d = lane; d < D; d += 64) vd[d * 4] = vn[d];
+        for (int i = 0; i < D / 64; ++i) vd[(64 * i + lane) * 4] = vw[i];
       }
     }
   }

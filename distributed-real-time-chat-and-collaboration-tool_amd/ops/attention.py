@@ -256,9 +256,9 @@ def fused_rope_variant(variant: int, D: int, max_parts: int) -> int:
     launch, or 0.  3 stays itself; 1 runs the shapes of 1 and 2: a workgroup per partition, so 8
     blocks are 2 per wave, and one launch instead of rope_kv, attention and decode_reduce.  Its merge
     holds up to 128 partitions.  32 heads of 128 over 8 kv heads, three launches against one:
-    1 x 266 tokens 19.1 -> 9.9 us, 1 x 16000 43.7 -> 27.0, 1 x 64000 95 -> 68, 8 x 4000 42.7 -> 31.8,
-    16 x 1000 26.4 -> 20.6; two launches (one partition) against one: 40 x 1000 47.2 -> 42.6,
-    64 x 300 23.2 -> 21.1, 128 x 1000 105 -> 98, 200 x 400 74.0 -> 74.5."""
+    1 x 2000 tokens 21.9 -> 11.3 us, 1 x 16000 43.7 -> 27.0, 1 x 64000 95 -> 68, 8 x 4000 42.7 -> 31.8,
+    16 x 1000 26.4 -> 19.9; two launches (one partition) against one: 40 x 1000 47.2 -> 41.8,
+    64 x 300 23.2 -> 20.6, 128 x 1000 105 -> 100, 200 x 400 74.0 -> 71.5."""
     if D not in (64, 128) or DECODE_VARIANT == 2:
         return 0
     return 3 if variant == 3 else 1 if max_parts <= (128 if FUSED_SPLIT_MERGE else 1) else 0
