@@ -495,6 +495,48 @@ def _nucleus_mask(logits, temp, top_p):
     return keep
 
 
+@pytest.mark.parametrize("k", [1, 2, 63, 64, 65, 100, 127, 128, 129])
+@pytest.mark.parametrize("ties", [False, True])
+def test_sample_topk_tokens(hipk, k, ties):
+    """The very token of the draw (the counter-based uniform over the kept candidates' cumulative weights in
+    64 bits), with one, two and more candidates to a lane and ties at and around the k-th value.
+    Draws closer to a boundary than the rounding of the 32-bit sums (128 terms) are left out."""
+    B, V, seed, step = 64, 1500, 7, 11
+    g = torch.Generator().manual_seed(k)
+    lg = (torch.randn(B, V, generator=g) * (1 if ties else 3)).to(torch.bfloat16)
+    if ties:
+        lg = ((lg.float() * 20).round() / 20).to(torch.bfloat16)
+    temp = torch.linspace(0.3, 1.5, B)
+    top_p = torch.where(torch.arange(B) % 3 == 0, 1.0, 0.2 + 0.7 * torch.rand(B, generator=g))
+    got = ops.sample(lg.to(DEV), temp.to(DEV), torch.full((B,), k, dtype=torch.int32, device=DEV), top_p.to(DEV),
+                     seed=seed, step=torch.tensor([step], device=DEV)).cpu()
+    M = (1 << 64) - 1
+
+    def mix(x):
+        for c in (0xff51afd7ed558ccd, 0xc4ceb9fe1a85ec53):
+            x = ((x ^ x >> 33) * c) & M
+        return x ^ x >> 33
+
+    checked = 0
+    for b in range(B):
+        row = lg[b].double()
+        kept = torch.nonzero(row >= row.topk(k).values[-1]).flatten().tolist()
+        if len(kept) > 1024:
+            continue
+        kept.sort(key=lambda i: (-float(row[i]), i))
+        w = ((row[kept] - row.max()) / float(temp[b])).exp().cumsum(0)
+        need = (float(top_p[b]) if top_p[b] < 1 else 1.0) * w[-1]
+        cut = min(int((w < need).sum()), len(kept) - 1)
+        u = float(torch.tensor((mix(seed ^ mix((step * 0x9E3779B97F4A7C15 + b) & M)) >> 40) + 0.5).float()) / 2 ** 24
+        at = int((w <= u * w[cut]).sum())
+        near = 1e-4 * w[-1]
+        if (w - need).abs().min() < near and top_p[b] < 1 or (w - u * w[cut]).abs().min() < near:
+            continue
+        checked += 1
+        assert int(got[b]) == kept[min(at, cut)], (b, len(kept))
+    assert checked >= B // 2
+
+
 def test_sample_top_p_full_vocab_exact(hipk):
     """top_k = 0: every draw lies in the exact nucleus of the full 128k vocab,
     and most draws are ranked below 1024 (nothing is truncated to a candidate
