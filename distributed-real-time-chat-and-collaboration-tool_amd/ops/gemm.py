@@ -5,7 +5,7 @@ shape (M, N, K, row stride of x) ONCE to a route, cached per shape (``route``):
 
   kind      kernel                                          taken for
   "w4"      gemm_w4.hip: 4-wave hand-scheduled MFMA GEMM,   prefill-sized passes (M >= W4_MIN_M,
-            persistent, 256 x 256 tiles (``mfma_gemm``)     K <= W4_MAX_K)
+            persistent, 256 x 256 tiles (``mfma_gemm``)     K <= W4_MAX_K or ``_w4_long``)
   "skinny"  gemv.hip weight-streaming kernels (M <= 16)     decode buckets where the table (or
                                                             ``skinny_variant`` untuned) says so
             gemm_stream.hip (variant STREAM, M <= 64)       where ``stream_ok`` says so
@@ -222,7 +222,9 @@ def _resolve(M: int, N: int, K: int, ldx: int) -> tuple[str, int]:
                 return ("xd", 141)
             return ("w4", 0)
         a = _prefill_algo(M, N, K, ldx, 0)
-        return ("lt", a) if a >= 0 else ("torch", 0)
+        if a >= 0:
+            return ("lt", a)
+        return ("w4", 0) if _w4_long(M, N, K) else ("torch", 0)
     if ldx % 8 == 0 and stream_ok(M, N, K):
         return ("skinny", STREAM)
     found = _decode_entry(M, N, K, ldx)
@@ -818,6 +820,17 @@ def w4_shape_ok(M: int, N: int, K: int) -> bool:
     """Shapes the prefill-sized hand GEMM takes (tensor strides / alignment aside)."""
     return (_w4_plain and _enabled and M >= W4_MIN_M and K <= W4_MAX_K and K % 64 == 0
             and N % 256 == 0)
+
+
+def _w4_long(M: int, N: int, K: int) -> bool:
+    """Whether gemm_w4 takes a K above W4_MAX_K that no tuned library solution covers: where its last
+    round of tiles leaves at most three tenths of the CUs idle on average.  4096 x 11264, us, the library's
+    own choice / gemm_w4: 6400 rows 672 / 489, 8960 912 / 682, 11520 1035 / 726, 14080 1105 / 965, 14848
+    1240 / 968, 16384 957 / 969, 7680 456 / 486; below the line, 5120 rows (0.62) 353 / 502."""
+    if not (_w4_plain and _enabled and M >= W4_MIN_M and K % 64 == 0 and N % 256 == 0):
+        return False
+    tiles = -(-M // 256) * (N // 256)
+    return tiles >= 0.7 * 256 * -(-tiles // 256)
 
 
 def w4_ok(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor | None = None) -> bool:

@@ -184,3 +184,19 @@ def test_gated_default_form(hipk, M, I, K, act):
     else:
         want = (torch.nn.functional.silu(a) if act == "silu" else torch.nn.functional.gelu(a, approximate="tanh")) * b
     assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,kind", [(5800, 2048, 8256, "w4"), (6144, 2048, 11264, "w4"), (4608, 4096, 8320, "torch"),
+                                        (4096, 512, 8256, "torch")])
+def test_long_k_prefill_route(hipk, M, N, K, kind):
+    """K above the limit of the measured shapes, without a tuned solution: gemm_w4 where its rounds of tiles are
+    full enough.  Rows against 64 bits: bf16 rounding of the result and fp32 sums of K products."""
+    G.reset()
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+    w = (torch.randn(N, K, device="cuda", generator=g) / K ** 0.5).to(torch.bfloat16)
+    assert G.route(M, N, K, K)[0] == kind
+    rows = torch.tensor([0, 255, 256, M // 2, M - 1], device="cuda")
+    want = x[rows].double() @ w.double().t()
+    assert ((ops.linear(x, w)[rows].double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-3).all()
