@@ -823,14 +823,17 @@ def w4_shape_ok(M: int, N: int, K: int) -> bool:
 
 
 def _w4_long(M: int, N: int, K: int) -> bool:
-    """Whether gemm_w4 takes a K above W4_MAX_K that no tuned library solution covers: where its last
-    round of tiles leaves at most three tenths of the CUs idle on average.  4096 x 11264, us, the library's
-    own choice / gemm_w4: 6400 rows 672 / 489, 8960 912 / 682, 11520 1035 / 726, 14080 1105 / 965, 14848
-    1240 / 968, 16384 957 / 969, 7680 456 / 486; below the line, 5120 rows (0.62) 353 / 502."""
-    if not (_w4_plain and _enabled and M >= W4_MIN_M and K % 64 == 0 and N % 256 == 0):
+    """Whether gemm_w4 takes a K above W4_MAX_K that no tuned library solution covers: from 4096 columns,
+    where the last round of tiles is a part of one and leaves at most three tenths of the CUs idle on average.
+    The library's own choice / gemm_w4, us: 4096 x 11264, 6400 rows 678 / 480, 11520 1044 / 718, 14848 1187 / 956,
+    7680 449 / 481; 4096 x 14336, 7680 rows 1012 / 615, 13000 1245 / 1122; 4096 x 18432, 8960 rows 1414 / 1143,
+    13000 1577 / 1620, 15616 1970 / 1684.  Below the line, 5120 x 4096 x 11264 (0.62): 353 / 502; whole rounds,
+    16384 rows, K 11264 963 / 985, 14336 1194 / 1240, 18432 1558 / 1736; 2048 columns, K 9216, 6400 rows 177 / 210,
+    13000 363 / 400."""
+    if not (_w4_plain and _enabled and M >= W4_MIN_M and K % 64 == 0 and N % 256 == 0 and N >= 4096):
         return False
     tiles = -(-M // 256) * (N // 256)
-    return tiles >= 0.7 * 256 * -(-tiles // 256)
+    return tiles % 256 != 0 and tiles >= 0.7 * 256 * -(-tiles // 256)
 
 
 def w4_ok(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor | None = None) -> bool:

@@ -187,11 +187,11 @@ def test_gated_default_form(hipk, M, I, K, act):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K,kind", [(5800, 2048, 8256, "w4"), (6144, 2048, 11264, "w4"), (4608, 4096, 8320, "torch"),
-                                        (4096, 512, 8256, "torch")])
+@pytest.mark.parametrize("M,N,K,kind", [(5889, 4096, 8256, "w4"), (7168, 4096, 11264, "w4"), (4608, 4096, 8320, "torch"),
+                                        (4096, 4096, 8256, "torch"), (6144, 2048, 11264, "torch")])
 def test_long_k_prefill_route(hipk, M, N, K, kind):
-    """K above the limit of the measured shapes, without a tuned solution: gemm_w4 where its rounds of tiles are
-    full enough.  Rows against 64 bits: bf16 rounding of the result and fp32 sums of K products."""
+    """K above the limit of the measured shapes, without a tuned solution: gemm_w4 where its last round of tiles
+    is a part of one and full enough (4608: not; 4096: whole), from 4096 columns.  Rows against 64 bits: bf16 rounding of the result and fp32 sums of K products."""
     G.reset()
     g = torch.Generator(device="cuda").manual_seed(M)
     x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
