@@ -248,7 +248,8 @@ __global__ __launch_bounds__(NT) void moe_plan_kernel(const L* __restrict__ logi
     p.local_range[0] = off[p.e_off];
     p.local_range[1] = off[p.e_off + p.e_local];
   }
-  if (p.grp_off != nullptr && t <= p.e_local) p.grp_off[t] = off[p.e_off + t];
+  if (p.grp_off != nullptr)  // one more than the experts: 257 at most
+    for (int i = t; i <= p.e_local; i += NT) p.grp_off[i] = off[p.e_off + i];
   for (int e = t; e < E; e += NT) {
     const int c = off[e + 1] - off[e], nt = toff[e + 1] - toff[e];
     for (int i = 0; i < nt && toff[e] + i < p.max_tiles; ++i) {

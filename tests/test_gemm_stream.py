@@ -165,6 +165,27 @@ def test_routing_plan(hipk, T, E, k, groups, keep):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,E,e_off", [(64, 256, 0), (256, 256, 0), (200, 255, 0), (300, 256, 0), (256, 256, 128)])
+def test_routing_plan_group_offsets(hipk, T, E, e_off):
+    """As many experts as threads: the end of the last expert's rows, which the grouped GEMM reads, over a
+    workspace of other bytes; hidden rows and outputs rounded to bf16 as in test_streamed_experts."""
+    H, I, k = 256, 128, 4
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn(T, H, device="cuda", generator=g).to(torch.bfloat16)
+    lg = torch.randn(T, E, device="cuda", generator=g)
+    lg[::3, E - 1] = 9.0
+    lg[::7, e_off] = 8.0
+    w_in = (torch.randn(E - e_off, 2 * I, H, device="cuda", generator=g) * 0.05).to(torch.bfloat16)
+    w_out = (torch.randn(E - e_off, H, I, device="cuda", generator=g) * 0.05).to(torch.bfloat16)
+    ws = ops.moe.make_workspace(T, H, I, E - e_off, k, "cuda")
+    want = ops.fused_moe_ref(x, lg, w_in, w_out, k, "silu", e_off).double()
+    for fill in (0xff, 0x00, 0x01):
+        ws.fill_(fill)
+        y = ops.fused_moe(x, lg, w_in, w_out, k, "silu", E, e_off, ws, variant=4).double()
+        assert (y - want).norm() <= 4e-3 * want.norm()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,I,K,act", [(17, 8192, 2048, "silu"), (33, 14336, 1024, "gelu_tanh"), (127, 10240, 4096, "silu"),
                                        (129, 3584, 4096, "silu"), (257, 7168, 1024, "clamped"), (511, 5632, 512, "silu"),
                                        (700, 1792, 2048, "silu"), (130, 28672, 512, "gelu_tanh")])
