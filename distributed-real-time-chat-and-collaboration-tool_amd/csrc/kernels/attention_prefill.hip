@@ -449,7 +449,7 @@ template <int D, int GH, bool PERSIST>
 __global__ __launch_bounds__(128 * GH, 2) void prefill_attn32_kernel(
     bf16_t* __restrict__ out, int out_stride, const bf16_t* __restrict__ qkv, int qkv_stride, int Hq, int Hkv,
     const int* __restrict__ cu_seqlens, const int* __restrict__ tile_seq, const int* __restrict__ tile_q0, int n_tiles,
-    float scale_log2e, int causal) {
+    float scale, float to_q, int causal) {
   using L = Prefill32<D, GH>;
   constexpr int KS = D / 16, NT = D / 32, VPR = D / 8, NV = kKT * VPR / L::NTHR;
   static_assert(NV >= 1 && (kKT * VPR) % L::NTHR == 0, "staging split");
@@ -457,8 +457,6 @@ __global__ __launch_bounds__(128 * GH, 2) void prefill_attn32_kernel(
   const int G = Hq / Hkv, groups = G / GH, n_hg = Hq / GH, n_work = n_tiles * n_hg;
   const int w = wave_id_uniform(), lane = threadIdx.x & 63;
   const int col = lane & 31, h = lane >> 5;
-  const float scale = fabsf(scale_log2e);
-  const unsigned flip = scale_log2e < 0.f ? 0x80008000u : 0u;  // the sign goes to Q: the largest score stays that
 
   struct Item {
     int s_begin, seqlen, q0, hq, hk, ntiles;
@@ -504,13 +502,11 @@ __global__ __launch_bounds__(128 * GH, 2) void prefill_attn32_kernel(
     }
   };
   auto turn = [&](bf16x8* qf) {
-    if (flip == 0) return;
+    if (to_q == 1.f) return;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      u32x4 t = __builtin_bit_cast(u32x4, qf[s]);
-      t ^= flip;
-      qf[s] = __builtin_bit_cast(bf16x8, t);
-    }
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) qf[s][j] = f2bf(bf2f(qf[s][j]) * to_q);
   };
   const int k_at = col * L::KROW + 8 * h;
   const int v_at = (4 * h + ((lane & 15) >> 2)) * L::VROW + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
@@ -630,6 +626,20 @@ __global__ __launch_bounds__(128 * GH, 2) void prefill_attn32_kernel(
   }
 }
 
+// prefill_attn32_kernel's scale and factor of Q for scores scaled by ``s``.  The kernel masks scores ahead
+// of the scale, which must keep a masked one (kNegBig) out of reach, and takes the largest one ahead of it
+// too: the sign goes to Q, and of scales below 2^-40 (0 as well) the power of two (exact where an element
+// of Q stays above 2^-126).
+static void split_scale(float s, float& scale, float& to_q) {
+  scale = fabsf(s);
+  to_q = 1.f;
+  if (scale < 0x1p-40f) {
+    to_q = scale < 0x1p-126f ? 0.f : ldexpf(1.f, ilogbf(scale));
+    scale = to_q > 0.f ? scale / to_q : 1.f;
+  }
+  if (s < 0.f) to_q = -to_q;
+}
+
 static int prefill_persist_grid(int n_work) {
   static int n_cu = 0;
   if (n_cu == 0) {
@@ -649,6 +659,8 @@ static void launch_tile(dim3 grid, hipStream_t st, bf16_t* out, int out_stride, 
   const int n_work = (int)(grid.x * grid.y);
   if constexpr (prefill32<D, GH>) {
     using L = Prefill32<D, GH>;
+    float scale, to_q;
+    split_scale(sl2, scale, to_q);
     if constexpr (GH == 4) {  // with fewer waves to a workgroup the others of its CU fill its gaps
       if (persist) {
         static int per_cu = 0;
@@ -658,12 +670,12 @@ static void launch_tile(dim3 grid, hipStream_t st, bf16_t* out, int out_stride, 
           per_cu = 1;
         const int n_wg = std::min(n_work, prefill_persist_grid(n_work * per_cu) * per_cu);
         prefill_attn32_kernel<D, GH, true><<<std::max(1, n_wg), L::NTHR, L::BYTES, st>>>(
-            out, out_stride, qkv, qkv_stride, Hq, Hkv, cu, ts, tq, (int)grid.x, sl2, causal);
+            out, out_stride, qkv, qkv_stride, Hq, Hkv, cu, ts, tq, (int)grid.x, scale, to_q, causal);
         return;
       }
     }
     prefill_attn32_kernel<D, GH, false><<<n_work, L::NTHR, L::BYTES, st>>>(
-        out, out_stride, qkv, qkv_stride, Hq, Hkv, cu, ts, tq, (int)grid.x, sl2, causal);
+        out, out_stride, qkv, qkv_stride, Hq, Hkv, cu, ts, tq, (int)grid.x, scale, to_q, causal);
   } else {
     constexpr size_t lds_bytes = PrefillLds<D, GH>::BYTES;
     if (persist) {

@@ -375,6 +375,29 @@ def test_prefill_rows32(hipk, D, Hq, Hkv, causal, sign, persist):
     _close(out, ref, 2e-2, 2e-2, "prefill")
 
 
+@pytest.mark.parametrize("D,Hq,Hkv", [(128, 16, 4), (128, 4, 2), (128, 2, 2), (64, 8, 4), (64, 2, 2), (256, 2, 1)])
+@pytest.mark.parametrize("scale", [0.0, 1e-30, -1e-30, 3e-39])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("persist", [True, False])
+def test_prefill_small_scales(hipk, D, Hq, Hkv, scale, causal, persist):
+    """Scales from 0 on: a masked key has no weight, however small the scale makes the scores.  Every other
+    query and all keys are 2^48 times larger, so that half of the rows see scores of about 1 at 1e-30 and
+    the others an average; tolerance of the tests above."""
+    lens = [1, 33, 64, 65, 200]
+    cu = [sum(lens[:i]) for i in range(len(lens) + 1)]
+    g = torch.Generator().manual_seed(4)
+    qkv = torch.randn(cu[-1], (Hq + 2 * Hkv) * D, generator=g)
+    qkv[::2, :Hq * D] *= 2.0 ** 48
+    qkv[:, Hq * D:(Hq + Hkv) * D] *= 2.0 ** 48
+    qkv = qkv.to(torch.bfloat16).to(DEV)
+    ops.set_prefill_persist(persist)
+    out = ops.prefill_attention(qkv, torch.tensor(cu, dtype=torch.int32, device=DEV), Hq, Hkv, D, scale, causal,
+                                cu_host=cu)
+    ops.set_prefill_persist(None)
+    ref = ops.prefill_attention_ref(qkv.double(), cu, Hq, Hkv, D, scale, causal)
+    _close(out, ref, 2e-2, 2e-2, "prefill")
+
+
 @pytest.mark.parametrize("persist", [True, False])
 def test_prefill_attention_shape_padding_rows_zero(hipk, persist):
     """A shape-padded chunk (T > cu[-1]): the op allocates its output, only the
