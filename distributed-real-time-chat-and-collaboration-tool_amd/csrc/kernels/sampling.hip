@@ -31,6 +31,7 @@
 // `step` lives in device memory so the kernel replays inside a hipGraph.
 // Keys: bf16 bit patterns mapped to unsigned 16-bit keys ordered like the
 // float values, so comparisons on keys are exact comparisons on logits.
+// A NaN or -inf is never drawn; a row of nothing else gets the token -1.
 #include "common.h"
 #include "launchers.h"
 
@@ -44,6 +45,7 @@ constexpr int kMaxRounds = 40;
 DRTC_DEVICE unsigned ord16(unsigned short b) {
   return (b & 0x8000u) ? (unsigned)(~b & 0xFFFFu) : (unsigned)(b | 0x8000u);
 }
+constexpr unsigned kLowKey = 0x80u, kTopKey = 0xff80u;  // keys of the numbers above -inf; NaNs lie on both sides
 DRTC_DEVICE float bits2f(unsigned short b) { return __uint_as_float((unsigned)b << 16); }
 
 DRTC_DEVICE uint64_t mix64(uint64_t x) {
@@ -180,7 +182,7 @@ DRTC_DEVICE void select_bin(SampShared& s, const unsigned* hist, int remaining) 
   __syncthreads();
 }
 
-// Exact key of the k-th largest element by a 16-bit radix select (two
+// Exact key of the k-th largest number by a 16-bit radix select (two
 // histogram passes over the row; per-wave histograms).
 template <int U>
 DRTC_DEVICE unsigned radix_kth(SampShared& s, const unsigned short* lr, int V, bool vec, int k) {
@@ -193,7 +195,7 @@ DRTC_DEVICE unsigned radix_kth(SampShared& s, const unsigned short* lr, int V, b
     unsigned* h = s.hist[wid];
     for_row<U>(lr, V, vec, [&](int, unsigned short b) {
       const unsigned key = ord16(b);
-      if ((key & mask) == prefix) atomicAdd(&h[(key >> pass) & 255u], 1u);
+      if ((key & mask) == prefix && key <= kTopKey) atomicAdd(&h[(key >> pass) & 255u], 1u);
     });
     __syncthreads();
     if (tid < 256) {
@@ -212,7 +214,7 @@ DRTC_DEVICE unsigned radix_kth(SampShared& s, const unsigned short* lr, int V, b
   return prefix;
 }
 
-// Gather every element with key >= thr into s.val / s.idx (ballot-compacted);
+// Gather every number with key >= thr into s.val / s.idx (ballot-compacted);
 // returns the number found (may exceed kCand: only the first kCand are kept).
 template <int U>
 DRTC_DEVICE int gather_ge(SampShared& s, const unsigned short* lr, int V, bool vec, unsigned thr) {
@@ -234,6 +236,7 @@ DRTC_DEVICE int gather_ge(SampShared& s, const unsigned short* lr, int V, bool v
       if (slot < kCand) { s.val[slot] = bits2f(b); s.idx[slot] = i; }
     }
   };
+  auto in = [&](unsigned short b) { return ord16(b) - thr <= kTopKey - thr; };
   // wave-uniform trip counts (the ballots need every lane): pad to whole waves
   const int w0 = tid & ~63;
   if (vec) {
@@ -253,7 +256,7 @@ DRTC_DEVICE int gather_ge(SampShared& s, const unsigned short* lr, int V, bool v
         any[u] = false;
         if (v < nv) {
 #pragma unroll
-          for (int j = 0; j < 8; ++j) any[u] |= ord16(x[u][j]) >= thr;
+          for (int j = 0; j < 8; ++j) any[u] |= in(x[u][j]);
         }
       }
 #pragma unroll
@@ -261,19 +264,19 @@ DRTC_DEVICE int gather_ge(SampShared& s, const unsigned short* lr, int V, bool v
         if (__ballot(any[u]) == 0) continue;  // wave-uniform
         const int v = v0 + u * kSampThreads + lane;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) put(v < nv && ord16(x[u][j]) >= thr, 8 * v + j, x[u][j]);
+        for (int j = 0; j < 8; ++j) put(v < nv && in(x[u][j]), 8 * v + j, x[u][j]);
       }
     }
     for (int i0 = (nv << 3) + w0; i0 < V; i0 += kSampThreads) {
       const int i = i0 + lane;
       const unsigned short b = i < V ? lr[i] : (unsigned short)0;
-      put(i < V && ord16(b) >= thr, i, b);
+      put(i < V && in(b), i, b);
     }
   } else {
     for (int i0 = w0; i0 < V; i0 += kSampThreads) {
       const int i = i0 + lane;
       const unsigned short b = i < V ? lr[i] : (unsigned short)0;
-      put(i < V && ord16(b) >= thr, i, b);
+      put(i < V && in(b), i, b);
     }
   }
   __syncthreads();
@@ -283,8 +286,10 @@ DRTC_DEVICE int gather_ge(SampShared& s, const unsigned short* lr, int V, bool v
 // The rest of sample_topk for up to 128 gathered candidates, n: each finds its place by counting those
 // ahead of it (8 threads to a candidate), then one wave does what is left, two candidates to a lane - the
 // same sums in the same order as the form below with two barriers instead of some fifty.  V 32000, top-k
-// 64, top-p 0.95: 1 row 15.0 -> 11.6 us, 1024 rows 39.7 -> 30.7; V 128256, 1024 rows 78.0 -> 70.4.
+// 64, top-p 0.95: 1 row 15.0 -> 11.2 us, 1024 rows 39.7 -> 31.2; V 128256, 1024 rows 78.0 -> 71.8.
 constexpr int kFew = 128;
+// against the largest: 1 for itself, at +inf too
+DRTC_DEVICE float weight(float v, float top, float inv_t) { return v == top ? 1.f : __expf((v - top) * inv_t); }
 DRTC_DEVICE void sample_few(SampShared& s, int* out_tokens, int row, float temp, int k, int n, float pp,
                             uint64_t seed, uint64_t st) {
   const int tid = threadIdx.x, lane = tid & 63, own = tid >> 3;
@@ -320,7 +325,7 @@ DRTC_DEVICE void sample_few(SampShared& s, int* out_tokens, int row, float temp,
   n = total_n;
   const float top = sv[0], inv_t = 1.f / temp;
 #pragma unroll
-  for (int z = 0; z < 2; ++z) x[z] = lane + 64 * z < n ? __expf((sv[min(lane + 64 * z, n - 1)] - top) * inv_t) : 0.f;
+  for (int z = 0; z < 2; ++z) x[z] = lane + 64 * z < n ? weight(sv[min(lane + 64 * z, n - 1)], top, inv_t) : 0.f;
   // inclusive scan over the next power of two
   for (int off = 1; off < n; off <<= 1) {
     const float a = off < 64 ? __shfl_up(x[0], off, 64) : 0.f, b = off < 64 ? __shfl_up(x[1], off, 64) : 0.f;
@@ -344,11 +349,14 @@ DRTC_DEVICE void sample_few(SampShared& s, int* out_tokens, int row, float temp,
     if (hit) cut = 64 * z + __ffsll((unsigned long long)hit) - 1;
   }
   const float target = uniform(seed, st, row, 0) * __shfl(cut >= 64 ? x[1] : x[0], cut & 63, 64);
+  int at = 0;  // (the first, where a temperature that is no number leaves no weights)
 #pragma unroll
   for (int z = 0; z < 2; ++z) {
     const int i = lane + 64 * z;
-    if (i <= cut && target >= lo[z] && (target < x[z] || i == cut)) out_tokens[row] = si[i];
+    const uint64_t hit = __ballot(i <= cut && target >= lo[z] && (target < x[z] || i == cut));
+    if (hit) at = 64 * z + 63 - __clzll((long long)hit);
   }
+  if (lane == 0) out_tokens[row] = si[at];
 }
 
 template <int U>
@@ -357,8 +365,9 @@ DRTC_DEVICE void sample_topk(SampShared& s, int* out_tokens, const unsigned shor
                              uint64_t st) {
   const int tid = threadIdx.x;
   // ---- pass 1: per-thread max key; tau0 = k-th largest of the thread maxima
-  unsigned tm = 0;
-  for_row<U>(lr, V, vec, [&](int, unsigned short b) { tm = max(tm, ord16(b)); });
+  float most = -INFINITY;  // (of floats: NaNs drop out, and +0 is above -0 as in the keys)
+  for_row<U>(lr, V, vec, [&](int, unsigned short b) { most = fmaxf(most, bits2f(b)); });
+  const unsigned tm = ord16((unsigned short)(__float_as_uint(most) >> 16));
   unsigned* h = &s.hist[0][0];
   h[tid] = tm;  // hist doubles as a 1024-key buffer here
   __syncthreads();
@@ -378,7 +387,8 @@ DRTC_DEVICE void sample_topk(SampShared& s, int* out_tokens, const unsigned shor
     remaining = s.misc[1];
     __syncthreads();
   }
-  // ---- gather key >= tau0 (>= k elements by construction).  Such an element
+  prefix = max(prefix, kLowKey);
+  // ---- gather key >= tau0 (>= k elements by construction, or all numbers).  Such an element
   // can only sit in a thread whose own max is >= tau0, so only those threads
   // (about k of the 1024) re-read their own elements: no second row pass.
   if (tid == 0) s.misc[2] = 0;
@@ -387,7 +397,7 @@ DRTC_DEVICE void sample_topk(SampShared& s, int* out_tokens, const unsigned shor
   __syncthreads();
   if (tm >= prefix) {
     for_row<U>(lr, V, vec, [&](int i, unsigned short b) {
-      if (ord16(b) >= prefix) {
+      if (ord16(b) - prefix <= kTopKey - prefix) {  // key in [prefix, kTopKey]
         const int slot = atomicAdd(&s.misc[2], 1);
         if (slot < kCand) { s.val[slot] = bits2f(b); s.idx[slot] = i; }
       }
@@ -398,6 +408,10 @@ DRTC_DEVICE void sample_topk(SampShared& s, int* out_tokens, const unsigned shor
   if (n > kCand) {  // heavy ties: exact k-th key by radix select, gather again
     const unsigned thr = radix_kth<U>(s, lr, V, vec, k);
     n = min(gather_ge<U>(s, lr, V, vec, thr), kCand);
+  }
+  if (n == 0) {
+    if (tid == 0) out_tokens[row] = -1;
+    return;
   }
   if (n <= kFew) {
     sample_few(s, out_tokens, row, temp, k, n, pp, seed, st);
@@ -435,7 +449,7 @@ DRTC_DEVICE void sample_topk(SampShared& s, int* out_tokens, const unsigned shor
   // ---- softmax + top-p + draw over the n candidates
   const float top = s.val[0];
   const float inv_t = 1.f / temp;
-  const float pv = (tid < n) ? __expf((s.val[tid] - top) * inv_t) : 0.f;
+  const float pv = (tid < n) ? weight(s.val[tid], top, inv_t) : 0.f;
   __syncthreads();
   s.val[tid] = pv;
   __syncthreads();
@@ -446,7 +460,10 @@ DRTC_DEVICE void sample_topk(SampShared& s, int* out_tokens, const unsigned shor
     __syncthreads();
   }
   const float total = s.val[n - 1];
-  if (tid == 0) s.misc[3] = n - 1;
+  if (tid == 0) {
+    s.misc[3] = n - 1;
+    s.misc[0] = 0;  // (the first, where a temperature that is no number leaves no weights)
+  }
   __syncthreads();
   {
     const float need = pp * total;
@@ -458,8 +475,10 @@ DRTC_DEVICE void sample_topk(SampShared& s, int* out_tokens, const unsigned shor
   const float target = uniform(seed, st, row, 0) * s.val[cut];
   if (tid <= cut) {
     const float lo = (tid == 0) ? 0.f : s.val[tid - 1];
-    if (target >= lo && (target < s.val[tid] || tid == cut)) out_tokens[row] = s.idx[tid];
+    if (target >= lo && (target < s.val[tid] || tid == cut)) s.misc[0] = tid;
   }
+  __syncthreads();
+  if (tid == 0) out_tokens[row] = s.idx[s.misc[0]];
 }
 
 template <int U>
@@ -596,7 +615,7 @@ __global__ __launch_bounds__(kSampThreads, 4 * OCC) void sample_kernel(
     if (tid == 0) {
       for (int w = 1; w < kSampWaves; ++w)
         if (s.val[w] > best || (s.val[w] == best && s.idx[w] < bi)) { best = s.val[w]; bi = s.idx[w]; }
-      out_tokens[row] = bi;
+      out_tokens[row] = bi < V ? bi : -1;
     }
     return;
   }

@@ -71,7 +71,8 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor | None = None,
     """logits [B, V] bf16 -> int32 token ids [B].
 
     temperature/top_k/top_p are per-row device tensors (float32 / int32 /
-    float32); ``step`` is an int64 device scalar the caller advances."""
+    float32); ``step`` is an int64 device scalar the caller advances.  On the GPU a
+    row without a number above -inf gets -1 (``sample_ref`` raises)."""
     if not on_gpu(logits):
         # counter-based like the HIP sampler: the draws are a function of (seed, step), so a
         # step re-run with the same counter (EP capacity redo) draws the same tokens
