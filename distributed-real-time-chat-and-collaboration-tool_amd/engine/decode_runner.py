@@ -33,6 +33,14 @@ from ..models.transformer import DecodeMeta, TransformerLM
 DEFAULT_BUCKETS = ops.gemm.DECODE_BUCKETS
 
 
+def check_tokens(ids: np.ndarray, vocab: int) -> None:
+    """Refuse tokens outside of the vocabulary while they are on the host: on the device a row
+    of such a token is NaN (ops.embed)."""
+    if ids.size and (ids.min() < 0 or ids.max() >= vocab):
+        bad = ids[(ids < 0) | (ids >= vocab)]
+        raise ValueError(f"token {bad[0]} outside of the vocabulary of {vocab}")
+
+
 class DecodeRunner:
     def __init__(self, model: TransformerLM, kv_cache, max_batch: int, max_blocks: int,
                  use_graphs: bool = True, seed: int = 0, buckets=DEFAULT_BUCKETS):
@@ -189,6 +197,8 @@ class DecodeRunner:
         (same slot order: a pipelined step).  Returns a handle for
         :meth:`wait`."""
         Bb = self.bucket(n)
+        if ids is not None:
+            check_tokens(ids[:n], self.model.cfg.vocab_size)
         B, MB = self.max_batch, self.max_blocks
         if self.use_graphs:
             self.capture(Bb)  # before the staging: it clears the device copies

@@ -38,7 +38,7 @@ from .. import ops
 from ..utils import tracing
 from ..utils.metrics import METRICS
 from ..models.transformer import DecodeMeta, PrefillMeta, TransformerLM
-from .decode_runner import DEFAULT_BUCKETS, DecodeRunner
+from .decode_runner import DEFAULT_BUCKETS, DecodeRunner, check_tokens
 from .request import Request, RequestState, SamplingParams
 
 BS = ops.KV_BLOCK
@@ -173,6 +173,7 @@ class LLMEngine:
             raise ValueError(f"prompt of {n} tokens exceeds max_model_len {self.max_model_len}")
         if n > self.max_prefill_tokens and not self.model.portions:
             raise ValueError("prompt exceeds max_prefill_tokens")
+        check_tokens(np.asarray(req.prompt_ids), self.cfg.vocab_size)
         with self.lock:
             req.state = RequestState.WAITING
             self.waiting.append(req)
@@ -590,6 +591,8 @@ class LLMEngine:
         Tp = _pad_tokens(T + Bb) - Bb
         ids = np.zeros(Tp, dtype=np.int32)
         ids[:T] = np.fromiter(itertools.chain.from_iterable(seqs), dtype=np.int32, count=T)
+        check_tokens(ids, self.cfg.vocab_size)
+        check_tokens(dec_ids, self.cfg.vocab_size)
         seq_of = np.repeat(np.arange(nseq), lens_a)
         p_tok = np.arange(T, dtype=np.int64) - np.repeat(cu_a[:-1] - starts, lens_a)
         pos = np.zeros(Tp, dtype=np.int32)

@@ -72,6 +72,39 @@ def test_engine_stop_conditions():
         eng.add_request(__import__("drtc_amd.engine", fromlist=["Request"]).Request([1] * 100))
 
 
+def test_tokens_outside_of_the_vocabulary_are_refused():
+    """By every entry that takes tokens from a caller, before anything runs on them; the engine goes on."""
+    import numpy as np
+    from drtc_amd.engine import Request
+
+    m = TransformerLM(TINY_LLAMA, "cpu", seed=4)
+    V = TINY_LLAMA.vocab_size
+    eng = LLMEngine(m, max_batch=4, max_model_len=64, num_blocks=32, use_graphs=False)
+    want = eng.generate([[1, V - 1, 0]], SamplingParams.greedy(4, ignore_eos=True))[0].output_ids
+    for bad in (V, -1, 1 << 30):
+        with pytest.raises(ValueError):
+            eng.add_request(Request([1, bad, 3]))
+        r = Request([])
+        with pytest.raises(ValueError):
+            eng.feed([(r, [2, bad], [1])])
+        with pytest.raises(ValueError):  # a decode row beside a prompt, and alone
+            eng.feed([(r, [2, 5], []), (Request([]), [bad], [])])
+        eng.release(r)
+        r = Request([])
+        eng.feed([(r, [2, 5], [])])
+        with pytest.raises(ValueError):
+            eng.feed([(r, [bad], [0])])
+        one = np.ones(1, np.int64)
+        with pytest.raises(ValueError):
+            eng.runner.launch(1, one * bad, 0 * one, one, -one, np.zeros((1, eng.max_blocks), np.int64), 0 * one,
+                              0 * one, one)
+        eng.release(r)
+        for x in list(eng.running):
+            eng.release(x)
+    assert eng.generate([[1, V - 1, 0]], SamplingParams.greedy(4, ignore_eos=True))[0].output_ids == want
+    assert eng.alloc.num_used == 0
+
+
 def test_pipelined_decode_matches_synchronous():
     """Pipelined decode (step t+1 enqueued before step t is read, tokens fed
     back on the device) produces exactly the synchronous engine's outputs,
