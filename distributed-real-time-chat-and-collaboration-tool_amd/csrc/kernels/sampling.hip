@@ -641,7 +641,7 @@ __global__ __launch_bounds__(256) void step_begin_kernel(int* __restrict__ ids, 
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i < B) {
     const int64_t s = src[i];
-    ids[i] = s >= 0 && s < B ? sampled[s] : host[i];
+    ids[i] = s < 0 ? host[i] : s < B ? sampled[s] : -1;  // -1: no such row, and no such token
   }
   if (i == 0) {
     const int64_t c = *counter;

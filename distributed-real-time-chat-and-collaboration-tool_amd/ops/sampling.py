@@ -102,7 +102,8 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor | None = None,
 def step_begin(ids: torch.Tensor, src: torch.Tensor, sampled: torch.Tensor, host: torch.Tensor,
                counter: torch.Tensor, position: torch.Tensor) -> None:
     """The tokens a decode step starts from, into ``ids``: ``sampled[src]``, or ``host`` where src is
-    negative (all int32 [B], src int64); then position = counter, counter += 1 (int64 [1])."""
+    negative (all int32 [B], src int64); then position = counter, counter += 1 (int64 [1]).  A src of
+    B or more is an error on the CPU and the token -1 on the GPU."""
     if not on_gpu(ids):
         ids.copy_(torch.where(src >= 0, sampled.index_select(0, src.clamp(min=0)), host))
         position.copy_(counter)

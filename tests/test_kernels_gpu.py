@@ -1125,3 +1125,17 @@ def test_step_begin(hipk, B):
         for a, b in zip(args, (want, src, sampled, host, ctr, at)):
             assert torch.equal(a.cpu(), b)
     assert int(at) == (1 << 40) + 1
+
+
+def test_step_begin_refuses_rows_beyond_the_batch(hipk):
+    """A source row that the last step does not have is no token of the host's."""
+    B = 70
+    src, sampled, host = torch.full((B,), B), torch.ones(B, dtype=torch.int32), torch.full((B,), 2, dtype=torch.int32)
+    src[::3], src[1::3], src[5] = -1, 0, 1 << 40
+    ctr, at, ids = torch.zeros(1).long(), torch.zeros(1).long(), torch.zeros(B, dtype=torch.int32)
+    with pytest.raises(IndexError):
+        ops.step_begin(ids, src, sampled, host, ctr, at)
+    args = [x.to(DEV) for x in (ids, src, sampled, host, ctr, at)]
+    ops.step_begin(*args)
+    want = torch.where(src < 0, 2, torch.where(src == 0, 1, -1))
+    assert torch.equal(args[0].cpu().long(), want)
