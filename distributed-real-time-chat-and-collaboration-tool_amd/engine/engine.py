@@ -44,6 +44,11 @@ from .request import Request, RequestState, SamplingParams
 BS = ops.KV_BLOCK
 
 
+def _check_sampled(toks: np.ndarray) -> None:
+    if (toks < 0).any():  # ops.sample; its CPU form raises by itself
+        raise RuntimeError("no token to draw: a row of logits holds no number above -inf")
+
+
 def _pad_tokens(T: int) -> int:
     """Prefill token-count bucket (< 256 padded rows above 256 tokens)."""
     if T <= 256:
@@ -702,6 +707,7 @@ class LLMEngine:
         """Slot assignment + first-token bookkeeping of one prefill chunk."""
         now = time.perf_counter()
         finished = []
+        _check_sampled(toks[:len(segs)])
         for (r, a, n), tok in zip(segs, toks):
             n += a
             if n < r.num_tokens:
@@ -975,6 +981,7 @@ class LLMEngine:
         toks = st["toks"] if st.get("handle") is None else self.runner.wait(st["handle"])
         n, reqs = st["n"], st["reqs"]
         live = np.fromiter((r.state != RequestState.FINISHED for r in reqs), dtype=bool, count=n)
+        _check_sampled(toks[:n][live])
         for r, tok, ok in zip(reqs, toks.tolist(), live.tolist()):
             if ok:
                 r.output_ids.append(tok)

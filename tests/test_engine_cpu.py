@@ -105,6 +105,27 @@ def test_tokens_outside_of_the_vocabulary_are_refused():
     assert eng.alloc.num_used == 0
 
 
+@pytest.mark.parametrize("call", [0, 2])
+def test_rows_without_a_token_stop_the_engine(monkeypatch, call):
+    """-1 from the sampler, for a prompt and for a decode step: an error, not a token of the output."""
+    m = TransformerLM(TINY_LLAMA, "cpu", seed=4)
+    eng = LLMEngine(m, max_batch=4, max_model_len=64, num_blocks=32, use_graphs=False)
+    eng.pipeline = False
+    real, n = ops.sample, [0]
+
+    def sample(*a, **k):
+        out = real(*a, **k)
+        if n[0] == call:
+            out[1] = -1
+        n[0] += 1
+        return out
+
+    monkeypatch.setattr(ops, "sample", sample)
+    with pytest.raises(RuntimeError, match="no number"):
+        eng.generate([[1, 2, 3], [4, 5]], SamplingParams.greedy(6, ignore_eos=True))
+    assert not any(t < 0 for r in eng.running for t in r.output_ids)
+
+
 def test_pipelined_decode_matches_synchronous():
     """Pipelined decode (step t+1 enqueued before step t is read, tokens fed
     back on the device) produces exactly the synchronous engine's outputs,
