@@ -178,13 +178,17 @@ def _chain_ok(w: DeltaWeights, decay: torch.Tensor, gate: torch.Tensor, p: Porti
             and p.max_len > 32 and p.row_state.numel() * w.heads <= 256 * p.max_len)
 
 
-def _chain_workspace(w: DeltaWeights, rows: int, n: int, dev) -> tuple[torch.Tensor, torch.Tensor]:
-    """(operands, outputs ahead of the norm) of delta_chain (delta_rule.hip: ChainEntry)."""
+def _chain_workspace(w: DeltaWeights, rows: int, n: int, dev) -> tuple[torch.Tensor, torch.Tensor] | None:
+    """(operands, outputs ahead of the norm) of delta_chain (delta_rule.hip: ChainEntry).  None where
+    memory does not hold them: the one-launch form needs none."""
     chunks, tiles = rows // 16 + n, 2 if w.dim <= 32 else 4 if w.dim <= 64 else 8
     head = chunks * (768 * tiles + 16 * tiles + 512)
     heads = min(w.heads, max(1, CHAIN_BYTES // (4 * head)))
-    return (torch.empty(heads * head, dtype=torch.float32, device=dev),
-            torch.empty(chunks * 16 * w.heads * (-(-w.vdim // 16) * 16), dtype=torch.float32, device=dev))
+    try:
+        return (torch.empty(heads * head, dtype=torch.float32, device=dev),
+                torch.empty(chunks * 16 * w.heads * (-(-w.vdim // 16) * 16), dtype=torch.float32, device=dev))
+    except torch.OutOfMemoryError:
+        return None
 
 
 def delta_decode(proj: torch.Tensor, off_b: int, w: DeltaWeights, ring: torch.Tensor,

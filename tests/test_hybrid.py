@@ -401,6 +401,35 @@ def test_delta_chains(target, case, monkeypatch):
 
 
 @on
+def test_delta_without_memory_for_the_chains(target, monkeypatch):
+    """Where the operands of the chunks do not fit, the one-launch form gives the same outputs and states."""
+    dev, dt = target
+    lens = [40, 70]
+    proj, off_b, w, decay, gate, want, states = _delta_case(dev, dt, 4, 2, 128, 128, 3, lens)
+    p, pos = _portions(dev, lens, [0, 0], [1, 0])
+    assert ops.delta._chain_ok(w, decay, gate, p) and ops.delta._chain_workspace(w, 110, 2, dev) is not None
+    ring, state = torch.zeros((2, 3, w.channels), dtype=dt, device=dev), torch.zeros((2, 4, 128, 128), device=dev)
+    conv = ops.short_conv(proj, w, ring, pos, p)
+    empty, asked = torch.empty, []
+
+    def refuse(*shape, **k):
+        if k.get("dtype") is torch.float32 and isinstance(shape[0], int):  # a workspace
+            asked.append(shape)
+            raise torch.OutOfMemoryError
+        return empty(*shape, **k)
+
+    monkeypatch.setattr(ops.delta.torch, "empty", refuse)
+    assert ops.delta._chain_workspace(w, 110, 2, dev) is None
+    out = ops.delta_scan(proj, off_b, conv, w, ring, state, decay, gate, p)
+    monkeypatch.undo()
+    assert len(asked) == (1 if dev == "cpu" else 2)
+    t = tol(dt, 5e-5, 3e-2)
+    close(out, want, t)
+    for s, S in zip((1, 0), states):
+        close(state[s], S, t)
+
+
+@on
 def test_delta_remembers_far_tokens(target):
     """Channels that hardly decay: a loud write hundreds of tokens back still shows."""
     dev, dt = target
