@@ -823,17 +823,24 @@ def w4_shape_ok(M: int, N: int, K: int) -> bool:
 
 
 def _w4_long(M: int, N: int, K: int) -> bool:
-    """Whether gemm_w4 takes a K above W4_MAX_K that no tuned library solution covers: from 4096 columns,
-    where the last round of tiles is a part of one and leaves at most three tenths of the CUs idle on average.
-    The library's own choice / gemm_w4, us: 4096 x 11264, 6400 rows 678 / 480, 11520 1044 / 718, 14848 1187 / 956,
-    7680 449 / 481; 4096 x 14336, 7680 rows 1012 / 615, 13000 1245 / 1122; 4096 x 18432, 8960 rows 1414 / 1143,
-    13000 1577 / 1620, 15616 1970 / 1684.  Below the line, 5120 x 4096 x 11264 (0.62): 353 / 502; whole rounds,
-    16384 rows, K 11264 963 / 985, 14336 1194 / 1240, 18432 1558 / 1736; 2048 columns, K 9216, 6400 rows 177 / 210,
-    13000 363 / 400."""
-    if not (_w4_plain and _enabled and M >= W4_MIN_M and K % 64 == 0 and N % 256 == 0 and N >= 4096):
+    """Whether gemm_w4 takes a K above W4_MAX_K that no tuned library solution covers.  The library's own
+    choice is as good where 256 x 256 tiles come to whole, quarter and three-quarter rounds of the CUs, and
+    falls off in between; which, and how far, depends on K and N.  The library's / gemm_w4's time at 4352 ..
+    16384 rows, K from 10240, 4096 .. 5120 columns (720 shapes): 0.94 .. 1.76, below 0.98 at six, 1.25 in
+    the mean; e.g. 4096 x 11264, 6400 rows 1.44, 8960 1.36, 11520 1.48, 15104 1.29.  Outside: whole and quarter
+    rounds there 0.83 .. 1.0, K 8704 and 9216 0.75 .. 1.56 with most below 1, 8192 columns 0.74 .. 1.1 past
+    three rounds, 2048 columns 0.84 .. 0.91; K above 16384 below half a round 0.86 .. 1.2."""
+    if not (_w4_plain and _enabled and M >= W4_MIN_M and max(10240, W4_MAX_K + 1) <= K <= 28672 and K % 64 == 0
+            and N % 256 == 0 and 4096 <= N <= 5120):
         return False
     tiles = -(-M // 256) * (N // 256)
-    return tiles % 256 != 0 and tiles >= 0.7 * 256 * -(-tiles // 256)
+    rounds, part = divmod(tiles, 256)
+    even = 256 % (N // 256) == 0  # a round ends with a row of tiles
+    if not 384 < tiles < 998 or part == 192:
+        return False
+    if part >= 128:
+        return part < (243 if even and rounds == 2 else 219)
+    return K <= 16384 and (0 < part < (51 if even else 38) or part > 76)
 
 
 def w4_ok(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor | None = None) -> bool:

@@ -208,11 +208,14 @@ def test_gated_default_form(hipk, M, I, K, act):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K,kind", [(5889, 4096, 8256, "w4"), (7168, 4096, 11264, "w4"), (4608, 4096, 8320, "torch"),
-                                        (4096, 4096, 8256, "torch"), (6144, 2048, 11264, "torch")])
+@pytest.mark.parametrize("M,N,K,kind", [(6145, 4096, 10304, "w4"), (7681, 4352, 11264, "w4"), (11520, 4096, 17472, "w4"),
+                                        (8960, 4096, 17472, "torch"), (9216, 4096, 11264, "torch"),
+                                        (4096, 4096, 10304, "torch"), (8192, 4096, 10304, "torch"),
+                                        (6400, 4096, 8256, "torch"), (6400, 2048, 11264, "torch")])
 def test_long_k_prefill_route(hipk, M, N, K, kind):
-    """K above the limit of the measured shapes, without a tuned solution: gemm_w4 where its last round of tiles
-    is a part of one and full enough (4608: not; 4096: whole), from 4096 columns.  Rows against 64 bits: bf16 rounding of the result and fp32 sums of K products."""
+    """K above the limit of the measured shapes, without a tuned solution: gemm_w4 between the quarter rounds of its
+    tiles (9216 rows: 2.25; 4096 and 8192: whole), from K 10240 and 4096 columns on.  Rows against 64 bits: bf16
+    rounding of the result and fp32 sums of K products."""
     G.reset()
     g = torch.Generator(device="cuda").manual_seed(M)
     x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
