@@ -94,7 +94,7 @@ def _activate() -> dict:
     with _lock:
         if _table is not None:
             return _table
-        tab: dict[tuple[int, int, int, int], tuple[int, int, int, int, int]] = {}
+        tab: dict[tuple[int, int, int, int], tuple[int, int, int, int, int, int]] = {}
         pre: dict[tuple[int, int, int], list[tuple[int, int, bool, bool]]] = {}
         if _enabled and torch.cuda.is_available():
             ver = str(hipk().lt_version())
@@ -109,13 +109,14 @@ def _activate() -> dict:
                     # a prefill-table shape that is also a decode batch above the buckets
                     # (Gemma-2B's 2048 rows) with a measured gemm_xd winner: the gemm_xd form
                     # only (its library algo stays with the prefill table)
-                    tab[(M, N, K, ldx)] = (-1, 0, 0, int(e["xd"]), 0)
+                    tab[(M, N, K, ldx)] = (-1, 0, 0, int(e["xd"]), 0, 1)
                     continue
                 nt_tuned = bool(e.get("nt_tuned"))
                 tab[(M, N, K, ldx)] = (int(e.get("algo", -1)), int(e.get("skinny", 0)),
                                        int(e.get("midm", 0)) if _midm_enabled else 0,
                                        _xd_policy(M, int(e.get("xd", 0)), nt_tuned),
-                                       _xd_policy(M, int(e.get("xd_glu", 0)), nt_tuned))
+                                       _xd_policy(M, int(e.get("xd_glu", 0)), nt_tuned),
+                                       int(e.get("stream", 1)))
         for v in pre.values():
             v.sort()
         _prefill.clear()
@@ -163,7 +164,7 @@ def set_enabled(on: bool) -> None:
 
 # ------------------------------------------------------------------ routing
 def _decode_entry(M: int, N: int, K: int,
-                  ldx: int) -> tuple[int, tuple[int, int, int, int, int]] | None:
+                  ldx: int) -> tuple[int, tuple[int, int, int, int, int, int]] | None:
     """(tuned bucket, entry) for a decode-sized shape, None for torch's (hipBLASLt heuristic)
     path.  The tuner measured every (model shape, DECODE_BUCKETS M) and kept an entry only
     where something beat the heuristic pick, so a bucket without an entry means "the
@@ -225,13 +226,14 @@ def _resolve(M: int, N: int, K: int, ldx: int) -> tuple[str, int]:
         if a >= 0:
             return ("lt", a)
         return ("w4", 0) if _w4_long(M, N, K) else ("torch", 0)
-    if ldx % 8 == 0 and stream_ok(M, N, K):
-        return ("skinny", STREAM)
     found = _decode_entry(M, N, K, ldx)
+    # the rule goes ahead of the table, but for entries that were measured faster ("stream": 0)
+    if ldx % 8 == 0 and stream_ok(M, N, K) and (found is None or found[1][5]):
+        return ("skinny", STREAM)
     if found is None:
         v = skinny_variant(M, N, K, ldx)
         return ("skinny", v) if v else ("torch", 0)
-    _, (algo, sk, midm, xd, _) = found
+    _, (algo, sk, midm, xd, _, _) = found
     if algo < 0 and not (sk or midm or xd):
         return ("torch", 0)  # measured: the library's heuristic pick beat every candidate
     if sk and M <= SKINNY_MAX_M and skinny_supports(sk, M, N, K, ldx):
@@ -470,15 +472,19 @@ def stream_ok(M: int, N: int, K: int, epi: str = "store") -> bool:
         33, 32000 51 / 65; 12800 27 / 26)
       33 .. 64 rows: 2048 columns and long W (64000 rows 59 / 71; 8192 15.7 / 12.6); gated where gemm_xd's
         form does not fill the chip (32768 rows 34.7, gemm_xd 32.5)
-      slices: adding the parts up costs about 3 us, and more for more rows: plain products of few
-        slices (4096 x 14336 25.4 / 27.8, 2048 x 16384 17.3 / 23.2, 2048 x 7168 also at 32 rows 15.4 / 18.4;
-        4096 x 14336 at 32 rows 30.3 / 29.1, 8192 x 28672 91 / 89)"""
+      slices: adding the parts up costs about 3 us, and more for more rows.  Plain products of two to four,
+        to 8 rows (2048 x 7168 11.5 / 13.9, 8192 x 8192 28.3 / 31.8, 5120 x 12288 27.0 / 42.0; 4096 x 7168, the
+        closest, 15.7 / 14.4); 9 .. 16 rows outside of the 2048 .. 5120 columns where the library's pick holds
+        (4096 x 8192 17.9 / 16.6, 2560 x 8192 16.8 / 14.0; 2048 x 7168 12.4 / 12.7, 5120 x 12288 27.6 / 33.5)
+        unless in four (4096 x 14336 25.2 / 27.3); above 16 rows they lose but for 32 rows of
+        two slices of 14 steps (2048 x 7168 15.7 / 18.6; 28 rows 14.9 / 12.9; 2048 x 8192 17.1 / 16.1)"""
     s = stream_slices(M, N, K, epi)
     if not s or M < 3 or SKINNY_MAX_M <= 0:
         return False
     rows = N * (1 + STREAM_ACT[epi][0])
     if s > 1:
-        return epi == "store" and s <= 4 and (M <= 16 or M <= 32 and s == 2 and N <= 2048)
+        return epi == "store" and s <= 4 and (M <= 8 or M <= 16 and (N <= 2048 or N >= 5120 or s == 4)
+                                              or M == 32 and N <= 2048 and K == 7168)
     if M <= 16:
         return rows * K >= 24_000_000
     if M <= 32:

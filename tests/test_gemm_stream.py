@@ -102,6 +102,24 @@ def test_routes_to_the_stream(hipk, M):
 
 
 @pytest.mark.gpu
+def test_measured_shapes_keep_their_kernels(hipk):
+    """Entries of the tuning table that say the streaming kernel is slower: the table's kernel, for the batches
+    that pad to the entry's bucket too; the bucket above takes the rule again."""
+    G.reset()
+    tab = {tuple(int(v) for v in k.split(",")) for k, e in G.load_table()[str(hipk.lt_version())].items()
+           if e.get("stream") == 0}
+    assert tab
+    for M, N, K, ldx in tab:
+        assert G.stream_ok(M, N, K) and G.route(M, N, K, ldx) != ("skinny", G.STREAM)
+    assert (4, 1280, 8192, 8192) in tab
+    assert G.route(3, 1280, 8192, 8192) != ("skinny", G.STREAM) and G.route(8, 1280, 8192, 8192) == ("skinny", G.STREAM)
+    x = torch.randn(3, 8192, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(1280, 8192, device="cuda") / 8192 ** 0.5).to(torch.bfloat16)
+    want = x.double() @ w.double().t()
+    assert ((ops.linear(x, w).double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-3).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T", [1, 5, 16, 37, 80, 150])
 @pytest.mark.parametrize("H,I,E,k,act,e_off", [(2048, 1792, 16, 4, "silu", 0), (4096, 3584, 20, 4, "relu2", 0),
                                               (2048, 4096, 8, 2, "gelu_tanh", 0), (1792, 2048, 24, 6, "clamped", 0),
