@@ -876,8 +876,8 @@ def w4_glu_ok(x: torch.Tensor, w: torch.Tensor, act: str) -> bool:
 
 def glu_form(M: int, N2: int, K: int, ldx: int, act: str = "silu") -> int:
     """gemm_xd gated form for a decode batch M through the [gate; up] weight [N2, K]: the one the
-    tuning table measured fastest (bucket-above for an off-bucket M), else ``_glu_default``; 0:
-    none."""
+    tuning table measured fastest (bucket-above for an off-bucket M), else ``_glu_default``, also
+    where the table has an entry for the plain product only; 0: none."""
     if not (_xd_enabled and _enabled) or M > DECODE_MAX_M:
         return 0
     found = _decode_entry(M, N2, K, ldx)
@@ -889,19 +889,22 @@ def glu_form(M: int, N2: int, K: int, ldx: int, act: str = "silu") -> int:
 
 def _glu_default(M: int, I: int, K: int) -> int:
     """gemm_xd gated form of a shape without a measured one, 0 where the library's product and an
-    activation pass, or above 640 rows gemm_w4, are as fast.  One launch and no [M, 2 I] intermediate
+    activation pass, or from W4_GLU_MIN_M rows gemm_w4, are as fast.  One launch and no [M, 2 I] intermediate
     win where ``xd_default_form``'s tiles fill the chip: 160 of them, 112 where K is short.  us,
-    library + pass / gemm_xd: 7168 x 2048 rows of W a half, 64 rows of x 22.8 / 16.6, 160 28.6 / 20.2, 512
-    38.5 / 32.4; 14336 x 4096, 64 rows 56.0 / 48.7; 11008 x 4096, 224 rows 64.9 / 56.6; too few tiles:
-    3584 x 4096, 64 rows 21.4 / 24.8.  Tiles of 128 columns a half lose to narrower ones up to 128 rows
-    (28672 x 8192 188 / 199, narrow 179) and to the library above 256 (14336 x 4096, 320 rows 82 / 97).
+    library + pass / gemm_xd: 7168 x 2048 rows of W a half, 64 rows of x 20.1 / 17.1, 160 29.2 / 20.9, 512
+    40.0 / 33.3; 14336 x 4096, 64 rows 59.2 / 48.8; 11008 x 4096, 224 rows 66.5 / 54.0; too few tiles:
+    3584 x 4096, 64 rows 21.4 / 24.8.  So do the table's buckets that were tuned without a gated form: 7168 x
+    4096, 128 rows 40.9 / 34.6, 448 62.9 / 56.5; 28672 x 8192, 24 rows 169 / 155, 96 199 / 177.
+    Tiles of 128 columns a half lose to narrower ones up to 128 rows (28672 x 8192 188 / 199, narrow 179),
+    with long K above them (20480 x 8192, 160 rows 179 / 203; 16384 x 4096 154 / 137) and to the library from
+    256 rows to gemm_w4's first (14336 x 4096, 320 rows 82 / 97; 7168 x 4096, 600 72 / 87, 5632 x 2048 39 / 48).
     Above 512 rows for the shapes that leave gemm_w4 fewer than three quarters of the CUs: 3584 x 2048, 768 rows
     90 / 29.6, 1024 49 / 30.7; 7168 x 2048, 1024 rows (224 tiles) 53.0 / 53.4."""
     if not 17 <= M <= DECODE_MAX_M or M > 512 and -(-M // 256) * (I // 128) > 176:
         return 0
     form = xd_default_form(M, I, K, True)
-    if form // 10 % 10 == 8 and M <= 512:
-        if M > 256:
+    if form // 10 % 10 == 8 and M < W4_GLU_MIN_M:
+        if M > 256 or M > 128 and K > 4096:
             return 0
         if M <= 128:
             form = 141

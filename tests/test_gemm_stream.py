@@ -225,6 +225,17 @@ def test_gated_default_form(hipk, M, I, K, act):
     assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all()
 
 
+def test_gated_default_leaves_what_the_library_does_faster():
+    """Tiles of 128 columns a half: not above 128 rows with long K, nor from 257 rows to gemm_w4's first; the
+    neighbours on the other side of each line keep theirs."""
+    none = [(160, 28672, 8192), (256, 20480, 8192), (320, 14336, 4096), (513, 7168, 4096), (600, 7168, 2048),
+            (639, 5632, 2048)]
+    assert not any(G._glu_default(*s) for s in none)
+    some = [(128, 28672, 8192), (160, 16384, 4096), (256, 32768, 4096), (512, 7168, 4096), (640, 7168, 4096),
+            (600, 3584, 2048)]
+    assert all(G._glu_default(*s) for s in some), [G._glu_default(*s) for s in some]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,kind", [(6145, 4096, 10304, "w4"), (7681, 4352, 11264, "w4"), (11520, 4096, 17472, "w4"),
                                         (8960, 4096, 17472, "torch"), (9216, 4096, 11264, "torch"),
