@@ -489,7 +489,7 @@ def stream_ok(M: int, N: int, K: int, epi: str = "store") -> bool:
         return rows * K >= 24_000_000
     if M <= 32:
         return rows >= (16384 if K > 2048 else 2048)
-    return rows >= 14336 and not (STREAM_ACT[epi][0] and _glu_default(M, N, K))
+    return rows >= 14336 and not (STREAM_ACT[epi][0] and glu_form(M, rows, K, K, epi))
 
 
 def stream_gemm(x: torch.Tensor, w: torch.Tensor, epi: str = "store", out: torch.Tensor | None = None,
@@ -881,13 +881,13 @@ def glu_form(M: int, N2: int, K: int, ldx: int, act: str = "silu") -> int:
     if not (_xd_enabled and _enabled) or M > DECODE_MAX_M:
         return 0
     found = _decode_entry(M, N2, K, ldx)
-    form = found[1][4] if found is not None and found[1][4] else _glu_default(M, N2 // 2, K)
-    if act == "clamped" and form // 10 % 10 not in XD_CLAMP_NF:
-        return 0
+    form = found[1][4] if found is not None else 0
+    if not form or act == "clamped" and form // 10 % 10 not in XD_CLAMP_NF:
+        form = _glu_default(M, N2 // 2, K, act)
     return form if form and xd_supported(M, N2 // 2, K, form, glu=True) else 0
 
 
-def _glu_default(M: int, I: int, K: int) -> int:
+def _glu_default(M: int, I: int, K: int, act: str = "silu") -> int:
     """gemm_xd gated form of a shape without a measured one, 0 where the library's product and an
     activation pass, or from W4_GLU_MIN_M rows gemm_w4, are as fast.  One launch and no [M, 2 I] intermediate
     win where ``xd_default_form``'s tiles fill the chip: 160 of them, 112 where K is short.  us,
@@ -899,7 +899,9 @@ def _glu_default(M: int, I: int, K: int) -> int:
     with long K above them (20480 x 8192, 160 rows 179 / 203; 16384 x 4096 154 / 137) and to the library from
     256 rows to gemm_w4's first (14336 x 4096, 320 rows 82 / 97; 7168 x 4096, 600 72 / 87, 5632 x 2048 39 / 48).
     Above 512 rows for the shapes that leave gemm_w4 fewer than three quarters of the CUs: 3584 x 2048, 768 rows
-    90 / 29.6, 1024 49 / 30.7; 7168 x 2048, 1024 rows (224 tiles) 53.0 / 53.4."""
+    90 / 29.6, 1024 49 / 30.7; 7168 x 2048, 1024 rows (224 tiles) 53.0 / 53.4.
+    The clamped activation has tiles of 64 and 128 columns only: 64 in place of 32 up to 128 rows (7168 x
+    2048, 40 rows 20.0 / 18.8, 128 23.7 / 22.1; above, 4096 x 2048, 160 rows 17.3 / 19.3)."""
     if not 17 <= M <= DECODE_MAX_M or M > 512 and -(-M // 256) * (I // 128) > 176:
         return 0
     form = xd_default_form(M, I, K, True)
@@ -908,6 +910,8 @@ def _glu_default(M: int, I: int, K: int) -> int:
             return 0
         if M <= 128:
             form = 141
+    if act == "clamped" and form // 10 % 10 not in XD_CLAMP_NF:
+        form = 141 if M <= 128 else 0
     if not form or not xd_supported(M, I, K, form, True):
         return 0
     mt, nf, _ = xd_form(form)

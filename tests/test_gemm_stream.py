@@ -236,6 +236,43 @@ def test_gated_default_leaves_what_the_library_does_faster():
     assert all(G._glu_default(*s) for s in some), [G._glu_default(*s) for s in some]
 
 
+@pytest.mark.parametrize("xd", [True, False])
+def test_streaming_yields_to_forms_that_run(monkeypatch, xd):
+    """Where a gated product of 33 to 64 rows leaves the streaming kernel for gemm_xd, gemm_xd has a form for its
+    activation; the clamped one gets a form of its own tiles; without gemm_xd the stream takes all it can."""
+    monkeypatch.setattr(G, "_xd_enabled", xd)
+    seen = set()
+    for act in G.GATED:
+        for M in (33, 48, 64):
+            for I in (1024, 3584, 5632, 7168, 8192, 14336, 16384):
+                for K in (2048, 4096):
+                    form = G.glu_form(M, 2 * I, K, K, act)
+                    assert not form or xd and G.xd_supported(M, I, K, form, True)
+                    assert act != "clamped" or not form or G.xd_form(form)[1] in G.XD_CLAMP_NF
+                    if G.stream_slices(M, I, K, act) == 1 and 2 * I >= 14336:
+                        assert G.stream_ok(M, I, K, act) != bool(form)
+                        seen.add((act, bool(form)))
+    assert seen >= {(a, xd) for a in G.GATED}
+    if xd:
+        assert G.glu_form(48, 14336, 2048, 2048, "clamped") == 1141 and G.glu_form(48, 14336, 2048, 2048, "silu") == 121
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [17, 64, 128])
+def test_clamped_default_form(hipk, M):
+    """A shape whose default tiles the clamped activation lacks, against 64 bits (bf16 rounding of the result)."""
+    I, K = 7168, 1024
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).bfloat16().to("cuda")
+    w = (torch.randn(2 * I, K, generator=g) / K ** 0.5).bfloat16().to("cuda")
+    assert G.glu_form(M, 2 * I, K, K, "clamped") == 1141
+    got = G.gated(x, w, "clamped", limit=1.0).double()
+    a, b = (x.double() @ w.double().t()).chunk(2, -1)
+    a, b = a.clamp(max=1.0), b.clamp(-1.0, 1.0)
+    want = a * torch.sigmoid(1.702 * a) * (b + 1)
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,kind", [(6145, 4096, 10304, "w4"), (7681, 4352, 11264, "w4"), (11520, 4096, 17472, "w4"),
                                         (8960, 4096, 17472, "torch"), (9216, 4096, 11264, "torch"),
