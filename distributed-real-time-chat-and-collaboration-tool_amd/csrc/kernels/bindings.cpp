@@ -199,6 +199,7 @@ PYBIND11_MODULE(_hipk, m) {
     return drtc::launch_stream_gemm(P<void>(y), P<const void>(x), P<const void>(w), M, N, K, ldx, ldy, glu, act, limit,
                                     slices, P<void>(slab), slab_bytes, P<void>(tickets), n_tickets, S(st));
   });
+  m.def("stream_moe_tiles", &drtc::stream_moe_tiles);  // (rows per expert, H, I, gated)
   m.def("midm_gemm", [](u64 y, u64 x, u64 w, u64 res, int M, int N, int K, int ldx, int ldy,
                         int ldr, int epi, int splits, u64 slab, int64_t slab_bytes, u64 st) {
     return drtc::launch_midm_gemm(P<void>(y), P<const void>(x), P<const void>(w),

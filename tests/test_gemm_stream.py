@@ -119,6 +119,14 @@ def test_measured_shapes_keep_their_kernels(hipk):
     assert ((ops.linear(x, w).double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-3).all()
 
 
+# tiles of 16 rows in an entry, 0: not taken; 2048 x 4096 and 4096 x 3584 leave registers for 32 rows (gated: 16)
+STREAMED_TILES = {(2048, "silu", 0): {1: 1, 5: 1, 16: 1, 37: 1, 80: 2, 150: 4},
+                  (4096, "relu2", 0): {1: 1, 5: 1, 16: 1, 37: 1, 80: 2, 150: 0},
+                  (2048, "gelu_tanh", 0): {1: 1, 5: 1, 16: 1, 37: 1, 80: 0, 150: 0},
+                  (1792, "clamped", 0): {1: 1, 5: 1, 16: 1, 37: 1, 80: 2, 150: 4},
+                  (2048, "silu", 4): {1: 1, 5: 1, 16: 1, 37: 2, 80: 4, 150: 0}}
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("T", [1, 5, 16, 37, 80, 150])
 @pytest.mark.parametrize("H,I,E,k,act,e_off", [(2048, 1792, 16, 4, "silu", 0), (4096, 3584, 20, 4, "relu2", 0),
@@ -142,10 +150,13 @@ def test_streamed_experts(hipk, T, H, I, E, k, act, e_off):
     def run(v=5):
         return ops.fused_moe(x, lg, w_in, w_out, k, act, E, e_off, ws, variant=v, limit=0.9)
 
-    try:
+    mt = hipk.stream_moe_tiles(T * k // e_local, H, I, act != "relu2")
+    assert mt == STREAMED_TILES[(H, act, e_off)][T]
+    if mt:
         y = run()
-    except RuntimeError:
-        assert T * k // e_local > 10  # entries of more rows than the registers hold
+    else:  # more rows to an expert than the registers hold
+        with pytest.raises(RuntimeError):
+            run()
         y = run(-1)
     want = ops.fused_moe_ref(x, lg, w_in, w_out, k, act, e_off, limit=0.9).double()
     # both round the hidden rows and the experts' outputs to bf16: a few of them differ by one unit
