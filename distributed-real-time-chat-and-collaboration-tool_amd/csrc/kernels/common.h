@@ -49,6 +49,11 @@ DRTC_DEVICE float wave_max(float v) {
   return v;
 }
 
+// Barrier that waits for this wave's LDS traffic only: loads from memory stay in flight.
+DRTC_DEVICE void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // 16x16x32 bf16 MFMA (gfx950).  Operand maps (cdna_hip_programming.md §3):
 //   A: lane l holds A[row l&15][k = 8*(l>>4) + j], j = 0..7
 //   B: lane l holds B[k = 8*(l>>4) + j][col l&15]

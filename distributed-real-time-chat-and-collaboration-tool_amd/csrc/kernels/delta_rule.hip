@@ -757,10 +757,6 @@ __global__ __launch_bounds__(NTHR, 2) void delta_chunk_kernel(DeltaArgs a) {
 // 4,000: 457 against 2,492.  With portions and heads enough for every CU delta_chunk keeps the fp32
 // units as busy without operands in memory (64 x 250, 32 heads: 959 against 1,249).
 // Chunks are numbered through the portions in their order: at most rows / 16 + nseg of them.
-// Waits for this wave's LDS traffic only: loads for the next chunk stay in flight.
-DRTC_DEVICE void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
 template <int DT>
 struct ChainEntry {  // floats of a (chunk, head)
   static constexpr int ek = 0, eq = 256 * DT, kd = 512 * DT;  // [DT][64 lanes][4]

@@ -1,5 +1,5 @@
 // Weight-streaming GEMM of decode batches (gfx950): y[M, N] = epi(x[M, K] @ W[N, K]^T), 1 <= M <= 64,
-// bf16 in and out, fp32 accumulation; optionally x = norm(x + residual) (RMSNorm) on the way in.
+// bf16 in and out, fp32 accumulation.
 //
 // The bound is one pass over W.  A persistent workgroup of 8 waves divides K: a wave keeps its
 // K / (8 slices) columns of all x rows in registers as MFMA operands, for as long as it lives, and
@@ -15,9 +15,10 @@
 // activation behind it; 32000 x 4096: 46 against 65 us; 64128 x 4096: 90 against 104.
 //   x:      lane (r = l & 15, g = l >> 4) holds k = 32 s + 8 g .. of token r; MT tiles of 16 tokens
 //   gated:  a gate tile and the up tile at the same rows, one after the other, then act(gate) * up
-//   slices: K too long for the registers is cut over workgroups; a wave that has summed its
-//           workgroup's part of a tile leaves it in the workspace (write-through), draws a ticket,
-//           and the last one adds the parts in the order of the slices.  No wave waits for another.
+//   slices: K too long for the registers is cut over up to four workgroups (plain products, M <= 32); a
+//           wave that has summed its workgroup's part of a tile leaves it in the workspace (write-through),
+//           draws a ticket, and the last one adds the parts in the order of the slices.  No wave waits for
+//           another.
 // Which shapes take it: ops/gemm.py stream_ok.
 #include "common.h"
 #include "launchers.h"
@@ -40,11 +41,72 @@ struct StreamArgs {
   int* tickets;
 };
 
-DRTC_DEVICE void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
 DRTC_DEVICE bf16x8 load_once(const bf16_t* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p));
+}
+
+// A tile of W past the x in registers, its fragments loaded again from na and nb as they are read.  The sums
+// of the wave go to red: products with W row r in row r, plus those in row r ^ 8, which lie 32 lanes away.
+template <int KS, int MT>
+DRTC_DEVICE void stream_tile(f32x4 (&red)[MT][64], bf16x8 (&wr)[KS], const bf16x8 (&xb)[MT][KS], bool low, int lane,
+                             const bf16_t* na, const bf16_t* nb) {
+  f32x4 acc[MT][2];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) acc[mt][0] = acc[mt][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < KS; s += 2) {
+    const u32x4 x = *(const u32x4*)&wr[s], z = *(const u32x4*)&wr[s + 1];
+    u32x4 f0, f1;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      f0[i] = low ? x[i] : z[i];
+      f1[i] = low ? z[i] : x[i];
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      acc[mt][0] = mfma16(*(const bf16x8*)&f0, xb[mt][s], acc[mt][0]);
+      acc[mt][1] = mfma16(*(const bf16x8*)&f1, xb[mt][s + 1], acc[mt][1]);
+    }
+    wr[s] = load_once(na + 32 * s);
+    wr[s + 1] = load_once(nb + 32 * s);
+    __builtin_amdgcn_sched_barrier(0);  // a load goes to the registers just read, no others
+  }
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    f32x4 v = acc[mt][0];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] += __shfl_xor(acc[mt][1][j], 32, 64);
+    red[mt][lane] = v;
+  }
+}
+
+// The waves' sums of token tile mt (gated: of gate and up), in the order of the waves.
+template <int NW, int TP, int MT>
+DRTC_DEVICE void stream_sum(f32x4 (&v)[TP], const f32x4 (&red)[NW][TP][MT][64], int mt, int lane) {
+#pragma unroll
+  for (int q = 0; q < TP; ++q) {
+    v[q] = red[0][q][mt][lane];
+#pragma unroll
+    for (int j = 1; j < NW; ++j) v[q] += red[j][q][mt][lane];
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// Four values of y.  gated: act 0 SiLU, 1 tanh-GELU, 2 clamped at limit; else squared relu or the sums.
+template <int TP>
+DRTC_DEVICE bf16x4 stream_value(const f32x4 (&v)[TP], int act, bool relu2, float limit) {
+  bf16x4 o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float f;
+    if constexpr (TP == 2)
+      f = act == 0 ? glu_value<0>(v[0][i], v[1][i], 0.f) : act == 1 ? glu_value<1>(v[0][i], v[1][i], 0.f)
+                                                         : glu_value<2>(v[0][i], v[1][i], limit);
+    else
+      f = relu2 ? fmaxf(v[0][i], 0.f) * fmaxf(v[0][i], 0.f) : v[0][i];
+    o[i] = f2bf(f);
+  }
+  return o;
 }
 
 template <int KS, int MT, bool GLU>
@@ -80,91 +142,46 @@ __global__ __launch_bounds__(512, KS * (1 + MT) <= 16 ? 4 : 2) void stream_gemm_
     for (int s = 0; s < KS; ++s)
       if (m >= a.M) xb[mt][s] = zero;
   }
-  // products of a tile: [0] with W row r in row r, [1] in row r ^ 8
-  f32x4 acc[MT][2];
-  auto pass = [&](bool more, int64_t next) {  // next: the rows after these
-    // behind the last tile: one line of W for all (two forms of the loop would share the selects, all of
-    // them ahead of the first load)
-    const bf16_t* na = more ? wa + next : a.w;
-    const bf16_t* nb = more ? wb + next : a.w;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[mt][0] = acc[mt][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < KS; s += 2) {
-      const u32x4 x = *(const u32x4*)&wr[s], z = *(const u32x4*)&wr[s + 1];
-      u32x4 f0, f1;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        f0[i] = low ? x[i] : z[i];
-        f1[i] = low ? z[i] : x[i];
-      }
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        acc[mt][0] = mfma16(*(const bf16x8*)&f0, xb[mt][s], acc[mt][0]);
-        acc[mt][1] = mfma16(*(const bf16x8*)&f1, xb[mt][s + 1], acc[mt][1]);
-      }
-      wr[s] = load_once(na + 32 * s);
-      wr[s + 1] = load_once(nb + 32 * s);
-      __builtin_amdgcn_sched_barrier(0);  // a load goes to the registers just read, no others
-    }
-  };
   auto finish = [&](int t, int mt, const f32x4 (&v)[TP]) {
     if (16 * mt + r >= a.M) return;
-    bf16x4 o;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float f;
-      if constexpr (GLU)
-        f = a.act == 0 ? glu_value<0>(v[0][i], v[1][i], 0.f) : a.act == 1 ? glu_value<1>(v[0][i], v[1][i], 0.f)
-                                                             : glu_value<2>(v[0][i], v[1][i], a.limit);
-      else
-        f = a.act == 1 ? fmaxf(v[0][i], 0.f) * fmaxf(v[0][i], 0.f) : v[0][i];
-      o[i] = f2bf(f);
-    }
-    *reinterpret_cast<bf16x4*>(a.y + (int64_t)(16 * mt + r) * a.ldy + 16 * t + 4 * g) = o;
+    *reinterpret_cast<bf16x4*>(a.y + (int64_t)(16 * mt + r) * a.ldy + 16 * t + 4 * g) =
+        stream_value<TP>(v, a.act, a.act == 1, a.limit);
   };
   // slices: this wave's part of token tile mt of tile t to the workspace; the last one adds them
-  const int64_t part = (int64_t)tiles * MT * TP * 256;
   auto publish = [&](int t, int mt, f32x4 (&v)[TP]) {
-    float* at = a.slab + (((int64_t)t * MT + mt) * TP) * 256 + 4 * lane;
+    const int64_t part = (int64_t)tiles * MT * 256;
+    float* at = a.slab + ((int64_t)t * MT + mt) * 256 + 4 * lane;
 #pragma unroll
-    for (int p = 0; p < TP; ++p)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        __hip_atomic_store(at + slice * part + p * 256 + i, v[p][i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int i = 0; i < 4; ++i)
+      __hip_atomic_store(at + slice * part + i, v[0][i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     int n = 0;
     int* ticket = a.tickets + t * MT + mt;
     if (lane == 0) n = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (__builtin_amdgcn_readfirstlane(n) != a.slices - 1) return;
     if (lane == 0) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-    for (int p = 0; p < TP; ++p) v[p] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    v[0] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
     for (int z = 0; z < a.slices; ++z)
 #pragma unroll
-      for (int p = 0; p < TP; ++p)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          v[p][i] += __hip_atomic_load(at + z * part + p * 256 + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (int i = 0; i < 4; ++i)
+        v[0][i] += __hip_atomic_load(at + z * part + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     finish(t, mt, v);
   };
-  // slices: a wave's sum waits here for the end (one at most, see go): publishing drains its loads
+  // slices: a wave's sum waits here for the end (one at most, see go): publishing drains its loads.  The
+  // branch stays in instances that are never cut: without it the gated ones came out 9 % slower (7168 x 2048,
+  // 8 rows 16.4 -> 17.9 us)
   f32x4 held[TP];
   int held_t = -1, held_mt = 0, buf = 0;
 #pragma unroll 1
   for (int u = 0;; ++u) {  // gated: u counts gate and up tiles
     const int i = u / TP, t = b + i * G, p = u % TP, p1 = (u + 1) % TP, t1 = b + (u + 1) / TP * G;
     if (t >= tiles) break;
-    pass(t1 < tiles, rows(t1, p1));
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      // rows r ^ 8 of the second sum lie 32 lanes away
-      f32x4 v = acc[mt][0];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] += __shfl_xor(acc[mt][1][j], 32, 64);
-      red[buf][wv][p][mt][lane] = v;
-    }
+    // behind the last tile: one line of W for all (two forms of the loop would share the selects, all of
+    // them ahead of the first load)
+    const int64_t next = rows(t1, p1);
+    const bool more = t1 < tiles;
+    stream_tile<KS, MT>(red[buf][wv][p], wr, xb, low, lane, more ? wa + next : a.w, more ? wb + next : a.w);
     if (p1 != 0) continue;
     lds_barrier();
     // lane l: y[16 mt + (l & 15)][16 t + 4 (l >> 4) ..]; the buffer is written again only behind the
@@ -172,19 +189,13 @@ __global__ __launch_bounds__(512, KS * (1 + MT) <= 16 ? 4 : 2) void stream_gemm_
     const int mt = (wv - MT * i) & (NW - 1);  // MT of the waves, others for the next tile
     if (mt < MT) {
       f32x4 v[TP];
-#pragma unroll
-      for (int q = 0; q < TP; ++q) {
-        v[q] = red[buf][0][q][mt][lane];
-#pragma unroll
-        for (int j = 1; j < NW; ++j) v[q] += red[buf][j][q][mt][lane];
-      }
+      stream_sum<NW, TP, MT>(v, red[buf], mt, lane);
       if (a.slices == 1) {
         finish(t, mt, v);
       } else {
         held_t = t;
         held_mt = mt;
-#pragma unroll
-        for (int q = 0; q < TP; ++q) held[q] = v[q];
+        held[0] = v[0];
       }
     }
     buf ^= 1;
@@ -262,36 +273,7 @@ __global__ __launch_bounds__(64 * NW, KS * (1 + MT) <= 16 && !GLU ? 4 : 2) void 
     }
     const bool more = u + 1 < q1 * TP;
     const int64_t next = p == TP - 1 ? rows(base, t, 0) : rows(b0, t0, 1);
-    const bf16_t* na = more ? wa + next : a.w;
-    const bf16_t* nb = more ? wb + next : a.w;
-    f32x4 acc[MT][2];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[mt][0] = acc[mt][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < KS; s += 2) {
-      const u32x4 x = *(const u32x4*)&wr[s], z = *(const u32x4*)&wr[s + 1];
-      u32x4 f0, f1;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        f0[i] = low ? x[i] : z[i];
-        f1[i] = low ? z[i] : x[i];
-      }
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        acc[mt][0] = mfma16(*(const bf16x8*)&f0, xb[mt][s], acc[mt][0]);
-        acc[mt][1] = mfma16(*(const bf16x8*)&f1, xb[mt][s + 1], acc[mt][1]);
-      }
-      wr[s] = load_once(na + 32 * s);
-      wr[s + 1] = load_once(nb + 32 * s);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      f32x4 v = acc[mt][0];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] += __shfl_xor(acc[mt][1][j], 32, 64);
-      red[buf][wv][p][mt][lane] = v;
-    }
+    stream_tile<KS, MT>(red[buf][wv][p], wr, xb, low, lane, more ? wa + next : a.w, more ? wb + next : a.w);
     if (p != TP - 1) continue;
     lds_barrier();
     int mt = wv - first;  // MT of the waves from ``first`` on, the next ones for the next tile
@@ -299,26 +281,10 @@ __global__ __launch_bounds__(64 * NW, KS * (1 + MT) <= 16 && !GLU ? 4 : 2) void 
     first = (first + MT) % NW;
     if (mt < MT) {
       f32x4 v[TP];
-#pragma unroll
-      for (int q = 0; q < TP; ++q) {
-        v[q] = red[buf][0][q][mt][lane];
-#pragma unroll
-        for (int j = 1; j < NW; ++j) v[q] += red[buf][j][q][mt][lane];
-      }
-      if (16 * mt + r < nr) {
-        bf16x4 o;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float f;
-          if constexpr (GLU)
-            f = a.act == 0 ? glu_value<0>(v[0][i], v[1][i], 0.f) : a.act == 1 ? glu_value<1>(v[0][i], v[1][i], 0.f)
-                                                                 : glu_value<2>(v[0][i], v[1][i], a.limit);
-          else
-            f = a.act == 3 ? fmaxf(v[0][i], 0.f) * fmaxf(v[0][i], 0.f) : v[0][i];
-          o[i] = f2bf(f);
-        }
-        *reinterpret_cast<bf16x4*>(a.y + (int64_t)(row0 + 16 * mt + r) * a.ldy + 16 * t0 + 4 * g) = o;
-      }
+      stream_sum<NW, TP, MT>(v, red[buf], mt, lane);
+      if (16 * mt + r < nr)
+        *reinterpret_cast<bf16x4*>(a.y + (int64_t)(row0 + 16 * mt + r) * a.ldy + 16 * t0 + 4 * g) =
+            stream_value<TP>(v, a.act, a.act == 3, a.limit);
     }
     buf ^= 1;
   }
@@ -357,7 +323,7 @@ int moe_go(const StreamMoe& a, hipStream_t st) {
   }
   DRTC_MOE_CUT(8, 8)
   DRTC_MOE_CUT(8, 7)
-  if constexpr (MT <= 2) {
+  if constexpr (MT == 1 || (MT == 2 && !GLU)) {  // (stream_moe_tiles)
     DRTC_MOE_CUT(16, 8)
     DRTC_MOE_CUT(14, 8)
   }
@@ -372,17 +338,17 @@ int moe_form(const StreamMoe& a, bool glu, bool gather, hipStream_t st) {
 
 }  // namespace
 
-// glu 0: act 0 store, 1 squared relu; glu 1: W holds N gate rows, then N up rows.  slices > 1: slab of
-// slices * N / 16 * tiles of M * (1 + glu) KB and N / 16 * tiles of M tickets, zero (they are left zero).
+// glu 0: act 0 store, 1 squared relu; glu 1: W holds N gate rows, then N up rows.  slices > 1 (glu 0, M <= 32):
+// slab of slices * N / 16 * tiles of M KB and N / 16 * tiles of M tickets, zero (they are left zero).
 int launch_stream_gemm(void* y, const void* x, const void* w, int M, int N, int K, int ldx, int ldy, int glu, int act,
                        float limit, int slices, void* slab, int64_t slab_bytes, void* tickets, int n_tickets,
                        hipStream_t st) {
   const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
-  if (M < 1 || M > 64 || N < 16 || N % 16 || slices < 1 || slices > 16 || K % (256 * slices) || ldx % 8 || ldy % 4 ||
-      act < 0 || act > (glu ? 2 : 1))
+  if (M < 1 || M > 64 || N < 16 || N % 16 || slices < 1 || slices > 4 || K % (256 * slices) || ldx % 8 || ldy % 4 ||
+      act < 0 || act > (glu ? 2 : 1) || (slices > 1 && (glu || mt > 2)))
     return -1;
   const int64_t parts = (int64_t)(N / 16) * mt;
-  if (slices > 1 && (!slab || !tickets || slab_bytes < slices * parts * (1 + (glu != 0)) * 1024 || n_tickets <= parts))
+  if (slices > 1 && (!slab || !tickets || slab_bytes < slices * parts * 1024 || n_tickets <= parts))
     return -2;
   const StreamArgs a{(bf16_t*)y, (const bf16_t*)x, (const bf16_t*)w, M, N, K, ldx, ldy, act, limit, slices,
                      (float*)slab, (int*)tickets};

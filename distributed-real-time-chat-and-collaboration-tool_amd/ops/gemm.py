@@ -443,6 +443,7 @@ def glu_linear(gu: torch.Tensor, w: torch.Tensor, act: str = "silu") -> torch.Te
 STREAM_MAX_M = 64
 # K steps of 32 that a wave's registers hold of 16, 32 or 64 rows of x (gemm_stream.hip instances)
 STREAM_KS = {1: (16, 14, 8), 2: (16, 14, 8), 4: (8,)}
+STREAM_MAX_SLICES = 4  # plain products up to 32 rows
 STREAM = 10  # as a variant of the skinny kernels in the router
 STREAM_ACT = {"store": (0, 0), "relu2": (0, 1), "silu": (1, 0), "gelu_tanh": (1, 1), "clamped": (1, 2)}
 
@@ -452,10 +453,10 @@ def stream_slices(M: int, N: int, K: int, epi: str = "store") -> int:
     if not (1 <= M <= STREAM_MAX_M and N % 16 == 0 and N >= 16 and epi in STREAM_ACT):
         return 0
     mt = 1 if M <= 16 else 2 if M <= 32 else 4
+    most = 1 if mt > 2 or STREAM_ACT[epi][0] else STREAM_MAX_SLICES
     for ks in STREAM_KS[mt]:
-        s = K // (256 * ks)
-        parts = N // 16 * mt * (1 + STREAM_ACT[epi][0])
-        if K % (256 * ks) == 0 and 1 <= s <= 16 and \
+        s, parts = K // (256 * ks), N // 16 * mt
+        if K % (256 * ks) == 0 and 1 <= s <= most and \
                 (s == 1 or (s * parts * 1024 <= WS_SLAB_BYTES and parts < WS_COUNTERS - 1)):
             return s
     return 0
@@ -483,8 +484,8 @@ def stream_ok(M: int, N: int, K: int, epi: str = "store") -> bool:
         return False
     rows = N * (1 + STREAM_ACT[epi][0])
     if s > 1:
-        return epi == "store" and s <= 4 and (M <= 8 or M <= 16 and (N <= 2048 or N >= 5120 or s == 4)
-                                              or M == 32 and N <= 2048 and K == 7168)
+        return epi == "store" and (M <= 8 or M <= 16 and (N <= 2048 or N >= 5120 or s == 4)
+                                   or M == 32 and N <= 2048 and K == 7168)
     if M <= 16:
         return rows * K >= 24_000_000
     if M <= 32:
