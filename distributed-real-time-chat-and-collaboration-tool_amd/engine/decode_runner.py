@@ -36,7 +36,10 @@ DEFAULT_BUCKETS = ops.gemm.DECODE_BUCKETS
 def check_tokens(ids: np.ndarray, vocab: int) -> None:
     """Refuse tokens outside of the vocabulary while they are on the host: on the device a row
     of such a token is NaN (ops.embed)."""
-    if ids.size and (ids.min() < 0 or ids.max() >= vocab):
+    if not ids.size:
+        return
+    # a negative one is a large unsigned one: one pass over the array
+    if ids.view(f"u{ids.itemsize}").max() >= vocab if ids.dtype.kind == "i" else ids.min() < 0 or ids.max() >= vocab:
         bad = ids[(ids < 0) | (ids >= vocab)]
         raise ValueError(f"token {bad[0]} outside of the vocabulary of {vocab}")
 
