@@ -52,6 +52,8 @@ _table: dict[tuple[int, int, int, int], tuple[int, int, int, int, int]] | None =
 _prefill: dict[tuple[int, int, int], list[tuple[int, int, bool, bool]]] = {}
 # (M, N, K, ldx, beta) -> algo chosen for a prefill-sized call (-1: torch's path)
 _prefill_pick: dict[tuple[int, int, int, int, int], int] = {}
+# (M, N, K, ldx) of entries that the weight-streaming GEMM leaves alone
+_kept: set[tuple[int, int, int, int]] = set()
 # (M, N, K, ldx) -> resolved route (kind, arg)
 _routes: dict[tuple[int, int, int, int], tuple[str, int]] = {}
 DECODE_MAX_M = 1024  # decode buckets end here; larger M are prefill (or mixed) passes
@@ -94,7 +96,8 @@ def _activate() -> dict:
     with _lock:
         if _table is not None:
             return _table
-        tab: dict[tuple[int, int, int, int], tuple[int, int, int, int, int, int]] = {}
+        tab: dict[tuple[int, int, int, int], tuple[int, int, int, int, int]] = {}
+        kept: set[tuple[int, int, int, int]] = set()
         pre: dict[tuple[int, int, int], list[tuple[int, int, bool, bool]]] = {}
         if _enabled and torch.cuda.is_available():
             ver = str(hipk().lt_version())
@@ -109,18 +112,21 @@ def _activate() -> dict:
                     # a prefill-table shape that is also a decode batch above the buckets
                     # (Gemma-2B's 2048 rows) with a measured gemm_xd winner: the gemm_xd form
                     # only (its library algo stays with the prefill table)
-                    tab[(M, N, K, ldx)] = (-1, 0, 0, int(e["xd"]), 0, 1)
+                    tab[(M, N, K, ldx)] = (-1, 0, 0, int(e["xd"]), 0)
                     continue
                 nt_tuned = bool(e.get("nt_tuned"))
                 tab[(M, N, K, ldx)] = (int(e.get("algo", -1)), int(e.get("skinny", 0)),
                                        int(e.get("midm", 0)) if _midm_enabled else 0,
                                        _xd_policy(M, int(e.get("xd", 0)), nt_tuned),
-                                       _xd_policy(M, int(e.get("xd_glu", 0)), nt_tuned),
-                                       int(e.get("stream", 1)))
+                                       _xd_policy(M, int(e.get("xd_glu", 0)), nt_tuned))
+                if e.get("stream") == 0:
+                    kept.add((M, N, K, ldx))
         for v in pre.values():
             v.sort()
         _prefill.clear()
         _prefill.update(pre)
+        _kept.clear()
+        _kept.update(kept)
         _prefill_pick.clear()
         _routes.clear()
         _table = tab
@@ -164,7 +170,7 @@ def set_enabled(on: bool) -> None:
 
 # ------------------------------------------------------------------ routing
 def _decode_entry(M: int, N: int, K: int,
-                  ldx: int) -> tuple[int, tuple[int, int, int, int, int, int]] | None:
+                  ldx: int) -> tuple[int, tuple[int, int, int, int, int]] | None:
     """(tuned bucket, entry) for a decode-sized shape, None for torch's (hipBLASLt heuristic)
     path.  The tuner measured every (model shape, DECODE_BUCKETS M) and kept an entry only
     where something beat the heuristic pick, so a bucket without an entry means "the
@@ -228,12 +234,12 @@ def _resolve(M: int, N: int, K: int, ldx: int) -> tuple[str, int]:
         return ("w4", 0) if _w4_long(M, N, K) else ("torch", 0)
     found = _decode_entry(M, N, K, ldx)
     # the rule goes ahead of the table, but for entries that were measured faster ("stream": 0)
-    if ldx % 8 == 0 and stream_ok(M, N, K) and (found is None or found[1][5]):
+    if ldx % 8 == 0 and stream_ok(M, N, K) and (found is None or (found[0], N, K, ldx) not in _kept):
         return ("skinny", STREAM)
     if found is None:
         v = skinny_variant(M, N, K, ldx)
         return ("skinny", v) if v else ("torch", 0)
-    _, (algo, sk, midm, xd, _, _) = found
+    _, (algo, sk, midm, xd, _) = found
     if algo < 0 and not (sk or midm or xd):
         return ("torch", 0)  # measured: the library's heuristic pick beat every candidate
     if sk and M <= SKINNY_MAX_M and skinny_supports(sk, M, N, K, ldx):
