@@ -563,6 +563,16 @@ DRTC_DEVICE void sample_topp_full(SampShared& s, int* out_tokens, const unsigned
     });
     float A, F;
     block_sum2(s, a_t, f_t, A, F);
+    if (A != A || F != F) {  // NaNs among the logits: once more without them
+      a_t = f_t = 0.f;
+      for_row<U>(lr, V, vec, [&](int, unsigned short b) {
+        const unsigned key = ord16(b);
+        const float w = bits2f(b) > -INFINITY ? __expf((bits2f(b) - m) * inv_t) : 0.f;
+        a_t += key > kj ? w : 0.f;
+        f_t += key > t ? w : 0.f;
+      });
+      block_sum2(s, a_t, f_t, A, F);
+    }
     if (A < P) {  // token j is inside the nucleus
       if (tid == 0) out_tokens[row] = j;
       return;

@@ -561,17 +561,18 @@ def test_sample_topk_tokens(hipk, k, ties):
 
 
 @pytest.mark.parametrize("V", [1500, 1501, 40000])
-@pytest.mark.parametrize("k", [1, 64, 128, 129, 300, 1000])
+@pytest.mark.parametrize("k", [0, 1, 64, 128, 129, 300, 1000])
 @pytest.mark.parametrize("nans", [0.01, 0.6, 0.999])
-def test_sample_topk_skips_nans(hipk, V, k, nans):
+def test_sample_skips_nans(hipk, V, k, nans):
     """NaNs of either sign are never drawn: the tokens of the same rows with -inf in their place, also where
-    fewer than k numbers are left, rows of +inf among them; -1 where none is left; always a token of the row."""
+    fewer than k numbers are left (k 0: over the whole row, finite), rows of +inf among them; -1 where none is left;
+    always a token of the row."""
     B = 24
     g = torch.Generator().manual_seed(V + k)
     lg = torch.randn(B, V, generator=g) * 3
     bad = torch.rand(B, V, generator=g) < nans
     bad[:, 7] = False
-    lg[3, 5] = lg[4, 7] = float("inf")
+    lg[3, 5] = lg[4, 7] = float("inf") if k else 300.0
     bad[3, 5] = False
     lg[:, 11] = float("-inf")
     bad[20], lg[21], bad[22, 100:], lg[22, :100] = True, float("-inf"), True, float("-inf")
@@ -580,7 +581,8 @@ def test_sample_topk_skips_nans(hipk, V, k, nans):
     neg = (torch.rand(B, V, generator=g) < 0.5) & bad
     lg = lg.view(torch.int16).masked_fill(neg, -0x40).view(torch.bfloat16).to(DEV)  # 0xffc0
     temp = torch.linspace(0.3, 1.5, B)
-    temp[10], temp[11], temp[12] = float("nan"), float("inf"), 1e-45
+    if k:
+        temp[10], temp[11], temp[12] = float("nan"), float("inf"), 1e-45
     top_p = torch.where(torch.arange(B) % 3 == 0, 1.0, 0.2 + 0.7 * torch.rand(B, generator=g)).to(DEV)
     kk = torch.full((B,), k, dtype=torch.int32, device=DEV)
     for step in (1, 2):
@@ -590,7 +592,7 @@ def test_sample_topk_skips_nans(hipk, V, k, nans):
         assert torch.equal(got, run(clean, temp))
         assert (got[20:23] == -1).all()
         greedy = run(lg, torch.zeros(B))
-        assert greedy[20] == -1 and int(got[3]) == 5 and int(got[4]) == 7 and got[10] == greedy[10]
+        assert greedy[20] == -1 and int(got[3]) == 5 and int(got[4]) == 7 and (got[10] == greedy[10] or not k)
         live = [b for b in range(B) if b not in (20, 21, 22)]
         assert ((got[live] >= 0) & (got[live] < V)).all()
         assert (clean.cpu()[live, got[live].long()] > float("-inf")).all()
