@@ -22,6 +22,8 @@ int configure_kernels() {
   if (e) return e;
   e = configure_memory();
   if (e) return e;
+  e = configure_ring_moe();
+  if (e) return e;
   return configure_gemm_xd();
 }
 }  // namespace drtc

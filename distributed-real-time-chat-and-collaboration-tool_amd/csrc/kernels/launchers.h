@@ -202,6 +202,13 @@ int stream_moe_tiles(int rows_e, int H, int I, bool glu);
 int launch_stream_moe(void* y, const void* x, const void* w, int N, int K, int ldx, int ldy, int mt, int act,
                       float limit, int64_t w_stride, const int* tok, const int* expert, const int* row0,
                       const int* rows, const int* n, hipStream_t st);
+// ... with up to kRingRows rows to a table entry (moe_ring.hip, moe.hip variant 6)
+constexpr int kRingRows = 128;
+bool ring_moe_ok(int T, int P, int H, int I, bool glu);
+int launch_ring_moe(void* y, const void* x, const void* w, int x_rows, int N, int K, int ldx, int ldy, int act, float limit,
+                    int64_t w_stride, const int* tok, const int* expert, const int* row0, const int* rows, const int* n,
+                    int entries, hipStream_t st);
+int configure_ring_moe();
 // medium-M decode GEMM (gemm_midm.hip)
 int64_t midm_slab_bytes(int M, int N, int S);
 int launch_midm_gemm(void* y, const void* x, const void* w, const void* res, int M, int N,

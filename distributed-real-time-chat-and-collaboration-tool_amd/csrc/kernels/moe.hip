@@ -1029,21 +1029,30 @@ int launch_moe(void* out, const void* x, const void* router_logits, const void* 
   const int P = T * k;
   // GEMM structure: 0 = 128-row 2-barrier (small tiles, decode), 1 = 128-row
   // 3-stage pipeline, 2 = 256-row 3-stage pipeline, 5 = gemm_stream's form for a few rows per expert
-  // (weights straight to registers), 3 = gemm_xd grouped mode (gate_up with
-  // the GLU in its epilogue and down, forms gu_form / dn_form; 0 = by rows per expert);
+  // (weights straight to registers), 6 = up to about a hundred rows per expert (moe_ring.hip),
+  // 3 = gemm_xd grouped mode (gate_up with the GLU in its epilogue and down, forms gu_form / dn_form;
+  // 0 = by rows per expert);
   // -1 = pick by rows per expert (scripts/moe_bench.py, Mixtral shapes)
   const int rows_e = P / e_local;
   const bool auto_v = variant < 0;
   // variant 4 from one 256-row tile per expert (gemm_w4's persistent 256 x 256 tiles over
   // expert-ordered rows; Mixtral shapes, profiles/r6j: 770 / 917 / 1061 TF/s at T = 1024 /
-  // 2048 / 4096 against 703 / 841 / 1019 on variant 3), gemm_xd's grouped forms from ~a
-  // 96-row tile
+  // 2048 / 4096 against 703 / 841 / 1019 on variant 3)
   const int stream_mt = opt.f32 ? 0 : stream_moe_tiles(rows_e, H, I, glu);
-  // ... below it where an expert's matrix is large (us of a layer, variants 1 / 3: 8 x 4096 x 14336, 16
-  // tokens 526 / 475, 256 tokens 561 / 535; 20 x 2048 x 3584 178 / 159; 16 x 2048 x 1792 102 / 107)
-  if (auto_v)
-    variant = rows_e >= kMoeW4Rows ? 4 : rows_e >= 96 ? 3 : stream_mt ? 5 : (int64_t)H * I >= 6 << 20 ? 3 : 1;
-  if (variant > 5 || (variant == 5 && !stream_mt)) return -1;
+  // ... below it the ring, to where most experts still fit one of its entries (100 rows 92 / 121 of variant 3, 128
+  // rows 134 / 123), but for a few rows per expert where gemm_stream's form takes the sizes: fewer pairs than experts (us of a layer,
+  // variants 5 / 6: 16 x 2048 x 1792, 1 token 30.5 / 46.0, 2 39.6 / 48.6; 4 61.9 / 59.1), and wide experts, gated (16 x 4096
+  // x 3584, 13 tokens 226.6 / 229.1) or with a row each (20 x 4096 x 3584, 8 tokens 157.0 / 158.5; 16 197 / 187).  A
+  // few of many large experts elsewhere: variant 3 (8 x 4096 x 14336, 1 token 156 / 175; 2 250 / 241)
+  const bool ring_ok = !opt.f32 && ring_moe_ok(T, P, H, I, glu), wide = H > 2048 || I > 2048;
+  if (auto_v) {
+    if (rows_e >= kMoeW4Rows) variant = 4;
+    else if (stream_mt == 1 && (rows_e == 0 || (wide && (glu || rows_e < 2)))) variant = 5;
+    else if (ring_ok && rows_e <= 104 && (4 * P > e_local || (int64_t)H * I < 6 << 20)) variant = 6;
+    // shapes past the ring's offsets, and sizes between it and gemm_w4
+    else variant = rows_e >= 96 || (int64_t)H * I >= 6 << 20 ? 3 : 1;
+  }
+  if (variant > 6 || (variant == 5 && !stream_mt) || (variant == 6 && !ring_ok)) return -1;
   // variant 4: the persistent GEMM's prologue stages two K tiles; the down reduction is I
   if (variant == 4 && (H / 64 < 2 || I % (glu ? 128 : 256) || I / 64 < 2 || H % 256)) {
     if (!auto_v) return -1;
@@ -1090,7 +1099,7 @@ int launch_moe(void* out, const void* x, const void* router_logits, const void* 
     }
   }
   const int bm = variant == 3 ? 128 * ((gu_form % 1000) / 100)
-                              : (variant == 2 || variant == 4 ? 256 : variant == 5 ? 16 * stream_mt : 128);
+                              : (variant == 2 || variant == 4 ? 256 : variant == 5 ? 16 * stream_mt : variant == 6 ? kRingRows : 128);
   const int max_tiles = (P + bm - 1) / bm + e_local;
   // workspace carve (all 256-B aligned)
   auto align = [](int64_t v) { return (v + 255) & ~int64_t(255); };
@@ -1218,6 +1227,13 @@ int launch_moe(void* out, const void* x, const void* router_logits, const void* 
     if (!e)
       e = launch_stream_moe(zbuf, hbuf, w_dn, H, I, I, H, stream_mt, 4, 0.f, (int64_t)H * I, nullptr, t_e, t_r0, t_n,
                             n_tiles, st);
+    if (e) return e;
+  } else if (variant == 6) {
+    int e = launch_ring_moe(hbuf, x, w_gu, T, I, H, H, I, act, opt.limit, (int64_t)up_rows * H, sorted_tok, t_e,
+                            t_r0, t_n, n_tiles, e_local, st);
+    if (!e)
+      e = launch_ring_moe(zbuf, hbuf, w_dn, P, H, I, I, H, 4, 0.f, (int64_t)H * I, nullptr, t_e, t_r0, t_n,
+                          n_tiles, e_local, st);
     if (e) return e;
   } else if (variant == 0) {
     hipLaunchKernelGGL((glu ? moe_gemm_kernel<0> : moe_gemm_kernel<2>), g_gu, dim3(256), 0, st, hbuf,

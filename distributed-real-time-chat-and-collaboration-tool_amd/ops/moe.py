@@ -37,8 +37,9 @@ MAX_TOP_K, MAX_GROUPS = 16, 64  # of the routing kernel
 # (csrc/kernels/gemm_xd.hip: XCD-partitioned tiles, GLU epilogue, split-K, non-temporal
 # weights where an expert's rows fit one tile), 4 = token rows gathered into expert order, then
 # gemm_w4's grouped persistent 256 x 256 form (csrc/kernels/gemm_w4.hip; prefill-sized rows per
-# expert), 5 = weights streamed past a few rows per expert (csrc/kernels/gemm_stream.hip), -1 = by rows
-# per expert (4 from 256 rows per expert, 3 from 96, below 5 where it takes the sizes).
+# expert), 5 = weights streamed past a few rows per expert (csrc/kernels/gemm_stream.hip), 6 = weights and
+# rows through an LDS ring (csrc/kernels/moe_ring.hip), -1 = by rows per expert (4 from 256 rows per
+# expert, 6 up to 104, 3 in between; 5 for the fewest).
 MOE_GEMM_VARIANT = int(os.environ.get("DRTC_MOE_VARIANT", "-1"))
 # gemm_xd forms of variant 3 (mt * 100 + nf * 10 + splitk, + 1000 non-temporal; 0 = by rows
 # per expert, csrc/kernels/moe.hip launch_moe)

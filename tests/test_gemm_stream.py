@@ -302,3 +302,47 @@ def test_long_k_prefill_route(hipk, M, N, K, kind):
     rows = torch.tensor([0, 255, 256, M // 2, M - 1], device="cuda")
     want = x[rows].double() @ w.double().t()
     assert ((ops.linear(x, w)[rows].double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-3).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,I,E,k,act,e_off,T", [
+    (128, 64, 4, 2, "silu", 0, 1),       # one K tile of the down projection, fewer columns than workgroups
+    (256, 192, 8, 2, "gelu_tanh", 0, 9),
+    (384, 320, 8, 4, "clamped", 4, 70),  # some of the experts on this rank
+    (2048, 1792, 16, 4, "silu", 0, 128), (2048, 1792, 20, 4, "relu2", 0, 129),  # tiles of 3 fragments and of 4
+    (1024, 640, 5, 3, "relu2", 0, 170),  # entries of all 128 rows, and of a few
+    (128, 128, 256, 4, "relu2", 0, 500),  # more entries than workgroups: runs over several of them
+    (192 * 2, 64, 130, 8, "silu", 0, 300),  # one workgroup to an entry, several tiles each
+])
+def test_ring_experts(hipk, H, I, E, k, act, e_off, T):
+    """The experts' ring at the edges of its tiles, entries and runs, against the fp32 oracle; the same bits
+    in replays of a graph, and with no row for any expert of this rank."""
+    e_local = E - e_off
+    g = torch.Generator(device="cuda").manual_seed(T + E)
+    x = torch.randn(T, H, device="cuda", generator=g).to(torch.bfloat16)
+    lg = torch.randn(T, E, device="cuda", generator=g)
+    lg[::3, e_off] = 9.0
+    n_in = I if act == "relu2" else 2 * I
+    w_in = (torch.randn(e_local, n_in, H, device="cuda", generator=g) * 0.02).to(torch.bfloat16)
+    w_out = (torch.randn(e_local, H, I, device="cuda", generator=g) * 0.02).to(torch.bfloat16)
+    ws = ops.moe.make_workspace(T, H, I, e_local, k, "cuda")
+    G.gemm_workspace(x.device)
+
+    def run():
+        return ops.fused_moe(x, lg, w_in, w_out, k, act, E, e_off, ws, variant=6, limit=0.9)
+
+    y = run()
+    want = ops.fused_moe_ref(x, lg, w_in, w_out, k, act, e_off, limit=0.9).double()
+    # both round the hidden rows and the experts' outputs to bf16: a few of them differ by one unit
+    assert (y.double() - want).norm() <= 2e-3 * want.norm() + 1e-6
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        z = run()
+    for _ in range(3):
+        x.normal_(generator=g)
+        lg.normal_(generator=g)
+        graph.replay()
+        assert torch.equal(z, run())
+    if e_off >= k:  # every token to the other rank
+        lg[:, :e_off] += 100.0
+        assert not run().any()
