@@ -483,14 +483,26 @@ __global__ __launch_bounds__(kXdThreads, 1) void gemm_xd_kernel(XdParams p) {
   f32x4 acc[FA][NF];  // written first by the K tile 0 MFMAs (onto a zero C operand)
 
   // ---- prologue: K tiles 0 .. S-1 into the S stages (the launcher guarantees nk > S)
+  // One row tile: every workgroup has its own columns of W, and each starts its K walk at another K tile.
+  // In step they would ask few memory channels at a time where rows of W lie a multiple of 4 KB apart
+  // (28672 x 4096 gated, 64 rows, tile 128 x 128: 47.5 -> 40.1 us; 32000 x 2048 28.1 -> 24.3; 256 x 128,
+  // 160 rows 55.5 -> 54.1).  Row tiles that share columns stay in step for the L2's sake (4096 x 4096, 1024 rows, each on
+  // its own: 39.6 -> 42.4).
+  unsigned kt = !G && p.tiles_m == 1 && !C::SPLIT ? (b >> 3) % nk : 0;
+  auto next_k = [&] {
+    const unsigned k = kt * 128u;
+    kt = kt + 1 == nk ? 0 : kt + 1;
+    return k;
+  };
 #pragma unroll
   for (int u = 0; u < C::S; ++u) {
+    const unsigned k = next_k();
 #pragma unroll
     for (int i = 0; i < C::DA; ++i)
-      xd_dma(d.lds_a + u * C::STAGE + 1024 * i, d.va[i], d.ra, (unsigned)u * 128u);
+      xd_dma(d.lds_a + u * C::STAGE + 1024 * i, d.va[i], d.ra, k);
 #pragma unroll
     for (int i = 0; i < C::DB; ++i)
-      xd_dma<C::NT>(d.lds_b + u * C::STAGE + 1024 * i, d.vb[i], d.rb, (unsigned)u * 128u);
+      xd_dma<C::NT>(d.lds_b + u * C::STAGE + 1024 * i, d.vb[i], d.rb, k);
   }
   xd_vmcnt<(C::S - 1) * C::D>();
   xd_barrier();
@@ -499,12 +511,12 @@ __global__ __launch_bounds__(kXdThreads, 1) void gemm_xd_kernel(XdParams p) {
 
   // ---- main loop: tile t in stage cur; its half 1 DMAs tile t + S into the same stage
   xd_tile<C, true, true, C::S - 2, true>(acc, fa0, fb0, fa1, fb1, lds, 0, C::STAGE % C::LDS,
-                                         (unsigned)C::S * 128u, f, d);
+                                         next_k(), f, d);
   int cur = C::STAGE % C::LDS;
   for (int t = 1; t + C::S < nk; ++t) {
     const int nxt = cur + C::STAGE == C::LDS ? 0 : cur + C::STAGE;
     xd_tile<C, true, true, C::S - 2>(acc, fa0, fb0, fa1, fb1, lds, cur, nxt,
-                                     (unsigned)(t + C::S) * 128u, f, d);
+                                     next_k(), f, d);
     cur = nxt;
   }
   xd_tail<C, C::S - 2>(acc, fa0, fb0, fa1, fb1, lds, cur, f, d);

@@ -233,6 +233,9 @@ def _resolve(M: int, N: int, K: int, ldx: int) -> tuple[str, int]:
             return ("lt", a)
         return ("w4", 0) if _w4_long(M, N, K) else ("torch", 0)
     found = _decode_entry(M, N, K, ldx)
+    wide = wide_form(M, N, K)
+    if wide and not (found is not None and found[1][3]):  # (entries of gemm_xd: measured against its other forms)
+        return ("xd", wide)
     # the rule goes ahead of the table, but for entries that were measured faster ("stream": 0)
     if ldx % 8 == 0 and stream_ok(M, N, K) and (found is None or (found[0], N, K, ldx) not in _kept):
         return ("skinny", STREAM)
@@ -254,6 +257,30 @@ def _resolve(M: int, N: int, K: int, ldx: int) -> tuple[str, int]:
                 return ("lt", algo)
     v = skinny_variant(M, N, K, ldx)
     return ("skinny", v) if v else ("torch", 0)
+
+
+def wide_form(M: int, N: int, K: int) -> int:
+    """gemm_xd form of a plain product of 24 .. 256 rows, one row tile, whose columns fill the CUs in whole
+    rounds: vocabulary heads above all.  Each workgroup walks K from another tile (gemm_xd.hip), which neither
+    the library nor the streaming GEMM does.  us, their best / this: 32000 x 2048, 24 rows 26.5 / 23.4, 64 32.6 / 24.3, 128
+    33.3 / 27.2, 192 36.0 / 34.9; 32000 x 4096, 17 46.0 / 47.5, 24 47.3 / 45.9, 64 58.1 / 47.2; 64128 x 4096, 32 91.2 /
+    82.7, 96 115.5 / 96.6; 128256 x 2048, 144 130 / 119; 57344 x 8192, 64 190 / 168, 192 235 / 203.  Rounds that are not
+    full: 50176 columns (0.77), 32 rows 39.4 / 40.0, 192 53.4 / 53.8; 27648 (0.84) 43.9 / 35.9, 61.4 / 55.2.  Short K:
+    64000 x 1024, 64 rows 27.8 / 29.3.  Above 128 rows tiles of 256 x 256, or 256 x 128 in one round (64128 columns, not a
+    multiple of 256, 256 rows 126.9 / 131.2)."""
+    if not (_xd_enabled and _enabled and 24 <= M <= 256 and K >= 2048):
+        return 0
+
+    def full(columns):
+        tiles = N // columns
+        return N % columns == 0 and tiles >= 0.84 * 256 * -(-tiles // 256)
+
+    if M <= 128:
+        form = 1141 if full(128) else 0
+    else:
+        form = 1281 if full(256) else 1241 if full(128) and N <= 256 * 128 else 0
+    form = form if _xd_nt else form % 1000
+    return form if form and xd_supported(M, N, K, form) else 0
 
 
 # DRTC_XD_BIG_M=0: decode batches above DECODE_MAX_M ignore tuned gemm_xd entries (A/B knob)

@@ -346,3 +346,26 @@ def test_ring_experts(hipk, H, I, E, k, act, e_off, T):
     if e_off >= k:  # every token to the other rank
         lg[:, :e_off] += 100.0
         assert not run().any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,form", [(23, 32768, 2048, 0), (24, 32768, 2048, 1141), (128, 27648, 2112, 1141),
+                                       (129, 27648, 2112, 1241), (256, 65536, 2048, 1281), (64, 32768, 1984, 0),
+                                       (64, 50176, 2048, 0), (129, 64128, 2048, 0), (65, 64128, 2048, 1141)])
+def test_wide_products(hipk, M, N, K, form):
+    """Both sides of the rule for wide plain products, and what linear then gives: every workgroup starts its walk
+    of K (33 tiles of 64 in two cases) elsewhere.  bf16 rounding of the result and fp32 sums of K products."""
+    G.reset()
+    assert G.wide_form(M, N, K) == form
+    kind = G.route(M, N, K, K)
+    assert not form or kind[0] == "xd"
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+    w = (torch.randn(N, K, device="cuda", generator=g) / K ** 0.5).to(torch.bfloat16)
+    got, want = ops.linear(x, w).double(), x.double() @ w.double().t()
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all()
+    if form:
+        glu = ops.gemm.xd_gemm(x, w[:N // 512 * 512], "silu", form=form)
+        a, b = (x.double() @ w[:N // 512 * 512].double().t()).chunk(2, -1)
+        want = a * torch.sigmoid(a) * b
+        assert ((glu.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all()
