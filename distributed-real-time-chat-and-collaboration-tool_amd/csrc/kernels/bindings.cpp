@@ -32,6 +32,11 @@ PYBIND11_MODULE(_hipk, m) {
                                       P<void>(w), rows, H, eps, x_stride,
                                       out_stride, res_stride, gemma, S(st));
         });
+  m.def("rmsnorm_parts", [](u64 out, u64 residual, u64 parts, int S_, u64 w, int rows, int H, float eps, int out_stride,
+                            int res_stride, bool gemma, u64 st) {
+    return drtc::launch_rmsnorm_parts(P<void>(out), P<void>(residual), P<const float>(parts), S_, P<const void>(w), rows, H,
+                                      eps, out_stride, res_stride, gemma, S(st));
+  });
   m.def("act_glu", [](u64 out, u64 gu, int64_t T, int I, int gu_stride, int act,
                       float limit, u64 st) {
     return drtc::launch_act_glu(P<void>(out), P<void>(gu), T, I, gu_stride, act, limit, S(st));
@@ -91,9 +96,9 @@ PYBIND11_MODULE(_hipk, m) {
                   int k, int e_off, int e_local, int act, u64 ws, int64_t ws_bytes, int variant,
                   int gu_form, int dn_form, u64 slab, int64_t slab_bytes, u64 counters,
                   int n_counters, int logit_ts, int logit_es, int f32, int logits_f32, int groups,
-                  int keep, float limit, u64 stream, u64 y, int ldy, int W, u64 st) {
+                  int keep, float limit, u64 stream, u64 y, int ldy, int W, int y_parts, u64 st) {
     const drtc::MoeOptions opt{f32, logits_f32, groups, keep, limit, P<float>(stream),
-                               P<const void>(y), ldy, W};
+                               P<const void>(y), ldy, W, y_parts};
     return drtc::launch_moe(P<void>(out), P<const void>(x), P<const void>(logits),
                             P<const void>(w_gu), P<const void>(w_dn), T, H, I, E, k, e_off,
                             e_local, act, P<void>(ws), ws_bytes, variant, gu_form, dn_form,
@@ -201,9 +206,9 @@ PYBIND11_MODULE(_hipk, m) {
   });
   m.def("stream_moe_tiles", &drtc::stream_moe_tiles);  // (rows per expert, H, I, gated)
   m.def("midm_gemm", [](u64 y, u64 x, u64 w, u64 res, int M, int N, int K, int ldx, int ldy,
-                        int ldr, int epi, int splits, u64 slab, int64_t slab_bytes, u64 st) {
+                        int ldr, int epi, int splits, int nf, u64 slab, int64_t slab_bytes, u64 st) {
     return drtc::launch_midm_gemm(P<void>(y), P<const void>(x), P<const void>(w),
-                                  P<const void>(res), M, N, K, ldx, ldy, ldr, epi, splits,
+                                  P<const void>(res), M, N, K, ldx, ldy, ldr, epi, splits, nf,
                                   P<void>(slab), slab_bytes, S(st));
   });
   m.def("midm_slab_bytes",

@@ -117,6 +117,10 @@ void bind_hybrid(py::module_& m) {
     return drtc::launch_dyt(f32, P<void>(out), P<float>(h), P<void>(y), ldy, P<const int>(ids),
                             P<void>(embed), P<float>(w), P<float>(b), alpha, rows, W, S(st));
   });
+  m.def("dyt_parts", [](u64 out, u64 h, u64 parts, int n, u64 w, u64 b, float alpha, int rows, int W, u64 st) {
+    return drtc::launch_dyt_parts(P<void>(out), P<float>(h), P<const float>(parts), n, P<const float>(w), P<const float>(b),
+                                  alpha, rows, W, S(st));
+  });
   m.def("act_glu_f32", [](u64 out, u64 gu, int64_t T, int I, int stride, int act, float limit,
                           u64 st) {
     return drtc::launch_act_glu_f32(P<float>(out), P<float>(gu), T, I, stride, act, limit, S(st));

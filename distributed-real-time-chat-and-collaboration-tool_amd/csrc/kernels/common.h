@@ -49,6 +49,28 @@ DRTC_DEVICE float wave_max(float v) {
   return v;
 }
 
+// v += 8 consecutive columns of the S <= 8 fp32 partial sums [S][..] of a product (gemm_midm.hip), in order;
+// every load is under way before the first add.
+constexpr int kMaxParts = 8;
+DRTC_DEVICE void add_parts(float (&v)[8], const float* p, int64_t stride, int S) {
+  f32x4 a[kMaxParts], b[kMaxParts];
+#pragma unroll
+  for (int s = 0; s < kMaxParts; ++s)
+    if (s < S) {
+      a[s] = *reinterpret_cast<const f32x4*>(p + s * stride);
+      b[s] = *reinterpret_cast<const f32x4*>(p + s * stride + 4);
+    }
+#pragma unroll
+  for (int s = 0; s < kMaxParts; ++s)
+    if (s < S) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        v[j] += a[s][j];
+        v[4 + j] += b[s][j];
+      }
+    }
+}
+
 // Barrier that waits for this wave's LDS traffic only: loads from memory stay in flight.
 DRTC_DEVICE void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");

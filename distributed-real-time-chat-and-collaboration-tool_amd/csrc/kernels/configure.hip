@@ -24,6 +24,8 @@ int configure_kernels() {
   if (e) return e;
   e = configure_ring_moe();
   if (e) return e;
+  e = configure_gemm_midm();
+  if (e) return e;
   return configure_gemm_xd();
 }
 }  // namespace drtc

@@ -1,170 +1,191 @@
-// Medium-M projection GEMM for decode batches 17..256: y[M, N] = x[M, K] @ W[N, K]^T,
-// bf16 in/out, fp32 accumulation, 16x16x32 bf16 MFMA.
+// Medium-M projection GEMM (gfx950): y[M, N] = epi(x[M, K] @ W[N, K]^T) for up to 256 rows, bf16 in and out,
+// fp32 accumulation, 16x16x32 MFMA.
 //
-// Regime: at these M the weights are read once per call and every weight byte is used
-// M times - far below the MFMA's arithmetic intensity - so the kernel is a weight
-// stream, and the library's 128-256-row output tiles leave most CUs idle on the
-// N = 4096-6144 projections (hipBLASLt at M = 128: o / qkv / down stream W at 2.3-2.4
-// TB/s, scripts/midm_probe.py).  Here:
-//   * a 256-thread workgroup owns 128 rows of W (4 waves x 2 MFMA row tiles) and one
-//     K-split of them; W goes straight from HBM to VGPRs through a D-chunk register
-//     ring (64-k chunks, compile-time ring slots), one pass, 16-byte loads;
-//   * the x chunk [0:M_pad, 64 k] is staged once per workgroup in LDS (double buffer,
-//     rows padded to 72 elements) and shared by the 4 waves; a wave multiplies each of
-//     its W fragments by MG x fragments (MG = ceil(M/16) column groups);
-//   * K is split over S workgroups so the grid fills every CU; splits write fp32
-//     partial tiles to a slab and `midm_reduce_kernel` sums them in fixed order and
-//     applies the epilogue (store, residual add, SiLU/GELU-gated [gate | up]).  With
-//     S = 1 and a plain / residual epilogue the GEMM kernel writes bf16 directly.
-//     No atomics or fences: the kernel boundary orders slab writes and reads, so the
-//     pair replays inside a hipGraph.
-// Operand mapping (as gemv.hip's MFMA form): A = W rows (lane row l & 15, k = 8 (l >> 4)
-// .. +8 of the 32-k substep), B = x^T (lane column m = l & 15 of the column group,
-// same k), so lane l holds D[n = 4 (l >> 4) + r][m = l & 15], r = 0..3: 4
-// consecutive output columns n of one row m (16-byte stores).
-#include "common.h"
+// What bounds it: W is read once (5.3 - 6 TB/s), and a CU takes in 50 - 70 GB/s of operands, from L2 as from
+// HBM, however many loads are in flight; less where both mix.  A tile of all M rows and TN columns over a K
+// slice costs its CU (M + TN) x slice x 2 bytes, so:
+//   * a tile holds all rows, in steps of 32 (rows past M are out of the descriptor's range: no memory access),
+//     and 64 or 128 columns of W;
+//   * K is cut into slices until the tiles fill the CUs (ops/gemm.py parts_form); the slices' fp32 tiles go
+//     to a slab, and the sum is taken by the kernel that reads y next - a residual add and norm - or by
+//     midm_reduce_kernel.  The kernel boundary orders them: no atomics, no waiting.  A 32-bit part is written and
+//     read instead of a bf16 row: 1 - 2 us against 3 - 8 for a pass, and one rounding less;
+//   * x and W pass through LDS (LDS-DMA, a ring of 64-deep K tiles, W non-temporal: every byte enters one CU
+//     once).  XCD x takes a contiguous range of the slice-major tile order, so its part of x stays in its L2, and
+//     its workgroups start their K walk at different tiles (rows of W a multiple of 4 KB apart, walked in step, ask few
+//     memory channels at a time: 32000 x 2048, 64 rows 30.6 -> 24.9 us);
+//   * 8 waves: 2 x 2 over the tile, times the two 32-deep halves of a K tile - a wave's fragments are read
+//     once for 16 FA x 16 NF outputs, and 8 waves issue loads.  The halves meet in LDS at the end.
+// us of the table's kernel / of the slices' sums: 4096 x 4096, 16 rows 11.1 / 8.5, 64 14.1 / 9.9, 160 19.5 / 15.0; 4096 x 14336
+// 24.2 / 19.8, 28.3 / 22.7, 39.0 / 30.8; 2048 x 7168 12.3 / 7.6, 22.0 / 9.1, 24.2 / 14.1.
+// Operands: MFMA A = W rows, B = x rows, so lane l holds 4 consecutive columns n = 4 (l >> 4) .. of the row
+// m = l & 15.  LDS rows are 128 bytes, 16-byte chunk c of row r at c ^ ((r >> 1) & 7): no bank conflicts.
+#include "lds_dma.h"
 #include "launchers.h"
 
 namespace drtc {
 namespace {
 
-constexpr int kMidThreads = 256;
-constexpr int kMidRows = 128;   // W rows per workgroup (4 waves x 2 tiles x 16)
-constexpr int kMidKC = 64;      // k per chunk
-constexpr int kMidXRow = 72;    // LDS x row stride (elements): 144 B breaks bank aliasing
-// W register ring depth (chunks in flight per wave): 4, or 2 where the accumulators of
-// 14-16 column groups leave no room for 4 (no scratch)
-template <int MG>
-constexpr int mid_depth() { return 4; }  // 8 measured slower (VGPRs, fewer valid splits)
+constexpr int kMidThreads = 512;
+enum { MID_STORE = 0, MID_RESIDUAL = 1, MID_SILU = 2, MID_GELU = 3, MID_SLAB = 4 };
 
-enum { MID_STORE = 0, MID_RESIDUAL = 1, MID_SLAB = 2 };
+struct MidArgs {
+  bf16_t* y;
+  float* slab;
+  const bf16_t* x;
+  const bf16_t* w;
+  const bf16_t* res;
+  int M, N, K, ldx, ldy, ldr;  // N: rows of W
+  int out;
+  int tiles, slices, per_xcd;
+};
 
-// Occupancy: 2 workgroups per CU up to 8 column groups (M <= 128); beyond that (the
-// 129-256-row buckets of the 70B decode) the 2 x MG accumulators need the AGPR half of the
-// register file and the x double buffer is up to 74 KiB of LDS, so one workgroup per CU.
-template <int MG>
-constexpr int mid_wgs_per_cu() { return MG > 8 ? 1 : 2; }
+template <int FA_, int NF_>
+struct MidCfg {
+  static constexpr int FA = FA_, NF = NF_;     // 16-row and 16-column fragments of a wave
+  static constexpr int TM = 32 * FA, TN = 32 * NF;
+  static constexpr int BOFF = TM * 128, STAGE = BOFF + TN * 128;
+  static constexpr int ODD = FA % 2;           // waves 4 .. 7 have one load of x less: one out of range instead
+  static constexpr int DA = (FA + 1) / 2, DB = NF / 2, D = DA + DB;  // LDS-DMA per wave and K tile
+  static constexpr int FIT = (160 * 1024 - 1024 * ODD) / STAGE;
+  static constexpr int ST = FIT < 6 ? FIT : 6;
+  static constexpr int LDS = ST * STAGE + 1024 * ODD;
+  static_assert(FA * NF * 4096 <= LDS && ST >= 3, "the halves' exchange fits the ring");
+};
 
-template <int MG, int OUT>
-__global__ __launch_bounds__(kMidThreads, mid_wgs_per_cu<MG>()) void midm_kernel(
-    bf16_t* __restrict__ y, float* __restrict__ slab, const bf16_t* __restrict__ x,
-    const bf16_t* __restrict__ w, const bf16_t* __restrict__ res, int M, int N, int K,
-    int ldx, int ldy, int ldr, int n_blocks, int kps) {
-  constexpr int MP = MG * 16;
-  constexpr int kMidD = mid_depth<MG>();
-  __shared__ __attribute__((aligned(16))) bf16_t xs[2][MP * kMidXRow];
-  const int nb = blockIdx.x % n_blocks;
-  const int s = blockIdx.x / n_blocks;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int r = lane & 15, g = lane >> 4;
-  const int n0 = nb * kMidRows + wv * 32;
-  const int k_begin = s * kps;
-  const int nc = kps / kMidKC;
+template <class C, bool GLU>
+__global__ __launch_bounds__(kMidThreads, 1) void midm_kernel(MidArgs a) {
+  constexpr int FA = C::FA, NF = C::NF;
+  extern __shared__ __attribute__((aligned(16))) char mid_lds[];
+  const int b = blockIdx.x, item = (b & 7) * a.per_xcd + (b >> 3);
+  if (item >= a.tiles * a.slices) return;
+  const int slice = item / a.tiles, tile = item - slice * a.tiles;
+  const int nkt = a.K >> 6, kt0 = slice * nkt / a.slices, nk = (slice + 1) * nkt / a.slices - kt0;
+  constexpr int TNO = GLU ? C::TN / 2 : C::TN;  // output columns of a tile
+  const int n0 = tile * TNO, up = a.N / 2;
+  const int lane = threadIdx.x & 63, wv = wave_id_uniform();
+  const int kg = wv >> 2, wm = (wv >> 1) & 1, wn = wv & 1, r = lane & 15, g = lane >> 4;
 
-  // ---- W register ring: [slot][tile][substep] 16-B fragments
-  bf16x8 wr[kMidD][2][2];
-  const bf16_t* wp0 = w + (int64_t)(n0 + r) * K + k_begin + 8 * g;
-  const bf16_t* wp1 = wp0 + (int64_t)16 * K;
-  auto load_w = [&](bf16x8 (&dst)[2][2], int c) {
-    const int k = c * kMidKC;
-    dst[0][0] = load_bf16x8(wp0 + k);
-    dst[0][1] = load_bf16x8(wp0 + k + 32);
-    dst[1][0] = load_bf16x8(wp1 + k);
-    dst[1][1] = load_bf16x8(wp1 + k + 32);
-  };
-  // ---- x staging: MP rows x 64 k = MP * 8 16-B vectors, MG / 2 per thread
-  constexpr int XV = MP * 8 / kMidThreads;  // = MG / 2
-  static_assert(MG % 2 == 0 && XV >= 1, "MG must be even");
-  // x register ring of 2 chunks: chunk j is loaded at iteration j - 2 into slot j & 1 and
-  // written to LDS buffer j & 1 at iteration j - 1, so a whole iteration hides its latency
-  bf16x8 xr[2][XV];
-  auto load_x = [&](bf16x8 (&dst)[XV], int c) {
-    const int k = k_begin + c * kMidKC;
+  // ---- loads: an instruction fills 8 rows of 128 bytes; wave wv takes the groups wv, wv + 8, ..
+  const __amdgpu_buffer_rsrc_t ra = dma_rsrc(a.x + (int64_t)kt0 * 64);
+  const __amdgpu_buffer_rsrc_t rb = dma_rsrc(a.w + (int64_t)n0 * a.K + (int64_t)kt0 * 64);
+  const unsigned lds0 = (unsigned)(uintptr_t)(lds_ptr)mid_lds;
+  unsigned va[C::DA], vb[C::DB];
 #pragma unroll
-    for (int i = 0; i < XV; ++i) {
-      const int v = tid + i * kMidThreads;
-      const int m = v >> 3, kk = (v & 7) * 8;
-      if (m < M) {
-        dst[i] = load_bf16x8(x + (int64_t)m * ldx + k + kk);
-      } else {
+  for (int i = 0; i < C::DA; ++i) {
+    const int R = 8 * (wv + 8 * i) + (lane >> 3), c = (lane & 7) ^ ((R >> 1) & 7);
+    va[i] = R < C::TM && R < a.M ? (unsigned)(R * a.ldx * 2 + c * 16) : kNoRow;
+  }
 #pragma unroll
-        for (int j = 0; j < 8; ++j) dst[i][j] = f2bf(0.f);
-      }
+  for (int i = 0; i < C::DB; ++i) {
+    const int R = 8 * (wv + 8 * i) + (lane >> 3), c = (lane & 7) ^ ((R >> 1) & 7);
+    int src = R;
+    if constexpr (GLU) {  // fragments 2 j and 2 j + 1 of a wave: gate and up rows of the same columns
+      const int w = R / (16 * NF), j = R % (16 * NF) / 16;
+      src = w * 8 * NF + j / 2 * 16 + (R & 15) + (j & 1 ? up : 0);
+    }
+    vb[i] = (unsigned)src * (unsigned)(a.K * 2) + c * 16;
+  }
+  const int turn = (b >> 3) % nk;
+  auto load = [&](int t, int slot) {
+    const int kt = t + turn;
+    const unsigned at = lds0 + slot * C::STAGE, k = (unsigned)(kt < nk ? kt : kt - nk) * 128u;
+#pragma unroll
+    for (int i = 0; i < C::DB; ++i) dma16<true>(at + C::BOFF + 1024 * (wv + 8 * i), vb[i], rb, k);
+#pragma unroll
+    for (int i = 0; i < C::DA; ++i) {
+      unsigned dst = at + 1024 * (wv + 8 * i);
+      if (C::ODD && i == C::DA - 1 && wv >= 4) dst = lds0 + C::ST * C::STAGE;
+      dma16<false>(dst, va[i], ra, k);
     }
   };
-  auto store_x = [&](const bf16x8 (&src)[XV], int buf) {
+  int issued = 0, fill = 0;
+#pragma unroll 1
+  for (; issued < min(C::ST - 1, nk); ++issued, ++fill) load(issued, fill);
+
+  const int fx = (r >> 1) & 7, ch = ((4 * kg + g) ^ fx) * 16;
+  const char* xa = mid_lds + (16 * FA * wm + r) * 128 + ch;
+  const char* wa = mid_lds + C::BOFF + (16 * NF * wn + r) * 128 + ch;
+  f32x4 acc[FA][NF];
 #pragma unroll
-    for (int i = 0; i < XV; ++i) {
-      const int v = tid + i * kMidThreads;
-      const int m = v >> 3, kk = (v & 7) * 8;
-      store_bf16x8(&xs[buf][m * kMidXRow + kk], src[i]);
+  for (int i = 0; i < FA; ++i)
+#pragma unroll
+    for (int j = 0; j < NF; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  int at = 0;
+#pragma unroll 1
+  for (int t = 0; t < nk; ++t) {
+    wait_groups<C::D, C::ST - 2>(issued - t - 1);
+    // everyone's part of tile t is there, and everyone has read tile t - 1, whose stage is filled next
+    lds_barrier();
+    if (issued < nk) {
+      load(issued, fill);
+      ++issued;
+      fill = fill + 1 == C::ST ? 0 : fill + 1;
     }
-  };
-
-  f32x4 acc[2][MG];
+    bf16x8 fb[NF], fa[FA];
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+    for (int j = 0; j < NF; ++j) fb[j] = *reinterpret_cast<const bf16x8*>(wa + at + 2048 * j);
 #pragma unroll
-    for (int q = 0; q < MG; ++q) acc[t][q] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-  // The loop body is branch-free (nc is a multiple of kMidD, enforced by the launcher;
-  // prefetches past the last chunk re-load the last chunk instead of being skipped), so
-  // hipcc can count the loads still in flight: each chunk waits for its own W fragments
-  // only (counted vmcnt), not for the ring's younger loads (a conditional load made it
-  // emit vmcnt(0) before every chunk - one full HBM latency per 64-k chunk).
-  load_x(xr[0], 0);
+    for (int i = 0; i < FA; ++i) fa[i] = *reinterpret_cast<const bf16x8*>(xa + at + 2048 * i);
 #pragma unroll
-  for (int d = 0; d < kMidD; ++d) load_w(wr[d], d);
-  load_x(xr[1], min(1, nc - 1));
-  store_x(xr[0], 0);
-  __syncthreads();
-
-  static_assert(kMidD % 2 == 0, "ring phases must keep the x slot compile-time");
-  for (int c0 = 0; c0 < nc; c0 += kMidD) {
+    for (int i = 0; i < FA; ++i)
 #pragma unroll
-    for (int ph = 0; ph < kMidD; ++ph) {
-      const int c = c0 + ph;
-      {
-        const int buf = ph & 1;  // == c & 1 (c0 is a multiple of kMidD, which is even)
-        load_x(xr[buf], min(c + 2, nc - 1));  // slot of chunk c: stored last iteration
-        const bf16_t* xb = &xs[buf][0];
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub) {
-#pragma unroll
-          for (int q = 0; q < MG; ++q) {
-            const bf16x8 xf = load_bf16x8(xb + (q * 16 + r) * kMidXRow + sub * 32 + 8 * g);
-            acc[0][q] = mfma16(wr[ph][0][sub], xf, acc[0][q]);
-            acc[1][q] = mfma16(wr[ph][1][sub], xf, acc[1][q]);
-          }
-        }
-        load_w(wr[ph], min(c + kMidD, nc - 1));
-        store_x(xr[buf ^ 1], buf ^ 1);  // chunk c + 1, loaded an iteration ago
-        __syncthreads();
-      }
-    }
+      for (int j = 0; j < NF; ++j) acc[i][j] = mfma16(fb[j], fa[i], acc[i][j]);
+    at = at + C::STAGE == C::ST * C::STAGE ? 0 : at + C::STAGE;
   }
 
-  // ---- epilogue: lane holds rows n = n0 + 16 t + 4 g + 0..3 of column m = 16 q + r
+  // ---- the two halves of K: wave kg 0 gets the sums of the row fragments below FI, kg 1 the others
+  constexpr int FI = (FA + 1) / 2;
+  lds_barrier();  // everyone has read the last tile
+  {
+    f32x4* to = reinterpret_cast<f32x4*>(mid_lds) + (wv & 3) * (FA * NF * 64) + lane;
 #pragma unroll
-  for (int q = 0; q < MG; ++q) {
-    const int m = q * 16 + r;
-    if (m >= M) continue;
+    for (int i = 0; i < FA; ++i)
+      if ((i < FI) == (kg == 1))
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int n = n0 + 16 * t + 4 * g;
-      if constexpr (OUT == MID_SLAB) {
-        *reinterpret_cast<f32x4*>(slab + ((int64_t)s * M + m) * N + n) = acc[t][q];
-      } else {
-        f32x4 v = acc[t][q];
-        if constexpr (OUT == MID_RESIDUAL) {
-          const bf16x4 rv = *reinterpret_cast<const bf16x4*>(res + (int64_t)m * ldr + n);
+        for (int j = 0; j < NF; ++j) to[(i * NF + j) * 64] = acc[i][j];
+    lds_barrier();
 #pragma unroll
-          for (int j = 0; j < 4; ++j) v[j] += bf2f(rv[j]);
+    for (int i = 0; i < FA; ++i)
+      if ((i < FI) == (kg == 0))
+#pragma unroll
+        for (int j = 0; j < NF; ++j) acc[i][j] += to[(i * NF + j) * 64];
+  }
+
+#pragma unroll
+  for (int i = 0; i < FA; ++i) {
+    const int m = 16 * (FA * wm + i) + r;
+    if ((i < FI) != (kg == 0) || m >= a.M) continue;
+    if (a.out == MID_SLAB) {
+#pragma unroll
+      for (int j = 0; j < NF; ++j) {
+        const int n = GLU ? n0 + 8 * NF * wn + j / 2 * 16 + (j & 1 ? up : 0) : n0 + 16 * (NF * wn + j);
+        *reinterpret_cast<f32x4*>(a.slab + ((int64_t)slice * a.M + m) * a.N + n + 4 * g) = acc[i][j];
+      }
+    } else if constexpr (GLU) {
+#pragma unroll
+      for (int j = 0; j < NF; j += 2) {
+        bf16x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          o[e] = f2bf(a.out == MID_SILU ? glu_value<0>(acc[i][j][e], acc[i][j + 1][e], 0.f)
+                                        : glu_value<1>(acc[i][j][e], acc[i][j + 1][e], 0.f));
+        *reinterpret_cast<bf16x4*>(a.y + (int64_t)m * a.ldy + n0 + 8 * NF * wn + 8 * j + 4 * g) = o;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < NF; ++j) {
+        const int n = n0 + 16 * (NF * wn + j) + 4 * g;
+        f32x4 v = acc[i][j];
+        if (a.out == MID_RESIDUAL) {
+          const bf16x4 rv = *reinterpret_cast<const bf16x4*>(a.res + (int64_t)m * a.ldr + n);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] += bf2f(rv[e]);
         }
         bf16x4 o;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) o[j] = f2bf(v[j]);
-        *reinterpret_cast<bf16x4*>(y + (int64_t)m * ldy + n) = o;
+        for (int e = 0; e < 4; ++e) o[e] = f2bf(v[e]);
+        *reinterpret_cast<bf16x4*>(a.y + (int64_t)m * a.ldy + n) = o;
       }
     }
   }
@@ -185,6 +206,7 @@ __global__ __launch_bounds__(256) void midm_reduce_kernel(bf16_t* __restrict__ y
   const int m = (int)(i / per_row);
   const int n = (int)(i - (int64_t)m * per_row) * 4;
   f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
   for (int s = 0; s < S; ++s) {
     const float* row = slab + ((int64_t)s * M + m) * N;
     a += *reinterpret_cast<const f32x4*>(row + n);
@@ -195,82 +217,80 @@ __global__ __launch_bounds__(256) void midm_reduce_kernel(bf16_t* __restrict__ y
   for (int j = 0; j < 4; ++j) {
     float v = a[j];
     if constexpr (EPI == 1) v += bf2f(res[(int64_t)m * ldr + n + j]);
-    if constexpr (EPI == 2) v = act_value<0>(bf2f(f2bf(a[j]))) * bf2f(f2bf(b[j]));
-    if constexpr (EPI == 3) v = act_value<1>(bf2f(f2bf(a[j]))) * bf2f(f2bf(b[j]));
+    if constexpr (EPI == 2) v = act_value<0>(a[j]) * b[j];
+    if constexpr (EPI == 3) v = act_value<1>(a[j]) * b[j];
     o[j] = f2bf(v);
   }
   *reinterpret_cast<bf16x4*>(y + (int64_t)m * ldy + n) = o;
 }
 
-template <int MG>
-int launch_mg(bf16_t* y, float* slab, const bf16_t* x, const bf16_t* w, const bf16_t* res, int M,
-              int N, int K, int ldx, int ldy, int ldr, int S, int out, hipStream_t st) {
-  const int n_blocks = N / kMidRows;
-  const dim3 grid(n_blocks * S), block(kMidThreads);
-  const int kps = K / S;
-  switch (out) {
-    case MID_STORE:
-      midm_kernel<MG, MID_STORE><<<grid, block, 0, st>>>(y, slab, x, w, res, M, N, K, ldx, ldy, ldr, n_blocks, kps);
-      break;
-    case MID_RESIDUAL:
-      midm_kernel<MG, MID_RESIDUAL><<<grid, block, 0, st>>>(y, slab, x, w, res, M, N, K, ldx, ldy, ldr, n_blocks, kps);
-      break;
-    default:
-      midm_kernel<MG, MID_SLAB><<<grid, block, 0, st>>>(y, slab, x, w, res, M, N, K, ldx, ldy, ldr, n_blocks, kps);
-      break;
-  }
-  return 0;
+template <class C>
+int mid_launch(const MidArgs& a, bool glu, hipStream_t st) {
+  const dim3 grid(8 * a.per_xcd), block(kMidThreads);
+  if (glu) midm_kernel<C, true><<<grid, block, C::LDS, st>>>(a);
+  else midm_kernel<C, false><<<grid, block, C::LDS, st>>>(a);
+  return (int)hipGetLastError();
 }
+template <class C>
+int mid_cfg() {
+  return (int)hipFuncSetAttribute((const void*)midm_kernel<C, true>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS) |
+         (int)hipFuncSetAttribute((const void*)midm_kernel<C, false>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
+}
+#define DRTC_MID_ROWS(X, NF) X(1, NF) X(2, NF) X(3, NF) X(4, NF) X(5, NF) X(6, NF) X(7, NF) X(8, NF)
 
 }  // namespace
 
 int64_t midm_slab_bytes(int M, int N, int S) { return (int64_t)S * M * N * 4; }
 
-// epi: 0 store, 1 residual add (res may alias y), 2 SiLU-GLU, 3 GELU-GLU (N = 2 I,
-// y has N / 2 columns).  S = number of K splits (K % (64 S) == 0); S > 1 or a GLU
-// epilogue needs `slab` (midm_slab_bytes) and runs the reduce kernel.
+// epi: 0 store, 1 residual add (res may alias y), 2 SiLU-GLU, 3 GELU-GLU (N = 2 I, y has N / 2 columns),
+// 4: the slices' fp32 sums stay in the slab [S][M][N], y is not written.  nf: 16-column fragments of a
+// wave, 2 or 4.  S K slices (at most K / 64); S > 1 or epi 4 needs `slab` (midm_slab_bytes).
 int launch_midm_gemm(void* y, const void* x, const void* w, const void* res, int M, int N,
-                     int K, int ldx, int ldy, int ldr, int epi, int S, void* slab,
+                     int K, int ldx, int ldy, int ldr, int epi, int S, int nf, void* slab,
                      int64_t slab_bytes, hipStream_t st) {
-  // K per split: whole register rings (4 chunks of 64)
-  if (M < 1 || M > 256 || N % kMidRows || S < 1 || K % (4 * kMidKC * S) || ldx % 8 ||
-      ldy % 4 ||
-      epi < 0 || epi > 3 || (epi == 1 && (res == nullptr || ldr % 4)) ||
-      (epi >= 2 && (N / 2) % 4))
+  const bool glu = epi == MID_SILU || epi == MID_GELU;
+  if (M < 1 || M > 256 || (nf != 2 && nf != 4) || N < 1 || N % (32 * nf) || K < 64 || K % 64 || S < 1 ||
+      S > K / 64 || ldx % 8 || ldy % 4 || epi < 0 || epi > MID_SLAB ||
+      (epi == MID_RESIDUAL && (res == nullptr || ldr % 4)))
     return -1;
-  const bool use_slab = S > 1 || epi >= 2;
+  if ((uintptr_t)x % 16 || (uintptr_t)w % 16 || (uintptr_t)y % 8 || (uintptr_t)res % 8) return -1;
+  // 32-bit offsets from the tile's first row
+  if ((int64_t)M * ldx * 2 >= (1ll << 31) || ((int64_t)(glu ? N / 2 : 0) + 32 * nf) * K * 2 >= (1ll << 31)) return -1;
+  const bool use_slab = S > 1 || epi == MID_SLAB;
   if (use_slab && (slab == nullptr || slab_bytes < midm_slab_bytes(M, N, S))) return -2;
-  const int out = use_slab ? MID_SLAB : (epi == 1 ? MID_RESIDUAL : MID_STORE);
-  int mg = (M + 15) / 16;
-  mg += mg & 1;  // even column-group counts only
+  const int tiles = N / (32 * nf);
+  if ((int64_t)tiles * S >= (1 << 24)) return -1;
+  const MidArgs a{(bf16_t*)y, (float*)slab, (const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)res,
+                  M, N, K, ldx, ldy, ldr, use_slab ? (int)MID_SLAB : epi, tiles, S, (tiles * S + 7) / 8};
+  int e = -1;
+#define DRTC_MID(FA, NF) \
+  if ((M + 31) / 32 == FA && nf == NF) e = mid_launch<MidCfg<FA, NF>>(a, glu, st);
+  DRTC_MID_ROWS(DRTC_MID, 2)
+  DRTC_MID_ROWS(DRTC_MID, 4)
+#undef DRTC_MID
+  if (e || !use_slab || epi == MID_SLAB) return e;
+  const int NO = glu ? N / 2 : N;
+  const int64_t items = (int64_t)M * (NO / 4);
+  const dim3 rgrid((unsigned)((items + 255) / 256)), rblock(256);
   bf16_t* yy = (bf16_t*)y;
-  float* sl = (float*)slab;
-  const bf16_t* xx = (const bf16_t*)x;
-  const bf16_t* ww = (const bf16_t*)w;
+  const float* sl = (const float*)slab;
   const bf16_t* rr = (const bf16_t*)res;
-  switch (mg) {
-    case 2: launch_mg<2>(yy, sl, xx, ww, rr, M, N, K, ldx, ldy, ldr, S, out, st); break;
-    case 4: launch_mg<4>(yy, sl, xx, ww, rr, M, N, K, ldx, ldy, ldr, S, out, st); break;
-    case 6: launch_mg<6>(yy, sl, xx, ww, rr, M, N, K, ldx, ldy, ldr, S, out, st); break;
-    case 8: launch_mg<8>(yy, sl, xx, ww, rr, M, N, K, ldx, ldy, ldr, S, out, st); break;
-    case 10: launch_mg<10>(yy, sl, xx, ww, rr, M, N, K, ldx, ldy, ldr, S, out, st); break;
-    case 12: launch_mg<12>(yy, sl, xx, ww, rr, M, N, K, ldx, ldy, ldr, S, out, st); break;
-    case 14: launch_mg<14>(yy, sl, xx, ww, rr, M, N, K, ldx, ldy, ldr, S, out, st); break;
-    case 16: launch_mg<16>(yy, sl, xx, ww, rr, M, N, K, ldx, ldy, ldr, S, out, st); break;
-    default: return -1;
-  }
-  if (use_slab) {
-    const int NO = epi >= 2 ? N / 2 : N;
-    const int64_t items = (int64_t)M * (NO / 4);
-    const dim3 rgrid((unsigned)((items + 255) / 256)), rblock(256);
-    switch (epi) {
-      case 0: midm_reduce_kernel<0><<<rgrid, rblock, 0, st>>>(yy, sl, rr, M, N, S, ldy, ldr); break;
-      case 1: midm_reduce_kernel<1><<<rgrid, rblock, 0, st>>>(yy, sl, rr, M, N, S, ldy, ldr); break;
-      case 2: midm_reduce_kernel<2><<<rgrid, rblock, 0, st>>>(yy, sl, rr, M, N, S, ldy, ldr); break;
-      default: midm_reduce_kernel<3><<<rgrid, rblock, 0, st>>>(yy, sl, rr, M, N, S, ldy, ldr); break;
-    }
+  switch (epi) {
+    case MID_STORE: midm_reduce_kernel<0><<<rgrid, rblock, 0, st>>>(yy, sl, rr, M, N, S, ldy, ldr); break;
+    case MID_RESIDUAL: midm_reduce_kernel<1><<<rgrid, rblock, 0, st>>>(yy, sl, rr, M, N, S, ldy, ldr); break;
+    case MID_SILU: midm_reduce_kernel<2><<<rgrid, rblock, 0, st>>>(yy, sl, rr, M, N, S, ldy, ldr); break;
+    default: midm_reduce_kernel<3><<<rgrid, rblock, 0, st>>>(yy, sl, rr, M, N, S, ldy, ldr); break;
   }
   return (int)hipGetLastError();
+}
+
+int configure_gemm_midm() {
+  int e = 0;
+#define DRTC_MID(FA, NF) e |= mid_cfg<MidCfg<FA, NF>>();
+  DRTC_MID_ROWS(DRTC_MID, 2)
+  DRTC_MID_ROWS(DRTC_MID, 4)
+#undef DRTC_MID
+  return e;
 }
 
 }  // namespace drtc

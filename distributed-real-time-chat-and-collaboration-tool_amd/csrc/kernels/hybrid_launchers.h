@@ -12,6 +12,8 @@ namespace drtc {
 int launch_dyt(int f32, void* out, float* h, const void* y, int ldy, const int* ids,
                const void* embed, const float* w, const float* b, float alpha, int rows, int W,
                hipStream_t st);
+int launch_dyt_parts(void* out, float* h, const float* parts, int S, const float* w, const float* b, float alpha, int rows,
+                     int W, hipStream_t st);
 int launch_act_glu_f32(float* out, const float* gu, int64_t T, int I, int gu_stride, int act,
                        float limit, hipStream_t st);
 

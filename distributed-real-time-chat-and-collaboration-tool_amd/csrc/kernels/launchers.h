@@ -15,6 +15,8 @@ int launch_rmsnorm(void* out, void* residual, const void* x, const void* w,
                    int rows, int H, float eps, int x_stride, int out_stride,
                    int res_stride, bool gemma, hipStream_t st);
 
+int launch_rmsnorm_parts(void* out, void* residual, const float* parts, int S, const void* w, int rows, int H, float eps,
+                         int out_stride, int res_stride, bool gemma, hipStream_t st);
 int launch_act_glu(void* out, const void* gu, int64_t T, int I, int gu_stride,
                    int act, float limit, hipStream_t st);
 
@@ -67,6 +69,7 @@ struct MoeOptions {
   const void* y = nullptr;
   int ldy = 0;
   int W = 0;
+  int y_parts = 0;  // > 0: y is that many fp32 partial sums [y_parts][T][ldy]
 };
 // variant 0 / 1 / 2: the moe.hip grouped GEMMs; 3: gemm_xd grouped mode with xd forms gu_form
 // (gated gate_up) / dn_form (down), 0 = by rows per expert; slab / counters: the split-K
@@ -212,8 +215,9 @@ int configure_ring_moe();
 // medium-M decode GEMM (gemm_midm.hip)
 int64_t midm_slab_bytes(int M, int N, int S);
 int launch_midm_gemm(void* y, const void* x, const void* w, const void* res, int M, int N,
-                     int K, int ldx, int ldy, int ldr, int epi, int S, void* slab,
+                     int K, int ldx, int ldy, int ldr, int epi, int S, int nf, void* slab,
                      int64_t slab_bytes, hipStream_t st);
+int configure_gemm_midm();
 int configure_moe();
 
 }  // namespace drtc

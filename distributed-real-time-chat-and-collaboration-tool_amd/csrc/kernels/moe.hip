@@ -897,18 +897,25 @@ __global__ __launch_bounds__(256) void moe_combine_f32_kernel(
 
 // As the combine kernels, added to the residual stream h [T, W] together with y; the first W of H
 // columns.  out (bf16): the stream after the add, or null.
-template <class T>
+// PARTS: y is the S fp32 partial sums [S][T][ldy] of that sublayer's product.
+template <class T, bool PARTS = false>
 __global__ __launch_bounds__(256) void moe_combine_stream_kernel(
-    bf16_t* __restrict__ out, float* __restrict__ h, const T* __restrict__ y, int64_t ldy,
+    bf16_t* __restrict__ out, float* __restrict__ h, const void* __restrict__ yv, int64_t ldy, int S,
     const T* __restrict__ z, const T* __restrict__ z2, const float* __restrict__ topk_w,
     const int* __restrict__ inv_pos, int W, int H, int k) {
   const int t = blockIdx.x;
   float* hr = h + (int64_t)t * W;
-  const T* yr = y + (int64_t)t * ldy;
+  const T* yr = (const T*)yv + (int64_t)t * ldy;
   if (W % 8 == 0 && ldy % 8 == 0) {
     for (int c = threadIdx.x * 8; c < W; c += 256 * 8) {
       float s[8], d[8];
-      load8(s, yr + c);
+      if constexpr (PARTS) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) s[q] = 0.f;
+        add_parts(s, (const float*)yv + t * ldy + c, (int64_t)gridDim.x * ldy, S);
+      } else {
+        load8(s, yr + c);
+      }
       for (int j = 0; j < k; ++j) {
         const int64_t p = inv_pos[t * k + j];
         const float w = topk_w[t * k + j];
@@ -930,6 +937,7 @@ __global__ __launch_bounds__(256) void moe_combine_stream_kernel(
     }
     return;
   }
+  if constexpr (PARTS) return;  // (whole vectors only)
   for (int c = threadIdx.x; c < W; c += 256) {
     float s = to_f32(yr[c]);
     for (int j = 0; j < k; ++j) {
@@ -1018,6 +1026,7 @@ int launch_moe(void* out, const void* x, const void* router_logits, const void* 
   if (opt.stream && (opt.y == nullptr || opt.W < 1 || opt.W > H || opt.ldy < opt.W || e_off != 0 ||
                      e_local != E))
     return -1;
+  if (opt.y_parts && (!opt.stream || opt.f32 || opt.y_parts < 0 || opt.y_parts > kMaxParts || opt.W % 8 || opt.ldy % 8)) return -1;
   if (opt.groups < 1 || opt.groups > kMoeMaxGroups || E % opt.groups || opt.keep < 1 ||
       opt.keep > opt.groups || k > opt.keep * (E / opt.groups))
     return -1;
@@ -1178,7 +1187,7 @@ int launch_moe(void* out, const void* x, const void* router_logits, const void* 
         I, H, 0, 0.f);
     if (opt.stream) {
       moe_combine_stream_kernel<float><<<dim3(T), dim3(256), 0, st>>>(
-          nullptr, opt.stream, (const float*)opt.y, opt.ldy, (const float*)zbuf, nullptr, topk_w,
+          nullptr, opt.stream, opt.y, opt.ldy, 0, (const float*)zbuf, nullptr, topk_w,
           inv_pos, opt.W, H, k);
       return (int)hipGetLastError();
     }
@@ -1262,8 +1271,8 @@ int launch_moe(void* out, const void* x, const void* router_logits, const void* 
                        n_tiles, I, H, I, H, max_tiles, 0, 0.f);
   }
   if (opt.stream) {
-    moe_combine_stream_kernel<bf16_t><<<dim3(T), dim3(256), 0, st>>>(
-        (bf16_t*)out, opt.stream, (const bf16_t*)opt.y, opt.ldy, zbuf,
+    (opt.y_parts ? moe_combine_stream_kernel<bf16_t, true> : moe_combine_stream_kernel<bf16_t>)<<<dim3(T), dim3(256), 0, st>>>(
+        (bf16_t*)out, opt.stream, opt.y, opt.ldy, opt.y_parts, zbuf,
         dn_split ? (const bf16_t*)zbuf2 : nullptr, topk_w, inv_pos, opt.W, H, k);
     return (int)hipGetLastError();
   }

@@ -23,9 +23,10 @@ DRTC_DEVICE float tanh_as<bf16_t>(float x) { return tanh_exp(x); }
 template <>
 DRTC_DEVICE float tanh_as<float>(float x) { return tanhf(x); }
 
-template <class T>
+// PARTS: y is the S fp32 partial sums [S][rows][W] of the product ahead
+template <class T, bool PARTS = false>
 __global__ __launch_bounds__(256) void dyt_vec_kernel(
-    T* __restrict__ out, float* __restrict__ h, const T* __restrict__ y, int ldy,
+    T* __restrict__ out, float* __restrict__ h, const void* __restrict__ yv, int ldy, int S,
     const int* __restrict__ ids, const T* __restrict__ embed, const float* __restrict__ w,
     const float* __restrict__ b, float alpha, int64_t nvec, int vpr) {
   const int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -41,9 +42,12 @@ __global__ __launch_bounds__(256) void dyt_vec_kernel(
     store8(h + at, x);
   } else {
     load8(x, h + at);
-    if (y) {
+    if constexpr (PARTS) {
+      add_parts(x, (const float*)yv + at, nvec * 8, S);
+      store8(h + at, x);
+    } else if (yv) {
       float d[8];
-      load8(d, y + row * ldy + c);
+      load8(d, (const T*)yv + row * ldy + c);
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] += d[j];
       store8(h + at, x);
@@ -83,7 +87,7 @@ static void dyt_t(void* out, float* h, const void* y, int ldy, const int* ids, c
   if (W % 8 == 0 && ldy % 8 == 0) {
     const int64_t n = (int64_t)rows * (W / 8);
     dyt_vec_kernel<T><<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st>>>(
-        (T*)out, h, (const T*)y, ldy, ids, (const T*)embed, w, b, alpha, n, W / 8);
+        (T*)out, h, y, ldy, 0, ids, (const T*)embed, w, b, alpha, n, W / 8);
   } else {
     const int64_t n = (int64_t)rows * W;
     dyt_any_kernel<T><<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st>>>(
@@ -97,6 +101,16 @@ int launch_dyt(int f32, void* out, float* h, const void* y, int ldy, const int* 
   if (rows == 0) return 0;
   if (f32) dyt_t<float>(out, h, y, ldy, ids, embed, w, b, alpha, rows, W, st);
   else dyt_t<bf16_t>(out, h, y, ldy, ids, embed, w, b, alpha, rows, W, st);
+  return (int)hipGetLastError();
+}
+
+int launch_dyt_parts(void* out, float* h, const float* parts, int S, const float* w, const float* b, float alpha, int rows,
+                     int W, hipStream_t st) {
+  if (W % 8 || S < 1 || S > kMaxParts) return -1;
+  if (rows == 0) return 0;
+  const int64_t n = (int64_t)rows * (W / 8);
+  dyt_vec_kernel<bf16_t, true><<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st>>>(
+      (bf16_t*)out, h, parts, 0, S, nullptr, nullptr, w, b, alpha, n, W / 8);
   return (int)hipGetLastError();
 }
 

@@ -379,18 +379,19 @@ class HybridLM:
         cfg = self.cfg
         h = torch.empty((ids.shape[0], cfg.hidden_size), dtype=torch.float32, device=self.device)
         y, by, last = None, None, len(self.layers) - 1
+        linear = ops.linear_parts if isinstance(self.final, Dyt) else ops.linear  # (every norm is of one kind)
         for i, (l, L) in enumerate(zip(cfg.layers, self.layers)):
             x = self._enter(L["norm1"], h, y, by, ids=ids if i == 0 else None)
             a = mix(i, L["mixer"], x)
             if i == last and rows is not None:
                 a, h = a.index_select(0, rows), h.index_select(0, rows)
-            y, by = ops.linear(a, L["mixer"].o), L.get("add1")
+            y, by = linear(a, L["mixer"].o), L.get("add1")
             if l.experts:
                 x = self._enter(L["norm2"], h, y, by, width=self._moe_width)
                 y, by = self._experts(L, l, x), L["add2"]
             elif l.ff:
                 x = self._enter(L["norm2"], h, y, by)
-                y = ops.linear(ops.gated(x, L["gate_up"], cfg.act, l.limit), L["down"])
+                y = linear(ops.gated(x, L["gate_up"], cfg.act, l.limit), L["down"])
                 by = L.get("add2")
         return ops.linear(self._enter(self.final, h, y, by), self.lm_head)
 
@@ -458,11 +459,10 @@ class HybridLM:
                 x = wide[:, :W]
             if "up" in L:
                 ops.squared_relu(x, L["up"], a[:, off:])
-            y = ops.linear(a, L["out"])
             if l.experts:
-                x = self._experts(L, l, wide, stream=h, y=y)
+                x = self._experts(L, l, wide, stream=h, y=ops.linear_parts(a, L["out"]))
             else:
-                x = ops.stream_add(h, y)
+                x = ops.stream_add(h, ops.linear(a, L["out"]))
             z = zn = None
             if cfg.side_dim:
                 g = ops.side_input(x, L["side_gate"], self.side_embed, ids, i)

@@ -294,16 +294,24 @@ class TransformerLM:
             res = self._fusable_residual(h, x)
             if res is not None:
                 return ops.linear_residual(h, L["down"], res), True
+            if self.pc.tp_size == 1:
+                return ops.linear_parts(h, L["down"]), False
             y = ops.linear(h, L["down"])
         else:
             gu = ops.norm_linear(x, L["gate_up"])
             res = self._fusable_residual(gu, x)
             if res is not None:
                 return ops.linear_residual(ops.act_glu(gu, self.cfg.act), L["down"], res), True
-            y = ops.glu_linear(gu, L["down"], self.cfg.act)
+            y = ops.glu_linear(gu, L["down"], self.cfg.act, parts=self.pc.tp_size == 1)
         if decode and self.pc.tp_size > 1:
             return y, False, True  # reduced by the next norm (fused all-reduce + add + norm)
         return self.pc.all_reduce_tp(y), False
+
+    def _to_norm(self, a: torch.Tensor, w: torch.Tensor):
+        """A projection whose output goes into the next residual add and norm."""
+        if self.pc.tp_size == 1:
+            return ops.linear_parts(a, w)
+        return self.pc.all_reduce_tp(ops.linear(a, w))
 
     def _fusable_residual(self, a: torch.Tensor, x: ops.PendingNorm) -> torch.Tensor | None:
         """The residual stream the o / down projection may add into inside its
@@ -448,7 +456,7 @@ class TransformerLM:
             res = self._fusable_residual(a, x)
             if res is not None:
                 return ops.linear_residual(a, L["o"], res), True
-            return self.pc.all_reduce_tp(ops.linear(a, L["o"])), False
+            return self._to_norm(a, L["o"]), False
 
         last = len(self.layers) - 1
         x = self._layers(self._embed(ids), attn)
@@ -572,10 +580,10 @@ class TransformerLM:
                                                 meta.context_lens, cfg.attn_scale, out=attn_out,
                                                 blocks_per_part=meta.blocks_per_part,
                                                 workspace=meta.workspace)
-            o = ops.linear(a.view(B, sh.hq * D), L["o"])
+            a = a.view(B, sh.hq * D)
             if self.pc.tp_size > 1:
-                return o, False, True  # reduced by the next norm (fused all-reduce + add + norm)
-            return o, False
+                return ops.linear(a, L["o"]), False, True  # reduced by the next norm (fused all-reduce + add + norm)
+            return ops.linear_parts(a, L["o"]), False
 
         if self.decode_micro_ok(B):
             return self._forward_decode_micro(ids, meta, kv_caches, attn_out)

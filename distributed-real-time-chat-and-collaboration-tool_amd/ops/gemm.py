@@ -9,7 +9,9 @@ shape (M, N, K, row stride of x) ONCE to a route, cached per shape (``route``):
   "skinny"  gemv.hip weight-streaming kernels (M <= 16)     decode buckets where the table (or
                                                             ``skinny_variant`` untuned) says so
             gemm_stream.hip (variant STREAM, M <= 64)       where ``stream_ok`` says so
-  "midm"    gemm_midm.hip medium-M kernel (M <= 256)        decode buckets where the table says so
+  "midm"    gemm_midm.hip medium-M kernel (M <= 256)        decode buckets where the table says so;
+                                                            K slices' sums for the op behind
+                                                            (``linear_parts``): ``parts_form``
   "xd"      gemm_xd.hip: 128-row tiles, full K, tile order  decode buckets where the table says so
             partitioned by XCD (``xd_gemm``)                (full-batch qkv / o / down)
   "lt"      hipBLASLt with the per-shape measured solution  the other decode buckets, and
@@ -160,6 +162,7 @@ def reset() -> None:
     with _lock:
         _table = None
         _routes.clear()
+        _parts_forms.clear()
 
 
 def set_enabled(on: bool) -> None:
@@ -453,10 +456,11 @@ _fuse_glu = os.environ.get("DRTC_FUSED_GLU_GEMM", "1") != "0"
 GLU_FUSE_MAX_M = 1
 
 
-def glu_linear(gu: torch.Tensor, w: torch.Tensor, act: str = "silu") -> torch.Tensor:
-    """y = (act(gu[:, :I]) * gu[:, I:]) @ w.T (the down projection of a gated MLP).  When the
+def glu_linear(gu: torch.Tensor, w: torch.Tensor, act: str = "silu", parts: bool = False):
+    """y = (act(gu[:, :I]) * gu[:, I:]) @ w.T (the down projection of a gated MLP), by ``linear`` or
+    (``parts``) ``linear_parts`` behind ops.act_glu.  When the
     projection would run on the skinny dot2 kernel the activation is computed inside it while
-    loading its input (gemv.hip, no act_glu launch); otherwise ops.act_glu + linear."""
+    loading its input (gemv.hip, no act_glu launch)."""
     from .activation import act_glu
 
     if _fuse_glu and _gpu_bf16(gu, w) and act in ("silu", "gelu_tanh"):
@@ -469,7 +473,7 @@ def glu_linear(gu: torch.Tensor, w: torch.Tensor, act: str = "silu") -> torch.Te
                                          gu.stride(0), N, 0 if act == "silu" else 1,
                                          stream_ptr(gu)), "skinny_glu_gemm")
             return y
-    return linear(act_glu(gu, act), w)
+    return (linear_parts if parts else linear)(act_glu(gu, act), w)
 
 
 # ------------------------------------------------------------------ weight-streaming decode GEMM
@@ -1131,14 +1135,13 @@ def xd_gemm(x: torch.Tensor, w: torch.Tensor, epi: str = "store",
 
 
 # ------------------------------------------------------------------ medium-M decode GEMM
-MIDM_EPI = {"store": 0, "residual": 1, "silu": 2, "gelu_tanh": 3}  # gemm_midm.hip accepts 0-3
+MIDM_EPI = {"store": 0, "residual": 1, "silu": 2, "gelu_tanh": 3}  # 4: partial sums (``linear_parts``)
 MIDM_MAX_M = 256
 
 
 def midm_splits(M: int, N: int, K: int, target_wgs: int | None = None) -> int:
-    """K splits of the medium-M GEMM: the largest S <= 16 with K a multiple of 256 S (whole
-    4-chunk register rings per split) and at most ~2 workgroups per CU (one above 128 rows,
-    where the kernel runs one workgroup per CU)."""
+    """K splits of the medium-M GEMM: the largest S <= 16 with K a multiple of 256 S and at most two
+    workgroups per CU (one above 128 rows)."""
     if target_wgs is None:
         target_wgs = 256 if M > 128 else 512
     nb = N // 128
@@ -1151,24 +1154,23 @@ def midm_splits(M: int, N: int, K: int, target_wgs: int | None = None) -> int:
 
 
 def midm_depth(M: int) -> int:
-    """Chunks of 64 k in flight per wave (gemm_midm.hip mid_depth)."""
+    """K tiles of 64 that a split of ``midm_splits`` is a multiple of."""
     return 4
 
 
 def midm_supported(M: int, N: int, K: int, epi: str = "store") -> bool:
-    return (1 <= M <= MIDM_MAX_M and N % 128 == 0 and K % (64 * midm_depth(M)) == 0
+    return (1 <= M <= MIDM_MAX_M and N % 128 == 0 and K % 64 == 0
             and epi in MIDM_EPI
             and (epi not in ("silu", "gelu_tanh") or (N // 2) % 4 == 0))
 
 
 def midm_gemm(x: torch.Tensor, w: torch.Tensor, epi: str = "store",
               residual: torch.Tensor | None = None, out: torch.Tensor | None = None,
-              splits: int | None = None) -> torch.Tensor:
-    """Medium-M (17..256 rows) decode GEMM, csrc/kernels/gemm_midm.hip: y = x @ w^T with a
+              splits: int | None = None, nf: int = 4) -> torch.Tensor:
+    """Medium-M (up to 256 rows) decode GEMM, csrc/kernels/gemm_midm.hip: y = x @ w^T with a
     store / residual (y = residual + x w^T, in place when out is residual) / SiLU- or
-    GELU-gated [gate | up] epilogue.  W streams once from HBM into registers, x is shared
-    through LDS, K is split over workgroups and the fp32 partials summed by a second small
-    kernel."""
+    GELU-gated [gate | up] epilogue.  Tiles of all rows and 32 ``nf`` (2, 4) columns, K split over
+    workgroups, the fp32 partials summed by a second small kernel."""
     M, K = x.shape
     N = w.shape[0]
     assert x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_cuda
@@ -1187,12 +1189,80 @@ def midm_gemm(x: torch.Tensor, w: torch.Tensor, epi: str = "store",
     slab = gemm_workspace(x.device)[0]
     check(hipk().midm_gemm(out.data_ptr(), x.data_ptr(), w.data_ptr(), ptr(residual), M, N, K,
                            x.stride(0), out.stride(0),
-                           residual.stride(0) if residual is not None else 0, MIDM_EPI[epi], S,
+                           residual.stride(0) if residual is not None else 0, MIDM_EPI[epi], S, nf,
                            slab.data_ptr(), slab.numel() * 4, stream_ptr(x)), "midm_gemm")
     return out
 
 
-__all__ = ["linear", "route", "norm_linear", "glu_linear", "norm_glu", "fused_glu_ok",
+class Parts:
+    """x @ w.T as the fp32 sums of its K slices, ``slab`` [S, M, N], for an op that adds them up while it
+    reads its input (``PendingNorm`` with a residual, ``dyt``, ``fused_moe``'s ``y``)."""
+
+    __slots__ = ("slab", "dtype")
+
+    def __init__(self, slab: torch.Tensor, dtype: torch.dtype):
+        self.slab, self.dtype = slab, dtype
+
+    @property
+    def shape(self) -> torch.Size:
+        return self.slab.shape[1:]
+
+    def tensor(self) -> torch.Tensor:
+        return self.slab.sum(0).to(self.dtype)
+
+
+MAX_PARTS = 8  # common.h kMaxParts
+_parts_enabled = os.environ.get("DRTC_PARTS", "1") != "0"
+# (M, N, K) -> (16-column fragments, K slices) of ``linear_parts``, None: ``linear``
+_parts_forms: dict[tuple[int, int, int], tuple[int, int] | None] = {}
+
+
+def parts_form(M: int, N: int, K: int) -> tuple[int, int] | None:
+    """How ``linear_parts`` cuts a product of M rows, None where ``linear`` is as fast.  us of ``linear`` / of
+    the parts, to which reading them adds 0.3 - 2:
+      K from 5120 on, 3 rows to 256: 4096 x 14336, 4 rows 22.7 / 19.8, 16 24.2 / 19.8, 64 28.3 / 22.7, 160 39.0 / 30.8, 256
+        58.0 / 38.6; 2048 x 7168, 4 rows 11.0 / 7.4, 160 24.2 / 14.1; 2048 x 5632, 256 rows 20.9 / 16.0; two rows and one
+        stay with the dot2 form (2048 x 7168 8.4 / 7.4, 7.5 / 7.3)
+      K from 4096 on to 160 rows: 4096 x 4096, 4 rows 9.7 / 8.4, 16 11.1 / 8.5, 64 14.1 / 9.9, 160 19.5 / 15.0; 200 18.8 / 17.3
+      K from 2048 on, 17 rows to 64, 128 where narrow: 2048 x 2048, 16 rows 6.2 / 4.8, 24 7.6 / 5.0, 64 10.7 / 5.9, 128 10.7 /
+        7.6, 160 10.5 / 8.7; 3584 x 2048, 64 rows 9.4 / 7.0, 96 9.2 / 8.3
+    The cut: the least of a workgroup's operands at 50 GB/s or its weights at 24, a quarter of a microsecond to
+    a slice, and the parts read again by the whole chip or by a row's CU."""
+    key = (M, N, K)
+    if key in _parts_forms:
+        return _parts_forms[key]
+    rows = (3, 256) if K >= 5120 else (3, 160) if K >= 4096 else (17, 128 if N <= 2048 else 64) if K >= 2048 else (1, 0)
+    best = None
+    if _parts_enabled and _midm_enabled and K % 64 == 0 and 1024 <= N <= 8192 and rows[0] <= M <= rows[1]:
+        for nf in (2, 4):
+            for s in range(2, MAX_PARTS + 1):
+                tiles = N // (32 * nf) * s
+                if N % (32 * nf) or tiles > 256 or K // 64 // s < 4:
+                    continue
+                cost = (max(K / s * (M + 32 * nf) * 2 / 50e3, K / s * 32 * nf * 2 / 24e3) + 0.25 * s
+                        + max(s * M * N * 4 / 8e6, s * N * 4 / 65e3))
+                if best is None or cost < best[0]:
+                    best = cost, (nf, s)
+    form = best[1] if best else None
+    _parts_forms[key] = form
+    return form
+
+
+def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | Parts:
+    """``linear``, or its K slices' sums (csrc/kernels/gemm_midm.hip) where ``parts_form`` says so."""
+    if _gpu_bf16(x, w) and w.shape[1] == x.shape[1] and _aligned(x, w):
+        (M, K), N = x.shape, w.shape[0]
+        form = parts_form(M, N, K) if M * x.stride(0) < 1 << 30 else None
+        if form is not None:
+            nf, S = form
+            slab = torch.empty((S, M, N), dtype=torch.float32, device=x.device)
+            check(hipk().midm_gemm(0, x.data_ptr(), w.data_ptr(), 0, M, N, K, x.stride(0), N, 0, 4, S, nf,
+                                   slab.data_ptr(), slab.numel() * 4, stream_ptr(x)), "midm_gemm")
+            return Parts(slab, x.dtype)
+    return linear(x, w)
+
+
+__all__ = ["linear", "linear_parts", "parts_form", "Parts", "route", "norm_linear", "glu_linear", "norm_glu", "fused_glu_ok",
            "linear_residual",
            "residual_fusable", "w4_glu_ok", "w4_ok", "w4_shape_ok", "squared_relu", "w4_group_m", "mfma_gemm",
            "mfma_gemm_grouped",

@@ -22,6 +22,7 @@ import torch.nn.functional as F
 
 from ._ext import check, hipk, on_gpu, stream_ptr
 from .activation import ACTS, act_glu_ref
+from .gemm import Parts
 
 # Largest token chunk per kernel call: bounds the workspace (P = chunk * k rows of [I] and [H]
 # intermediates: ~3 GB for Mixtral).  One Mixtral prefill step (ModelConfig.prefill_chunk,
@@ -158,7 +159,7 @@ def fused_moe(x: torch.Tensor, router_logits: torch.Tensor, w_gu: torch.Tensor,
     """y[t] = sum_j w[t,j] * down_e(act(gate_e x_t) * up_e x_t) over the top-k experts; act
     "relu2": down_e(relu(up_e x_t)^2), w_gu [E_local, I, H].
 
-    ``stream`` [T, W <= H] fp32: the result is added to it together with ``y`` [T, W], and the
+    ``stream`` [T, W <= H] fp32: the result is added to it together with ``y`` [T, W] (or its ``Parts``), and the
     stream is returned in x's type (itself in fp32).
 
     x [T, H] bf16 (H % 128 == 0, I % 64 == 0) or fp32 (any size); router_logits [T, E] bf16 or
@@ -194,10 +195,17 @@ def fused_moe(x: torch.Tensor, router_logits: torch.Tensor, w_gu: torch.Tensor,
     assert 1 <= groups <= MAX_GROUPS and E % groups == 0 and 1 <= keep <= groups
     assert top_k <= keep * (E // groups)
     W = H
+    y_parts = 0
     if stream is not None:
         W = stream.shape[1]
+        if isinstance(y, Parts):
+            if f32 or W % 8 or T > MOE_CHUNK:
+                y = y.tensor()
+            else:
+                y_parts, slab_y = y.slab.shape[0], y.slab
+                assert y.shape == (T, W) and slab_y.is_contiguous()
         assert stream.shape == y.shape == (T, W) and W <= H and stream.is_contiguous()
-        assert stream.dtype == torch.float32 and y.dtype == x.dtype and y.stride(1) == 1
+        assert stream.dtype == torch.float32 and y.dtype == x.dtype and (y_parts or y.stride(1) == 1)
         assert out is None and (e_off, e_local) == (0, E)
         out = stream if f32 else x.new_empty(T, W)
     elif out is None:
@@ -231,7 +239,7 @@ def fused_moe(x: torch.Tensor, router_logits: torch.Tensor, w_gu: torch.Tensor,
                       cnt.numel() if cnt is not None else 0, lts, les, int(f32),
                       int(router_logits.dtype == torch.float32), groups, keep, float(limit),
                       0 if stream is None else stream[t0].data_ptr(),
-                      0 if stream is None else y[t0].data_ptr(),
-                      0 if stream is None else y.stride(0), W, st), "moe")
+                      0 if stream is None else slab_y.data_ptr() if y_parts else y[t0].data_ptr(),
+                      0 if stream is None else W if y_parts else y.stride(0), W, y_parts, st), "moe")
     return out
 

@@ -6,6 +6,7 @@ from __future__ import annotations
 import torch
 
 from ._ext import check, hipk, on_gpu, ptr, stream_ptr
+from .gemm import Parts
 
 
 def rmsnorm_ref(x: torch.Tensor, w: torch.Tensor, eps: float, gemma: bool = False,
@@ -50,6 +51,18 @@ def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, gemma: bool = False,
     return out
 
 
+def rmsnorm_parts(x: Parts, w: torch.Tensor, eps: float, gemma: bool, residual: torch.Tensor) -> torch.Tensor:
+    """``rmsnorm`` of the sum of x's parts and the residual, without rounding the sum in between."""
+    S, rows, H = x.slab.shape
+    assert w.shape == (H,) and w.dtype == torch.bfloat16 and w.is_contiguous() and H % 8 == 0 and H <= 8192 * 2
+    assert residual.shape == (rows, H) and residual.stride(1) == 1 and residual.dtype == torch.bfloat16
+    out = torch.empty((rows, H), dtype=torch.bfloat16, device=residual.device)
+    check(hipk().rmsnorm_parts(out.data_ptr(), residual.data_ptr(), x.slab.data_ptr(), S, w.data_ptr(), rows, H,
+                               float(eps), out.stride(0), residual.stride(0), bool(gemma), stream_ptr(residual)),
+          "rmsnorm_parts")
+    return out
+
+
 def embed(ids: torch.Tensor, table: torch.Tensor) -> torch.Tensor:
     """table[ids] of token ids [rows] (int32 or int64)."""
     if not (on_gpu(table) and ids.device == table.device and ids.dim() == 1 and ids.is_contiguous()
@@ -79,6 +92,16 @@ def dyt(h: torch.Tensor, w: torch.Tensor, b: torch.Tensor, alpha: float,
     if not on_gpu(h):
         return dyt_ref(h, w, b, alpha, y, ids, embed, dtype)
     rows, W = h.shape
+    if isinstance(y, Parts):
+        if dtype == torch.bfloat16 and W % 8 == 0:
+            S = y.slab.shape[0]
+            assert y.shape == (rows, W) and ids is None and h.is_contiguous() and w.is_contiguous() and b.is_contiguous()
+            assert h.dtype == w.dtype == b.dtype == torch.float32 and w.numel() == b.numel() == W
+            out = torch.empty((rows, W), dtype=dtype, device=h.device)
+            check(hipk().dyt_parts(out.data_ptr(), h.data_ptr(), y.slab.data_ptr(), S, w.data_ptr(), b.data_ptr(),
+                                   float(alpha), rows, W, stream_ptr(h)), "dyt_parts")
+            return out
+        y = y.tensor()
     assert h.dtype == w.dtype == b.dtype == torch.float32 and h.is_contiguous()
     assert w.numel() == b.numel() == W and w.is_contiguous() and b.is_contiguous()
     assert y is None or (y.shape == (rows, W) and y.stride(1) == 1 and y.dtype == dtype)
@@ -147,6 +170,8 @@ class PendingNorm:
         self.pc = pc
         self._h: torch.Tensor | None = None
         self._out: torch.Tensor | None = None
+        if isinstance(x, Parts):  # K slices of the product ahead: added up by the norm
+            self.materialize()
 
     def applied(self, h: torch.Tensor) -> None:
         """Record that a fused consumer computed h = x (+ residual)."""
@@ -158,6 +183,8 @@ class PendingNorm:
             if self.pc is not None:
                 self._out = self.pc.reduce_norm(self.x, res, self.w, self.eps, self.gemma)
                 self.pc = None
+            elif isinstance(self.x, Parts):
+                self._out = rmsnorm_parts(self.x, self.w, self.eps, self.gemma, res)
             else:
                 self._out = rmsnorm(self.x, self.w, self.eps, self.gemma, residual=res)
             self._h = res if res is not None else self.x  # rmsnorm updated res in place

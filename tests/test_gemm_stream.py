@@ -369,3 +369,72 @@ def test_wide_products(hipk, M, N, K, form):
         a, b = (x.double() @ w[:N // 512 * 512].double().t()).chunk(2, -1)
         want = a * torch.sigmoid(a) * b
         assert ((glu.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all()
+
+
+def test_parts_forms():
+    """The cut of every shape that the rule takes fits the kernel; what lies outside of it stays with linear."""
+    seen = set()
+    for K in (2048, 2112, 3584, 4096, 5120, 5632, 8192, 14336, 28672):
+        for N in (1024, 1088, 2048, 4096, 5120, 8192):
+            for M in (1, 2, 3, 16, 17, 33, 64, 65, 128, 129, 160, 161, 256, 257):
+                form = G.parts_form(M, N, K)
+                if form:
+                    nf, s = form
+                    assert nf in (2, 4) and N % (32 * nf) == 0 and 2 <= s <= G.MAX_PARTS and K // 64 // s >= 4
+                    assert N // (32 * nf) * s <= 256 and 3 <= M <= 256
+                    seen.add(form)
+    assert len(seen) > 6
+    assert not any(G.parts_form(*s) for s in [(2, 4096, 14336), (257, 4096, 14336), (161, 4096, 4096), (16, 2048, 2048),
+                                              (65, 4096, 2048), (64, 4096, 1984), (64, 8256, 4096), (64, 4096, 4104)])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,form", [(1, 1024, 256, (2, 1)), (17, 1088, 320, (2, 5)), (33, 2048, 4096, (2, 8)),
+                                       (64, 4096, 704, (4, 8)), (96, 1024, 2112, (4, 3)), (150, 4096, 5632, (2, 4)),
+                                       (160, 2048, 1024, (4, 2)), (200, 1152, 7168, (4, 7)), (256, 1024, 448, (4, 1))])
+def test_product_parts(hipk, M, N, K, form):
+    """K slices at the edges of the tiles and rings (fewer K tiles than stages, slices of unequal length, rows
+    that are no multiple of 32) and the three ops that add them up, each against 64 bits."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    buf = torch.randn(M, K + 8, device="cuda", generator=g).to(torch.bfloat16)
+    x = buf[:, :K]
+    w = (torch.randn(N, K, device="cuda", generator=g) / K ** 0.5).to(torch.bfloat16)
+    nf, s = form
+    slab = torch.full((s, M, N), float("nan"), device="cuda")
+    assert hipk.midm_gemm(0, x.data_ptr(), w.data_ptr(), 0, M, N, K, x.stride(0), N, 0, 4, s, nf, slab.data_ptr(),
+                          slab.numel() * 4, torch.cuda.current_stream().cuda_stream) == 0
+    want = x.double() @ w.double().t()
+    # fp32 sums of K products in whatever order
+    assert (slab.double().sum(0) - want).abs().max() <= 2.0 ** -24 * K ** 0.5 * 16
+    parts = G.Parts(slab, torch.bfloat16)
+    near = 2.0 ** -8  # of a rounding to bf16
+    # residual add and RMS norm
+    res = torch.randn(M, N, device="cuda", generator=g).to(torch.bfloat16)
+    nw = (1 + 0.1 * torch.randn(N, device="cuda", generator=g)).to(torch.bfloat16)
+    h = want + res.double()
+    for gemma in (False, True):
+        r = res.clone()
+        p = ops.PendingNorm(parts, r, nw, 1e-5, gemma)
+        assert p.stream().data_ptr() == r.data_ptr()
+        assert ((r.double() - h).abs() <= near * h.abs() + 1e-5).all()
+        n = h * torch.rsqrt((h * h).mean(-1, keepdim=True) + 1e-5) * (nw.double() + gemma)
+        assert ((p.materialize().double() - n).abs() <= 2 * near * n.abs() + 1e-4).all()
+    # Dynamic Tanh on the 32-bit stream
+    st, b = res.float(), torch.randn(N, device="cuda", generator=g)
+    out = ops.dyt(st, nw.float(), b, 0.7, y=parts)
+    assert (st.double() - h).abs().max() <= 1e-5
+    t = torch.tanh(0.7 * h) * nw.double() + b.double()
+    assert ((out.double() - t).abs() <= near * t.abs() + 1e-5).all()
+    # the experts' combine: experts that return zeros leave the sum alone
+    if N % 128 == 0:
+        st = res.float()
+        zero = torch.zeros(2, 128, N, device="cuda", dtype=torch.bfloat16)
+        out = ops.fused_moe(res, torch.randn(M, 2, device="cuda", generator=g), zero, zero.transpose(1, 2).contiguous(), 1,
+                            "relu2", stream=st, y=parts)
+        assert (st.double() - h).abs().max() <= 1e-5 and torch.equal(out, st.to(torch.bfloat16))
+    # a K slice's sums do not depend on what else is in the batch
+    if M > 32:
+        few = torch.empty(s, 32, N, device="cuda")
+        assert hipk.midm_gemm(0, x.data_ptr(), w.data_ptr(), 0, 32, N, K, x.stride(0), N, 0, 4, s, nf, few.data_ptr(),
+                              few.numel() * 4, torch.cuda.current_stream().cuda_stream) == 0
+        assert torch.equal(few, slab[:, :32])
