@@ -32,6 +32,12 @@ PYBIND11_MODULE(_hipk, m) {
                                       P<void>(w), rows, H, eps, x_stride,
                                       out_stride, res_stride, gemma, S(st));
         });
+  m.def("rmsnorm_router", [](u64 out, u64 residual, u64 x, int n_parts, u64 w, u64 router, u64 logits, int E, int rows, int H,
+                             float eps, int x_stride, int out_stride, int res_stride, u64 st) {
+    return drtc::launch_rmsnorm_router(P<void>(out), P<void>(residual), P<const void>(x), n_parts, P<const void>(w),
+                                       P<const void>(router), P<float>(logits), E, rows, H, eps, x_stride, out_stride,
+                                       res_stride, S(st));
+  });
   m.def("rmsnorm_parts", [](u64 out, u64 residual, u64 parts, int S_, u64 w, int rows, int H, float eps, int out_stride,
                             int res_stride, bool gemma, u64 st) {
     return drtc::launch_rmsnorm_parts(P<void>(out), P<void>(residual), P<const float>(parts), S_, P<const void>(w), rows, H,

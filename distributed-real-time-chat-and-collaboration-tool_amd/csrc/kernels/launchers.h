@@ -15,6 +15,9 @@ int launch_rmsnorm(void* out, void* residual, const void* x, const void* w,
                    int rows, int H, float eps, int x_stride, int out_stride,
                    int res_stride, bool gemma, hipStream_t st);
 
+int launch_rmsnorm_router(void* out, void* residual, const void* x, int S, const void* w, const void* router, float* logits,
+                          int E, int rows, int H, float eps, int x_stride, int out_stride, int res_stride,
+                          hipStream_t st);
 int launch_rmsnorm_parts(void* out, void* residual, const float* parts, int S, const void* w, int rows, int H, float eps,
                          int out_stride, int res_stride, bool gemma, hipStream_t st);
 int launch_act_glu(void* out, const void* gu, int64_t T, int I, int gu_stride,

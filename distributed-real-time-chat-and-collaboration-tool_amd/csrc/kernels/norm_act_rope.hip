@@ -47,13 +47,34 @@ int launch_embed(void* out, const void* ids, int wide, const void* table, int ro
 // ----------------------------------------------------------------- RMSNorm
 // PARTS: x is the S fp32 partial sums [S][rows][H] of the product ahead, added up here instead of in a pass of
 // its own (4096 columns: 16 rows of 4 parts 4.8 us against 4.7 from bf16 rows, 160 rows of 8 6.5 against 4.9; the pass takes 3 - 8).
-template <int VPT, bool GEMMA, bool RESID, bool PARTS = false>
+// ROUTER: and the logits of the E <= kRouterFuse experts of a mixture, logits[row] = router [E][H] . out[row] in
+// fp32 from the rounded row.  A router of its own reads as few bytes, but waits for the norm, its
+// launch and two round trips: 13 rows of 4096, 16 experts 4.8 + 13.7 us, now 7.9; 224 of 2048 5.0 + 10.0, now 7.6.  The
+// router's rows are asked for ahead of everything, by every row's workgroup: for decode batches only.
+constexpr int kRouterFuse = 32;
+template <int VPT, bool GEMMA, bool RESID, bool PARTS = false, bool ROUTER = false>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(
     bf16_t* __restrict__ out, bf16_t* __restrict__ residual,
     const void* __restrict__ xv, const bf16_t* __restrict__ w, int H,
-    float eps, int x_stride, int out_stride, int res_stride, int S) {
+    float eps, int x_stride, int out_stride, int res_stride, int S, const bf16_t* __restrict__ router = nullptr,
+    float* __restrict__ logits = nullptr, int E = 0) {
   const int row = blockIdx.x;
   const int tid = threadIdx.x;
+  constexpr int RE = 8;  // experts at a time
+  [[maybe_unused]] bf16x8 rw[ROUTER ? 2 : 1][RE][VPT];
+  auto load_router = [&](bf16x8 (&d)[RE][VPT], int e0) {
+#pragma unroll
+    for (int e = 0; e < RE; ++e)
+#pragma unroll
+      for (int i = 0; i < VPT; ++i) {
+        const int idx = (tid + i * 256) * 8;
+        if (idx < H) d[e][i] = load_bf16x8(router + (int64_t)min(e0 + e, E - 1) * H + idx);
+      }
+  };
+  if constexpr (ROUTER) {
+    load_router(rw[0], 0);
+    load_router(rw[1], RE);
+  }
   const bf16_t* xr = (const bf16_t*)xv + (int64_t)row * x_stride;
   float v[VPT][8];
   float ss = 0.f;
@@ -114,9 +135,47 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(
         float ww = bf2f(wv[i][j]);
         if constexpr (GEMMA) ww += 1.f;
         o[j] = f2bf(v[i][j] * rstd * ww);
+        if constexpr (ROUTER) v[i][j] = bf2f(o[j]);
       }
       store_bf16x8(orow + idx, o);
     }
+  }
+  if constexpr (ROUTER) {
+    __shared__ float dots[4][kRouterFuse + RE];
+    const int lane = tid & 63;
+    for (int e0 = 0; e0 < E; e0 += 2 * RE) {
+#pragma unroll
+      for (int z = 0; z < 2; ++z) {
+        if (e0 + z * RE >= E) break;
+        float p[RE];
+#pragma unroll
+        for (int e = 0; e < RE; ++e) {
+          p[e] = 0.f;
+#pragma unroll
+          for (int i = 0; i < VPT; ++i)
+            if ((tid + i * 256) * 8 < H)
+#pragma unroll
+              for (int j = 0; j < 8; ++j) p[e] += v[i][j] * bf2f(rw[z][e][i][j]);
+        }
+        if (e0 + (z + 2) * RE < E) load_router(rw[z], e0 + (z + 2) * RE);
+        // sums over the wave: each step halves the experts of a lane, lane 8 e + .. ends with expert e
+#pragma unroll
+        for (int n = RE / 2, o = 32; n > 0; n >>= 1, o >>= 1)
+#pragma unroll
+          for (int e = 0; e < n; ++e) {
+            const bool hi = lane & o;
+            const float keep = hi ? p[e + n] : p[e], give = hi ? p[e] : p[e + n];
+            p[e] = keep + __shfl_xor(give, o, 64);
+          }
+        float x = p[0];
+        x += __shfl_xor(x, 4, 64);
+        x += __shfl_xor(x, 2, 64);
+        x += __shfl_xor(x, 1, 64);
+        if ((lane & 7) == 0) dots[tid >> 6][e0 + z * RE + (lane >> 3)] = x;
+      }
+    }
+    __syncthreads();
+    if (tid < E) logits[(int64_t)row * E + tid] = dots[0][tid] + dots[1][tid] + dots[2][tid] + dots[3][tid];
   }
 }
 
@@ -131,7 +190,7 @@ static void launch_rmsnorm_t(bf16_t* out, bf16_t* residual, const void* x,
   case N:                                                                    \
     hipLaunchKernelGGL((rmsnorm_kernel<N, GEMMA, RESID, PARTS>), grid, block, \
                        0, st, out, residual, x, w, H, eps, x_stride,          \
-                       out_stride, res_stride, S);                            \
+                       out_stride, res_stride, S, nullptr, nullptr, 0);       \
     break;
   switch (vpt) {
     DRTC_RMS_CASE(1)
@@ -161,6 +220,24 @@ int launch_rmsnorm(void* out, void* residual, const void* x, const void* w,
     if (gemma) launch_rmsnorm_t<true, false>(o, r, x, ww, rows, H, eps, x_stride, out_stride, res_stride, 0, st);
     else launch_rmsnorm_t<false, false>(o, r, x, ww, rows, H, eps, x_stride, out_stride, res_stride, 0, st);
   }
+  return (int)hipGetLastError();
+}
+
+// residual += x [rows][H] (or S > 0: the sum of the fp32 parts x [S][rows][H]); out = norm(residual) * w;
+// logits [rows][E] = out . router
+int launch_rmsnorm_router(void* out, void* residual, const void* x, int S, const void* w, const void* router, float* logits,
+                          int E, int rows, int H, float eps, int x_stride, int out_stride, int res_stride,
+                          hipStream_t st) {
+  const int vpt = (H / 8 + 255) / 256;
+  if (H % 8 || vpt < 1 || vpt > 2 || S < 0 || S > kMaxParts || !residual || E < 1 || E > kRouterFuse) return -1;
+  if (rows == 0) return 0;
+#define DRTC_NORM_ROUTER(V, P)                                                                                    \
+  if (vpt == V && (S > 0) == P)                                                                                   \
+    rmsnorm_kernel<V, false, true, P, true><<<dim3(rows), dim3(256), 0, st>>>(                                    \
+        (bf16_t*)out, (bf16_t*)residual, x, (const bf16_t*)w, H, eps, x_stride, out_stride, res_stride, S,        \
+        (const bf16_t*)router, logits, E);
+  DRTC_NORM_ROUTER(1, false) DRTC_NORM_ROUTER(1, true) DRTC_NORM_ROUTER(2, false) DRTC_NORM_ROUTER(2, true)
+#undef DRTC_NORM_ROUTER
   return (int)hipGetLastError();
 }
 

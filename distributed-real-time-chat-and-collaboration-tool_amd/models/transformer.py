@@ -286,7 +286,10 @@ class TransformerLM:
 
     def _mlp(self, L: dict, x: ops.PendingNorm, decode: bool = False) -> torch.Tensor:
         if self.cfg.is_moe:
-            return self._moe(L, x.materialize(), decode), False
+            xn, logits = x.materialize_router(L["router"])
+            return self._moe(L, xn, decode, logits), False
+        if isinstance(x.x, ops.Parts):
+            x.materialize()
         if ops.fused_glu_ok(x.x, L["gate_up"], self.cfg.act):
             # prefill / decode batches with a fused form: gate_up GEMM with the GLU in its
             # epilogue (gemm_w4, or a tuned gated gemm_xd form)
@@ -350,8 +353,9 @@ class TransformerLM:
             self.ep_overflow.reduce(self.pc.ep_group)
         return logits
 
-    def _moe(self, L: dict, x: torch.Tensor, decode: bool = False) -> torch.Tensor:
-        """Top-k routed experts (Mixtral: softmax over the top-2 logits).
+    def _moe(self, L: dict, x: torch.Tensor, decode: bool = False, logits: torch.Tensor | None = None) -> torch.Tensor:
+        """Top-k routed experts (Mixtral: softmax over the top-2 logits); ``logits``: the router's, where the
+        norm ahead has them already.
 
         GPU: the fused HIP MoE (ops/moe.py: device-side routing + grouped
         MFMA GEMMs, static launch shapes -> the same code runs eagerly in
@@ -371,7 +375,8 @@ class TransformerLM:
             all_gather_into_tensor(out, y.contiguous(), group=pc.ep_group)
             return out
         if ops.on_gpu(x):
-            logits = ops.router_logits(x, L["router"], contiguous=False)  # [E, T] read in place
+            if logits is None:
+                logits = ops.router_logits(x, L["router"], contiguous=False)  # [E, T] read in place
             out = ops.fused_moe(x, logits, L["gate_up"], L["down"],
                                 cfg.experts_per_token, cfg.act, cfg.num_experts,
                                 sh.expert_offset, workspace=self.moe_ws)

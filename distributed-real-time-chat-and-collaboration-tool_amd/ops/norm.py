@@ -3,6 +3,8 @@ stream (+ fused residual add or embedding lookup) Dynamic Tanh: csrc/kernels/nor
 norms in groups: csrc/kernels/norm_group.hip."""
 from __future__ import annotations
 
+import os
+
 import torch
 
 from ._ext import check, hipk, on_gpu, ptr, stream_ptr
@@ -150,6 +152,21 @@ def group_rms(h: torch.Tensor, w: torch.Tensor, groups: int, eps: float,
     return out
 
 
+ROUTER_FUSE_MAX_M = 256  # rows: each reads the router's E rows again
+_fuse_router = os.environ.get("DRTC_FUSED_ROUTER", "1") != "0"
+
+
+def router_fusable(x: torch.Tensor | Parts, residual: torch.Tensor, router: torch.Tensor) -> bool:
+    """Whether the norm ahead of a mixture also computes its router's logits: decode batches and 9 to 32
+    experts (up to 8, every batch takes the same kernel: ``router_logits``) of up to 4096 columns."""
+    rows, H = residual.shape
+    return (_fuse_router and on_gpu(residual) and residual.dtype == router.dtype == x.dtype == torch.bfloat16
+            and 1 <= rows <= ROUTER_FUSE_MAX_M and 9 <= router.shape[0] <= 32 and router.shape[1] == H
+            and router.is_contiguous() and H % 8 == 0 and H <= 4096 and x.shape == residual.shape
+            and residual.stride(1) == 1 and residual.stride(0) % 8 == 0
+            and (isinstance(x, Parts) or x.stride(1) == 1 and x.stride(0) % 8 == 0))
+
+
 class PendingNorm:
     """A pre-norm sublayer input whose RMSNorm has not run yet: norm(x [+
     residual]) * w.  The consumer either fuses the norm into its projection
@@ -161,17 +178,16 @@ class PendingNorm:
 
     __slots__ = ("x", "residual", "w", "eps", "gemma", "_h", "_out", "pc")
 
-    def __init__(self, x: torch.Tensor, residual: torch.Tensor | None, w: torch.Tensor,
+    def __init__(self, x: torch.Tensor | Parts, residual: torch.Tensor | None, w: torch.Tensor,
                  eps: float, gemma: bool, pc=None):
-        """``pc``: a ParallelContext when ``x`` is still a tensor-parallel PARTIAL
+        """``x``: a tensor, or the K slices' sums of the product ahead, which the norm adds up (needs a
+        residual).  ``pc``: a ParallelContext when ``x`` is still a tensor-parallel PARTIAL
         sum: materialize() then runs the all-reduce fused with the residual add
         and the norm (ParallelContext.reduce_norm)."""
         self.x, self.residual, self.w, self.eps, self.gemma = x, residual, w, eps, gemma
         self.pc = pc
         self._h: torch.Tensor | None = None
         self._out: torch.Tensor | None = None
-        if isinstance(x, Parts):  # K slices of the product ahead: added up by the norm
-            self.materialize()
 
     def applied(self, h: torch.Tensor) -> None:
         """Record that a fused consumer computed h = x (+ residual)."""
@@ -190,6 +206,25 @@ class PendingNorm:
             self._h = res if res is not None else self.x  # rmsnorm updated res in place
             self.x, self.residual = self._h, None
         return self._out
+
+    def materialize_router(self, router: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor | None]:
+        """``materialize()`` and the router logits [rows, E] in fp32 of the normalised rows, computed by the norm;
+        None where it does not (``router_fusable``)."""
+        x, res = self.x, self.residual
+        if self._out is not None or self.pc is not None or res is None or self.gemma or not router_fusable(x, res, router):
+            return self.materialize(), None
+        parts = isinstance(x, Parts)
+        rows, H = res.shape
+        E = router.shape[0]
+        out = torch.empty((rows, H), dtype=res.dtype, device=res.device)
+        logits = torch.empty((rows, E), dtype=torch.float32, device=res.device)
+        src, stride = (x.slab, 0) if parts else (x, x.stride(0))
+        check(hipk().rmsnorm_router(out.data_ptr(), res.data_ptr(), src.data_ptr(), x.slab.shape[0] if parts else 0,
+                                    self.w.data_ptr(), router.data_ptr(), logits.data_ptr(), E, rows, H, float(self.eps),
+                                    stride, out.stride(0), res.stride(0), stream_ptr(res)), "rmsnorm_router")
+        self._out, self._h = out, res  # updated in place
+        self.x, self.residual = res, None
+        return out, logits
 
     def stream(self) -> torch.Tensor:
         if self._h is None:

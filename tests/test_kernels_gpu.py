@@ -1141,3 +1141,24 @@ def test_step_begin_refuses_rows_beyond_the_batch(hipk):
     ops.step_begin(*args)
     want = torch.where(src < 0, 2, torch.where(src == 0, 1, -1))
     assert torch.equal(args[0].cpu().long(), want)
+
+
+@pytest.mark.parametrize("rows,H,E", [(1, 128, 9), (13, 4096, 16), (224, 2048, 17), (256, 4096, 32), (5, 2056, 20)])
+@pytest.mark.parametrize("parts", [0, 3, 8])
+def test_norm_with_router(hipk, rows, H, E, parts):
+    """RMS norm after the residual add (of a bf16 row, or of K slices' sums) with the router's logits in the same
+    launch: the row as without them, the logits against 64 bits of the rounded row (fp32 sums of H products)."""
+    g = torch.Generator(device="cuda").manual_seed(rows + E)
+    wide = torch.randn(rows, H + 8, device="cuda", generator=g).to(torch.bfloat16)
+    x = wide[:, :H]
+    if parts:
+        x = ops.Parts(torch.randn(parts, rows, H, device="cuda", generator=g), torch.bfloat16)
+    res = torch.randn(rows, H, device="cuda", generator=g).to(torch.bfloat16)
+    w = (1 + 0.1 * torch.randn(H, device="cuda", generator=g)).to(torch.bfloat16)
+    r = (torch.randn(E, H, device="cuda", generator=g) / H ** 0.5).to(torch.bfloat16)
+    a, b = res.clone(), res.clone()
+    y, lg = ops.PendingNorm(x, a, w, 1e-5, False).materialize_router(r)
+    assert torch.equal(y, ops.PendingNorm(x, b, w, 1e-5, False).materialize()) and torch.equal(a, b)
+    assert (lg.double() - y.double() @ r.double().t()).abs().max() <= 1e-5
+    none = ops.PendingNorm(x, b, w, 1e-5, False).materialize_router(r[:8].contiguous())
+    assert none[1] is None
