@@ -72,6 +72,10 @@ struct MoeOptions {
   const void* y = nullptr;
   int ldy = 0;
   int W = 0;
+  // or a residual stream [T, H] that the result is added to in place; out is then its RMS norm times norm_w
+  void* residual = nullptr;
+  const void* norm_w = nullptr;
+  float eps = 0.f;
   int y_parts = 0;  // > 0: y is that many fp32 partial sums [y_parts][T][ldy]
 };
 // variant 0 / 1 / 2: the moe.hip grouped GEMMs; 3: gemm_xd grouped mode with xd forms gu_form

@@ -994,6 +994,78 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(
   }
 }
 
+// The combine with the residual add and RMS norm behind it: residual[t] += sum_j w z, out = norm(residual[t]) * nw; one
+// workgroup to a token, VPT vectors of 8 columns a thread.  In one launch: 224 tokens of 2048 4.7 + 4.8 -> 5.0 us,
+// 12288 of 4096 91 + 59 -> 124.
+template <int VPT>
+__global__ __launch_bounds__(256) void moe_combine_norm_kernel(
+    bf16_t* __restrict__ out, bf16_t* __restrict__ residual, const bf16_t* __restrict__ nw, float eps,
+    const bf16_t* __restrict__ zbuf, const bf16_t* __restrict__ zbuf2, const float* __restrict__ topk_w,
+    const int* __restrict__ inv_pos, const int* __restrict__ local_range, int H, int k) {
+  const int t = blockIdx.x, tid = threadIdx.x;
+  const int lo = local_range[0], hi = local_range[1];
+  bf16x8 wv[VPT], rv[VPT];
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int c = (tid + 256 * i) * 8;
+    if (c < H) {
+      wv[i] = load_bf16x8(nw + c);
+      rv[i] = load_bf16x8(residual + (int64_t)t * H + c);
+    }
+  }
+  float s[VPT][8], ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i)
+#pragma unroll
+    for (int q = 0; q < 8; ++q) s[i][q] = 0.f;
+  for (int j = 0; j < k; ++j) {
+    const int p = inv_pos[t * k + j];
+    if (p < lo || p >= hi) continue;  // pair routed to another EP rank
+    const float w = topk_w[t * k + j];
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+      const int c = (tid + 256 * i) * 8;
+      if (c >= H) continue;
+      const bf16x8 z = load_bf16x8(zbuf + (int64_t)p * H + c);
+      if (zbuf2 != nullptr) {  // down split over K: the two halves' partial products
+        const bf16x8 z2 = load_bf16x8(zbuf2 + (int64_t)p * H + c);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) s[i][q] += w * (bf2f(z[q]) + bf2f(z2[q]));
+      } else {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) s[i][q] += w * bf2f(z[q]);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int c = (tid + 256 * i) * 8;
+    if (c >= H) continue;
+    bf16x8 r;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      r[q] = f2bf(s[i][q] + bf2f(rv[i][q]));
+      s[i][q] = bf2f(r[q]);
+      ss += s[i][q] * s[i][q];
+    }
+    store_bf16x8(residual + (int64_t)t * H + c, r);
+  }
+  __shared__ float red[4];
+  ss = wave_sum(ss);
+  if ((tid & 63) == 0) red[tid >> 6] = ss;
+  __syncthreads();
+  const float rstd = rsqrtf((red[0] + red[1] + red[2] + red[3]) / (float)H + eps);
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int c = (tid + 256 * i) * 8;
+    if (c >= H) continue;
+    bf16x8 o;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) o[q] = f2bf(s[i][q] * rstd * bf2f(wv[i][q]));
+    store_bf16x8(out + (int64_t)t * H + c, o);
+  }
+}
+
 // Whether grouped gemm_xd form `form` takes an expert GEMM with N output columns (gated: I)
 // and reduction K (the 1x4 / 2x4 / 2x8 tiles launch_gemm_xd_grouped builds).
 static bool moe_xd_ok(int form, int N, int K, bool glu) {
@@ -1026,6 +1098,7 @@ int launch_moe(void* out, const void* x, const void* router_logits, const void* 
   if (opt.stream && (opt.y == nullptr || opt.W < 1 || opt.W > H || opt.ldy < opt.W || e_off != 0 ||
                      e_local != E))
     return -1;
+  if (opt.residual && (opt.stream || opt.f32 || !opt.norm_w || H > 8192)) return -1;
   if (opt.y_parts && (!opt.stream || opt.f32 || opt.y_parts < 0 || opt.y_parts > kMaxParts || opt.W % 8 || opt.ldy % 8)) return -1;
   if (opt.groups < 1 || opt.groups > kMoeMaxGroups || E % opt.groups || opt.keep < 1 ||
       opt.keep > opt.groups || k > opt.keep * (E / opt.groups))
@@ -1275,6 +1348,17 @@ int launch_moe(void* out, const void* x, const void* router_logits, const void* 
         (bf16_t*)out, opt.stream, opt.y, opt.ldy, opt.y_parts, zbuf,
         dn_split ? (const bf16_t*)zbuf2 : nullptr, topk_w, inv_pos, opt.W, H, k);
     return (int)hipGetLastError();
+  }
+  if (opt.residual) {
+#define DRTC_COMBINE_NORM(V)                                                                                           \
+  if (H <= 2048 * V) {                                                                                                 \
+    moe_combine_norm_kernel<V><<<dim3(T), dim3(256), 0, st>>>(                                                         \
+        (bf16_t*)out, (bf16_t*)opt.residual, (const bf16_t*)opt.norm_w, opt.eps, zbuf,                                 \
+        dn_split ? (const bf16_t*)zbuf2 : nullptr, topk_w, inv_pos, local_range, H, k);                                \
+    return (int)hipGetLastError();                                                                                     \
+  }
+    DRTC_COMBINE_NORM(1) DRTC_COMBINE_NORM(2) DRTC_COMBINE_NORM(4)
+#undef DRTC_COMBINE_NORM
   }
   hipLaunchKernelGGL(moe_combine_kernel, dim3(T), dim3(256), 0, st, (bf16_t*)out, zbuf,
                      dn_split ? (const bf16_t*)zbuf2 : nullptr, topk_w, inv_pos, local_range, T, H,

@@ -401,6 +401,24 @@ class TransformerLM:
             return self.pc.all_reduce_ep(out)
         return self.pc.all_reduce_tp(out)
 
+    def _moe_norm_ok(self, x: ops.PendingNorm) -> bool:
+        """Whether the experts' combine takes the residual add and the next norm along: one rank (their sum is
+        complete there), and more than the row whose norm its projection computes."""
+        h = x.x if x.residual is None else x.residual
+        return (self.pc.tp_size == 1 and self.pc.ep_size == 1 and not self.cfg.gemma_norm
+                and isinstance(h, torch.Tensor) and h.shape[0] > 1 and ops.moe_norm_ok(h))
+
+    def _moe_norm(self, L: dict, x: ops.PendingNorm, nxt: torch.Tensor) -> ops.PendingNorm:
+        """The experts of a layer, the residual add and the norm ``nxt`` behind it."""
+        cfg = self.cfg
+        xn, logits = x.materialize_router(L["router"])
+        if logits is None:
+            logits = ops.router_logits(xn, L["router"], contiguous=False)  # [E, T] read in place
+        h = x.stream()
+        out = ops.fused_moe(xn, logits, L["gate_up"], L["down"], cfg.experts_per_token, cfg.act, cfg.num_experts,
+                            self.sh.expert_offset, workspace=self.moe_ws, residual=h, norm_w=nxt, eps=cfg.rms_eps)
+        return ops.PendingNorm.done(out, h, nxt, cfg.rms_eps)
+
     def _layers(self, h: torch.Tensor, attn_fn, decode: bool = False) -> torch.Tensor:
         """Pre-norm residual stack.  Each sublayer receives its input as an
         ops.PendingNorm (norm(x + residual) not yet computed), so a small
@@ -416,8 +434,11 @@ class TransformerLM:
             o, added, *part = attn_fn(i, L, x)
             x = ops.PendingNorm(o, None if added else x.stream(), L["ln_post"], cfg.rms_eps,
                                 cfg.gemma_norm, pc=self.pc if part and part[0] else None)
-            m, added, *part = self._mlp(L, x, decode)
             nxt = self.layers[i + 1]["ln_in"] if i + 1 < n else self.final_norm
+            if cfg.is_moe and self._moe_norm_ok(x):
+                x = self._moe_norm(L, x, nxt)
+                continue
+            m, added, *part = self._mlp(L, x, decode)
             x = ops.PendingNorm(m, None if added else x.stream(), nxt, cfg.rms_eps, cfg.gemma_norm,
                                 pc=self.pc if part and part[0] else None)
         return x.materialize()

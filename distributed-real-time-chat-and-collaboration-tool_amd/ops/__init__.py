@@ -26,7 +26,7 @@ from .latent import (LatentDecodeWorkspace, PortionKeys, build_interleaved_rope,
                      latent_decode_attention, latent_gather, latent_prefill_attention,
                      latent_prep, latent_qtile, latent_width, portion_tiles, window_reach)
 from .memory import MemoryWeights, memory_decode, memory_scan, memory_slices
-from .moe import fused_moe, fused_moe_ref, router_logits, router_logits_f32
+from .moe import fused_moe, fused_moe_ref, moe_norm_ok, router_logits, router_logits_f32
 from .norm import PendingNorm, dyt, dyt_ref, embed, group_rms, rmsnorm, rmsnorm_ref
 from .norm_conv import (MAX_TAPS, ConvTiles, LayerNorm, conv_tile_rows, norm_conv, sinusoid_turns,
                         softcap_)
@@ -40,7 +40,7 @@ __all__ = [
     "on_gpu", "reference_mode", "linear", "linear_parts", "Parts", "norm_linear", "glu_linear", "norm_glu", "w4_glu_ok",
     "fused_glu_ok",
     "mfma_gemm", "linear_residual", "residual_fusable", "PendingNorm", "fused_moe", "router_logits",
-    "fused_moe_ref", "act_glu", "act_glu_ref", "KV_BLOCK", "DecodeWorkspace",
+    "fused_moe_ref", "moe_norm_ok", "act_glu", "act_glu_ref", "KV_BLOCK", "DecodeWorkspace",
     "decode_partitioning", "paged_decode_attention", "paged_decode_attention_rope",
     "paged_decode_ref", "prefill_attention", "prefill_attention_ref", "prefill_tiles",
     "set_prefill_persist", "rmsnorm", "rmsnorm_ref", "build_rope_cache", "rope_kv_",

@@ -20,7 +20,7 @@ import os
 import torch
 import torch.nn.functional as F
 
-from ._ext import check, hipk, on_gpu, stream_ptr
+from ._ext import check, hipk, on_gpu, ptr, stream_ptr
 from .activation import ACTS, act_glu_ref
 from .gemm import Parts
 
@@ -149,18 +149,28 @@ def router_logits_f32(x: torch.Tensor, w_router: torch.Tensor) -> torch.Tensor:
     return out.t()
 
 
+def moe_norm_ok(residual: torch.Tensor) -> bool:
+    """Whether ``fused_moe`` takes the residual add and RMS norm behind it along."""
+    return (on_gpu(residual) and residual.dtype == torch.bfloat16 and residual.is_contiguous()
+            and residual.shape[1] <= 8192)
+
+
 def fused_moe(x: torch.Tensor, router_logits: torch.Tensor, w_gu: torch.Tensor,
               w_dn: torch.Tensor, top_k: int, act: str = "silu", num_experts: int | None = None,
               e_off: int = 0, workspace: torch.Tensor | None = None,
               out: torch.Tensor | None = None, variant: int | None = None,
               gu_form: int | None = None, dn_form: int | None = None, groups: int = 1,
               keep: int = 1, limit: float = 0.0, stream: torch.Tensor | None = None,
-              y: torch.Tensor | None = None) -> torch.Tensor:
+              y: torch.Tensor | None = None, residual: torch.Tensor | None = None,
+              norm_w: torch.Tensor | None = None, eps: float = 0.0) -> torch.Tensor:
     """y[t] = sum_j w[t,j] * down_e(act(gate_e x_t) * up_e x_t) over the top-k experts; act
     "relu2": down_e(relu(up_e x_t)^2), w_gu [E_local, I, H].
 
     ``stream`` [T, W <= H] fp32: the result is added to it together with ``y`` [T, W] (or its ``Parts``), and the
     stream is returned in x's type (itself in fp32).
+
+    ``residual`` [T, H] bf16 (``moe_norm_ok``): the result is added to it, and its RMS norm times ``norm_w`` [H] is
+    returned.
 
     x [T, H] bf16 (H % 128 == 0, I % 64 == 0) or fp32 (any size); router_logits [T, E] bf16 or
     fp32, row-major or the transposed view of an [E, T] tensor (``router_logits(...,
@@ -208,7 +218,10 @@ def fused_moe(x: torch.Tensor, router_logits: torch.Tensor, w_gu: torch.Tensor,
         assert stream.dtype == torch.float32 and y.dtype == x.dtype and (y_parts or y.stride(1) == 1)
         assert out is None and (e_off, e_local) == (0, E)
         out = stream if f32 else x.new_empty(T, W)
-    elif out is None:
+    if residual is not None:
+        assert moe_norm_ok(residual) and residual.shape == (T, H) and residual.dtype == x.dtype and stream is None
+        assert norm_w.shape == (H,) and norm_w.dtype == x.dtype and norm_w.is_contiguous()
+    if out is None:
         out = torch.empty_like(x)
     assert out.is_contiguous() and out.shape == (T, W)
     chunk = min(T, MOE_CHUNK) if T else 1
@@ -240,6 +253,7 @@ def fused_moe(x: torch.Tensor, router_logits: torch.Tensor, w_gu: torch.Tensor,
                       int(router_logits.dtype == torch.float32), groups, keep, float(limit),
                       0 if stream is None else stream[t0].data_ptr(),
                       0 if stream is None else slab_y.data_ptr() if y_parts else y[t0].data_ptr(),
-                      0 if stream is None else W if y_parts else y.stride(0), W, y_parts, st), "moe")
+                      0 if stream is None else W if y_parts else y.stride(0), W, y_parts,
+                      0 if residual is None else residual[t0].data_ptr(), ptr(norm_w), float(eps), st), "moe")
     return out
 

@@ -189,6 +189,13 @@ class PendingNorm:
         self._h: torch.Tensor | None = None
         self._out: torch.Tensor | None = None
 
+    @classmethod
+    def done(cls, out: torch.Tensor, h: torch.Tensor, w: torch.Tensor, eps: float) -> PendingNorm:
+        """The norm ``out`` of the stream ``h``, computed by the op ahead."""
+        p = cls(h, None, w, eps, False)
+        p._out, p._h = out, h
+        return p
+
     def applied(self, h: torch.Tensor) -> None:
         """Record that a fused consumer computed h = x (+ residual)."""
         self._h, self.x, self.residual = h, h, None

@@ -1162,3 +1162,26 @@ def test_norm_with_router(hipk, rows, H, E, parts):
     assert (lg.double() - y.double() @ r.double().t()).abs().max() <= 1e-5
     none = ops.PendingNorm(x, b, w, 1e-5, False).materialize_router(r[:8].contiguous())
     assert none[1] is None
+
+
+@pytest.mark.parametrize("T,H,I,E,k,variant", [(2, 128, 64, 4, 2, -1), (37, 2176, 128, 9, 3, 6), (64, 4096, 128, 16, 4, 6),
+                                               (1030, 256, 256, 4, 2, 4), (300, 8192, 64, 3, 1, 1)])
+def test_moe_with_residual_and_norm(hipk, T, H, I, E, k, variant):
+    """The combine that adds to the residual stream and norms it, against the layer's output, an add and a norm (the
+    output is rounded to bf16 there, and the sum again); the split down projection of variant 4 too."""
+    g = torch.Generator(device="cuda").manual_seed(T + H)
+    x = torch.randn(T, H, device="cuda", generator=g).to(torch.bfloat16)
+    gu = (torch.randn(E, 2 * I, H, device="cuda", generator=g) / H ** 0.5).to(torch.bfloat16)
+    dn = (torch.randn(E, H, I, device="cuda", generator=g) / I ** 0.5).to(torch.bfloat16)
+    lg = torch.randn(T, E, device="cuda", generator=g)
+    w = (1 + 0.1 * torch.randn(H, device="cuda", generator=g)).to(torch.bfloat16)
+    res = torch.randn(T, H, device="cuda", generator=g).to(torch.bfloat16)
+    y = ops.fused_moe(x, lg, gu, dn, k, variant=variant).double()
+    h = res.clone()
+    out = ops.fused_moe(x, lg, gu, dn, k, variant=variant, residual=h, norm_w=w, eps=1e-5)
+    want = y + res.double()
+    near = 2.0 ** -8
+    assert ((h.double() - want).abs() <= near * (want.abs() + y.abs()) + 1e-5).all()
+    hd = h.double()
+    norm = hd * torch.rsqrt((hd * hd).mean(-1, keepdim=True) + 1e-5) * w.double()
+    assert ((out.double() - norm).abs() <= near * norm.abs() + 1e-4).all()
