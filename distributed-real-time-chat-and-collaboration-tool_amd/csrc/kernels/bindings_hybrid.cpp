@@ -71,7 +71,7 @@ void bind_hybrid(py::module_& m) {
     const Fields f{d};
     drtc::SideNormArgs a{};
     PTR(out); VAL(ldo); PTR(h); PTR(y); VAL(ldy); PTR(yw); PTR(ids); PTR(embed); VAL(embed_scale);
-    PTR(w); VAL(W); VAL(eps); VAL(rows);
+    PTR(w); VAL(W); VAL(eps); VAL(rows); PTR(router); VAL(ldr); PTR(logits); VAL(E);
     return drtc::launch_side_norm(f32, a, S(st));
   });
   m.def("stream_add", [](int f32, u64 out, u64 h, u64 y, int64_t ldy, int rows, int W, u64 st) {

@@ -365,6 +365,10 @@ struct SideNormArgs {
   int W;
   float eps;
   int rows;
+  const void* router;     // [E, ldr], W of the columns: its logits [rows, E] for the output rows (bf16); or null
+  int64_t ldr;
+  float* logits;
+  int E;
 };
 int launch_side_norm(int f32, const SideNormArgs& a, hipStream_t st);
 int launch_stream_add(int f32, void* out, float* h, const void* y, int64_t ldy, int rows, int W,

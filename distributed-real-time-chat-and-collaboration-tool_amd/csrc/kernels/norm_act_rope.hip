@@ -13,6 +13,7 @@
 //    cos/sin come from a host-precomputed fp32 table (no device trig).
 #include "common.h"
 #include "launchers.h"
+#include "router.h"
 
 namespace drtc {
 
@@ -51,7 +52,6 @@ int launch_embed(void* out, const void* ids, int wide, const void* table, int ro
 // fp32 from the rounded row.  A router of its own reads as few bytes, but waits for the norm, its
 // launch and two round trips: 13 rows of 4096, 16 experts 4.8 + 13.7 us, now 7.9; 224 of 2048 5.0 + 10.0, now 7.6.  The
 // router's rows are asked for ahead of everything, by every row's workgroup: for decode batches only.
-constexpr int kRouterFuse = 32;
 template <int VPT, bool GEMMA, bool RESID, bool PARTS = false, bool ROUTER = false>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(
     bf16_t* __restrict__ out, bf16_t* __restrict__ residual,
@@ -60,21 +60,8 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(
     float* __restrict__ logits = nullptr, int E = 0) {
   const int row = blockIdx.x;
   const int tid = threadIdx.x;
-  constexpr int RE = 8;  // experts at a time
-  [[maybe_unused]] bf16x8 rw[ROUTER ? 2 : 1][RE][VPT];
-  auto load_router = [&](bf16x8 (&d)[RE][VPT], int e0) {
-#pragma unroll
-    for (int e = 0; e < RE; ++e)
-#pragma unroll
-      for (int i = 0; i < VPT; ++i) {
-        const int idx = (tid + i * 256) * 8;
-        if (idx < H) d[e][i] = load_bf16x8(router + (int64_t)min(e0 + e, E - 1) * H + idx);
-      }
-  };
-  if constexpr (ROUTER) {
-    load_router(rw[0], 0);
-    load_router(rw[1], RE);
-  }
+  [[maybe_unused]] RouterDots<ROUTER ? VPT : 1> dots;
+  if constexpr (ROUTER) dots.start(router, H, H, E);
   const bf16_t* xr = (const bf16_t*)xv + (int64_t)row * x_stride;
   float v[VPT][8];
   float ss = 0.f;
@@ -140,43 +127,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(
       store_bf16x8(orow + idx, o);
     }
   }
-  if constexpr (ROUTER) {
-    __shared__ float dots[4][kRouterFuse + RE];
-    const int lane = tid & 63;
-    for (int e0 = 0; e0 < E; e0 += 2 * RE) {
-#pragma unroll
-      for (int z = 0; z < 2; ++z) {
-        if (e0 + z * RE >= E) break;
-        float p[RE];
-#pragma unroll
-        for (int e = 0; e < RE; ++e) {
-          p[e] = 0.f;
-#pragma unroll
-          for (int i = 0; i < VPT; ++i)
-            if ((tid + i * 256) * 8 < H)
-#pragma unroll
-              for (int j = 0; j < 8; ++j) p[e] += v[i][j] * bf2f(rw[z][e][i][j]);
-        }
-        if (e0 + (z + 2) * RE < E) load_router(rw[z], e0 + (z + 2) * RE);
-        // sums over the wave: each step halves the experts of a lane, lane 8 e + .. ends with expert e
-#pragma unroll
-        for (int n = RE / 2, o = 32; n > 0; n >>= 1, o >>= 1)
-#pragma unroll
-          for (int e = 0; e < n; ++e) {
-            const bool hi = lane & o;
-            const float keep = hi ? p[e + n] : p[e], give = hi ? p[e] : p[e + n];
-            p[e] = keep + __shfl_xor(give, o, 64);
-          }
-        float x = p[0];
-        x += __shfl_xor(x, 4, 64);
-        x += __shfl_xor(x, 2, 64);
-        x += __shfl_xor(x, 1, 64);
-        if ((lane & 7) == 0) dots[tid >> 6][e0 + z * RE + (lane >> 3)] = x;
-      }
-    }
-    __syncthreads();
-    if (tid < E) logits[(int64_t)row * E + tid] = dots[0][tid] + dots[1][tid] + dots[2][tid] + dots[3][tid];
-  }
+  if constexpr (ROUTER) dots.finish(v, logits + (int64_t)row * E);
 }
 
 template <bool GEMMA, bool RESID, bool PARTS = false>

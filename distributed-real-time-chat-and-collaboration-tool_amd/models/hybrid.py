@@ -404,9 +404,11 @@ class HybridLM:
                              embed=self.embed, embed_scale=cfg.embed_scale, width=width,
                              dtype=self.dtype)
 
-    def _experts(self, L: dict, l, x: torch.Tensor, **kw) -> torch.Tensor:
+    def _experts(self, L: dict, l, x: torch.Tensor, logits: torch.Tensor | None = None, **kw) -> torch.Tensor:
         e = l.experts
-        return ops.fused_moe(x, ops.router_logits_f32(x, L["router"]), L["experts_in"],
+        if logits is None:
+            logits = ops.router_logits_f32(x, L["router"])
+        return ops.fused_moe(x, logits, L["experts_in"],
                              L["experts_out"], e.top, self.cfg.act, e.count, workspace=self.moe_ws,
                              groups=e.groups, keep=e.keep, limit=l.limit, **kw)
 
@@ -447,8 +449,11 @@ class HybridLM:
         z, zn, last = None, None, len(self.layers) - 1
         for i, (l, L) in enumerate(zip(cfg.layers, self.layers)):
             first = {"ids": ids, "embed": self.embed, "embed_scale": cfg.embed_scale} if i == 0 else {}
-            wide = ops.side_norm(h, L["norm1"].w, eps, z, zn, dtype=dt,
+            # a prompt's last layer goes on with a few of these rows, larger steps have a router of their own
+            fuse = bool(l.experts) and not (i == last and rows is not None) and ops.side_router_ok(h, L["router"], dt)
+            wide = ops.side_norm(h, L["norm1"].w, eps, z, zn, dtype=dt, router=L["router"] if fuse else None,
                                  width=self._moe_width if l.experts else None, **first)
+            wide, logits = wide if fuse else (wide, None)
             x, mw, off = wide[:, :W], L["mixer"].width, pad_to(L["mixer"].width)
             a = torch.empty((ids.shape[0], L["out"].shape[1]), dtype=dt, device=self.device)
             if off > mw:
@@ -460,7 +465,7 @@ class HybridLM:
             if "up" in L:
                 ops.squared_relu(x, L["up"], a[:, off:])
             if l.experts:
-                x = self._experts(L, l, wide, stream=h, y=ops.linear_parts(a, L["out"]))
+                x = self._experts(L, l, wide, logits, stream=h, y=ops.linear_parts(a, L["out"]))
             else:
                 x = ops.stream_add(h, ops.linear(a, L["out"]))
             z = zn = None

@@ -9,7 +9,8 @@ shape (M, N, K, row stride of x) ONCE to a route, cached per shape (``route``):
   "skinny"  gemv.hip weight-streaming kernels (M <= 16)     decode buckets where the table (or
                                                             ``skinny_variant`` untuned) says so
             gemm_stream.hip (variant STREAM, M <= 64)       where ``stream_ok`` says so
-  "midm"    gemm_midm.hip medium-M kernel (M <= 256)        decode buckets where the table says so;
+  "midm"    gemm_midm.hip medium-M kernel (M <= 256)        decode buckets where the table says so, short K
+                                                            (``brief_ok``: 100 x fragments + slices);
                                                             K slices' sums for the op behind
                                                             (``linear_parts``): ``parts_form``
   "xd"      gemm_xd.hip: 128-row tiles, full K, tile order  decode buckets where the table says so
@@ -239,6 +240,8 @@ def _resolve(M: int, N: int, K: int, ldx: int) -> tuple[str, int]:
     wide = wide_form(M, N, K)
     if wide and not (found is not None and found[1][3]):  # (entries of gemm_xd: measured against its other forms)
         return ("xd", wide)
+    if brief_ok(M, N, K) and ldx % 8 == 0:
+        return ("midm", 201)
     # the rule goes ahead of the table, but for entries that were measured faster ("stream": 0)
     if ldx % 8 == 0 and stream_ok(M, N, K) and (found is None or (found[0], N, K, ldx) not in _kept):
         return ("skinny", STREAM)
@@ -260,6 +263,14 @@ def _resolve(M: int, N: int, K: int, ldx: int) -> tuple[str, int]:
                 return ("lt", algo)
     v = skinny_variant(M, N, K, ldx)
     return ("skinny", v) if v else ("torch", 0)
+
+
+def brief_ok(M: int, N: int, K: int) -> bool:
+    """Whether a product of a few K tiles takes gemm_midm in one slice and 64 columns to a workgroup: all of it is
+    launch, one round trip and the store.  us, the table's pick / this: 2048 x 128, 48 rows 6.6 / 3.8, 128 6.6 / 4.9, 256 7.1 /
+    6.8; 4096 x 256, 48 rows 6.4 / 4.4, 128 5.7 / 5.6, 200 6.4 / 7.1; 16 rows 2.6 / 3.5."""
+    return (_midm_enabled and _enabled and K % 64 == 0 and K <= 256 and 17 <= M <= 256 and M * K <= 32768
+            and N % 64 == 0 and 1024 <= N <= 8192)
 
 
 def wide_form(M: int, N: int, K: int) -> int:
@@ -326,8 +337,8 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         return y
     if kind == "skinny" and (arg != STREAM or _aligned(x, w)):
         return skinny_linear(x, w, arg)
-    if kind == "midm":
-        return midm_gemm(x, w, "store", splits=arg)
+    if kind == "midm" and (arg < 100 or _aligned(x, w)):
+        return midm_gemm(x, w, "store", splits=arg % 100, nf=arg // 100 or 4)
     if kind == "xd" and _aligned(x, w):
         return xd_gemm(x, w, form=arg)
     return F.linear(x, w)
@@ -1175,7 +1186,7 @@ def midm_gemm(x: torch.Tensor, w: torch.Tensor, epi: str = "store",
     N = w.shape[0]
     assert x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_cuda
     assert x.stride(1) == 1 and w.is_contiguous() and w.shape[1] == K
-    assert midm_supported(M, N, K, epi), (M, N, K, epi)
+    assert midm_supported(M, N, K, epi) or nf == 2 and N % 64 == 0 and midm_supported(M, 2 * N, K, epi), (M, N, K, epi)
     S = splits or midm_splits(M, N, K)
     while S > 1 and S * M * N * 4 > WS_SLAB_BYTES:
         S //= 2

@@ -11,15 +11,25 @@ import math
 import torch
 
 from ._ext import check, hipk, on_gpu, ptr, stream_ptr
+from .norm import ROUTER_FUSE_MAX_M, _fuse_router
+
+
+def side_router_ok(h: torch.Tensor, router: torch.Tensor, dtype) -> bool:
+    """Whether ``side_norm`` computes a router's logits along: decode batches and up to 32 experts."""
+    rows, W = h.shape
+    return (_fuse_router and on_gpu(h) and dtype == router.dtype == torch.bfloat16 and 1 <= rows <= ROUTER_FUSE_MAX_M
+            and router.shape[0] <= 32 and W % 8 == 0 and W <= 4096 and router.stride(1) == 1
+            and router.stride(0) % 8 == 0 and router.data_ptr() % 16 == 0)
 
 
 def side_norm(h: torch.Tensor, w: torch.Tensor, eps: float, y: torch.Tensor | None = None,
               y_norm: torch.Tensor | None = None, ids: torch.Tensor | None = None,
               embed: torch.Tensor | None = None, embed_scale: float = 1.0,
-              width: int | None = None, dtype=torch.bfloat16) -> torch.Tensor:
+              width: int | None = None, dtype=torch.bfloat16, router: torch.Tensor | None = None):
     """Layer norm (weight w, no bias) of the 32-bit residual stream h [rows, W], after
     h += y / sqrt(mean(y^2) + eps) * y_norm or h = embed_scale * embed[ids]; h is updated in
-    place.  w, y_norm: float32.  ``width`` > W: zeros behind the first W output columns."""
+    place.  w, y_norm: float32.  ``width`` > W: zeros behind the first W output columns.  ``router`` [E, width]
+    (``side_router_ok``): -> (output, its logits [rows, E] of the output rows in fp32)."""
     rows, W = h.shape
     N = width or W
     if not on_gpu(h):
@@ -40,11 +50,17 @@ def side_norm(h: torch.Tensor, w: torch.Tensor, eps: float, y: torch.Tensor | No
                            and embed.is_contiguous() and embed.dtype == dtype
                            and embed.shape[1] == W)
     out = torch.empty((rows, N), dtype=dtype, device=h.device)
+    logits, E = None, 0
+    if router is not None:
+        E = router.shape[0]
+        assert side_router_ok(h, router, dtype) and router.shape[1] >= W
+        logits = torch.empty((rows, E), dtype=torch.float32, device=h.device)
     check(hipk().side_norm(int(dtype == torch.float32), dict(
         out=out.data_ptr(), ldo=N, h=h.data_ptr(), y=ptr(y), ldy=y.stride(0) if y is not None else 0,
         yw=ptr(y_norm), ids=ptr(ids), embed=ptr(embed), embed_scale=float(embed_scale),
-        w=w.data_ptr(), W=W, eps=float(eps), rows=rows), stream_ptr(h)), "side_norm")
-    return out
+        w=w.data_ptr(), W=W, eps=float(eps), rows=rows, router=ptr(router), ldr=router.stride(0) if E else 0,
+        logits=ptr(logits), E=E), stream_ptr(h)), "side_norm")
+    return out if router is None else (out, logits)
 
 
 def stream_add(h: torch.Tensor, y: torch.Tensor) -> torch.Tensor:

@@ -438,3 +438,18 @@ def test_product_parts(hipk, M, N, K, form):
         assert hipk.midm_gemm(0, x.data_ptr(), w.data_ptr(), 0, 32, N, K, x.stride(0), N, 0, 4, s, nf, few.data_ptr(),
                               few.numel() * 4, torch.cuda.current_stream().cuda_stream) == 0
         assert torch.equal(few, slab[:, :32])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(17, 1024, 64), (64, 4096, 256), (128, 1088, 256), (170, 2048, 192), (256, 2048, 128)])
+def test_short_k_products(hipk, M, N, K):
+    """Products of one to four K tiles, fewer than the ring has stages, as linear routes them; rows of a wider
+    buffer.  bf16 rounding of the result; unaligned rows through another route."""
+    G.reset()
+    assert G.brief_ok(M, N, K) and not G.brief_ok(M, N, K + 256) and not G.brief_ok(16, N, K) and not G.brief_ok(M, 512, K)
+    g = torch.Generator(device="cuda").manual_seed(M)
+    wide = torch.randn(M, K + 72, device="cuda", generator=g).to(torch.bfloat16)
+    w = (torch.randn(N, K, device="cuda", generator=g) / K ** 0.5).to(torch.bfloat16)
+    for x in (wide[:, 8:K + 8], wide[:, 3:K + 3], wide[:, :K].contiguous()):
+        got, want = ops.linear(x, w).double(), x.double() @ w.double().t()
+        assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all()

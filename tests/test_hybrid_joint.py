@@ -477,3 +477,22 @@ def test_squared_relu_on_xcd_tiles(form):
     ops.gemm.xd_gemm(x, w, "relu2", out=a[:, 8:8 + N], form=form)
     close(a[:, 8:8 + N], torch.relu(x64 @ w64.T).square(), 1e-2)
     assert (a[:, :8] == 5).all() and (a[:, 8 + N:] == 5).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,W,N,E", [(1, 64, 64, 1), (13, 2048, 2048, 20), (224, 4096, 4096, 32), (256, 1032, 1152, 9)])
+@pytest.mark.parametrize("y", [False, True])
+def test_side_norm_with_router(rows, W, N, E, y):
+    """The norm with a router's logits in the same launch: the rows as without them, the logits against 64 bits of
+    the rounded rows (fp32 sums of W products); a router wider than the stream reads its first W columns."""
+    g = torch.Generator(device="cuda").manual_seed(rows + W)
+    h = torch.randn(rows, W, device="cuda", generator=g)
+    w = 1 + 0.1 * torch.randn(W, device="cuda", generator=g)
+    kw = {"y": torch.randn(rows, W, device="cuda", generator=g).to(torch.bfloat16), "y_norm": w} if y else {}
+    r = torch.zeros(E, N, device="cuda", dtype=torch.bfloat16)
+    r[:, :W] = (torch.randn(E, W, device="cuda", generator=g) / W ** 0.5).to(torch.bfloat16)
+    a, b = h.clone(), h.clone()
+    assert ops.side_router_ok(a, r, torch.bfloat16) and not ops.side_router_ok(a.new_zeros(257, W), r, torch.bfloat16)
+    out, lg = ops.side_norm(a, w, 1e-5, width=N, router=r, **kw)
+    assert torch.equal(out, ops.side_norm(b, w, 1e-5, width=N, **kw)) and torch.equal(a, b)
+    assert (lg.double() - out.double() @ r.double().t()).abs().max() <= 1e-5
