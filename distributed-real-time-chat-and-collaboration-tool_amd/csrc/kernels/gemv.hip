@@ -159,22 +159,26 @@ int launch_skinny_glu_gemm(void* y, const void* gu, const void* w, int M, int N,
 // decode, profiles/r1l_skinny_gemm.md): a win at M = 1 only - at M = 2..4 the
 // per-workgroup re-read of the M x K input costs what the saved launch gains
 // (also with 8 W rows per workgroup), so ops.norm_linear fuses at M = 1.
-template <int MT, int CPW, bool GEMMA, int R>
+//
+// ACT >= 0: w holds gate over up (N rows each), the R rows are R / 2 of either and y = act(gate) * up [M, N]:
+// the next product reads a row instead of making it in each of its workgroups (2048 x 7168, one row: 9.5 us
+// with the activation in it, 7.1 without; this kernel 12.1 and 12.9).
+template <int MT, int CPW, bool GEMMA, int R, int ACT = -1>
 __global__ __launch_bounds__(256) void skinny_norm_gemm_kernel(
     bf16_t* __restrict__ y, bf16_t* __restrict__ h_out, const bf16_t* __restrict__ x,
     const bf16_t* __restrict__ res, const bf16_t* __restrict__ nw,
-    const bf16_t* __restrict__ w, int M, int K, int ldx, int ldr, int ldh, int ldy, float eps) {
-  constexpr int CH = 512;
+    const bf16_t* __restrict__ w, int M, int N, int K, int ldx, int ldr, int ldh, int ldy, float eps) {
+  constexpr int CH = 512, OUT = ACT < 0 ? R : R / 2;  // output columns
   __shared__ float red[4][MT];
   __shared__ float part[4][R * MT];
-  const int n0 = blockIdx.x * R;
+  const int n0 = blockIdx.x * OUT;
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   bf16x8 wa[CPW][R];
 #pragma unroll
   for (int j = 0; j < CPW; ++j)
 #pragma unroll
     for (int r = 0; r < R; ++r)
-      wa[j][r] = load_bf16x8(w + (int64_t)(n0 + r) * K + (wv + 4 * j) * CH + lane * 8);
+      wa[j][r] = load_bf16x8(w + (int64_t)(r < OUT ? n0 + r : N + n0 + r - OUT) * K + (wv + 4 * j) * CH + lane * 8);
   bf16x8 hx[MT][CPW];
   float ss[MT];
 #pragma unroll
@@ -244,51 +248,50 @@ __global__ __launch_bounds__(256) void skinny_norm_gemm_kernel(
   }
   __syncthreads();
   const int t = threadIdx.x;
-  if (t < R * MT) {
+  if (t < OUT * MT) {
     const int r = t / MT, m = t - r * MT;
     if (m < M) {
-      const float s = part[0][t] + part[1][t] + part[2][t] + part[3][t];
+      float s = part[0][t] + part[1][t] + part[2][t] + part[3][t];
+      if constexpr (ACT >= 0) {
+        const int q = t + OUT * MT;
+        s = act_value<ACT>(s) * (part[0][q] + part[1][q] + part[2][q] + part[3][q]);
+      }
       y[(int64_t)m * ldy + n0 + r] = f2bf(s);
     }
   }
 }
 
-template <int MT, bool GEMMA>
+template <int MT, bool GEMMA, int ACT = -1>
 static int launch_norm_mt(bf16_t* y, bf16_t* h, const bf16_t* x, const bf16_t* res,
                           const bf16_t* nw, const bf16_t* w, int M, int N, int K, int ldx, int ldr,
                           int ldh, int ldy, float eps, hipStream_t st) {
-  const dim3 grid(N / 4), block(256);
+  const dim3 grid(ACT < 0 ? N / 4 : N / 2), block(256);
   switch (K / 2048) {
-    case 1: skinny_norm_gemm_kernel<MT, 1, GEMMA, 4><<<grid, block, 0, st>>>(y, h, x, res, nw, w, M, K, ldx, ldr, ldh, ldy, eps); break;
-    case 2: skinny_norm_gemm_kernel<MT, 2, GEMMA, 4><<<grid, block, 0, st>>>(y, h, x, res, nw, w, M, K, ldx, ldr, ldh, ldy, eps); break;
-    case 4: skinny_norm_gemm_kernel<MT, 4, GEMMA, 4><<<grid, block, 0, st>>>(y, h, x, res, nw, w, M, K, ldx, ldr, ldh, ldy, eps); break;
+    case 1: skinny_norm_gemm_kernel<MT, 1, GEMMA, 4, ACT><<<grid, block, 0, st>>>(y, h, x, res, nw, w, M, N, K, ldx, ldr, ldh, ldy, eps); break;
+    case 2: skinny_norm_gemm_kernel<MT, 2, GEMMA, 4, ACT><<<grid, block, 0, st>>>(y, h, x, res, nw, w, M, N, K, ldx, ldr, ldh, ldy, eps); break;
+    case 4: skinny_norm_gemm_kernel<MT, 4, GEMMA, 4, ACT><<<grid, block, 0, st>>>(y, h, x, res, nw, w, M, N, K, ldx, ldr, ldh, ldy, eps); break;
     default: return -1;
   }
   return 0;
 }
 
+// act: 0 silu, 1 gelu (tanh), -1 none.  N: output columns, of two rows of w each with an activation
 int launch_skinny_norm_gemm(void* y, void* h_out, const void* x, const void* res, const void* nw,
                             const void* w, int M, int N, int K, int ldx, int ldr, int ldh,
-                            int ldy, float eps, bool gemma, hipStream_t st) {
-  if (M < 1 || M > 4 || K % 2048 != 0 || N % 4 != 0 || ldx % 8 || (res && (ldr % 8 || ldh % 8)) ||
-      (res && !h_out))
+                            int ldy, float eps, bool gemma, int act, hipStream_t st) {
+  if (M < 1 || M > 4 || K % 2048 != 0 || N % (act < 0 ? 4 : 2) != 0 || ldx % 8 ||
+      (res && (ldr % 8 || ldh % 8)) || (res && !h_out) || act > 1 || (act >= 0 && M > 1))
     return -1;
-  bf16_t* yy = (bf16_t*)y;
-  bf16_t* hh = (bf16_t*)h_out;
-  const bf16_t* xx = (const bf16_t*)x;
-  const bf16_t* rr = (const bf16_t*)res;
-  const bf16_t* gg = (const bf16_t*)nw;
-  const bf16_t* ww = (const bf16_t*)w;
+  const auto run = [&](auto launch) {
+    return launch((bf16_t*)y, (bf16_t*)h_out, (const bf16_t*)x, (const bf16_t*)res, (const bf16_t*)nw,
+                  (const bf16_t*)w, M, N, K, ldx, ldr, ldh, ldy, eps, st);
+  };
   int rc;
-  if (M == 1)
-    rc = gemma ? launch_norm_mt<1, true>(yy, hh, xx, rr, gg, ww, M, N, K, ldx, ldr, ldh, ldy, eps, st)
-               : launch_norm_mt<1, false>(yy, hh, xx, rr, gg, ww, M, N, K, ldx, ldr, ldh, ldy, eps, st);
-  else if (M == 2)
-    rc = gemma ? launch_norm_mt<2, true>(yy, hh, xx, rr, gg, ww, M, N, K, ldx, ldr, ldh, ldy, eps, st)
-               : launch_norm_mt<2, false>(yy, hh, xx, rr, gg, ww, M, N, K, ldx, ldr, ldh, ldy, eps, st);
-  else
-    rc = gemma ? launch_norm_mt<4, true>(yy, hh, xx, rr, gg, ww, M, N, K, ldx, ldr, ldh, ldy, eps, st)
-               : launch_norm_mt<4, false>(yy, hh, xx, rr, gg, ww, M, N, K, ldx, ldr, ldh, ldy, eps, st);
+  if (act == 0) rc = run(gemma ? launch_norm_mt<1, true, 0> : launch_norm_mt<1, false, 0>);
+  else if (act == 1) rc = run(gemma ? launch_norm_mt<1, true, 1> : launch_norm_mt<1, false, 1>);
+  else if (M == 1) rc = run(gemma ? launch_norm_mt<1, true> : launch_norm_mt<1, false>);
+  else if (M == 2) rc = run(gemma ? launch_norm_mt<2, true> : launch_norm_mt<2, false>);
+  else rc = run(gemma ? launch_norm_mt<4, true> : launch_norm_mt<4, false>);
   return rc ? rc : (int)hipGetLastError();
 }
 

@@ -140,10 +140,11 @@ int launch_skinny_gemm(void* y, const void* x, const void* w, int M, int N, int 
 int launch_skinny_glu_gemm(void* y, const void* gu, const void* w, int M, int N, int K, int ldx,
                            int ldy, int act, hipStream_t st);
 // RMSNorm (+ residual add) fused into the skinny dot2 GEMM (gemv.hip): y = norm(x [+ res]) @ W^T,
-// h_out = x + res (written when res is given); M <= 4, K % 2048 == 0.
+// h_out = x + res (written when res is given); M <= 4, K 2048, 4096 or 8192.  act >= 0: W = [gate; up] of
+// 2N rows, y = act(gate) * up, M = 1.
 int launch_skinny_norm_gemm(void* y, void* h_out, const void* x, const void* res, const void* nw,
                             const void* w, int M, int N, int K, int ldx, int ldr, int ldh,
-                            int ldy, float eps, bool gemma, hipStream_t st);
+                            int ldy, float eps, bool gemma, int act, hipStream_t st);
 
 // 4-wave hand-scheduled GEMM (gemm_w4.hip): c[M,N] = epi(a[M,K] . b[N,K]^T); epi 0 store,
 // 1 + r (residual, may alias c), 2/3 SiLU/GELU gated (b rows [0,up_off) gate, [up_off, 2 up_off)

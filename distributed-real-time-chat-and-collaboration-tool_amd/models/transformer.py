@@ -300,6 +300,8 @@ class TransformerLM:
             if self.pc.tp_size == 1:
                 return ops.linear_parts(h, L["down"]), False
             y = ops.linear(h, L["down"])
+        elif (h := ops.norm_glu_row(x, L["gate_up"], self.cfg.act)) is not None:  # a decode step of one row
+            y = (ops.linear_parts if self.pc.tp_size == 1 else ops.linear)(h, L["down"])
         else:
             gu = ops.norm_linear(x, L["gate_up"])
             res = self._fusable_residual(gu, x)
@@ -419,7 +421,7 @@ class TransformerLM:
                             self.sh.expert_offset, workspace=self.moe_ws, residual=h, norm_w=nxt, eps=cfg.rms_eps)
         return ops.PendingNorm.done(out, h, nxt, cfg.rms_eps)
 
-    def _layers(self, h: torch.Tensor, attn_fn, decode: bool = False) -> torch.Tensor:
+    def _layers(self, h: torch.Tensor, attn_fn, decode: bool = False) -> ops.PendingNorm:
         """Pre-norm residual stack.  Each sublayer receives its input as an
         ops.PendingNorm (norm(x + residual) not yet computed), so a small
         decode batch can fuse the norm into the first projection."""
@@ -441,10 +443,11 @@ class TransformerLM:
             m, added, *part = self._mlp(L, x, decode)
             x = ops.PendingNorm(m, None if added else x.stream(), nxt, cfg.rms_eps, cfg.gemma_norm,
                                 pc=self.pc if part and part[0] else None)
-        return x.materialize()
+        return x
 
-    def _logits(self, x: torch.Tensor) -> torch.Tensor:
-        logits = ops.linear(x, self.lm_head)
+    def _logits(self, x: torch.Tensor | ops.PendingNorm) -> torch.Tensor:
+        """Logits of normalised rows, or of rows whose last norm is pending."""
+        logits = ops.norm_linear(x, self.lm_head) if isinstance(x, ops.PendingNorm) else ops.linear(x, self.lm_head)
         return self.pc.all_gather_tp_lastdim(logits)
 
     def forward_prefill(self, ids: torch.Tensor, meta: PrefillMeta, kv_caches) -> torch.Tensor:
@@ -562,7 +565,7 @@ class TransformerLM:
                 m, added = self._mlp(L, xr)
                 xf = ops.PendingNorm(m, None if added else xr.stream(), self.final_norm,
                                      cfg.rms_eps, cfg.gemma_norm)
-                return self._logits(xf.materialize())
+                return self._logits(xf)
             o_rows = pc.reduce_scatter_rows(ops.linear(a, L["o"]))
             x = ops.PendingNorm(o_rows, x.stream(), L["ln_post"], cfg.rms_eps, cfg.gemma_norm)
             if cfg.is_moe and moe_a2a:

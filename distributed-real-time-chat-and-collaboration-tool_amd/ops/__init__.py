@@ -19,7 +19,7 @@ from .delta import DeltaWeights, Portions, delta_decode, delta_scan, short_conv
 from .gated_average import (SCAN_CHUNK, AverageWeights, ScanChunks, chunk_scan, gated_decode,
                             gated_scan)
 from .gemm import (Parts, fused_glu_ok, gated, glu_linear, linear, linear_parts, linear_residual, mfma_gemm, norm_glu,
-                   norm_linear, residual_fusable, squared_relu, w4_glu_ok)
+                   norm_glu_row, norm_linear, residual_fusable, squared_relu, w4_glu_ok)
 from .grouped import (GroupedDecodeWorkspace, GroupedPortions, GroupedWeights, attn_prep,
                       grouped_decode, grouped_prefill, grouped_qtile, prep_tile_rows)
 from .latent import (LatentDecodeWorkspace, PortionKeys, build_interleaved_rope, head_linear,

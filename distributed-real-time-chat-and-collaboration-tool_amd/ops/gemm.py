@@ -436,6 +436,32 @@ _fuse_norm = os.environ.get("DRTC_FUSED_NORM_GEMM", "1") != "0"
 NORM_FUSE_MAX_M = 1
 
 
+def _norm_fused(p, w: torch.Tensor, act: int = -1):
+    """norm(p) @ w.T, gated with ``act`` >= 0, in one launch (``skinny_norm_gemm_kernel``), or None where the
+    projection would not run on the skinny dot2 kernel."""
+    x, res = p.x, p.residual
+    if not (_fuse_norm and p._out is None and p.pc is None and isinstance(x, torch.Tensor)
+            and _gpu_bf16(x, w) and p.w.is_contiguous()
+            and (res is None or (res.stride(1) == 1 and res.shape == x.shape))):
+        return None
+    M, K = x.shape
+    N = w.shape[0]
+    if not (M <= (NORM_FUSE_MAX_M if act < 0 else 1) and K in (2048, 4096, 8192) and N % 4 == 0
+            and x.stride(0) % 8 == 0 and (res is None or res.stride(0) % 8 == 0)
+            and _choice(M, N, K, K) == 1):
+        return None
+    if act >= 0:
+        N //= 2
+    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    h = torch.empty((M, K), dtype=x.dtype, device=x.device) if res is not None else None
+    check(hipk().skinny_norm_gemm(
+        y.data_ptr(), ptr(h), x.data_ptr(), ptr(res), p.w.data_ptr(), w.data_ptr(), M, N,
+        K, x.stride(0), res.stride(0) if res is not None else 0, K, N, float(p.eps),
+        bool(p.gemma), act, stream_ptr(x)), "skinny_norm_gemm")
+    p.applied(h if h is not None else x)
+    return y
+
+
 def norm_linear(p, w: torch.Tensor) -> torch.Tensor:
     """y = rmsnorm(p.x [+ p.residual]) @ w.T for an ``ops.PendingNorm`` p.
 
@@ -443,24 +469,15 @@ def norm_linear(p, w: torch.Tensor) -> torch.Tensor:
     measured per shape) the norm is fused into it (gemv.hip ``skinny_norm_gemm_kernel``):
     one launch instead of two, and the new residual stream is written by the GEMM.
     Otherwise the norm is materialised and ``linear`` runs."""
-    x, res = p.x, p.residual
-    if (_fuse_norm and p._out is None and p.pc is None and isinstance(x, torch.Tensor)
-            and _gpu_bf16(x, w) and p.w.is_contiguous()
-            and (res is None or (res.stride(1) == 1 and res.shape == x.shape))):
-        M, K = x.shape
-        N = w.shape[0]
-        if (M <= NORM_FUSE_MAX_M and K % 2048 == 0 and K <= 8192 and N % 4 == 0
-                and x.stride(0) % 8 == 0 and (res is None or res.stride(0) % 8 == 0)
-                and _choice(M, N, K, K) == 1):
-            y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-            h = torch.empty((M, K), dtype=x.dtype, device=x.device) if res is not None else None
-            check(hipk().skinny_norm_gemm(
-                y.data_ptr(), ptr(h), x.data_ptr(), ptr(res), p.w.data_ptr(), w.data_ptr(), M, N,
-                K, x.stride(0), res.stride(0) if res is not None else 0, K, N, float(p.eps),
-                bool(p.gemma), stream_ptr(x)), "skinny_norm_gemm")
-            p.applied(h if h is not None else x)
-            return y
-    return linear(p.materialize(), w)
+    y = _norm_fused(p, w)
+    return linear(p.materialize(), w) if y is None else y
+
+
+def norm_glu_row(p, w: torch.Tensor, act: str = "silu"):
+    """act(norm(p) @ gate.T) * (norm(p) @ up.T) of one row in one launch, the fused [gate; up] weight on the skinny
+    dot2 kernel; None where another kernel takes the product (``norm_glu``)."""
+    code = {"silu": 0, "gelu_tanh": 1}.get(act)
+    return None if code is None or not _fuse_glu else _norm_fused(p, w, code)
 
 
 _fuse_glu = os.environ.get("DRTC_FUSED_GLU_GEMM", "1") != "0"
@@ -1273,7 +1290,7 @@ def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | Parts:
     return linear(x, w)
 
 
-__all__ = ["linear", "linear_parts", "parts_form", "Parts", "route", "norm_linear", "glu_linear", "norm_glu", "fused_glu_ok",
+__all__ = ["linear", "linear_parts", "parts_form", "Parts", "route", "norm_linear", "glu_linear", "norm_glu_row", "norm_glu", "fused_glu_ok",
            "linear_residual",
            "residual_fusable", "w4_glu_ok", "w4_ok", "w4_shape_ok", "squared_relu", "w4_group_m", "mfma_gemm",
            "mfma_gemm_grouped",

@@ -1038,6 +1038,42 @@ def test_skinny_glu_gemm(hipk, M, I, act):
         gemm._routes.clear()
 
 
+@pytest.mark.parametrize("K", [2048, 4096, 8192])
+@pytest.mark.parametrize("act,resid,gemma", [("silu", True, False), ("gelu_tanh", False, False), ("silu", True, True)])
+def test_skinny_norm_glu_gemm(hipk, K, act, resid, gemma):
+    """One row's norm, gated projection and activation in one launch: the stream exactly, the row to its bf16
+    rounding and that of the normed input (2^-9 of each of K products, root-sum-square)."""
+    from drtc_amd.ops import gemm
+
+    torch.manual_seed(K)
+    I = 1030
+    x = torch.randn(1, K, device=DEV).to(torch.bfloat16)
+    res = torch.randn(1, K, device=DEV).to(torch.bfloat16) if resid else None
+    nw = (torch.randn(K, device=DEV) * 0.1 + (0.0 if gemma else 1.0)).to(torch.bfloat16)
+    w = (torch.randn(2 * I, K, device=DEV) / K ** 0.5).to(torch.bfloat16)
+    h = (x.float() + res.float()).to(torch.bfloat16) if resid else x
+    gu = ops.rmsnorm_ref(h, nw, 1e-5, gemma).float() @ w.float().t()
+    g, u = gu[:, :I].double(), gu[:, I:].double()
+    want = (torch.nn.functional.silu(g) if act == "silu" else torch.nn.functional.gelu(g, approximate="tanh")) * u
+    saved = gemm._table
+    try:
+        gemm._table = {(1, 2 * I, K, K): (-1, 1, 0, 0, 0)}  # measured pick: dot2 kernel
+        gemm._routes.clear()
+        p = ops.PendingNorm(x, res.clone() if resid else None, nw, 1e-5, gemma)
+        y = ops.norm_glu_row(p, w, act)
+        assert y is not None and torch.equal(p.stream(), h)
+        # an element of the normed row may round the other way (rstd): 2^-8 of it; gate and up are about 1 wide
+        assert ((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -8).all()
+        two = ops.PendingNorm(x.repeat(2, 1), None, nw, 1e-5, gemma)
+        assert ops.norm_glu_row(two, w, act) is None and ops.norm_glu_row(p, w, "relu2") is None
+        gemm._table = {(1, 2 * I, K, K): (-1, 0, 0, 0, 0)}
+        gemm._routes.clear()
+        assert ops.norm_glu_row(p, w, act) is None
+    finally:
+        gemm._table = saved
+        gemm._routes.clear()
+
+
 @pytest.mark.parametrize("e_off,e_local", [(0, 8), (2, 3)])
 def test_moe_large_eager_call_fused(hipk, e_off, e_local):
     """A prefill-sized eager MoE call (more tokens than one kernel chunk) on the fused
