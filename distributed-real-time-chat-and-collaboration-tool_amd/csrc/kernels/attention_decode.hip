@@ -637,7 +637,7 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_wave_kerne
 //     from registers instead: k rotated the same way, q.k reduced over the 4 lane groups,
 //     m = that score, p = 1, o = its v row;
 //   * that item also writes the rotated k row and the v row into the paged cache (slot from
-//     `slots`) for the next steps - the same bytes rope_kv_kernel_v2 writes.
+//     `slots`) for the next steps - the same bytes rope_kv_kernel writes.
 // One LDS-DMA wave-instruction of one dword per lane: 256 contiguous bytes land at the LDS byte
 // address `dst` (M0 saved and restored).  Counts in vmcnt like any vector load.
 DRTC_DEVICE void dma_dword_lds(unsigned dst, unsigned voff, __amdgpu_buffer_rsrc_t rsrc) {

@@ -47,25 +47,17 @@ PYBIND11_MODULE(_hipk, m) {
                       float limit, u64 st) {
     return drtc::launch_act_glu(P<void>(out), P<void>(gu), T, I, gu_stride, act, limit, S(st));
   });
-  m.def("rope_kv", [](u64 qkv, int T, int qkv_stride, u64 positions, u64 slots,
-                      u64 cos_sin, int Hq, int Hkv, int D, u64 k_cache,
-                      u64 v_cache, int block_size, int write_v, u64 st) {
-    return drtc::launch_rope_kv(P<void>(qkv), T, qkv_stride, P<const int>(positions),
-                                P<const int64_t>(slots), P<const float>(cos_sin), Hq,
-                                Hkv, D, P<void>(k_cache), P<void>(v_cache),
-                                block_size, write_v, S(st));
+  m.def("rope_kv", [](u64 qkv, int T, int qkv_stride, u64 positions, u64 slots, u64 cos_sin, int Hq, int Hkv, int D,
+                      u64 k_cache, u64 v_cache, int block_size, int write_v, u64 seg_tok, u64 seg_len, u64 seg_blk,
+                      int nseg, u64 pad, int pad_rows, int pad_cols, int64_t pad_stride, u64 st) {
+    return drtc::launch_rope_kv({P<void>(qkv), T, qkv_stride, P<const int>(positions), P<const int64_t>(slots),
+                                 P<const float>(cos_sin), Hq, Hkv, D, P<void>(k_cache), P<void>(v_cache), block_size,
+                                 write_v, P<const int>(seg_tok), P<const int>(seg_len), P<const int>(seg_blk), nseg,
+                                 P<void>(pad), pad_rows, pad_cols, pad_stride}, S(st));
   });
-  m.def("set_rope_variant", [](int v) { drtc::set_rope_variant(v); });
   m.def("w4_set_krot", [](int k) { drtc::w4_set_krot(k); });
   m.def("w4_krot", []() { return drtc::w4_krot(); });
   m.def("w4_set_grouped_rot", [](int r) { drtc::w4_set_grouped_rot(r); });
-  m.def("kv_write_v", [](u64 v_cache, u64 qkv, int qkv_stride, u64 seg_tok, u64 seg_len,
-                         u64 seg_blk, int nseg, int Hq, int Hkv, int D, int block_size,
-                         u64 st) {
-    return drtc::launch_kv_write_v(P<void>(v_cache), P<const void>(qkv), qkv_stride,
-                                   P<const int>(seg_tok), P<const int>(seg_len),
-                                   P<const int>(seg_blk), nseg, Hq, Hkv, D, block_size, S(st));
-  });
   m.def("paged_decode",
         [](u64 out, u64 part_o, u64 part_ml, u64 counters, u64 q, int q_stride, u64 k_cache,
            u64 v_cache, u64 block_tables, int bt_stride, u64 context_lens, int B,

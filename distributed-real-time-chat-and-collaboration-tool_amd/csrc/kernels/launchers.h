@@ -23,15 +23,25 @@ int launch_rmsnorm_parts(void* out, void* residual, const float* parts, int S, c
 int launch_act_glu(void* out, const void* gu, int64_t T, int I, int gu_stride,
                    int act, float limit, hipStream_t st);
 
-void set_rope_variant(int v);
-int launch_rope_kv(void* qkv, int T, int qkv_stride, const int* positions,
-                   const int64_t* slots, const float* cos_sin, int Hq, int Hkv,
-                   int D, void* k_cache, void* v_cache, int block_size, int write_v,
-                   hipStream_t st);
-
-int launch_kv_write_v(void* v_cache, const void* qkv, int qkv_stride, const int* seg_tok,
-                      const int* seg_len, const int* seg_blk, int nseg, int Hq, int Hkv,
-                      int D, int block_size, hipStream_t st);
+struct RopeArgs {
+  void* qkv;               // [T][qkv_stride], q and k rotated in place
+  int T, qkv_stride;
+  const int* positions;
+  const int64_t* slots;    // [T] cache slots of the tokens (-1: none), or null
+  const float* cos_sin;
+  int Hq, Hkv, D;
+  void* k_cache;
+  void* v_cache;
+  int block_size, write_v;
+  const int* seg_tok;      // nseg cache blocks of prompts to write V of: first token, tokens, block
+  const int* seg_len;
+  const int* seg_blk;
+  int nseg;
+  void* pad;               // pad_rows rows of pad_cols to clear, or null
+  int pad_rows, pad_cols;
+  int64_t pad_stride;
+};
+int launch_rope_kv(const RopeArgs& a, hipStream_t st);
 
 int launch_paged_decode_rope(void* out, float* part_o, float* part_ml, const void* q,
                              int q_stride, void* k_cache, void* v_cache,

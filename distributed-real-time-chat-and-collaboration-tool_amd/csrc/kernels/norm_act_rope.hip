@@ -248,91 +248,48 @@ int launch_act_glu(void* out, const void* gu, int64_t T, int I, int gu_stride,
 // ------------------------------------------------------ RoPE + KV write
 // qkv: [T][qkv_stride] with heads laid out q(Hq) | k(Hkv) | v(Hkv), each D.
 // cos_sin: [max_pos][D] fp32, first D/2 = cos, last D/2 = sin (NeoX halves).
+//
+// Blocks [0, nseg Hkv): V of a prompt's cache blocks (write_v_block).  Then one a token: a single pass over rope
+// items + V items where those are written by the token (threads = their count rounded up to whole waves, looping
+// only past 1024), cos/sin read as 16-B vectors, and the V scatter mapped one cache dim per lane: a wave's
+// stores then hit 64 consecutive 8-B slots of the dim-major V group (4 cache lines) instead of 8 dims per lane
+// (every store instruction spread over 32 lines).  Then one for each row of `pad` to clear.  All three in a
+// launch, since each of them is mostly launch where a prompt is short (160 rows, 32 + 8 heads of 128: 4.8 + 3.9
+// + 1.8 us in three, now 4.8).
 template <int D>
-__global__ __launch_bounds__(256) void rope_kv_kernel(
-    bf16_t* __restrict__ qkv, int qkv_stride, const int* __restrict__ positions,
-    const int64_t* __restrict__ slots, const float* __restrict__ cos_sin,
-    int Hq, int Hkv, bf16_t* __restrict__ k_cache,
-    bf16_t* __restrict__ v_cache, int block_size, int write_v) {
-  constexpr int HV = D / 16;  // 8-wide vectors per half-head
-  const int t = blockIdx.x;
-  const int pos = positions[t];
-  const int64_t slot = slots ? slots[t] : -1;
-  bf16_t* row = qkv + (int64_t)t * qkv_stride;
-  const float* cs = cos_sin + (int64_t)pos * D;
-  int64_t blk = 0, off = 0;
-  if (slot >= 0) {
-    blk = slot / block_size;
-    off = slot - blk * block_size;
-  }
-  const int n_rope = (Hq + Hkv) * HV;
-  for (int item = threadIdx.x; item < n_rope; item += 256) {
-    const int head = item / HV;
-    const int vi = item - head * HV;
-    bf16_t* base = row + head * D + vi * 8;
-    bf16x8 x1 = load_bf16x8(base);
-    bf16x8 x2 = load_bf16x8(base + D / 2);
-    bf16x8 o1, o2;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float c = cs[vi * 8 + j];
-      const float s = cs[D / 2 + vi * 8 + j];
-      const float a = bf2f(x1[j]), b = bf2f(x2[j]);
-      o1[j] = f2bf(a * c - b * s);
-      o2[j] = f2bf(b * c + a * s);
-    }
-    store_bf16x8(base, o1);
-    store_bf16x8(base + D / 2, o2);
-    if (head >= Hq && slot >= 0) {
-      const int h = head - Hq;
-      bf16_t* kd = k_cache + ((blk * Hkv + h) * block_size + off) * D + vi * 8;
-      store_bf16x8(kd, o1);
-      store_bf16x8(kd + D / 2, o2);
-    }
-  }
-  if (slot < 0 || !write_v) return;
-  const int n_v = Hkv * (D / 8);
-  for (int item = threadIdx.x; item < n_v; item += 256) {
-    const int h = item / (D / 8);
-    const int c = (item - h * (D / 8)) * 8;
-    bf16x8 v = load_bf16x8(row + (Hq + Hkv + h) * D + c);
-    // V block layout: [block_size/4 groups][D][4 tokens] (see kv_write_v)
-    bf16_t* vd = v_cache + (blk * Hkv + h) * D * block_size + (off >> 2) * (4 * D) + c * 4 +
-                 (off & 3);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) vd[4 * j] = v[j];
-  }
-}
+DRTC_DEVICE void write_v_block(const RopeArgs& a, int seg, int h, bf16_t* tile);
 
-// v2: a single pass over rope items + V items (block = their count rounded
-// up to whole waves, looping only past 1024), cos/sin read as 16-B vectors,
-// and the V scatter mapped one cache dim per lane: a wave's stores then hit
-// 64 consecutive 8-B slots of the dim-major V group (4 cache lines) instead of
-// 8 dims per lane (every store instruction spread over 32 lines).  Same math
-// and cache contents as rope_kv_kernel.
 template <int D>
-__global__ __launch_bounds__(1024) void rope_kv_kernel_v2(
-    bf16_t* __restrict__ qkv, int qkv_stride, const int* __restrict__ positions,
-    const int64_t* __restrict__ slots, const float* __restrict__ cos_sin,
-    int Hq, int Hkv, bf16_t* __restrict__ k_cache,
-    bf16_t* __restrict__ v_cache, int block_size, int write_v) {
+__global__ __launch_bounds__(1024) void rope_kv_kernel(RopeArgs a) {
   constexpr int HV = D / 16;
-  const int t = blockIdx.x;
+  __shared__ bf16_t tile[32 * (D + 2)];
+  int t = blockIdx.x;
+  const int Hq = a.Hq, Hkv = a.Hkv, nv = a.nseg * Hkv;
+  if (t < nv) {
+    write_v_block<D>(a, t / Hkv, t % Hkv, tile);
+    return;
+  }
+  t -= nv;
+  if (t >= a.T) {
+    bf16_t* row = (bf16_t*)a.pad + (int64_t)(t - a.T) * a.pad_stride;
+    for (int i = threadIdx.x; i < a.pad_cols; i += blockDim.x) row[i] = f2bf(0.f);
+    return;
+  }
   const int n_rope = (Hq + Hkv) * HV;
-  const int pos = positions[t];
-  const int64_t slot = slots ? slots[t] : -1;
-  const int n_items = n_rope + ((slot >= 0 && write_v) ? Hkv * (D / 2) : 0);
-  bf16_t* row = qkv + (int64_t)t * qkv_stride;
+  const int pos = a.positions[t];
+  const int64_t slot = a.slots ? a.slots[t] : -1;
+  const int n_items = n_rope + ((slot >= 0 && a.write_v) ? Hkv * (D / 2) : 0);
+  bf16_t* row = (bf16_t*)a.qkv + (int64_t)t * a.qkv_stride;
   int64_t blk = 0, off = 0;
   if (slot >= 0) {
-    blk = slot / block_size;
-    off = slot - blk * block_size;
+    blk = slot / a.block_size;
+    off = slot - blk * a.block_size;
   }
   for (int item = threadIdx.x; item < n_items; item += blockDim.x) {
     if (item < n_rope) {
       const int head = item / HV;
       const int vi = item - head * HV;
-      const float* cs = cos_sin + (int64_t)pos * D + vi * 8;
+      const float* cs = a.cos_sin + (int64_t)pos * D + vi * 8;
       const f32x4 ca = *reinterpret_cast<const f32x4*>(cs);
       const f32x4 cb = *reinterpret_cast<const f32x4*>(cs + 4);
       const f32x4 sa = *reinterpret_cast<const f32x4*>(cs + D / 2);
@@ -345,24 +302,24 @@ __global__ __launch_bounds__(1024) void rope_kv_kernel_v2(
       for (int j = 0; j < 8; ++j) {
         const float c = j < 4 ? ca[j] : cb[j - 4];
         const float sn = j < 4 ? sa[j] : sb[j - 4];
-        const float a = bf2f(x1[j]), b = bf2f(x2[j]);
-        o1[j] = f2bf(a * c - b * sn);
-        o2[j] = f2bf(b * c + a * sn);
+        const float p = bf2f(x1[j]), q = bf2f(x2[j]);
+        o1[j] = f2bf(p * c - q * sn);
+        o2[j] = f2bf(q * c + p * sn);
       }
       store_bf16x8(base, o1);
       store_bf16x8(base + D / 2, o2);
       if (head >= Hq && slot >= 0) {
-        bf16_t* kd = k_cache + ((blk * Hkv + (head - Hq)) * block_size + off) * D + vi * 8;
+        bf16_t* kd = (bf16_t*)a.k_cache + ((blk * Hkv + (head - Hq)) * a.block_size + off) * D + vi * 8;
         store_bf16x8(kd, o1);
         store_bf16x8(kd + D / 2, o2);
       }
     } else {
-      // V block layout: [block_size/4 groups][D][4 tokens] (see kv_write_v)
+      // V block layout: [block_size/4 groups][D][4 tokens] (see write_v_block)
       const int vitem = item - n_rope;
       const int h = vitem / (D / 2);
       const int d = vitem - h * (D / 2);
       const bf16_t* src = row + (Hq + Hkv + h) * D + d;
-      bf16_t* vd = v_cache + (blk * Hkv + h) * D * block_size + (off >> 2) * (4 * D) + d * 4 +
+      bf16_t* vd = (bf16_t*)a.v_cache + (blk * Hkv + h) * D * a.block_size + (off >> 2) * (4 * D) + d * 4 +
                    (off & 3);
       const bf16_t v0 = src[0], v1 = src[D / 2];
       vd[0] = v0;
@@ -371,52 +328,8 @@ __global__ __launch_bounds__(1024) void rope_kv_kernel_v2(
   }
 }
 
-static int g_rope_variant = 2;
-void set_rope_variant(int v) { g_rope_variant = v; }
-
-int launch_rope_kv(void* qkv, int T, int qkv_stride, const int* positions,
-                   const int64_t* slots, const float* cos_sin, int Hq, int Hkv,
-                   int D, void* k_cache, void* v_cache, int block_size, int write_v,
-                   hipStream_t st) {
-  if (T == 0) return 0;
-  const int items = (Hq + Hkv) * (D / 16) + (slots && write_v ? Hkv * (D / 2) : 0);
-  if (g_rope_variant == 2) {
-    dim3 grid(T), block(std::min(1024, (items + 63) / 64 * 64));
-    switch (D) {
-      case 64:
-        hipLaunchKernelGGL(rope_kv_kernel_v2<64>, grid, block, 0, st, (bf16_t*)qkv, qkv_stride, positions, slots, cos_sin, Hq, Hkv, (bf16_t*)k_cache, (bf16_t*)v_cache, block_size, write_v);
-        break;
-      case 128:
-        hipLaunchKernelGGL(rope_kv_kernel_v2<128>, grid, block, 0, st, (bf16_t*)qkv, qkv_stride, positions, slots, cos_sin, Hq, Hkv, (bf16_t*)k_cache, (bf16_t*)v_cache, block_size, write_v);
-        break;
-      case 256:
-        hipLaunchKernelGGL(rope_kv_kernel_v2<256>, grid, block, 0, st, (bf16_t*)qkv, qkv_stride, positions, slots, cos_sin, Hq, Hkv, (bf16_t*)k_cache, (bf16_t*)v_cache, block_size, write_v);
-        break;
-      default:
-        return -1;
-    }
-    return (int)hipGetLastError();
-  }
-  dim3 grid(T), block(256);
-  switch (D) {
-    case 64:
-      hipLaunchKernelGGL(rope_kv_kernel<64>, grid, block, 0, st, (bf16_t*)qkv, qkv_stride, positions, slots, cos_sin, Hq, Hkv, (bf16_t*)k_cache, (bf16_t*)v_cache, block_size, write_v);
-      break;
-    case 128:
-      hipLaunchKernelGGL(rope_kv_kernel<128>, grid, block, 0, st, (bf16_t*)qkv, qkv_stride, positions, slots, cos_sin, Hq, Hkv, (bf16_t*)k_cache, (bf16_t*)v_cache, block_size, write_v);
-      break;
-    case 256:
-      hipLaunchKernelGGL(rope_kv_kernel<256>, grid, block, 0, st, (bf16_t*)qkv, qkv_stride, positions, slots, cos_sin, Hq, Hkv, (bf16_t*)k_cache, (bf16_t*)v_cache, block_size, write_v);
-      break;
-    default:
-      return -1;
-  }
-  return (int)hipGetLastError();
-}
-
-// ------------------------------------------- prefill V write (transposed)
-// V cache block layout (per kv head): 8 groups of 4 tokens, each group
-// dim-major [D][4] - the decode kernel's P.V operand wants 4 consecutive
+// V of a prompt's cache block, transposed.  V cache block layout (per kv head): 8 groups of 4 tokens, each
+// group dim-major [D][4] - the decode kernel's P.V operand wants 4 consecutive
 // tokens of one dim in 8 contiguous bytes, and a decode-time write of ONE
 // token then touches D 8-byte slots inside a 2*D-byte span (a plain [D][32]
 // dim-major block scatters it over D separate 64-B rows: ~8x the HBM write
@@ -425,28 +338,23 @@ int launch_rope_kv(void* qkv, int T, int qkv_stride, const int* positions,
 // [32][D] tile in LDS and writes the block with 16-byte stores (two dims x
 // 4 tokens each).
 template <int D>
-__global__ __launch_bounds__(256) void kv_write_v_kernel(
-    bf16_t* __restrict__ v_cache, const bf16_t* __restrict__ qkv, int qkv_stride,
-    const int* __restrict__ seg_tok, const int* __restrict__ seg_len,
-    const int* __restrict__ seg_blk, int Hq, int Hkv) {
+DRTC_DEVICE void write_v_block(const RopeArgs& a, int seg, int h, bf16_t* tile) {
   constexpr int BS = 32;
   constexpr int ROW = D + 2;  // padded LDS row (elements)
-  __shared__ bf16_t tile[BS * ROW];
-  const int seg = blockIdx.x, h = blockIdx.y;
-  const int t0 = seg_tok[seg], n = seg_len[seg];
-  const int64_t blk = seg_blk[seg];
-  const int voff = (Hq + Hkv + h) * D;
-  for (int v = threadIdx.x; v < BS * (D / 8); v += 256) {
+  const int t0 = a.seg_tok[seg], n = a.seg_len[seg];
+  const int64_t blk = a.seg_blk[seg];
+  const int voff = (a.Hq + a.Hkv + h) * D;
+  for (int v = threadIdx.x; v < BS * (D / 8); v += blockDim.x) {
     const int t = v / (D / 8), c = (v - t * (D / 8)) * 8;
     bf16x8 x;
-    if (t < n) x = load_bf16x8(qkv + (int64_t)(t0 + t) * qkv_stride + voff + c);
+    if (t < n) x = load_bf16x8((const bf16_t*)a.qkv + (int64_t)(t0 + t) * a.qkv_stride + voff + c);
     else for (int j = 0; j < 8; ++j) x[j] = f2bf(0.f);
 #pragma unroll
     for (int j = 0; j < 8; ++j) tile[t * ROW + c + j] = x[j];
   }
   __syncthreads();
-  bf16_t* dst = v_cache + (blk * Hkv + h) * (int64_t)D * BS;
-  for (int v = threadIdx.x; v < (BS / 4) * (D / 2); v += 256) {
+  bf16_t* dst = (bf16_t*)a.v_cache + (blk * a.Hkv + h) * (int64_t)D * BS;
+  for (int v = threadIdx.x; v < (BS / 4) * (D / 2); v += blockDim.x) {
     const int q4 = v / (D / 2), d = (v - q4 * (D / 2)) * 2;
     bf16x8 y;
 #pragma unroll
@@ -455,24 +363,17 @@ __global__ __launch_bounds__(256) void kv_write_v_kernel(
   }
 }
 
-int launch_kv_write_v(void* v_cache, const void* qkv, int qkv_stride, const int* seg_tok,
-                      const int* seg_len, const int* seg_blk, int nseg, int Hq, int Hkv,
-                      int D, int block_size, hipStream_t st) {
-  if (nseg == 0) return 0;
-  if (block_size != 32) return -1;
-  dim3 grid(nseg, Hkv), block(256);
-  switch (D) {
-    case 64:
-      hipLaunchKernelGGL(kv_write_v_kernel<64>, grid, block, 0, st, (bf16_t*)v_cache, (const bf16_t*)qkv, qkv_stride, seg_tok, seg_len, seg_blk, Hq, Hkv);
-      break;
-    case 128:
-      hipLaunchKernelGGL(kv_write_v_kernel<128>, grid, block, 0, st, (bf16_t*)v_cache, (const bf16_t*)qkv, qkv_stride, seg_tok, seg_len, seg_blk, Hq, Hkv);
-      break;
-    case 256:
-      hipLaunchKernelGGL(kv_write_v_kernel<256>, grid, block, 0, st, (bf16_t*)v_cache, (const bf16_t*)qkv, qkv_stride, seg_tok, seg_len, seg_blk, Hq, Hkv);
-      break;
-    default:
-      return -1;
+int launch_rope_kv(const RopeArgs& a, hipStream_t st) {
+  if (a.nseg && a.block_size != 32) return -1;
+  const int pad = a.pad ? a.pad_rows : 0, grid = a.nseg * a.Hkv + a.T + pad;
+  if (grid == 0) return 0;
+  const int items = a.T == 0 ? 256 : (a.Hq + a.Hkv) * (a.D / 16) + (a.slots && a.write_v ? a.Hkv * (a.D / 2) : 0);
+  const int threads = std::max(a.nseg ? 256 : 64, std::min(1024, (items + 63) / 64 * 64));
+  switch (a.D) {
+    case 64: rope_kv_kernel<64><<<grid, threads, 0, st>>>(a); break;
+    case 128: rope_kv_kernel<128><<<grid, threads, 0, st>>>(a); break;
+    case 256: rope_kv_kernel<256><<<grid, threads, 0, st>>>(a); break;
+    default: return -1;
   }
   return (int)hipGetLastError();
 }

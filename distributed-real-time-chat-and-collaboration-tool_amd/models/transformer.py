@@ -462,19 +462,7 @@ class TransformerLM:
 
         def attn(i, L, x):
             qkv = ops.norm_linear(x, L["qkv"])
-            kc, vc = kv_caches[i] if kv_caches is not None else (None, None)
-            blockwise_v = kc is not None and meta.v_segs is not None
-            ops.rope_kv_(qkv, meta.positions, meta.slots if kc is not None else None,
-                         self.cos_sin, sh.hq, sh.hkv, D, kc, vc, ops.KV_BLOCK,
-                         write_v=not blockwise_v)
-            if blockwise_v:
-                ops.kv_write_v(vc, qkv, meta.v_segs, sh.hq, sh.hkv, D)
-            if meta.decode is None:
-                a = ops.prefill_attention(qkv, meta.cu_seqlens, sh.hq, sh.hkv, D,
-                                          cfg.attn_scale, True, tiles=meta.tiles,
-                                          cu_host=meta.cu_host, max_len=meta.max_len)
-            else:
-                a = self._attn_mixed(qkv, meta, kc, vc)
+            a = self._attend_prefill(i, qkv, meta, kv_caches)
             if i == last:
                 # Every position's K/V is cached and attended to by now; only
                 # each sequence's last token feeds the logits, so the last
@@ -491,21 +479,23 @@ class TransformerLM:
         x = self._layers(self._embed(ids), attn)
         return self._ep_end(self._logits(x))
 
-    def _attn_mixed(self, qkv: torch.Tensor, meta: PrefillMeta, kc, vc) -> torch.Tensor:
+    def _attn_mixed(self, qkv: torch.Tensor, meta: PrefillMeta, kc, vc, a: torch.Tensor | None = None) -> torch.Tensor:
         """Attention of a mixed step: causal varlen attention over the prefill
         rows, paged-cache attention for the decode rows (their K/V were just
-        written by rope_kv_), both into one [T, hq * D] buffer."""
+        written by rope_kv_), both into one [T, hq * D] buffer, ``a`` where its padding rows are cleared."""
         cfg, sh = self.cfg, self.sh
         D, Tp, dm = cfg.head_dim, meta.n_prefill, meta.decode
         T = qkv.shape[0]
         Bd = T - Tp
-        a = qkv.new_empty((T, sh.hq * D))
+        clear = a is None
+        if clear:
+            a = qkv.new_empty((T, sh.hq * D))
         ap = ops.prefill_attention(qkv[:Tp], meta.cu_seqlens, sh.hq, sh.hkv, D, cfg.attn_scale,
                                    True, tiles=meta.tiles, cu_host=meta.cu_host,
                                    max_len=meta.max_len, out=a[:Tp])
         if ap.data_ptr() != a.data_ptr():  # CPU reference returns a new tensor
             a[:Tp].copy_(ap)
-        if meta.cu_host[-1] < Tp:
+        if clear and meta.cu_host[-1] < Tp:
             a[meta.cu_host[-1]:Tp].zero_()  # shape-padding rows: never written by the kernel
         q = qkv[Tp:].as_strided((Bd, sh.hq, D), (qkv.stride(0), D, 1))
         ops.paged_decode_attention(q, kc, vc, dm.block_tables, dm.context_lens, cfg.attn_scale,
@@ -516,18 +506,28 @@ class TransformerLM:
     def _attn_prefill(self, i: int, L: dict, xn: torch.Tensor, meta: PrefillMeta, kv_caches):
         """QKV + RoPE/KV write + causal attention of a packed prefill chunk on
         this rank's heads; returns the attention output [T, hq * D]."""
+        return self._attend_prefill(i, ops.linear(xn, L["qkv"]), meta, kv_caches)
+
+    def _attend_prefill(self, i: int, qkv: torch.Tensor, meta: PrefillMeta, kv_caches) -> torch.Tensor:
+        """RoPE, KV write and attention of a packed prefill pass; a mixed step's decode rows too."""
         cfg, sh = self.cfg, self.sh
-        D = cfg.head_dim
-        qkv = ops.linear(xn, L["qkv"])
+        D, T = cfg.head_dim, qkv.shape[0]
         kc, vc = kv_caches[i] if kv_caches is not None else (None, None)
         blockwise_v = kc is not None and meta.v_segs is not None
+        out = pad = None
+        if ops.on_gpu(qkv):
+            out = qkv.new_empty((T, sh.hq * D))
+            rows = T if meta.decode is None else meta.n_prefill
+            if meta.cu_host[-1] < rows:
+                pad = out[meta.cu_host[-1]:rows]  # shape-padding rows: not written by the attention
         ops.rope_kv_(qkv, meta.positions, meta.slots if kc is not None else None,
-                     self.cos_sin, sh.hq, sh.hkv, D, kc, vc, ops.KV_BLOCK, write_v=not blockwise_v)
-        if blockwise_v:
-            ops.kv_write_v(vc, qkv, meta.v_segs, sh.hq, sh.hkv, D)
+                     self.cos_sin, sh.hq, sh.hkv, D, kc, vc, ops.KV_BLOCK, write_v=not blockwise_v,
+                     v_segs=meta.v_segs if blockwise_v else None, pad=pad)
+        if meta.decode is not None:
+            return self._attn_mixed(qkv, meta, kc, vc, out)
         return ops.prefill_attention(qkv, meta.cu_seqlens, sh.hq, sh.hkv, D, cfg.attn_scale,
                                      True, tiles=meta.tiles, cu_host=meta.cu_host,
-                                     max_len=meta.max_len)
+                                     max_len=meta.max_len, out=out)
 
     def _forward_prefill_sp(self, ids: torch.Tensor, meta: PrefillMeta, kv_caches) -> torch.Tensor:
         """Sequence-parallel TP prefill (tp | T).  Rank r holds rows

@@ -92,32 +92,42 @@ def kv_write_v_ref(v_cache, qkv, seg_tok, seg_len, seg_blk, Hq, Hkv, D):
         v_cache[b] = v_block_storage(blk)
 
 
+def _segments(segs) -> tuple:
+    seg_tok, seg_len, seg_blk = segs
+    for t in segs:
+        assert t.dtype == torch.int32 and t.is_cuda and t.numel() == seg_tok.numel()
+    return seg_tok.data_ptr(), seg_len.data_ptr(), seg_blk.data_ptr(), seg_tok.numel()
+
+
 def kv_write_v(v_cache: torch.Tensor, qkv: torch.Tensor, segs, Hq: int, Hkv: int, D: int) -> None:
     """Prefill V write: ``segs`` = (tok_start, n_tokens, block) int32 tensors,
     one entry per 32-token cache block of the packed prompt batch."""
-    seg_tok, seg_len, seg_blk = segs
     if not on_gpu(qkv):
-        kv_write_v_ref(v_cache, qkv, seg_tok, seg_len, seg_blk, Hq, Hkv, D)
+        kv_write_v_ref(v_cache, qkv, *segs, Hq, Hkv, D)
         return
     nb, hkv, d, bs = v_cache.shape
     assert hkv == Hkv and d == D and v_cache.is_contiguous() and qkv.stride(1) == 1
-    for t in segs:
-        assert t.dtype == torch.int32 and t.is_cuda and t.numel() == seg_tok.numel()
-    check(hipk().kv_write_v(v_cache.data_ptr(), qkv.data_ptr(), qkv.stride(0), seg_tok.data_ptr(),
-                            seg_len.data_ptr(), seg_blk.data_ptr(), seg_tok.numel(), Hq, Hkv, D, bs,
-                            stream_ptr(qkv)), "kv_write_v")
+    check(hipk().rope_kv(qkv.data_ptr(), 0, qkv.stride(0), 0, 0, 0, Hq, Hkv, D, 0, v_cache.data_ptr(), bs, 0,
+                         *_segments(segs), 0, 0, 0, 0, stream_ptr(qkv)), "rope_kv")
 
 
 def rope_kv_(qkv: torch.Tensor, positions: torch.Tensor, slots: torch.Tensor | None,
              cos_sin: torch.Tensor, Hq: int, Hkv: int, D: int,
              k_cache: torch.Tensor | None, v_cache: torch.Tensor | None,
-             block_size: int, write_v: bool = True) -> torch.Tensor:
+             block_size: int, write_v: bool = True, v_segs: tuple | None = None,
+             pad: torch.Tensor | None = None) -> torch.Tensor:
     """Rotate q/k heads of ``qkv`` [T, (Hq+2Hkv)*D] in place; write k (and v,
     unless ``write_v`` is False) of tokens with ``slots[t] >= 0`` into the
-    paged cache."""
+    paged cache.  In the same launch: v of whole cache blocks (``v_segs``: ``kv_write_v``) and zeros into the
+    rows of ``pad`` (bf16)."""
     if not on_gpu(qkv):
-        return rope_kv_ref(qkv, positions, slots, cos_sin, Hq, Hkv, D, k_cache,
-                           v_cache if write_v else None, block_size)
+        rope_kv_ref(qkv, positions, slots, cos_sin, Hq, Hkv, D, k_cache,
+                    v_cache if write_v else None, block_size)
+        if v_segs is not None:
+            kv_write_v_ref(v_cache, qkv, *v_segs, Hq, Hkv, D)
+        if pad is not None:
+            pad.zero_()
+        return qkv
     T = qkv.shape[0]
     assert qkv.dtype == torch.bfloat16 and qkv.stride(1) == 1
     assert qkv.shape[1] >= (Hq + 2 * Hkv) * D
@@ -127,8 +137,14 @@ def rope_kv_(qkv: torch.Tensor, positions: torch.Tensor, slots: torch.Tensor | N
         assert slots.dtype == torch.int64 and slots.numel() >= T
         assert k_cache is not None and v_cache is not None
         assert k_cache.shape[1:] == (Hkv, block_size, D) and k_cache.is_contiguous()
+    if slots is not None or v_segs is not None:
         assert v_cache.shape[1:] == (Hkv, D, block_size) and v_cache.is_contiguous()
+    rows = cols = stride = 0
+    if pad is not None:
+        assert pad.is_cuda and pad.dtype == torch.bfloat16 and pad.stride(1) == 1
+        (rows, cols), stride = pad.shape, pad.stride(0)
     check(hipk().rope_kv(qkv.data_ptr(), T, qkv.stride(0), positions.data_ptr(), ptr(slots),
                          cos_sin.data_ptr(), Hq, Hkv, D, ptr(k_cache), ptr(v_cache),
-                         block_size, int(write_v), stream_ptr(qkv)), "rope_kv")
+                         block_size, int(write_v), *(_segments(v_segs) if v_segs is not None else (0, 0, 0, 0)),
+                         ptr(pad), rows, cols, stride, stream_ptr(qkv)), "rope_kv")
     return qkv

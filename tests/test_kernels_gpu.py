@@ -1221,3 +1221,34 @@ def test_moe_with_residual_and_norm(hipk, T, H, I, E, k, variant):
     hd = h.double()
     norm = hd * torch.rsqrt((hd * hd).mean(-1, keepdim=True) + 1e-5) * w.double()
     assert ((out.double() - norm).abs() <= near * norm.abs() + 1e-4).all()
+
+
+@pytest.mark.parametrize("D,Hq,Hkv", [(64, 8, 2), (128, 32, 8), (256, 2, 1)])
+@pytest.mark.parametrize("lens,pad", [([1], 0), ([70, 32, 1, 33], 24), ([148], 12)])
+def test_rope_kv_v_and_padding_in_one_launch(hipk, D, Hq, Hkv, lens, pad):
+    """RoPE + K write, V of whole cache blocks and the cleared rows of another tensor, as by the three ops."""
+    torch.manual_seed(D + sum(lens))
+    n, bs = sum(lens), ops.KV_BLOCK
+    T = n + pad
+    tok, ln, blk, slots, pos, a, b = [], [], [], [], [], 0, 1
+    for m in lens:
+        for j in range(0, m, bs):
+            tok.append(a + j), ln.append(min(bs, m - j)), blk.append(b + j // bs)
+        slots += [b * bs + j for j in range(m)]
+        pos += list(range(m))
+        a, b = a + m, b + -(-m // bs)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    segs, pos = (i32(tok), i32(ln), i32(blk)), i32(pos + [0] * pad)
+    slots = torch.tensor(slots + [-1] * pad, device=DEV)
+    qkv = torch.randn(T, (Hq + 2 * Hkv) * D, device=DEV).to(torch.bfloat16)
+    cs = ops.build_rope_cache(256, D, 1e4, device=DEV)
+    kc, vc = (torch.randn(b + 1, Hkv, *d, device=DEV).to(torch.bfloat16) for d in ((bs, D), (D, bs)))
+    rows = torch.full((T + 3, 3 * D), float("nan"), device=DEV, dtype=torch.bfloat16)
+    q2, k2, v2 = qkv.clone(), kc.clone(), vc.clone()
+    ops.rope_kv_(qkv, pos, slots, cs, Hq, Hkv, D, kc, vc, bs, write_v=False, v_segs=segs,
+                 pad=rows[n:T, D:2 * D + 8] if pad else None)
+    ops.rope_kv_(q2, pos, slots, cs, Hq, Hkv, D, k2, v2, bs, write_v=False)
+    ops.kv_write_v(v2, q2, segs, Hq, Hkv, D)
+    assert torch.equal(qkv, q2) and torch.equal(kc, k2) and torch.equal(vc, v2)
+    z = rows[n:T, D:2 * D + 8]
+    assert (z == 0).all() and int(rows.isnan().sum()) == rows.numel() - z.numel()
