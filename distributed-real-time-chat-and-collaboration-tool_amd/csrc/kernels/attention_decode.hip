@@ -25,6 +25,7 @@
 //   Columns are query heads: G <= 16 (Llama-3 4, 70B 8, Gemma-2B 8).
 #include "common.h"
 #include "launchers.h"
+#include "lds_dma.h"
 
 typedef __attribute__((address_space(3))) void* ad_lds_ptr;
 
@@ -119,6 +120,50 @@ DRTC_DEVICE void load_kv_block_n(KVRegs<D>& r, const bf16_t* kb, const bf16_t* v
   }
 }
 
+// K of a block into a wave's LDS, whole rows to an instruction (fragments from memory are 64 bytes of each of 16
+// rows: half a cache line, whose other half is asked for again): 16-byte chunk p of row t lies at p ^ turn(t), so
+// that the 16 lanes of a fragment read as many banks.  Rows past the context are the last one's again: their
+// scores are masked.
+template <int D>
+struct KLds {
+  static constexpr int CPR = D / 8;  // chunks to a row
+  DRTC_DEVICE static int turn(int t) { return CPR >= 16 ? t & 15 : (t >> 1) & 7; }
+  DRTC_DEVICE static void load(unsigned dst, const bf16_t* kb, int lane, int nvalid) {
+    const __amdgpu_buffer_rsrc_t rsrc = dma_rsrc(kb);
+    const int last = max(min(nvalid, kBS) - 1, 0);
+#pragma unroll
+    for (int j = 0; j < kBS * CPR / 64; ++j) {
+      const int t = (64 * j + lane) / CPR, p = lane & (CPR - 1);
+      dma16<true>(dst + 1024 * j, (unsigned)(min(t, last) * CPR + (p ^ turn(t))) * 16u, rsrc, 0u);
+    }
+  }
+  DRTC_DEVICE static bf16x8 frag(const char* lds, int t, int s, int g) {
+    return *reinterpret_cast<const bf16x8*>(lds + (t * CPR + ((4 * s + g) ^ turn(t))) * 16);
+  }
+};
+template <int D>
+struct VRegs {
+  bf16x4 lo[D / 16], hi[D / 16];
+};
+DRTC_DEVICE bf16x4 load_once(const bf16_t* p) { return __builtin_nontemporal_load(reinterpret_cast<const bf16x4*>(p)); }
+template <int D>
+DRTC_DEVICE void load_v_block(VRegs<D>& r, const bf16_t* vb, int lane, int nvalid) {
+  const int t = lane & 15, g = lane >> 4;
+  if (nvalid < kBS) {  // a group past the context: zeros, which keep 0 * V finite
+    const bf16x4 zero = {};
+#pragma unroll
+    for (int i = 0; i < D / 16; ++i) r.lo[i] = r.hi[i] = zero;
+  }
+  if (nvalid >= kBS || 4 * g < nvalid) {
+#pragma unroll
+    for (int i = 0; i < D / 16; ++i) r.lo[i] = load_once(vb + g * (4 * D) + (16 * i + t) * 4);
+  }
+  if (nvalid >= kBS || 16 + 4 * g < nvalid) {
+#pragma unroll
+    for (int i = 0; i < D / 16; ++i) r.hi[i] = load_once(vb + (4 + g) * (4 * D) + (16 * i + t) * 4);
+  }
+}
+
 // The step's token for kernels that rotate and write it themselves (see the persistent kernel)
 struct DecodeRope {
   const int* positions;
@@ -153,31 +198,39 @@ DRTC_DEVICE void rope_frags(bf16x8* f, const float* __restrict__ cos_sin, int po
   }
 }
 
-// the same from cos | sin held in registers
+// One LDS-DMA wave-instruction of one dword per lane: 256 contiguous bytes land at the LDS byte
+// address `dst` (M0 saved and restored).  Counts in vmcnt like any vector load.
+DRTC_DEVICE void dma_dword_lds(unsigned dst, unsigned voff, __amdgpu_buffer_rsrc_t rsrc) {
+  unsigned keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\t"
+               "buffer_load_dword %2, %3, %4 offen lds\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep)
+               : "s"(dst), "v"(voff), "s"(rsrc), "s"(0u)
+               : "memory");
+}
+
+// rope_frags with the position's cos | sin row read from LDS (the staged row of the item)
 template <int D>
-struct RopeRegs {
-  f32x4 c[D / 64][2], s[D / 64][2];
-  DRTC_DEVICE void load(const float* __restrict__ cos_sin, int pos, int g) {
-    const float* cs = cos_sin + (int64_t)pos * D + 8 * g;
+DRTC_DEVICE void rope_frags_lds(bf16x8* f, const float* cs_row, int g) {
+  constexpr int KS = D / 32;
+  const float* cs = cs_row + 8 * g;
 #pragma unroll
-    for (int i = 0; i < D / 64; ++i)
+  for (int s = 0; s < KS / 2; ++s) {
+    const f32x4 ca = *reinterpret_cast<const f32x4*>(cs + 32 * s);
+    const f32x4 cb = *reinterpret_cast<const f32x4*>(cs + 32 * s + 4);
+    const f32x4 sa = *reinterpret_cast<const f32x4*>(cs + D / 2 + 32 * s);
+    const f32x4 sb = *reinterpret_cast<const f32x4*>(cs + D / 2 + 32 * s + 4);
 #pragma unroll
-      for (int z = 0; z < 2; ++z) {
-        c[i][z] = *reinterpret_cast<const f32x4*>(cs + 32 * i + 4 * z);
-        s[i][z] = *reinterpret_cast<const f32x4*>(cs + D / 2 + 32 * i + 4 * z);
-      }
+    for (int j = 0; j < 8; ++j) {
+      const float c = j < 4 ? ca[j] : cb[j - 4];
+      const float sn = j < 4 ? sa[j] : sb[j - 4];
+      const float a = bf2f(f[s][j]), b = bf2f(f[s + KS / 2][j]);
+      f[s][j] = f2bf(a * c - b * sn);
+      f[s + KS / 2][j] = f2bf(b * c + a * sn);
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
-  DRTC_DEVICE void turn(bf16x8* f) const {
-#pragma unroll
-    for (int i = 0; i < D / 64; ++i)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float a = bf2f(f[i][j]), b = bf2f(f[i + D / 64][j]), cc = c[i][j >> 2][j & 3], sn = s[i][j >> 2][j & 3];
-        f[i][j] = f2bf(a * cc - b * sn);
-        f[i + D / 64][j] = f2bf(b * cc + a * sn);
-      }
-  }
-};
+}
 
 DRTC_DEVICE void store_part(float* p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -185,15 +238,15 @@ DRTC_DEVICE void store_part(float* p, float v) {
 DRTC_DEVICE float load_part(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// ROPE (decode batches too small for the persistent kernel): q, k and v of the step's token come
-// unrotated, as there; wave 0 of the last partition opens its softmax with that token and writes its
-// rows, the cache is read up to the token ahead of it.  Bound by its chain of round trips (table,
-// K / V, partials, count, merge), not by bytes, until a batch fills the chip: one sequence of 2000 tokens
-// 11.3 us, 16 of 1000 19.9 us for 65 MB (rope_kv + a wave per partition + reduce: 21.9 and 26.4), 128 of
-// 1000 100 us (5.2 TB/s; rope_kv + this without ROPE 105).  cos | sin and the token's rows asked for
-// behind the first block: 200 of 400 75.8 us, now 71.5.
+// ROPE: q, k and v of the step's token come unrotated, as in the persistent kernel; wave 0 of the last partition
+// opens its softmax with that token and writes its rows, the cache is read up to the token ahead of it.
+// A block of K goes through LDS (KLds), V into registers, both asked for again as soon as they are used: with no
+// second block held the kernel fits 128 registers, so that four workgroups of a CU cover for each other, where two
+// blocks in registers left two.  Small batches are bound by the chain of round trips (table, K / V, partials, count,
+// merge), full ones by memory.  32 heads over 8 kv heads, us, two blocks in registers / this: 16 x 1000 tokens 24.5 /
+// 19.0, 64 x 300 21.3 / 18.4, 200 x 400 70.5 / 60.5 (5.4 TB/s), 1024 x 150 139 (persistent) / 115.8 (5.4 TB/s).
 template <int D, bool ROPE>
-__global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_kernel(
+__global__ __launch_bounds__(256, D >= 256 ? 2 : 4) void paged_decode_kernel(
     bf16_t* __restrict__ out, float* __restrict__ part_o,
     float* __restrict__ part_ml, int* __restrict__ counters, const bf16_t* __restrict__ q,
     int q_stride, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
@@ -202,12 +255,12 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_kernel(
     int max_parts, int blocks_per_part, DecodeRope rope) {
   constexpr int NT = D / 16;  // output d-tiles
   constexpr int KS = D / 32;  // k-steps of the QK product
-  const int b = blockIdx.x / Hkv;
-  const int h = blockIdx.x - b * Hkv;
   const int p = blockIdx.y;
   const int G = Hq / Hkv;
   const int lane = threadIdx.x & 63;
   const int w = wave_id_uniform();
+  const int b = blockIdx.x / Hkv;
+  const int h = blockIdx.x - b * Hkv;
   const int col = lane & 15, g = lane >> 4;
   const int blk_begin = p * blocks_per_part;
   // Issue every load that does not depend on the context length first: the
@@ -224,21 +277,6 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_kernel(
     if (col < G) qf[s] = load_bf16x8(qrow + 32 * s + 8 * g);
     else for (int j = 0; j < 8; ++j) qf[s][j] = f2bf(0.f);
   }
-  // the step's own k and v rows (wave 0: it takes the token, if this is the last partition)
-  [[maybe_unused]] bf16x8 kf[ROPE ? KS : 1];
-  [[maybe_unused]] bf16x4 vf[ROPE ? NT : 1];
-  [[maybe_unused]] bf16_t vw[ROPE ? D / 64 : 1];
-  if constexpr (ROPE) {
-    if (w == 0) {
-      const bf16_t* kn = q + (int64_t)b * q_stride + (int64_t)(Hq + h) * D;
-#pragma unroll
-      for (int s = 0; s < KS; ++s) kf[s] = load_bf16x8(kn + 32 * s + 8 * g);
-#pragma unroll
-      for (int i = 0; i < NT; ++i) vf[i] = load_bf16x4(kn + (int64_t)Hkv * D + 16 * i + 4 * g);
-#pragma unroll
-      for (int i = 0; i < D / 64; ++i) vw[i] = kn[(int64_t)Hkv * D + 64 * i + lane];
-    }
-  }
   const int ctx = context_lens[b];
   const int nc = ROPE ? ctx - 1 : ctx;  // tokens read from the cache
   const int pos = ROPE ? rope.positions[b] : 0;
@@ -253,6 +291,8 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_kernel(
     return;
   }
   if (p >= nparts) return;
+  const bool alone = nblk == 1;  // wave 0 has it all, and nothing to merge (1024 x 20: 57 -> 47 us)
+  if (alone && w != 0) return;
 
   const int blk_end = min(nblk, blk_begin + blocks_per_part);
 
@@ -262,29 +302,54 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_kernel(
   float m = kNegBig, lsum = 0.f;
 
   const int64_t blk_elems = (int64_t)kBS * D;
-  auto load_block = [&](KVRegs<D>& r, int64_t phys, int blk) {
-    const bf16_t* kb = k_cache + (phys * Hkv + h) * blk_elems;
-    const bf16_t* vb = v_cache + (phys * Hkv + h) * blk_elems;
-    if constexpr (ROPE) load_kv_block_n<D>(r, kb, vb, lane, nc - blk * kBS);
-    else load_kv_block<D>(r, kb, vb, lane);
+  // [4][16] m, [4][16] l, then each wave's K block, later its sums [D][16]
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  char* const klds = reinterpret_cast<char*>(smem + 128) + w * (D * 64);
+  const unsigned kdst = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(ad_lds_ptr)klds);
+  VRegs<D> v;
+  auto load_k = [&](int phys, int blk) {
+    KLds<D>::load(kdst, k_cache + ((int64_t)__builtin_amdgcn_readfirstlane(phys) * Hkv + h) * blk_elems, lane,
+                  nc - blk * kBS);
   };
-  // cos | sin ahead of the cache: memory answers in order, q and k turn while the block arrives
-  [[maybe_unused]] RopeRegs<D> cs;
+  auto load_v = [&](int phys, int blk) {
+    load_v_block<D>(v, v_cache + ((int64_t)phys * Hkv + h) * blk_elems, lane, nc - blk * kBS);
+  };
+  // ROPE: cos | sin of the position, and for the wave that takes the step's token its k and v, through LDS ahead of
+  // the cache (memory answers in order): held in registers they would cost a wave per SIMD
+  [[maybe_unused]] char* const stage = reinterpret_cast<char*>(smem + 128 + 64 * D) + 1024 * w;
+  [[maybe_unused]] const bool taker = ROPE && w == 0 && p == nparts - 1;
   if constexpr (ROPE) {
-    cs.load(rope.cos_sin, pos, g);
-    __builtin_amdgcn_sched_barrier(0);
+    const unsigned dst = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(ad_lds_ptr)stage), at = lane * 4u;
+    const __amdgpu_buffer_rsrc_t rc = dma_rsrc(rope.cos_sin + (int64_t)__builtin_amdgcn_readfirstlane(pos) * D);
+#pragma unroll
+    for (int i = 0; i < D / 64; ++i) dma_dword_lds(dst + 512 + 256 * i, at + 256u * i, rc);
+    if (taker) {
+      const __amdgpu_buffer_rsrc_t rq = dma_rsrc(q + (int64_t)b * q_stride + (int64_t)(Hq + h) * D);
+      const unsigned in = lane < D / 2 ? at : kNoRow;  // a row: D / 2 dwords
+      dma_dword_lds(dst, in, rq);
+      dma_dword_lds(dst + 256, lane < D / 2 ? at + (unsigned)(Hkv * D) * 2u : kNoRow, rq);
+    }
   }
-  KVRegs<D> cur, nxt;
   int blk = blk_begin + w;
-  int ph_next = ph_b;  // table entry of block blk + 4, loaded one step ahead
+  int ph_next = ph_b;  // table entry of the wave's next block, loaded one step ahead
   if (blk < blk_end) {
-    const int64_t phys = ph_a;
-    load_block(cur, phys, blk);
+    load_k(ph_a, blk);
+    load_v(ph_a, blk);
   }
   if constexpr (ROPE) {
-    cs.turn(qf);
-    if (w == 0 && p == nparts - 1) {
-      cs.turn(kf);
+    // q and what was staged have landed; of a whole block at most V is still on its way
+    if (blk < blk_end && nc - blk * kBS >= kBS) wait_vm<2 * NT>();
+    else wait_vm<0>();
+    asm volatile("" ::: "memory");
+    const float* cs = reinterpret_cast<const float*>(stage + 512);
+    rope_frags_lds<D>(qf, cs, g);
+    if (taker) {
+      const bf16_t* kn = reinterpret_cast<const bf16_t*>(stage);
+      const bf16_t* vn = kn + 128;
+      bf16x8 kf[KS];
+#pragma unroll
+      for (int s = 0; s < KS; ++s) kf[s] = load_bf16x8(kn + 32 * s + 8 * g);
+      rope_frags_lds<D>(kf, cs, g);
       float dot = 0.f;
 #pragma unroll
       for (int s = 0; s < KS; ++s)
@@ -301,29 +366,32 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_kernel(
         for (int s = 0; s < KS; ++s) store_bf16x8(kd + 32 * s, kf[s]);
       }
 #pragma unroll
-      for (int i = 0; i < NT; ++i)
+      for (int i = 0; i < NT; ++i) {
+        const bf16x4 vf = load_bf16x4(vn + 16 * i + 4 * g);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[i][r] = bf2f(vf[i][r]);
+        for (int r = 0; r < 4; ++r) o[i][r] = bf2f(vf[r]);
+      }
       if (slot >= 0) {  // V block [8 groups of 4 tokens][D][4]
         bf16_t* vd = rope.v_cache + (cblk * Hkv + h) * blk_elems + (off >> 2) * (4 * D) + (off & 3);
 #pragma unroll
-        for (int i = 0; i < D / 64; ++i) vd[(64 * i + lane) * 4] = vw[i];
+        for (int i = 0; i < D / 64; ++i) vd[(64 * i + lane) * 4] = vn[64 * i + lane];
       }
     }
   }
-  vm_wait_all();  // the first block lands before the loop (vm_wait_all)
   for (; blk < blk_end; blk += 4) {
-    const int nb = blk + 4;
-    if (nb < blk_end) {  // register double-buffer: next block in flight
-      const int64_t phys = ph_next;
-      load_block(nxt, phys, nb);
-      ph_next = bt[min(nb + 4, bt_stride - 1)];
-    }
+    const int nb = blk + 4, phys = ph_next;
+    ph_next = bt[min(nb + 4, bt_stride - 1)];
+    vm_wait_all();  // K and V of this block have landed
+    asm volatile("" ::: "memory");
     f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
-      s0 = mfma16(cur.k0[s], qf[s], s0);
-      s1 = mfma16(cur.k1[s], qf[s], s1);
+      s0 = mfma16(KLds<D>::frag(klds, col, s, g), qf[s], s0);
+      s1 = mfma16(KLds<D>::frag(klds, 16 + col, s, g), qf[s], s1);
+    }
+    if (nb < blk_end) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before it is written again
+      load_k(phys, nb);
     }
     const int tok0 = blk * kBS + 4 * g;
     float bmax = kNegBig;
@@ -359,18 +427,32 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_kernel(
       bf16x8 a;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        a[j] = cur.vlo[i][j];
-        a[4 + j] = cur.vhi[i][j];
+        a[j] = v.lo[i][j];
+        a[4 + j] = v.hi[i][j];
       }
       o[i] = mfma16(a, pf, o[i]);
     }
-    if (nb < blk_end) cur = nxt;
+    if (nb < blk_end) load_v(phys, nb);
   }
   lsum += __shfl_xor(lsum, 16, 64);
   lsum += __shfl_xor(lsum, 32, 64);
 
+  if (alone) {
+    if (col < G) {
+      const float inv = 1.f / lsum;
+      bf16_t* orow = out + ((int64_t)b * Hq + h * G + col) * D + 4 * g;
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        bf16x4 y;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y[r] = f2bf(o[i][r] * inv);
+        *reinterpret_cast<bf16x4*>(orow + 16 * i) = y;
+      }
+    }
+    return;
+  }
+
   // ---- merge the 4 waves through LDS
-  extern __shared__ __attribute__((aligned(16))) float smem[];
   float* sm_m = smem;              // [4][16]
   float* sm_l = smem + 64;         // [4][16]
   float* sm_o = smem + 128;        // [4][D][16]
@@ -638,40 +720,6 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_wave_kerne
 //     m = that score, p = 1, o = its v row;
 //   * that item also writes the rotated k row and the v row into the paged cache (slot from
 //     `slots`) for the next steps - the same bytes rope_kv_kernel writes.
-// One LDS-DMA wave-instruction of one dword per lane: 256 contiguous bytes land at the LDS byte
-// address `dst` (M0 saved and restored).  Counts in vmcnt like any vector load.
-DRTC_DEVICE void dma_dword_lds(unsigned dst, unsigned voff, __amdgpu_buffer_rsrc_t rsrc) {
-  unsigned keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\t"
-               "buffer_load_dword %2, %3, %4 offen lds\n\ts_mov_b32 m0, %0"
-               : "=&s"(keep)
-               : "s"(dst), "v"(voff), "s"(rsrc), "s"(0u)
-               : "memory");
-}
-
-// rope_frags with the position's cos | sin row read from LDS (the staged row of the item)
-template <int D>
-DRTC_DEVICE void rope_frags_lds(bf16x8* f, const float* cs_row, int g) {
-  constexpr int KS = D / 32;
-  const float* cs = cs_row + 8 * g;
-#pragma unroll
-  for (int s = 0; s < KS / 2; ++s) {
-    const f32x4 ca = *reinterpret_cast<const f32x4*>(cs + 32 * s);
-    const f32x4 cb = *reinterpret_cast<const f32x4*>(cs + 32 * s + 4);
-    const f32x4 sa = *reinterpret_cast<const f32x4*>(cs + D / 2 + 32 * s);
-    const f32x4 sb = *reinterpret_cast<const f32x4*>(cs + D / 2 + 32 * s + 4);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float c = j < 4 ? ca[j] : cb[j - 4];
-      const float sn = j < 4 ? sa[j] : sb[j - 4];
-      const float a = bf2f(f[s][j]), b = bf2f(f[s + KS / 2][j]);
-      f[s][j] = f2bf(a * c - b * sn);
-      f[s + KS / 2][j] = f2bf(b * c + a * sn);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  }
-}
-
 template <int D, bool ROPE>
 __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_persist_kernel(
     bf16_t* __restrict__ out, float* __restrict__ part_o,
@@ -1113,7 +1161,7 @@ int launch_paged_decode_rope(void* out, float* part_o, float* part_ml, const voi
     if (max_parts > 1 && !counters) return -2;
     if (max_parts > kFusedMergeParts) return -1;
     const dim3 grid(B * Hkv, max_parts);
-    const size_t lds = (128 + 4 * (size_t)D * 16) * sizeof(float);
+    const size_t lds = (128 + 4 * (size_t)D * 16) * sizeof(float) + 4096;  // and the staged rows
     (D == 64 ? paged_decode_kernel<64, true> : paged_decode_kernel<128, true>)<<<grid, pblock, lds, st>>>(
         (bf16_t*)out, part_o, part_ml, counters, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache,
         (const bf16_t*)v_cache, block_tables, bt_stride, context_lens, Hq, Hkv, sl2, max_parts, blocks_per_part, r);

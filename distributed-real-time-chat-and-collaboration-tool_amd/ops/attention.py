@@ -143,6 +143,20 @@ def decode_variant(batch: int, Hkv: int, D: int, max_blocks: int) -> int:
     if items < 256 and max_blocks > 8:
         return 2
     return 1
+
+
+def launch_variant(variant: int, max_blocks: int, max_parts: int, max_wgs: int = 0) -> int:
+    """The kernel that runs where ``decode_variant`` says ``variant``: 1, since its K passes through LDS in whole rows
+    and four of its workgroups fit a CU, where the others hold two blocks in registers - 32 heads over 8 kv heads, us,
+    1024 x 150 tokens 115 (3: 139), 256 x 1000 171 (206), 256 x 150 33 (41), 224 x 300 28 (39).  Left to the others: a
+    choice by hand, a grid capped by ``max_wgs``, more partitions than the merge holds, and tables of up to three
+    blocks, where not all of its four waves have work (1024 x 40: 59, 3: 52; 1024 x 20: 47, 38; 512 x 60: 37, 37; from
+    four blocks, 2048 x 90: 147, 173)."""
+    if DECODE_VARIANT or max_wgs or max_parts > (128 if FUSED_SPLIT_MERGE else 1):
+        return variant
+    return variant if variant == 3 and max_blocks <= 3 else 1
+
+
 # variant 1 merges split-K partitions inside the attention kernel (last
 # workgroup to finish) instead of a separate decode_reduce launch
 FUSED_SPLIT_MERGE = os.environ.get("DRTC_DECODE_FUSED_MERGE", "1") != "0"
@@ -159,8 +173,11 @@ def decode_partitioning(batch: int, Hkv: int, max_blocks: int, target_wgs: int =
     partitions shorter than ~8 blocks losing to the merge overhead (batch 8 at
     4k tokens: 28 us with 32-block parts vs 40 us with 4-block parts)."""
     variant = variant or decode_variant(batch, Hkv, D, max_blocks)
-    per_wg = 4 if variant in (2, 3) else 1
-    parts_wanted = max(1, math.ceil(target_wgs * per_wg / max(1, batch * Hkv)))
+    # a split context is some 384 workgroups, 1.5 a CU, of four waves each (launch_variant): with 1024 (one a wave)
+    # 16 x 1000 tokens of 8 kv heads took 21.0 us in 5 parts, with 384 18.6 in 3; 8 x 4000 33.7 / 31.4, 1 x 16000
+    # 28.9 / 25.2, 13 x 700 15.4 / 15.4
+    wanted = 1.5 * target_wgs if variant == 2 else target_wgs * (4 if variant == 3 else 1)
+    parts_wanted = max(1, math.ceil(wanted / max(1, batch * Hkv)))
     bpp = max(8, math.ceil(max_blocks / parts_wanted))
     bpp = ((bpp + 3) // 4) * 4
     max_parts = max(1, math.ceil(max_blocks / bpp))
@@ -228,10 +245,11 @@ def paged_decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
     assert block_tables.dtype == torch.int32 and block_tables.stride(1) == 1
     assert context_lens.dtype == torch.int32 and context_lens.numel() >= B
     max_blocks = block_tables.shape[1]
-    variant = variant or decode_variant(B, Hkv, D, block_tables.shape[1])
+    picked = variant or decode_variant(B, Hkv, D, max_blocks)
     if blocks_per_part is None or workspace is None:
-        blocks_per_part, max_parts = decode_partitioning(B, Hkv, max_blocks, variant=variant, D=D)
+        blocks_per_part, max_parts = decode_partitioning(B, Hkv, max_blocks, variant=picked, D=D)
         workspace = DecodeWorkspace(B, Hq, D, max_parts, q.device)
+    variant = variant or launch_variant(picked, max_blocks, workspace.max_parts)
     if out is None:
         out = torch.empty((B, Hq, D), dtype=q.dtype, device=q.device)
     assert out.is_contiguous() and out.shape == (B, Hq, D)
@@ -251,17 +269,18 @@ def paged_decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
 FUSED_ROPE = os.environ.get("DRTC_DECODE_FUSED_ROPE", "1") != "0"
 
 
-def fused_rope_variant(variant: int, D: int, max_parts: int) -> int:
+def fused_rope_variant(variant: int, D: int, max_parts: int, max_blocks: int = 0, max_wgs: int = 0) -> int:
     """The kernel that takes RoPE, the KV write and the merge of the partitions into the attention
-    launch, or 0.  3 stays itself; 1 runs the shapes of 1 and 2: a workgroup per partition, so 8
+    launch, or 0: 1 or 3 (``launch_variant``), a workgroup per partition of 1, so 8
     blocks are 2 per wave, and one launch instead of rope_kv, attention and decode_reduce.  Its merge
     holds up to 128 partitions.  32 heads of 128 over 8 kv heads, three launches against one:
     1 x 2000 tokens 21.9 -> 11.3 us, 1 x 16000 43.7 -> 27.0, 1 x 64000 95 -> 68, 8 x 4000 42.7 -> 31.8,
     16 x 1000 26.4 -> 19.9; two launches (one partition) against one: 40 x 1000 47.2 -> 41.8,
-    64 x 300 23.2 -> 20.6, 128 x 1000 105 -> 100, 200 x 400 74.0 -> 71.5."""
+    64 x 300 23.2 -> 20.6, 128 x 1000 105 -> 100, 200 x 400 74.0 -> 71.5 (all before K went through LDS)."""
     if D not in (64, 128) or DECODE_VARIANT == 2:
         return 0
-    return 3 if variant == 3 else 1 if max_parts <= (128 if FUSED_SPLIT_MERGE else 1) else 0
+    variant = launch_variant(variant, max_blocks, max_parts, max_wgs)
+    return variant if variant != 2 else 1 if max_parts <= (128 if FUSED_SPLIT_MERGE else 1) else 0
 
 
 def paged_decode_attention_rope(qkv: torch.Tensor, positions: torch.Tensor, slots: torch.Tensor,
@@ -288,7 +307,7 @@ def paged_decode_attention_rope(qkv: torch.Tensor, positions: torch.Tensor, slot
     if on_gpu(qkv) and FUSED_ROPE:
         max_parts = (workspace.max_parts if blocks_per_part is not None and workspace is not None
                      else decode_partitioning(B, Hkv, block_tables.shape[1], variant=variant, D=D)[1])
-        fused = fused_rope_variant(variant, D, max_parts)
+        fused = fused_rope_variant(variant, D, max_parts, block_tables.shape[1], max_wgs)
     if not fused:
         rope_kv_(qkv, positions, slots, cos_sin, Hq, Hkv, D, k_cache, v_cache, KV_BLOCK)
         return paged_decode_attention(q, k_cache, v_cache, block_tables, context_lens, scale,

@@ -1252,3 +1252,52 @@ def test_rope_kv_v_and_padding_in_one_launch(hipk, D, Hq, Hkv, lens, pad):
     assert torch.equal(qkv, q2) and torch.equal(kc, k2) and torch.equal(vc, v2)
     z = rows[n:T, D:2 * D + 8]
     assert (z == 0).all() and int(rows.isnan().sum()) == rows.numel() - z.numel()
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,rope", [(64, 8, 2, True), (128, 32, 8, True), (64, 4, 4, False), (128, 16, 1, False),
+                                           (256, 8, 1, False)])
+@pytest.mark.parametrize("bpp", [64, 4])
+def test_paged_decode_reads_no_row_past_the_context(hipk, D, Hq, Hkv, rope, bpp):
+    """K through LDS, a block at a time: contexts of one block (one wave, no merge) to several a wave, NaN in every K
+    row and whole V group behind the context, in one or several partitions; rounding of the tests above."""
+    from drtc_amd.ops import attention as attn_ops
+
+    ctx_lens = [1, 2, 4, 0, 31, 32, 33, 36, 64, 65, 127, 128, 129, 160, 161, 290]
+    B, bs = len(ctx_lens), ops.KV_BLOCK
+    q, kc, vc, bt, cl = _paged_setup(B, Hq, Hkv, D, ctx_lens, seed=31)
+    kn, vn = kc.clone(), vc.clone()
+    for b, c in enumerate(ctx_lens):
+        have = c - 1 if rope else c  # rows in the cache
+        for j in range(-(-c // bs)):
+            n = max(have - j * bs, 0)
+            if n < bs:
+                blk = int(bt[b, j])
+                kn[blk, :, n:] = float("nan")
+                vn[blk].view(Hkv, bs // 4, D, 4)[:, -(-n // 4):] = float("nan")
+    mp = -(-bt.shape[1] // bpp)
+    assert attn_ops.launch_variant(attn_ops.decode_variant(B, Hkv, D, bt.shape[1]), bt.shape[1], mp) == 1
+    kw = dict(blocks_per_part=bpp, workspace=ops.DecodeWorkspace(B, Hq, D, mp, DEV))
+    if not rope:
+        out = ops.paged_decode_attention(q, kn, vn, bt, cl, D ** -0.5, **kw)
+    else:
+        qkv = torch.cat([q.flatten(1), torch.randn(B, 2 * Hkv * D, device=DEV).to(torch.bfloat16)], 1)
+        pos = (cl - 1).clamp(min=0)
+        slots = torch.tensor([int(bt[b, (c - 1) // bs]) * bs + (c - 1) % bs if c else -1
+                              for b, c in enumerate(ctx_lens)], device=DEV)
+        cs = ops.build_rope_cache(512, D, 1e4, device=DEV)
+        out = ops.paged_decode_attention_rope(qkv, pos, slots, cs, Hq, Hkv, D, kn, vn, bt, cl, D ** -0.5, **kw)
+        ops.rope_kv_ref(qkv, pos, slots, cs, Hq, Hkv, D, kc, vc, bs)
+        q = qkv[:, :Hq * D].reshape(B, Hq, D)
+    _close(out, ops.paged_decode_ref(q, kc, vc, bt, cl, D ** -0.5), 2e-2, 2e-2, "attention")
+
+
+def test_decode_kernel_by_table_width():
+    """The kernel that runs: 1 but for a choice by hand, a capped grid, a table of up to three blocks and more
+    partitions than its merge holds."""
+    from drtc_amd.ops import attention as a
+
+    assert a.launch_variant(3, 64, 1) == a.launch_variant(2, 64, 8) == a.launch_variant(1, 2, 1) == 1
+    assert a.launch_variant(3, 3, 1) == a.launch_variant(3, 64, 1, max_wgs=256) == 3
+    assert a.launch_variant(2, 4096, 129) == 2 and a.launch_variant(2, 2, 1) == 1
+    assert a.fused_rope_variant(3, 128, 1, 64) == a.fused_rope_variant(2, 64, 5, 64) == 1
+    assert a.fused_rope_variant(3, 128, 1, 2) == 3 and a.fused_rope_variant(1, 256, 1, 64) == 0
