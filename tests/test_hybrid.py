@@ -994,3 +994,33 @@ def test_limits_are_errors():
     with pytest.raises(ValueError):
         build_model(TINY_MEBALORN, "cpu", pc=ParallelContext(tp_size=2, tp_rank=0))
     assert math.isclose(config_from_dict(config(16, 16, latent(1, 8, 8, 8, 8, 3))).layers[0].mixer.scale, 0.25)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,R", [(1, 512), (16, 512), (16, 256), (20, 512), (32, 256), (40, 256), (64, 512)])
+@pytest.mark.parametrize("parts", [1, 3])
+def test_latent_decode_in_pairs_of_blocks(H, R, parts):
+    """Rows of whole cache lines, two blocks at a time: one block, odd and even counts, a table of more than 64
+    entries, windows, splits that end within a pair, rows with no context; rounding of the test above."""
+    dev, dt, rot, nb = "cuda", torch.bfloat16, 64, 74
+    LW = ops.latent_width(R, rot)
+    assert LW == R + 64
+    ctx = [1, 32, 33, 64, 65, 96, 97, 0, 2079, 2080, 2081, 2330]
+    B = len(ctx)
+    g = torch.Generator().manual_seed(R + H)
+    cache = (torch.randn(B * nb + 1, 32, LW, generator=g) * 0.5).to(dt)
+    bt = torch.randperm(B * nb, generator=g).view(B, nb).to(torch.int32) + 1
+    qa = (torch.randn(B, H, LW, generator=g) * 0.5).to(dt)
+    for window in (None, 40, 2070):
+        ws = ops.LatentDecodeWorkspace(B, H, R, window, nb, dev)
+        ws.per, ws.splits = -(-nb // parts), parts
+        ws.part_o, ws.part_ml = torch.empty(B, H, parts, R, device=dev), torch.empty(B, H, parts, 2, device=dev)
+        out = ops.latent_decode_attention(qa.to(dev), cache.to(dev), R, bt.to(dev),
+                                          torch.tensor(ctx, dtype=torch.int32, device=dev), window, 0.05, None, ws)
+        for b, n in enumerate(ctx):
+            if n == 0:
+                assert (out[b] == 0).all()
+                continue
+            rows = cache[bt[b].long()].reshape(-1, LW)[max(0, n - (window or n)):n].double()
+            p = (qa[b].double() @ rows.T * 0.05).softmax(-1)
+            close(out[b], p @ rows[:, :R], 2e-2)
