@@ -957,11 +957,61 @@ __global__ __launch_bounds__(256) void head_gemm_kernel(
   }
 }
 
+// The same for long K on a chip with room: a workgroup's waves share its 16 output dims and take every fourth
+// 128 of K, their sums meet in LDS: one round trip to memory where a wave alone makes K / 128.  128 dims from 512, us:
+// 200 rows of 16 heads 11.3 -> 7.2, 64 of 32 11.2 -> 4.8.
+template <int NBT>
+__global__ __launch_bounds__(256) void head_gemm_shared_kernel(
+    bf16_t* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, int B,
+    int N, int K, int64_t yb, int64_t yh, int64_t xb, int64_t xh) {
+  __shared__ f32x4 sums[4][NBT][64];
+  const int h = blockIdx.z, b0 = blockIdx.y * 16 * NBT, n0 = blockIdx.x * 16;
+  const int wv = wave_id_uniform(), lane = threadIdx.x & 63;
+  const int col = lane & 15, g = lane >> 4;
+  const bf16_t* wr = w + ((int64_t)h * N + min(n0 + col, N - 1)) * K;
+  const bf16_t* xr[NBT];
+#pragma unroll
+  for (int i = 0; i < NBT; ++i) xr[i] = x + (int64_t)min(b0 + 16 * i + col, B - 1) * xb + h * xh;
+  f32x4 acc[NBT];
+#pragma unroll
+  for (int i = 0; i < NBT; ++i) acc[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  for (int k = 128 * wv; k < K; k += 512) {
+    bf16x8 wf[4], xf[4][NBT];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      wf[s] = load_bf16x8(wr + k + 32 * s + 8 * g);
+#pragma unroll
+      for (int i = 0; i < NBT; ++i) xf[s][i] = load_bf16x8(xr[i] + k + 32 * s + 8 * g);
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int i = 0; i < NBT; ++i) acc[i] = mfma16(wf[s], xf[s][i], acc[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < NBT; ++i) sums[wv][i][lane] = acc[i];
+  __syncthreads();
+  for (int i = wv; i < NBT; i += 4) {
+    const f32x4 s = (sums[0][i][lane] + sums[1][i][lane]) + (sums[2][i][lane] + sums[3][i][lane]);
+    const int b = b0 + 16 * i + col, n = n0 + 4 * g;
+    if (b < B && n < N) {
+      bf16x4 v;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = f2bf(s[r]);
+      *reinterpret_cast<bf16x4*>(y + b * yb + h * yh + n) = v;
+    }
+  }
+}
+
 template <int NBT>
 static void head_gemm_go(bf16_t* y, const bf16_t* x, const bf16_t* w, int B, int H, int N, int K,
                          int64_t yb, int64_t yh, int64_t xb, int64_t xh, hipStream_t st) {
   const dim3 grid((N + 63) / 64, (B + 16 * NBT - 1) / (16 * NBT), H);
-  if (K % 128 == 0)
+  // shared where a CU would have half a workgroup: 128 dims from 512 of 32 heads, 128 rows 11.4 / 8.4 us, 200 (one a
+  // CU) 12.4 / 13.7; with fewer rows to a workgroup up to one a CU: 256 dims of 64 heads, 32 rows 8.8 / 8.3
+  if (K % 128 == 0 && K >= 256 && (int64_t)grid.x * grid.y * H <= (NBT == 4 ? 128 : 256))
+    head_gemm_shared_kernel<NBT><<<dim3((N + 15) / 16, grid.y, H), dim3(256), 0, st>>>(y, x, w, B, N, K, yb, yh, xb, xh);
+  else if (K % 128 == 0)
     head_gemm_kernel<NBT, true><<<grid, dim3(256), 0, st>>>(y, x, w, B, N, K, yb, yh, xb, xh);
   else
     head_gemm_kernel<NBT, false><<<grid, dim3(256), 0, st>>>(y, x, w, B, N, K, yb, yh, xb, xh);

@@ -1024,3 +1024,16 @@ def test_latent_decode_in_pairs_of_blocks(H, R, parts):
             rows = cache[bt[b].long()].reshape(-1, LW)[max(0, n - (window or n)):n].double()
             p = (qa[b].double() @ rows.T * 0.05).softmax(-1)
             close(out[b], p @ rows[:, :R], 2e-2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,N,K", [(1, 3, 64, 256), (17, 2, 20, 384), (70, 4, 128, 512), (128, 2, 36, 640), (32, 4, 16, 1024)])
+def test_head_linear_with_shared_k(B, H, N, K):
+    """Heads whose products a workgroup's waves share, K in 2 to 8 parts of 128: bf16 rounding of the result."""
+    g = torch.Generator(device="cuda").manual_seed(B + K)
+    x = torch.randn(B, H, K + 8, device="cuda", generator=g).to(torch.bfloat16)
+    w = (torch.randn(H, N, K, device="cuda", generator=g) / K ** 0.5).to(torch.bfloat16)
+    out = torch.full((B, H, N + 8), 5.0, dtype=torch.bfloat16, device="cuda")
+    ops.head_linear(x, w, out=out)
+    want = torch.stack([x[:, h, :K].double() @ w[h].double().t() for h in range(H)], 1)
+    assert ((out[..., :N].double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all() and (out[..., N:] == 5).all()
