@@ -7,7 +7,8 @@
 // set by the operand bytes each CU must read: (rows + columns of its tile) x K x 2.  This
 // kernel picks the tile per shape:
 //
-//   * 128 MT x 32 NF output tiles (MT 1 / 2, NF 2 / 4 / 6 / 8), K split over splitk = 1..8 slices
+//   * 64 x 32 NF output tiles (MT 0, NF 1 / 2 / 4; plain products of up to 256 rows on a workgroup a CU or fewer:
+//     3584 x 2048, 224 rows 10.7 us in tiles of 128 x 64, 8.9 of 64 x 64), or 128 MT x 32 NF (MT 1 / 2, NF 2 / 4 / 6 / 8), K split over splitk = 1..8 slices
 //     (whole K tiles, as even as they divide), one workgroup per (tile, slice) and per CU
 //     (o / down at M = 1024: 8 x 32 tiles of 128 x 128, or 4 x 32 x 2 slices of 256 x 128;
 //     qkv N = 6144: 8 x 32 of 128 x 192; Llama-3-70B at M = 256: 256 x 128 x 3-4 slices;
@@ -19,7 +20,7 @@
 //     panels and ALL row tiles of each.  Every weight byte is fetched from HBM into ONE XCD's
 //     L2, and the workgroups that share a panel stream it through that L2 in K-lockstep (the
 //     activations, 1-8 MB, are read by every XCD from the Infinity Cache).
-//   * 4 waves, one per SIMD, 64 MT x 16 NF outputs per wave (4 MT x NF MFMA 16x16x32 tiles);
+//   * 4 waves, one per SIMD, 64 MT x 16 NF outputs per wave (4 MT x NF MFMA 16x16x32 tiles; MT 0: 2 x NF);
 //     the 16x16x32 form, not 32x32x16: same LDS bytes per FLOP at a given wave tile, and the
 //     bf16 16x16x32 loop holds a 12-15 % higher clock on random data (MI355X_MICROARCH.md,
 //     DVFS give-back item 7).
@@ -68,20 +69,20 @@ struct XdCfg {
   static constexpr int MT = MT_, NF = NF_, S = S_;
   static constexpr bool SPLIT = SPLIT_;            // split-K combine compiled in
   static constexpr bool NT = NT_;                  // weight (B) LDS-DMA non-temporal
-  static constexpr int TM = 128 * MT;              // tile rows
+  static constexpr int FA = MT ? 4 * MT : 2;       // A fragments per wave (16 rows each); MT 0: 64-row tiles
+  static constexpr int TM = 32 * FA;               // tile rows
   static constexpr int TN = 32 * NF;               // tile columns
-  static constexpr int FA = 4 * MT;                // A fragments per wave (16 rows each)
   static constexpr int H = FA * NF;                // MFMAs per 32-deep K half (per wave)
-  static constexpr int DA = 4 * MT, DB = NF, D = DA + DB;  // LDS-DMA per wave per K tile
+  static constexpr int DA = FA, DB = NF, D = DA + DB;  // LDS-DMA per wave per K tile
   static constexpr int NR = FA + NF;               // fragment reads per wave per K half
   static constexpr int BOFF = TM * 128;            // B region within a stage
   static constexpr int STAGE = BOFF + TN * 128;
   static constexpr int LDS = S * STAGE;            // the K-tile ring
   static constexpr int PITCH = 32 * NF + 16;       // epilogue bytes per wave-tile row (padded)
-  static constexpr int IMAGE = 4 * 64 * MT * PITCH;  // the epilogue's bf16 tile image
+  static constexpr int IMAGE = 4 * 16 * FA * PITCH;  // the epilogue's bf16 tile image
   static constexpr int ALLOC = LDS > IMAGE ? LDS : IMAGE;
   static_assert(ALLOC <= 160 * 1024, "LDS exceeds the CU's 160 KiB");
-  static_assert(NR < H, "half-0 fragment reads must fit the half");
+  static_assert(NR < H || MT == 0, "half-0 fragment reads, one behind an MFMA, must fit the half");
 };
 
 struct XdParams {
@@ -120,7 +121,7 @@ struct XdDma {
   unsigned lds_a, lds_b;  // LDS byte address of this wave's first DMA block in stage 0
 };
 
-// Fragment read offsets within a stage (bytes): row 64 MT wm + l16 (A) / 16 NF wn + l16 (B),
+// Fragment read offsets within a stage (bytes): row 16 FA wm + l16 (A) / 16 NF wn + l16 (B),
 // 16-B chunk 4 h + g stored at chunk ^ ((row >> 1) & 7); + 2048 per 16-row fragment.
 struct XdFrag {
   int ra0, ra1, rb0, rb1;
@@ -230,7 +231,9 @@ DRTC_DEVICE void xd_step(f32x4 (&acc)[C::FA][C::NF], bf16x8 (&fa0)[C::FA], bf16x
   else
     acc[i][j] = mfma16(fa1[i], fb1[j], acc[i][j]);
   // ---- half 0: fragments of this tile's half 1 (one per MFMA from step 1)
-  if constexpr (h == 0 && Q >= 1 && Q <= C::NR)
+  if constexpr (C::MT == 0 && h == 0)  // (of a few MFMAs: spread over all)
+    xd_reads<C, (rem * C::NR + H - 1) / H, ((rem + 1) * C::NR + H - 1) / H>(fa1, fb1, lds, cur, f.ra1, f.rb1);
+  else if constexpr (h == 0 && Q >= 1 && Q <= C::NR)
     xd_read<C, Q - 1>(fa1, fb1, lds, cur, f.ra1, f.rb1);
   // ---- boundary: tile t + 1 landed for every wave; every read of this stage is done
   if constexpr (NEXT && Q == H - 1) {
@@ -399,7 +402,7 @@ DRTC_DEVICE void xd_sum_frags(const XdParams& p, const __amdgpu_buffer_rsrc_t& s
 }
 template <class C, int EPI, bool G = false>
 __global__ __launch_bounds__(kXdThreads, 1) void gemm_xd_kernel(XdParams p) {
-  constexpr int MT = C::MT, NF = C::NF, FA = C::FA;
+  constexpr int NF = C::NF, FA = C::FA;
   extern __shared__ __attribute__((aligned(16))) char xd_lds[];
   // ---- work item: XCD label x = b % 8 takes the items [x per_xcd, (x + 1) per_xcd) of the
   // slice-major, column-major order (item = slice * tiles + tile; all row tiles of a weight
@@ -433,7 +436,7 @@ __global__ __launch_bounds__(kXdThreads, 1) void gemm_xd_kernel(XdParams p) {
   const int wm = wv >> 1, wn = wv & 1, l16 = lane & 15, g = lane >> 4;
   const int64_t k0 = (int64_t)kt0 * 64;
 
-  // ---- DMA plan: instruction i of wave wv fills stage rows 32 MT wv + 8 i + (lane >> 3)
+  // ---- DMA plan: instruction i of wave wv fills stage rows 8 FA wv + 8 i + (lane >> 3)
   // (A) / 8 NF wv + 8 i + (lane >> 3) (B), lane's LDS chunk lane & 7 <- source chunk ^
   // swizzle.  A rows past M read row M - 1 (valid bytes, never stored).
   XdDma<C> d;
@@ -447,7 +450,7 @@ __global__ __launch_bounds__(kXdThreads, 1) void gemm_xd_kernel(XdParams p) {
     d.rb = __builtin_amdgcn_make_buffer_rsrc((void*)bbase, (short)0, 0x7FFFFFFF, 0x00020000);
 #pragma unroll
     for (int i = 0; i < C::DA; ++i) {
-      const int R = 32 * MT * wv + 8 * i + (lane >> 3);
+      const int R = 8 * FA * wv + 8 * i + (lane >> 3);
       const int c = (lane & 7) ^ ((R >> 1) & 7);
       const int row = min(R, rows_a - 1);
       const int src = gather ? p.g_aidx[m0 + row] : row;  // A row (a token, grouped mode)
@@ -467,14 +470,14 @@ __global__ __launch_bounds__(kXdThreads, 1) void gemm_xd_kernel(XdParams p) {
       }
       d.vb[i] = (unsigned)(src * p.ldb * 2 + c * 16);
     }
-    d.lds_a = __builtin_amdgcn_readfirstlane(lds0 + 32 * MT * wv * 128);
+    d.lds_a = __builtin_amdgcn_readfirstlane(lds0 + 8 * FA * wv * 128);
     d.lds_b = __builtin_amdgcn_readfirstlane(lds0 + C::BOFF + 8 * NF * wv * 128);
   }
   XdFrag f;
   {
     const int fx = (l16 >> 1) & 7;
-    f.ra0 = (64 * MT * wm + l16) * 128 + ((0 + g) ^ fx) * 16;
-    f.ra1 = (64 * MT * wm + l16) * 128 + ((4 + g) ^ fx) * 16;
+    f.ra0 = (16 * FA * wm + l16) * 128 + ((0 + g) ^ fx) * 16;
+    f.ra1 = (16 * FA * wm + l16) * 128 + ((4 + g) ^ fx) * 16;
     f.rb0 = C::BOFF + (16 * NF * wn + l16) * 128 + ((0 + g) ^ fx) * 16;
     f.rb1 = C::BOFF + (16 * NF * wn + l16) * 128 + ((4 + g) ^ fx) * 16;
   }
@@ -532,18 +535,18 @@ __global__ __launch_bounds__(kXdThreads, 1) void gemm_xd_kernel(XdParams p) {
   }
 
   // ---- epilogue: the wave's tile as bf16 into LDS, then 16-B global stores of whole row
-  // segments (acc[i][j][r] = C[64 MT wm + 16 i + 4 g + r][16 NF wn + 16 j + l16]; gated:
+  // segments (acc[i][j][r] = C[16 FA wm + 16 i + 4 g + r][16 NF wn + 16 j + l16]; gated:
   // output column 8 NF wn + 16 j + l16 = act(acc[i][j]) * acc[i][j + NF / 2], j < NF / 2)
   __syncthreads();  // every wave is done reading the stages
   constexpr int OC = xd_glu<EPI>() ? 8 * NF : 16 * NF;  // output columns per wave
   constexpr int PITCH = 2 * OC + 16;
-  char* ep = xd_lds + wv * 64 * MT * PITCH;
+  char* ep = xd_lds + wv * 16 * FA * PITCH;
   const __amdgpu_buffer_rsrc_t slab = xd_slab(p);
   // split-K combine groups (the sums are consumed here, the accumulators stay in place): a
   // row block's fragments x 4 slice positions in flight, NF 6 / 8 one position at a time
   // (more spills: those kernels hold 192 / 256 accumulator registers)
   constexpr int QG = NF >= 6 ? 1 : 4;
-  constexpr int NP = NF >= 8 ? 4 : NF / 2;  // gated: column pairs per group
+  constexpr int NP = NF >= 8 ? 4 : NF >= 2 ? NF / 2 : 1;  // gated: column pairs per group
   constexpr int JB = NF >= 8 ? 8 : NF;      // plain: fragments per group
   static_assert(NF % JB == 0 && (NF / 2) % NP == 0, "combine groups tile the fragments");
 #pragma unroll
@@ -600,11 +603,11 @@ __global__ __launch_bounds__(kXdThreads, 1) void gemm_xd_kernel(XdParams p) {
   __syncthreads();
   constexpr int CPR = OC / 8;  // 16-B chunks per wave-tile row
 #pragma unroll
-  for (int s = 0; s < CPR * MT; ++s) {
+  for (int s = 0; s < CPR * FA / 4; ++s) {
     const int q = lane + 64 * s;
     const int row = q / CPR, ch = q - row * CPR;
-    if (64 * MT * wm + row >= rows_a) continue;
-    const int m = m0 + 64 * MT * wm + row;
+    if (16 * FA * wm + row >= rows_a) continue;
+    const int m = m0 + 16 * FA * wm + row;
     const int n = n0 + OC * wn + 8 * ch;
     bf16x8 v = *reinterpret_cast<const bf16x8*>(ep + row * PITCH + ch * 16);
     if constexpr (EPI == XD_RESIDUAL) {
@@ -625,7 +628,14 @@ int xd_launch_e(const XdParams& p, hipStream_t st) {
 
 template <class C>
 int xd_launch(const XdParams& p, int epi, hipStream_t st) {
-  switch (epi) {
+  if constexpr (C::MT == 0) {  // plain products only
+    switch (epi) {
+      case XD_STORE: return xd_launch_e<C, XD_STORE>(p, st);
+      case XD_RESIDUAL: return xd_launch_e<C, XD_RESIDUAL>(p, st);
+      case XD_RELU2: return xd_launch_e<C, XD_RELU2>(p, st);
+      default: return -1;
+    }
+  } else switch (epi) {
     case XD_STORE: return xd_launch_e<C, XD_STORE>(p, st);
     case XD_RESIDUAL: return xd_launch_e<C, XD_RESIDUAL>(p, st);
     case XD_SILU: return xd_launch_e<C, XD_SILU>(p, st);
@@ -654,6 +664,12 @@ int xd_launch_g(const XdParams& p, int epi, hipStream_t st) {
 template <class C>
 int xd_cfg() {
   int e = 0;
+  if constexpr (C::MT == 0) {
+    for (const void* f : {(const void*)gemm_xd_kernel<C, XD_STORE>, (const void*)gemm_xd_kernel<C, XD_RESIDUAL>,
+                          (const void*)gemm_xd_kernel<C, XD_RELU2>})
+      e |= (int)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, C::ALLOC);
+    return e;
+  } else {
   for (const void* f : {(const void*)gemm_xd_kernel<C, XD_STORE>,
                         (const void*)gemm_xd_kernel<C, XD_RESIDUAL>,
                         (const void*)gemm_xd_kernel<C, XD_SILU>,
@@ -664,6 +680,7 @@ int xd_cfg() {
     e |= (int)hipFuncSetAttribute((const void*)gemm_xd_kernel<C, XD_CLAMP>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, C::ALLOC);
   return e;
+  }
 }
 template <class C>
 int xd_cfg_g() {
@@ -694,7 +711,16 @@ using Xd2x6 = XdCfg<2, 6, 2, SP, NT>;
 template <bool SP, bool NT = false>
 using Xd2x8 = XdCfg<2, 8, 2, SP, NT>;
 
+// 64-row tiles of 32, 64 and 128 columns (six stages; four of 24 KiB), without either
+template <bool NT = false>
+using Xd0x1 = XdCfg<0, 1, 6, false, NT>;
+template <bool NT = false>
+using Xd0x2 = XdCfg<0, 2, 6, false, NT>;
+template <bool NT = false>
+using Xd0x4 = XdCfg<0, 4, 4, false, NT>;
+
 int xd_stages(int mt, int nf) {
+  if (mt == 0) return nf == 1 || nf == 2 ? 6 : (nf == 4 ? 4 : 0);
   if (mt == 1) return nf == 6 ? 3 : (nf == 2 || nf == 4 ? 4 : 0);
   if (mt == 2) return nf == 4 ? 3 : (nf == 6 || nf == 8 ? 2 : 0);
   return 0;
@@ -702,6 +728,18 @@ int xd_stages(int mt, int nf) {
 
 template <bool SP>
 int xd_dispatch(const XdParams& p, int mt, int nf, bool nt, int epi, hipStream_t st) {
+  if (mt == 0) {
+    if constexpr (SP) return -1;
+    else switch (nf + (nt ? 10 : 0)) {
+      case 1: return xd_launch<Xd0x1<>>(p, epi, st);
+      case 2: return xd_launch<Xd0x2<>>(p, epi, st);
+      case 4: return xd_launch<Xd0x4<>>(p, epi, st);
+      case 11: return xd_launch<Xd0x1<true>>(p, epi, st);
+      case 12: return xd_launch<Xd0x2<true>>(p, epi, st);
+      case 14: return xd_launch<Xd0x4<true>>(p, epi, st);
+      default: return -1;
+    }
+  }
   if (nt) {
     switch (mt * 10 + nf) {
       case 14: return xd_launch<Xd1x4<SP, true>>(p, epi, st);
@@ -745,7 +783,7 @@ int splitk_spin_limit() { return g_spin_limit; }
 void set_splitk_spin_limit(int limit) { g_spin_limit = limit; }
 
 int64_t gemm_xd_workspace_bytes(int M, int N, int mt, int nf, int splitk, int glu) {
-  if (splitk < 2 || mt < 1 || nf < 1) return 0;
+  if (splitk < 2 || mt < 1 || nf < 1) return 0;  // (64-row tiles have no slices)
   const int tno = glu ? 16 * nf : 32 * nf;
   const int64_t tiles = (int64_t)((M + 128 * mt - 1) / (128 * mt)) * (N / tno);
   return tiles * splitk * (128 * mt) * (32 * nf) * 4;
@@ -764,7 +802,8 @@ int launch_gemm_xd(void* c, const void* a, const void* b, const void* r, int M, 
   if (lda % 8 || ldb % 8 || ldc % 8) return -1;
   if ((uintptr_t)a % 16 || (uintptr_t)b % 16 || (uintptr_t)c % 16) return -1;
   if (epi == XD_RESIDUAL && (r == nullptr || ldr % 8 || (uintptr_t)r % 16)) return -1;
-  const int tm_rows = 128 * mt, tno = glu ? 16 * nf : 32 * nf;
+  if (mt == 0 && (glu || splitk > 1)) return -1;
+  const int tm_rows = mt ? 128 * mt : 64, tno = glu ? 16 * nf : 32 * nf;
   // shape contract: whole column tiles, every slice more K tiles than the ring holds (the
   // first K tile is peeled), 32-bit buffer offsets from the tile bases
   if (M <= 0 || N <= 0 || N % tno || K % 64 || K / 64 / splitk <= stages) return -1;
@@ -818,7 +857,7 @@ int launch_gemm_xd_grouped(void* c, const void* a, const void* b, int a_rows, in
   if (epi < XD_STORE || epi > XD_RELU2 || epi == XD_RESIDUAL) return -1;
   const bool glu = epi != XD_STORE && epi != XD_RELU2;
   const int stages = xd_stages(mt, nf);
-  if (stages == 0 || splitk < 1 || splitk > 8 || (glu && nf % 2)) return -1;
+  if (mt == 0 || stages == 0 || splitk < 1 || splitk > 8 || (glu && nf % 2)) return -1;
   if (lda % 8 || ldb % 8 || ldc % 8 || max_tiles < 1 || a_rows < 1) return -1;
   if ((uintptr_t)a % 16 || (uintptr_t)b % 16 || (uintptr_t)c % 16) return -1;
   if (tile_row0 == nullptr || tile_rows == nullptr || tile_expert == nullptr || n_tiles == nullptr)
@@ -872,7 +911,8 @@ int configure_gemm_xd() {
                 xd_cfg_g<Xd2x8<false, true>>() | xd_cfg_g<Xd1x4<true, true>>() |
                 xd_cfg_g<Xd2x4<true, true>>() | xd_cfg_g<Xd2x8<true, true>>();
   if (g) return g;
-  return xd_cfg<Xd1x2<false>>() | xd_cfg<Xd1x4<false>>() | xd_cfg<Xd1x6<false>>() |
+  return xd_cfg<Xd0x1<>>() | xd_cfg<Xd0x2<>>() | xd_cfg<Xd0x4<>>() | xd_cfg<Xd0x1<true>>() | xd_cfg<Xd0x2<true>>() |
+         xd_cfg<Xd0x4<true>>() | xd_cfg<Xd1x2<false>>() | xd_cfg<Xd1x4<false>>() | xd_cfg<Xd1x6<false>>() |
          xd_cfg<Xd2x4<false>>() | xd_cfg<Xd2x6<false>>() | xd_cfg<Xd1x2<true>>() |
          xd_cfg<Xd1x4<true>>() | xd_cfg<Xd1x6<true>>() | xd_cfg<Xd2x4<true>>() |
          xd_cfg<Xd2x6<true>>() | xd_cfg<Xd2x8<false>>() | xd_cfg<Xd2x8<true>>() |

@@ -240,6 +240,9 @@ def _resolve(M: int, N: int, K: int, ldx: int) -> tuple[str, int]:
     wide = wide_form(M, N, K)
     if wide and not (found is not None and found[1][3]):  # (entries of gemm_xd: measured against its other forms)
         return ("xd", wide)
+    small = small_form(M, N, K)
+    if small and ldx % 8 == 0:
+        return ("xd", small)
     if brief_ok(M, N, K) and ldx % 8 == 0:
         return ("midm", 201)
     # the rule goes ahead of the table, but for entries that were measured faster ("stream": 0)
@@ -263,6 +266,28 @@ def _resolve(M: int, N: int, K: int, ldx: int) -> tuple[str, int]:
                 return ("lt", algo)
     v = skinny_variant(M, N, K, ldx)
     return ("skinny", v) if v else ("torch", 0)
+
+
+def small_form(M: int, N: int, K: int) -> int:
+    """gemm_xd form of 64-row tiles for a plain product of 17 .. 256 rows that they cut into at most a workgroup a CU, of
+    32 columns or else 64: what a workgroup reads, at 45 - 65 GB/s, is the time of such a product, and its other forms and
+    the library's leave half the chip idle or read all rows everywhere.  us, the best of those / this: 3584 x 2048, 64 rows
+    9.5 / 7.7, 128 10.9 / 7.8, 224 10.7 / 8.9; 2048 x 2048, 224 10.5 / 7.8; 3840 x 2048, 100 14.0 / 8.2; 6912 x 4096, 32 15.5 / 13.6,
+    100 20.3 / 18.9; 12800 x 4096, 32 23.7 / 19.7, 64 25.3 / 23.4; 4096 x 4096, 160 19.7 / 17.5.
+    Not where K slices fill the chip better: long K on half the CUs (4096 x 4096, 64 rows 14.3 / 16.8), nor for long K and
+    whole row tiles, several of them (6144 x 4096, 100 rows 20.1 / 18.6, 128 20.8 / 21.1), nor 64 columns
+    where up to 32 rows stream (8448 x 2048, 32 rows 12.2 / 13.6).  Weights of 32 MiB on, one row tile: non-temporal (6912 x 4096, 64 rows 18.6 /
+    17.1; 8192 x 2048 11.8 / 10.1; 3840 x 2048 9.4 / 9.7)."""
+    if not (_xd_enabled and _enabled and 17 <= M <= 256 and 2048 <= K <= 4096 and N >= 2048):
+        return 0
+    tiles = -(-M // 64)
+    nf = next((n for n in (1, 2) if N % (32 * n) == 0 and tiles * (N // (32 * n)) <= 256), 0)
+    items = tiles * (N // (32 * nf)) if nf else 0
+    if not nf or (K > 2048 and (items < 160 or M > 64 and (M - 1) % 64 >= 48)) or (
+            nf == 2 and M <= 32 and stream_ok(M, N, K)):
+        return 0
+    form = 10 * nf + 1 + (1000 if _xd_nt and tiles == 1 and N * K >= 1 << 24 else 0)
+    return form if xd_supported(M, N, K, form) else 0
 
 
 def brief_ok(M: int, N: int, K: int) -> bool:
@@ -1071,15 +1096,15 @@ def squared_relu(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.T
 
 # ------------------------------------------------------------------ XCD-partitioned decode GEMM
 XD_EPI = {"store": 0, "residual": 1, "silu": 2, "gelu_tanh": 3, "clamped": 4, "relu2": 5}
-# tile shapes built in gemm_xd.hip, (mt, nf) -> LDS ring depth (128 mt x 32 nf tiles); a form
+# tile shapes built in gemm_xd.hip, (mt, nf) -> LDS ring depth (128 mt x 32 nf tiles, mt 0: 64 rows); a form
 # is mt * 100 + nf * 10 + splitk (K split over 1..8 slices), + 1000 for non-temporal weight
 # loads (the tiles of XD_NT_TILES)
-XD_TILES = {(1, 2): 4, (1, 4): 4, (1, 6): 3, (2, 4): 3, (2, 6): 2, (2, 8): 2}
+XD_TILES = {(0, 1): 6, (0, 2): 6, (0, 4): 4, (1, 2): 4, (1, 4): 4, (1, 6): 3, (2, 4): 3, (2, 6): 2, (2, 8): 2}
 XD_CLAMP_NF = (4, 8)  # tile widths the clamped epilogue is built for
-XD_NT_TILES = {(1, 4), (1, 6), (2, 4), (2, 6), (2, 8)}
+XD_NT_TILES = {(0, 1), (0, 2), (0, 4), (1, 4), (1, 6), (2, 4), (2, 6), (2, 8)}
 XD_MAX_SPLITK = 8
 # the forms the tuner (scripts/tune_xd.py) measures
-XD_FORMS = tuple(sorted([mt * 100 + nf * 10 + 1 for mt, nf in XD_TILES] +
+XD_FORMS = tuple(sorted([mt * 100 + nf * 10 + 1 for mt, nf in XD_TILES if mt] +
                         [200 + nf * 10 + sk for nf in (4, 6, 8) for sk in (2, 3, 4)]))
 
 
@@ -1096,7 +1121,7 @@ def xd_supported(M: int, N: int, K: int, form: int, glu: bool = False) -> bool:
     """Shapes gemm_xd.hip takes in ``form`` (mt * 100 + nf * 10 + splitk); N = output
     columns (gated: half the rows of the [gate; up] weight)."""
     mt, nf, sk = xd_form(form)
-    if (mt, nf) not in XD_TILES or not 1 <= sk <= XD_MAX_SPLITK or (glu and nf % 2):
+    if (mt, nf) not in XD_TILES or not 1 <= sk <= XD_MAX_SPLITK or (glu and nf % 2) or mt == 0 and (glu or sk > 1):
         return False
     if form // 1000 > 1 or (xd_nt(form) and (mt, nf) not in XD_NT_TILES):
         return False
@@ -1104,7 +1129,7 @@ def xd_supported(M: int, N: int, K: int, form: int, glu: bool = False) -> bool:
     if not (M >= 1 and N % tno == 0 and K % 64 == 0 and K // 64 // sk > XD_TILES[(mt, nf)]):
         return False
     # split-K: the partial slots and tile counters fit the device workspace
-    tiles = -(-M // (128 * mt)) * (N // tno)
+    tiles = -(-M // (128 * max(mt, 1))) * (N // tno)
     return sk == 1 or (tiles * sk * (128 * mt) * (32 * nf) * 4 <= WS_SLAB_BYTES
                        and 2 * tiles + 2 <= WS_COUNTERS)  # + the fault word (last counter)
 
@@ -1134,7 +1159,7 @@ def xd_gemm(x: torch.Tensor, w: torch.Tensor, epi: str = "store",
             limit: float = 0.0) -> torch.Tensor:
     """Decode-shaped hand GEMM, csrc/kernels/gemm_xd.hip: y = epi(x @ w.T) on 128 mt x 32 nf
     tiles, K split over 1..8 slices, with the tile order partitioned by XCD (each XCD streams
-    its own weight column panels through its L2 for every row tile).  epi "store";
+    its own weight column panels through its L2 for every row tile); mt 0: 64 rows, plain, one slice.  epi "store";
     "residual" (``out`` may be ``residual``); "silu" / "gelu_tanh": w is the fused [gate; up]
     weight [2I, K] and y[:, n] = act(x . gate_n) * (x . up_n); "clamped": bounded by ``limit``
     (tiles of XD_CLAMP_NF); "relu2": relu(x @ w.T)^2.  ``form`` = mt * 100 + nf * 10 + splitk (+ 1000: non-temporal weight loads; 0: ``xd_default_form``)."""

@@ -453,3 +453,34 @@ def test_short_k_products(hipk, M, N, K):
     for x in (wide[:, 8:K + 8], wide[:, 3:K + 3], wide[:, :K].contiguous()):
         got, want = ops.linear(x, w).double(), x.double() @ w.double().t()
         assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 17, 63, 64, 65, 200, 256])
+@pytest.mark.parametrize("form", [11, 21, 41, 1011, 1021, 1041])
+@pytest.mark.parametrize("N,K", [(256, 512), (384, 2048)])
+def test_row_tiles_of_64(hipk, M, form, N, K):
+    """gemm_xd on tiles of 64 rows: one row tile (each workgroup starts K at another tile) and several, rows of a
+    wider buffer, residual and squared epilogues.  bf16 rounding of the result (twice with the residual)."""
+    g = torch.Generator(device="cuda").manual_seed(M + form)
+    x = torch.randn(M, K + 8, device="cuda", generator=g).to(torch.bfloat16)[:, :K]
+    w = (torch.randn(N, K, device="cuda", generator=g) / K ** 0.5).to(torch.bfloat16)
+    res = torch.randn(M, N, device="cuda", generator=g).to(torch.bfloat16)
+    want = x.double() @ w.double().t()
+    near = lambda got, ref, add=0.0: bool(((got.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + add + 1e-5).all())
+    assert near(G.xd_gemm(x, w, form=form), want)
+    assert near(G.xd_gemm(x, w, "relu2", form=form), want.clamp(min=0) ** 2, 1e-5 * want.abs().max())
+    assert near(G.xd_gemm(x, w, "residual", residual=res.clone(), form=form), want + res.double(), 2.0 ** -8 * want.abs())
+    assert not G.xd_supported(M, N, K, form + 1) and not G.xd_supported(M, N, K, form, glu=True)
+
+
+def test_small_products_rule():
+    """Which products the 64-row tiles take: at most a workgroup a CU of their tiles, long K on more than half of
+    them."""
+    forms = {(M, N, K): G.small_form(M, N, K) for M in (16, 17, 32, 64, 100, 128, 224, 256, 257)
+             for N in (1024, 2048, 3584, 6144, 8448, 32000) for K in (1984, 2048, 4096, 4160)}
+    assert not any(f for (M, N, K), f in forms.items() if M in (16, 257) or N in (1024, 32000) or K in (1984, 4160))
+    assert forms[64, 3584, 2048] == 11 and forms[224, 3584, 2048] == 21 and forms[224, 2048, 2048] == 11
+    assert forms[64, 6144, 4096] == 1011 and forms[100, 6144, 4096] == 21 and forms[128, 6144, 4096] == 0
+    assert forms[32, 8448, 2048] == 0 and forms[64, 8448, 2048] == 1021 and forms[224, 8448, 2048] == 0
+    assert forms[64, 2048, 4096] == 0 and forms[128, 8448, 2048] == 0
