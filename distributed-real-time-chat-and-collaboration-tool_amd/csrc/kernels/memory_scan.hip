@@ -833,7 +833,8 @@ __global__ __launch_bounds__(256) void memory_decode_kernel(MemoryArgs a) {
           y[v] = s[j][v] * da + k * u[v];
           o[v] += q * y[v];
         }
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, y), buf, mine, j * step, 0);
+        // (no scalar offset in a register: delta_rule.hip, move_all)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, y), buf, mine + j * step, 0, 0);
         __builtin_amdgcn_sched_barrier(0);  // a row at a time: few registers
       }
     } else for (int r0 = rg; r0 < a.dim; r0 += RG * U) {

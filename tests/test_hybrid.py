@@ -1037,3 +1037,31 @@ def test_head_linear_with_shared_k(B, H, N, K):
     ops.head_linear(x, w, out=out)
     want = torch.stack([x[:, h, :K].double() @ w[h].double().t() for h in range(H)], 1)
     assert ((out[..., :N].double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all() and (out[..., N:] == 5).all()
+
+
+@pytest.mark.gpu
+def test_delta_decode_large_steps(hipk):
+    """A step that keeps the whole chip's memory busy, against the same sequences one by one, a first token over a
+    state of NaN and a row without a state among them.  Inputs kept in bf16: the same; outputs: to their rounding;
+    states: sums of 128 products of about 1, whose multiply-adds two kernels may contract differently (128 roundings
+    of 2^-24)."""
+    B, H, d, taps, dev = 50, 32, 128, 4, "cuda"
+    g = torch.Generator(device=dev).manual_seed(5)
+    r = lambda *s, std=1.0: torch.randn(*s, generator=g, device=dev) * std
+    C = 3 * H * d
+    proj, decay, gate = r(B, C + H).to(BF16), r(B, H * d).to(BF16), r(B, H * d).to(BF16)
+    w = ops.DeltaWeights(r(taps, C, std=0.5), torch.linspace(-1, 1, H, device=dev).exp(), r(H * d) - 2, 1 + 0.1 * r(d), 1e-5, H,
+                         H, d, d)
+    ring, state = r(B, taps, C).to(BF16), r(B, H, d, d)
+    state[2] = float("nan")
+    pos = torch.arange(B, dtype=torch.int32, device=dev).roll(2)  # row 2 (state 2): its first token
+    slot = torch.arange(B, dtype=torch.int32, device=dev)
+    slot[7] = -1
+    outs = []
+    for parts in ((slice(0, B),), tuple(slice(i, i + 1) for i in range(B))):
+        rg, sg = ring.clone(), state.clone()
+        o = torch.cat([ops.delta_decode(proj[p], C, w, rg, sg, decay[p], gate[p], pos[p], slot[p]) for p in parts])
+        outs.append((o, rg, sg))
+    (o, rg, sg), (o2, rg2, sg2) = outs
+    assert torch.equal(rg, rg2) and sg.isfinite().all() and ((sg - sg2).abs() <= 2.0 ** -17 * (1 + sg2.abs())).all()
+    assert ((o.float() - o2.float()).abs() <= 2.0 ** -8 * o2.float().abs() + 1e-5).all()
