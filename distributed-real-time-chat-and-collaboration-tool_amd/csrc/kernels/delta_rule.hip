@@ -190,8 +190,8 @@ struct StateTile {
         s[i][c] = r < dim && col + c < vdim ? S[(int64_t)r * vdim + col + c] : 0.f;
     }
   }
-  // of a state that fills the tiles: one register of addresses
-  template <bool STORE>
+  // of a state that fills the tiles: one register of addresses.  NT: non-temporal
+  template <bool STORE, bool NT = false>
   DRTC_DEVICE void move_all(float* S, int col, int p, int vdim) {
     static_assert(CPL % 4 == 0, "16-byte pieces");
     const __amdgpu_buffer_rsrc_t at =
@@ -209,9 +209,9 @@ struct StateTile {
           // the whole offset in a register of the lanes: behind a 16-byte store whose scalar offset is a register
           // the compiler writes the data's registers again at once, and the store, read late on a busy chip,
           // took lanes 12 - 15 of each 16 from there
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), at, off + 4 * c + so, 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), at, off + 4 * c + so, 0, NT ? 2 : 0);
         } else {
-          v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(at, off + 4 * c, so, 0));
+          v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(at, off + 4 * c, so, NT ? 2 : 0));
 #pragma unroll
           for (int j = 0; j < 4; ++j) s[i][c + j] = v[j];
         }
@@ -1160,9 +1160,10 @@ __global__ __launch_bounds__(256) void delta_read_kernel(DeltaArgs a) {
 // Bound by the state, read and written once; everything a token needs besides it is asked for ahead of
 // it, so that the token is prepared while it arrives (memory answers in order).  EXACT: the state fills
 // the lanes' tiles, so no load of it stands behind a condition and the waits can count them.  64 sequences x 32 heads of
-// 128 x 128 58.7 -> 53.7 us (5.0 TB/s), 256 x 32 284 -> 223 (4.8).
+// 128 x 128 58.7 -> 53.7 us (5.0 TB/s), 256 x 32 284 -> 223 (4.8).  NT: the states past the caches, which hold a step's
+// weights instead; in the pass of 64 x 32 heads 60.5 -> 54 and the kernels around it 2 % (the rule: kStatesPastCaches).
 constexpr int kDecodeTaps = 4;  // taps whose inputs are fetched ahead; more are read where they are used
-template <class T, int DPL, int CPL, bool EXACT>
+template <class T, int DPL, int CPL, bool EXACT, bool NT = false>
 __global__ __launch_bounds__(512) void delta_decode_kernel(DeltaArgs a) {
   constexpr int DP = 8 * DPL;
   extern __shared__ __attribute__((aligned(16))) float sm[];
@@ -1225,7 +1226,7 @@ __global__ __launch_bounds__(512) void delta_decode_kernel(DeltaArgs a) {
   const float dt0 = a.dt_bias[h * a.dim + i0];
   __builtin_amdgcn_sched_barrier(0);
   StateTile<DPL, CPL> st;
-  if constexpr (EXACT) st.template move_all<false>(S, col, p, a.vdim);
+  if constexpr (EXACT) st.template move_all<false, NT>(S, col, p, a.vdim);
   else if (pos > 0) st.load(S, col, p, a.dim, a.vdim);
   __builtin_amdgcn_sched_barrier(0);
   float sq = 0.f, sk = 0.f, dot = 0.f;
@@ -1271,7 +1272,7 @@ __global__ __launch_bounds__(512) void delta_decode_kernel(DeltaArgs a) {
 #pragma unroll
     for (int c = 0; c < CPL; ++c) v[c] = col + c < a.vdim ? vs[col + c] : 0.f;
     st.token(ks, qs, gs, p, beta, qk, v, o);
-    if constexpr (EXACT) st.template move_all<true>(S, col, p, a.vdim);
+    if constexpr (EXACT) st.template move_all<true, NT>(S, col, p, a.vdim);
     else st.store(S, col, p, a.dim, a.vdim);
 #pragma unroll
     for (int c = 0; c < CPL; ++c)
@@ -1380,6 +1381,10 @@ int launch_delta_scan(int f32, const DeltaArgs& a, int cpl, hipStream_t st) {
   return rc ? rc : (int)hipGetLastError();
 }
 
+// Bytes of a step's states from which on they go past the caches.  us a step of four layers, two of them these, through /
+// past: 128 MiB (64 sequences, 32 heads, width 4096) 617 / 597, 96 547 / 541, 80 528 / 538, 64 486 / 498; on width 2048, whose
+// weights a cache holds, 128 MiB 496 / 462, 64 366 / 335.
+constexpr int64_t kStatesPastCaches = 96ll << 20;
 template <class T, int DPL, int CPL>
 static int decode_go(const DeltaArgs& a, hipStream_t st) {
   const int waves = (a.vdim + 8 * CPL - 1) / (8 * CPL);
@@ -1387,7 +1392,9 @@ static int decode_go(const DeltaArgs& a, hipStream_t st) {
   if (waves > 8) return -1;
   if constexpr (DPL <= 16) {
     if (a.dim == 8 * DPL && a.vdim == 8 * CPL * waves) {
-      delta_decode_kernel<T, DPL, CPL, true><<<dim3(a.rows, a.H), dim3(64 * waves), lds, st>>>(a);
+      const bool past = (int64_t)a.rows * a.H * a.dim * a.vdim * 4 >= kStatesPastCaches;
+      (past ? delta_decode_kernel<T, DPL, CPL, true, true> : delta_decode_kernel<T, DPL, CPL, true>)
+          <<<dim3(a.rows, a.H), dim3(64 * waves), lds, st>>>(a);
       return 0;
     }
   }

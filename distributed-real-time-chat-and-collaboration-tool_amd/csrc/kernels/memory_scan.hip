@@ -703,7 +703,8 @@ __global__ __launch_bounds__(64 * NW, 2) void memory_chunk_kernel(MemoryArgs a) 
 // flight while queries and keys are prepared.  Bound by the state, read and written once: 200 sequences x
 // 16 heads of 128 x 128 66 us (6.3 TB/s), 256 x 32 213 (5.0); with the token's inputs asked for behind the
 // state and loads behind conditions 74 and 231.
-template <class T, int V, bool EXACT>
+// NT: the states past the caches, which hold a step's weights instead.
+template <class T, int V, bool EXACT, bool NT = false>
 __global__ __launch_bounds__(256) void memory_decode_kernel(MemoryArgs a) {
   constexpr int U = 16;
   __shared__ float ks[256], qs[256], part[256 * V], os[1024], red[16];
@@ -774,7 +775,7 @@ __global__ __launch_bounds__(256) void memory_decode_kernel(MemoryArgs a) {
   if constexpr (EXACT) {
 #pragma unroll
     for (int i = 0; i < U; ++i) {
-      const f32x4 y = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(buf, mine, i * step, 0));
+      const f32x4 y = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(buf, mine, i * step, NT ? 2 : 0));
 #pragma unroll
       for (int v = 0; v < V; ++v) s[i][v] = y[v];
     }
@@ -834,7 +835,7 @@ __global__ __launch_bounds__(256) void memory_decode_kernel(MemoryArgs a) {
           o[v] += q * y[v];
         }
         // (no scalar offset in a register: delta_rule.hip, move_all)
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, y), buf, mine + j * step, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, y), buf, mine + j * step, 0, NT ? 2 : 0);
         __builtin_amdgcn_sched_barrier(0);  // a row at a time: few registers
       }
     } else for (int r0 = rg; r0 < a.dim; r0 += RG * U) {
@@ -972,12 +973,17 @@ int launch_memory_decode(int f32, const MemoryArgs& a, hipStream_t st) {
   const bool vec = a.vdim % 4 == 0;
   // 16 rows of 4 columns to a thread are the whole state
   const bool exact = vec && a.vdim <= 256 && 256 % (a.vdim / 4) == 0 && a.dim == 16 * (256 / (a.vdim / 4));
+  // us a step of four layers, two of them these, through the caches / past them: 200 MiB of states (200 sequences,
+  // 16 heads, width 2048) 943 / 898, 100 761 / 715, 80 694 / 668, on width 4096 1434 / 1392; 64 641 / 621 and 1338 / 1352,
+  // 40 594 / 600
+  const bool past = (int64_t)a.rows * a.H * a.dim * a.vdim * 4 > 64ll << 20;
   if (f32) {
     if (exact) memory_decode_kernel<float, 4, true><<<grid, blk, 0, st>>>(a);
     else if (vec) memory_decode_kernel<float, 4, false><<<grid, blk, 0, st>>>(a);
     else memory_decode_kernel<float, 1, false><<<grid, blk, 0, st>>>(a);
   } else {
-    if (exact) memory_decode_kernel<bf16_t, 4, true><<<grid, blk, 0, st>>>(a);
+    if (exact && past) memory_decode_kernel<bf16_t, 4, true, true><<<grid, blk, 0, st>>>(a);
+    else if (exact) memory_decode_kernel<bf16_t, 4, true><<<grid, blk, 0, st>>>(a);
     else if (vec) memory_decode_kernel<bf16_t, 4, false><<<grid, blk, 0, st>>>(a);
     else memory_decode_kernel<bf16_t, 1, false><<<grid, blk, 0, st>>>(a);
   }

@@ -1041,8 +1041,8 @@ def test_head_linear_with_shared_k(B, H, N, K):
 
 @pytest.mark.gpu
 def test_delta_decode_large_steps(hipk):
-    """A step that keeps the whole chip's memory busy, against the same sequences one by one, a first token over a
-    state of NaN and a row without a state among them.  Inputs kept in bf16: the same; outputs: to their rounding;
+    """A step that keeps the whole chip's memory busy, its states past the caches, against the same sequences one by
+    one, a first token over a state of NaN and a row without a state among them.  Inputs kept in bf16: the same; outputs: to their rounding;
     states: sums of 128 products of about 1, whose multiply-adds two kernels may contract differently (128 roundings
     of 2^-24)."""
     B, H, d, taps, dev = 50, 32, 128, 4, "cuda"

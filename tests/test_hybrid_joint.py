@@ -496,3 +496,25 @@ def test_side_norm_with_router(rows, W, N, E, y):
     out, lg = ops.side_norm(a, w, 1e-5, width=N, router=r, **kw)
     assert torch.equal(out, ops.side_norm(b, w, 1e-5, width=N, **kw)) and torch.equal(a, b)
     assert (lg.double() - out.double() @ r.double().t()).abs().max() <= 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["retention", "memory"])
+def test_memory_decode_states_past_the_caches(kind):
+    """A step whose states are large enough to go past the caches, against the same sequences in two smaller
+    steps, a first token and a row without a state among them.  Outputs to their rounding; states: a product and a sum,
+    whose contraction may differ (two roundings of 2^-24)."""
+    B, H, d = 34, 32, 128
+    proj, w, _, fresh = memory("cuda", torch.bfloat16, kind, (H, d, d, d), B)
+    pos, slot = i32([(i + 4) % B for i in range(B)], "cuda"), i32([i if i != 7 else -1 for i in range(B)], "cuda")
+    states = fresh(B, 0.5)
+    outs = []
+    for parts in ((slice(0, B),), (slice(0, 17), slice(17, B))):
+        s = [None if x is None else x.clone() for x in states]
+        o = torch.full((B, H * d), 7.0, dtype=torch.bfloat16, device="cuda")
+        for p in parts:
+            ops.memory_decode(proj[p], w, s, pos[p], slot[p], o[p])
+        outs.append([o] + [x for x in s if x is not None])
+    for k, (a, b) in enumerate(zip(*outs)):
+        a, b = a.float(), b.float()
+        assert ((a - b).abs() <= (2.0 ** -22 if k else 2.0 ** -8) * (1 + b.abs())).all()
