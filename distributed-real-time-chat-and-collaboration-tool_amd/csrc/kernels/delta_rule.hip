@@ -754,11 +754,14 @@ __global__ __launch_bounds__(NTHR, 2) void delta_chunk_kernel(DeltaArgs a) {
 //                layout is also a B operand
 //   delta_read   output norm and gate, rings
 // The chain is bound by the fp32 MFMA (32 cycles each, 64 + 32 of them per chunk and column tile, over
-// NW waves) and by two exchanges through LDS, about 700 cycles a chunk: 1.5 us per 16 tokens at CT = 2
-// against 10.3 us of delta_chunk, whose five barriers also wait for the staging.  Heads of 128,
-// 4 x 3,500 tokens, 16 heads: 664 us (prep 197, chain 397, read 65), delta_chunk 2,244; one portion of
-// 4,000: 457 against 2,492.  With portions and heads enough for every CU delta_chunk keeps the fp32
-// units as busy without operands in memory (64 x 250, 32 heads: 959 against 1,249).
+// NW waves) and by two exchanges through LDS.  Only the keys' products are ahead of the first: the queries' run while
+// the parts come back.  The operands of two chunks are under way at any time, which the compiler's waits count only
+// since nothing older than they is pending in the loop (S is waited for ahead of it, pointers are uniform): before, every
+// second chunk waited for all loads, 1.6 us per 16 tokens, now 1.0 at CT = 1 and 1.4 at CT = 2, 10.3 in delta_chunk,
+// whose five barriers also wait for the staging.  Heads of 128, 4 x 3,500 tokens, 16 heads: 640 us (prep 190,
+// chain 446 -> 387, read 64), delta_chunk 2,244; one portion of 4,000: 364 (chain 417 -> 262) against
+// 2,492.  With portions and heads enough for every CU delta_chunk keeps the fp32 units as busy without
+// operands in memory (64 x 250, 32 heads: 959 against 1,249).
 // Chunks are numbered through the portions in their order: at most rows / 16 + nseg of them.
 template <int DT>
 struct ChainEntry {  // floats of a (chunk, head)
@@ -964,9 +967,12 @@ __global__ __launch_bounds__(64 * chain_waves(DT), 2) void delta_chain_kernel(De
   static_assert(CT <= NW, "a wave to a column tile");
   __shared__ __attribute__((aligned(16))) float part[NW * 2 * CT * 256], us[CT * 256];
   const int seg = blockIdx.x / nh, hh = blockIdx.x % nh, h = h0 + hh;
-  const int slot = a.seg_state[seg];
+  // uniform, and in scalar registers: the loads of a chunk advance a scalar pointer past fixed lane offsets
+  auto uniform = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+  const int slot = uniform(a.seg_state[seg]);
   if (slot < 0) return;
-  const int n = a.seg_len[seg], row0 = a.seg_row[seg], pos0 = a.seg_pos[seg], nch = (n + 15) / 16;
+  const int n = uniform(a.seg_len[seg]), row0 = uniform(a.seg_row[seg]), pos0 = uniform(a.seg_pos[seg]);
+  const int nch = (n + 15) / 16;
   const int w = wave_id_uniform(), lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
   const int x0 = 16 * CT * blockIdx.y;
   int entry = 0;
@@ -987,13 +993,28 @@ __global__ __launch_bounds__(64 * chain_waves(DT), 2) void delta_chain_kernel(De
   };
   f32x4 st[TW][CT];
   state([&](int t, int ct, int r, bool in, float* at) { st[t][ct][r] = pos0 > 0 && in ? *at : 0.f; });
+  // S is there before the loop: else its first use in there waits for all loads, those of the chunks ahead too
+#pragma unroll
+  for (int t = 0; t < TW; ++t)
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) asm volatile("" : "+v"(st[t][ct]));
+  entry = uniform(entry);
   const float* p = a.ws + ((int64_t)entry * nh + hh) * E::N;
-  // wave w < CT: R, U and O of column tile w
-  const int xo = x0 + 16 * min(w, CT - 1) + col;
-  const T* v = (const T*)a.conv + (int64_t)row0 * a.C + 2 * a.Hk * a.dim + h * a.vdim + min(xo, a.vdim - 1);
+  // a wave of its own for R, U and O of column tile wc
+  const int wc = (w + NW - (CT == 1 ? (blockIdx.y + blockIdx.y / NW * 2) % NW : 0)) % NW;
+  const bool lead = wc < CT;
+  const int xo = x0 + 16 * min(wc, CT - 1) + col;
+  const T* v = (const T*)a.conv + (int64_t)row0 * a.C + 2 * a.Hk * a.dim + h * a.vdim;
+  unsigned vrow[4], vlast[4];  // of a lane's rows of a chunk; of the last one, where rows behind the end are the last row
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    vrow[r] = (4 * g + r) * a.C + min(xo, a.vdim - 1);
+    vlast[r] = min(4 * g + r, (n - 1) & 15) * a.C + min(xo, a.vdim - 1);
+  }
   const int64_t ldo = (int64_t)a.H * a.vdim16;
-  float* o = a.ws_o + ((int64_t)entry * 16 + 4 * g) * ldo + h * a.vdim16 + xo;
-  const bool mine = w < CT && xo < a.vdim16;
+  float* o = a.ws_o + (int64_t)entry * 16 * ldo + h * a.vdim16;
+  const unsigned orow = 4 * g * (unsigned)ldo + xo;
+  const bool mine = lead && xo < a.vdim16;
   // operands of two chunks: each part is loaded again, two chunks ahead, where it has been read
   // (one chunk is shorter than a load from HBM takes)
   struct Ops {
@@ -1003,22 +1024,24 @@ __global__ __launch_bounds__(64 * chain_waves(DT), 2) void delta_chain_kernel(De
   auto load_k = [&](Ops& x, const float* p) {
 #pragma unroll
     for (int t = 0; t < TW; ++t) {
-      x.ek[t] = *(const f32x4*)(p + E::ek + 256 * (TW * w + t) + 4 * lane);
-      x.eq[t] = *(const f32x4*)(p + E::eq + 256 * (TW * w + t) + 4 * lane);
+      x.ek[t] = *(const f32x4*)(p + E::ek + 256 * (TW * w + t) + 4u * lane);
+      x.eq[t] = *(const f32x4*)(p + E::eq + 256 * (TW * w + t) + 4u * lane);
     }
   };
   auto load_u = [&](Ops& x, const float* p) {
 #pragma unroll
     for (int t = 0; t < TW; ++t) {
-      x.kd[t] = *(const f32x4*)(p + E::kd + 256 * (TW * w + t) + 4 * lane);
-      x.gt[t] = *(const f32x4*)(p + E::gt + 16 * (TW * w + t) + 4 * g);
+      x.kd[t] = *(const f32x4*)(p + E::kd + 256 * (TW * w + t) + 4u * lane);
+      x.gt[t] = *(const f32x4*)(p + E::gt + 16 * (TW * w + t) + 4u * g);
     }
   };
-  auto load_m = [&](Ops& x, const float* p, int t0) {  // rows behind the portion's end: its last one
-    x.mu = *(const f32x4*)(p + E::mu + 4 * lane);
-    x.mo = *(const f32x4*)(p + E::mo + 4 * lane);
+  auto load_m = [&](Ops& x, const float* p, int c) {
+    x.mu = *(const f32x4*)(p + E::mu + 4u * lane);
+    x.mo = *(const f32x4*)(p + E::mo + 4u * lane);
+    const bool last = c >= nch - 1;
+    const T* at = v + (int64_t)(16 * min(c, nch - 1)) * a.C;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) x.v[r] = v[(int64_t)min(t0 + 4 * g + r, n - 1) * a.C];
+    for (int r = 0; r < 4; ++r) x.v[r] = at[last ? vlast[r] : vrow[r]];
   };
   Ops even, odd;
   auto chunk = [&](int c) { return p + (int64_t)min(c, nch - 1) * nh * E::N; };
@@ -1027,11 +1050,11 @@ __global__ __launch_bounds__(64 * chain_waves(DT), 2) void delta_chain_kernel(De
     load_m(even, chunk(0), 0);
     load_u(even, chunk(0));
     load_k(odd, chunk(1));
-    load_m(odd, chunk(1), 16);
+    load_m(odd, chunk(1), 1);
     load_u(odd, chunk(1));
   }
   float* mypart = part + w * 2 * CT * 256 + 4 * lane;
-  const float* sums = part + 256 * min(w, CT - 1) + 4 * lane;
+  const float* sums = part + 256 * min(wc, CT - 1) + 4 * lane;
   auto compute = [&](int c, Ops& x) {
     const float* ahead = chunk(c + 2);
     f32x4 rk[CT], ok[CT];
@@ -1042,37 +1065,44 @@ __global__ __launch_bounds__(64 * chain_waves(DT), 2) void delta_chain_kernel(De
 #pragma unroll
       for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-          rk[ct] = mfma_f32(x.ek[t][r], st[t][ct][r], rk[ct]);
-          ok[ct] = mfma_f32(x.eq[t][r], st[t][ct][r], ok[ct]);
-        }
-    load_k(x, ahead);
+        for (int ct = 0; ct < CT; ++ct) rk[ct] = mfma_f32(x.ek[t][r], st[t][ct][r], rk[ct]);
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
-      *(f32x4*)(mypart + 256 * ct) = rk[ct];
-      *(f32x4*)(mypart + 256 * (CT + ct)) = ok[ct];
-    }
+    for (int ct = 0; ct < CT; ++ct) *(f32x4*)(mypart + 256 * ct) = rk[ct];
     lds_barrier();
-    f32x4 res, y;
-    if (w < CT) {
-      f32x4 rs = *(const f32x4*)sums;
-      y = *(const f32x4*)(sums + 256 * CT);
+    // the queries' products run while the keys' parts come back from LDS
+    f32x4 rs[NW];
+    if (lead) {
 #pragma unroll
-      for (int i = 1; i < NW; ++i) {
-        rs += *(const f32x4*)(sums + i * 2 * CT * 256);
-        y += *(const f32x4*)(sums + i * 2 * CT * 256 + 256 * CT);
-      }
+      for (int i = 0; i < NW; ++i) rs[i] = *(const f32x4*)(sums + i * 2 * CT * 256);
+    }
+#pragma unroll
+    for (int t = 0; t < TW; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) ok[ct] = mfma_f32(x.eq[t][r], st[t][ct][r], ok[ct]);
+    load_k(x, ahead);
+    f32x4 res;
+    if (lead) {
+#pragma unroll
+      for (int i = 1; i < NW; ++i) rs[0] += rs[i];
       f32x4 u = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int r = 0; r < 4; ++r) res[r] = 16 * c + 4 * g + r < n ? to_f32(x.v[r]) - rs[r] : 0.f;
+      for (int r = 0; r < 4; ++r) res[r] = 16 * c + 4 * g + r < n ? to_f32(x.v[r]) - rs[0][r] : 0.f;
 #pragma unroll
       for (int r = 0; r < 4; ++r) u = mfma_f32(x.mu[r], res[r], u);
-      *(f32x4*)(us + 256 * w + 4 * lane) = u;
+      *(f32x4*)(us + 256 * wc + 4 * lane) = u;
     }
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) *(f32x4*)(mypart + 256 * (CT + ct)) = ok[ct];
     lds_barrier();
-    f32x4 u[CT];
+    f32x4 u[CT], ys[NW];
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) u[ct] = *(const f32x4*)(us + 256 * ct + 4 * lane);
+    if (lead) {
+#pragma unroll
+      for (int i = 0; i < NW; ++i) ys[i] = *(const f32x4*)(sums + i * 2 * CT * 256 + 256 * CT);
+    }
 #pragma unroll
     for (int t = 0; t < TW; ++t)
 #pragma unroll
@@ -1084,19 +1114,24 @@ __global__ __launch_bounds__(64 * chain_waves(DT), 2) void delta_chain_kernel(De
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) st[t][ct] = mfma_f32(x.kd[t][r], u[ct][r], st[t][ct]);
     load_u(x, ahead);
-    if (w < CT) {
+    if (lead) {
+      f32x4 y = ys[0];
+#pragma unroll
+      for (int i = 1; i < NW; ++i) y += ys[i];
 #pragma unroll
       for (int r = 0; r < 4; ++r) y = mfma_f32(x.mo[r], res[r], y);
       if (mine)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[(int64_t)(16 * c + r) * ldo] = y[r];
+        for (int r = 0; r < 4; ++r) (o + (16 * c + r) * ldo)[orow] = y[r];
     }
-    load_m(x, ahead, 16 * (c + 2));
+    load_m(x, ahead, c + 2);
   };
-  for (int c = 0; c < nch; c += 2) {
+#pragma unroll 1
+  for (int c = 0; c + 1 < nch; c += 2) {
     compute(c, even);
-    if (c + 1 < nch) compute(c + 1, odd);
+    compute(c + 1, odd);
   }
+  if (nch & 1) compute(nch - 1, even);
   state([&](int t, int ct, int r, bool in, float* at) {
     if (in) *at = st[t][ct][r];
   });
@@ -1340,12 +1375,17 @@ static int chain_go(const DeltaArgs& a, hipStream_t st) {
   for (int h0 = 0; h0 < a.H; h0 += nh) {
     const int m = std::min(nh, a.H - h0);
     delta_prep_kernel<T, DT><<<dim3(entries, m), dim3(256), 0, st>>>(a, h0);
-    // 64 columns to a workgroup read the operands half as often; 32 where that would leave CUs idle
     constexpr int NW = chain_waves(DT);
-    if (NW == 4 && (int64_t)a.nseg * m * ((a.vdim16 + 63) / 64) >= 512)
-      delta_chain_kernel<T, DT, NW><<<dim3(a.nseg * m, (a.vdim16 + 16 * NW - 1) / (16 * NW)), dim3(64 * NW), 0, st>>>(a, h0, m);
-    else
-      delta_chain_kernel<T, DT, 2><<<dim3(a.nseg * m, (a.vdim16 + 31) / 32), dim3(64 * NW), 0, st>>>(a, h0, m);
+    auto go = [&](auto kernel, int columns) {
+      kernel<<<dim3(a.nseg * m, (a.vdim16 + columns - 1) / columns), dim3(64 * NW), 0, st>>>(a, h0, m);
+    };
+    // The fewest columns to a workgroup wait least between its products and overlap with a CU's other ones; more
+    // read the operands less often.  Heads of 128, us with 16 / 32 columns: 16 chains of 4,000 tokens 262 / 371, 32 of 868
+    // 64 / 86, 64 of 3,500 387 / 390, 96 of 2,000 334 / 358, 144 of 1,000 269 / 231.
+    const int64_t chains = (int64_t)a.nseg * m;
+    if (chains * ((a.vdim16 + 15) / 16) <= 768) go(delta_chain_kernel<T, DT, 1>, 16);
+    else if (NW == 4 && chains * ((a.vdim16 + 63) / 64) >= 512) go(delta_chain_kernel<T, DT, NW>, 16 * NW);
+    else go(delta_chain_kernel<T, DT, 2>, 32);
   }
   if (a.vdim <= 128) delta_read_kernel<T, 1><<<dim3(entries, (a.H + 3) / 4), dim3(256), 0, st>>>(a);
   else delta_read_kernel<T, 2><<<dim3(entries, (a.H + 3) / 4), dim3(256), 0, st>>>(a);

@@ -327,7 +327,9 @@ def test_delta_rule(target, shape, columns):
 CHAIN_CASES = [  # heads, key heads, dim, vdim, lengths in the order of the portions, chunk bytes
     (2, 1, 128, 128, [33, 16, 49], 1 << 30), (3, 3, 40, 24, [64, 1, 17, 15], 1 << 30),
     (2, 2, 24, 8, [47], 1 << 30), (4, 2, 128, 72, [40, 34], 40000 * 4),  # one head at a time
-    (16, 4, 128, 256, [34, 33, 35, 17, 32, 31, 20, 34], 1 << 30), (4, 4, 64, 136, [80, 2], 1 << 30)]
+    (16, 4, 128, 256, [34, 33, 35, 17, 32, 31, 20, 34], 1 << 30), (4, 4, 64, 136, [80, 2], 1 << 30),
+    # 32 columns to a workgroup, the last with 16 and with 8; two waves
+    (16, 4, 64, 136, [34, 33, 35, 17, 32, 31, 20, 34], 1 << 30), (16, 2, 24, 104, [34, 33, 35, 17, 32, 31, 20, 34], 1 << 30)]
 
 
 @pytest.mark.gpu
@@ -363,7 +365,7 @@ def test_delta_decode_state_ahead(hipk, dt, H, Hk, d, dv, taps):
 @pytest.mark.parametrize("case", CHAIN_CASES, ids=str)
 def test_delta_chains(target, case, monkeypatch):
     """A few long portions (chunks prepared ahead): lengths around the chunks of 16, head sizes that
-    pad, heads in several passes, 64 columns to a workgroup; portions not in the order of their rows,
+    pad, heads in several passes, 16, 32 and 64 columns to a workgroup; portions not in the order of their rows,
     a padding portion, and the second half of every sequence continuing the first's state."""
     dev, dt = target
     *shape, lens, most = case
