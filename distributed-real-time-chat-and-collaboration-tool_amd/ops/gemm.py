@@ -7,7 +7,8 @@ shape (M, N, K, row stride of x) ONCE to a route, cached per shape (``route``):
   "w4"      gemm_w4.hip: 4-wave hand-scheduled MFMA GEMM,   prefill-sized passes (M >= W4_MIN_M,
             persistent, 256 x 256 tiles (``mfma_gemm``)     K <= W4_MAX_K or ``_w4_long``)
   "skinny"  gemv.hip weight-streaming kernels (M <= 16)     decode buckets where the table (or
-                                                            ``skinny_variant`` untuned) says so
+                                                            ``skinny_variant`` untuned) says so; one
+                                                            or two rows by ``dot2_ok``
             gemm_stream.hip (variant STREAM, M <= 64)       where ``stream_ok`` says so
   "midm"    gemm_midm.hip medium-M kernel (M <= 256)        decode buckets where the table says so, short K
                                                             (``brief_ok``: 100 x fragments + slices);
@@ -236,6 +237,8 @@ def _resolve(M: int, N: int, K: int, ldx: int) -> tuple[str, int]:
         if a >= 0:
             return ("lt", a)
         return ("w4", 0) if _w4_long(M, N, K) else ("torch", 0)
+    if dot2_ok(M, N, K, ldx):
+        return ("skinny", 1)
     found = _decode_entry(M, N, K, ldx)
     wide = wide_form(M, N, K)
     if wide and not (found is not None and found[1][3]):  # (entries of gemm_xd: measured against its other forms)
@@ -288,6 +291,15 @@ def small_form(M: int, N: int, K: int) -> int:
         return 0
     form = 10 * nf + 1 + (1000 if _xd_nt and tiles == 1 and N * K >= 1 << 24 else 0)
     return form if xd_supported(M, N, K, form) else 0
+
+
+def dot2_ok(M: int, N: int, K: int, ldx: int) -> bool:
+    """Whether one or two rows go to the dot2 kernel ahead of the table, whose entries were measured before its
+    weights went past the caches.  us, the MFMA form or the library / this: one row 32000 x 4096 43.7 / 40.5, 64128 x
+    4096 83.2 / 77.9, 128256 x 2048 82.8 / 76.9, 256000 x 2048 162 / 152, 57344 x 8192 157 / 143, 128256 x 8192 346 / 314;
+    two rows 16384 x 4096 24.1 / 22.2, 32000 x 4096 43.3 / 39.3, 57344 x 8192 154 / 134.  Smaller products gain less (two rows of
+    8192 x 2048 8.3 / 8.3, 4096 x 3584 8.2 / 7.8, 3584 x 2048 5.5 / 5.7) and stay with the table."""
+    return _enabled and M <= min(2, SKINNY_MAX_M) and N * K >= 1 << 25 and skinny_supports(1, M, N, K, ldx)
 
 
 def brief_ok(M: int, N: int, K: int) -> bool:

@@ -484,3 +484,32 @@ def test_small_products_rule():
     assert forms[64, 6144, 4096] == 1011 and forms[100, 6144, 4096] == 21 and forms[128, 6144, 4096] == 0
     assert forms[32, 8448, 2048] == 0 and forms[64, 8448, 2048] == 1021 and forms[224, 8448, 2048] == 0
     assert forms[64, 2048, 4096] == 0 and forms[128, 8448, 2048] == 0
+
+
+def test_dot2_rule():
+    """One and two rows from 2^25 weights on, K in whole waves and N in whole rows of them; rows 16 bytes apart."""
+    assert G.dot2_ok(1, 8192, 4096, 4096) and G.dot2_ok(2, 65536, 512, 520)
+    for M, N, K, ldx in ((3, 8192, 4096, 4096), (2, 8188, 4096, 4096), (2, 65538, 512, 512), (1, 32768, 1088, 1088),
+                         (2, 8192, 4096, 4100)):
+        assert not G.dot2_ok(M, N, K, ldx)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 2])
+@pytest.mark.parametrize("N,K", [(8192, 4096), (65540, 512), (16388, 2048), (2624, 12800)])
+def test_dot2_rule_products(hipk, M, N, K):
+    """The rule's products, and one row's with its norm, against fp32: twice the 2^-9 of a bf16 result, and fp32 sums;
+    with the norm its bf16 rows too (2^-9 of every product, signs at random: of the products' norm, 12 deviations)."""
+    g = torch.Generator(device="cuda").manual_seed(N + M)
+    x, w = (torch.randn(*s, device="cuda", generator=g).bfloat16() for s in ((M, K), (N, K)))
+    assert G.route(M, N, K, K) == ("skinny", 1)
+    want = x.float() @ w.float().T
+    assert ((ops.linear(x, w).float() - want).abs() <= 2 ** -8 * want.abs() + 1e-6 * K).all()
+    if K > 8192:  # no norm of such rows
+        return
+    nw = torch.rand(K, device="cuda", generator=g).bfloat16()
+    y = ops.norm_linear(ops.PendingNorm(x, None, nw, 1e-5, False), w).float()
+    xf = x.float()
+    n = xf * (xf.pow(2).mean(-1, keepdim=True) + 1e-5).rsqrt() * nw.float()
+    want = n @ w.float().T
+    assert ((y - want).abs() <= 2 ** -8 * want.abs() + 6 * 2 ** -8 * (n.pow(2) @ w.float().pow(2).T).sqrt()).all()
