@@ -244,7 +244,12 @@ DRTC_DEVICE float load_part(const float* p) {
 // second block held the kernel fits 128 registers, so that four workgroups of a CU cover for each other, where two
 // blocks in registers left two.  Small batches are bound by the chain of round trips (table, K / V, partials, count,
 // merge), full ones by memory.  32 heads over 8 kv heads, us, two blocks in registers / this: 16 x 1000 tokens 24.5 /
-// 19.0, 64 x 300 21.3 / 18.4, 200 x 400 70.5 / 60.5 (5.4 TB/s), 1024 x 150 139 (persistent) / 115.8 (5.4 TB/s).
+// 19.0, 64 x 300 21.3 / 18.4, 200 x 400 70.5 / 60.5 (5.4 TB/s), 1024 x 150 139 (persistent) / 115.8 (5.4 TB/s).  (D 256:
+// two workgroups, for their LDS.)
+// pack > 1 (pack_heads): a context of one block gives each of that many kv heads one wave of a workgroup, one of two
+// blocks two heads two waves each, where a workgroup to a head would leave three waves or two without work and
+// four or eight at work on a CU: 1024 x 20 tokens 45.8 -> 33.6 us (persistent: 36.7), x 40 58.3 -> 47.9 (51.8), x 60
+// 64.3 -> 61.5 (66.8), 512 x 20 24.7 -> 19.9 (20.7), 256 x 40 18.3 -> 16.8 (17.4); 256 x 20 13.8 -> 13.4 (12.0).
 template <int D, bool ROPE>
 __global__ __launch_bounds__(256, D >= 256 ? 2 : 4) void paged_decode_kernel(
     bf16_t* __restrict__ out, float* __restrict__ part_o,
@@ -252,7 +257,7 @@ __global__ __launch_bounds__(256, D >= 256 ? 2 : 4) void paged_decode_kernel(
     int q_stride, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     const int* __restrict__ block_tables, int bt_stride,
     const int* __restrict__ context_lens, int Hq, int Hkv, float scale_log2e,
-    int max_parts, int blocks_per_part, DecodeRope rope) {
+    int max_parts, int blocks_per_part, int pack, DecodeRope rope) {
   constexpr int NT = D / 16;  // output d-tiles
   constexpr int KS = D / 32;  // k-steps of the QK product
   const int p = blockIdx.y;
@@ -260,7 +265,7 @@ __global__ __launch_bounds__(256, D >= 256 ? 2 : 4) void paged_decode_kernel(
   const int lane = threadIdx.x & 63;
   const int w = wave_id_uniform();
   const int b = blockIdx.x / Hkv;
-  const int h = blockIdx.x - b * Hkv;
+  int h = blockIdx.x - b * Hkv;
   const int col = lane & 15, g = lane >> 4;
   const int blk_begin = p * blocks_per_part;
   // Issue every load that does not depend on the context length first: the
@@ -268,7 +273,7 @@ __global__ __launch_bounds__(256, D >= 256 ? 2 : 4) void paged_decode_kernel(
   // row: speculative, used only if the blocks exist) and Q.  The critical
   // path becomes max(ctx, table) -> K/V instead of ctx -> table -> K/V.
   const int* bt = block_tables + (int64_t)b * bt_stride;
-  const int ph_a = bt[min(blk_begin + w, bt_stride - 1)];
+  int ph_a = bt[min(blk_begin + w, bt_stride - 1)];
   const int ph_b = bt[min(blk_begin + w + 4, bt_stride - 1)];
   bf16x8 qf[KS];  // Q^T B-operand fragments (zero for padding columns col >= G)
   const bf16_t* qrow = q + (int64_t)b * q_stride + (int64_t)(h * G + col) * D;
@@ -291,8 +296,23 @@ __global__ __launch_bounds__(256, D >= 256 ? 2 : 4) void paged_decode_kernel(
     return;
   }
   if (p >= nparts) return;
-  const bool alone = nblk == 1;  // wave 0 has it all, and nothing to merge (1024 x 20: 57 -> 47 us)
-  if (alone && w != 0) return;
+  // heads to a workgroup, waves to a head, and which of them this one is
+  const int heads = D >= 256 ? 1 : nblk == 1 ? pack : nblk == 2 ? min(pack, 2) : 1;
+  const int wph = 4 / heads, sub = heads == 1 ? w : w & (wph - 1);
+  if (heads > 1) {
+    // one workgroup of theirs has all of them: another one from sequence to sequence, since a turn of the dispatch
+    // over XCDs, their engines and CUs is a power of two long (always the first one: 1024 x 20 70 us)
+    if ((h ^ b ^ b >> 2 ^ b >> 4 ^ b >> 6) & (heads - 1)) return;
+    const int mine = (h & -heads) + w / wph;
+    if (col < G) {
+#pragma unroll
+      for (int s = 0; s < KS; ++s) qf[s] = load_bf16x8(qrow + (mine - h) * G * D + 32 * s + 8 * g);
+    }
+    h = mine;
+    ph_a = bt[min(sub, bt_stride - 1)];
+  }
+  const bool alone = nblk == 1;  // one wave has it all, and nothing to merge
+  if (alone && sub != 0) return;
 
   const int blk_end = min(nblk, blk_begin + blocks_per_part);
 
@@ -317,7 +337,7 @@ __global__ __launch_bounds__(256, D >= 256 ? 2 : 4) void paged_decode_kernel(
   // ROPE: cos | sin of the position, and for the wave that takes the step's token its k and v, through LDS ahead of
   // the cache (memory answers in order): held in registers they would cost a wave per SIMD
   [[maybe_unused]] char* const stage = reinterpret_cast<char*>(smem + 128 + 64 * D) + 1024 * w;
-  [[maybe_unused]] const bool taker = ROPE && w == 0 && p == nparts - 1;
+  [[maybe_unused]] const bool taker = ROPE && sub == 0 && p == nparts - 1;
   if constexpr (ROPE) {
     const unsigned dst = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(ad_lds_ptr)stage), at = lane * 4u;
     const __amdgpu_buffer_rsrc_t rc = dma_rsrc(rope.cos_sin + (int64_t)__builtin_amdgcn_readfirstlane(pos) * D);
@@ -330,7 +350,7 @@ __global__ __launch_bounds__(256, D >= 256 ? 2 : 4) void paged_decode_kernel(
       dma_dword_lds(dst + 256, lane < D / 2 ? at + (unsigned)(Hkv * D) * 2u : kNoRow, rq);
     }
   }
-  int blk = blk_begin + w;
+  int blk = blk_begin + sub;
   int ph_next = ph_b;  // table entry of the wave's next block, loaded one step ahead
   if (blk < blk_end) {
     load_k(ph_a, blk);
@@ -378,7 +398,7 @@ __global__ __launch_bounds__(256, D >= 256 ? 2 : 4) void paged_decode_kernel(
       }
     }
   }
-  for (; blk < blk_end; blk += 4) {
+  for (; blk < blk_end; blk += 4) {  // (heads > 1: one block to a wave)
     const int nb = blk + 4, phys = ph_next;
     ph_next = bt[min(nb + 4, bt_stride - 1)];
     vm_wait_all();  // K and V of this block have landed
@@ -452,7 +472,7 @@ __global__ __launch_bounds__(256, D >= 256 ? 2 : 4) void paged_decode_kernel(
     return;
   }
 
-  // ---- merge the 4 waves through LDS
+  // ---- merge the waves of a head through LDS
   float* sm_m = smem;              // [4][16]
   float* sm_l = smem + 64;         // [4][16]
   float* sm_o = smem + 128;        // [4][D][16]
@@ -467,6 +487,17 @@ __global__ __launch_bounds__(256, D >= 256 ? 2 : 4) void paged_decode_kernel(
       sm_o[(w * D + 16 * i + 4 * g + r) * 16 + col] = o[i][r];
   __syncthreads();
 
+  if (heads == 2) {  // two blocks: this wave's head is in waves 2 (w / 2) and the next one
+    for (int item = threadIdx.x & 127; item < G * D; item += 128) {
+      const int hh = item / D, d = item - hh * D, wa = w & 2, wb = wa + 1;
+      const float M = fmaxf(sm_m[wa * 16 + hh], sm_m[wb * 16 + hh]);
+      const float fa = fast_exp2(sm_m[wa * 16 + hh] - M), fb = fast_exp2(sm_m[wb * 16 + hh] - M);
+      const float L = sm_l[wa * 16 + hh] * fa + sm_l[wb * 16 + hh] * fb;
+      const float O = sm_o[(wa * D + d) * 16 + hh] * fa + sm_o[(wb * D + d) * 16 + hh] * fb;
+      out[((int64_t)b * Hq + h * G + hh) * D + d] = f2bf(O / L);
+    }
+    return;
+  }
   const bool single = (nparts == 1);
   for (int item = threadIdx.x; item < G * D; item += 256) {
     const int hh = item / D;
@@ -1038,6 +1069,13 @@ __global__ __launch_bounds__(256) void decode_reduce_kernel(
   }
 }
 
+// Kv heads that a workgroup of paged_decode_kernel may take where a context has few blocks: from twice the workgroups
+// that the chip holds at a time, at heads of 64 four times (256 x 20 tokens, 8 kv heads: 9.7 us, 10.5 packed).
+static int pack_heads(int items, int Hkv, int D, int max_parts) {
+  if (max_parts > 1 || items < (D < 128 ? 4096 : 2048)) return 1;
+  return Hkv % 4 == 0 ? 4 : Hkv % 2 == 0 ? 2 : 1;
+}
+
 int launch_paged_decode(void* out, float* part_o, float* part_ml, int* counters, const void* q,
                         int q_stride, const void* k_cache, const void* v_cache,
                         const int* block_tables, int bt_stride,
@@ -1107,15 +1145,16 @@ int launch_paged_decode(void* out, float* part_o, float* part_ml, int* counters,
   if (max_parts > kFusedMergeParts) counters = nullptr;
   dim3 grid(B * Hkv, max_parts), block(256);
   const size_t lds = (128 + 4 * (size_t)D * 16) * sizeof(float);
+  const int pack = pack_heads(B * Hkv, Hkv, D, max_parts);
   switch (D) {
     case 64:
-      hipLaunchKernelGGL((paged_decode_kernel<64, false>), grid, block, lds, st, (bf16_t*)out, part_o, part_ml, counters, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, bt_stride, context_lens, Hq, Hkv, sl2, max_parts, blocks_per_part, DecodeRope{});
+      hipLaunchKernelGGL((paged_decode_kernel<64, false>), grid, block, lds, st, (bf16_t*)out, part_o, part_ml, counters, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, bt_stride, context_lens, Hq, Hkv, sl2, max_parts, blocks_per_part, pack, DecodeRope{});
       break;
     case 128:
-      hipLaunchKernelGGL((paged_decode_kernel<128, false>), grid, block, lds, st, (bf16_t*)out, part_o, part_ml, counters, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, bt_stride, context_lens, Hq, Hkv, sl2, max_parts, blocks_per_part, DecodeRope{});
+      hipLaunchKernelGGL((paged_decode_kernel<128, false>), grid, block, lds, st, (bf16_t*)out, part_o, part_ml, counters, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, bt_stride, context_lens, Hq, Hkv, sl2, max_parts, blocks_per_part, pack, DecodeRope{});
       break;
     case 256:
-      hipLaunchKernelGGL((paged_decode_kernel<256, false>), grid, block, lds, st, (bf16_t*)out, part_o, part_ml, counters, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, bt_stride, context_lens, Hq, Hkv, sl2, max_parts, blocks_per_part, DecodeRope{});
+      hipLaunchKernelGGL((paged_decode_kernel<256, false>), grid, block, lds, st, (bf16_t*)out, part_o, part_ml, counters, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, bt_stride, context_lens, Hq, Hkv, sl2, max_parts, blocks_per_part, pack, DecodeRope{});
       break;
     default:
       return -1;
@@ -1164,7 +1203,8 @@ int launch_paged_decode_rope(void* out, float* part_o, float* part_ml, const voi
     const size_t lds = (128 + 4 * (size_t)D * 16) * sizeof(float) + 4096;  // and the staged rows
     (D == 64 ? paged_decode_kernel<64, true> : paged_decode_kernel<128, true>)<<<grid, pblock, lds, st>>>(
         (bf16_t*)out, part_o, part_ml, counters, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache,
-        (const bf16_t*)v_cache, block_tables, bt_stride, context_lens, Hq, Hkv, sl2, max_parts, blocks_per_part, r);
+        (const bf16_t*)v_cache, block_tables, bt_stride, context_lens, Hq, Hkv, sl2, max_parts, blocks_per_part,
+        pack_heads(B * Hkv, Hkv, D, max_parts), r);
     return (int)hipGetLastError();
   }
   switch (D) {

@@ -148,10 +148,11 @@ def decode_variant(batch: int, Hkv: int, D: int, max_blocks: int) -> int:
 def launch_variant(variant: int, max_blocks: int, max_parts: int, max_wgs: int = 0) -> int:
     """The kernel that runs where ``decode_variant`` says ``variant``: 1, since its K passes through LDS in whole rows
     and four of its workgroups fit a CU, where the others hold two blocks in registers - 32 heads over 8 kv heads, us,
-    1024 x 150 tokens 115 (3: 139), 256 x 1000 171 (206), 256 x 150 33 (41), 224 x 300 28 (39).  Left to the others: a
-    choice by hand, a grid capped by ``max_wgs``, more partitions than the merge holds, and tables of up to three
-    blocks, where not all of its four waves have work (1024 x 40: 59, 3: 52; 1024 x 20: 47, 38; 512 x 60: 37, 37; from
-    four blocks, 2048 x 90: 147, 173)."""
+    1024 x 150 tokens 115 (3: 139), 256 x 1000 171 (206), 256 x 150 33 (41), 224 x 300 28 (39).  The table says nothing
+    of the contexts in it: where they are of one or two blocks in a batch of 3, the kernel's waves take several heads to a
+    workgroup (1024 x 20: 34, 3: 37; 1024 x 40: 49, 52; 512 x 20: 20, 21; 512 x 40: 27, 30; 256 x 40: 17, 17; but 256 x 20: 14,
+    12).  Left to the others: a choice by hand, a grid capped by ``max_wgs``, more partitions than the merge holds, and
+    tables of up to three blocks, since a context of three leaves a wave without work."""
     if DECODE_VARIANT or max_wgs or max_parts > (128 if FUSED_SPLIT_MERGE else 1):
         return variant
     return variant if variant == 3 and max_blocks <= 3 else 1

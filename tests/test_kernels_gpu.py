@@ -1291,6 +1291,47 @@ def test_paged_decode_reads_no_row_past_the_context(hipk, D, Hq, Hkv, rope, bpp)
     _close(out, ops.paged_decode_ref(q, kc, vc, bt, cl, D ** -0.5), 2e-2, 2e-2, "attention")
 
 
+@pytest.mark.parametrize("D,Hq,Hkv,rope", [(128, 32, 8, True), (64, 8, 4, True), (128, 16, 2, True), (128, 24, 6, False),
+                                           (64, 16, 16, False), (128, 12, 3, True), (256, 8, 4, False)])
+def test_decode_of_short_contexts_in_full_batches(hipk, D, Hq, Hkv, rope):
+    """From 2048 (sequence, kv head) items on (heads of 64: 4096) a workgroup takes up to four kv heads of a context of one block, two of
+    two blocks: contexts of either among longer ones, NaN in every K row and whole V group behind them, every
+    cached row written; rounding of the tests above."""
+    from drtc_amd.ops import attention as attn_ops
+
+    bs, B = ops.KV_BLOCK, -(-(4096 if D == 64 else 2048) // Hkv) + 3
+    some = [1, 2, 5, 31, 32, 33, 34, 48, 0, 63, 64, 65, 97, 20, 140, 40]
+    ctx_lens = [some[(i * 5 + i // 16) % 16] for i in range(B)]
+    q, kc, vc, bt, cl = _paged_setup(B, Hq, Hkv, D, ctx_lens, seed=32)
+    kn, vn = kc.clone(), vc.clone()
+    for b, c in enumerate(ctx_lens):
+        n = c - 1 if rope else c  # rows in the cache
+        j = n // bs
+        if j < -(-c // bs):
+            blk, n = int(bt[b, j]), n - j * bs
+            kn[blk, :, n:] = float("nan")
+            vn[blk].view(Hkv, bs // 4, D, 4)[:, -(-n // 4):] = float("nan")
+    kw = dict(blocks_per_part=bt.shape[1] + 3, workspace=ops.DecodeWorkspace(B, Hq, D, 1, DEV))
+    assert attn_ops.launch_variant(attn_ops.decode_variant(B, Hkv, D, bt.shape[1]), bt.shape[1], 1) == 1
+    if not rope:
+        out = ops.paged_decode_attention(q, kn, vn, bt, cl, D ** -0.5, **kw)
+    else:
+        qkv = torch.cat([q.flatten(1), torch.randn(B, 2 * Hkv * D, device=DEV).to(torch.bfloat16)], 1)
+        pos = (cl - 1).clamp(min=0)
+        slots = torch.tensor([int(bt[b, (c - 1) // bs]) * bs + (c - 1) % bs if c else -1
+                              for b, c in enumerate(ctx_lens)], device=DEV)
+        cs = ops.build_rope_cache(512, D, 1e4, device=DEV)
+        out = ops.paged_decode_attention_rope(qkv, pos, slots, cs, Hq, Hkv, D, kn, vn, bt, cl, D ** -0.5, **kw)
+        ops.rope_kv_ref(qkv, pos, slots, cs, Hq, Hkv, D, kc, vc, bs)
+        q = qkv[:, :Hq * D].reshape(B, Hq, D)
+        live = torch.tensor([b for b, c in enumerate(ctx_lens) if c], device=DEV)
+        blk, off = slots[live] // bs, slots[live] % bs
+        _close(kn[blk, :, off], kc[blk, :, off], 1e-2, 1e-2, "rows of k")
+        assert torch.equal(vn.view(-1, Hkv, bs // 4, D, 4)[blk, :, off // 4, :, off % 4],
+                           vc.view(-1, Hkv, bs // 4, D, 4)[blk, :, off // 4, :, off % 4])
+    _close(out, ops.paged_decode_ref(q, kc, vc, bt, cl, D ** -0.5), 2e-2, 2e-2, "attention")
+
+
 def test_decode_kernel_by_table_width():
     """The kernel that runs: 1 but for a choice by hand, a capped grid, a table of up to three blocks and more
     partitions than its merge holds."""
