@@ -374,10 +374,11 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         return y
     if kind == "skinny" and (arg != STREAM or _aligned(x, w)):
         return skinny_linear(x, w, arg)
-    if kind == "midm" and (arg < 100 or _aligned(x, w)):
+    # LDS-DMA: whole 16-byte pieces, 32-bit offsets of up to 256 rows
+    if kind in ("midm", "xd") and _aligned(x, w) and x.stride(0) < 1 << 22:
+        if kind == "xd":
+            return xd_gemm(x, w, form=arg)
         return midm_gemm(x, w, "store", splits=arg % 100, nf=arg // 100 or 4)
-    if kind == "xd" and _aligned(x, w):
-        return xd_gemm(x, w, form=arg)
     return F.linear(x, w)
 
 

@@ -164,6 +164,26 @@ def test_linear_dispatches_midm_from_table(hipk):
     assert _rel(got, x.float() @ w.float().t()) < 1e-2
 
 
+@pytest.mark.parametrize("M,N,K,kind", [(24, 8192, 1024, "midm"), (64, 4096, 14336, "midm"), (48, 2048, 128, "midm"),
+                                        (64, 3584, 2048, "xd"), (24, 32000, 2048, "xd")])
+def test_linear_takes_rows_at_any_address(hipk, M, N, K, kind):
+    """Inputs and weights that start off 16 bytes, and rows too far apart for 32-bit offsets, at shapes that the table and
+    the rules send to kernels which load whole 16-byte pieces into LDS: another kernel takes them."""
+    G.reset()
+    if G.route(M, N, K, K)[0] != kind:
+        pytest.skip("no such entry for this hipBLASLt version")
+    g = torch.Generator(device="cuda").manual_seed(M)
+    flat = torch.randn(M * K + 8, device="cuda", generator=g).to(torch.bfloat16)
+    wide = torch.randn(M, K + 8, device="cuda", generator=g).to(torch.bfloat16)
+    weights = (torch.randn(N * K + 8, device="cuda", generator=g) * K ** -0.5).to(torch.bfloat16)
+    w = weights[:N * K].view(N, K)
+    far = torch.empty((M - 1 << 24) + K, dtype=torch.bfloat16, device="cuda").as_strided((M, K), (1 << 24, 1))
+    far.copy_(wide[:, :K])
+    for x, w in ((flat[3:3 + M * K].view(M, K), w), (wide[:, 4:4 + K], w), (far, w),
+                 (wide[:, :K], weights[1:1 + N * K].view(N, K))):
+        assert _rel(G.linear(x, w), x.float() @ w.float().t()) < 1e-2
+
+
 @pytest.mark.parametrize("epi", ["store", "residual", "silu"])
 @pytest.mark.parametrize("M,N,K,splitk,gm", [(1024, 4096, 4096, 4, -4), (1024, 4096, 4096, 2, -2),
                                              (512, 2048, 1024, 8, -2), (1000, 1024, 2048, 4, -1)])
