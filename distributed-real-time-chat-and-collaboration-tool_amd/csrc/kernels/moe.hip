@@ -1126,10 +1126,12 @@ int launch_moe(void* out, const void* x, const void* router_logits, const void* 
   // variants 5 / 6: 16 x 2048 x 1792, 1 token 30.5 / 46.0, 2 39.6 / 48.6; 4 61.9 / 59.1), and wide experts, gated (16 x 4096
   // x 3584, 13 tokens 226.6 / 229.1) or with a row each (20 x 4096 x 3584, 8 tokens 157.0 / 158.5; 16 197 / 187).  A
   // few of many large experts elsewhere: variant 3 (8 x 4096 x 14336, 1 token 156 / 175; 2 250 / 241)
-  const bool ring_ok = !opt.f32 && ring_moe_ok(T, P, H, I, glu), wide = H > 2048 || I > 2048;
+  // The ring loads 16-byte pieces into LDS; gemm_stream's form, into registers, takes rows at any address.
+  const bool whole = ((uintptr_t)x | (uintptr_t)w_gu | (uintptr_t)w_dn) % 16 == 0;
+  const bool ring_ok = !opt.f32 && whole && ring_moe_ok(T, P, H, I, glu), wide = H > 2048 || I > 2048;
   if (auto_v) {
     if (rows_e >= kMoeW4Rows) variant = 4;
-    else if (stream_mt == 1 && (rows_e == 0 || (wide && (glu || rows_e < 2)))) variant = 5;
+    else if (stream_mt && (!ring_ok || (stream_mt == 1 && (rows_e == 0 || (wide && (glu || rows_e < 2)))))) variant = 5;
     else if (ring_ok && rows_e <= 104 && (4 * P > e_local || (int64_t)H * I < 6 << 20)) variant = 6;
     // shapes past the ring's offsets, and sizes between it and gemm_w4
     else variant = rows_e >= 96 || (int64_t)H * I >= 6 << 20 ? 3 : 1;

@@ -474,6 +474,27 @@ def test_row_tiles_of_64(hipk, M, form, N, K):
     assert not G.xd_supported(M, N, K, form + 1) and not G.xd_supported(M, N, K, form, glu=True)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,act", [(4, "silu"), (24, "silu"), (128, "silu"), (64, "relu2")])
+def test_experts_at_any_address(hipk, T, act):
+    """Rows or weights that start off 16 bytes, at sizes that the ring of LDS pieces takes otherwise: the form that
+    streams into registers takes them, within the tolerance of the tests above."""
+    E, k, H, I = 16, 4, 2048, 1792
+    g = torch.Generator(device="cuda").manual_seed(T)
+
+    def at(off, scale, *shape):
+        n = torch.Size(shape).numel()
+        flat = torch.randn(n + 8, device="cuda", generator=g).mul_(scale).to(torch.bfloat16)
+        return flat[off:off + n].view(shape)
+
+    lg = torch.randn(T, E, device="cuda", generator=g).to(torch.bfloat16)
+    n_in = I if act == "relu2" else 2 * I
+    for ox, oi, oo in ((3, 0, 0), (0, 5, 0), (0, 0, 1), (0, 0, 0)):
+        x, w_in, w_out = at(ox, 1.0, T, H), at(oi, 0.02, E, n_in, H), at(oo, 0.02, E, H, I)
+        got, want = ops.fused_moe(x, lg, w_in, w_out, k, act).double(), ops.fused_moe_ref(x, lg, w_in, w_out, k, act).double()
+        assert (got - want).norm() <= 1e-2 * want.norm()
+
+
 def test_small_products_rule():
     """Which products the 64-row tiles take: at most a workgroup a CU of their tiles, long K on more than half of
     them."""
