@@ -1085,6 +1085,7 @@ int launch_paged_decode(void* out, float* part_o, float* part_ml, int* counters,
   if (B == 0) return 0;
   if (Hkv <= 0 || Hq % Hkv != 0 || Hq / Hkv > 16) return -1;
   if (max_parts > 1 && (!part_o || !part_ml)) return -2;
+  if (variant == 1 && (uintptr_t)k_cache % 16) variant = 2;  // K into LDS by whole 16-byte pieces
   const float sl2 = scale * kLog2e;
   if (variant == 3) {
     static int n_cu = 0;

@@ -305,7 +305,9 @@ def paged_decode_attention_rope(qkv: torch.Tensor, positions: torch.Tensor, slot
     q = qkv.as_strided((B, Hq, D), (qkv.stride(0), D, 1))
     variant = decode_variant(B, Hkv, D, block_tables.shape[1]) if on_gpu(qkv) else 0
     fused = 0
-    if on_gpu(qkv) and FUSED_ROPE:
+    # staged into LDS: a row by whole words, K by 16-byte pieces
+    whole = qkv.data_ptr() % 4 == 0 and qkv.stride(0) % 2 == 0 and k_cache.data_ptr() % 16 == 0
+    if on_gpu(qkv) and FUSED_ROPE and whole:
         max_parts = (workspace.max_parts if blocks_per_part is not None and workspace is not None
                      else decode_partitioning(B, Hkv, block_tables.shape[1], variant=variant, D=D)[1])
         fused = fused_rope_variant(variant, D, max_parts, block_tables.shape[1], max_wgs)

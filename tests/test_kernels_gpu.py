@@ -1332,6 +1332,35 @@ def test_decode_of_short_contexts_in_full_batches(hipk, D, Hq, Hkv, rope):
     _close(out, ops.paged_decode_ref(q, kc, vc, bt, cl, D ** -0.5), 2e-2, 2e-2, "attention")
 
 
+@pytest.mark.parametrize("ctx_lens", [[1, 20, 64, 0, 290], [33] * 300])
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("cache_off,row_off", [(1, 0), (4, 0), (0, 1)])
+def test_paged_decode_at_any_address(hipk, rope, ctx_lens, cache_off, row_off):
+    """Caches that start off 16 bytes and rows that start off a word: other kernels take them; rounding of the
+    tests above."""
+    B, Hq, Hkv, D, bs = len(ctx_lens), 32, 8, 128, ops.KV_BLOCK
+    q, kc, vc, bt, cl = _paged_setup(B, Hq, Hkv, D, ctx_lens, seed=33)
+
+    def at(t, off, cols=0):
+        flat = torch.empty(t.shape[0] * (t[0].numel() + cols) + 8, dtype=t.dtype, device=DEV)[off:]
+        return flat[:t.numel() + t.shape[0] * cols].view(t.shape[0], -1)[:, :t[0].numel()].copy_(t.flatten(1))
+
+    kn, vn = at(kc, cache_off).view(kc.shape), at(vc, cache_off).view(vc.shape)
+    qkv = torch.cat([q.flatten(1), torch.randn(B, 2 * Hkv * D, device=DEV).to(torch.bfloat16)], 1)
+    rows = at(qkv, row_off, row_off)
+    if not rope:
+        out = ops.paged_decode_attention(rows.as_strided((B, Hq, D), (rows.stride(0), D, 1)), kn, vn, bt, cl, D ** -0.5)
+    else:
+        pos = (cl - 1).clamp(min=0)
+        slots = torch.tensor([int(bt[b, (c - 1) // bs]) * bs + (c - 1) % bs if c else -1
+                              for b, c in enumerate(ctx_lens)], device=DEV)
+        cs = ops.build_rope_cache(512, D, 1e4, device=DEV)
+        out = ops.paged_decode_attention_rope(rows, pos, slots, cs, Hq, Hkv, D, kn, vn, bt, cl, D ** -0.5)
+        ops.rope_kv_ref(qkv, pos, slots, cs, Hq, Hkv, D, kc, vc, bs)
+        q = qkv[:, :Hq * D].reshape(B, Hq, D)
+    _close(out, ops.paged_decode_ref(q, kc, vc, bt, cl, D ** -0.5), 2e-2, 2e-2, "attention")
+
+
 def test_decode_kernel_by_table_width():
     """The kernel that runs: 1 but for a choice by hand, a capped grid, a table of up to three blocks and more
     partitions than its merge holds."""
