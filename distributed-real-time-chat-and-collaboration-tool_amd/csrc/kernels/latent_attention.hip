@@ -863,7 +863,8 @@ static void lat_decode_go(const LatentDecodeArgs& a, hipStream_t st) {
   const size_t lds = (size_t)2 * kLB * (a.LW + kLatPad) * 2;
   const dim3 grid(a.B, (a.H + 16 * NH - 1) / (16 * NH), a.nsplits), block(64 * NH * ND);
   if constexpr (RT >= 4) {
-    if (a.R == 64 * RT && a.LW == 32 * (2 * RT + 2)) {
+    // (into LDS by whole 16-byte pieces)
+    if (a.R == 64 * RT && a.LW == 32 * (2 * RT + 2) && (uintptr_t)a.cache % 16 == 0) {
       constexpr int NP = NH == 2 ? 4 : ND;  // eight waves where the heads fill two tiles
       latent_decode_pair_kernel<RT, NH, NP><<<grid, dim3(64 * NH * NP), LatPair<RT, NH, NP>::BYTES, st>>>(a);
       return;

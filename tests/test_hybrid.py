@@ -1029,6 +1029,23 @@ def test_latent_decode_in_pairs_of_blocks(H, R, parts):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H,R", [(16, 256), (32, 512), (40, 512)])
+def test_latent_decode_of_a_cache_at_any_address(H, R):
+    """Rows of whole cache lines in a cache that starts off 16 bytes: rounding of the test above."""
+    LW, nb, ctx = ops.latent_width(R, 64), 4, [1, 40, 97, 0, 128]
+    g = torch.Generator().manual_seed(R + H)
+    cache = torch.randn(len(ctx) * nb + 1, 32, LW, generator=g).mul_(0.5).to(torch.bfloat16)
+    moved = torch.empty(cache.numel() + 8, dtype=cache.dtype, device="cuda")[3:3 + cache.numel()].view(cache.shape).copy_(cache)
+    bt = torch.randperm(len(ctx) * nb, generator=g).view(len(ctx), nb).to(torch.int32) + 1
+    qa = torch.randn(len(ctx), H, LW, generator=g).mul_(0.5).to(torch.bfloat16)
+    out = ops.latent_decode_attention(qa.cuda(), moved, R, bt.cuda(), torch.tensor(ctx, dtype=torch.int32, device="cuda"),
+                                      None, 0.05, None)
+    for b, n in enumerate(ctx):
+        rows = cache[bt[b].long()].reshape(-1, LW)[:n].double()
+        close(out[b], (qa[b].double() @ rows.T * 0.05).softmax(-1) @ rows[:, :R], 2e-2)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("B,H,N,K", [(1, 3, 64, 256), (17, 2, 20, 384), (70, 4, 128, 512), (128, 2, 36, 640), (32, 4, 16, 1024)])
 def test_head_linear_with_shared_k(B, H, N, K):
     """Heads whose products a workgroup's waves share, K in 2 to 8 parts of 128: bf16 rounding of the result."""
