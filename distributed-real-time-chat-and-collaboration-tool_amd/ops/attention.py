@@ -281,7 +281,9 @@ def fused_rope_variant(variant: int, D: int, max_parts: int, max_blocks: int = 0
     if D not in (64, 128) or DECODE_VARIANT == 2:
         return 0
     variant = launch_variant(variant, max_blocks, max_parts, max_wgs)
-    return variant if variant != 2 else 1 if max_parts <= (128 if FUSED_SPLIT_MERGE else 1) else 0
+    if variant == 3:
+        return 3
+    return 1 if max_parts <= (128 if FUSED_SPLIT_MERGE else 1) else 0
 
 
 def paged_decode_attention_rope(qkv: torch.Tensor, positions: torch.Tensor, slots: torch.Tensor,

@@ -432,6 +432,24 @@ def test_backend_timeout_aborts_request():
         be.close()
 
 
+def test_fused_rope_within_the_merge(monkeypatch):
+    """The launch that rotates and merges takes no more partitions than its merge holds, also where its kernel was
+    chosen by hand, and none to merge where the merge in the kernel is switched off."""
+    from drtc_amd.ops import attention as a
+
+    assert a.decode_partitioning(1, 1, 4000, variant=1)[1] > 128
+    for by_hand in (0, 1):
+        monkeypatch.setattr(a, "DECODE_VARIANT", by_hand)
+        for variant in (1, 2):
+            assert a.fused_rope_variant(variant, 128, 128, 4000) == 1
+            assert a.fused_rope_variant(variant, 128, 129, 4000) == 0
+        monkeypatch.setattr(a, "FUSED_SPLIT_MERGE", False)
+        assert a.fused_rope_variant(1, 128, 1, 64) == 1 and a.fused_rope_variant(1, 128, 2, 64) == 0
+        monkeypatch.setattr(a, "FUSED_SPLIT_MERGE", True)
+    monkeypatch.setattr(a, "DECODE_VARIANT", 3)
+    assert a.fused_rope_variant(3, 128, 1, 64) == 3
+
+
 def test_decode_kernel_choice_per_geometry():
     """The measured decode-attention variant table (profiles/r2g, r2l) at the
     engine's decode buckets: static per graph, chosen from (batch, kv heads, D)
