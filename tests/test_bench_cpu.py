@@ -1,7 +1,9 @@
 """bench.py's driver contract on CPU (gloo): one JSON line from rank 0 with the
 whole-job value, max-over-ranks timing and DP global batch."""
+import glob
 import json
 import os
+import re
 import socket
 import subprocess
 import sys
@@ -136,3 +138,19 @@ def test_bench_self_launch_tp_ep_mixtral():
     assert r["config"]["parallelism"] == "tp4" and r["config"]["model"] == "tiny-mixtral"
     assert r["rccl_world"] == 4 and len(r["devices"]) == 4
     assert r["engine_stats"]["decode_tokens"] >= 4 * 3
+
+
+def test_scripts_call_bindings_that_exist():
+    """What the scripts and the package call on the kernel extension is bound there."""
+    package = os.path.join(ROOT, "distributed-real-time-chat-and-collaboration-tool_amd")
+    bound = set()
+    for path in glob.glob(os.path.join(package, "csrc", "kernels", "bindings*.cpp")):
+        with open(path) as f:
+            bound |= set(re.findall(r'm\.def\(\s*"(\w+)"', f.read()))
+    called = set()
+    for path in (glob.glob(os.path.join(ROOT, "scripts", "*.py")) + glob.glob(os.path.join(ROOT, "*.py"))
+                 + glob.glob(os.path.join(package, "**", "*.py"), recursive=True)):
+        with open(path) as f:
+            called |= {(os.path.basename(path), n) for n in re.findall(r"\bhipk\(\)\.(\w+)\(", f.read())}
+    assert len(bound) > 50 and len(called) > 50
+    assert not sorted(c for c in called if c[1] not in bound)
