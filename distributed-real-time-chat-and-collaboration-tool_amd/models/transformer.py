@@ -286,6 +286,8 @@ class TransformerLM:
 
     def _mlp(self, L: dict, x: ops.PendingNorm, decode: bool = False) -> torch.Tensor:
         if self.cfg.is_moe:
+            if self._moe_a2a(x.x.shape[0], decode):  # each rank routes its own rows there
+                return self._moe(L, x.materialize(), decode), False
             xn, logits = x.materialize_router(L["router"])
             return self._moe(L, xn, decode, logits), False
         if isinstance(x.x, ops.Parts):
@@ -355,6 +357,12 @@ class TransformerLM:
             self.ep_overflow.reduce(self.pc.ep_group)
         return logits
 
+    def _moe_a2a(self, T: int, decode: bool) -> bool:
+        """Whether T rows reach the EP group's experts over all-to-all, a slice from each rank."""
+        pc = self.pc
+        return (pc.ep_size > 1 and T % pc.ep_size == 0
+                and (pc.ep_combine == "a2a" if not decode else _EP_DECODE_A2A))
+
     def _moe(self, L: dict, x: torch.Tensor, decode: bool = False, logits: torch.Tensor | None = None) -> torch.Tensor:
         """Top-k routed experts (Mixtral: softmax over the top-2 logits); ``logits``: the router's, where the
         norm ahead has them already.
@@ -367,9 +375,7 @@ class TransformerLM:
         all-to-all form and all-gathered afterwards."""
         cfg, sh, pc = self.cfg, self.sh, self.pc
         T = x.shape[0]
-        a2a = (pc.ep_size > 1 and T % pc.ep_size == 0 and
-               (pc.ep_combine == "a2a" if not decode else _EP_DECODE_A2A))
-        if a2a:
+        if self._moe_a2a(T, decode):
             t = T // pc.ep_size
             rows = x[pc.ep_rank * t:(pc.ep_rank + 1) * t]
             y = self._moe_ep_a2a(L, rows, static=decode)

@@ -318,3 +318,28 @@ def test_tp_device_checks():
         check_devices([6, 8], 8, lambda a, b: True)
     with pytest.raises(RuntimeError, match="peer access"):
         check_devices([0, 1, 2], 8, lambda a, b: {a, b} != {1, 2})
+
+
+def test_norm_leaves_the_router_to_ranks_that_exchange_tokens(monkeypatch):
+    """The norm ahead of a mixture computes the router's logits only where this rank routes all of the rows: over
+    all-to-all each rank routes its own slice again."""
+    sys.path.insert(0, ROOT)
+    from drtc_amd import ops
+    from drtc_amd.models import transformer
+    from drtc_amd.models.config import TINY_MIXTRAL
+
+    model = transformer.TransformerLM(TINY_MIXTRAL, torch.device("cpu"), seed=0)
+    asked = []
+    monkeypatch.setattr(ops.PendingNorm, "materialize_router", lambda x, w: asked.append(1) or (x.materialize(), None))
+    monkeypatch.setattr(transformer.TransformerLM, "_moe", lambda self, L, x, *a: x)
+    monkeypatch.setattr(model.pc, "ep_size", 2)
+    L = model.layers[0]
+    for combine, decode_a2a, rows, decode, want in (("a2a", True, 4, False, 0), ("a2a", False, 4, False, 0),
+                                                    ("a2a", True, 4, True, 0), ("a2a", False, 4, True, 1),
+                                                    ("allreduce", True, 4, False, 1), ("a2a", True, 5, True, 1)):
+        monkeypatch.setattr(model.pc, "ep_combine", combine)
+        monkeypatch.setattr(transformer, "_EP_DECODE_A2A", decode_a2a)
+        asked.clear()
+        h = torch.randn(rows, TINY_MIXTRAL.hidden_size).to(torch.bfloat16)
+        model._mlp(L, ops.PendingNorm(h, h.clone(), L["ln_post"], 1e-5, False), decode)
+        assert len(asked) == want, (combine, decode_a2a, rows, decode)
