@@ -495,6 +495,15 @@ def test_experts_at_any_address(hipk, T, act):
         assert (got - want).norm() <= 1e-2 * want.norm()
 
 
+def test_medium_m_cuts_fill_the_chip_once():
+    """The K slices that the medium-M kernel takes by itself: one workgroup to a CU, all of whose LDS its ring takes."""
+    for M in (17, 64, 128, 129, 256):
+        for N, K in ((4096, 4096), (4096, 14336), (6144, 4096), (8192, 28672), (2048, 16384), (65536, 4096)):
+            s = G.midm_splits(M, N, K)
+            assert K % (256 * s) == 0 and (s == 1 or N // 128 * s <= 256)
+    assert G.midm_splits(64, 4096, 4096) == 8 and G.midm_splits(64, 8192, 28672) == 4
+
+
 def test_small_products_rule():
     """Which products the 64-row tiles take: at most a workgroup a CU of their tiles, long K on more than half of
     them."""
