@@ -2,7 +2,7 @@
 """Measure the medium-M decode GEMM (csrc/kernels/gemm_midm.hip) against the
 engine's current path (ops.linear: tuned hipBLASLt / F.linear) for every decode
 projection of a model at the decode buckets 17..256, and write a tuning entry
-{"midm": S} (K splits) where the hand kernel wins by at least --min-gain.
+{"midm": cut} (100 x fragments + K slices) where the hand kernel wins by at least --min-gain.
 
 W is rotated over copies (>= 512 MB in all) so it streams from HBM, as in a
 decode step, not from the 256 MB Infinity Cache; arms are interleaved.
@@ -74,17 +74,17 @@ def main() -> None:
                 lib = time_arm(lambda w: G.linear(x, w), ws)
                 ref = x.float() @ ws[0].float().t()
                 best = None
-                ring = 64 * G.midm_depth(M)
-                for S in range(1, 17):
-                    if K % (ring * S) or S * M * N * 4 > G.WS_SLAB_BYTES or (N // 128) * S > 1024:
-                        continue
-                    y = G.midm_gemm(x, ws[0], splits=S)
+                # cuts: 100 x fragments + K slices (4 fragments: the slices alone), a workgroup to a CU at most
+                cuts = [S if nf == 4 else 100 * nf + S for nf in (2, 4) for S in range(1, 17)
+                        if N // (32 * nf) * S <= 256 and K // 64 // S >= 3 and S * M * N * 4 <= G.WS_SLAB_BYTES]
+                for S in cuts:
+                    y = G.midm_gemm(x, ws[0], splits=S % 100, nf=S // 100 or 4)
                     err = ((y.float() - ref).abs().max() / ref.abs().max()).item()
                     if err > 2e-2:
                         print(json.dumps({"model": model, "tp": tp, "gemm": name, "M": M,
                                           "S": S, "err": err, "FAILED": True}), flush=True)
                         continue
-                    us = time_arm(lambda w, S=S: G.midm_gemm(x, w, splits=S), ws)
+                    us = time_arm(lambda w, S=S: G.midm_gemm(x, w, splits=S % 100, nf=S // 100 or 4), ws)
                     if best is None or us < best[1]:
                         best = (S, us)
                 rec = {"model": model, "tp": int(tp), "gemm": name, "M": M, "N": N, "K": K,

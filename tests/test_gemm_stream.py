@@ -504,6 +504,25 @@ def test_medium_m_cuts_fill_the_chip_once():
     assert G.midm_splits(64, 4096, 4096) == 8 and G.midm_splits(64, 8192, 28672) == 4
 
 
+def test_medium_m_entries_decide():
+    """The tuning table's medium-M cuts: shapes that no rule ahead of the table takes, at most a workgroup to a CU,
+    whole K tiles to a slice, faster than what the table has otherwise."""
+    seen = 0
+    for entries in G.load_table().values():
+        for key, e in entries.items():
+            cut = e.get("midm")
+            if not cut:
+                continue
+            M, N, K, ldx = (int(v) for v in key.split(","))
+            nf, s = cut // 100 or 4, cut % 100
+            assert G.midm_supported(M, N, K) and N % (32 * nf) == 0 and nf in (2, 4) and 1 <= s <= K // 64
+            assert N // (32 * nf) * s <= 256, key
+            assert not (G.wide_form(M, N, K) or G.small_form(M, N, K) or G.brief_ok(M, N, K) or e.get("xd")), key
+            assert e["midm_us"] < e["midm_base_us"]
+            seen += 1
+    assert seen
+
+
 def test_small_products_rule():
     """Which products the 64-row tiles take: at most a workgroup a CU of their tiles, long K on more than half of
     them."""
