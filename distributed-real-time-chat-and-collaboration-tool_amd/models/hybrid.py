@@ -382,6 +382,7 @@ class HybridLM:
         linear = ops.linear_parts if isinstance(self.final, Dyt) else ops.linear  # (every norm is of one kind)
         for i, (l, L) in enumerate(zip(cfg.layers, self.layers)):
             x = self._enter(L["norm1"], h, y, by, ids=ids if i == 0 else None)
+            y = None  # K slices' sums live until the norm has read them
             a = mix(i, L["mixer"], x)
             if i == last and rows is not None:
                 a, h = a.index_select(0, rows), h.index_select(0, rows)
@@ -391,6 +392,7 @@ class HybridLM:
                 y, by = self._experts(L, l, x), L["add2"]
             elif l.ff:
                 x = self._enter(L["norm2"], h, y, by)
+                y = None
                 y = linear(ops.gated(x, L["gate_up"], cfg.act, l.limit), L["down"])
                 by = L.get("add2")
         return ops.linear(self._enter(self.final, h, y, by), self.lm_head)

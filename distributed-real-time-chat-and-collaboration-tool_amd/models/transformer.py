@@ -442,6 +442,7 @@ class TransformerLM:
             o, added, *part = attn_fn(i, L, x)
             x = ops.PendingNorm(o, None if added else x.stream(), L["ln_post"], cfg.rms_eps,
                                 cfg.gemma_norm, pc=self.pc if part and part[0] else None)
+            del o  # K slices' sums live until the norm has read them, not until the next ones
             nxt = self.layers[i + 1]["ln_in"] if i + 1 < n else self.final_norm
             if cfg.is_moe and self._moe_norm_ok(x):
                 x = self._moe_norm(L, x, nxt)
@@ -449,6 +450,7 @@ class TransformerLM:
             m, added, *part = self._mlp(L, x, decode)
             x = ops.PendingNorm(m, None if added else x.stream(), nxt, cfg.rms_eps, cfg.gemma_norm,
                                 pc=self.pc if part and part[0] else None)
+            del m
         return x
 
     def _logits(self, x: torch.Tensor | ops.PendingNorm) -> torch.Tensor:
@@ -701,6 +703,7 @@ class TransformerLM:
                     mo, added, *_ = self._mlp(L, x, decode=True)
                     xs[j] = ops.PendingNorm(mo, None if added else x.stream(), nxt, cfg.rms_eps,
                                             cfg.gemma_norm)
+                    del mo
         finals = []
         for j in (0, 1):
             with torch.cuda.stream(streams[j]), ops.gemm.private_workspace(wss[j]):

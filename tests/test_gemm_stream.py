@@ -441,6 +441,39 @@ def test_product_parts(hipk, M, N, K, form):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("family", ["llama", "ralesun"])
+def test_slices_sums_live_until_their_norm(hipk, monkeypatch, family):
+    """A layer stack holds the sums of one product's K slices at a time."""
+    import weakref
+
+    from drtc_amd.engine import LLMEngine, Request
+    from drtc_amd.models import build_model
+    from drtc_amd.models.config import HybridConfig, LatentAttention, Layer, ModelConfig
+
+    if family == "llama":
+        cfg = ModelConfig("three layers", 512, 2048, 7168, 3, 16, 4, 128)
+    else:
+        att = LatentAttention(16, 128, 64, 128, 512, 192 ** -0.5, 1024, 500000.0, 64)
+        cfg = HybridConfig("three layers", 512, 2048, (Layer(att, 7168),) * 3, norm_eps=1e-5)
+    real, live, seen = G.linear_parts, [], []
+
+    def watch(x, w):
+        assert not [r for r in live if r() is not None]
+        y = real(x, w)
+        if isinstance(y, ops.Parts):
+            live.append(weakref.ref(y.slab))
+            seen.append(y.shape)
+        return y
+
+    eng = LLMEngine(build_model(cfg, "cuda", seed=1), max_batch=4, max_model_len=128, num_blocks=16)
+    monkeypatch.setattr(ops, "linear_parts", watch)
+    monkeypatch.setattr(G, "linear_parts", watch)
+    eng.feed([(Request([]), list(range(3, 51)), [47])])
+    torch.cuda.synchronize()
+    assert len(seen) >= 4
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(17, 1024, 64), (64, 4096, 256), (128, 1088, 256), (170, 2048, 192), (256, 2048, 128)])
 def test_short_k_products(hipk, M, N, K):
     """Products of one to four K tiles, fewer than the ring has stages, as linear routes them; rows of a wider
