@@ -36,6 +36,7 @@ projections with the residual add in their epilogue do not go through ``linear``
 """
 from __future__ import annotations
 
+import functools
 import json
 import math
 import os
@@ -1147,6 +1148,7 @@ def xd_supported(M: int, N: int, K: int, form: int, glu: bool = False) -> bool:
                        and 2 * tiles + 2 <= WS_COUNTERS)  # + the fault word (last counter)
 
 
+@functools.lru_cache(maxsize=4096)
 def xd_default_form(M: int, N: int, K: int, glu: bool = False) -> int:
     """Form of an untuned shape, by a per-CU operand-bytes model (profiles/r4i): a CU's
     time ~ (tile rows + columns) x (K / splitk) x 2 B per round of 256 work items, plus the
@@ -1315,6 +1317,8 @@ def parts_form(M: int, N: int, K: int) -> tuple[int, int] | None:
 
 def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | Parts:
     """``linear``, or its K slices' sums (csrc/kernels/gemm_midm.hip) where ``parts_form`` says so."""
+    if x.shape[0] > MIDM_MAX_M:  # (a prompt's host path is as long as its kernels up to some 600 rows)
+        return linear(x, w)
     if _gpu_bf16(x, w) and w.shape[1] == x.shape[1] and _aligned(x, w):
         (M, K), N = x.shape, w.shape[0]
         form = parts_form(M, N, K) if M * x.stride(0) < 1 << 30 else None

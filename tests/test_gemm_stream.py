@@ -556,6 +556,22 @@ def test_medium_m_entries_decide():
     assert seen
 
 
+def test_prompts_ask_once(monkeypatch):
+    """What a prompt's products ask for on the host: no K slices above the rows that they take, and a shape's tile once."""
+    asked = []
+    real = G._gpu_bf16
+    monkeypatch.setattr(G, "_gpu_bf16", lambda x, w: asked.append(x.shape[0]) or real(x, w))
+    w = torch.randn(64, 128)
+    for rows in (G.MIDM_MAX_M + 1, 1000):
+        x = torch.randn(rows, 128)
+        assert torch.equal(ops.linear_parts(x, w), ops.linear(x, w))
+    assert len(asked) == 4
+    supported = G.xd_supported
+    monkeypatch.setattr(G, "xd_supported", lambda *a: asked.append(a) or supported(*a))
+    first, n = G.xd_default_form(397, 2048, 2048, True), len(asked)
+    assert n > 4 and G.xd_default_form(397, 2048, 2048, True) == first and len(asked) == n
+
+
 def test_small_products_rule():
     """Which products the 64-row tiles take: at most a workgroup a CU of their tiles, long K on more than half of
     them."""
