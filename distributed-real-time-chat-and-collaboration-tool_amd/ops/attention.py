@@ -122,7 +122,8 @@ DECODE_VARIANT = int(os.environ.get("DRTC_DECODE_VARIANT", "0"))
 
 
 def decode_variant(batch: int, Hkv: int, D: int, max_blocks: int) -> int:
-    """Kernel variant per decode shape (profiles/r2g_decode_persistent.md):
+    """Shape class of a decode step, named by the kernel that was the faster one for it before ``launch_variant``,
+    which picks the kernel that runs; ``decode_partitioning`` cuts contexts by it (profiles/r2g_decode_persistent.md):
     3 (persistent waves, next item prefetched) when there are >= 4096
     (sequence, kv head) items and D <= 128 - the serving batches (B 1024 x 8
     kv heads: 141 vs 150 us); 2 (wave per item) when the context must be
@@ -132,7 +133,7 @@ def decode_variant(batch: int, Hkv: int, D: int, max_blocks: int) -> int:
     r2l (profiles/r2l_decode_geometries.md): from 2048 items v3 also wins at
     chat lengths (Mixtral / 70B heads at B 256: 38.4 vs 40.1 / 38.9 vs 41.2 us);
     at D = 256 (Gemma-2B, one kv head) v2 wins from 1024 items (B 1024: 34.2 vs
-    49.5 us; v3 holds ~400 registers there and spills)."""
+    49.5 us; v3 holds ~400 registers there and spills).  All figures: from before kernel 1 took K through LDS."""
     if DECODE_VARIANT:
         return DECODE_VARIANT
     items = batch * Hkv
@@ -147,11 +148,18 @@ def decode_variant(batch: int, Hkv: int, D: int, max_blocks: int) -> int:
 
 def launch_variant(variant: int, max_blocks: int, max_parts: int, max_wgs: int = 0) -> int:
     """The kernel that runs where ``decode_variant`` says ``variant``: 1, since its K passes through LDS in whole rows
-    and four of its workgroups fit a CU, where the others hold two blocks in registers - 32 heads over 8 kv heads, us,
-    1024 x 150 tokens 115 (3: 139), 256 x 1000 171 (206), 256 x 150 33 (41), 224 x 300 28 (39).  The table says nothing
-    of the contexts in it: where they are of one or two blocks in a batch of 3, the kernel's waves take several heads to a
-    workgroup (1024 x 20: 34, 3: 37; 1024 x 40: 49, 52; 512 x 20: 20, 21; 512 x 40: 27, 30; 256 x 40: 17, 17; but 256 x 20: 14,
-    12).  Left to the others: a choice by hand, a grid capped by ``max_wgs``, more partitions than the merge holds, and
+    and four of its workgroups fit a CU (two at heads of 256, for their LDS), where the others hold two blocks in
+    registers.  us:
+      32 heads of 128 over 8 kv heads, 3 / 1: 1024 x 150 tokens 139 / 115, 256 x 1000 206 / 171, 256 x 150 41 / 33, 224 x 300
+        39 / 28
+      32 heads of 64 over 8, 3 / 1: 256 x 150 21.6 / 20.3, 1024 x 90 52 / 48.5, 1024 x 150 76 / 69, 1024 x 500 200 / 184
+      8 heads of 256 over 1, contexts of three to five quarters of the mean, rotation apart, 2 / 1: 1024 x 60 27.4 / 26.1,
+        1024 x 150 44.8 / 41.5, 1024 x 400 99.8 / 80.5, 2048 x 150 82 / 72; 1024 x 20 14.6 / 15.7, and 1024 equal contexts, all of
+        whose waves end together, x 150 33.7 / 37.6, x 500 102 / 91
+    The table says nothing of the contexts in it: where they are of one or two blocks in a batch of 3, the kernel's waves
+    take several heads to a workgroup (3 / 1: 1024 x 20 37 / 34, 1024 x 40 52 / 49, 512 x 20 21 / 20, 512 x 40 30 / 27, 256 x 40
+    17 / 17; but 256 x 20 12 / 14).
+    Left to the others: a choice by hand, a grid capped by ``max_wgs``, more partitions than the merge holds, and
     tables of up to three blocks, since a context of three leaves a wave without work."""
     if DECODE_VARIANT or max_wgs or max_parts > (128 if FUSED_SPLIT_MERGE else 1):
         return variant
