@@ -27,8 +27,6 @@
 #include "launchers.h"
 #include "lds_dma.h"
 
-typedef __attribute__((address_space(3))) void* ad_lds_ptr;
-
 namespace {
 // s_waitcnt vmcnt(0): every vector-memory load of this wave has landed.  Used right after the
 // first K/V block of a register double-buffered block loop is issued (see the persistent
@@ -325,7 +323,7 @@ __global__ __launch_bounds__(256, D >= 256 ? 2 : 4) void paged_decode_kernel(
   // [4][16] m, [4][16] l, then each wave's K block, later its sums [D][16]
   extern __shared__ __attribute__((aligned(16))) float smem[];
   char* const klds = reinterpret_cast<char*>(smem + 128) + w * (D * 64);
-  const unsigned kdst = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(ad_lds_ptr)klds);
+  const unsigned kdst = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(lds_ptr)klds);
   VRegs<D> v;
   auto load_k = [&](int phys, int blk) {
     KLds<D>::load(kdst, k_cache + ((int64_t)__builtin_amdgcn_readfirstlane(phys) * Hkv + h) * blk_elems, lane,
@@ -339,7 +337,7 @@ __global__ __launch_bounds__(256, D >= 256 ? 2 : 4) void paged_decode_kernel(
   [[maybe_unused]] char* const stage = reinterpret_cast<char*>(smem + 128 + 64 * D) + 1024 * w;
   [[maybe_unused]] const bool taker = ROPE && sub == 0 && p == nparts - 1;
   if constexpr (ROPE) {
-    const unsigned dst = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(ad_lds_ptr)stage), at = lane * 4u;
+    const unsigned dst = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(lds_ptr)stage), at = lane * 4u;
     const __amdgpu_buffer_rsrc_t rc = dma_rsrc(rope.cos_sin + (int64_t)__builtin_amdgcn_readfirstlane(pos) * D);
 #pragma unroll
     for (int i = 0; i < D / 64; ++i) dma_dword_lds(dst + 512 + 256 * i, at + 256u * i, rc);
@@ -829,7 +827,7 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void paged_decode_persist_ke
   __shared__ __attribute__((aligned(16))) char rope_lds[STAGE ? 4 * 1024 : 16];
   char* const slot_lds = rope_lds + (STAGE ? 1024 * wave_id_uniform() : 0);
   const unsigned slot_dst =
-      __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(ad_lds_ptr)slot_lds);
+      __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(lds_ptr)slot_lds);
   const __amdgpu_buffer_rsrc_t rsrc_q =
       __builtin_amdgcn_make_buffer_rsrc((void*)q, (short)0, 0x7FFFFFFF, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsrc_cs = __builtin_amdgcn_make_buffer_rsrc(

@@ -46,14 +46,13 @@
 //     2) of the SAME 8 NF output columns, so the gate value meets its up value in a lane.
 #include "common.h"
 #include "launchers.h"
+#include "lds_dma.h"
 
 #include <cstdlib>
 #include <utility>
 
 namespace drtc {
 namespace {
-
-typedef __attribute__((address_space(3))) void* xd_lds_ptr;
 
 constexpr int kXdThreads = 256;
 enum { XD_STORE = 0, XD_RESIDUAL = 1, XD_SILU = 2, XD_GELU = 3, XD_CLAMP = 4, XD_RELU2 = 5 };
@@ -131,35 +130,9 @@ DRTC_DEVICE void xd_barrier() {
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 }
-template <int N>
-DRTC_DEVICE void xd_vmcnt() {
-  constexpr int imm = (N & 0xF) | (0x7 << 4) | (0xF << 8) | ((N >> 4) << 14);
-  __builtin_amdgcn_s_waitcnt(imm);
-}
 DRTC_DEVICE void xd_lgkm0() { __builtin_amdgcn_s_waitcnt(0xC07F); }
 DRTC_DEVICE bf16x8 xd_rd(const char* lds, int off) {
   return *reinterpret_cast<const bf16x8*>(lds + off);
-}
-
-// One LDS-DMA wave-instruction outside the main loop: M0 saved and restored.  NT: the
-// non-temporal policy (a weight byte that one CU reads once, MI355X_MICROARCH.md nt-weights).
-template <bool NT = false>
-DRTC_DEVICE void xd_dma(unsigned dst, unsigned voff, __amdgpu_buffer_rsrc_t rsrc, unsigned soff) {
-  unsigned keep;
-  if constexpr (NT)
-    asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\t"
-        "buffer_load_dwordx4 %2, %3, %4 offen nt lds\n\ts_mov_b32 m0, %0"
-        : "=&s"(keep)
-        : "s"(dst), "v"(voff), "s"(rsrc), "s"(soff)
-        : "memory");
-  else
-    asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\t"
-        "buffer_load_dwordx4 %2, %3, %4 offen lds\n\ts_mov_b32 m0, %0"
-        : "=&s"(keep)
-        : "s"(dst), "v"(voff), "s"(rsrc), "s"(soff)
-        : "memory");
 }
 
 // Fragment r of a K half in consumption order (A row block 0, every B column block, then the
@@ -237,7 +210,7 @@ DRTC_DEVICE void xd_step(f32x4 (&acc)[C::FA][C::NF], bf16x8 (&fa0)[C::FA], bf16x
     xd_read<C, Q - 1>(fa1, fb1, lds, cur, f.ra1, f.rb1);
   // ---- boundary: tile t + 1 landed for every wave; every read of this stage is done
   if constexpr (NEXT && Q == H - 1) {
-    xd_vmcnt<WT * C::D>();  // WT younger K tiles of this wave may still be in flight
+    wait_vm<WT * C::D>();  // WT younger K tiles of this wave may still be in flight
     xd_lgkm0();
     xd_barrier();
   }
@@ -440,7 +413,7 @@ __global__ __launch_bounds__(kXdThreads, 1) void gemm_xd_kernel(XdParams p) {
   // (A) / 8 NF wv + 8 i + (lane >> 3) (B), lane's LDS chunk lane & 7 <- source chunk ^
   // swizzle.  A rows past M read row M - 1 (valid bytes, never stored).
   XdDma<C> d;
-  const unsigned lds0 = (unsigned)(uintptr_t)(xd_lds_ptr)xd_lds;
+  const unsigned lds0 = (unsigned)(uintptr_t)(lds_ptr)xd_lds;
   {
     const bool gather = G && p.g_aidx != nullptr;
     const char* abase =
@@ -502,12 +475,12 @@ __global__ __launch_bounds__(kXdThreads, 1) void gemm_xd_kernel(XdParams p) {
     const unsigned k = next_k();
 #pragma unroll
     for (int i = 0; i < C::DA; ++i)
-      xd_dma(d.lds_a + u * C::STAGE + 1024 * i, d.va[i], d.ra, k);
+      dma16<false>(d.lds_a + u * C::STAGE + 1024 * i, d.va[i], d.ra, k);
 #pragma unroll
     for (int i = 0; i < C::DB; ++i)
-      xd_dma<C::NT>(d.lds_b + u * C::STAGE + 1024 * i, d.vb[i], d.rb, k);
+      dma16<C::NT>(d.lds_b + u * C::STAGE + 1024 * i, d.vb[i], d.rb, k);
   }
-  xd_vmcnt<(C::S - 1) * C::D>();
+  wait_vm<(C::S - 1) * C::D>();
   xd_barrier();
   bf16x8 fa0[FA], fb0[NF], fa1[FA], fb1[NF];
   xd_reads<C, 0, C::NR>(fa0, fb0, lds, 0, f.ra0, f.rb0);
@@ -523,7 +496,7 @@ __global__ __launch_bounds__(kXdThreads, 1) void gemm_xd_kernel(XdParams p) {
     cur = nxt;
   }
   xd_tail<C, C::S - 2>(acc, fa0, fb0, fa1, fb1, lds, cur, f, d);
-  xd_vmcnt<0>();
+  wait_vm<0>();
 
   bool part = false;   // split-K: this workgroup adds the other slices' partials
   bool rearm = false;  // ... and re-arms the tile's counters (not after a fault)
