@@ -247,7 +247,7 @@ def _resolve(M: int, N: int, K: int, ldx: int) -> tuple[str, int]:
     small = small_form(M, N, K)
     if small and ldx % 8 == 0:
         return ("xd", small)
-    if brief_ok(M, N, K) and ldx % 8 == 0:
+    if brief_ok(M, N, K) and ldx % 8 == 0 and brief_pays(M, N, K, found is not None and found[1][0] >= 0):
         return ("midm", 201)
     # the rule goes ahead of the table, but for entries that were measured faster ("stream": 0)
     if ldx % 8 == 0 and stream_ok(M, N, K) and (found is None or (found[0], N, K, ldx) not in _kept):
@@ -304,11 +304,19 @@ def dot2_ok(M: int, N: int, K: int, ldx: int) -> bool:
 
 
 def brief_ok(M: int, N: int, K: int) -> bool:
-    """Whether a product of a few K tiles takes gemm_midm in one slice and 64 columns to a workgroup: all of it is
-    launch, one round trip and the store.  us, the table's pick / this: 2048 x 128, 48 rows 6.6 / 3.8, 128 6.6 / 4.9, 256 7.1 /
-    6.8; 4096 x 256, 48 rows 6.4 / 4.4, 128 5.7 / 5.6, 200 6.4 / 7.1; 16 rows 2.6 / 3.5."""
+    """Whether gemm_midm takes a product of a few K tiles in one slice and 64 columns to a workgroup: all of it is
+    launch, one round trip and the store."""
     return (_midm_enabled and _enabled and K % 64 == 0 and K <= 256 and 17 <= M <= 256 and M * K <= 32768
             and N % 64 == 0 and 1024 <= N <= 8192)
+
+
+def brief_pays(M: int, N: int, K: int, listed: bool) -> bool:
+    """... and is the faster kernel for it, against the library's pick or (``listed``) the table's.  us, the pick /
+    this: 1024 x 64, 17 rows 3.5 / 2.9, 64 3.6 / 3.3; 2560 x 128, 17 rows 4.0 / 3.2, 64 4.2 / 3.8, 80 4.0 / 4.2, 112 4.4 / 4.7;
+    5120 x 256, 64 rows 5.4 / 4.7, 112 5.7 / 5.9, 128 6.2 / 6.1; 3072 x 192, 72 rows 0.92 of it, 128 0.94.  It reads all rows in
+    every workgroup, so many of them lose: 1024 x 128, 160 rows 3.7 / 4.9, 256 3.7 / 6.5.  The table's, 2048 x 128: 48 rows 6.2 /
+    3.5, 128 6.3 / 4.6, 200 7.0 / 5.8, 256 6.8 / 6.4; 4096 x 256, 48 rows 6.5 / 4.5, 128 5.9 / 6.0."""
+    return M <= 64 or M <= 128 and N * K >= 3072 * 192 or listed
 
 
 def wide_form(M: int, N: int, K: int) -> int:

@@ -572,6 +572,16 @@ def test_prompts_ask_once(monkeypatch):
     assert n > 4 and G.xd_default_form(397, 2048, 2048, True) == first and len(asked) == n
 
 
+def test_short_k_rule():
+    """Short K stays with the library's pick where many rows lose: above 64, wide products 128, but for shapes
+    whose tuned solution is slower."""
+    for M, N, K in ((17, 1024, 64), (64, 1024, 256), (64, 8192, 64), (112, 6144, 128), (128, 3072, 192), (128, 8192, 256)):
+        assert G.brief_ok(M, N, K) and G.brief_pays(M, N, K, False) and G._resolve(M, N, K, K) == ("midm", 201)
+    for M, N, K in ((65, 1024, 128), (128, 1024, 256), (112, 2048, 192), (160, 4096, 192), (200, 8192, 128), (256, 1536, 128)):
+        assert G.brief_ok(M, N, K) and not G.brief_pays(M, N, K, False) and G.brief_pays(M, N, K, True)
+        assert G._resolve(M, N, K, K) == ("torch", 0)  # (no such shape in the table)
+
+
 def test_small_products_rule():
     """Which products the 64-row tiles take: at most a workgroup a CU of their tiles, long K on more than half of
     them."""
