@@ -205,6 +205,7 @@ PYBIND11_MODULE(_hipk, m) {
                                     slices, P<void>(slab), slab_bytes, P<void>(tickets), n_tickets, S(st));
   });
   m.def("stream_moe_tiles", &drtc::stream_moe_tiles);  // (rows per expert, H, I, gated)
+  m.def("moe_variant", &drtc::moe_variant);  // (T, pairs, experts, H, I, gated, 16-byte pieces)
   m.def("midm_gemm", [](u64 y, u64 x, u64 w, u64 res, int M, int N, int K, int ldx, int ldy,
                         int ldr, int epi, int splits, int nf, u64 slab, int64_t slab_bytes, u64 st) {
     return drtc::launch_midm_gemm(P<void>(y), P<const void>(x), P<const void>(w),

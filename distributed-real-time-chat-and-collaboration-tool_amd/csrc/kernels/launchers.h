@@ -93,6 +93,7 @@ struct MoeOptions {
 // workspace of the gemm_xd forms (may be null: no split-K); 4: rows gathered into expert order,
 // then gemm_w4's grouped persistent form (prefill-sized rows per expert); -1: by rows per
 // expert
+int moe_variant(int T, int P, int E, int H, int I, bool glu, bool whole);  // of -1, bf16
 int launch_moe(void* out, const void* x, const void* router_logits, const void* w_gu,
                const void* w_dn, int T, int H, int I, int E, int k, int e_off, int e_local,
                int act, void* workspace, int64_t ws_bytes, int variant, int gu_form, int dn_form,

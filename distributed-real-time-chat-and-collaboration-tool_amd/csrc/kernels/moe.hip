@@ -1083,6 +1083,29 @@ static void moe_xd_form(int form, int& mt, int& nf, int& sk) {
   sk = form % 10;
 }
 
+// The variant of a layer of T tokens and P pairs over E experts, bf16; whole: rows and weights start at 16 bytes.
+//   * 4 from one 256-row tile per expert (gemm_w4's persistent 256 x 256 tiles over
+//     expert-ordered rows; Mixtral shapes, profiles/r6j: 770 / 917 / 1061 TF/s at T = 1024 /
+//     2048 / 4096 against 703 / 841 / 1019 on variant 3).
+//   * below it the ring, to where most experts still fit one of its entries (100 rows 92 / 121 of variant 3, 128
+//     rows 134 / 123), but for a few rows per expert where gemm_stream's form takes the sizes: fewer pairs than experts (us of a layer,
+//     variants 5 / 6: 16 x 2048 x 1792, 1 token 30.5 / 46.0, 2 39.6 / 48.6; 4 61.9 / 59.1), and wide experts, gated (16 x 4096
+//     x 3584, 13 tokens 226.6 / 229.1) or with a row each (20 x 4096 x 3584, 8 tokens 157.0 / 158.5; 16 197 / 187).  (wide:
+//     of the four widths that gemm_stream's form has, the upper two.)  Elsewhere a few pairs of large experts: variant 3,
+//     to seven of them and a pair an expert (3 / 6: 8 x 4096 x 14336, 2 per token, 1 token 152 / 176, 2 241 / 244, 4 364 / 328;
+//     4 x 2048 x 5632, 1 58.6 / 74.3, 2 80.7 / 76.2, 3 90.9 / 80.0; 12 x 1536 x 4096, 2 49.6 / 61.8, 3 71.4 / 68.4, 4 77.5 / 78.0; 16 x
+//     3072 x 2560, 3 63.5 / 70.0, 4 102 / 77; 64 x 2560 x 2816, 2 71.1 / 78.7, 4 99.3 / 86.9, 16 245 / 207)
+//     The ring loads 16-byte pieces into LDS; gemm_stream's form, into registers, takes rows at any address.
+int moe_variant(int T, int P, int E, int H, int I, bool glu, bool whole) {
+  const int rows_e = P / E, stream_mt = stream_moe_tiles(rows_e, H, I, glu);
+  const bool ring_ok = whole && ring_moe_ok(T, P, H, I, glu), wide = H > 2048 || I > 2048;
+  if (rows_e >= kMoeW4Rows) return 4;
+  if (stream_mt && (!ring_ok || (stream_mt == 1 && (rows_e == 0 || (wide && (glu || rows_e < 2)))))) return 5;
+  if (ring_ok && rows_e <= 104 && (P >= 8 || P > E || (int64_t)H * I < 6 << 20)) return 6;
+  // shapes past the ring's offsets, and sizes between it and gemm_w4
+  return rows_e >= 96 || (int64_t)H * I >= 6 << 20 ? 3 : 1;
+}
+
 int launch_moe(void* out, const void* x, const void* router_logits, const void* w_gu,
                const void* w_dn, int T, int H, int I, int E, int k, int e_off, int e_local,
                int act, void* workspace, int64_t ws_bytes, int variant, int gu_form, int dn_form,
@@ -1117,25 +1140,10 @@ int launch_moe(void* out, const void* x, const void* router_logits, const void* 
   // -1 = pick by rows per expert (scripts/moe_bench.py, Mixtral shapes)
   const int rows_e = P / e_local;
   const bool auto_v = variant < 0;
-  // variant 4 from one 256-row tile per expert (gemm_w4's persistent 256 x 256 tiles over
-  // expert-ordered rows; Mixtral shapes, profiles/r6j: 770 / 917 / 1061 TF/s at T = 1024 /
-  // 2048 / 4096 against 703 / 841 / 1019 on variant 3)
   const int stream_mt = opt.f32 ? 0 : stream_moe_tiles(rows_e, H, I, glu);
-  // ... below it the ring, to where most experts still fit one of its entries (100 rows 92 / 121 of variant 3, 128
-  // rows 134 / 123), but for a few rows per expert where gemm_stream's form takes the sizes: fewer pairs than experts (us of a layer,
-  // variants 5 / 6: 16 x 2048 x 1792, 1 token 30.5 / 46.0, 2 39.6 / 48.6; 4 61.9 / 59.1), and wide experts, gated (16 x 4096
-  // x 3584, 13 tokens 226.6 / 229.1) or with a row each (20 x 4096 x 3584, 8 tokens 157.0 / 158.5; 16 197 / 187).  A
-  // few of many large experts elsewhere: variant 3 (8 x 4096 x 14336, 1 token 156 / 175; 2 250 / 241)
-  // The ring loads 16-byte pieces into LDS; gemm_stream's form, into registers, takes rows at any address.
   const bool whole = ((uintptr_t)x | (uintptr_t)w_gu | (uintptr_t)w_dn) % 16 == 0;
-  const bool ring_ok = !opt.f32 && whole && ring_moe_ok(T, P, H, I, glu), wide = H > 2048 || I > 2048;
-  if (auto_v) {
-    if (rows_e >= kMoeW4Rows) variant = 4;
-    else if (stream_mt && (!ring_ok || (stream_mt == 1 && (rows_e == 0 || (wide && (glu || rows_e < 2)))))) variant = 5;
-    else if (ring_ok && rows_e <= 104 && (4 * P > e_local || (int64_t)H * I < 6 << 20)) variant = 6;
-    // shapes past the ring's offsets, and sizes between it and gemm_w4
-    else variant = rows_e >= 96 || (int64_t)H * I >= 6 << 20 ? 3 : 1;
-  }
+  if (auto_v) variant = moe_variant(T, P, e_local, H, I, glu, whole);
+  const bool ring_ok = !opt.f32 && whole && ring_moe_ok(T, P, H, I, glu);
   if (variant > 6 || (variant == 5 && !stream_mt) || (variant == 6 && !ring_ok)) return -1;
   // variant 4: the persistent GEMM's prologue stages two K tiles; the down reduction is I
   if (variant == 4 && (H / 64 < 2 || I % (glu ? 128 : 256) || I / 64 < 2 || H % 256)) {

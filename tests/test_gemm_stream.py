@@ -508,6 +508,20 @@ def test_row_tiles_of_64(hipk, M, form, N, K):
 
 
 @pytest.mark.gpu
+def test_variants_by_pairs(hipk):
+    """A few pairs of large experts are gemm_xd's, from eight on or more than one an expert the ring's, as are small
+    experts; few rows an expert of gemm_stream's widths its form; nothing off 16 bytes the ring's."""
+    v = lambda T, k, E, H, I, glu=True, whole=True: hipk.moe_variant(T, T * k, E, H, I, glu, whole)
+    assert [v(T, 2, 4, 2048, 5632) for T in (1, 2, 3)] == [3, 3, 6]
+    assert [v(T, 2, 12, 1536, 4096) for T in (1, 2, 3, 4)] == [3, 3, 3, 6]
+    assert [v(T, 2, 64, 2560, 2816) for T in (2, 3, 4, 16)] == [3, 3, 6, 6]
+    assert [v(T, 2, 8, 4096, 14336) for T in (1, 3, 4, 16, 500, 2000)] == [3, 3, 6, 6, 3, 4]
+    assert v(1, 2, 16, 1024, 1024) == 6 and v(1, 2, 16, 1024, 1024, whole=False) == 1
+    assert [v(T, 4, 16, 2048, 1792) for T in (1, 4, 224)] == [5, 6, 6] and v(224, 4, 16, 2048, 1792, whole=False) == 1
+    assert v(13, 4, 16, 4096, 3584) == 5 and v(16, 4, 20, 4096, 3584, glu=False) == 6
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T,act", [(4, "silu"), (24, "silu"), (128, "silu"), (64, "relu2")])
 def test_experts_at_any_address(hipk, T, act):
     """Rows or weights that start off 16 bytes, at sizes that the ring of LDS pieces takes otherwise: the form that
