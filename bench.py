@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Headline benchmark: smart-reply serving throughput on MI355X.
 
-Metric (BASELINE.json): "smart-reply tokens/sec (whole node) + p50 suggestion
+Metric: "smart-reply tokens/sec (whole node) + p50 suggestion
 latency, Llama-3-8B TP=1".
 
 Workload per GPU (one engine replica per GPU, DP over the node = weak

@@ -1,6 +1,6 @@
 """drtc_amd: an MI355X-native distributed real-time chat & collaboration stack.
 
-Layers (see SURVEY.md §1 for the reference's layer map):
+Layers:
 
 * control plane (CPU): ``protos`` (wire contract), ``raft`` (consensus core,
   replicated chat state machine, persistence), ``server`` (gRPC services),

@@ -1,7 +1,6 @@
 """Interactive chat client: ``python -m drtc_amd.client.cli [--server host:port]``.
 
-Same command set as the reference CLI (client/chat_client.py:466-1783, SURVEY
-§2.9): signup, login, logout, channels, create_channel, switch, join, send,
+Same command set as the reference CLI (client/chat_client.py:466-1783): signup, login, logout, channels, create_channel, switch, join, send,
 dm, conversations, back, history, users, reconnect, status, clear, upload,
 download, files, smart_reply, ask, suggest, summarize, add_user,
 remove_user, members, help, help_all - plus ``exit``/``quit``/EOF, which the

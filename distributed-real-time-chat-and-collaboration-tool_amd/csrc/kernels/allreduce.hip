@@ -1,4 +1,4 @@
-// One-shot peer-to-peer all-reduce for tensor-parallel decode (SURVEY X1).
+// One-shot peer-to-peer all-reduce for tensor-parallel decode.
 //
 // TP=8 decode issues 2 all-reduces per layer of [batch, hidden] bf16 - small
 // messages for which a ring (2(N-1) latency-bound steps, per-link bound on the

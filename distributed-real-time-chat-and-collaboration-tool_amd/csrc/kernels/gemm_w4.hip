@@ -6,8 +6,8 @@
 // This is the GEMM of the engine's prefill and full-batch decode passes (replacing the model
 // hop of ref llm_server/llm_server.py:231 / :287 with on-node compute).
 //
-// Why this layout: 8-wave forms (2 waves per SIMD, 128 x 64 per wave; round 2, removed in
-// round 4) reached 0.76-0.81x of hipBLASLt on the Llama shapes (profiles/r2a_hand_gemm.md):
+// Why this layout: 8-wave forms (2 waves per SIMD, 128 x 64 per wave), since
+// removed, reached 0.76-0.81x of hipBLASLt on the Llama shapes (profiles/r2a_hand_gemm.md):
 // parked at barriers (SQ_WAIT_ANY 9x the library's) and issuing 1.5x the LDS reads per
 // MFMA.  This kernel uses the layout that reads the least LDS per FLOP - one wave per SIMD,
 // 128 x 128 outputs per wave (64 MFMA 16x16x32 tiles = 256 accumulator registers, the AGPR

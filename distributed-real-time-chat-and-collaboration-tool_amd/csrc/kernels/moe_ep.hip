@@ -1,4 +1,4 @@
-// Expert-parallel dispatch / combine for the MoE all-to-all (SURVEY X2, ref call site
+// Expert-parallel dispatch / combine for the MoE all-to-all (ref call site
 // replaced: llm_server/llm_server.py:403, the hosted context-suggestion model).
 //
 // A rank holds T tokens routed to k experts each (P = T k pairs) and ships every pair to the

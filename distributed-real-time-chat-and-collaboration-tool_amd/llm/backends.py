@@ -3,7 +3,7 @@
 * ``EngineBackend``   - the on-GPU engine in this process (continuous batching
   through an EngineLoop thread; concurrent RPCs share decode steps).
 * ``ReplicaRouter``   - data parallelism: N engine replicas, one process per
-  GPU (``WorkerPool``), least-outstanding-requests routing (SURVEY X3).
+  GPU (``WorkerPool``), least-outstanding-requests routing.
 * ``ScriptedBackend`` - deterministic, format-correct text for CPU tests and
   the "LLM disabled" plumbing configuration (no model at all).
 
@@ -104,8 +104,7 @@ def _worker_main(rank: int, device: str, model_name: str, engine_kw: dict, inq, 
     completions of each engine step go back on ``outqs[fe]`` (one front-end, index 0, in
     this service).  Besides results, the worker sends a heartbeat with its engine
     counters every ``hb_interval`` s on ``ctlq``; the owner's health monitor evicts a replica
-    whose process died or whose heartbeats stopped (SURVEY §5 failure detection: per-GPU
-    replica eviction)."""
+    whose process died or whose heartbeats stopped."""
     import torch
 
     from ..engine.engine import EngineLoop, LLMEngine, freeze_gc

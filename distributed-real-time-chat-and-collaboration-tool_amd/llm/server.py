@@ -11,14 +11,14 @@ on-node inference:
                      (RCCL all-reduce over xGMI), e.g. Llama-3-70B TP=8;
   --backend scripted deterministic format-correct text (no model; CPU tests).
   --serve FEATURE=MODEL[@GPUS][:tpN][:mem=F] (repeatable) hosts one engine group per
-                     feature on GPUs of the node: the per-feature model matrix of
-                     BASELINE.json (Gemma-2B smart reply, Llama-3-8B summarize,
-                     Llama-3-70B TP=8 ask-AI, Mixtral suggestions) behind ONE service
+                     feature on GPUs of the node: Gemma-2B smart
+                     reply, Llama-3-8B summarize, Llama-3-70B TP=8 ask-AI,
+                     Mixtral suggestions, for instance, behind ONE service
                      address (features without a --serve use --model).  Groups may share
                      a GPU only with an explicit HBM budget each (mem=F: the fraction of
                      the GPU's total HBM the group may hold - weights, KV cache,
                      workspaces; at most 0.95 per GPU in all), so the split does not
-                     depend on start order.  The five BASELINE configs on one 8-GPU node:
+                     depend on start order.  Four features' models on one 8-GPU node:
                        --serve answer=llama-3-70b@0-7:tp8:mem=0.35
                        --serve smart=gemma-2b@0,4:mem=0.6
                        --serve summary=llama-3-8b@1,5:mem=0.6
@@ -52,7 +52,7 @@ log = logging.getLogger("drtc_amd.llm.server")
 # Engine batch (max concurrent requests per replica) when --max-batch is not given: the
 # measured throughput knee on one MI355X that still answers inside the reference's
 # per-feature node->LLM deadlines (20 s smart reply / suggestions, 10 s summarize and
-# ask-AI: ref server/raft_node.py:2018,2084,2126,2187).  BASELINE.md: Llama-3-8B smart
+# ask-AI: ref server/raft_node.py:2018,2084,2126,2187).  Llama-3-8B smart
 # reply at 1024 (p50 2.5 s; 1536 adds ~1 %), Gemma-2B at 2048 (p50 1.5 s, +7.7 % over 1024),
 # Mixtral suggestions at 1024 (p50 8.9 s, +11 % over 512, +40 % over 256), Llama-3-70B
 # ask-AI on one GPU at 224 (p50 9.15 s, 3,663 tok/s; 256: p50 9.83 s, too close to the 10 s

@@ -45,7 +45,7 @@ def _backend_for(backend, feature: str):
 class FeatureRouter:
     """One LLM service hosting several models: each feature ("smart", "summary", "answer",
     "suggest") is served by its own backend (an engine replica pool or a TP group on its
-    share of the node's GPUs), as BASELINE.json assigns a model per feature.  Backends
+    share of the node's GPUs).  Backends
     shared by several features are listed once in ``backends``."""
 
     FEATURES = ("smart", "summary", "answer", "suggest")

@@ -1,6 +1,6 @@
 """Model configurations (public architecture hyper-parameters; random-init weights).
 
-The four families BASELINE.json names for the LLM service:
+The four families of the LLM service:
   * Llama-3-8B  (smart reply / summarize, TP=1)        - flagship bench model
   * Llama-3-70B (ask-AI, TP=8 over xGMI)
   * Gemma-2B    (smart reply, TP=1; MQA, head_dim 256, GELU-tanh, (1+w) norm)

@@ -52,7 +52,7 @@ from .config import ModelConfig
 _EP_DECODE_A2A = os.environ.get("DRTC_EP_DECODE", "a2a") == "a2a"
 _EP_PREFILL = os.environ.get("DRTC_EP_PREFILL", "cap")
 
-# Two-stream micro-batched decode (VERDICT r5 item 1): the step's rows in two halves, one per
+# Two-stream micro-batched decode: the step's rows in two halves, one per
 # stream inside the captured graph, with each half's paged attention (HBM-bound) ordered to
 # run beside the other half's projections (per-CU operand-ingest bound).  DRTC_DECODE_MICRO=2
 # enables it for decode batches of at least DECODE_MICRO_MIN_B rows (dense TP=1 models);

@@ -892,7 +892,7 @@ def save_entries(entries: dict[str, dict], path: str | None = None) -> str:
 # per-tile form in one process (profiles/r3r/probe.log): prefill qkv +0.5 %, o +2.0 %,
 # gate_up+GLU +0.9 %, a 4400-row chunk's gate_up+GLU +2.3 %, decode gate_up+GLU at M = 1024
 # +4.0 %.  DRTC_W4_PERSIST=0 restores the per-tile form (variant 7).
-# Variant 31 (the default since round 4) adds the per-XCD K rotation: each XCD label starts its
+# Variant 31 (the default) adds the per-XCD K rotation: each XCD label starts its
 # K loop at its own eighth of K, so the eight XCDs' epilogue store bursts do not coincide.
 # Same box, interleaved (profiles/r4d/seam.log): decode gate_up + GLU at M = 1024 207.4 vs
 # 231.1 us (v15), prefill shapes within +-1 % (K = 14336 1.2 % faster).  Fewer than 8 tiles
@@ -929,7 +929,7 @@ def w4_group_m(M: int, N: int, K: int, glu: bool = False) -> int:
     """Row-tile group of the XCD-aware tile order.  An XCD's 32 workgroups take 32 consecutive
     tiles: with groups of 8 (4) rows that is an 8 x 4 (4 x 8) block of tiles, whose 12 operand
     panels stream through the XCD's L2 per K step, against 18 for the 2 x 16 block of groups
-    of 2 (round 5, profiles/r5c: hipBLASLt's down kernel 23.4 M L2 misses, gemm_w4 at group 2
+    of 2 (profiles/r5c: hipBLASLt's down kernel 23.4 M L2 misses, gemm_w4 at group 2
     34.1 M).  Interleaved on one box (profiles/r5d): down at K = 14336 1217 us at 8 vs 1247 at
     2; qkv 524 vs 532 at 4; o + residual 376 vs 378; the gated gate_up 2513 at 4 vs 2537 at 8."""
     return 4 if glu else 8

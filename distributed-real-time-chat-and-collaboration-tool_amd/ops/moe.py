@@ -4,7 +4,7 @@ HIP kernels: csrc/kernels/moe.hip.  One call enqueues four kernels with
 static launch shapes (the per-expert tile table lives on the device), so the
 layer is hipGraph-capturable and the Mixtral decode step replays with no
 host synchronisation and exact sparse FLOPs (the earlier graph path ran every
-expert on every token).  SURVEY.md §2 K8.
+expert on every token).
 
 Routing semantics: top-k of the router logits, softmax over the selected k logits (as much as a
 softmax over all experts divided by the chosen ones' sum); ties pick the lower expert id.  With
@@ -102,7 +102,7 @@ def make_workspace(tokens: int, hidden: int, inter: int, e_local: int, top_k: in
 
 
 # fused_moe reads the router GEMM's [E, T] output in place (DRTC_ROUTER_VIEW=0: the
-# transposed copy of round 5's first router form, for A/B)
+# transposed copy of an earlier router form, for comparison)
 ROUTER_VIEW = os.environ.get("DRTC_ROUTER_VIEW", "1") != "0"
 
 

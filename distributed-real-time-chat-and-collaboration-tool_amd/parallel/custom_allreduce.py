@@ -1,4 +1,4 @@
-"""One-/two-shot P2P all-reduce for tensor-parallel messages (SURVEY X1, §7.3).
+"""One-/two-shot P2P all-reduce for tensor-parallel messages.
 
 Kernel + memory protocol: csrc/kernels/allreduce.hip.  Each rank allocates
 one uncached device buffer (flags + double-buffered staging), exports it as

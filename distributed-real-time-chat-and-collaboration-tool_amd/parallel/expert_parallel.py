@@ -1,4 +1,4 @@
-"""Expert parallelism with token dispatch/combine over all-to-all (SURVEY X2).
+"""Expert parallelism with token dispatch/combine over all-to-all.
 
 Served form (models/transformer.py, ``ep_size > 1``): every rank owns E/ep
 experts and a SHARD of the tokens - the sequence-parallel rows of a prefill

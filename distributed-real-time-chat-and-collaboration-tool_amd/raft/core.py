@@ -21,7 +21,7 @@ Behaviour vs the reference (server/raft_node.py:469-1194):
   * AppendEntries batches are bounded in bytes (quirk Q12) and rejected
     followers are probed with exponential back-off instead of one entry
     per round trip;
-  * log compaction (the reference has none, SURVEY §5 "Checkpoint"): the
+  * log compaction (the reference has none): the
     runtime snapshots the state machine at an applied index and calls
     ``compact``; entries up to it leave the log (``snap_index`` /
     ``snap_term`` remember the boundary).  A follower whose next entry was

@@ -1,6 +1,6 @@
 """Deterministic in-memory network for RaftCore (fault-injection test harness).
 
-The reference has no fault injection at all (SURVEY §5); this simulator
+The reference has no fault injection at all; this simulator
 drives N cores on a virtual clock and lets tests drop, delay, duplicate and
 reorder messages and partition the cluster.
 """

@@ -1,9 +1,9 @@
 """Replicated chat state machine (the apply side of the Raft log).
 
-Log-entry commands and their JSON payloads are the reference's (SURVEY §2.7,
-server/raft_node.py:1196-1397); in-memory records keep the reference's dict
+Log-entry commands and their JSON payloads are the reference's
+(server/raft_node.py:1196-1397); in-memory records keep the reference's dict
 schemas so the app-state pickles (users/channels/messages/direct_messages)
-stay byte-compatible (SURVEY §2.8).  Differences, all deliberate:
+stay byte-compatible.  Differences, all deliberate:
 
 * idempotency by id *sets* (O(1)) instead of linear scans (raft_node.py:1354,1376);
 * secondary indexes for the read RPCs (DMs by user pair / by user id);
@@ -184,7 +184,7 @@ class ChatState:
         """The default users/channels as log entries (CREATE_USER /
         CREATE_CHANNEL) for whatever is still missing: proposed once by the
         first leader of a fresh cluster, so every replica applies the same
-        bcrypt hashes and timestamps (byte-identical pickles; SURVEY Q11).
+        bcrypt hashes and timestamps (byte-identical pickles).
         Ids are the names, as in the reference (server/raft_node.py:426-467)."""
         out = []
         ids = [name for name, _ in DEFAULT_USERS]

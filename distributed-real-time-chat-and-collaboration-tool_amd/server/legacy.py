@@ -1,6 +1,6 @@
 """Legacy single-node ``chat.ChatService`` (no Raft) with real-time streaming.
 
-Capabilities of the reference's server/app_server.py (SURVEY C27/C28):
+Capabilities of the reference's server/app_server.py:
 signup with validation (username 3-20 ``[A-Za-z0-9_]``, e-mail regex,
 password 6-50 with a digit/special), login/logout, channels with admin
 management (``ManageChannel`` add_user/remove_user), channel posts, DMs,

@@ -1,8 +1,8 @@
 """``raft.RaftNode`` gRPC service: the chat application over Raft.
 
 RPC semantics, response messages and log-entry payloads follow the reference
-handlers (server/raft_node.py:1401-2347, SURVEY §2.6); deliberate fixes are
-marked with the survey quirk they address:
+handlers (server/raft_node.py:1401-2347); deliberate fixes are
+numbered by the quirk of the reference they address:
 
   Q1  writes are acknowledged after majority commit (RaftConfig.local_commit
       restores leader-local commit);
@@ -82,7 +82,7 @@ class NodeConfig:
         "smart": 20.0, "summary": 10.0, "answer": 10.0, "suggest": 20.0})
     # per-feature LLM services (None: ``llm_address``, the reference's single LLM server,
     # ref server/raft_node.py:372).  One node can route each AI RPC to the engine group
-    # serving that feature's model (BASELINE: Gemma-2B smart reply, 8B summarize, 70B ask,
+    # serving that feature's model (for instance Gemma-2B smart reply, 8B summarize, 70B ask,
     # Mixtral suggestions) - ref call sites :2018 / :2084 / :2126 / :2187.
     llm_smart: str | None = None
     llm_summary: str | None = None
@@ -172,7 +172,7 @@ class ChatNode:
         self.rt.stop()
 
     def _genesis_loop(self) -> None:
-        """Seed the default users/channels through the log (SURVEY Q11): once
+        """Seed the default users/channels through the log: once
         this node leads and has applied its whole log (its NOOP committed, so
         every earlier entry is in the state), propose whatever default record
         is still missing.  Apply is idempotent by username / channel id, so a

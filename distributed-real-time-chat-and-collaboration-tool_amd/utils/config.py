@@ -1,10 +1,10 @@
-"""Config files for the CLIs (SURVEY §5 "Config / flags").
+"""Config files for the CLIs.
 
 The reference hardcodes everything but ``--node-id/--port`` (server) and
 ``--server`` (client).  Here every entry point's flags can also come from a
 JSON or YAML file (``--config node1.yaml``); values on the command line
 override the file, and the file overrides the built-in defaults (which equal
-the reference's values where the reference has one, SURVEY §2.10).  Keys are
+the reference's values where the reference has one).  Keys are
 the flags' destination names, e.g. ``node_id``, ``election_timeout``,
 ``snapshot_every``; an unknown key is an error, not silently ignored.
 YAML is read with ``yaml.safe_load`` (no object construction).

@@ -1,6 +1,6 @@
 """Process-wide metrics registry: counters and latency histograms.
 
-The reference has only ad-hoc log lines (SURVEY §5 "Metrics"); every server
+The reference has only ad-hoc log lines; every server
 here records RPC latencies, Raft proposals, engine tokens/s, TTFT/TPOT and
 KV occupancy into this registry, which the bench harness and the
 ``status`` RPCs dump.  Histograms keep a bounded reservoir so percentiles

@@ -1,4 +1,4 @@
-"""Byte-compatible pickle I/O for the reference's on-disk formats (SURVEY §2.8).
+"""Byte-compatible pickle I/O for the reference's on-disk formats.
 
 Writers pin protocol 4 (the default of the CPython 3.8-3.13 interpreters the
 reference ran on).  Readers NEVER execute code from a file: ``safe_load``

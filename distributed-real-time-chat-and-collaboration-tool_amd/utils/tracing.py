@@ -1,4 +1,4 @@
-"""Tracing: roctx ranges + an in-process span recorder (SURVEY §5 "Tracing").
+"""Tracing: roctx ranges + an in-process span recorder.
 
 The reference has no tracing (an unused ``PerformanceLogger``,
 utils/logger_config.py:102-123).  Here:
