@@ -1293,14 +1293,20 @@ _parts_forms: dict[tuple[int, int, int], tuple[int, int] | None] = {}
 
 
 def parts_form(M: int, N: int, K: int) -> tuple[int, int] | None:
-    """How ``linear_parts`` cuts a product of M rows, None where ``linear`` is as fast.  us of ``linear`` / of
-    the parts, to which reading them adds 0.3 - 2:
+    """How ``linear_parts`` cuts a product of M rows, None where ``linear`` is as fast.  us of ``linear`` as it was before
+    ``small_form`` / of the parts, to which reading them adds 0.3 - 2:
       K from 5120 on, 3 rows to 256: 4096 x 14336, 4 rows 22.7 / 19.8, 16 24.2 / 19.8, 64 28.3 / 22.7, 160 39.0 / 30.8, 256
         58.0 / 38.6; 2048 x 7168, 4 rows 11.0 / 7.4, 160 24.2 / 14.1; 2048 x 5632, 256 rows 20.9 / 16.0; two rows and one
         stay with the dot2 form (2048 x 7168 8.4 / 7.4, 7.5 / 7.3)
       K from 4096 on to 160 rows: 4096 x 4096, 4 rows 9.7 / 8.4, 16 11.1 / 8.5, 64 14.1 / 9.9, 160 19.5 / 15.0; 200 18.8 / 17.3
       K from 2048 on, 17 rows to 64, 128 where narrow: 2048 x 2048, 16 rows 6.2 / 4.8, 24 7.6 / 5.0, 64 10.7 / 5.9, 128 10.7 /
         7.6, 160 10.5 / 8.7; 3584 x 2048, 64 rows 9.4 / 7.0, 96 9.2 / 8.3
+    Product and norm together, ``linear`` as it is / the parts: over 1224 shapes of K 2048 to 28672 1 / 0.72; 4096 x 14336,
+      4 rows 27.2 / 25.6, 64 31.1 / 29.6, 256 52.1 / 49.3; 2048 x 7168, 160 rows 26.7 / 20.7; 4096 x 4096, 16 rows 14.2 / 12.5, 64
+      17.2 / 14.9; 2048 x 2048, 24 rows 9.7 / 8.0, 64 10.8 / 9.3.  The 64-row tiles of ``small_form`` are the faster product in
+      52 of them, most of K up to 4096 from 96 rows on (4096 x 4096, 144 rows 20.2 / 23.8; 2048 x 2048, 128 rows 10.9 / 12.6),
+      and for 256 rows at K near 5120 (1024 x 5120 17.0 / 19.7).  The parts stay there: the norm reads these sums in 32 bits,
+      and a product's rows would be rounded to 16 in between.
     The cut: the least of a workgroup's operands at 50 GB/s or its weights at 24, a quarter of a microsecond to
     a slice, and the parts read again by the whole chip or by a row's CU."""
     key = (M, N, K)
