@@ -1261,6 +1261,15 @@ def midm_gemm(x: torch.Tensor, w: torch.Tensor, epi: str = "store",
     assert out.shape == (M, NO) and out.stride(1) == 1
     if epi == "residual":
         assert residual is not None and residual.shape == (M, N) and residual.stride(1) == 1
+    # whole 16-byte pieces into LDS at 32-bit offsets, residual and y by four values: what lies otherwise is copied
+    if x.stride(0) % 8 == 0 and (x.data_ptr() % 16 or x.stride(0) >= 1 << 22):
+        x = torch.empty((M, K), dtype=x.dtype, device=x.device).copy_(x)
+    if w.data_ptr() % 16:
+        w = w.clone()
+    if residual is not None and residual.stride(0) % 4 == 0 and residual.data_ptr() % 8:
+        residual = torch.empty((M, N), dtype=x.dtype, device=x.device).copy_(residual)
+    if out.stride(0) % 4 == 0 and out.data_ptr() % 8:
+        return out.copy_(midm_gemm(x, w, epi, residual, torch.empty((M, NO), dtype=x.dtype, device=x.device), splits, nf))
     slab = gemm_workspace(x.device)[0]
     check(hipk().midm_gemm(out.data_ptr(), x.data_ptr(), w.data_ptr(), ptr(residual), M, N, K,
                            x.stride(0), out.stride(0),

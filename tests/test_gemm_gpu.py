@@ -184,6 +184,28 @@ def test_linear_takes_rows_at_any_address(hipk, M, N, K, kind):
         assert _rel(G.linear(x, w), x.float() @ w.float().t()) < 1e-2
 
 
+@pytest.mark.parametrize("M,splits", [(33, 1), (200, 4)])
+def test_midm_takes_operands_at_any_address(hipk, M, splits):
+    """Input and weights off 16 bytes, residual and output (also in place) off 8, and rows too far apart for 32-bit offsets."""
+    N, K = 512, 1024
+    g = torch.Generator(device="cuda").manual_seed(M)
+
+    def off(rows, cols, by, scale=1.0):
+        flat = (torch.randn(rows * cols + 8, device="cuda", generator=g) * scale).to(torch.bfloat16)
+        return flat[by:by + rows * cols].view(rows, cols)
+
+    x, w, res = off(M, K, 3), off(N, K, 1, K ** -0.5), off(M, N, 2)
+    far = torch.empty((M - 1 << 24) + K, dtype=torch.bfloat16, device="cuda").as_strided((M, K), (1 << 24, 1)).copy_(x)
+    y, ref = off(M, N, 1), x.float() @ w.float().t()
+    for xx in (x, far):
+        assert _rel(G.midm_gemm(xx, w, splits=splits), ref) < 1e-2
+    assert G.midm_gemm(x, w, "residual", residual=res, out=y, splits=splits) is y
+    assert _rel(y, ref + res.float()) < 1e-2
+    ref = ref + res.float()
+    assert G.midm_gemm(x, w, "residual", residual=res, splits=splits) is res
+    assert _rel(res, ref) < 1e-2
+
+
 @pytest.mark.parametrize("epi", ["store", "residual", "silu"])
 @pytest.mark.parametrize("M,N,K,splitk,gm", [(1024, 4096, 4096, 4, -4), (1024, 4096, 4096, 2, -2),
                                              (512, 2048, 1024, 8, -2), (1000, 1024, 2048, 4, -1)])
