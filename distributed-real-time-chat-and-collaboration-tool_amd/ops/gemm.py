@@ -70,7 +70,7 @@ _prefill_enabled = os.environ.get("DRTC_PREFILL_TUNED", "1") != "0"
 _midm_enabled = os.environ.get("DRTC_MIDM_GEMM", "1") != "0"
 _xd_enabled = os.environ.get("DRTC_XD_GEMM", "1") != "0"
 # tuned gemm_xd forms whose batch fits one row tile take non-temporal weight loads (each weight
-# byte enters one CU once: MI355X_MICROARCH.md nt-weights; profiles/r4aa: Llama-3-70B down at
+# byte enters one CU once; profiles/r4aa: Llama-3-70B down at
 # M = 256 159.6 -> 136.8 us, gated gate_up 265.7 -> 230.2, the 70B ask wave +5.2 %)
 _xd_nt = os.environ.get("DRTC_XD_NT", "1") != "0"
 # decode batches up to this many rows may take the skinny kernel: the table's choice where
@@ -1135,7 +1135,7 @@ def xd_form(form: int) -> tuple[int, int, int]:
 
 
 def xd_nt(form: int) -> bool:
-    """Form with non-temporal weight loads (MI355X_MICROARCH.md nt-weights)."""
+    """Form with non-temporal weight loads."""
     return form >= 1000
 
 
