@@ -49,6 +49,15 @@ def test_packed_prefill_last_layer_pruning(cfg):
         assert (got[j] - ref).abs().max() <= 2e-2 * max(1.0, ref.abs().max().item())
 
 
+def test_prefill_buckets():
+    from drtc_amd.engine.engine import _pad_tokens
+
+    padded = [_pad_tokens(T) for T in range(1, 20000)]
+    for T, Tp in enumerate(padded, 1):
+        assert T <= Tp < T + (32 if T <= 1024 else T / 16) and Tp % 32 == 0
+    assert padded == sorted(padded) and len(set(padded)) < 150
+
+
 def test_engine_preemption_and_recompute():
     m = TransformerLM(TINY_LLAMA, "cpu", seed=3)
     eng = LLMEngine(m, max_batch=8, max_model_len=512, num_blocks=12, use_graphs=False)

@@ -25,6 +25,23 @@ def test_prefill_logits_match_reference(hipk, cfg):
         assert err < 0.05 * max(1.0, b.float().abs().max().item()), err
 
 
+@pytest.mark.parametrize("tokens", [257, 288, 1025, 2049])
+def test_packed_prompts_off_the_bucket(hipk, tokens):
+    """Logits of packed prompts that leave most of a bucket's rows, one or none as padding."""
+    from drtc_amd.engine import Request
+
+    cfg = TINY_MIXTRAL.replace(experts_per_token=TINY_MIXTRAL.num_experts)  # no routing discontinuity
+    m = TransformerLM(cfg, "cuda", seed=5)
+    eng = LLMEngine(m, max_batch=16, max_model_len=512, num_blocks=128, use_graphs=False)
+    seqs = [[(7 * i + j) % 500 + 3 for j in range(n)] for i, n in enumerate([tokens % 200] + [200] * (tokens // 200))]
+    got = eng.feed([(Request([]), s, [len(s) - 1]) for s in seqs])
+    with ops.reference_mode():
+        ref = m.forward_reference(seqs)
+    for a, b in zip(got, ref):
+        err = (a[-1].float() - b[-1].float()).abs().max().item()
+        assert err < 0.05 * max(1.0, b[-1].float().abs().max().item()), err
+
+
 @pytest.mark.parametrize("cfg", [TINY_LLAMA, TINY_GEMMA, TINY_MIXTRAL], ids=lambda c: c.name)
 def test_engine_decode_matches_reference(hipk, cfg):
     """Greedy decode through paged KV + graphs agrees with a full-sequence
