@@ -11,6 +11,8 @@
 //     3584 x 2048, 224 rows 10.7 us in tiles of 128 x 64, 8.9 of 64 x 64), or 128 MT x 32 NF (MT 1 / 2, NF 2 / 4 / 6 / 8), K split over splitk = 1..8 slices
 //     (whole K tiles, as even as they divide), one workgroup per (tile, slice) and per CU
 //     (o / down at M = 1024: 8 x 32 tiles of 128 x 128, or 4 x 32 x 2 slices of 256 x 128;
+//     or one tile of 160, 192 or 224 rows x 32 NF (MT 3 .. 5; 28672 x 4096 gated, 160 rows: 57 us padded to 256, 50;
+//     32000 x 4096, 192 rows 60 / 56) in rings of what the LDS holds;
 //     qkv N = 6144: 8 x 32 of 128 x 192; Llama-3-70B at M = 256: 256 x 128 x 3-4 slices;
 //     gated gate_up at M = 512-1024: 256 x 256).  Per shape the tuning table picks the form
 //     (scripts/tune_xd.py, ops/gemm.py route / glu_form).
@@ -62,12 +64,15 @@ DRTC_DEVICE constexpr bool xd_glu() {
 template <int EPI>
 DRTC_DEVICE constexpr int xd_act() { return EPI == XD_SILU ? 0 : EPI == XD_GELU ? 1 : 2; }
 
+// 16-row fragments of a wave in tile MT: tiles have 32 times as many rows
+constexpr int xd_fa(int mt) { return mt == 0 ? 2 : mt <= 2 ? 4 * mt : mt + 2; }
+
 template <int MT_, int NF_, int S_, bool SPLIT_, bool NT_ = false>
 struct XdCfg {
   static constexpr int MT = MT_, NF = NF_, S = S_;
   static constexpr bool SPLIT = SPLIT_;            // split-K combine compiled in
   static constexpr bool NT = NT_;                  // weight (B) LDS-DMA non-temporal
-  static constexpr int FA = MT ? 4 * MT : 2;       // A fragments per wave (16 rows each); MT 0: 64-row tiles
+  static constexpr int FA = xd_fa(MT);             // A fragments per wave (16 rows each)
   static constexpr int TM = 32 * FA;               // tile rows
   static constexpr int TN = 32 * NF;               // tile columns
   static constexpr int H = FA * NF;                // MFMAs per 32-deep K half (per wave)
@@ -575,9 +580,10 @@ __global__ __launch_bounds__(kXdThreads, 1) void gemm_xd_kernel(XdParams p) {
   __syncthreads();
   constexpr int CPR = OC / 8;  // 16-B chunks per wave-tile row
 #pragma unroll
-  for (int s = 0; s < CPR * FA / 4; ++s) {
+  for (int s = 0; s < (CPR * FA + 3) / 4; ++s) {
     const int q = lane + 64 * s;
     const int row = q / CPR, ch = q - row * CPR;
+    if (CPR * FA % 4 && row >= 16 * FA) continue;
     if (16 * FA * wm + row >= rows_a) continue;
     const int m = m0 + 16 * FA * wm + row;
     const int n = n0 + OC * wn + 8 * ch;
@@ -690,10 +696,16 @@ template <bool NT = false>
 using Xd0x2 = XdCfg<0, 2, 6, false, NT>;
 template <bool NT = false>
 using Xd0x4 = XdCfg<0, 4, 4, false, NT>;
+// one row tile of 160, 192 and 224 rows, non-temporal weights
+using Xd3x2 = XdCfg<3, 2, 5, false, true>;
+using Xd3x4 = XdCfg<3, 4, 4, false, true>;
+using Xd4x4 = XdCfg<4, 4, 4, false, true>;
+using Xd5x4 = XdCfg<5, 4, 3, false, true>;
 
 int xd_stages(int mt, int nf) {
   if (mt == 0) return nf == 1 || nf == 2 ? 6 : (nf == 4 ? 4 : 0);
   if (mt == 1) return nf == 6 ? 3 : (nf == 2 || nf == 4 ? 4 : 0);
+  if (mt >= 3 && mt <= 5) return nf == 4 ? (mt == 5 ? 3 : 4) : nf == 2 && mt == 3 ? 5 : 0;
   if (mt == 2) return nf == 4 ? 3 : (nf == 6 || nf == 8 ? 2 : 0);
   return 0;
 }
@@ -714,6 +726,10 @@ int xd_dispatch(const XdParams& p, int mt, int nf, bool nt, int epi, hipStream_t
   }
   if (nt) {
     switch (mt * 10 + nf) {
+      case 32: if constexpr (!SP) return xd_launch<Xd3x2>(p, epi, st); else return -1;
+      case 34: if constexpr (!SP) return xd_launch<Xd3x4>(p, epi, st); else return -1;
+      case 44: if constexpr (!SP) return xd_launch<Xd4x4>(p, epi, st); else return -1;
+      case 54: if constexpr (!SP) return xd_launch<Xd5x4>(p, epi, st); else return -1;
       case 14: return xd_launch<Xd1x4<SP, true>>(p, epi, st);
       case 16: return xd_launch<Xd1x6<SP, true>>(p, epi, st);
       case 24: return xd_launch<Xd2x4<SP, true>>(p, epi, st);
@@ -757,8 +773,9 @@ void set_splitk_spin_limit(int limit) { g_spin_limit = limit; }
 int64_t gemm_xd_workspace_bytes(int M, int N, int mt, int nf, int splitk, int glu) {
   if (splitk < 2 || mt < 1 || nf < 1) return 0;  // (64-row tiles have no slices)
   const int tno = glu ? 16 * nf : 32 * nf;
-  const int64_t tiles = (int64_t)((M + 128 * mt - 1) / (128 * mt)) * (N / tno);
-  return tiles * splitk * (128 * mt) * (32 * nf) * 4;
+  const int rows = 32 * xd_fa(mt);
+  const int64_t tiles = (int64_t)((M + rows - 1) / rows) * (N / tno);
+  return tiles * splitk * rows * (32 * nf) * 4;
 }
 
 int launch_gemm_xd(void* c, const void* a, const void* b, const void* r, int M, int N, int K,
@@ -775,7 +792,7 @@ int launch_gemm_xd(void* c, const void* a, const void* b, const void* r, int M, 
   if ((uintptr_t)a % 16 || (uintptr_t)b % 16 || (uintptr_t)c % 16) return -1;
   if (epi == XD_RESIDUAL && (r == nullptr || ldr % 8 || (uintptr_t)r % 16)) return -1;
   if (mt == 0 && (glu || splitk > 1)) return -1;
-  const int tm_rows = mt ? 128 * mt : 64, tno = glu ? 16 * nf : 32 * nf;
+  const int tm_rows = 32 * xd_fa(mt), tno = glu ? 16 * nf : 32 * nf;
   // shape contract: whole column tiles, every slice more K tiles than the ring holds (the
   // first K tile is peeled), 32-bit buffer offsets from the tile bases
   if (M <= 0 || N <= 0 || N % tno || K % 64 || K / 64 / splitk <= stages) return -1;
@@ -834,7 +851,7 @@ int launch_gemm_xd_grouped(void* c, const void* a, const void* b, int a_rows, in
   if ((uintptr_t)a % 16 || (uintptr_t)b % 16 || (uintptr_t)c % 16) return -1;
   if (tile_row0 == nullptr || tile_rows == nullptr || tile_expert == nullptr || n_tiles == nullptr)
     return -1;
-  const int tm_rows = 128 * mt, tno = glu ? 16 * nf : 32 * nf;
+  const int tm_rows = 32 * xd_fa(mt), tno = glu ? 16 * nf : 32 * nf;
   if (N <= 0 || N % tno || K % 64 || K / 64 / splitk <= stages) return -1;
   // 32-bit buffer offsets: a gathered A row anywhere in A, a tile's rows of contiguous A, the
   // weight rows of one expert
@@ -883,7 +900,7 @@ int configure_gemm_xd() {
                 xd_cfg_g<Xd2x8<false, true>>() | xd_cfg_g<Xd1x4<true, true>>() |
                 xd_cfg_g<Xd2x4<true, true>>() | xd_cfg_g<Xd2x8<true, true>>();
   if (g) return g;
-  return xd_cfg<Xd0x1<>>() | xd_cfg<Xd0x2<>>() | xd_cfg<Xd0x4<>>() | xd_cfg<Xd0x1<true>>() | xd_cfg<Xd0x2<true>>() |
+  return xd_cfg<Xd3x2>() | xd_cfg<Xd3x4>() | xd_cfg<Xd4x4>() | xd_cfg<Xd5x4>() | xd_cfg<Xd0x1<>>() | xd_cfg<Xd0x2<>>() | xd_cfg<Xd0x4<>>() | xd_cfg<Xd0x1<true>>() | xd_cfg<Xd0x2<true>>() |
          xd_cfg<Xd0x4<true>>() | xd_cfg<Xd1x2<false>>() | xd_cfg<Xd1x4<false>>() | xd_cfg<Xd1x6<false>>() |
          xd_cfg<Xd2x4<false>>() | xd_cfg<Xd2x6<false>>() | xd_cfg<Xd1x2<true>>() |
          xd_cfg<Xd1x4<true>>() | xd_cfg<Xd1x6<true>>() | xd_cfg<Xd2x4<true>>() |

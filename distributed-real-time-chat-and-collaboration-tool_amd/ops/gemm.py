@@ -141,7 +141,7 @@ def _activate() -> dict:
 def xd_nt_ok(M: int, form: int) -> bool:
     """Whether ``form`` (plain) has a non-temporal build and M fits one of its row tiles."""
     mt, nf, _ = xd_form(form)
-    return form < 1000 and (mt, nf) in XD_NT_TILES and M <= 128 * mt
+    return form < 1000 and (mt, nf) in XD_NT_TILES and M <= XD_ROWS[mt]
 
 
 def _xd_policy(M: int, form: int, nt_tuned: bool = False) -> int:
@@ -240,6 +240,9 @@ def _resolve(M: int, N: int, K: int, ldx: int) -> tuple[str, int]:
         return ("w4", 0) if _w4_long(M, N, K) else ("torch", 0)
     if dot2_ok(M, N, K, ldx):
         return ("skinny", 1)
+    tall = tall_form(M, N, K)
+    if tall and ldx % 8 == 0:
+        return ("xd", tall)
     found = _decode_entry(M, N, K, ldx)
     wide = wide_form(M, N, K)
     if wide and not (found is not None and found[1][3]):  # (entries of gemm_xd: measured against its other forms)
@@ -317,6 +320,25 @@ def brief_pays(M: int, N: int, K: int, listed: bool) -> bool:
     every workgroup, so many of them lose: 1024 x 128, 160 rows 3.7 / 4.9, 256 3.7 / 6.5.  The table's, 2048 x 128: 48 rows 6.2 /
     3.5, 128 6.3 / 4.6, 200 7.0 / 5.8, 256 6.8 / 6.4; 4096 x 256, 48 rows 6.5 / 4.5, 128 5.9 / 6.0."""
     return M <= 64 or M <= 128 and N * K >= 3072 * 192 or listed
+
+
+def tall_form(M: int, N: int, K: int, glu: bool = False, act: str = "silu") -> int:
+    """gemm_xd form of one row tile of 160, 192 or 224 rows for a product of 129 .. 224 rows (N output columns, gated: of a
+    half) that tiles of 128 rows of W cut into one well filled round of the CUs; 160 rows also where tiles of 64 do, nearly
+    full.  Other forms pad the rows to 256, or read W twice.  us, the best of them / this: 28672 x 4096 gated, 132 rows
+    58.4 / 48.0, 160 56.9 / 50.9, 192 56.2 / 54.2, 224 57.8 / 57.7; 32000 x 4096, 144 rows 60.6 / 53.1, 208 61.0 / 58.4; 32000 x
+    2048, 160 33.4 / 30.3; 25600 x 4096, 224 57.2 / 54.2; 20480 x 2048 (160 tiles), 160 28.2 / 26.4, 224 30.0 / 29.2; in tiles of
+    64: 14336 x 2048 gated, 132 rows 22.3 / 18.3, 160 20.4 / 19.4, 12800 x 2048 20.1 / 19.0, 16384 x 4096 gated 39.1 / 36.7.
+    More than a round: 57344 x 4096 gated, 176 rows 100.6 / 109; fewer tiles: 16384 x 4096 gated, 160 rows 39.1 / 48.4, and of 64
+    8448 x 2048, 160 rows 17.6 / 17.9; 192 rows in tiles of 64 12800 x 2048 21.5 / 21.4."""
+    if not (_xd_enabled and _enabled and _xd_nt and 129 <= M <= 224 and K >= 2048):
+        return 0
+    mt, rows = 3 if M <= 160 else 4 if M <= 192 else 5, 2 * N if glu else N
+    nf = 4 if rows % 128 == 0 and 160 <= rows // 128 <= 256 else 2 if mt == 3 and rows % 64 == 0 and 192 <= rows // 64 <= 256 else 0
+    if not nf or act == "clamped" and nf not in XD_CLAMP_NF:
+        return 0
+    form = 1001 + 100 * mt + 10 * nf
+    return form if xd_supported(M, N, K, form, glu) else 0
 
 
 def wide_form(M: int, N: int, K: int) -> int:
@@ -988,11 +1010,14 @@ def w4_glu_ok(x: torch.Tensor, w: torch.Tensor, act: str) -> bool:
 
 
 def glu_form(M: int, N2: int, K: int, ldx: int, act: str = "silu") -> int:
-    """gemm_xd gated form for a decode batch M through the [gate; up] weight [N2, K]: the one the
+    """gemm_xd gated form for a decode batch M through the [gate; up] weight [N2, K]: ``tall_form``'s, or the one the
     tuning table measured fastest (bucket-above for an off-bucket M), else ``_glu_default``, also
     where the table has an entry for the plain product only; 0: none."""
     if not (_xd_enabled and _enabled) or M > DECODE_MAX_M:
         return 0
+    tall = tall_form(M, N2 // 2, K, True, act)
+    if tall:
+        return tall
     found = _decode_entry(M, N2, K, ldx)
     form = found[1][4] if found is not None else 0
     if not form or act == "clamped" and form // 10 % 10 not in XD_CLAMP_NF:
@@ -1118,15 +1143,16 @@ def squared_relu(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.T
 
 # ------------------------------------------------------------------ XCD-partitioned decode GEMM
 XD_EPI = {"store": 0, "residual": 1, "silu": 2, "gelu_tanh": 3, "clamped": 4, "relu2": 5}
-# tile shapes built in gemm_xd.hip, (mt, nf) -> LDS ring depth (128 mt x 32 nf tiles, mt 0: 64 rows); a form
+# tile shapes built in gemm_xd.hip, (mt, nf) -> LDS ring depth (XD_ROWS[mt] x 32 nf tiles); a form
 # is mt * 100 + nf * 10 + splitk (K split over 1..8 slices), + 1000 for non-temporal weight
 # loads (the tiles of XD_NT_TILES)
-XD_TILES = {(0, 1): 6, (0, 2): 6, (0, 4): 4, (1, 2): 4, (1, 4): 4, (1, 6): 3, (2, 4): 3, (2, 6): 2, (2, 8): 2}
+XD_TILES = {(0, 1): 6, (0, 2): 6, (0, 4): 4, (3, 2): 5, (3, 4): 4, (4, 4): 4, (5, 4): 3, (1, 2): 4, (1, 4): 4, (1, 6): 3, (2, 4): 3, (2, 6): 2, (2, 8): 2}
+XD_ROWS = {0: 64, 1: 128, 2: 256, 3: 160, 4: 192, 5: 224}  # mt -> rows of a tile
 XD_CLAMP_NF = (4, 8)  # tile widths the clamped epilogue is built for
-XD_NT_TILES = {(0, 1), (0, 2), (0, 4), (1, 4), (1, 6), (2, 4), (2, 6), (2, 8)}
+XD_NT_TILES = {(0, 1), (0, 2), (0, 4), (3, 2), (3, 4), (4, 4), (5, 4), (1, 4), (1, 6), (2, 4), (2, 6), (2, 8)}
 XD_MAX_SPLITK = 8
 # the forms the tuner (scripts/tune_xd.py) measures
-XD_FORMS = tuple(sorted([mt * 100 + nf * 10 + 1 for mt, nf in XD_TILES if mt] +
+XD_FORMS = tuple(sorted([mt * 100 + nf * 10 + 1 for mt, nf in XD_TILES if 1 <= mt <= 2] +
                         [200 + nf * 10 + sk for nf in (4, 6, 8) for sk in (2, 3, 4)]))
 
 
@@ -1144,6 +1170,8 @@ def xd_supported(M: int, N: int, K: int, form: int, glu: bool = False) -> bool:
     columns (gated: half the rows of the [gate; up] weight)."""
     mt, nf, sk = xd_form(form)
     if (mt, nf) not in XD_TILES or not 1 <= sk <= XD_MAX_SPLITK or (glu and nf % 2) or mt == 0 and (glu or sk > 1):
+        return False
+    if mt > 2 and not (xd_nt(form) and sk == 1 and M <= XD_ROWS[mt]):  # one row tile, non-temporal
         return False
     if form // 1000 > 1 or (xd_nt(form) and (mt, nf) not in XD_NT_TILES):
         return False

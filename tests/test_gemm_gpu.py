@@ -399,6 +399,42 @@ def test_xd_gemm_glu_matches_fp32(hipk, act, form, M, I, K):
     _check(out, _ref(x, w, act, None))
 
 
+@pytest.mark.parametrize("epi", ["store", "residual", "relu2", "silu", "gelu_tanh", "clamped"])
+@pytest.mark.parametrize("form,M", [(1321, 129), (1321, 160), (1341, 1), (1341, 160), (1441, 161), (1441, 192),
+                                    (1541, 193), (1541, 224)])
+@pytest.mark.parametrize("K", [384, 1024])  # 384: one K tile more than the deepest ring
+def test_xd_gemm_one_tall_tile(hipk, form, M, K, epi):
+    """One row tile of 160, 192 or 224 rows: every output written, against fp32."""
+    glu, N = epi in G.GATED, 384
+    assert G.xd_supported(M, N, K, form, glu)
+    if epi == "clamped" and G.xd_form(form)[1] not in G.XD_CLAMP_NF:
+        pytest.skip("tile without the clamped epilogue")
+    g = torch.Generator(device="cuda").manual_seed(M + K + form)
+    x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+    w = (torch.randn(2 * N if glu else N, K, device="cuda", generator=g) * 0.05).to(torch.bfloat16)
+    res = torch.randn(M, N, device="cuda", generator=g).to(torch.bfloat16) if epi == "residual" else None
+    out = torch.full((M, N), float("nan"), device="cuda", dtype=torch.bfloat16)
+    G.xd_gemm(x, w, epi, residual=res, out=out, form=form, limit=7.0)
+    ref = _ref(x, w, epi, res)
+    if epi == "relu2":
+        ref = ref.relu().square()
+    elif epi == "clamped":
+        gate, up = ref[:, :N].clamp(max=7.0), ref[:, N:].clamp(-7.0, 7.0)
+        ref = gate * torch.sigmoid(1.702 * gate) * (up + 1)
+    _check(out, ref)
+
+
+@pytest.mark.parametrize("M,N,K", [(129, 32000, 2048), (160, 12800, 2048), (192, 20480, 2048), (224, 32000, 2048)])
+def test_linear_on_one_tall_tile(hipk, M, N, K):
+    """The rule's products, aligned ones on its form, others as before."""
+    g = torch.Generator(device="cuda").manual_seed(M)
+    buf = torch.randn(M, K + 8, device="cuda", generator=g).to(torch.bfloat16)
+    w = (torch.randn(N, K, device="cuda", generator=g) * 0.02).to(torch.bfloat16)
+    for x in (buf[:, :K].contiguous(), buf[:, 8:], buf[:, 1:K + 1]):
+        assert G.route(M, N, K, x.stride(0)) == ("xd", G.tall_form(M, N, K))
+        assert _rel(G.linear(x, w), x.float() @ w.float().t()) < 1e-2
+
+
 @pytest.mark.parametrize("epi", ["store", "residual", "silu"])
 @pytest.mark.parametrize("form", [1141, 1161, 1241, 1244, 1261, 1281, 1282])
 def test_xd_gemm_nontemporal_weights_match_fp32(hipk, epi, form):

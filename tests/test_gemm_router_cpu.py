@@ -20,6 +20,21 @@ def test_nontemporal_forms_only_for_built_tiles():
     assert not G.xd_supported(256, 1536, 2048, 2244)  # not a form
 
 
+@pytest.mark.parametrize("M,N,K,glu,want", [
+    (129, 14336, 4096, True, 1341), (160, 14336, 4096, True, 1341), (161, 14336, 4096, True, 1441), (193, 14336, 4096, True, 1541),
+    (224, 32000, 2048, False, 1541), (160, 7168, 2048, True, 1321), (161, 7168, 2048, True, 0), (128, 32000, 4096, False, 0),
+    (225, 32000, 4096, False, 0), (160, 28672, 4096, True, 0), (160, 32000, 1024, False, 0), (160, 8448, 2048, False, 0),
+    (160, 32016, 4096, False, 0),
+])
+def test_tall_tiles_rule(monkeypatch, M, N, K, glu, want):
+    monkeypatch.setattr(G, "_xd_nt", True)
+    monkeypatch.setattr(G, "_xd_enabled", True)
+    assert G.tall_form(M, N, K, glu) == want
+    if want:
+        assert not G.xd_supported(G.XD_ROWS[want // 100 % 10] + 1, N, K, want, glu)  # one row tile
+        assert not G.xd_supported(M, N, K, want - 1000, glu) and not G.xd_supported(M, N, K, want + 1, glu)
+
+
 @pytest.mark.parametrize("M,form,want", [
     (256, 244, 1244),   # one 256-row tile: every weight byte read once
     (128, 141, 1141),
