@@ -701,10 +701,13 @@ using Xd3x2 = XdCfg<3, 2, 5, false, true>;
 using Xd3x4 = XdCfg<3, 4, 4, false, true>;
 using Xd4x4 = XdCfg<4, 4, 4, false, true>;
 using Xd5x4 = XdCfg<5, 4, 3, false, true>;
+// 128 x 256, grouped
+template <bool NT = false>
+using Xd1x8 = XdCfg<1, 8, 3, false, NT>;
 
 int xd_stages(int mt, int nf) {
   if (mt == 0) return nf == 1 || nf == 2 ? 6 : (nf == 4 ? 4 : 0);
-  if (mt == 1) return nf == 6 ? 3 : (nf == 2 || nf == 4 ? 4 : 0);
+  if (mt == 1) return nf == 6 || nf == 8 ? 3 : (nf == 2 || nf == 4 ? 4 : 0);
   if (mt >= 3 && mt <= 5) return nf == 4 ? (mt == 5 ? 3 : 4) : nf == 2 && mt == 3 ? 5 : 0;
   if (mt == 2) return nf == 4 ? 3 : (nf == 6 || nf == 8 ? 2 : 0);
   return 0;
@@ -749,10 +752,12 @@ int xd_dispatch(const XdParams& p, int mt, int nf, bool nt, int epi, hipStream_t
   }
 }
 
-// grouped (MoE) mode: the 128 x 128, 256 x 128 and 256 x 256 tiles
+// grouped (MoE) mode: the 128 x 128, 128 x 256, 256 x 128 and 256 x 256 tiles
 template <bool SP>
 int xd_dispatch_g(const XdParams& p, int mt, int nf, bool nt, int epi, hipStream_t st) {
   switch (mt * 10 + nf + (nt ? 100 : 0)) {
+    case 18: if constexpr (!SP) return xd_launch_g<Xd1x8<>>(p, epi, st); else return -1;
+    case 118: if constexpr (!SP) return xd_launch_g<Xd1x8<true>>(p, epi, st); else return -1;
     case 14: return xd_launch_g<Xd1x4<SP>>(p, epi, st);
     case 24: return xd_launch_g<Xd2x4<SP>>(p, epi, st);
     case 28: return xd_launch_g<Xd2x8<SP>>(p, epi, st);
@@ -897,7 +902,7 @@ int configure_gemm_xd() {
   const int g = xd_cfg_g<Xd1x4<false>>() | xd_cfg_g<Xd2x4<false>>() | xd_cfg_g<Xd2x8<false>>() |
                 xd_cfg_g<Xd1x4<true>>() | xd_cfg_g<Xd2x4<true>>() | xd_cfg_g<Xd2x8<true>>() |
                 xd_cfg_g<Xd1x4<false, true>>() | xd_cfg_g<Xd2x4<false, true>>() |
-                xd_cfg_g<Xd2x8<false, true>>() | xd_cfg_g<Xd1x4<true, true>>() |
+                xd_cfg_g<Xd1x8<>>() | xd_cfg_g<Xd1x8<true>>() | xd_cfg_g<Xd2x8<false, true>>() | xd_cfg_g<Xd1x4<true, true>>() |
                 xd_cfg_g<Xd2x4<true, true>>() | xd_cfg_g<Xd2x8<true, true>>();
   if (g) return g;
   return xd_cfg<Xd3x2>() | xd_cfg<Xd3x4>() | xd_cfg<Xd4x4>() | xd_cfg<Xd5x4>() | xd_cfg<Xd0x1<>>() | xd_cfg<Xd0x2<>>() | xd_cfg<Xd0x4<>>() | xd_cfg<Xd0x1<true>>() | xd_cfg<Xd0x2<true>>() |

@@ -24,6 +24,9 @@
 // loop), 16 MFMA 16x16x32 per wave per k-step.
 #include "common.h"
 #include "launchers.h"
+
+#include <algorithm>
+#include <cmath>
 #include "typed.h"
 
 #include <initializer_list>
@@ -1070,10 +1073,10 @@ __global__ __launch_bounds__(256) void moe_combine_norm_kernel(
 // and reduction K (the 1x4 / 2x4 / 2x8 tiles launch_gemm_xd_grouped builds).
 static bool moe_xd_ok(int form, int N, int K, bool glu) {
   const int mt = (form % 1000) / 100, nf = form / 10 % 10, sk = form % 10;
-  const int st = mt == 1 ? (nf == 4 ? 4 : 0) : (mt == 2 ? (nf == 4 ? 3 : (nf == 8 ? 2 : 0)) : 0);
+  const int st = mt == 1 ? (nf == 4 ? 4 : nf == 8 ? 3 : 0) : (mt == 2 ? (nf == 4 ? 3 : (nf == 8 ? 2 : 0)) : 0);
   if (st == 0 || sk < 1 || sk > 8 || form >= 2000) return false;
   const int tno = glu ? 16 * nf : 32 * nf;
-  return N % tno == 0 && K % 64 == 0 && K / 64 / sk > st;
+  return N % tno == 0 && K % 64 == 0 && K / 64 / sk > st && (sk == 1 || mt != 1 || nf != 8);
 }
 
 // xd form (mt * 100 + nf * 10 + splitk, + 1000 non-temporal weights) -> launcher fields
@@ -1083,12 +1086,39 @@ static void moe_xd_form(int form, int& mt, int& nf, int& sk) {
   sk = form % 10;
 }
 
+// Row tiles of bm rows that an expert of `rows` rows in the mean has, if tokens choose by themselves (a spread of
+// sqrt(rows)).
+static double moe_tiles(double rows, int bm) {
+  const double s = sqrt(rows > 1. ? rows : 1.);
+  double t = 1.;
+  for (int at = bm; at < rows + 2 * s; at += bm) t += std::min(1., 0.5 + (rows - at) / (4 * s));
+  return t;
+}
+// us of both products of E experts in gemm_xd's grouped tiles of bm x 256: whole rounds of 256 workgroups, each the time of
+// a tile's products, 1.1 PFLOP/s by the whole chip in 128 rows and 1.35 in 256.
+static double moe_xd_us(int E, double rows, int bm, int H, int I, bool glu) {
+  const double tiles = E * moe_tiles(rows, bm), per = bm == 128 ? 0.0146 : 0.0244;
+  const double up = ceil(tiles * (glu ? 2 * I : I) / 65536 - 0.02), down = ceil(tiles * H / 65536 - 0.02);
+  const bool split = bm == 256 && rows < kMoeW4Rows && tiles * H <= 32768;  // down in two K slices (launch_moe)
+  return up * (per * H + 3) + down * (split ? per * I / 2 + 20 : per * I + 3);
+}
+// Whether tiles of 128 rows are the faster ones: fewer rows of padding, or a round less.  us of a layer, 256 rows (variant
+// 3 or 4) / 128: 20 x 2048 x 1792, squared relu, 640 tokens 150 / 102, 1536 222 / 156, 896 127 / 148; 20 x 4096 x 3584, 640 tokens
+// 385 / 313, 1536 556 / 495; 16 x 4096 x 3584, gated, 640 tokens 337 / 388, 1152 572 / 550, 1536 633 / 651.  whole: gemm_xd
+// loads 16-byte pieces at 32-bit offsets of x and of an expert's matrix, which gemm_w4 behind its gather need not.
+static bool moe_half_tiles(int T, int E, int rows, int H, int I, bool glu, bool whole) {
+  const int64_t most = 1 << 30;
+  return whole && (int64_t)T * H < most && (int64_t)(I + 256) * H < most && (int64_t)(H + 256) * I < most && moe_xd_ok(181, I, H, glu) && moe_xd_ok(181, H, I, false) &&
+         moe_xd_us(E, rows, 128, H, I, glu) < 0.96 * moe_xd_us(E, rows, 256, H, I, glu);
+}
+
 // The variant of a layer of T tokens and P pairs over E experts, bf16; whole: rows and weights start at 16 bytes.
 //   * 4 from one 256-row tile per expert (gemm_w4's persistent 256 x 256 tiles over
 //     expert-ordered rows; Mixtral shapes, profiles/r6j: 770 / 917 / 1061 TF/s at T = 1024 /
-//     2048 / 4096 against 703 / 841 / 1019 on variant 3).
-//   * below it the ring, to where most experts still fit one of its entries (100 rows 92 / 121 of variant 3, 128
-//     rows 134 / 123), but for a few rows per expert where gemm_stream's form takes the sizes: fewer pairs than experts (us of a layer,
+//     2048 / 4096 against 703 / 841 / 1019 on variant 3), but where tiles of 128 rows are the faster ones.
+//   * below it the ring, to where most experts still fit one of its entries (100 rows 92 / 121 of variant 3, 112 105 / 125,
+//     128 134 / 123; many experts, of which some need a second entry, leave fewer workgroups to each: 128 x 2048 x 768, 112 rows
+//     506 / 470), but for a few rows per expert where gemm_stream's form takes the sizes: fewer pairs than experts (us of a layer,
 //     variants 5 / 6: 16 x 2048 x 1792, 1 token 30.5 / 46.0, 2 39.6 / 48.6; 4 61.9 / 59.1), and wide experts, gated (16 x 4096
 //     x 3584, 13 tokens 226.6 / 229.1) or with a row each (20 x 4096 x 3584, 8 tokens 157.0 / 158.5; 16 197 / 187).  (wide:
 //     of the four widths that gemm_stream's form has, the upper two.)  Elsewhere a few pairs of large experts: variant 3,
@@ -1099,9 +1129,9 @@ static void moe_xd_form(int form, int& mt, int& nf, int& sk) {
 int moe_variant(int T, int P, int E, int H, int I, bool glu, bool whole) {
   const int rows_e = P / E, stream_mt = stream_moe_tiles(rows_e, H, I, glu);
   const bool ring_ok = whole && ring_moe_ok(T, P, H, I, glu), wide = H > 2048 || I > 2048;
-  if (rows_e >= kMoeW4Rows) return 4;
+  if (rows_e >= kMoeW4Rows) return rows_e < 768 && moe_half_tiles(T, E, rows_e, H, I, glu, whole) ? 3 : 4;
   if (stream_mt && (!ring_ok || (stream_mt == 1 && (rows_e == 0 || (wide && (glu || rows_e < 2)))))) return 5;
-  if (ring_ok && rows_e <= 104 && (P >= 8 || P > E || (int64_t)H * I < 6 << 20)) return 6;
+  if (ring_ok && rows_e <= (E <= 64 ? 112 : 104) && (P >= 8 || P > E || (int64_t)H * I < 6 << 20)) return 6;
   // shapes past the ring's offsets, and sizes between it and gemm_w4
   return rows_e >= 96 || (int64_t)H * I >= 6 << 20 ? 3 : 1;
 }
@@ -1156,26 +1186,31 @@ int launch_moe(void* out, const void* x, const void* router_logits, const void* 
     variant = 3;  // a down form requested for variant 3 (DRTC_MOE_DN_FORM) keeps its variant
   }
   if (variant == 3) {
-    // 256-row tiles from ~1.5 tiles of rows per expert, else 128-row; 256 gated columns
-    // (128 outputs) for gate_up where I allows; down with split-K 2 while the grid is below
-    // ~2 rounds of CUs; non-temporal weights where an expert's rows fit one tile (each
+    // 256-row tiles from ~1.5 tiles of rows per expert, but where moe_half_tiles says 128, else 128-row; 256 gated columns
+    // (128 outputs) for gate_up where I allows; down with split-K 2 where that leaves one round of
+    // CUs; non-temporal weights where an expert's rows fit one tile (each
     // weight byte is read by one workgroup)
     const bool gu_auto = gu_form == 0;  // an explicitly requested form runs as given
-    if (gu_auto) {
+    const bool half = gu_auto && dn_form == 0 && rows_e >= 96 && moe_half_tiles(T, e_local, rows_e, H, I, glu, whole);
+    if (half) {
+      const int nt = moe_tiles(rows_e, 128) < 1.1 ? 1000 : 0;
+      gu_form = dn_form = 181 + nt;
+    } else if (gu_auto) {
       for (int f : rows_e >= 96 ? std::initializer_list<int>{281, 241} :
                                   std::initializer_list<int>{141})
         if (moe_xd_ok(f, I, H, glu)) { gu_form = f; break; }
     }
     const int mt0 = (gu_form % 1000) / 100, bm0 = 128 * mt0;
-    if (gu_auto && gu_form && gu_form < 1000 && rows_e <= bm0) gu_form += 1000;
+    if (gu_auto && !half && gu_form && gu_form < 1000 && rows_e <= bm0) gu_form += 1000;
     if (dn_form == 0 && gu_form) {
       const int64_t max_t = (P + bm0 - 1) / bm0 + e_local;
       for (int f : mt0 == 2 ? std::initializer_list<int>{282, 281, 242, 241} :
                               std::initializer_list<int>{142, 141}) {
-        // split-K 2 while the grid is below ~2 rounds of CUs and its fp32 partial slots fit
+        // split-K 2 while its workgroups are one round of CUs and the fp32 partial slots fit (20 x 2048 x 1792, squared
+        // relu, 640 tokens, 160 tiles: 150 us split, 127 not)
         const int nf = f / 10 % 10;
         const int64_t tiles = max_t * (H / (32 * nf));
-        const bool split = tiles < 512 && slab != nullptr && n_counters >= 2 * tiles + 2 &&
+        const bool split = 2 * e_local * moe_tiles(rows_e, bm0) * (H / (32 * nf)) <= 256 && slab != nullptr && n_counters >= 2 * tiles + 2 &&
                            slab_bytes >= tiles * 2 * bm0 * (32 * nf) * 4;
         if (!split && f % 10 > 1) continue;
         if (moe_xd_ok(f, H, I, false)) { dn_form = f; break; }

@@ -746,6 +746,35 @@ def test_fused_moe_grouped_xd_forms(hipk, T, H, I, E, k, gu, dn, act):
     G.check_splitk_fault()
 
 
+@pytest.mark.parametrize("T,H,I,E,k,gu,dn", [
+    (300, 512, 256, 4, 2, 181, 181),     # 150 rows an expert: a second tile of a few rows
+    (256, 256, 512, 4, 2, 1181, 181),    # about a whole tile
+    (64, 512, 768, 8, 2, 1181, 1181),    # few rows, more column tiles than one
+    (3, 512, 256, 16, 1, 181, 181),      # experts without a row
+])
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh", "relu2"])
+def test_fused_moe_128_x_256_tiles(hipk, T, H, I, E, k, gu, dn, act):
+    """Experts in gemm_xd's tiles of 128 x 256: against the fp32 reference."""
+    x, lg, wgu, wdn = _moe_inputs(T, H, I, E, seed=T)
+    if act == "relu2":
+        wgu = wgu[:, :I].contiguous()
+    y = ops.fused_moe(x, lg, wgu, wdn, k, act, variant=3, gu_form=gu, dn_form=dn)
+    _close(y, ops.fused_moe_ref(x, lg, wgu, wdn, k, act), 3e-2, 3e-2, f"moe xd {gu}/{dn}")
+
+
+def test_tile_height_of_the_experts(hipk):
+    """Rows per expert a little above a multiple of 256: tiles of 128 rows (variant 3), but for rows or weights off 16
+    bytes and sizes past 32-bit offsets; the layer by itself against the reference at both sides of the rule."""
+    v = lambda T, k, E, H, I, glu=True, whole=True: hipk.moe_variant(T, T * k, E, H, I, glu, whole)
+    assert [v(T, 4, 20, 2048, 1792, False) for T in (1408, 1536, 3072)] == [3, 3, 4]
+    assert [v(T, 4, 16, 4096, 3584) for T in (1088, 1152, 2048, 12288)] == [3, 3, 4, 4]
+    assert v(1536, 4, 20, 2048, 1792, False, False) == 4 and v(600000, 1, 2048, 2048, 1792, False) == 4
+    assert [v(T, 4, 16, 2048, 1792) for T in (448, 452)] == [6, 3] and [v(T, 8, 128, 2048, 768) for T in (1664, 1680)] == [6, 3]
+    for T in (600, 1408):
+        x, lg, wgu, wdn = _moe_inputs(T, 512, 512, 20, seed=T)
+        _close(ops.fused_moe(x, lg, wgu, wdn, 4, "silu"), ops.fused_moe_ref(x, lg, wgu, wdn, 4, "silu"), 3e-2, 3e-2, "moe")
+
+
 @pytest.mark.parametrize("T,H,I,E,k,e_off,e_local", [
     (4096, 1024, 512, 8, 2, 0, 8),       # ~1k rows per expert: the auto pick
     (3000, 512, 384, 4, 2, 0, 4),        # row tails in every expert
