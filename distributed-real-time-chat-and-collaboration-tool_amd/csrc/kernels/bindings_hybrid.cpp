@@ -125,13 +125,13 @@ void bind_hybrid(py::module_& m) {
                           u64 st) {
     return drtc::launch_act_glu_f32(P<float>(out), P<float>(gu), T, I, stride, act, limit, S(st));
   });
-  m.def("latent_prep", [](int f32, const py::dict& d, u64 st) {
+  m.def("latent_prep", [](int f32, const py::dict& d, u64 w, u64 st) {  // w: also the queries' way down (decode)
     const Fields f{d};
     drtc::LatentPrepArgs a{};
     PTR(proj); VAL(ldp); VAL(off_kv); VAL(H); VAL(dim); VAL(rot); VAL(rot_dims); VAL(R); VAL(LW);
     PTR(norm_w); VAL(eps); PTR(cos_sin); PTR(positions); PTR(slots); PTR(lat); PTR(cache);
     PTR(qa); VAL(rows);
-    return drtc::launch_latent_prep(f32, a, S(st));
+    return w ? drtc::launch_latent_front(f32, a, P<void>(w), S(st)) : drtc::launch_latent_prep(f32, a, S(st));
   });
   m.def("latent_gather", [](u64 out, u64 cache, u64 slots, int rows, int row_bytes, u64 st) {
     return drtc::launch_latent_gather(P<void>(out), P<void>(cache), P<const int64_t>(slots), rows,
@@ -146,13 +146,14 @@ void bind_hybrid(py::module_& m) {
     PTR(gate); VAL(ldg);
     return drtc::launch_latent_prefill(f32, a, S(st));
   });
-  m.def("latent_decode", [](int f32, const py::dict& d, u64 st) {
+  m.def("latent_decode", [](int f32, const py::dict& d, u64 y, u64 w, int N, int64_t yb, int64_t yh, u64 st) {
     const Fields f{d};
     drtc::LatentDecodeArgs a{};
     PTR(out); PTR(part_o); PTR(part_ml); PTR(qa); PTR(cache); PTR(block_tables); VAL(bt_stride);
     PTR(context_lens); VAL(B); VAL(H); VAL(R); VAL(LW); VAL(window); VAL(tiles_per_split);
     VAL(nsplits); VAL(scale); PTR(sink); PTR(gate); VAL(ldg);
-    return drtc::launch_latent_decode(f32, a, S(st));
+    return w ? drtc::launch_latent_decode_up(f32, a, P<void>(y), P<void>(w), N, yb, yh, S(st))
+             : drtc::launch_latent_decode(f32, a, S(st));
   });
   m.def("head_gemm", [](int f32, u64 y, u64 x, u64 w, int B, int H, int N, int K, int64_t yb,
                         int64_t yh, int64_t xb, int64_t xh, u64 st) {

@@ -32,6 +32,7 @@ struct LatentPrepArgs {
   int rows;
 };
 int launch_latent_prep(int f32, const LatentPrepArgs& a, hipStream_t st);
+int launch_latent_front(int f32, const LatentPrepArgs& a, const void* w, hipStream_t st);
 int launch_latent_gather(void* out, const void* cache, const int64_t* slots, int rows,
                          int row_bytes, hipStream_t st);
 
@@ -73,6 +74,8 @@ struct LatentDecodeArgs {
   int ldg;
 };
 int launch_latent_decode(int f32, const LatentDecodeArgs& a, hipStream_t st);
+int launch_latent_decode_up(int f32, const LatentDecodeArgs& a, void* y, const void* w, int N, int64_t yb, int64_t yh,
+                            hipStream_t st);
 int launch_head_gemm(int f32, void* y, const void* x, const void* w, int B, int H, int N, int K,
                      int64_t yb, int64_t yh, int64_t xb, int64_t xh, hipStream_t st);
 int configure_latent();

@@ -64,9 +64,9 @@ DRTC_DEVICE void lat_store(T* p, const float (&v)[V]) {
 }
 
 template <class T, int V>
-__global__ __launch_bounds__(256) void latent_prep_kernel(LatentPrepArgs a) {
+DRTC_DEVICE void latent_prep_row(const LatentPrepArgs& a, int row) {
   __shared__ float red[16];
-  const int row = blockIdx.x, tid = threadIdx.x;
+  const int tid = threadIdx.x;
   T* pr = (T*)a.proj + (int64_t)row * a.ldp;
   const T* kv = pr + a.off_kv;
   const int half = a.rot_dims >> 1;
@@ -145,10 +145,22 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(LatentPrepArgs a) {
   }
 }
 
+template <class T, int V>
+__global__ __launch_bounds__(256) void latent_prep_kernel(LatentPrepArgs a) {
+  latent_prep_row<T, V>(a, blockIdx.x);
+}
+
+static bool lat_prep_whole(const LatentPrepArgs& a) {  // vectors of 8
+  return a.R % 8 == 0 && a.rot % 8 == 0 && a.dim % 8 == 0 && a.ldp % 8 == 0 && (a.off_kv < 0 || a.off_kv % 8 == 0) &&
+         a.LW % 8 == 0;
+}
+static bool lat_prep_takes(const LatentPrepArgs& a) {
+  return a.rot_dims <= a.rot && a.rot_dims % 2 == 0 && a.R + a.rot <= a.LW && a.R % 2 == 0 && a.rot % 2 == 0 && a.LW % 2 == 0;
+}
+
 template <class T>
 static void lat_prep_t(const LatentPrepArgs& a, hipStream_t st) {
-  if (a.R % 8 == 0 && a.rot % 8 == 0 && a.dim % 8 == 0 && a.ldp % 8 == 0 &&
-      (a.off_kv < 0 || a.off_kv % 8 == 0) && a.LW % 8 == 0)
+  if (lat_prep_whole(a))
     latent_prep_kernel<T, 8><<<dim3(a.rows), dim3(256), 0, st>>>(a);
   else
     latent_prep_kernel<T, 2><<<dim3(a.rows), dim3(256), 0, st>>>(a);
@@ -156,9 +168,7 @@ static void lat_prep_t(const LatentPrepArgs& a, hipStream_t st) {
 
 int launch_latent_prep(int f32, const LatentPrepArgs& a, hipStream_t st) {
   if (a.rows == 0) return 0;
-  if (a.rot_dims > a.rot || a.rot_dims % 2 || a.R + a.rot > a.LW || a.R % 2 || a.rot % 2 ||
-      a.LW % 2)
-    return -1;
+  if (!lat_prep_takes(a)) return -1;
   if (f32) lat_prep_t<float>(a, st);
   else lat_prep_t<bf16_t>(a, st);
   return (int)hipGetLastError();
@@ -883,15 +893,23 @@ static void lat_decode_h(const LatentDecodeArgs& a, hipStream_t st) {
   else lat_decode_go<RT, 4, 2>(a, st);
 }
 
+static int lat_decode_need(const LatentDecodeArgs& a) { return std::max((a.R + 63) / 64, (a.LW / 32 - 1) / 2); }
+static bool lat_decode_mfma(int f32, const LatentDecodeArgs& a) {
+  return !f32 && a.R % 8 == 0 && a.LW % 32 == 0 && lat_decode_need(a) <= 8 && a.R <= 512;
+}
+static bool lat_decode_split(int f32, const LatentDecodeArgs& a) { return lat_decode_mfma(f32, a) && a.nsplits > 1; }
+static void lat_decode_parts(const LatentDecodeArgs& a, hipStream_t st) {
+  const int need = lat_decode_need(a);
+  if (need <= 1) lat_decode_h<1>(a, st);
+  else if (need <= 2) lat_decode_h<2>(a, st);
+  else if (need <= 4) lat_decode_h<4>(a, st);
+  else lat_decode_h<8>(a, st);
+}
+
 int launch_latent_decode(int f32, const LatentDecodeArgs& a, hipStream_t st) {
   if (a.B == 0) return 0;
-  const int ks = a.LW / 32;
-  const int need = std::max((a.R + 63) / 64, (ks - 1) / 2);
-  if (!f32 && a.R % 8 == 0 && a.LW % 32 == 0 && need <= 8 && a.R <= 512) {
-    if (need <= 1) lat_decode_h<1>(a, st);
-    else if (need <= 2) lat_decode_h<2>(a, st);
-    else if (need <= 4) lat_decode_h<4>(a, st);
-    else lat_decode_h<8>(a, st);
+  if (lat_decode_mfma(f32, a)) {
+    lat_decode_parts(a, st);
     if (a.nsplits > 1) latent_merge_kernel<<<dim3(a.B, a.H), dim3(128), 0, st>>>(a);
   } else {
     if (a.R > 1024) return -1;
@@ -906,14 +924,19 @@ int launch_latent_decode(int f32, const LatentDecodeArgs& a, hipStream_t st) {
 // workgroup sharing each weight fragment; operands straight from global memory (the weights
 // are read once per 64 rows and stay in L2).
 // WHOLE: K % 128 == 0 - four steps' loads ahead of their products.
+struct HeadGemm {
+  bf16_t* y;
+  const bf16_t *x, *w;
+  int B, N, K;
+  int64_t yb, yh, xb, xh;
+};
 template <int NBT, bool WHOLE>
-__global__ __launch_bounds__(256) void head_gemm_kernel(
-    bf16_t* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, int B,
-    int N, int K, int64_t yb, int64_t yh, int64_t xb, int64_t xh) {
-  const int h = blockIdx.z, b0 = blockIdx.y * 16 * NBT;
+DRTC_DEVICE void head_gemm_tile(const HeadGemm& q, int tile, int rows, int h) {
+  const auto [y, x, w, B, N, K, yb, yh, xb, xh] = q;
+  const int b0 = rows * 16 * NBT;
   const int wv = wave_id_uniform(), lane = threadIdx.x & 63;
   const int col = lane & 15, g = lane >> 4;
-  const int n0 = (blockIdx.x * 4 + wv) * 16;
+  const int n0 = (tile * 4 + wv) * 16;
   if (n0 >= N) return;
   const bf16_t* wr = w + ((int64_t)h * N + min(n0 + col, N - 1)) * K;
   const bf16_t* xr[NBT];
@@ -962,9 +985,8 @@ __global__ __launch_bounds__(256) void head_gemm_kernel(
 // 128 of K, their sums meet in LDS: one round trip to memory where a wave alone makes K / 128.  128 dims from 512, us:
 // 200 rows of 16 heads 11.3 -> 7.2, 64 of 32 11.2 -> 4.8.
 template <int NBT>
-__global__ __launch_bounds__(256) void head_gemm_shared_kernel(
-    bf16_t* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, int B,
-    int N, int K, int64_t yb, int64_t yh, int64_t xb, int64_t xh) {
+__global__ __launch_bounds__(256) void head_gemm_shared_kernel(HeadGemm q) {
+  const auto [y, x, w, B, N, K, yb, yh, xb, xh] = q;
   __shared__ f32x4 sums[4][NBT][64];
   const int h = blockIdx.z, b0 = blockIdx.y * 16 * NBT, n0 = blockIdx.x * 16;
   const int wv = wave_id_uniform(), lane = threadIdx.x & 63;
@@ -1004,18 +1026,114 @@ __global__ __launch_bounds__(256) void head_gemm_shared_kernel(
   }
 }
 
+// The shared form for up to 16 rows behind a split window (LatentDecodeArgs a), K = a.R: each workgroup adds the
+// splits up itself, into LDS, while its weights are on their way.
+constexpr int kUpParts = 1024;  // rows times splits
+template <int KMAX>
+__global__ __launch_bounds__(256) void latent_up_kernel(LatentDecodeArgs a, HeadGemm q) {
+  __shared__ f32x4 sums[4][64];
+  __shared__ float factor[kUpParts];
+  __shared__ int count[16];
+  __shared__ __attribute__((aligned(16))) bf16_t xs[16][KMAX + 8];
+  const int h = blockIdx.y, n0 = blockIdx.x * 16, K = q.K, N = q.N, B = q.B;
+  const int wv = wave_id_uniform(), lane = threadIdx.x & 63;
+  const int col = lane & 15, g = lane >> 4;
+  const bf16_t* wr = q.w + ((int64_t)h * N + min(n0 + col, N - 1)) * K + 128 * wv + 8 * g;
+  bf16x8 wf[KMAX / 512][4];
+#pragma unroll
+  for (int j = 0; j < KMAX / 512; ++j)
+#pragma unroll
+    for (int s = 0; s < 4; ++s) wf[j][s] = 128 * wv + 512 * j < K ? load_bf16x8(wr + 512 * j + 32 * s) : zero8();
+  for (int b = wv; b < B; b += 4) {
+    const int ctx = a.context_lens[b], lo = a.window > 0 ? max(0, ctx - a.window) : 0;
+    const int n = ctx <= 0 ? 0 : ((ctx + kLB - 1) / kLB - lo / kLB + a.tiles_per_split - 1) / a.tiles_per_split;
+    const float* ml = a.part_ml + ((int64_t)b * a.H + h) * a.nsplits * 2;
+    if (lane == 0) count[b] = n;
+    if (n < 2) continue;
+    float top = kNegBig, l = 0.f;
+    for (int p = lane; p < n; p += 64) top = fmaxf(top, ml[2 * p]);
+    top = wave_max(top);
+    for (int p = lane; p < n; p += 64) l += ml[2 * p + 1] * fast_exp2(ml[2 * p] - top);
+    l = wave_sum(l) + (a.sink ? fast_exp2(a.sink[h] * kLog2e - top) : 0.f);
+    const float inv = head_gate<bf16_t>(a.gate, (int64_t)b * a.ldg + h) / l;
+    for (int p = lane; p < n; p += 64) factor[b * a.nsplits + p] = fast_exp2(ml[2 * p] - top) * inv;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < B * (K / 4); i += 256) {
+    const int b = i / (K / 4), d = 4 * (i - b * (K / 4)), n = count[b];
+    const int64_t row = (int64_t)b * a.H + h;
+    bf16x4 v;
+    if (n == 1) {  // (written as it is)
+      v = load_bf16x4((const bf16_t*)a.out + row * K + d);
+    } else {
+      const float* po = a.part_o + row * a.nsplits * K + d;
+      f32x4 s = {0.f, 0.f, 0.f, 0.f};
+      for (int p0 = 0; p0 < n; p0 += 8) {  // eight on their way
+        f32x4 t[8];
+#pragma unroll
+        for (int p = 0; p < 8; ++p) t[p] = *reinterpret_cast<const f32x4*>(po + (int64_t)min(p0 + p, n - 1) * K);
+#pragma unroll
+        for (int p = 0; p < 8; ++p) s += t[p] * (p0 + p < n ? factor[b * a.nsplits + p0 + p] : 0.f);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = f2bf(s[r]);
+    }
+    *reinterpret_cast<bf16x4*>(&xs[b][d]) = v;
+  }
+  __syncthreads();
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < KMAX / 512; ++j) {
+    if (128 * wv + 512 * j >= K) continue;
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      acc = mfma16(wf[j][s], load_bf16x8(&xs[min(col, B - 1)][128 * wv + 512 * j + 32 * s + 8 * g]), acc);
+  }
+  sums[wv][lane] = acc;
+  __syncthreads();
+  if (wv) return;
+  const f32x4 s = (sums[0][lane] + sums[1][lane]) + (sums[2][lane] + sums[3][lane]);
+  const int n = n0 + 4 * g;
+  if (col < B && n < N) {
+    bf16x4 v;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = f2bf(s[r]);
+    *reinterpret_cast<bf16x4*>(q.y + col * q.yb + h * q.yh + n) = v;
+  }
+}
+template <int NBT, bool WHOLE>
+__global__ __launch_bounds__(256) void head_gemm_kernel(HeadGemm q) {
+  head_gemm_tile<NBT, WHOLE>(q, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+
+// A decode step's preparation and its queries' way down into the latent space, which read and write other columns: the
+// rows' workgroups, then the product's.  Both are a round trip to memory and their launch, and one of them is saved: 2.2 us
+// a layer at 1 to 200 rows.
 template <int NBT>
-static void head_gemm_go(bf16_t* y, const bf16_t* x, const bf16_t* w, int B, int H, int N, int K,
-                         int64_t yb, int64_t yh, int64_t xb, int64_t xh, hipStream_t st) {
-  const dim3 grid((N + 63) / 64, (B + 16 * NBT - 1) / (16 * NBT), H);
+__global__ __launch_bounds__(256) void latent_front_kernel(LatentPrepArgs a, HeadGemm q) {
+  if ((int)blockIdx.x < a.rows) {
+    latent_prep_row<bf16_t, 8>(a, blockIdx.x);
+    return;
+  }
+  const int i = blockIdx.x - a.rows, gx = (q.N + 63) / 64, t = i / gx, gy = (q.B + 16 * NBT - 1) / (16 * NBT);
+  head_gemm_tile<NBT, true>(q, i - t * gx, t % gy, t / gy);
+}
+
+static bool head_gemm_shares(const HeadGemm& q, int H, int nbt) {
   // shared where a CU would have half a workgroup: 128 dims from 512 of 32 heads, 128 rows 11.4 / 8.4 us, 200 (one a
   // CU) 12.4 / 13.7; with fewer rows to a workgroup up to one a CU: 256 dims of 64 heads, 32 rows 8.8 / 8.3
-  if (K % 128 == 0 && K >= 256 && (int64_t)grid.x * grid.y * H <= (NBT == 4 ? 128 : 256))
-    head_gemm_shared_kernel<NBT><<<dim3((N + 15) / 16, grid.y, H), dim3(256), 0, st>>>(y, x, w, B, N, K, yb, yh, xb, xh);
-  else if (K % 128 == 0)
-    head_gemm_kernel<NBT, true><<<grid, dim3(256), 0, st>>>(y, x, w, B, N, K, yb, yh, xb, xh);
+  return q.K % 128 == 0 && q.K >= 256 &&
+         (int64_t)((q.N + 63) / 64) * ((q.B + 16 * nbt - 1) / (16 * nbt)) * H <= (nbt == 4 ? 128 : 256);
+}
+template <int NBT>
+static void head_gemm_go(const HeadGemm& q, int H, hipStream_t st) {
+  const dim3 grid((q.N + 63) / 64, (q.B + 16 * NBT - 1) / (16 * NBT), H);
+  if (head_gemm_shares(q, H, NBT))
+    head_gemm_shared_kernel<NBT><<<dim3((q.N + 15) / 16, grid.y, H), dim3(256), 0, st>>>(q);
+  else if (q.K % 128 == 0)
+    head_gemm_kernel<NBT, true><<<grid, dim3(256), 0, st>>>(q);
   else
-    head_gemm_kernel<NBT, false><<<grid, dim3(256), 0, st>>>(y, x, w, B, N, K, yb, yh, xb, xh);
+    head_gemm_kernel<NBT, false><<<grid, dim3(256), 0, st>>>(q);
 }
 
 template <class T>
@@ -1031,15 +1149,17 @@ __global__ __launch_bounds__(256) void head_gemm_any_kernel(
   y[b * yb + h * yh + n] = from_f32<T>(s);
 }
 
+static bool head_gemm_whole(int N, int K, int64_t yb, int64_t yh, int64_t xb, int64_t xh) {
+  return K % 8 == 0 && N % 4 == 0 && yb % 4 == 0 && yh % 4 == 0 && xb % 8 == 0 && xh % 8 == 0;
+}
 int launch_head_gemm(int f32, void* y, const void* x, const void* w, int B, int H, int N, int K,
                      int64_t yb, int64_t yh, int64_t xb, int64_t xh, hipStream_t st) {
   if (B == 0) return 0;
-  if (!f32 && K % 8 == 0 && N % 4 == 0 && yb % 4 == 0 && yh % 4 == 0 && xb % 8 == 0 &&
-      xh % 8 == 0) {
-    const bf16_t *xx = (const bf16_t*)x, *ww = (const bf16_t*)w;
-    if (B <= 16) head_gemm_go<1>((bf16_t*)y, xx, ww, B, H, N, K, yb, yh, xb, xh, st);
-    else if (B <= 32) head_gemm_go<2>((bf16_t*)y, xx, ww, B, H, N, K, yb, yh, xb, xh, st);
-    else head_gemm_go<4>((bf16_t*)y, xx, ww, B, H, N, K, yb, yh, xb, xh, st);
+  if (!f32 && head_gemm_whole(N, K, yb, yh, xb, xh)) {
+    const HeadGemm q{(bf16_t*)y, (const bf16_t*)x, (const bf16_t*)w, B, N, K, yb, yh, xb, xh};
+    if (B <= 16) head_gemm_go<1>(q, H, st);
+    else if (B <= 32) head_gemm_go<2>(q, H, st);
+    else head_gemm_go<4>(q, H, st);
   } else {
     const dim3 grid(B, H, (N + 255) / 256);
     if (f32)
@@ -1049,6 +1169,41 @@ int launch_head_gemm(int f32, void* y, const void* x, const void* w, int B, int 
       head_gemm_any_kernel<bf16_t><<<grid, dim3(256), 0, st>>>(
           (bf16_t*)y, (const bf16_t*)x, (const bf16_t*)w, N, K, yb, yh, xb, xh);
   }
+  return (int)hipGetLastError();
+}
+
+// Decode: launch_latent_prep, and qa[b, h, :R] = w[h] proj[b, h, :dim] for w [H, R, dim].
+int launch_latent_front(int f32, const LatentPrepArgs& a, const void* w, hipStream_t st) {
+  if (a.rows == 0) return 0;
+  if (!a.qa || !lat_prep_takes(a)) return -1;
+  const int dq = a.dim + a.rot;
+  const HeadGemm q{(bf16_t*)a.qa, (const bf16_t*)a.proj, (const bf16_t*)w, a.rows, a.R, a.dim,
+                   (int64_t)a.H * a.LW, a.LW, a.ldp, dq};
+  const int nbt = a.rows <= 16 ? 1 : a.rows <= 32 ? 2 : 4;
+  if (f32 || !lat_prep_whole(a) || !head_gemm_whole(q.N, q.K, q.yb, q.yh, q.xb, q.xh) || a.dim % 128 ||
+      head_gemm_shares(q, a.H, nbt)) {
+    const int e = launch_latent_prep(f32, a, st);
+    return e ? e : launch_head_gemm(f32, a.qa, a.proj, w, a.rows, a.H, a.R, a.dim, q.yb, q.yh, q.xb, q.xh, st);
+  }
+  const int grid = a.rows + (a.R + 63) / 64 * ((a.rows + 16 * nbt - 1) / (16 * nbt)) * a.H;
+  (nbt == 1 ? latent_front_kernel<1> : nbt == 2 ? latent_front_kernel<2> : latent_front_kernel<4>)<<<dim3(grid), dim3(256), 0, st>>>(a, q);
+  return (int)hipGetLastError();
+}
+
+// Decode: launch_latent_decode, and y[b, h, :] = w[h] out[b, h, :] for w [H, N, R].
+int launch_latent_decode_up(int f32, const LatentDecodeArgs& a, void* y, const void* w, int N, int64_t yb, int64_t yh,
+                            hipStream_t st) {
+  if (a.B == 0) return 0;
+  const HeadGemm q{(bf16_t*)y, (const bf16_t*)a.out, (const bf16_t*)w, a.B, N, a.R, yb, yh, (int64_t)a.H * a.R, a.R};
+  // few rows: the product adds up the splits itself, in each of its workgroups again, up to 64 KB each (a step of one row at
+  // 3500, two such layers 381 -> 364 us with the launch below; 16 rows, 128 KB, 436 -> 439)
+  if (!lat_decode_split(f32, a) || !head_gemm_whole(N, a.R, yb, yh, q.xb, q.xh) || a.R % 128 || a.B > 16 ||
+      a.B * a.nsplits > kUpParts || (int64_t)a.B * a.nsplits * a.R > 16384) {
+    const int e = launch_latent_decode(f32, a, st);
+    return e ? e : launch_head_gemm(f32, y, a.out, w, a.B, a.H, N, a.R, yb, yh, q.xb, q.xh, st);
+  }
+  lat_decode_parts(a, st);
+  latent_up_kernel<512><<<dim3((N + 15) / 16, a.H), dim3(256), 0, st>>>(a, q);
   return (int)hipGetLastError();
 }
 

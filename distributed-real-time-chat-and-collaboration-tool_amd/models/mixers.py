@@ -116,13 +116,11 @@ class LatentMixer(Mixer):
         B = proj.shape[0]
         qa = proj.new_empty(B, m.heads, cache.shape[-1])
         ops.latent_prep(proj, self.off_kv, m.heads, m.dim, m.rot_dim, m.rot_dims, m.kv_rank,
-                        self.c_norm, self.eps, self.rope, positions, slots, cache, qa=qa)
-        dq = m.dim + m.rot_dim
-        ops.head_linear(proj[:, :m.heads * dq].unflatten(1, (m.heads, dq)), self.uk_t, out=qa)
-        o = ops.latent_decode_attention(qa, cache, m.kv_rank, dm.block_tables, dm.context_lens,
-                                        m.window, m.scale, self.sink,
-                                        dm.workspace[m.heads, m.kv_rank, m.window], self._gate(proj))
-        ops.head_linear(o, self.uv, out=out.unflatten(1, (m.heads, m.vdim)))
+                        self.c_norm, self.eps, self.rope, positions, slots, cache, qa=qa, down=self.uk_t)
+        ops.latent_decode_attention(qa, cache, m.kv_rank, dm.block_tables, dm.context_lens,
+                                    m.window, m.scale, self.sink,
+                                    dm.workspace[m.heads, m.kv_rank, m.window], self._gate(proj),
+                                    up=self.uv, out=out.unflatten(1, (m.heads, m.vdim)))
 
     def _latents(self, proj, meta, cache, carry):
         """Latent rows of the portions' keys; queries are rotated in place.  Layers that read the

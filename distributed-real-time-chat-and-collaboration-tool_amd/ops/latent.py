@@ -64,11 +64,12 @@ def latent_prep(proj: torch.Tensor, off_kv: int | None, heads: int, dim: int, ro
                 rot_dims: int, kv_rank: int, norm_w: torch.Tensor | None, eps: float,
                 cos_sin: torch.Tensor, positions: torch.Tensor, slots: torch.Tensor | None,
                 cache: torch.Tensor | None, lat: torch.Tensor | None = None,
-                qa: torch.Tensor | None = None) -> None:
+                qa: torch.Tensor | None = None, down: torch.Tensor | None = None) -> None:
     """Rows of the fused projection [queries | latent, key part]: RMS-norm the latent, rotate
     the key part, write both to ``lat`` [rows, LW] and to the cache rows ``slots`` (-1: none).
     The queries' rotated parts go to ``qa`` [rows, heads, LW] at column kv_rank (zeros
-    behind), or are rotated in place.  ``off_kv`` None: queries only."""
+    behind), or are rotated in place.  ``off_kv`` None: queries only.  ``down`` [heads, kv_rank, dim] (with ``qa``): the
+    queries' other parts go there too, times it, in the same launch."""
     rows = proj.shape[0]
     own = off_kv is not None
     LW = (cache if cache is not None else lat if lat is not None else qa).shape[-1]
@@ -89,6 +90,8 @@ def latent_prep(proj: torch.Tensor, off_kv: int | None, heads: int, dim: int, ro
                 cache.view(-1, LW)[slots[:rows][ok]] = full[ok]
         q = proj[:, :heads * dq].unflatten(1, (heads, dq))
         r = rotate_pairs_ref(q[..., dim:], cs, rot_dims)
+        if down is not None:
+            head_linear(q, down, out=qa)
         if qa is not None:
             qa[..., kv_rank:] = 0
             qa[..., kv_rank:kv_rank + rot_dim] = r
@@ -106,13 +109,15 @@ def latent_prep(proj: torch.Tensor, off_kv: int | None, heads: int, dim: int, ro
         assert t is None or (t.is_contiguous() and t.shape[-1] == LW and t.dtype == proj.dtype)
     assert lat is None or lat.shape[0] == rows
     assert qa is None or qa.shape[:2] == (rows, heads)
+    assert down is None or (qa is not None and down.shape == (heads, kv_rank, dim) and down.is_contiguous()
+                            and down.dtype == proj.dtype)
     if cache is not None:
         assert slots is not None and slots.dtype == torch.int64 and slots.numel() >= rows
     check(hipk().latent_prep(int(proj.dtype == torch.float32), dict(
         proj=proj.data_ptr(), ldp=proj.stride(0), off_kv=off_kv if own else -1, H=heads, dim=dim,
         rot=rot_dim, rot_dims=rot_dims, R=kv_rank, LW=LW, norm_w=ptr(norm_w), eps=float(eps),
         cos_sin=cos_sin.data_ptr(), positions=positions.data_ptr(), slots=ptr(slots),
-        lat=ptr(lat), cache=ptr(cache), qa=ptr(qa), rows=rows), stream_ptr(proj)), "latent_prep")
+        lat=ptr(lat), cache=ptr(cache), qa=ptr(qa), rows=rows), ptr(down), stream_ptr(proj)), "latent_prep")
 
 
 def latent_gather(cache: torch.Tensor, slots: torch.Tensor) -> torch.Tensor:
@@ -270,12 +275,18 @@ def latent_decode_attention(qa: torch.Tensor, cache: torch.Tensor, kv_rank: int,
                             block_tables: torch.Tensor, context_lens: torch.Tensor,
                             window: int | None, scale: float, sink: torch.Tensor | None,
                             workspace: LatentDecodeWorkspace | None = None,
-                            gate: torch.Tensor | None = None) -> torch.Tensor:
+                            gate: torch.Tensor | None = None, up: torch.Tensor | None = None,
+                            out: torch.Tensor | None = None) -> torch.Tensor:
     """One query per sequence in the latent space, qa [B, heads, LW], against the cache rows of
     its last ``window`` tokens (its own included: context_lens counts it).  Rows with context 0
-    give zeros.  ``gate`` [B, heads]: results times its sigmoid.  Returns [B, heads, kv_rank]."""
+    give zeros.  ``gate`` [B, heads]: results times its sigmoid.  Returns [B, heads, kv_rank], or with ``up`` [heads, N,
+    kv_rank] ``out`` [B, heads, >= N]: ``head_linear`` of it, which adds up the splits of few rows."""
     B, H, LW = qa.shape
+    assert (up is None) == (out is None)
     if not on_gpu(qa):
+        if up is not None:
+            return head_linear(latent_decode_attention(qa, cache, kv_rank, block_tables, context_lens, window, scale, sink,
+                                                       workspace, gate), up, out=out)
         out = qa.new_zeros(B, H, kv_rank)
         flat = cache.view(-1, LW)
         for b in range(B):
@@ -299,15 +310,21 @@ def latent_decode_attention(qa: torch.Tensor, cache: torch.Tensor, kv_rank: int,
     ws = workspace or LatentDecodeWorkspace(B, H, kv_rank, window, block_tables.shape[1], qa.device)
     assert ws.splits == 1 or (ws.part_o is not None and ws.part_o.shape[:2] == (B, H)
                               and ws.part_o.shape[3] == kv_rank)
+    y = out
     out = torch.empty((B, H, kv_rank), dtype=qa.dtype, device=qa.device)
+    if up is not None:
+        N = up.shape[1]
+        assert up.is_contiguous() and up.shape == (H, N, kv_rank) and up.dtype == y.dtype == qa.dtype
+        assert y.shape[:2] == (B, H) and y.shape[2] >= N and y.stride(2) == 1
     check(hipk().latent_decode(int(qa.dtype == torch.float32), dict(
         out=out.data_ptr(), part_o=ptr(ws.part_o), part_ml=ptr(ws.part_ml), qa=qa.data_ptr(),
         cache=cache.data_ptr(), block_tables=block_tables.data_ptr(),
         bt_stride=block_tables.stride(0), context_lens=context_lens.data_ptr(), B=B, H=H,
         R=kv_rank, LW=LW, window=window or 0, tiles_per_split=ws.per, nsplits=ws.splits,
         scale=float(scale), sink=ptr(sink), gate=ptr(gate),
-        ldg=gate.stride(0) if gate is not None else 0), stream_ptr(qa)), "latent_decode")
-    return out
+        ldg=gate.stride(0) if gate is not None else 0), ptr(y), ptr(up), 0 if up is None else up.shape[1],
+        0 if y is None else y.stride(0), 0 if y is None else y.stride(1), stream_ptr(qa)), "latent_decode")
+    return out if y is None else y
 
 
 def head_linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:

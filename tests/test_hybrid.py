@@ -1029,6 +1029,54 @@ def test_latent_decode_in_pairs_of_blocks(H, R, parts):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("B", [1, 3, 16, 17, 65])
+@pytest.mark.parametrize("H,R,dim,vdim,splits,gated", [(16, 512, 128, 128, 20, True), (4, 256, 128, 40, 3, False),
+                                                        (5, 128, 256, 64, 2, True), (20, 448, 128, 128, 4, True),
+                                                        (3, 52, 12, 20, 3, False), (2, 384, 128, 16, 64, False)])
+def test_latent_ways_down_and_up(B, H, R, dim, vdim, splits, gated):
+    """The queries' way down in the preparation's launch, the same bits as by itself; the results' way up that adds up
+    the splits, against the merged result's within two roundings to bf16 of each addend's size."""
+    rot, nb = 64 if R != 52 else 6, 2 * splits
+    LW, dq, dev = ops.latent_width(R, rot), dim + rot, "cuda"
+    g = torch.Generator().manual_seed(B + R)
+    rand = lambda *shape, std=1.0: (torch.randn(*shape, generator=g) * std).to(torch.bfloat16).to(dev)
+    kv = -(-H * dq // 8) * 8
+    proj = rand(B, kv + -(-(R + rot) // 8) * 8 + H)
+    uk, uv = rand(H, R, dim, std=dim ** -0.5), rand(H, vdim, R, std=R ** -0.5)
+    norm, angle = torch.rand(R, generator=g).to(dev) + 0.5, torch.rand(4096, rot // 2, generator=g)
+    cs = torch.cat([angle.cos(), angle.sin()], 1).to(dev)
+    ctx = [1, 32 * nb, 33, 70, 0, 64, 32 * nb - 1][:B] + [(37 * i) % (32 * nb) for i in range(7, B)]
+    bt = (torch.randperm(B * nb, generator=g).view(B, nb) + 1).to(torch.int32).to(dev)
+    pos = torch.tensor([max(0, n - 1) for n in ctx], dtype=torch.int32, device=dev)
+    ctx_t = torch.tensor(ctx, dtype=torch.int32, device=dev)
+    slots = torch.tensor([int(bt[b, (n - 1) // 32]) * 32 + (n - 1) % 32 if n else -1 for b, n in enumerate(ctx)],
+                         dtype=torch.int64, device=dev)
+    caches, rows = [rand(B * nb + 1, 32, LW)], []
+    caches.append(caches[0].clone())
+    for cache, down in zip(caches, (None, uk)):
+        qa = torch.full((B, H, LW), float("nan"), dtype=torch.bfloat16, device=dev)
+        ops.latent_prep(proj, kv, H, dim, rot, rot, R, norm, 1e-5, cs, pos, slots, cache, qa=qa, down=down)
+        if down is None:
+            ops.head_linear(proj[:, :H * dq].unflatten(1, (H, dq)), uk, out=qa)
+        rows.append(qa)
+    assert torch.equal(*rows) and torch.equal(*caches) and not rows[0].isnan().any()
+    gate, sink = (proj[:, -H:], rand(H).float()) if gated else (None, None)
+    for window in (None, 50):
+        ws = ops.LatentDecodeWorkspace(B, H, R, window, nb, dev)
+        ws.per, ws.splits = 2, splits
+        ws.part_o, ws.part_ml = torch.full((B, H, splits, R), 1e3, device=dev), torch.zeros(B, H, splits, 2, device=dev)
+        args = (rows[0], caches[0], R, bt, ctx_t, window, 0.05, sink, ws, gate)
+        merged = ops.latent_decode_attention(*args)
+        out = torch.full((B, H + 1, vdim + 4), 7.0, dtype=torch.bfloat16, device=dev)
+        assert ops.latent_decode_attention(*args, up=uv, out=out[:, :H, :vdim]) is not None
+        want = torch.einsum("bhr,hnr->bhn", merged.float().cpu(), uv.float().cpu())
+        size = torch.einsum("bhr,hnr->bhn", merged.float().abs().cpu(), uv.float().abs().cpu())
+        got = out[:, :H, :vdim].float().cpu()
+        assert ((got - want).abs() <= 2 ** -8 * (want.abs() + size) + 1e-6).all()
+        assert (out[:, H] == 7).all() and (out[:, :, vdim:] == 7).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,R", [(16, 256), (32, 512), (40, 512)])
 def test_latent_decode_of_a_cache_at_any_address(H, R):
     """Rows of whole cache lines in a cache that starts off 16 bytes: rounding of the test above."""
