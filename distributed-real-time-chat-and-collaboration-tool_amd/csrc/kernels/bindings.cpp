@@ -234,9 +234,10 @@ PYBIND11_MODULE(_hipk, m) {
                                          M, N, K, ldx, ldr, ldh, ldy, eps, gemma, act, S(st));
   });
   m.def("skinny_gemm", [](u64 y, u64 x, u64 w, int M, int N, int K, int ldx, int ldy,
-                          int variant, u64 st) {
+                          int variant, u64 y2, u64 x2, u64 w2, int N2, int ldx2, int ldy2, int relu2, u64 st) {
     return drtc::launch_skinny_gemm(P<void>(y), P<const void>(x), P<const void>(w), M, N, K, ldx,
-                                    ldy, variant, S(st));
+                                    ldy, variant, P<void>(y2), P<const void>(x2), P<const void>(w2), N2, ldx2, ldy2, relu2,
+                                    S(st));
   });
   m.def("lt_tune", [](u64 y, u64 x, u64 w, int64_t M, int64_t N, int64_t K, int64_t ldx,
                       int64_t ldy, int iters, int max_candidates, u64 st) {

@@ -56,14 +56,31 @@ DRTC_DEVICE bf16x8 load_x8(const bf16_t* p, int K) {
   }
 }
 
-template <int MT, int R, int ACT = -1>
-__global__ __launch_bounds__(256) void skinny_gemm_kernel(bf16_t* __restrict__ y,
-                                                          const bf16_t* __restrict__ x,
-                                                          const bf16_t* __restrict__ w, int M,
-                                                          int K, int ldx, int ldy) {
+// A second product of as many rows and the same K in the same launch, from workgroup `first` on: neither waits for the
+// other, and what a launch costs a chain of small kernels, 2 us, is paid once.  relu2: bit 0 squares the first's relu, bit 1
+// the second's.  (Four layers with two such pairs in a step of one row: 364 -> 344 us.)
+struct SkinnyBeside {
+  bf16_t* y;
+  const bf16_t *x, *w;
+  int ldx, ldy, first, relu2;
+};
+DRTC_DEVICE float relu2_if(float v, bool on) {
+  const float r = fmaxf(v, 0.f);
+  return on ? r * r : v;
+}
+
+template <int MT, int R, int ACT = -1, bool TWO = false>
+__global__ __launch_bounds__(256) void skinny_gemm_kernel(bf16_t* y, const bf16_t* x, const bf16_t* w, int M, int K, int ldx,
+                                                          int ldy, SkinnyBeside s) {
   constexpr int CH = 512;  // k elements per chunk (64 lanes x 8)
   __shared__ float part[4][R * MT];
-  const int n0 = blockIdx.x * R;
+  int n0 = blockIdx.x * R;
+  bool relu2 = TWO && (s.relu2 & 1);
+  if (TWO && (int)blockIdx.x >= s.first) {
+    n0 -= s.first * R;
+    y = s.y, x = s.x, w = s.w, ldx = s.ldx, ldy = s.ldy;
+    relu2 = s.relu2 & 2;
+  }
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int nch = K / CH;
   float acc[R][MT];
@@ -129,8 +146,8 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(bf16_t* __restrict__ y
   if (t < R * MT) {
     const int r = t / MT, m = t - r * MT;
     if (m < M) {
-      const float s = part[0][t] + part[1][t] + part[2][t] + part[3][t];
-      y[(int64_t)m * ldy + n0 + r] = f2bf(s);
+      const float sum = part[0][t] + part[1][t] + part[2][t] + part[3][t];
+      y[(int64_t)m * ldy + n0 + r] = f2bf(relu2_if(sum, relu2));
     }
   }
 }
@@ -143,12 +160,13 @@ int launch_skinny_glu_gemm(void* y, const void* gu, const void* w, int M, int N,
   bf16_t* yy = (bf16_t*)y;
   const bf16_t* xx = (const bf16_t*)gu;
   const bf16_t* ww = (const bf16_t*)w;
+  const SkinnyBeside none{nullptr, nullptr, nullptr, 0, 0, N / 4, 0};
   if (M == 1) {
-    if (act == 0) skinny_gemm_kernel<1, 4, 0><<<grid, block, 0, st>>>(yy, xx, ww, M, K, ldx, ldy);
-    else skinny_gemm_kernel<1, 4, 1><<<grid, block, 0, st>>>(yy, xx, ww, M, K, ldx, ldy);
+    if (act == 0) skinny_gemm_kernel<1, 4, 0><<<grid, block, 0, st>>>(yy, xx, ww, M, K, ldx, ldy, none);
+    else skinny_gemm_kernel<1, 4, 1><<<grid, block, 0, st>>>(yy, xx, ww, M, K, ldx, ldy, none);
   } else {
-    if (act == 0) skinny_gemm_kernel<2, 4, 0><<<grid, block, 0, st>>>(yy, xx, ww, M, K, ldx, ldy);
-    else skinny_gemm_kernel<2, 4, 1><<<grid, block, 0, st>>>(yy, xx, ww, M, K, ldx, ldy);
+    if (act == 0) skinny_gemm_kernel<2, 4, 0><<<grid, block, 0, st>>>(yy, xx, ww, M, K, ldx, ldy, none);
+    else skinny_gemm_kernel<2, 4, 1><<<grid, block, 0, st>>>(yy, xx, ww, M, K, ldx, ldy, none);
   }
   return (int)hipGetLastError();
 }
@@ -313,16 +331,21 @@ int launch_skinny_norm_gemm(void* y, void* h_out, const void* x, const void* res
 // g = l >> 4 takes k = 32 s + 8 g .. +8 - the same k for the A and B
 // fragments, so the product is exact; this order makes the 4 lanes of a row
 // read 64 contiguous bytes per load instruction.
-template <int T, int NW, int KS>
-__global__ __launch_bounds__(NW * 64) void skinny_mfma_kernel(bf16_t* __restrict__ y,
-                                                             const bf16_t* __restrict__ x,
-                                                             const bf16_t* __restrict__ w, int M,
-                                                             int K, int ldx, int ldy) {
+template <int T, int NW, int KS, bool TWO>
+__global__ __launch_bounds__(NW * 64) void skinny_mfma_kernel(bf16_t* y, const bf16_t* x, const bf16_t* w, int M, int K,
+                                                              int ldx, int ldy, SkinnyBeside beside) {
   constexpr int STEP = 128, RG = NW / KS;
   __shared__ f32x4 red[NW][T][64];
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int ks = wv % KS, rg = wv / KS;
-  const int n0 = (blockIdx.x * RG + rg) * (16 * T);
+  int blk = blockIdx.x;
+  bool relu2 = TWO && (beside.relu2 & 1);
+  if (TWO && blk >= beside.first) {
+    blk -= beside.first;
+    y = beside.y, x = beside.x, w = beside.w, ldx = beside.ldx, ldy = beside.ldy;
+    relu2 = beside.relu2 & 2;
+  }
+  const int n0 = (blk * RG + rg) * (16 * T);
   const int r = lane & 15, g = lane >> 4;
   const bool xv = r < M;
   const int nst = K / STEP;
@@ -368,7 +391,9 @@ __global__ __launch_bounds__(NW * 64) void skinny_mfma_kernel(bf16_t* __restrict
   }
   // C layout: lane l holds D[row 4*(l>>4) + v][col l&15] = y[m = l&15][n0 + 16t + 4(l>>4) + v]
   auto store = [&](f32x4 v, int row0, int l) {
-    const bf16x4 o = {f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
+    bf16x4 o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = f2bf(relu2_if(v[i], relu2));
     *reinterpret_cast<bf16x4*>(y + (int64_t)(l & 15) * ldy + row0 + 4 * (l >> 4)) = o;
   };
   if constexpr (KS == 1) {
@@ -386,56 +411,61 @@ __global__ __launch_bounds__(NW * 64) void skinny_mfma_kernel(bf16_t* __restrict
       f32x4 sum = red[q * KS][t][l];
 #pragma unroll
       for (int j = 1; j < KS; ++j) sum += red[q * KS + j][t][l];
-      store(sum, (blockIdx.x * RG + q) * (16 * T) + 16 * t, l);
+      store(sum, (blk * RG + q) * (16 * T) + 16 * t, l);
     }
   }
 }
 
 template <int T, int NW, int KS>
 static int launch_mfma(bf16_t* y, const bf16_t* x, const bf16_t* w, int M, int N, int K, int ldx,
-                       int ldy, hipStream_t st) {
+                       int ldy, SkinnyBeside s, int N2, hipStream_t st) {
   constexpr int ROWS = 16 * T * (NW / KS);
-  if (N % ROWS != 0) return -1;
-  skinny_mfma_kernel<T, NW, KS><<<dim3(N / ROWS), dim3(NW * 64), 0, st>>>(y, x, w, M, K, ldx, ldy);
+  if (N % ROWS != 0 || N2 % ROWS != 0) return -1;
+  s.first = N / ROWS;
+  (N2 || s.relu2 ? skinny_mfma_kernel<T, NW, KS, true> : skinny_mfma_kernel<T, NW, KS, false>)<<<dim3((N + N2) / ROWS), dim3(NW * 64), 0, st>>>(
+      y, x, w, M, K, ldx, ldy, s);
   return 0;
 }
 
 // variant: 0 = by shape, 1 = dot2 form, 2.. = MFMA form (T, NW, KS):
 //   2 (1,4,4)  3 (1,8,8)  4 (2,4,4)  5 (2,8,8)  6 (1,16,16)  7 (1,8,2)  8 (1,8,1)  9 (1,16,4)
+// y2 [M, N2] = x2 w2^T beside it (N2 0: none), relu2 as SkinnyBeside's
 int launch_skinny_gemm(void* y, const void* x, const void* w, int M, int N, int K, int ldx,
-                       int ldy, int variant, hipStream_t st) {
+                       int ldy, int variant, void* y2, const void* x2, const void* w2, int N2, int ldx2, int ldy2,
+                       int relu2, hipStream_t st) {
   constexpr int R = 4;
   bf16_t* yy = (bf16_t*)y;
   const bf16_t* xx = (const bf16_t*)x;
   const bf16_t* ww = (const bf16_t*)w;
-  if (M < 1 || M > 16 || ldx % 8 != 0 || ldy % 4 != 0) return -1;
+  if (M < 1 || M > 16 || ldx % 8 != 0 || ldy % 4 != 0 || N2 < 0 || ldx2 % 8 != 0 || ldy2 % 4 != 0 ||
+      (N2 > 0 && (!y2 || !x2 || !w2)))
+    return -1;
+  SkinnyBeside s{(bf16_t*)y2, (const bf16_t*)x2, (const bf16_t*)w2, ldx2, ldy2, 0, relu2};
   if (variant == 0) variant = (M <= 2 && K % 512 == 0) ? 1 : 3;
   if (variant >= 2) {
     if (K % 128 != 0) return -1;
     int rc = -1;
     switch (variant) {
-      case 2: rc = launch_mfma<1, 4, 4>(yy, xx, ww, M, N, K, ldx, ldy, st); break;
-      case 3: rc = launch_mfma<1, 8, 8>(yy, xx, ww, M, N, K, ldx, ldy, st); break;
-      case 4: rc = launch_mfma<2, 4, 4>(yy, xx, ww, M, N, K, ldx, ldy, st); break;
-      case 5: rc = launch_mfma<2, 8, 8>(yy, xx, ww, M, N, K, ldx, ldy, st); break;
-      case 6: rc = launch_mfma<1, 16, 16>(yy, xx, ww, M, N, K, ldx, ldy, st); break;
-      case 7: rc = launch_mfma<1, 8, 2>(yy, xx, ww, M, N, K, ldx, ldy, st); break;
-      case 8: rc = launch_mfma<1, 8, 1>(yy, xx, ww, M, N, K, ldx, ldy, st); break;
-      case 9: rc = launch_mfma<1, 16, 4>(yy, xx, ww, M, N, K, ldx, ldy, st); break;
+      case 2: rc = launch_mfma<1, 4, 4>(yy, xx, ww, M, N, K, ldx, ldy, s, N2, st); break;
+      case 3: rc = launch_mfma<1, 8, 8>(yy, xx, ww, M, N, K, ldx, ldy, s, N2, st); break;
+      case 4: rc = launch_mfma<2, 4, 4>(yy, xx, ww, M, N, K, ldx, ldy, s, N2, st); break;
+      case 5: rc = launch_mfma<2, 8, 8>(yy, xx, ww, M, N, K, ldx, ldy, s, N2, st); break;
+      case 6: rc = launch_mfma<1, 16, 16>(yy, xx, ww, M, N, K, ldx, ldy, s, N2, st); break;
+      case 7: rc = launch_mfma<1, 8, 2>(yy, xx, ww, M, N, K, ldx, ldy, s, N2, st); break;
+      case 8: rc = launch_mfma<1, 8, 1>(yy, xx, ww, M, N, K, ldx, ldy, s, N2, st); break;
+      case 9: rc = launch_mfma<1, 16, 4>(yy, xx, ww, M, N, K, ldx, ldy, s, N2, st); break;
       default: return -1;
     }
     return rc ? rc : (int)hipGetLastError();
   }
-  if (M > 8 || K % 512 != 0 || N % R != 0) return -1;
-  const dim3 grid(N / R), block(256);
-  if (M == 1)
-    skinny_gemm_kernel<1, R><<<grid, block, 0, st>>>(yy, xx, ww, M, K, ldx, ldy);
-  else if (M == 2)
-    skinny_gemm_kernel<2, R><<<grid, block, 0, st>>>(yy, xx, ww, M, K, ldx, ldy);
-  else if (M <= 4)
-    skinny_gemm_kernel<4, R><<<grid, block, 0, st>>>(yy, xx, ww, M, K, ldx, ldy);
-  else
-    skinny_gemm_kernel<8, R><<<grid, block, 0, st>>>(yy, xx, ww, M, K, ldx, ldy);
+  if (M > 8 || K % 512 != 0 || N % R != 0 || N2 % R != 0) return -1;
+  const dim3 grid((N + N2) / R), block(256);
+  s.first = N / R;
+  const auto go = [&](auto one, auto two) { (N2 || relu2 ? two : one)<<<grid, block, 0, st>>>(yy, xx, ww, M, K, ldx, ldy, s); };
+  if (M == 1) go(skinny_gemm_kernel<1, R>, skinny_gemm_kernel<1, R, -1, true>);
+  else if (M == 2) go(skinny_gemm_kernel<2, R>, skinny_gemm_kernel<2, R, -1, true>);
+  else if (M <= 4) go(skinny_gemm_kernel<4, R>, skinny_gemm_kernel<4, R, -1, true>);
+  else go(skinny_gemm_kernel<8, R>, skinny_gemm_kernel<8, R, -1, true>);
   return (int)hipGetLastError();
 }
 

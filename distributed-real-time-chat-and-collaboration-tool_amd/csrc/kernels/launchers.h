@@ -144,7 +144,8 @@ std::vector<std::pair<int, float>> lt_tune(void* y, const void* x, const void* w
 // Skinny projection GEMM for decode batches M <= 16 (gemv.hip): y[M,N] = x[M,K] @ W[N,K]^T.
 // variant 0 = by shape; returns -1 for a shape the chosen form does not cover.
 int launch_skinny_gemm(void* y, const void* x, const void* w, int M, int N, int K, int ldx,
-                       int ldy, int variant, hipStream_t st);
+                       int ldy, int variant, void* y2, const void* x2, const void* w2, int N2, int ldx2, int ldy2,
+                       int relu2, hipStream_t st);
 
 // Gated activation fused into the skinny dot2 GEMM (gemv.hip): y = (act(gu[:, :K]) * gu[:, K:2K]) @ W^T,
 // gu row stride ldx; M <= 2, K % 512 == 0, act 0 = SiLU, 1 = tanh-GELU.

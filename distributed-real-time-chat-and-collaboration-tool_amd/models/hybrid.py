@@ -444,8 +444,9 @@ class HybridLM:
         logits = ops.linear(x, self.lm_head)
         return ops.softcap_(logits, cfg.logit_softcap) if cfg.logit_softcap else logits
 
-    def _joint(self, ids: torch.Tensor, mix, rows: torch.Tensor | None) -> torch.Tensor:
-        """As _serial: one norm for both sublayers, one add, then the token's input to the layer."""
+    def _joint(self, ids: torch.Tensor, mix, rows: torch.Tensor | None, carry: dict | None = None) -> torch.Tensor:
+        """As _serial: one norm for both sublayers, one add, then the token's input to the layer.  ``carry``: of a decode
+        step, where a mixer may take the shared expert's first product along with its own."""
         cfg, dt, eps, W = self.cfg, self.dtype, self.cfg.norm_eps, self.cfg.hidden_size
         h = torch.empty((ids.shape[0], W), dtype=torch.float32, device=self.device)
         z, zn, last = None, None, len(self.layers) - 1
@@ -460,11 +461,14 @@ class HybridLM:
             a = torch.empty((ids.shape[0], L["out"].shape[1]), dtype=dt, device=self.device)
             if off > mw:
                 a[:, mw:off].zero_()
+            if carry is not None and "up" in L:
+                carry["beside"] = (L["up"], a[:, off:])
             mix(i, L["mixer"], x, a[:, :mw])
+            taken = carry is not None and carry.pop("beside", None) is None
             if i == last and rows is not None:
                 ids, h, a, wide = (t.index_select(0, rows) for t in (ids, h, a, wide))
                 x = wide[:, :W]
-            if "up" in L:
+            if "up" in L and not taken:
                 ops.squared_relu(x, L["up"], a[:, off:])
             if l.experts:
                 x = self._experts(L, l, wide, logits, stream=h, y=ops.linear_parts(a, L["out"]))
@@ -499,7 +503,7 @@ class HybridLM:
             return mixer.decode(x, meta, kv[i], out, carry)
 
         if self.cfg.block != "parallel":
-            return (self._joint if self.cfg.block == "joint" else self._serial)(ids, mix, None)
+            return self._joint(ids, mix, None, carry) if self.cfg.block == "joint" else self._serial(ids, mix, None)
         return self._parallel(ids, mix, None, meta.positions, kv, row_state=meta.state)
 
     # ------------------------------------------------------------ reference

@@ -72,6 +72,11 @@ class Mixer:
                                   ops.GroupedWeights, ops.MemoryWeights)) else []
         return ts
 
+    def _project_in(self, x, carry) -> torch.Tensor:
+        """The input projection, along with the product that the step's ``carry`` has for it under "beside"."""
+        beside = carry.pop("beside", None) if carry else None
+        return ops.linear(x, self.proj) if beside is None else ops.linear_beside(x, self.proj, x, *beside, relu2=True)[0]
+
     def _out(self, x, out) -> torch.Tensor:
         return x.new_empty(x.shape[0], self.width) if out is None else out
 
@@ -157,7 +162,7 @@ class LatentMixer(Mixer):
 
     def decode(self, x, meta, cache, out=None, carry=None):
         a = self._out(x, out)
-        self._decode(ops.linear(x, self.proj), meta.positions, meta.slots, cache, meta, a)
+        self._decode(self._project_in(x, carry), meta.positions, meta.slots, cache, meta, a)
         return a
 
 
@@ -187,8 +192,8 @@ class DeltaMixer(Mixer):
 
     def _project(self, x):
         proj = ops.linear(x, self.proj)
-        decay = ops.linear(proj[:, self.off_a:self.off_a + self.a2.shape[1]], self.a2)
-        gate = ops.linear(proj[:, self.off_g:self.off_g + self.g2.shape[1]], self.g2)
+        decay, gate = ops.linear_beside(proj[:, self.off_a:self.off_a + self.a2.shape[1]], self.a2,
+                                        proj[:, self.off_g:self.off_g + self.g2.shape[1]], self.g2)
         return proj, decay, gate
 
     def prefill(self, x, meta, cache, out=None, carry=None):
@@ -401,7 +406,7 @@ class MemoryMixer(Mixer):
 
     def decode(self, x, meta, cache, out=None, carry=None):
         a = self._out(x, out)
-        ops.memory_decode(ops.linear(x, self.proj), self.w, self._states(cache), meta.positions,
+        ops.memory_decode(self._project_in(x, carry), self.w, self._states(cache), meta.positions,
                           meta.state, a)
         return a
 

@@ -18,7 +18,7 @@ from .attention import (KV_BLOCK, DecodeWorkspace, decode_partitioning, paged_de
 from .delta import DeltaWeights, Portions, delta_decode, delta_scan, short_conv
 from .gated_average import (SCAN_CHUNK, AverageWeights, ScanChunks, chunk_scan, gated_decode,
                             gated_scan)
-from .gemm import (Parts, fused_glu_ok, gated, glu_linear, linear, linear_parts, linear_residual, mfma_gemm, norm_glu,
+from .gemm import (Parts, fused_glu_ok, gated, glu_linear, linear, linear_beside, linear_parts, linear_residual, mfma_gemm, norm_glu,
                    norm_glu_row, norm_linear, residual_fusable, squared_relu, w4_glu_ok)
 from .grouped import (GroupedDecodeWorkspace, GroupedPortions, GroupedWeights, attn_prep,
                       grouped_decode, grouped_prefill, grouped_qtile, prep_tile_rows)
@@ -37,7 +37,7 @@ from .talking import (MIX_TILE, STATS_TILE, TalkDecodeWorkspace, TalkPortions, T
                       head_prep, pad8, talk_cache_shapes, talk_decode, talk_prefill)
 
 __all__ = [
-    "on_gpu", "reference_mode", "linear", "linear_parts", "Parts", "norm_linear", "glu_linear", "norm_glu", "w4_glu_ok",
+    "on_gpu", "reference_mode", "linear", "linear_beside", "linear_parts", "Parts", "norm_linear", "glu_linear", "norm_glu", "w4_glu_ok",
     "fused_glu_ok",
     "mfma_gemm", "linear_residual", "residual_fusable", "PendingNorm", "fused_moe", "router_logits",
     "fused_moe_ref", "moe_norm_ok", "act_glu", "act_glu_ref", "KV_BLOCK", "DecodeWorkspace",

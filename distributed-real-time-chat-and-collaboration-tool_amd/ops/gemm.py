@@ -414,6 +414,7 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 
 # ------------------------------------------------------------------ skinny decode kernels
+DUAL = range(1, 10)  # skinny variants that take a second product along
 # rows of W per workgroup of each MFMA variant (gemv.hip launch_skinny_gemm)
 SKINNY_ROWS = {2: 16, 3: 16, 4: 32, 5: 32, 6: 16, 7: 64, 8: 128, 9: 64}
 
@@ -451,8 +452,32 @@ def skinny_linear(x: torch.Tensor, w: torch.Tensor, variant: int = 0) -> torch.T
     variant = variant or skinny_variant(M, N, K, x.stride(0))
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
     check(hipk().skinny_gemm(y.data_ptr(), x.data_ptr(), w.data_ptr(), M, N, K, x.stride(0), N,
-                             variant, stream_ptr(x)), "skinny_gemm")
+                             variant, 0, 0, 0, 0, 0, 0, 0, stream_ptr(x)), "skinny_gemm")
     return y
+
+
+def linear_beside(x: torch.Tensor, w: torch.Tensor, x2: torch.Tensor, w2: torch.Tensor, out2: torch.Tensor | None = None,
+                  relu2: bool = False) -> tuple[torch.Tensor, torch.Tensor]:
+    """``linear(x, w)``, and ``linear(x2, w2)`` or (``relu2``, into ``out2``) ``squared_relu``: in one launch where both are
+    products of the same K that the skinny kernels take (gemv.hip SkinnyBeside), by the first's choice of them."""
+    if _gpu_bf16(x, w) and _gpu_bf16(x2, w2) and x.shape == x2.shape and x.shape[0] <= SKINNY_MAX_M:
+        (M, K), N, N2 = x.shape, w.shape[0], w2.shape[0]
+        v, v2 = _choice(M, N, K, x.stride(0)), _choice(M, N2, K, x2.stride(0))
+        if v in DUAL and v2 in DUAL and (v == v2 or v != 1 != v2) and skinny_supports(v, M, N2, K, x2.stride(0)) and (
+                out2 is None or out2.stride(1) == 1 and out2.stride(0) % 4 == 0 and out2.data_ptr() % 8 == 0):
+            y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+            if out2 is None:
+                out2 = torch.empty((M, N2), dtype=x.dtype, device=x.device)
+            assert out2.shape == (M, N2) and out2.dtype == x.dtype
+            check(hipk().skinny_gemm(y.data_ptr(), x.data_ptr(), w.data_ptr(), M, N, K, x.stride(0), N, v,
+                                     out2.data_ptr(), x2.data_ptr(), w2.data_ptr(), N2, x2.stride(0), out2.stride(0),
+                                     2 if relu2 else 0, stream_ptr(x)), "skinny_gemm")
+            return y, out2
+    y = linear(x, w)
+    if relu2:
+        return y, squared_relu(x2, w2, out2)
+    y2 = linear(x2, w2)
+    return y, y2 if out2 is None else out2.copy_(y2)
 
 
 def _choice(M: int, N: int, K: int, ldx: int) -> int:
@@ -1135,6 +1160,11 @@ def squared_relu(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.T
             return stream_gemm(x, w, "relu2", out=out)
         if kind == "xd":
             return xd_gemm(x, w, "relu2", out=out, form=form)
+        if kind == "skinny" and out.dtype == x.dtype:
+            N = w.shape[0]
+            check(hipk().skinny_gemm(out.data_ptr(), x.data_ptr(), w.data_ptr(), M, N, K, x.stride(0), out.stride(0), form,
+                                     0, 0, 0, 0, 0, 0, 1, stream_ptr(x)), "skinny_gemm")
+            return out
     y = linear(x, w)
     check(hipk().relu2(int(y.dtype == torch.float32), out.data_ptr(), out.stride(0), y.data_ptr(),
                        M, w.shape[0], stream_ptr(x)), "relu2")
@@ -1382,7 +1412,7 @@ def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | Parts:
     return linear(x, w)
 
 
-__all__ = ["linear", "linear_parts", "parts_form", "Parts", "route", "norm_linear", "glu_linear", "norm_glu_row", "norm_glu", "fused_glu_ok",
+__all__ = ["linear", "linear_beside", "linear_parts", "parts_form", "Parts", "route", "norm_linear", "glu_linear", "norm_glu_row", "norm_glu", "fused_glu_ok",
            "linear_residual",
            "residual_fusable", "w4_glu_ok", "w4_ok", "w4_shape_ok", "squared_relu", "w4_group_m", "mfma_gemm",
            "mfma_gemm_grouped",

@@ -424,6 +424,37 @@ def test_xd_gemm_one_tall_tile(hipk, form, M, K, epi):
     _check(out, ref)
 
 
+@pytest.mark.parametrize("v", range(1, 10))
+@pytest.mark.parametrize("M", [1, 2, 3, 8, 9, 16])
+@pytest.mark.parametrize("N,N2,K,relu2", [(256, 128, 512, True), (128, 384, 1536, False), (512, 256, 128, True)])
+def test_two_products_in_a_skinny_launch(hipk, monkeypatch, v, M, N, N2, K, relu2):
+    """Both products on every skinny kernel, or (a shape it does not take) each by itself: fp32 sums rounded once."""
+    monkeypatch.setattr(G, "_choice", lambda *a: v)
+    g = torch.Generator(device="cuda").manual_seed(v + M + K)
+    buf = torch.randn(M, 2 * K, device="cuda", generator=g).to(torch.bfloat16)
+    w, w2 = ((torch.randn(n, K, device="cuda", generator=g) * K ** -0.5).to(torch.bfloat16) for n in (N, N2))
+    wide = torch.full((M, N2 + 16), 7.0, device="cuda", dtype=torch.bfloat16)
+    y, y2 = G.linear_beside(buf[:, :K], w, buf[:, K:], w2, wide[:, 8:8 + N2] if relu2 else None, relu2)
+    want, want2 = buf[:, :K].double() @ w.double().t(), buf[:, K:].double() @ w2.double().t()
+    if relu2:
+        want2 = want2.relu().square()
+        assert y2.data_ptr() == wide[:, 8:].data_ptr() and (wide[:, :8] == 7).all() and (wide[:, 8 + N2:] == 7).all()
+    for got, ref in ((y, want), (y2, want2)):  # one rounding to bf16, two where the pass behind the product squares
+        assert ((got.double() - ref).abs() <= 2.0 ** -6 * ref.abs() + 1e-4).all()
+
+
+def test_squared_relu_of_few_rows(hipk):
+    """Into columns of a wider operand, by the skinny kernels at any of their row counts, against fp64."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    w = (torch.randn(3584, 2048, device="cuda", generator=g) * 0.02).to(torch.bfloat16)
+    for M in (1, 2, 5, 8, 16):
+        x = torch.randn(M, 2048, device="cuda", generator=g).to(torch.bfloat16)
+        a = torch.full((M, 2048 + 3584), 7.0, device="cuda", dtype=torch.bfloat16)
+        G.squared_relu(x, w, a[:, 2048:])
+        want = (x.double() @ w.double().t()).relu().square()
+        assert ((a[:, 2048:].double() - want).abs() <= 2.0 ** -6 * want + 1e-4).all() and (a[:, :2048] == 7).all()
+
+
 @pytest.mark.parametrize("M,N,K", [(129, 32000, 2048), (160, 12800, 2048), (192, 20480, 2048), (224, 32000, 2048)])
 def test_linear_on_one_tall_tile(hipk, M, N, K):
     """The rule's products, aligned ones on its form, others as before."""
