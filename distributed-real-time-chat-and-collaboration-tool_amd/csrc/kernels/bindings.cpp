@@ -248,16 +248,34 @@ PYBIND11_MODULE(_hipk, m) {
   m.def("embed", [](u64 out, u64 ids, int wide, u64 table, int rows, int V, int H, u64 st) {
     return drtc::launch_embed(P<void>(out), P<const void>(ids), wide, P<const void>(table), rows, V, H, S(st));
   });
+  static const auto stage_ranges = [](const std::vector<std::pair<unsigned, unsigned>>& ranges) {
+    drtc::StageRanges r{};
+    if (ranges.size() > drtc::kStageRanges) r.n = -1;
+    else for (const auto& [first, words] : ranges) {
+      r.first[r.n] = first;
+      r.words[r.n++] = words;
+    }
+    return r;
+  };
+  m.def("stage_rows", [](u64 dst, u64 host, const std::vector<std::pair<unsigned, unsigned>>& ranges, u64 st) {
+    return drtc::launch_stage_rows(P<void>(dst), P<const void>(host), stage_ranges(ranges), S(st));
+  });
+  m.def("step_stage", [](u64 dst, u64 host0, u64 host1, const std::vector<std::pair<unsigned, unsigned>>& ranges, u64 ids,
+                         u64 sampled, unsigned src, unsigned host, int B, u64 counter, u64 position, u64 turn, u64 st) {
+    const drtc::StepTokens t{P<int>(ids), P<const int>(sampled), src, host, B, P<int64_t>(counter), P<int64_t>(position)};
+    return drtc::launch_step_stage(P<void>(dst), P<const void>(host0), P<const void>(host1), stage_ranges(ranges), t,
+                                   P<int>(turn), S(st));
+  });
   m.def("step_begin", [](u64 ids, u64 src, u64 sampled, u64 host, int B, u64 counter, u64 position, u64 st) {
     return drtc::launch_step_begin(P<int>(ids), P<const int64_t>(src), P<const int>(sampled), P<const int>(host), B,
                                    P<int64_t>(counter), P<int64_t>(position), S(st));
   });
   m.def("sample", [](u64 out_tokens, u64 logits, int B, int V, int ld,
                      u64 temperature, u64 top_k, u64 top_p, uint64_t seed,
-                     u64 step, u64 st) {
+                     u64 step, u64 turn, u64 host0, u64 host1, u64 st) {
     return drtc::launch_sample(P<int>(out_tokens), P<const void>(logits), B, V, ld,
                                P<const float>(temperature), P<const int>(top_k),
                                P<const float>(top_p), seed,
-                               P<const int64_t>(step), S(st));
+                               P<const int64_t>(step), {P<const int>(turn), {P<int>(host0), P<int>(host1)}}, S(st));
   });
 }

@@ -64,11 +64,32 @@ int launch_prefill_attn(void* out, int out_stride, const void* qkv,
                         hipStream_t st);
 
 int launch_embed(void* out, const void* ids, int wide, const void* table, int rows, int V, int H, hipStream_t st);
+// ranges of words that a step's staging copies, first and count of each
+constexpr int kStageRanges = 12;
+struct StageRanges {
+  int n;
+  unsigned first[kStageRanges], words[kStageRanges];
+};
+int launch_stage_rows(void* dst, const void* host, const StageRanges& r, hipStream_t st);
+// step_begin's, its src and host arrays as words of the staging sets
+struct StepTokens {
+  int* ids;
+  const int* sampled;
+  unsigned src, host;
+  int B;
+  int64_t *counter, *position;
+};
+int launch_step_stage(void* dst, const void* host0, const void* host1, const StageRanges& r, const StepTokens& t, int* turn,
+                      hipStream_t st);
 int launch_step_begin(int* ids, const int64_t* src, const int* sampled, const int* host, int B, int64_t* counter,
                       int64_t* position, hipStream_t st);
+struct SampleMirror {  // launch_step_stage's turn, and the host's token buffers of its two sets (turn null: none)
+  const int* turn;
+  int* host[2];
+};
 int launch_sample(int* out_tokens, const void* logits, int B, int V, int ld,
                   const float* temperature, const int* top_k, const float* top_p,
-                  uint64_t seed, const int64_t* step, hipStream_t st);
+                  uint64_t seed, const int64_t* step, const SampleMirror& mirror, hipStream_t st);
 
 struct MoeOptions {
   int f32 = 0;         // operands fp32 (any sizes); else bf16

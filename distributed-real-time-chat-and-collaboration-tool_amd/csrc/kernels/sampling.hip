@@ -102,6 +102,16 @@ DRTC_DEVICE float wave_max(float x) {
   return x;
 }
 
+// Where a row's token goes: device memory, and for a step's graph the host's buffer of the staging set that it read, which
+// waits for the step anyway (a copy behind the step is 4 us more).
+struct TokenOut {
+  int *tokens, *host;
+  DRTC_DEVICE void put(int row, int token) const {
+    tokens[row] = token;
+    if (host) __hip_atomic_store(host + row, token, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+};
+
 struct SampShared {
   float val[kCand];
   int idx[kCand];
@@ -290,7 +300,7 @@ DRTC_DEVICE int gather_ge(SampShared& s, const unsigned short* lr, int V, bool v
 constexpr int kFew = 128;
 // against the largest: 1 for itself, at +inf too
 DRTC_DEVICE float weight(float v, float top, float inv_t) { return v == top ? 1.f : __expf((v - top) * inv_t); }
-DRTC_DEVICE void sample_few(SampShared& s, int* out_tokens, int row, float temp, int k, int n, float pp,
+DRTC_DEVICE void sample_few(SampShared& s, const TokenOut& out, int row, float temp, int k, int n, float pp,
                             uint64_t seed, uint64_t st) {
   const int tid = threadIdx.x, lane = tid & 63, own = tid >> 3;
   float* const sv = reinterpret_cast<float*>(&s.hist[8][0]);
@@ -356,11 +366,11 @@ DRTC_DEVICE void sample_few(SampShared& s, int* out_tokens, int row, float temp,
     const uint64_t hit = __ballot(i <= cut && target >= lo[z] && (target < x[z] || i == cut));
     if (hit) at = 64 * z + 63 - __clzll((long long)hit);
   }
-  if (lane == 0) out_tokens[row] = si[at];
+  if (lane == 0) out.put(row, si[at]);
 }
 
 template <int U>
-DRTC_DEVICE void sample_topk(SampShared& s, int* out_tokens, const unsigned short* lr, int V,
+DRTC_DEVICE void sample_topk(SampShared& s, const TokenOut& out, const unsigned short* lr, int V,
                              bool vec, int row, float temp, int k, float pp, uint64_t seed,
                              uint64_t st) {
   const int tid = threadIdx.x;
@@ -410,11 +420,11 @@ DRTC_DEVICE void sample_topk(SampShared& s, int* out_tokens, const unsigned shor
     n = min(gather_ge<U>(s, lr, V, vec, thr), kCand);
   }
   if (n == 0) {
-    if (tid == 0) out_tokens[row] = -1;
+    if (tid == 0) out.put(row, -1);
     return;
   }
   if (n <= kFew) {
-    sample_few(s, out_tokens, row, temp, k, n, pp, seed, st);
+    sample_few(s, out, row, temp, k, n, pp, seed, st);
     return;
   }
   int np2 = 1;
@@ -478,11 +488,11 @@ DRTC_DEVICE void sample_topk(SampShared& s, int* out_tokens, const unsigned shor
     if (target >= lo && (target < s.val[tid] || tid == cut)) s.misc[0] = tid;
   }
   __syncthreads();
-  if (tid == 0) out_tokens[row] = s.idx[s.misc[0]];
+  if (tid == 0) out.put(row, s.idx[s.misc[0]]);
 }
 
 template <int U>
-DRTC_DEVICE void sample_topp_full(SampShared& s, int* out_tokens, const unsigned short* lr, int V,
+DRTC_DEVICE void sample_topp_full(SampShared& s, const TokenOut& out, const unsigned short* lr, int V,
                                   bool vec, int row, float temp, float pp, uint64_t seed,
                                   uint64_t st) {
   const int tid = threadIdx.x;
@@ -547,7 +557,7 @@ DRTC_DEVICE void sample_topp_full(SampShared& s, int* out_tokens, const unsigned
     const unsigned kj = (unsigned)s.misc[1];
     __syncthreads();
     if (pp >= 1.f || kj >= H || round == kMaxRounds - 1) {
-      if (tid == 0) out_tokens[row] = j;
+      if (tid == 0) out.put(row, j);
       return;
     }
     // ---- verify: mass above key_j, plus the bisection key between L and H
@@ -574,7 +584,7 @@ DRTC_DEVICE void sample_topp_full(SampShared& s, int* out_tokens, const unsigned
       block_sum2(s, a_t, f_t, A, F);
     }
     if (A < P) {  // token j is inside the nucleus
-      if (tid == 0) out_tokens[row] = j;
+      if (tid == 0) out.put(row, j);
       return;
     }
     // key_j and everything below it is outside
@@ -597,7 +607,7 @@ __global__ __launch_bounds__(kSampThreads, 4 * OCC) void sample_kernel(
     int* __restrict__ out_tokens, const bf16_t* __restrict__ logits, int V,
     int ld, const float* __restrict__ temperature, const int* __restrict__ top_k,
     const float* __restrict__ top_p, uint64_t seed,
-    const int64_t* __restrict__ step) {
+    const int64_t* __restrict__ step, SampleMirror mirror) {
   constexpr int U = OCC == 1 ? kUnroll : 2;
   const int row = blockIdx.x;
   const int tid = threadIdx.x;
@@ -605,6 +615,7 @@ __global__ __launch_bounds__(kSampThreads, 4 * OCC) void sample_kernel(
   const unsigned short* lr = (const unsigned short*)(logits + (int64_t)row * ld);
   const bool vec = ((reinterpret_cast<uintptr_t>(lr) & 15) == 0);
   const float temp = temperature ? temperature[row] : 0.f;
+  const TokenOut out{out_tokens, mirror.turn ? mirror.host[~*mirror.turn & 1] : nullptr};  // (the turn is the next step's)
   __shared__ SampShared s;
 
   if (temp <= 0.f) {  // ---------------------------------- greedy argmax
@@ -625,7 +636,7 @@ __global__ __launch_bounds__(kSampThreads, 4 * OCC) void sample_kernel(
     if (tid == 0) {
       for (int w = 1; w < kSampWaves; ++w)
         if (s.val[w] > best || (s.val[w] == best && s.idx[w] < bi)) { best = s.val[w]; bi = s.idx[w]; }
-      out_tokens[row] = bi < V ? bi : -1;
+      out.put(row, bi < V ? bi : -1);
     }
     return;
   }
@@ -634,9 +645,9 @@ __global__ __launch_bounds__(kSampThreads, 4 * OCC) void sample_kernel(
   int k = top_k ? top_k[row] : 0;
   if (k >= V) k = 0;
   if (k > 0) {
-    sample_topk<U>(s, out_tokens, lr, V, vec, row, temp, min(k, kCand), pp, seed, st);
+    sample_topk<U>(s, out, lr, V, vec, row, temp, min(k, kCand), pp, seed, st);
   } else {
-    sample_topp_full<U>(s, out_tokens, lr, V, vec, row, temp, pp, seed, st);
+    sample_topp_full<U>(s, out, lr, V, vec, row, temp, pp, seed, st);
   }
 }
 
@@ -660,6 +671,98 @@ __global__ __launch_bounds__(256) void step_begin_kernel(int* __restrict__ ids, 
   }
 }
 
+// A step's inputs from pinned host memory: the words of a few ranges, as far as the batch uses them, read over the bus by
+// the chip itself, at system scope (nothing of the step before stays in a cache).  A copy of the whole staging buffer is
+// handed to the copy engines from some ten kilobytes on, which the chain of a step waits for.
+DRTC_DEVICE unsigned host_word(const unsigned* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+DRTC_DEVICE void stage_words(unsigned* dst, const unsigned* host, unsigned first, unsigned words) {
+  const unsigned i = blockIdx.x * 1024 + threadIdx.x;
+  unsigned v[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (i + 256 * j < words) v[j] = host_word(host + first + i + 256 * j);
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (i + 256 * j < words) dst[first + i + 256 * j] = v[j];
+}
+__global__ __launch_bounds__(256) void stage_rows_kernel(unsigned* __restrict__ dst, const unsigned* host, StageRanges r) {
+  stage_words(dst, host, r.first[blockIdx.y], r.words[blockIdx.y]);
+}
+
+// The same along with the start of the step, the first node of its graph: the two staging sets take turns, and the last
+// workgroup to have looked whose turn it is gives it to the other (turn: set, workgroups that have looked).  Steps, us, with the
+// copies and step_begin / with this and the sampler's own writes to the host: one row 190.1 / 187.6, alone on the chip 211 /
+// 204; 224 of 256 rows 627 / 612, 64 of 64 597 / 582.
+__global__ __launch_bounds__(256) void step_stage_kernel(unsigned* __restrict__ dst, const unsigned* host0, const unsigned* host1,
+                                                         StageRanges r, StepTokens t, int* turn) {
+  // the tokens are what a step waits for: both sets' are on their way with the turn, one trip over the bus
+  unsigned ahead[6];
+  const int first = blockIdx.x * 1024 + threadIdx.x;
+  if ((int)blockIdx.y == r.n && first < t.B) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const unsigned* h = k ? host1 : host0;
+      ahead[3 * k] = host_word(h + t.src + 2 * first);
+      ahead[3 * k + 1] = host_word(h + t.src + 2 * first + 1);
+      ahead[3 * k + 2] = host_word(h + t.host + first);
+    }
+  }
+  const int set = __hip_atomic_load(turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const unsigned* host = set & 1 ? host1 : host0;
+  __syncthreads();
+  if (threadIdx.x == 0 &&
+      __hip_atomic_fetch_add(turn + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)(gridDim.x * gridDim.y) - 1) {
+    __hip_atomic_store(turn + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(turn, set ^ 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if ((int)blockIdx.y < r.n) {
+    stage_words(dst, host, r.first[blockIdx.y], r.words[blockIdx.y]);
+    return;
+  }
+  for (int i = blockIdx.x * 1024 + threadIdx.x; i < min(t.B, (int)(blockIdx.x + 1) * 1024); i += 256) {
+    const int e = i - blockIdx.x * 1024 >= 256;  // (the first ones are asked for ahead)
+    unsigned lo = ahead[0], hi = ahead[1], id = ahead[2];
+    if (e) {
+      lo = host_word(host + t.src + 2 * i), hi = host_word(host + t.src + 2 * i + 1), id = host_word(host + t.host + i);
+    } else if (set & 1) {
+      lo = ahead[3], hi = ahead[4], id = ahead[5];
+    }
+    const int64_t s = (int64_t)((uint64_t)hi << 32 | lo);
+    t.ids[i] = s < 0 ? (int)id : s < t.B ? t.sampled[s] : -1;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    const int64_t c = *t.counter;
+    *t.position = c;
+    *t.counter = c + 1;
+  }
+}
+
+static bool stage_ok(const void* dst, const StageRanges& r, unsigned& most) {
+  most = 0;
+  if (r.n < 0 || r.n > kStageRanges || (uintptr_t)dst % 4) return false;
+  for (int i = 0; i < r.n; ++i) most = std::max(most, r.words[i]);
+  return true;
+}
+
+int launch_stage_rows(void* dst, const void* host, const StageRanges& r, hipStream_t st) {
+  unsigned most;
+  if (!stage_ok(dst, r, most) || (uintptr_t)host % 4) return -1;
+  if (most == 0) return 0;
+  stage_rows_kernel<<<dim3((most + 1023) / 1024, r.n), 256, 0, st>>>((unsigned*)dst, (const unsigned*)host, r);
+  return (int)hipGetLastError();
+}
+
+int launch_step_stage(void* dst, const void* host0, const void* host1, const StageRanges& r, const StepTokens& t, int* turn,
+                      hipStream_t st) {
+  unsigned most;
+  if (!stage_ok(dst, r, most) || (uintptr_t)host0 % 4 || (uintptr_t)host1 % 4 || t.B <= 0) return -1;
+  step_stage_kernel<<<dim3((std::max(most, (unsigned)t.B) + 1023) / 1024, r.n + 1), 256, 0, st>>>(
+      (unsigned*)dst, (const unsigned*)host0, (const unsigned*)host1, r, t, turn);
+  return (int)hipGetLastError();
+}
+
 int launch_step_begin(int* ids, const int64_t* src, const int* sampled, const int* host, int B, int64_t* counter,
                       int64_t* position, hipStream_t st) {
   if (B <= 0) return B == 0 ? 0 : -1;
@@ -669,8 +772,9 @@ int launch_step_begin(int* ids, const int64_t* src, const int* sampled, const in
 
 int launch_sample(int* out_tokens, const void* logits, int B, int V, int ld,
                   const float* temperature, const int* top_k, const float* top_p,
-                  uint64_t seed, const int64_t* step, hipStream_t st) {
+                  uint64_t seed, const int64_t* step, const SampleMirror& mirror, hipStream_t st) {
   if (B == 0) return 0;
+  if (mirror.turn && (!mirror.host[0] || !mirror.host[1])) return -1;
   // two workgroups per CU by default: B = 1024, V = 128k, top-k 64 / top-p 0.95 in 76.5 vs
   // 106.0 us, greedy 44.8 vs 58.1, full-vocabulary top-p 179 vs 237 (profiles/r3v);
   // DRTC_SAMPLER_OCC=1 restores one per CU
@@ -680,10 +784,10 @@ int launch_sample(int* out_tokens, const void* logits, int B, int V, int ld,
   }();
   if (occ == 2)
     hipLaunchKernelGGL(sample_kernel<2>, dim3(B), dim3(kSampThreads), 0, st, out_tokens,
-                       (const bf16_t*)logits, V, ld, temperature, top_k, top_p, seed, step);
+                       (const bf16_t*)logits, V, ld, temperature, top_k, top_p, seed, step, mirror);
   else
     hipLaunchKernelGGL(sample_kernel<1>, dim3(B), dim3(kSampThreads), 0, st, out_tokens,
-                       (const bf16_t*)logits, V, ld, temperature, top_k, top_p, seed, step);
+                       (const bf16_t*)logits, V, ld, temperature, top_k, top_p, seed, step, mirror);
   return (int)hipGetLastError();
 }
 

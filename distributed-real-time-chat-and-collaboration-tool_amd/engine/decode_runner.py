@@ -93,8 +93,11 @@ class DecodeRunner:
         self.h_out = [torch.zeros(B, dtype=torch.int32, pin_memory=pin) for _ in range(2)]
         self.events = [torch.cuda.Event() if pin else None for _ in range(2)]
         self._k = 0
+        # the set that the next replay reads (ops.step_stage), on the device and as the host has it
+        self.turn, self._turn = torch.zeros(2, dtype=torch.int32, device=dev), 0
         self.n_i32 = n_i32
         self._metas = {}
+        self._stagings: dict[tuple[int, int], ops.StageRows] = {}
         self._graphs = {}
         self._pool = None
         # DRTC_TIME_DECODE=1: GPU time of every replay (hipEvents), for host-
@@ -124,6 +127,18 @@ class DecodeRunner:
         return (stage[:16 * B].view(torch.int64), stage[16 * B:-8 * B].view(torch.int32),
                 stage[-8 * B:].view(torch.float32))
 
+    def _staging(self, Bb: int, k: int) -> ops.StageRows:
+        """The copy of what a step of Bb rows reads of staging set k."""
+        r = self._stagings.get((Bb, k))
+        if r is None:
+            B, MB = self.max_batch, self.max_blocks
+            i32, f32 = 16 * B, 16 * B + 4 * self.n_i32
+            at = [(8 * B * j, 8 * Bb) for j in (0, 1)] + [(i32 + 4 * B * j, 4 * Bb) for j in range(4)]
+            at += [(i32 + 16 * B, 4 * Bb * MB), (i32 + 4 * B * (4 + MB), 4 * Bb)]
+            at += [(f32 + 4 * B * j, 4 * Bb) for j in (0, 1)]
+            r = self._stagings[Bb, k] = ops.StageRows(self.stage, self.h_stage[k], [(a, a + n) for a, n in at])
+        return r
+
     # ------------------------------------------------------------------
     def bucket(self, n: int) -> int:
         i = bisect.bisect_left(self.buckets, n)
@@ -141,12 +156,17 @@ class DecodeRunner:
             self._metas[Bb] = m
         return m
 
-    def _forward(self, Bb: int) -> None:
+    def _forward(self, Bb: int, stage: bool = False) -> None:
+        """A step of the device's staging buffer, or (``stage``, in a graph) of the set whose turn it is."""
         meta = self._meta(Bb)
         # input tokens: the previous step's samples still on the device
         # (pipelined steps, src >= 0) or host-provided ids (src = -1)
         ids = self.ids_used[:Bb]
-        ops.step_begin(ids, self.src[:Bb], self.out[:Bb], self.ids[:Bb], self.step_ctr, self.step_at)
+        if stage:
+            ops.step_stage([self._staging(Bb, k) for k in (0, 1)], ids, 8 * self.max_batch, 16 * self.max_batch,
+                           self.out[:Bb], self.step_ctr, self.step_at, self.turn)
+        else:
+            ops.step_begin(ids, self.src[:Bb], self.out[:Bb], self.ids[:Bb], self.step_ctr, self.step_at)
         if not (self.device.type == "cuda" and torch.cuda.is_current_stream_capturing()):
             self._ctr += 1
         logits = self.model.forward_decode(ids, meta, self.kv,
@@ -154,7 +174,7 @@ class DecodeRunner:
         if self.keep_logits:
             self.logits[Bb] = logits
         ops.sample(logits.to(torch.bfloat16), self.temp[:Bb], self.topk[:Bb], self.topp[:Bb], seed=self.seed,
-                   step=self.step_at, out=self.out[:Bb])
+                   step=self.step_at, out=self.out[:Bb], mirror=(self.turn, self.h_out) if stage else None)
 
     def capture(self, Bb: int) -> None:
         if not self.use_graphs or Bb in self._graphs:
@@ -175,7 +195,7 @@ class DecodeRunner:
             self._pool = torch.cuda.graph_pool_handle()
         g = torch.cuda.CUDAGraph()
         with torch.cuda.graph(g, pool=self._pool):
-            self._forward(Bb)
+            self._forward(Bb, stage=True)
         torch.cuda.synchronize(self.device)
         self._graphs[Bb] = g
 
@@ -234,8 +254,11 @@ class DecodeRunner:
         hf[B:B + n] = topp
         hf[B + n:B + Bb] = 1.0
         nb = self.device.type == "cuda"
-        self.stage.copy_(self.h_stage[k], non_blocking=nb)
         g = self._graphs.get(Bb)
+        if g is None:
+            self._staging(Bb, k)()
+        elif self._turn != k:  # a step without a graph came between
+            self.turn[:1].fill_(k)
         timing = nb and self.time_gpu
         if timing:
             ev0 = torch.cuda.Event(enable_timing=True)
@@ -245,21 +268,24 @@ class DecodeRunner:
         with tracing.span("decode.graph_replay" if g is not None else "decode.eager", bucket=Bb):
             if g is not None:
                 g.replay()
+                self._turn = k ^ 1
                 self._ctr += 1
             else:
                 self._forward(Bb)
         if timing:
             ev1.record()
             self._timing[k] = (ev0, ev1)
-        self._readback(n, k)
+        self._readback(n, k, g is None)
         self._pending.append({"n": n, "k": k, "Bb": Bb, "step": self._step_no, "ctr": ctr})
         del self._pending[:-2]  # two staging sets: at most two steps in flight
         self._step_no += 1
         return n, k
 
-    def _readback(self, n: int, k: int) -> None:
+    def _readback(self, n: int, k: int, tokens: bool = True) -> None:
+        """What the host reads of a step; ``tokens``: not written there by the step itself."""
         nb = self.device.type == "cuda"
-        self.h_out[k][:n].copy_(self.out[:n], non_blocking=nb)
+        if tokens:
+            self.h_out[k][:n].copy_(self.out[:n], non_blocking=nb)
         if self.ep:
             self.h_in[k][:n].copy_(self.ids_used[:n], non_blocking=nb)
             self.h_ovf[k].copy_(self.model.ep_overflow.count, non_blocking=nb)

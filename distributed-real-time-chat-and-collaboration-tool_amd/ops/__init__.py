@@ -32,7 +32,7 @@ from .norm_conv import (MAX_TAPS, ConvTiles, LayerNorm, conv_tile_rows, norm_con
                         softcap_)
 from .norm_side import side_gate, side_input, side_norm, side_router_ok, stream_add
 from .rope import build_rope_cache, kv_write_v, kv_write_v_ref, rope_kv_, rope_kv_ref
-from .sampling import sample, sample_ref, step_begin
+from .sampling import StageRows, sample, sample_ref, step_begin, step_stage
 from .talking import (MIX_TILE, STATS_TILE, TalkDecodeWorkspace, TalkPortions, TalkWeights,
                       head_prep, pad8, talk_cache_shapes, talk_decode, talk_prefill)
 
@@ -44,7 +44,7 @@ __all__ = [
     "decode_partitioning", "paged_decode_attention", "paged_decode_attention_rope",
     "paged_decode_ref", "prefill_attention", "prefill_attention_ref", "prefill_tiles",
     "set_prefill_persist", "rmsnorm", "rmsnorm_ref", "build_rope_cache", "rope_kv_",
-    "rope_kv_ref", "kv_write_v", "kv_write_v_ref", "sample", "sample_ref", "step_begin", "dyt", "dyt_ref",
+    "rope_kv_ref", "kv_write_v", "kv_write_v_ref", "sample", "sample_ref", "StageRows", "step_begin", "step_stage", "dyt", "dyt_ref",
     "embed",
     "gated", "DeltaWeights", "Portions", "delta_decode", "delta_scan", "short_conv",
     "LatentDecodeWorkspace", "PortionKeys", "build_interleaved_rope", "head_linear",

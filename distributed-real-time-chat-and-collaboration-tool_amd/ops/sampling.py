@@ -67,8 +67,12 @@ def sample_ref(logits: torch.Tensor, temperature: torch.Tensor | None = None,
 def sample(logits: torch.Tensor, temperature: torch.Tensor | None = None,
            top_k: torch.Tensor | None = None, top_p: torch.Tensor | None = None,
            seed: int = 0, step: torch.Tensor | None = None,
-           out: torch.Tensor | None = None) -> torch.Tensor:
+           out: torch.Tensor | None = None,
+           mirror: tuple[torch.Tensor, list[torch.Tensor]] | None = None) -> torch.Tensor:
     """logits [B, V] bf16 -> int32 token ids [B].
+
+    ``mirror``: (turn, two pinned int32 buffers), behind ``step_stage`` on the GPU: the tokens go to the buffer of the set
+    that it read as well.
 
     temperature/top_k/top_p are per-row device tensors (float32 / int32 /
     float32); ``step`` is an int64 device scalar the caller advances.  On the GPU a
@@ -93,10 +97,50 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor | None = None,
     if out is None:
         out = torch.empty(B, dtype=torch.int32, device=logits.device)
     assert out.dtype == torch.int32 and out.is_contiguous()
+    turn, hosts = mirror or (None, (None, None))
+    assert turn is None or turn.dtype == torch.int32 and turn.is_cuda
+    for h in hosts if mirror else ():
+        assert h.dtype == torch.int32 and h.is_contiguous() and h.numel() >= B and h.is_pinned()
     check(hipk().sample(out.data_ptr(), logits.data_ptr(), B, V, logits.stride(0),
                         ptr(temperature), ptr(top_k), ptr(top_p), int(seed) & ((1 << 64) - 1),
-                        ptr(step), stream_ptr(logits)), "sample")
+                        ptr(step), ptr(turn), ptr(hosts[0]), ptr(hosts[1]), stream_ptr(logits)), "sample")
     return out
+
+
+class StageRows:
+    """``dst[a:b] = host[a:b]`` for the byte ranges (a, b), multiples of 4, of two uint8 buffers of one size, at every call.
+    On the GPU ``host`` is pinned, and a kernel reads it: it stays unchanged until the stream is past it."""
+
+    def __init__(self, dst: torch.Tensor, host: torch.Tensor, ranges: list[tuple[int, int]]):
+        assert dst.shape == host.shape and dst.dtype == host.dtype == torch.uint8
+        assert dst.is_contiguous() and host.is_contiguous()
+        assert all(0 <= a <= b <= dst.numel() and a % 4 == b % 4 == 0 for a, b in ranges)
+        self.dst, self.host, self.ranges = dst, host, ranges
+        self.kernel = on_gpu(dst) and host.is_pinned()
+        self.args = dst.data_ptr(), host.data_ptr(), [(a // 4, (b - a) // 4) for a, b in ranges]
+
+    def __call__(self) -> None:
+        if self.kernel:
+            check(hipk().stage_rows(*self.args, stream_ptr(self.dst)), "stage_rows")
+            return
+        for a, b in self.ranges:
+            self.dst[a:b].copy_(self.host[a:b])
+
+
+def step_stage(stages: list[StageRows], ids: torch.Tensor, src: int, host: int, sampled: torch.Tensor,
+               counter: torch.Tensor, position: torch.Tensor, turn: torch.Tensor) -> None:
+    """One of two ``StageRows`` of one destination and ranges, and ``step_begin`` with src and host at these byte offsets of
+    its staging set, in one launch: the set is ``turn[0]``, which the launch gives to the other one (int32 [2], [1] 0)."""
+    a, b = stages
+    B, size = ids.numel(), a.dst.numel()
+    assert a.kernel and b.kernel and a.dst is b.dst and a.ranges == b.ranges and src % 8 == host % 4 == 0
+    assert 0 <= src <= size - 8 * B and 0 <= host <= size - 4 * B
+    for t, dt, n in ((ids, torch.int32, B), (sampled, torch.int32, B), (counter, torch.int64, 1),
+                     (position, torch.int64, 1), (turn, torch.int32, 2)):
+        assert t.dtype == dt and t.is_contiguous() and t.numel() == n and t.is_cuda
+    check(hipk().step_stage(a.args[0], a.args[1], b.args[1], a.args[2], ids.data_ptr(), sampled.data_ptr(), src // 4,
+                            host // 4, B, counter.data_ptr(), position.data_ptr(), turn.data_ptr(), stream_ptr(ids)),
+          "step_stage")
 
 
 def step_begin(ids: torch.Tensor, src: torch.Tensor, sampled: torch.Tensor, host: torch.Tensor,

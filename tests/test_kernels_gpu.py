@@ -1,6 +1,7 @@
 """Numerics of every HIP kernel against the fp32 PyTorch reference of the same op."""
 import math
 
+import numpy as np
 import pytest
 import torch
 
@@ -744,6 +745,76 @@ def test_fused_moe_grouped_xd_forms(hipk, T, H, I, E, k, gu, dn, act):
     y = ops.fused_moe(x, lg, wgu, wdn, k, act, variant=3, gu_form=gu, dn_form=dn)
     _close(y, ops.fused_moe_ref(x, lg, wgu, wdn, k, act), 3e-2, 3e-2, f"moe xd {gu}/{dn}")
     G.check_splitk_fault()
+
+
+@pytest.mark.parametrize("B,extra", [(1, 0), (5, 3), (256, 5000), (1500, 40000)])
+def test_step_stage_takes_turns(hipk, B, extra):
+    """Staging sets in turn, from a graph: the copied ranges, the tokens as step_begin gives them, the counter."""
+    n = 8 * B + 4 * B + 4 * extra + 4
+    hosts = [torch.zeros(n, dtype=torch.uint8, pin_memory=True) for _ in range(2)]
+    dst = torch.zeros(n, dtype=torch.uint8, device=DEV)
+    ranges = [(0, 8 * B), (8 * B, 12 * B), (12 * B, n - 4)]
+    stages = [ops.StageRows(dst, h, ranges) for h in hosts]
+    sampled = torch.arange(100, 100 + B, dtype=torch.int32, device=DEV)
+    ids = torch.zeros(B, dtype=torch.int32, device=DEV)
+    counter, position = torch.full((1,), 7, dtype=torch.int64, device=DEV), torch.zeros(1, dtype=torch.int64, device=DEV)
+    turn = torch.zeros(2, dtype=torch.int32, device=DEV)
+    outs = [torch.full((B + 3,), -7, dtype=torch.int32, pin_memory=True) for _ in range(2)]
+    logits = torch.randn(B, 512, device=DEV).to(torch.bfloat16)
+    picks = torch.zeros(B, dtype=torch.int32, device=DEV)
+    temp, top_k = torch.arange(B, device=DEV).remainder(3) * 0.5, torch.arange(B, device=DEV).remainder(5).int() * 40
+
+    def step():
+        ops.step_stage(stages, ids, 0, 8 * B, sampled, counter, position, turn)
+        ops.sample(logits, temp.float(), top_k, None, seed=3, step=position, out=picks, mirror=(turn, outs))
+
+    step()  # (warm, on the second set after it)
+    turn.zero_()
+    counter.fill_(7)
+    torch.cuda.synchronize()
+    gr = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(gr):
+        step()
+    rng = np.random.default_rng(B)
+    for i in range(12):
+        h = hosts[i & 1].numpy()
+        src = rng.integers(-1, B + 2, B)
+        h[:8 * B] = src.astype(np.int64).view(np.uint8)
+        host_ids = rng.integers(0, 9999, B).astype(np.int32)
+        h[8 * B:12 * B] = host_ids.view(np.uint8)
+        h[12 * B:] = rng.integers(0, 256, n - 12 * B)
+        gr.replay()
+        torch.cuda.synchronize()
+        want = np.where(src < 0, host_ids, np.where(src < B, 100 + src, -1))
+        assert (ids.cpu().numpy() == want).all()
+        assert (dst[:n - 4].cpu().numpy() == h[:n - 4]).all() and not dst[n - 4:].any()
+        assert (int(position), int(counter), turn.tolist()) == (7 + i, 8 + i, [(i + 1) & 1, 0])
+        assert torch.equal(outs[i & 1][:B], picks.cpu()) and (outs[i & 1][B:] == -7).all()
+        assert torch.equal(picks, ops.sample(logits, temp.float(), top_k, None, seed=3, step=position))
+        outs[i & 1].fill_(-7)
+
+
+@pytest.mark.parametrize("n", [12, 4096, 300000])
+def test_stage_rows_reads_what_the_host_wrote_last(hipk, n):
+    """Ranges of a pinned buffer, rewritten between the launches that read them; bytes outside stay as they were."""
+    n = n // 4 * 4
+    host = torch.zeros(n, dtype=torch.uint8, pin_memory=True)
+    dst = torch.full((n,), 255, dtype=torch.uint8, device=DEV)
+    ranges = [(0, 4), (n // 8 * 4, n // 8 * 4), (n // 8 * 4 + 4, n)]
+    seen = dst.clone()
+    copy = ops.StageRows(dst, host, ranges)
+    for step in range(50):
+        host.fill_(step + 1)
+        host[-1] = step
+        copy()
+        torch.cuda.synchronize()
+        for a, b in ranges:
+            seen[a:b] = step + 1
+        seen[-1] = step
+        assert torch.equal(dst, seen)
+    with pytest.raises(AssertionError):
+        ops.StageRows(dst, host, [(0, n + 4)])
+    assert hipk.stage_rows(dst.data_ptr(), host.data_ptr(), [(0, 1)] * 13, 0) == -1
 
 
 @pytest.mark.parametrize("T,H,I,E,k,gu,dn", [
