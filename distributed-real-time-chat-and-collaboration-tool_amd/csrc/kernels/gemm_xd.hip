@@ -33,6 +33,8 @@
 //     [vmcnt: own DMA of tile t + 1 landed, lgkmcnt(0), ONE barrier: everyone's tile t + 1
 //     landed and every read of stage t done]; half 1 MFMAs | LDS-DMA of tile t + S into stage
 //     t + ds_read of tile t + 1 half 0.  The first K tile accumulates onto a zero C operand.
+//     Rings of two stages: a second barrier right behind half 1's fragment reads, and the
+//     LDS-DMA of tile t + 2 from there on.
 //   * Split-K with a ticket-first combine: each slice draws a ticket when its K loop ends;
 //     tickets 0 .. splitk - 2 write their fp32 tile to their slice's slab slot (write-through
 //     sc1 stores, drained, barrier) and count themselves ready; the last ticket (resident, and
@@ -78,6 +80,14 @@ struct XdCfg {
   static constexpr int H = FA * NF;                // MFMAs per 32-deep K half (per wave)
   static constexpr int DA = FA, DB = NF, D = DA + DB;  // LDS-DMA per wave per K tile
   static constexpr int NR = FA + NF;               // fragment reads per wave per K half
+  // The MFMA behind which a stage is free (half 1's fragments have been read).  Its next K tile's loads are spread over
+  // those from there on, EARLY of them ahead of the boundary of the halves.  In a ring of two stages they are due at
+  // the next boundary: from half 1 on alone the boundary waited for them (256 x 256: 14336 x 4096 gated, 1024 rows
+  // 104 -> 96 us, 512 rows 90 -> 84; 32000 x 2048, 1024 rows 124 -> 115).  Deeper rings gain nothing from it (256 x 128
+  // 43.6 / 43.5, 128 x 128 42.5 / 42.7, 128 x 192 52.4 / 53.0) and stay with one barrier.
+  static constexpr int FREE = S == 2 ? NR + 3 : H - 1;
+  static constexpr int LOADS = 2 * H - 1 - FREE;   // MFMAs that loads are spread over
+  static constexpr int EARLY = FREE < H - 1 ? (D * (H - 2 - FREE) + LOADS - 1) / LOADS : 0;
   static constexpr int BOFF = TM * 128;            // B region within a stage
   static constexpr int STAGE = BOFF + TN * 128;
   static constexpr int LDS = S * STAGE;            // the K-tile ring
@@ -212,16 +222,23 @@ DRTC_DEVICE void xd_step(f32x4 (&acc)[C::FA][C::NF], bf16x8 (&fa0)[C::FA], bf16x
     xd_reads<C, (rem * C::NR + H - 1) / H, ((rem + 1) * C::NR + H - 1) / H>(fa1, fb1, lds, cur, f.ra1, f.rb1);
   else if constexpr (h == 0 && Q >= 1 && Q <= C::NR)
     xd_read<C, Q - 1>(fa1, fb1, lds, cur, f.ra1, f.rb1);
-  // ---- boundary: tile t + 1 landed for every wave; every read of this stage is done
-  if constexpr (NEXT && Q == H - 1) {
-    wait_vm<WT * C::D>();  // WT younger K tiles of this wave may still be in flight
+  // ---- every read of this stage is done
+  if constexpr (DMA && Q == C::FREE && C::FREE < H - 1) {
     xd_lgkm0();
     xd_barrier();
   }
-  // ---- half 1: DMA of tile t + S into this stage, spread over the half; the next tile's
-  // half-0 fragments in between
-  if constexpr (DMA && h == 1)
-    xd_dmas<C, (rem * C::D + H - 1) / H, ((rem + 1) * C::D + H - 1) / H>(d, cur, kb);
+  // ---- boundary: tile t + 1 landed for every wave
+  if constexpr (NEXT && Q == H - 1) {
+    // WT younger K tiles of this wave may still be in flight, and what this one has asked for
+    wait_vm<WT * C::D + (DMA ? C::EARLY : 0)>();
+    if constexpr (!DMA || C::FREE == H - 1) xd_lgkm0();
+    xd_barrier();
+  }
+  // ---- DMA of tile t + S into this stage, from when it is free; in half 1 the next tile's half-0 fragments in between
+  if constexpr (DMA && Q > C::FREE) {
+    constexpr int u = Q - C::FREE - 1;
+    xd_dmas<C, (u * C::D + C::LOADS - 1) / C::LOADS, ((u + 1) * C::D + C::LOADS - 1) / C::LOADS>(d, cur, kb);
+  }
   if constexpr (NEXT && h == 1)
     xd_reads<C, (rem * C::NR + H - 1) / H, ((rem + 1) * C::NR + H - 1) / H>(fa0, fb0, lds, nxt,
                                                                            f.ra0, f.rb0);
