@@ -128,7 +128,7 @@ PYBIND11_MODULE(_hipk, m) {
     return drtc::launch_gemm_w4_grouped(P<void>(c), P<const void>(a), P<const void>(b),
                                         P<const int>(grp), n_grp, max_rows, N, K, lda, ldb, ldc,
                                         b_grp, epi, up_off, group_m, ksplit, c_split, limit,
-                                        S(st));
+                                        nullptr, 0, S(st));
   });
   // gemm_xd (ops.gemm.xd_gemm): decode-shaped tiles, XCD-partitioned order, split-K 1..8
   m.def("gemm_xd", [](u64 c, u64 a, u64 b, u64 r, int M, int N, int K, int lda, int ldb, int ldc,

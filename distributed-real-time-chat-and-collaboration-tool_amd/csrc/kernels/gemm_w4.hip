@@ -59,6 +59,7 @@ constexpr int kW4BOff = 32768;                 // B region within a stage
 constexpr int kW4BBlk = 1040;                  // bytes per 8-row B block
 constexpr int kW4Stage = kW4BOff + 32 * kW4BBlk;  // 66048
 constexpr int kW4Lds = 2 * kW4Stage;
+constexpr int kW4Rows = 1024;  // V & 128: a tile's row indexes behind the ring, 64 words a wave
 
 enum { W4_STORE = 0, W4_RESIDUAL = 1, W4_SILU = 2, W4_GELU = 3, W4_RELU2 = 4, W4_CLAMP = 5 };
 
@@ -91,6 +92,9 @@ struct W4Params {
   int ksplit;
   int64_t c_split;
   float limit;  // W4_CLAMP: bound of the gate and up values
+  // V & 128: row r of the groups is row aidx[r] of A, which has a_bytes
+  const int* aidx;
+  unsigned a_bytes;
 };
 
 // Position of one output tile: row tile tm, column tile tn; grouped form: rows [row0,
@@ -205,6 +209,7 @@ struct W4Tile {
 //          MFMA 63) instead of one per MFMA at 104-119: the burst ran the LDS array at its
 //          256 B/clk limit beside the landing LDS-DMA (PMC: +72 % SQ_WAIT_INST_LDS against
 //          hipBLASLt's kernel of the same tile, profiles/r4j)
+//   V & 64 grouped form; V & 128 its A rows are read through an index list
 template <int V, bool DMA, bool NEXT, bool Z, int Q>
 DRTC_DEVICE void w4_step(f32x4 (&acc)[8][8], bf16x8 (&fa0)[8], bf16x8 (&fb0)[8],
                          bf16x8 (&fa1)[8], bf16x8 (&fb1)[8], const W4Tile& T, const W4Dma& d) {
@@ -257,8 +262,8 @@ DRTC_DEVICE void w4_step(f32x4 (&acc)[8][8], bf16x8 (&fa0)[8], bf16x8 (&fb0)[8],
     if constexpr (DMA && Z) {
       // first K step of a persistent tile: the previous tile's epilogue stores sit between
       // the DMA of K step 1 (needed now) and this step's DMA - do not wait for them
-      if (T.seam)
-        w4_vmcnt<32 + kYoung>();
+      if (T.seam)  // (V & 128: and the next tile's row indexes)
+        w4_vmcnt<32 + ((V & 128) != 0) + kYoung>();
       else
         w4_vmcnt<kYoung>();
     } else if constexpr (DMA) {
@@ -630,13 +635,16 @@ DRTC_DEVICE void w4_plan(W4Dma& d, const W4Params& p, const W4Pos& q, int wv, in
   const int chunk = (lane & 7) ^ ((4 * wv + (lane >> 4)) & 7);  // logical chunk of this lane
   const int row0 = w4_row0<V>(q);
   const int rows_a = min(256, w4_mend<V>(p, q) - row0);
-  const bf16_t* abase = p.a + (int64_t)row0 * p.lda + k_base;
-  d.na = (unsigned)(rows_a * p.lda * 2 - k_base * 2);
+  constexpr bool kIdx = (V & 128) != 0;  // (lane offsets: w4_rows)
+  const bf16_t* abase = p.a + (kIdx ? 0 : (int64_t)row0 * p.lda) + k_base;
+  d.na = (kIdx ? p.a_bytes : (unsigned)(rows_a * p.lda * 2)) - (unsigned)(k_base * 2);
   d.ra = __builtin_amdgcn_make_buffer_rsrc((void*)abase, (short)0, (int)d.na, 0x00020000);
   // tile-independent lane offsets: rows past the tile's valid rows fall outside `na`
+  if constexpr (!kIdx) {
 #pragma unroll
-  for (int s = 0; s < 8; ++s)
-    d.va[s] = (unsigned)((32 * s + 8 * wv + r8) * p.lda * 2 + chunk * 16);
+    for (int s = 0; s < 8; ++s)
+      d.va[s] = (unsigned)((32 * s + 8 * wv + r8) * p.lda * 2 + chunk * 16);
+  }
   // B: fragment j of wave column half h reads LDS rows 128 h + 8 l + j (l = lane & 15),
   // so lane l16 of the MFMA output holds the 8 CONSECUTIVE columns 8 l16 .. 8 l16 + 7 over
   // j = 0..7 (16-B epilogue stores).  Plain tiles keep tile row = LDS row.  Gated tiles:
@@ -664,6 +672,43 @@ DRTC_DEVICE void w4_plan(W4Dma& d, const W4Params& p, const W4Pos& q, int wv, in
   d.vb = (unsigned)(brow * p.ldb * 2 + (lane & 7) * 16);  // B: chunks in natural order
   d.lds_a = __builtin_amdgcn_readfirstlane(lds0 + 8 * wv * 128);
   d.lds_b = __builtin_amdgcn_readfirstlane(lds0 + kW4BOff + wv * kW4BBlk);
+}
+
+// The lane index re-derived (opaque to hipcc): kept live across the K loop it is spilled, and its
+// reload's vmcnt(0) would wait for the next tile's DMA.
+DRTC_DEVICE int w4_lane() {
+  int ln;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
+  return ln;
+}
+
+// V & 128: this wave's 64 rows of the tile at q, row 32 s + 8 wv + r in lane 8 s + r.  Their indexes go into the wave's
+// own 256 B behind the ring by one LDS-DMA a tile, issued a whole tile ahead: a load into registers would have to drain
+// the ring when its result is used.
+DRTC_DEVICE void w4_rows_ask(const W4Params& p, const W4Pos& q, int wv, unsigned lds0) {
+  const int lane = w4_lane();
+  const int row = 32 * (lane >> 3) + 8 * wv + (lane & 7);
+  const __amdgpu_buffer_rsrc_t ri = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(p.aidx + q.row0), (short)0, min(256, q.mend - q.row0) * 4, 0x00020000);
+  unsigned keep;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\t"
+      "buffer_load_dword %2, %3, 0 offen lds\n\ts_mov_b32 m0, %0"
+      : "=&s"(keep)
+      : "s"(lds0 + kW4Lds + 256 * wv), "v"(row * 4), "s"(ri)
+      : "memory");
+}
+// The lane offsets of A's DMA instructions from those indexes (landed: the wait is the caller's); rows past the tile's
+// valid ones lie outside A: read as 0.
+DRTC_DEVICE void w4_rows(W4Dma& d, const W4Params& p, const W4Pos& q, int wv, const char* lds) {
+  asm volatile("" ::: "memory");  // the reads stay behind that wait
+  const int lane = w4_lane();
+  const int r8 = lane >> 3, rows = q.mend - q.row0;
+  const int chunk = (lane & 7) ^ ((4 * wv + (lane >> 4)) & 7);
+  const int* at = reinterpret_cast<const int*>(lds + kW4Lds + 256 * wv) + r8;
+#pragma unroll
+  for (int s = 0; s < 8; ++s)
+    d.va[s] = 32 * s + 8 * wv + r8 < rows ? (unsigned)(at[8 * s] * p.lda * 2 + chunk * 16) : 0x80000000u;
 }
 
 // Select of two DMA plans on a wave-uniform condition: only the operand bases and the valid-A
@@ -720,6 +765,11 @@ __global__ __launch_bounds__(kW4Threads, 1) void gemm_w4_kernel(W4Params p) {
   W4Dma d;
   const unsigned lds0 = (unsigned)(uintptr_t)(w4_lds_ptr)w4_lds;
   w4_plan<EPI, V>(d, p, q, wv, lane, k_base, lds0);
+  if constexpr ((V & 128) != 0) {
+    w4_rows_ask(p, q, wv, lds0);
+    w4_vmcnt<0>();
+    w4_rows(d, p, q, wv, w4_lds);
+  }
   // fragment read offsets (bytes within a stage): row 128 w + l16 (+ 16 per fragment), the
   // 16-B chunk 4 h + g stored at chunk ^ ((row >> 1) & 7)
   const int fx = (l16 >> 1) & 7;
@@ -782,6 +832,7 @@ __global__ __launch_bounds__(kW4Threads, 1) void gemm_w4_kernel(W4Params p) {
       if (more) q2 = w4_pos_of<V>(p, tnext);
       W4Dma dn;
       w4_plan<EPI, V>(dn, p, q2, wv, lane, 0, lds0);
+      if constexpr ((V & 128) != 0) w4_rows_ask(p, q2, wv, lds0);  // (also where unused: the seam's wait counts it)
       // K step t + 2 of this tile, or step t + 2 - nk of the next one; the very last tile
       // re-stages its final K tile (valid bytes, never read) as the plain form does.  Step 0
       // starts the accumulators from 0 (MFMA with a zero C operand: no separate zeroing of the
@@ -796,6 +847,9 @@ __global__ __launch_bounds__(kW4Threads, 1) void gemm_w4_kernel(W4Params p) {
       }
       for (int t = 1; t < nk; ++t) {
         const bool own = t + 2 < nk;
+        if constexpr ((V & 128) != 0) {  // the last two K steps load the next tile's rows
+          if (t == nk - 2 && more) w4_rows(d, p, q2, wv, w4_lds);
+        }
         int t2 = own ? t + 2 : (more ? t + 2 - nk : nk - 1);
         t2 += kst;
         t2 -= t2 >= nk ? nk : 0;
@@ -806,10 +860,7 @@ __global__ __launch_bounds__(kW4Threads, 1) void gemm_w4_kernel(W4Params p) {
       // one epilogue call site (two would make hipcc copy all 256 accumulators out of the
       // AGPRs ahead of the branch between them, and spill)
       if (!more) w4_vmcnt<0>();  // no LDS-DMA may still be landing when the workgroup leaves
-      // the lane index re-derived here (opaque to hipcc): kept live across the K loop it is
-      // spilled, and its reload's vmcnt(0) would wait for the next tile's DMA
-      int ln;
-      asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
+      const int ln = w4_lane();
       w4_epilogue<EPI, V>(p, w4_cop<V>(p, q), acc, w4_row0<V>(q), w4_mend<V>(p, q), q.tn, wm, wn,
                           ln & 15, ln >> 4, 0);
       if (!more) break;
@@ -817,7 +868,7 @@ __global__ __launch_bounds__(kW4Threads, 1) void gemm_w4_kernel(W4Params p) {
       par ^= nk & 1;
       tt = tnext;
       q = q2;
-      d = dn;
+      d = w4_pick(false, d, dn);
     }
     return;
   }
@@ -879,7 +930,10 @@ int w4_launch(const W4Params& p, int v, hipStream_t st) {
 static int g_w4_grouped_rot = 0;
 template <int EPI>
 int w4_launch_grouped(const W4Params& p, int nwg, hipStream_t st) {
-  if (g_w4_grouped_rot)
+  if (EPI != W4_STORE && p.aidx != nullptr)
+    hipLaunchKernelGGL((gemm_w4_kernel<EPI, EPI == W4_STORE ? 104 : 232>), dim3(nwg), dim3(kW4Threads),
+                       kW4Lds + kW4Rows, st, p);
+  else if (g_w4_grouped_rot)
     hipLaunchKernelGGL((gemm_w4_kernel<EPI, 120>), dim3(nwg), dim3(kW4Threads), kW4Lds, st, p);
   else
     hipLaunchKernelGGL((gemm_w4_kernel<EPI, 104>), dim3(nwg), dim3(kW4Threads), kW4Lds, st, p);
@@ -901,6 +955,11 @@ template <int EPI, int V>
 int w4_cfg_one() {
   return (int)hipFuncSetAttribute((const void*)gemm_w4_kernel<EPI, V>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, kW4Lds);
+}
+template <int EPI>
+int w4_cfg_idx() {
+  return (int)hipFuncSetAttribute((const void*)gemm_w4_kernel<EPI, 232>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  kW4Lds + kW4Rows);
 }
 template <int EPI>
 int w4_cfg() {
@@ -1006,8 +1065,11 @@ int launch_gemm_w4(void* c, const void* a, const void* b, const void* r, int M, 
 int launch_gemm_w4_grouped(void* c, const void* a, const void* b, const int* grp, int n_grp,
                            int max_rows, int N, int K, int lda, int ldb, int ldc, int64_t b_grp,
                            int epi, int up_off, int group_m, int ksplit, int64_t c_split,
-                           float limit, hipStream_t st) {
+                           float limit, const int* aidx, int a_rows, hipStream_t st) {
   const bool glu = epi == W4_SILU || epi == W4_GELU || epi == W4_CLAMP;
+  // (three K tiles: the first one's wait covers the indexes, the last two's loads use them)
+  if (aidx != nullptr && (epi == W4_STORE || K < 192 || a_rows < 1 || (int64_t)a_rows * lda * 2 >= (1ll << 31)))
+    return -1;
   if (epi != W4_STORE && epi != W4_RELU2 && !glu) return -1;
   if (ksplit < 1 || (epi != W4_STORE && ksplit != 1)) return -1;  // an activation cannot be split
   if (grp == nullptr || n_grp < 1 || max_rows < 1 || K % 64 || (K / 64) % ksplit ||
@@ -1038,6 +1100,8 @@ int launch_gemm_w4_grouped(void* c, const void* a, const void* b, const int* grp
   p.b_grp = b_grp;
   p.ksplit = ksplit;
   p.c_split = c_split;
+  p.aidx = aidx;
+  p.a_bytes = aidx != nullptr ? (unsigned)(((int64_t)(a_rows - 1) * lda + K) * 2) : 0;
   // the most row tiles n_grp groups of max_rows rows in total can make
   const int64_t tiles = (int64_t)(p.tiles_m + n_grp - 1) * p.tiles_n * ksplit;
   int nwg = (int)(tiles < w4_num_cus() ? tiles : w4_num_cus());
@@ -1064,6 +1128,7 @@ int configure_gemm_w4() {
          w4_cfg_one<W4_STORE, 104>() | w4_cfg_one<W4_SILU, 104>() | w4_cfg_one<W4_GELU, 104>() |
          w4_cfg_one<W4_CLAMP, 0>() | w4_cfg_one<W4_CLAMP, 40>() | w4_cfg_one<W4_CLAMP, 56>() |
          w4_cfg_one<W4_CLAMP, 104>() | w4_cfg_one<W4_CLAMP, 120>() |
+         w4_cfg_idx<W4_SILU>() | w4_cfg_idx<W4_GELU>() | w4_cfg_idx<W4_CLAMP>() | w4_cfg_idx<W4_RELU2>() |
          w4_cfg_one<W4_STORE, 120>() | w4_cfg_one<W4_SILU, 120>() | w4_cfg_one<W4_GELU, 120>();
 }
 

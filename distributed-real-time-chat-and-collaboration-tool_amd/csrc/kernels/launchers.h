@@ -194,11 +194,11 @@ int launch_gemm_w4(void* c, const void* a, const void* b, const void* r, int M, 
 // Grouped persistent form: rows [grp[g], grp[g + 1]) of a / c (grp: n_grp + 1 row offsets in
 // DEVICE memory) times weight b + g * b_grp; epi 0 store or 2/3 gated; max_rows >= grp[n_grp]
 // sizes the grid.  ksplit > 1 (store only): K cut into ksplit slices, slice s written as bf16
-// partial products to c + s * c_split elements.
+// partial products to c + s * c_split elements.  aidx (2 / 3 / 4 / 5): row r is row aidx[r] of a, which has a_rows.
 int launch_gemm_w4_grouped(void* c, const void* a, const void* b, const int* grp, int n_grp,
                            int max_rows, int N, int K, int lda, int ldb, int ldc, int64_t b_grp,
                            int epi, int up_off, int group_m, int ksplit, int64_t c_split,
-                           float limit, hipStream_t st);
+                           float limit, const int* aidx, int a_rows, hipStream_t st);
 int64_t gemm_w4_workspace_bytes(int64_t M, int64_t N, int splitk);
 int configure_gemm_w4();
 

@@ -953,7 +953,7 @@ __global__ __launch_bounds__(256) void moe_combine_stream_kernel(
   }
 }
 
-// Variant 4: the pairs' token rows copied into expert order, xs[p] = x[sorted_tok[p]] for this
+// Variant 4, rows gemm_w4 does not read by the list: the pairs' token rows copied into expert order, xs[p] = x[sorted_tok[p]] for this
 // rank's positions (16 B per lane; a row of H bf16 per workgroup pass).
 __global__ __launch_bounds__(256) void moe_gather_kernel(bf16_t* __restrict__ xs,
                                                          const bf16_t* __restrict__ x,
@@ -1314,13 +1314,17 @@ int launch_moe(void* out, const void* x, const void* router_logits, const void* 
     return (int)hipGetLastError();
   }
   if (variant == 4) {
-    // xs (expert-ordered token rows) lives in zbuf: gate_up consumes it before down writes Z
-    bf16_t* xs = zbuf;
-    hipLaunchKernelGGL(moe_gather_kernel, dim3(min(P, 8192)), dim3(256), 0, st, xs,
-                       (const bf16_t*)x, sorted_tok, local_range, P, H);
-    int e = launch_gemm_w4_grouped(hbuf, xs, w_gu, grp_off, e_local, P, I, H, H, H, I,
+    // gate_up reads the token rows through the list: a pass of copying them in expert order first took 119 us a layer of
+    // 12,160 tokens of 4096, two experts each (pass of three layers 14.59 -> 14.31 ms), 144 us of 15,000 with two
+    // of 16 (20.84 -> 20.34 ms).  Still copied, into zbuf, which gate_up has consumed before down writes Z: tokens past a
+    // descriptor's 2 GiB or off 16 bytes.
+    const bool listed = (int64_t)T * H * 2 < (1ll << 31) && (uintptr_t)x % 16 == 0;
+    if (!listed)
+      hipLaunchKernelGGL(moe_gather_kernel, dim3(min(P, 8192)), dim3(256), 0, st, zbuf,
+                         (const bf16_t*)x, sorted_tok, local_range, P, H);
+    int e = launch_gemm_w4_grouped(hbuf, listed ? x : zbuf, w_gu, grp_off, e_local, P, I, H, H, H, I,
                                    (int64_t)up_rows * H, epi_gu, glu ? I : 0, g_moe_gm_gu, 1, 0,
-                                   opt.limit, st);
+                                   opt.limit, listed ? sorted_tok : nullptr, T, st);
     if (e) return e;
     if (dn_form) {
       // down on gemm_xd's grouped split-K forms over the 256-row tile table (few rows per
@@ -1333,7 +1337,7 @@ int launch_moe(void* out, const void* x, const void* router_logits, const void* 
     } else {
       e = launch_gemm_w4_grouped(zbuf, hbuf, w_dn, grp_off, e_local, P, H, I, I, I, H,
                                  (int64_t)H * I, 0, 0, g_moe_gm_dn, dn_split ? 2 : 1,
-                                 dn_split ? (int64_t)(zbuf2 - zbuf) : 0, 0.f, st);
+                                 dn_split ? (int64_t)(zbuf2 - zbuf) : 0, 0.f, nullptr, 0, st);
     }
     if (e) return e;
   } else if (variant == 3) {

@@ -846,6 +846,23 @@ def test_tile_height_of_the_experts(hipk):
         _close(ops.fused_moe(x, lg, wgu, wdn, 4, "silu"), ops.fused_moe_ref(x, lg, wgu, wdn, 4, "silu"), 3e-2, 3e-2, "moe")
 
 
+@pytest.mark.parametrize("T,H,I,E,k,act,off", [
+    (2500, 256, 4096, 4, 2, "silu", 0),      # a workgroup has several tiles of four K tiles
+    (1000, 512, 256, 3, 3, "gelu_tanh", 0),  # every expert has every token
+    (300, 256, 512, 2, 1, "relu2", 0),       # last tiles of few rows
+    (300, 256, 512, 2, 1, "silu", 4),        # tokens off 16 bytes: copied
+])
+def test_fused_moe_reads_tokens_by_the_list(hipk, T, H, I, E, k, act, off):
+    """Variant 4 on tokens that lie among others' bytes: against the fp32 reference."""
+    x, lg, wgu, wdn = _moe_inputs(T, H, I, E, seed=T)
+    if act == "relu2":
+        wgu = wgu[:, :I].contiguous()
+    buf = torch.full((T * H + 16,), float("nan"), device="cuda", dtype=torch.bfloat16)
+    buf[off:off + T * H] = x.flatten()
+    y = ops.fused_moe(buf[off:off + T * H].view(T, H), lg, wgu, wdn, k, act, variant=4)
+    _close(y, ops.fused_moe_ref(x, lg, wgu, wdn, k, act), 3e-2, 3e-2, f"moe list {T}")
+
+
 @pytest.mark.parametrize("T,H,I,E,k,e_off,e_local", [
     (4096, 1024, 512, 8, 2, 0, 8),       # ~1k rows per expert: the auto pick
     (3000, 512, 384, 4, 2, 0, 4),        # row tails in every expert
