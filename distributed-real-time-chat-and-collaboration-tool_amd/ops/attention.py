@@ -32,6 +32,22 @@ def prefill_persist_for(max_len: int) -> bool:
     return forced if forced is not None else max_len <= PERSIST_MAX_LEN
 
 
+def prefill_form(max_len: int, ntiles: int, Hq: int, Hkv: int, D: int) -> int:
+    """Launch form of the prefill attention: 1 persistent workgroups, + 2 the next tile's scores ahead (four heads of 128
+    to a KV head).  us, plain / persistent / ahead / both.  A workgroup an item: persistent ones gain nothing, and ahead
+    pays from 320 tokens (one prompt, 16 heads: 200 12.7 / 13.3 / 12.9 / 13.4, 256 14.8 / 15.4 / 14.8 / 15.3, 320 16.7 / 17.6 / 16.3 /
+    16.8, 700 27.6 / 29.6 / 25.4 / 26.1, 2000 64 / 71 / 58 / 59).  More: from 640 (32 heads: 20 x 384 64 / 60 / 66 / 61, 16 x 512
+    90 / 80 / 94 / 84, 12 x 640 76 / 73.5 / 78 / 72.4, 8 x 1000 103 / 101 / 101 / 96.5, 4 x 3000 340 / 349 / 321 / 320)."""
+    persist = prefill_persist_for(max_len)
+    G = Hq // Hkv
+    if D != 128 or G % 4:
+        return int(persist)
+    one = ntiles * (Hq // 4) <= 256  # CUs
+    if one and _prefill_persist[0] is None:
+        persist = False
+    return int(persist) | (2 if max_len >= (320 if one else 640) else 0)
+
+
 # ----------------------------------------------------------------- prefill
 def prefill_tiles(cu_seqlens: list[int]) -> tuple[list[int], list[int]]:
     """Host-side 64-row query tile map for a packed batch, longest sequences
@@ -102,13 +118,12 @@ def prefill_attention(qkv: torch.Tensor, cu_seqlens: torch.Tensor, Hq: int, Hkv:
         tiles = (torch.tensor(ts, dtype=torch.int32, device=dev),
                  torch.tensor(tq, dtype=torch.int32, device=dev))
     ntiles = tiles[0].numel()
-    if max_len is None and _prefill_persist[0] is None:
-        max_len = max(b - a for a, b in zip(cu, cu[1:]))
-    persist = prefill_persist_for(max_len or 0)
+    if max_len is None:
+        max_len = max((b - a for a, b in zip(cu, cu[1:])), default=0)
     check(hipk().prefill_attn(out.data_ptr(), out.stride(0), qkv.data_ptr(), qkv.stride(0),
                               Hq, Hkv, D, cu_seqlens.data_ptr(), tiles[0].data_ptr(),
                               tiles[1].data_ptr(), ntiles, float(scale), int(causal),
-                              int(persist), stream_ptr(qkv)), "prefill_attn")
+                              prefill_form(max_len, ntiles, Hq, Hkv, D), stream_ptr(qkv)), "prefill_attn")
     return out
 
 
