@@ -331,7 +331,7 @@ def tall_form(M: int, N: int, K: int, glu: bool = False, act: str = "silu") -> i
     64: 14336 x 2048 gated, 132 rows 22.3 / 18.3, 160 20.4 / 19.4, 12800 x 2048 20.1 / 19.0, 16384 x 4096 gated 39.1 / 36.7.
     More than a round: 57344 x 4096 gated, 176 rows 100.6 / 109; fewer tiles: 16384 x 4096 gated, 160 rows 39.1 / 48.4, and of 64
     8448 x 2048, 160 rows 17.6 / 17.9; 192 rows in tiles of 64 12800 x 2048 21.5 / 21.4."""
-    if not (_xd_enabled and _enabled and _xd_nt and 129 <= M <= 224 and K >= 2048):
+    if not (129 <= M <= 224 and K >= 2048 and _xd_enabled and _enabled and _xd_nt):
         return 0
     mt, rows = 3 if M <= 160 else 4 if M <= 192 else 5, 2 * N if glu else N
     nf = 4 if rows % 128 == 0 and 160 <= rows // 128 <= 256 else 2 if mt == 3 and rows % 64 == 0 and 192 <= rows // 64 <= 256 else 0
@@ -1195,6 +1195,7 @@ def xd_nt(form: int) -> bool:
     return form >= 1000
 
 
+@functools.lru_cache(maxsize=4096)  # (asked several times a layer; of its arguments alone)
 def xd_supported(M: int, N: int, K: int, form: int, glu: bool = False) -> bool:
     """Shapes gemm_xd.hip takes in ``form`` (mt * 100 + nf * 10 + splitk); N = output
     columns (gated: half the rows of the [gate; up] weight)."""
