@@ -454,6 +454,10 @@ __global__ __launch_bounds__(128 * GH, 2) void prefill_attn32_kernel(
     float scale, float to_q, int causal) {
   using L = Prefill32<D, GH>;
   constexpr int KS = D / 16, NT = D / 32, VPR = D / 8, NV = kKT * VPR / L::NTHR;
+  // LDS reads in flight ahead of the MFMAs, in pinned order: left alone the compiler reads an operand or two ahead, and
+  // each MFMA waits for most of the LDS's latency (128: 15 x 1000 of 16 heads over 4 108 -> 102 us, 148 of 32 11.2 ->
+  // 10.6, 8 x 2000 of 16 over 8 181 -> 176; 64 loses, 8 x 2000 of 16 over 8 112 -> 119)
+  constexpr int AHEAD = D == 128 ? 4 : 0;
   static_assert(NV >= 1 && (kKT * VPR) % L::NTHR == 0, "staging split");
   extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
   const int G = Hq / Hkv, groups = G / GH, n_hg = Hq / GH, n_work = n_tiles * n_hg;
@@ -552,13 +556,24 @@ __global__ __launch_bounds__(128 * GH, 2) void prefill_attn32_kernel(
         if constexpr (PERSIST) load_q(qn, nxt);
       }
       f32x16 sc[2];
+      bf16x8 kf[2 * KS], vf[4 * NT];
+      auto read_k = [&](int n) { kf[n] = load_bf16x8(kb + 32 * (n / KS) * L::KROW + k_at + 16 * (n % KS)); };
+      auto read_v = [&](int n) {
+        const bf16_t* p = vb + 16 * (n % 4) * L::VROW + 32 * (n / 4);
+        const bf16x4 lo = lds_read_tr16(p), hi = lds_read_tr16(p + 8 * L::VROW);
 #pragma unroll
-      for (int st = 0; st < 2; ++st) {
+        for (int j = 0; j < 4; ++j) { vf[n][j] = lo[j]; vf[n][4 + j] = hi[j]; }
+      };
 #pragma unroll
-        for (int r = 0; r < 16; ++r) sc[st][r] = 0.f;
+      for (int n = 0; n < AHEAD; ++n) read_k(n);
 #pragma unroll
-        for (int s = 0; s < KS; ++s)
-          sc[st] = mfma32(load_bf16x8(kb + 32 * st * L::KROW + k_at + 16 * s), qf[s], sc[st]);
+      for (int n = 0; n < 2 * KS; ++n) {
+        if constexpr (AHEAD > 0) __builtin_amdgcn_sched_barrier(0);
+        if (n + AHEAD < 2 * KS) read_k(n + AHEAD);
+        if (n % KS == 0)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) sc[n / KS][r] = 0.f;
+        sc[n / KS] = mfma32(kf[n], qf[n % KS], sc[n / KS]);
       }
       const int k0 = kt * kKT;
       if (k0 + kKT > open) {
@@ -593,16 +608,13 @@ __global__ __launch_bounds__(128 * GH, 2) void prefill_attn32_kernel(
         }
       lsum += (psum[0] + psum[1]) + (psum[2] + psum[3]);
 #pragma unroll
-      for (int i = 0; i < NT; ++i)
+      for (int n = 0; n < AHEAD; ++n) read_v(n);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const bf16x4 lo = lds_read_tr16(vb + 16 * t * L::VROW + 32 * i);
-          const bf16x4 hi = lds_read_tr16(vb + (16 * t + 8) * L::VROW + 32 * i);
-          bf16x8 a;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) { a[j] = lo[j]; a[4 + j] = hi[j]; }
-          o[i] = mfma32(a, pf[t], o[i]);
-        }
+      for (int n = 0; n < 4 * NT; ++n) {
+        if constexpr (AHEAD > 0) __builtin_amdgcn_sched_barrier(0);
+        if (n + AHEAD < 4 * NT) read_v(n + AHEAD);
+        o[n / 4] = mfma32(vf[n], pf[n % 4], o[n / 4]);
+      }
     }
     lsum += __shfl_xor(lsum, 32, 64);
     if (qrow < cur.seqlen) {
@@ -635,40 +647,36 @@ DRTC_DEVICE void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier
 // the outputs of this one.  What bounds a wave above is that its matrix instructions and its softmax follow one
 // another, and the barrier of each tile keeps the two waves of a SIMD in step.  (Matrix cores busy 42.6 -> 48 %, cycles
 // 660,000 -> 588,000 at 4 x 4000 tokens of 16 heads; the clock falls from 2.2 to 2.05 GHz, power bounds the rest.)
-// us, above / this: 4 x 4000 of 16 heads over 4 301 / 287, 4 x 4096 of 32 over 8 607 / 577, 627 of 32 27.3 / 24.1,
-// 8 x 500 of 16 27.3 / 25.1, 16 x 1000 of 32 persistent 225 / 212.  Few tiles do not pay for the first one's scores
-// by themselves (148 of 32 11.8 / 12.4, 300 x 148 157 / 163), two heads not for the registers (8 x 2000 180 / 258):
-// the caller picks by the longest sequence.  Every sum is the one above's, in its order.
-template <bool PERSIST>
+// us, above / this: 4 x 4000 of 16 heads over 4 281 / 274, 4 x 3000 of 32 over 8 324 / 316, one of 700 26.4 / 25.7, of 2000
+// 64 / 58 (above without its pinned reads).  Few tiles do not pay for the first one's scores by themselves (one of 256
+// 14.2 / 14.7, 16 x 512 90 / 94), two heads not for the registers (8 x 2000 180 / 258), persistent workgroups not for
+// theirs (8 x 1000 50.3 / 52.3, 16 x 512 of 32 82.5 / 85.4): the caller picks by the longest sequence.  Every sum is the
+// one above's, in its order.
 __global__ __launch_bounds__(512, 2) void prefill_ahead_kernel(
     bf16_t* __restrict__ out, int out_stride, const bf16_t* __restrict__ qkv, int qkv_stride, int Hq, int Hkv,
-    const int* __restrict__ cu_seqlens, const int* __restrict__ tile_seq, const int* __restrict__ tile_q0, int n_tiles,
+    const int* __restrict__ cu_seqlens, const int* __restrict__ tile_seq, const int* __restrict__ tile_q0,
     float scale, float to_q, int causal) {
   constexpr int D = 128, GH = 4;
   using L = Prefill32<D, GH>;
   constexpr int KS = D / 16, NT = D / 32, VPR = D / 8, NV = kKT * VPR / L::NTHR;
   extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
-  const int G = Hq / Hkv, groups = G / GH, n_hg = Hq / GH, n_work = n_tiles * n_hg;
+  const int G = Hq / Hkv, groups = G / GH, n_hg = Hq / GH;
   const int w = wave_id_uniform(), lane = threadIdx.x & 63;
   const int col = lane & 31, h = lane >> 5;
 
-  struct Item {
-    int s_begin, seqlen, q0, hq, hk, ntiles;
-  };
-  auto info = [&](int item) -> Item {
-    const int tile = item / n_hg, hg = item - tile * n_hg, hk = hg / groups;
-    const int seq = tile_seq[tile], q0 = tile_q0[tile], s_begin = cu_seqlens[seq];
-    const int seqlen = cu_seqlens[seq + 1] - s_begin;
-    const int kv_end = causal ? min(seqlen, q0 + kQT) : seqlen;
-    return Item{s_begin, seqlen, q0, hk * G + (hg - hk * groups) * GH + (w >> 1), hk, (kv_end + kKT - 1) / kKT};
-  };
+  const int tile = blockIdx.x / n_hg, hg = blockIdx.x - tile * n_hg, hk = hg / groups;
+  const int hq = hk * G + (hg - hk * groups) * GH + (w >> 1);
+  const int seq = tile_seq[tile], q0 = tile_q0[tile], s_begin = cu_seqlens[seq];
+  const int seqlen = cu_seqlens[seq + 1] - s_begin;
+  const int ntiles = ((causal ? min(seqlen, q0 + kQT) : seqlen) + kKT - 1) / kKT;
+  const int qrow = q0 + 32 * (w & 1) + col;
   // tile kt of K (at = Hq + hk) or V (Hkv further), kept in registers until its place in the LDS is free
-  auto issue = [&](bf16x8 (&x)[NV], const Item& it, int at, int kt) {
-    const bf16_t* base = qkv + (int64_t)(it.s_begin + kt * kKT) * qkv_stride + at * D;
+  auto issue = [&](bf16x8 (&x)[NV], int at, int kt) {
+    const bf16_t* base = qkv + (int64_t)(s_begin + kt * kKT) * qkv_stride + at * D;
 #pragma unroll
     for (int n = 0; n < NV; ++n) {
       const int v = threadIdx.x + n * L::NTHR, key = v / VPR, c = (v - key * VPR) * 8;
-      if (kt * kKT + key < it.seqlen) {
+      if (kt * kKT + key < seqlen) {
         x[n] = load_bf16x8(base + key * qkv_stride + c);
       } else {
 #pragma unroll
@@ -685,200 +693,167 @@ __global__ __launch_bounds__(512, 2) void prefill_ahead_kernel(
   };
   auto ks = [&](int kt) { return lds + (kt & 1) * L::BUF; };
   auto vs = [&](int kt) { return lds + (kt & 1) * L::BUF + L::K_ELEMS; };
-  auto load_q = [&](bf16x8* qf, const Item& it) {
-    const int qrow = it.q0 + 32 * (w & 1) + col;
-    const bf16_t* qp = qkv + (int64_t)(it.s_begin + qrow) * qkv_stride + it.hq * D + 8 * h;
+  const int k_at = col * L::KROW + 8 * h;
+  const int v_at = (4 * h + ((lane & 15) >> 2)) * L::VROW + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+
+  bf16x8 kr[NV], k2[NV], vr[NV], qf[KS];
+  issue(kr, Hq + hk, 0);
+  issue(vr, Hq + Hkv + hk, 0);
+  if (ntiles > 1) issue(k2, Hq + hk, 1);
+  const bf16_t* qp = qkv + (int64_t)(s_begin + qrow) * qkv_stride + hq * D + 8 * h;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      if (qrow < it.seqlen) qf[s] = load_bf16x8(qp + 16 * s);
-      else for (int j = 0; j < 8; ++j) qf[s][j] = f2bf(0.f);
-    }
-  };
-  auto turn = [&](bf16x8* qf) {
-    if (to_q == 1.f) return;
+  for (int s = 0; s < KS; ++s) {
+    if (qrow < seqlen) qf[s] = load_bf16x8(qp + 16 * s);
+    else for (int j = 0; j < 8; ++j) qf[s][j] = f2bf(0.f);
+  }
+  if (to_q != 1.f) {
 #pragma unroll
     for (int s = 0; s < KS; ++s)
 #pragma unroll
       for (int j = 0; j < 8; ++j) qf[s][j] = f2bf(bf2f(qf[s][j]) * to_q);
-  };
-  const int k_at = col * L::KROW + 8 * h;
-  const int v_at = (4 * h + ((lane & 15) >> 2)) * L::VROW + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+  }
+  // keys below `open` need no mask for any row of the workgroup
+  const int open = causal ? min(seqlen, q0 + 1) : seqlen;
+  const int last = causal ? min(seqlen - 1, qrow) : seqlen - 1;  // last key of this row
+  f32x16 o[NT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
+  float m = kNegBig, lsum = 0.f;
 
-  const int nwg = gridDim.x;
-  auto item_of = [&](int round) -> int {
-    const int slot = (round & 1) ? nwg - 1 - (int)blockIdx.x : (int)blockIdx.x;
-    return round * nwg + slot;
-  };
-  int round = 0;
-  if (item_of(0) >= n_work) return;
-  Item cur = info(item_of(0));
-  bf16x8 kr[NV], k2[NV], vr[NV], qf[KS];
-  auto first = [&](const Item& it) {  // an item's first tiles: K 0 and 1, V 0
-    issue(kr, it, Hq + it.hk, 0);
-    issue(vr, it, Hq + Hkv + it.hk, 0);
-    if (it.ntiles > 1) issue(k2, it, Hq + it.hk, 1);
-  };
-  first(cur);
-  load_q(qf, cur);
-  while (true) {
-    turn(qf);
-    const int qrow = cur.q0 + 32 * (w & 1) + col;
-    // keys below `open` need no mask for any row of the workgroup
-    const int open = causal ? min(cur.seqlen, cur.q0 + 1) : cur.seqlen;
-    const int last = causal ? min(cur.seqlen - 1, qrow) : cur.seqlen - 1;  // last key of this row
-    f32x16 o[NT];
+  // Tile kt: the softmax and the output of its scores `sc`, and (NEXT) the scores of tile kt + 1 into `sn`.  A slot of
+  // the stream holds a score MFMA, an output MFMA of the 16 keys before and the exponentials of 2 keys a
+  // lane between them; operands are read two slots ahead.
+  auto step = [&](auto next, f32x16 (&sc)[2], f32x16 (&sn)[2], int kt) {
+    constexpr bool NEXT = decltype(next)::value;
+    constexpr int U = KS / 2, E = 8 / U;  // slots to 16 keys, scores a lane to a slot
+    static_assert(NT == U, "an output MFMA to a score MFMA");
+    const bf16_t* kb = ks(kt + 1) + k_at;
+    const bf16_t* vb = vs(kt) + v_at;
+    bf16x8 kf[2 * KS], vf[4 * NT];
+    auto read_k = [&](int n) { kf[n] = load_bf16x8(kb + 32 * (n / KS) * L::KROW + 16 * (n % KS)); };
+    auto read_v = [&](int n) {  // keys 16 (n / NT).., columns 32 (n % NT)..
+      const bf16_t* p = vb + 16 * (n / NT) * L::VROW + 32 * (n % NT);
+      const bf16x4 lo = lds_read_tr16(p), hi = lds_read_tr16(p + 8 * L::VROW);
 #pragma unroll
-    for (int i = 0; i < NT; ++i)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
-    float m = kNegBig, lsum = 0.f;
-    const bool have_next = PERSIST && item_of(round + 1) < n_work;
-    Item nxt = cur;
-
-    // Tile kt: the softmax and the output of its scores `sc`, and (NEXT) the scores of tile kt + 1 into `sn`.  A slot of
-    // the stream holds a score MFMA, an output MFMA of the 16 keys before and the exponentials of 2 keys a
-    // lane between them; operands are read two slots ahead.
-    auto step = [&](auto next, f32x16 (&sc)[2], f32x16 (&sn)[2], int kt) {
-      constexpr bool NEXT = decltype(next)::value;
-      constexpr int U = KS / 2, E = 8 / U;  // slots to 16 keys, scores a lane to a slot
-      static_assert(NT == U, "an output MFMA to a score MFMA");
-      const bf16_t* kb = ks(kt + 1) + k_at;
-      const bf16_t* vb = vs(kt) + v_at;
-      bf16x8 kf[2 * KS], vf[4 * NT];
-      auto read_k = [&](int n) { kf[n] = load_bf16x8(kb + 32 * (n / KS) * L::KROW + 16 * (n % KS)); };
-      auto read_v = [&](int n) {  // keys 16 (n / NT).., columns 32 (n % NT)..
-        const bf16_t* p = vb + 16 * (n / NT) * L::VROW + 32 * (n % NT);
-        const bf16x4 lo = lds_read_tr16(p), hi = lds_read_tr16(p + 8 * L::VROW);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) { vf[n][j] = lo[j]; vf[n][4 + j] = hi[j]; }
-      };
-      if constexpr (NEXT) { read_k(0); read_k(1); }
-      const int k0 = kt * kKT;
-      if (k0 + kKT > open) {
-        const int past = last - k0 - 4 * h;
-#pragma unroll
-        for (int st = 0; st < 2; ++st)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) sc[st][r] = 32 * st + 8 * (r / 4) + r % 4 <= past ? sc[st][r] : kNegBig;
-      }
-      float top = kNegBig;
+      for (int j = 0; j < 4; ++j) { vf[n][j] = lo[j]; vf[n][4 + j] = hi[j]; }
+    };
+    if constexpr (NEXT) { read_k(0); read_k(1); }
+    const int k0 = kt * kKT;
+    if (k0 + kKT > open) {
+      const int past = last - k0 - 4 * h;
 #pragma unroll
       for (int st = 0; st < 2; ++st)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) top = fmaxf(top, sc[st][r]);
-      const float m_new = fmaxf(m, half_max(top) * scale);
-      if (__any(m != m_new)) {
-        const float alpha = fast_exp2(m - m_new);
-        lsum *= alpha;
+        for (int r = 0; r < 16; ++r) sc[st][r] = 32 * st + 8 * (r / 4) + r % 4 <= past ? sc[st][r] : kNegBig;
+    }
+    float top = kNegBig;
 #pragma unroll
-        for (int i = 0; i < NT; ++i) o[i] *= alpha;
-      }
-      m = m_new;
-      __builtin_amdgcn_sched_barrier(0);
-      float psum[4] = {0.f, 0.f, 0.f, 0.f};
-      bf16x8 pf[4];
+    for (int st = 0; st < 2; ++st)
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
+      for (int r = 0; r < 16; ++r) top = fmaxf(top, sc[st][r]);
+    const float m_new = fmaxf(m, half_max(top) * scale);
+    if (__any(m != m_new)) {
+      const float alpha = fast_exp2(m - m_new);
+      lsum *= alpha;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const int n = U * c + u;
-          if constexpr (NEXT) {
-            if (n + 2 < 2 * KS) read_k(n + 2);
-          }
-          if (n + 2 >= U) read_v(n + 2 - U);
-          if constexpr (NEXT) {
-            if (n % KS == 0)
+      for (int i = 0; i < NT; ++i) o[i] *= alpha;
+    }
+    m = m_new;
+    __builtin_amdgcn_sched_barrier(0);
+    float psum[4] = {0.f, 0.f, 0.f, 0.f};
+    bf16x8 pf[4];
 #pragma unroll
-              for (int r = 0; r < 16; ++r) sn[n / KS][r] = 0.f;
-            sn[n / KS] = mfma32(kf[n], qf[n % KS], sn[n / KS]);
-          }
-#pragma unroll
-          for (int e = 0; e < E; ++e) {
-            if (e == E / 2) {
-              __builtin_amdgcn_sched_barrier(0);
-              if (c > 0) o[u] = mfma32(vf[n - U], pf[c - 1], o[u]);
-            }
-            const int r = 8 * (c & 1) + E * u + e;
-            const float p = fast_exp2(__builtin_fmaf(sc[c >> 1][r], scale, -m));
-            psum[r & 3] += p;
-            pf[c][r & 7] = f2bf(p);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      lsum += (psum[0] + psum[1]) + (psum[2] + psum[3]);
+    for (int c = 0; c < 4; ++c)
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        if (u + 2 < U) read_v(3 * U + u + 2);
-        o[u] = mfma32(vf[3 * U + u], pf[3], o[u]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    };
-    // what the LDS holds is read and written a tile apart: K a tile ahead of V
-    auto turnover = [&](int kt) {
-      lds_barrier();
-      if (kt + 2 < cur.ntiles) commit(kr, ks(kt), L::KROW);
-      commit(vr, vs(kt + 1), L::VROW);
-      if (kt + 3 < cur.ntiles) issue(kr, cur, Hq + cur.hk, kt + 3);
-      if (kt + 2 < cur.ntiles) issue(vr, cur, Hq + Hkv + cur.hk, kt + 2);
-    };
-    if (round > 0) lds_barrier();
-    commit(kr, ks(0), L::KROW);
-    commit(vr, vs(0), L::VROW);
-    if (cur.ntiles > 1) {
-      commit(k2, ks(1), L::KROW);
-      issue(vr, cur, Hq + Hkv + cur.hk, 1);
-      if (cur.ntiles > 2) issue(kr, cur, Hq + cur.hk, 2);
-    }
-    lds_barrier();
-    f32x16 sa[2], sb[2];
-#pragma unroll
-    for (int st = 0; st < 2; ++st) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) sa[st][r] = 0.f;
-#pragma unroll
-      for (int s = 0; s < KS; ++s)
-        sa[st] = mfma32(load_bf16x8(ks(0) + 32 * st * L::KROW + k_at + 16 * s), qf[s], sa[st]);
-    }
-    int kt = 0;
-    for (; kt + 2 < cur.ntiles; kt += 2) {
-      turnover(kt);
-      step(std::true_type{}, sa, sb, kt);
-      turnover(kt + 1);
-      step(std::true_type{}, sb, sa, kt + 1);
-    }
-    if (kt + 1 < cur.ntiles) {
-      turnover(kt);
-      step(std::true_type{}, sa, sb, kt);
-      sa[0] = sb[0];
-      sa[1] = sb[1];
-      ++kt;
-    }
-    lds_barrier();
-    if (have_next) {
-      nxt = info(item_of(round + 1));
-      first(nxt);
-      load_q(qf, nxt);  // (the last tile's step has no use for Q)
-    }
-    step(std::false_type{}, sa, sb, kt);
-    lsum += __shfl_xor(lsum, 32, 64);
-    if (qrow < cur.seqlen) {
-      const float inv = 1.f / lsum;
-      bf16_t* op = out + (int64_t)(cur.s_begin + qrow) * out_stride + cur.hq * D + 4 * h;
-#pragma unroll
-      for (int i = 0; i < NT; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          bf16x4 v;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] = f2bf(o[i][4 * q + r] * inv);
-          *reinterpret_cast<bf16x4*>(op + 32 * i + 8 * q) = v;
+        const int n = U * c + u;
+        if constexpr (NEXT) {
+          if (n + 2 < 2 * KS) read_k(n + 2);
         }
+        if (n + 2 >= U) read_v(n + 2 - U);
+        if constexpr (NEXT) {
+          if (n % KS == 0)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sn[n / KS][r] = 0.f;
+          sn[n / KS] = mfma32(kf[n], qf[n % KS], sn[n / KS]);
+        }
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          if (e == E / 2) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (c > 0) o[u] = mfma32(vf[n - U], pf[c - 1], o[u]);
+          }
+          const int r = 8 * (c & 1) + E * u + e;
+          const float p = fast_exp2(__builtin_fmaf(sc[c >> 1][r], scale, -m));
+          psum[r & 3] += p;
+          pf[c][r & 7] = f2bf(p);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    lsum += (psum[0] + psum[1]) + (psum[2] + psum[3]);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (u + 2 < U) read_v(3 * U + u + 2);
+      o[u] = mfma32(vf[3 * U + u], pf[3], o[u]);
     }
-    if (!have_next) break;
-    if constexpr (PERSIST) {
-      cur = nxt;
-      ++round;
-    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // what the LDS holds is read and written a tile apart: K a tile ahead of V
+  auto turnover = [&](int kt) {
+    lds_barrier();
+    if (kt + 2 < ntiles) commit(kr, ks(kt), L::KROW);
+    commit(vr, vs(kt + 1), L::VROW);
+    if (kt + 3 < ntiles) issue(kr, Hq + hk, kt + 3);
+    if (kt + 2 < ntiles) issue(vr, Hq + Hkv + hk, kt + 2);
+  };
+  commit(kr, ks(0), L::KROW);
+  commit(vr, vs(0), L::VROW);
+  if (ntiles > 1) {
+    commit(k2, ks(1), L::KROW);
+    issue(vr, Hq + Hkv + hk, 1);
+    if (ntiles > 2) issue(kr, Hq + hk, 2);
+  }
+  lds_barrier();
+  f32x16 sa[2], sb[2];
+#pragma unroll
+  for (int st = 0; st < 2; ++st) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sa[st][r] = 0.f;
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      sa[st] = mfma32(load_bf16x8(ks(0) + 32 * st * L::KROW + k_at + 16 * s), qf[s], sa[st]);
+  }
+  int kt = 0;
+  for (; kt + 2 < ntiles; kt += 2) {
+    turnover(kt);
+    step(std::true_type{}, sa, sb, kt);
+    turnover(kt + 1);
+    step(std::true_type{}, sb, sa, kt + 1);
+  }
+  if (kt + 1 < ntiles) {
+    turnover(kt);
+    step(std::true_type{}, sa, sb, kt);
+    sa[0] = sb[0];
+    sa[1] = sb[1];
+    ++kt;
+  }
+  lds_barrier();
+  step(std::false_type{}, sa, sb, kt);
+  lsum += __shfl_xor(lsum, 32, 64);
+  if (qrow < seqlen) {
+    const float inv = 1.f / lsum;
+    bf16_t* op = out + (int64_t)(s_begin + qrow) * out_stride + hq * D + 4 * h;
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        bf16x4 v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = f2bf(o[i][4 * q + r] * inv);
+        *reinterpret_cast<bf16x4*>(op + 32 * i + 8 * q) = v;
+      }
   }
 }
 
@@ -918,27 +893,22 @@ static void launch_tile(dim3 grid, hipStream_t st, bf16_t* out, int out_stride, 
     float scale, to_q;
     split_scale(sl2, scale, to_q);
     if constexpr (GH == 4) {  // with fewer waves to a workgroup the others of its CU fill its gaps
-      if (persist & 1) {
+      if (persist == 1) {
         static int per_cu = 0;
         if (per_cu == 0 && (hipOccupancyMaxActiveBlocksPerMultiprocessor(
                                 &per_cu, prefill_attn32_kernel<D, GH, true>, L::NTHR, L::BYTES) != hipSuccess ||
                             per_cu <= 0))
           per_cu = 1;
         const int n_wg = std::min(n_work, prefill_persist_grid(n_work * per_cu) * per_cu);
-        if (persist & 2) {  // (as many to a CU: the LDS and the launch bounds are the same)
-          prefill_ahead_kernel<true><<<std::max(1, n_wg), L::NTHR, L::BYTES, st>>>(
-              out, out_stride, qkv, qkv_stride, Hq, Hkv, cu, ts, tq, (int)grid.x, scale, to_q, causal);
-          return;
-        }
         prefill_attn32_kernel<D, GH, true><<<std::max(1, n_wg), L::NTHR, L::BYTES, st>>>(
             out, out_stride, qkv, qkv_stride, Hq, Hkv, cu, ts, tq, (int)grid.x, scale, to_q, causal);
         return;
       }
     }
     if constexpr (GH == 4) {
-      if (persist & 2) {
-        prefill_ahead_kernel<false><<<n_work, L::NTHR, L::BYTES, st>>>(
-            out, out_stride, qkv, qkv_stride, Hq, Hkv, cu, ts, tq, (int)grid.x, scale, to_q, causal);
+      if (persist == 2) {
+        prefill_ahead_kernel<<<n_work, L::NTHR, L::BYTES, st>>>(out, out_stride, qkv, qkv_stride, Hq, Hkv, cu, ts, tq, scale,
+                                                                to_q, causal);
         return;
       }
     }
@@ -946,7 +916,7 @@ static void launch_tile(dim3 grid, hipStream_t st, bf16_t* out, int out_stride, 
         out, out_stride, qkv, qkv_stride, Hq, Hkv, cu, ts, tq, (int)grid.x, scale, to_q, causal);
   } else {
     constexpr size_t lds_bytes = PrefillLds<D, GH>::BYTES;
-    if (persist & 1) {
+    if (persist == 1) {
       // resident workgroups per CU for this instantiation (VGPRs / LDS / waves)
       static int per_cu = 0;
       if (per_cu == 0) {
@@ -1022,8 +992,7 @@ static int set_lds() {
     e = set(prefill_attn32_kernel<D, GH, false>, Prefill32<D, GH>::BYTES);
     if constexpr (GH == 4) {
       if (!e) e = set(prefill_attn32_kernel<D, GH, true>, Prefill32<D, GH>::BYTES);
-      if (!e) e = set(prefill_ahead_kernel<false>, Prefill32<D, GH>::BYTES);
-      if (!e) e = set(prefill_ahead_kernel<true>, Prefill32<D, GH>::BYTES);
+      if (!e) e = set(prefill_ahead_kernel, Prefill32<D, GH>::BYTES);
     }
   } else {
     e = set(prefill_attn_kernel<D, GH>, PrefillLds<D, GH>::BYTES);

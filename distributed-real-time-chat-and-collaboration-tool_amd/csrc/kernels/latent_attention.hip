@@ -280,6 +280,10 @@ __global__ __launch_bounds__(64 * NW, NB == 1 ? 2 : 1) void latent_prefill_kerne
   constexpr int KS = DKP / 32, NT = DVP / 16;
   constexpr int NK = kLK * (DKP / 8) / NTHR, NV = kLK * (DVP / 8) / NTHR;
   constexpr int QT = 16 * NW * QF;
+  // LDS reads in flight ahead of the MFMAs, in pinned order: left alone the compiler reads two operands and waits for
+  // them (192 / 128, window 1024, 256 rows: 4 x 3500 tokens of 16 heads 234 -> 220 us, 15 x 1000 of 32 386 -> 362, 8 x 300
+  // of 16 21.9 -> 21.2).  128 rows have no registers for it (64 x 150 of 16 heads 73.8 -> 76.3).
+  constexpr int AHEAD = NW == 8 ? 4 : 0;
   static_assert(NK * NTHR == kLK * (DKP / 8) && NV * NTHR == kLK * (DVP / 8), "staging split");
   extern __shared__ __attribute__((aligned(16))) bf16_t lat_lds[];
 
@@ -374,15 +378,19 @@ __global__ __launch_bounds__(64 * NW, NB == 1 ? 2 : 1) void latent_prefill_kerne
     const bool whole = k0 + kLK - 1 <= q_first && k0 > q_last - win;
 
     f32x4 sc[QF][4];
+    bf16x8 kf[4 * KS];
+    auto read_k = [&](int n) { kf[n] = load_bf16x8(kb + (16 * (n / KS) + col) * L::KROW + 32 * (n % KS) + 8 * g); };
 #pragma unroll
-    for (int st = 0; st < 4; ++st) {
+    for (int n = 0; n < AHEAD; ++n) read_k(n);
 #pragma unroll
-      for (int f = 0; f < QF; ++f) sc[f][st] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int n = 0; n < 4 * KS; ++n) {
+      if constexpr (AHEAD > 0) __builtin_amdgcn_sched_barrier(0);
+      if (n + AHEAD < 4 * KS) read_k(n + AHEAD);
+      const int st = n / KS, s = n % KS;
 #pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        const bf16x8 kf = load_bf16x8(kb + (16 * st + col) * L::KROW + 32 * s + 8 * g);
-#pragma unroll
-        for (int f = 0; f < QF; ++f) sc[f][st] = mfma16(kf, qf[f][s], sc[f][st]);
+      for (int f = 0; f < QF; ++f) {
+        if (s == 0) sc[f][st] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        sc[f][st] = mfma16(kf[n], qf[f][s], sc[f][st]);
       }
     }
     if (!whole) {
@@ -436,18 +444,21 @@ __global__ __launch_bounds__(64 * NW, NB == 1 ? 2 : 1) void latent_prefill_kerne
 #pragma unroll
         for (int i = 0; i < NT; ++i) o[f][i] *= alpha[f];
     }
+    bf16x8 vf[2 * NT];
+    auto read_v = [&](int n) {
+      const bf16_t* p = vb + tr_off + 32 * (n % 2) * L::VROW + 16 * (n / 2);
+      const bf16x4 lo = lat_read_tr16(p), hi = lat_read_tr16(p + 16 * L::VROW);
 #pragma unroll
-    for (int i = 0; i < NT; ++i) {
+      for (int j = 0; j < 4; ++j) { vf[n][j] = lo[j]; vf[n][4 + j] = hi[j]; }
+    };
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        const bf16x4 lo = lat_read_tr16(vb + tr_off + 32 * ks * L::VROW + 16 * i);
-        const bf16x4 hi = lat_read_tr16(vb + tr_off + (32 * ks + 16) * L::VROW + 16 * i);
-        bf16x8 vf;
+    for (int n = 0; n < AHEAD; ++n) read_v(n);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) { vf[j] = lo[j]; vf[4 + j] = hi[j]; }
+    for (int n = 0; n < 2 * NT; ++n) {
+      if constexpr (AHEAD > 0) __builtin_amdgcn_sched_barrier(0);
+      if (n + AHEAD < 2 * NT) read_v(n + AHEAD);
 #pragma unroll
-        for (int f = 0; f < QF; ++f) o[f][i] = mfma16(vf, pf[f][ks], o[f][i]);
-      }
+      for (int f = 0; f < QF; ++f) o[f][n / 2] = mfma16(vf[n], pf[f][n % 2], o[f][n / 2]);
     }
   }
 #pragma unroll

@@ -33,19 +33,19 @@ def prefill_persist_for(max_len: int) -> bool:
 
 
 def prefill_form(max_len: int, ntiles: int, Hq: int, Hkv: int, D: int) -> int:
-    """Launch form of the prefill attention: 1 persistent workgroups, + 2 the next tile's scores ahead (four heads of 128
-    to a KV head).  us, plain / persistent / ahead / both.  A workgroup an item: persistent ones gain nothing, and ahead
-    pays from 320 tokens (one prompt, 16 heads: 200 12.7 / 13.3 / 12.9 / 13.4, 256 14.8 / 15.4 / 14.8 / 15.3, 320 16.7 / 17.6 / 16.3 /
-    16.8, 700 27.6 / 29.6 / 25.4 / 26.1, 2000 64 / 71 / 58 / 59).  More: from 640 (32 heads: 20 x 384 64 / 60 / 66 / 61, 16 x 512
-    90 / 80 / 94 / 84, 12 x 640 76 / 73.5 / 78 / 72.4, 8 x 1000 103 / 101 / 101 / 96.5, 4 x 3000 340 / 349 / 321 / 320)."""
+    """Launch form of the prefill attention: 1 persistent workgroups, 2 the next tile's scores ahead (four heads of 128 to a
+    KV head), 0 neither.  us, plain / persistent / ahead.  A workgroup an item: persistent ones gain nothing, and ahead pays
+    from 512 tokens (one prompt, 16 heads: 256 14.2 / 14.7 / 14.7, 384 17.7 / 18.2 / 17.9, 512 21.4 / 22.1 / 21.2, 700 26.4 / 27.6 /
+    25.7).  More: where persistent ones lose (32 heads: 16 x 512 90 / 82 / 94, 8 x 1000 99 / 97 / 100, 8 x 1200 133.5 / 132.0 / 133.3,
+    4 x 3000 324 / 334 / 317)."""
     persist = prefill_persist_for(max_len)
     G = Hq // Hkv
     if D != 128 or G % 4:
         return int(persist)
     one = ntiles * (Hq // 4) <= 256  # CUs
-    if one and _prefill_persist[0] is None:
-        persist = False
-    return int(persist) | (2 if max_len >= (320 if one else 640) else 0)
+    if persist and (not one or _prefill_persist[0] is not None):
+        return 1
+    return 2 if not one or max_len >= 512 else 0
 
 
 # ----------------------------------------------------------------- prefill

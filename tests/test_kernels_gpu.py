@@ -404,8 +404,8 @@ def test_prefill_small_scales(hipk, D, Hq, Hkv, scale, causal, persist):
 @pytest.mark.parametrize("sign", [1, -1])
 @pytest.mark.parametrize("inf", [False, True])
 def test_prefill_scores_ahead(hipk, Hq, Hkv, causal, sign, inf):
-    """The next tile's scores ahead, an item a workgroup or several: the sums of the kernel without, in its order, at every
-    number of tiles and remainder."""
+    """The next tile's scores ahead, persistent workgroups: the sums of the kernel without, in its order, at every number of
+    tiles and remainder."""
     from drtc_amd.ops.attention import prefill_tiles
     lens = [1, 63, 64, 65, 127, 128, 129, 192, 193, 256, 300, 385, 700]
     cu, D = [sum(lens[:i]) for i in range(len(lens) + 1)], 128
@@ -417,7 +417,7 @@ def test_prefill_scores_ahead(hipk, Hq, Hkv, causal, sign, inf):
     cu_d = torch.tensor(cu, dtype=torch.int32, device=DEV)
     ts, tq = (torch.tensor(t, dtype=torch.int32, device=DEV) for t in prefill_tiles(cu))
     outs = []
-    for form in range(4):
+    for form in range(3):
         outs.append(torch.full((cu[-1], Hq * D + 8), 7.0, device=DEV, dtype=torch.bfloat16))
         assert hipk.prefill_attn(outs[-1].data_ptr(), Hq * D + 8, qkv.data_ptr(), qkv.stride(0), Hq, Hkv, D, cu_d.data_ptr(),
                                  ts.data_ptr(), tq.data_ptr(), ts.numel(), sign * D ** -0.5, int(causal), form,
@@ -428,8 +428,8 @@ def test_prefill_scores_ahead(hipk, Hq, Hkv, causal, sign, inf):
 
 def test_prefill_form_rule():
     from drtc_amd.ops.attention import prefill_form
-    assert [prefill_form(n, 3, 32, 8, 128) for n in (148, 256, 320, 1000, 4000)] == [0, 0, 2, 2, 2]
-    assert [prefill_form(n, 500, 32, 8, 128) for n in (148, 500, 640, 1000, 1025)] == [1, 1, 3, 3, 2]
+    assert [prefill_form(n, 3, 32, 8, 128) for n in (148, 511, 512, 1000, 4000)] == [0, 0, 2, 2, 2]
+    assert [prefill_form(n, 500, 32, 8, 128) for n in (148, 640, 1024, 1025)] == [1, 1, 1, 2]
     assert [prefill_form(n, 3, 16, 8, 128) for n in (148, 1000, 4000)] == [1, 1, 0]  # two heads
     assert [prefill_form(n, 3, 32, 8, 64) for n in (148, 4000)] == [1, 0]
 
