@@ -256,6 +256,9 @@ def _resolve(M: int, N: int, K: int, ldx: int) -> tuple[str, int]:
     if ldx % 8 == 0 and stream_ok(M, N, K) and (found is None or (found[0], N, K, ldx) not in _kept):
         return ("skinny", STREAM)
     if found is None:
+        deep = deep_form(M, N, K)
+        if deep and ldx % 8 == 0:
+            return ("xd", deep)
         v = skinny_variant(M, N, K, ldx)
         return ("skinny", v) if v else ("torch", 0)
     _, (algo, sk, midm, xd, _) = found
@@ -339,6 +342,36 @@ def tall_form(M: int, N: int, K: int, glu: bool = False, act: str = "silu") -> i
         return 0
     form = 1001 + 100 * mt + 10 * nf
     return form if xd_supported(M, N, K, form, glu) else 0
+
+
+DEEP_FORMS = (122, 123, 124, 142, 143, 144, 162, 163, 164, 242, 243, 244)
+
+
+@functools.lru_cache(maxsize=4096)
+def _deep_form(M: int, N: int, K: int) -> int:
+    best, cost = 0, 0.0
+    for form in DEEP_FORMS:
+        mt, nf, sk = xd_form(form)
+        tm, tn = XD_ROWS[mt], 32 * nf
+        items = -(-M // tm) * (N // tn) * sk
+        if not 100 <= items <= 256 or not xd_supported(M, N, K, form):
+            continue
+        us = 7 + (tm + tn) * K / sk / 1e6 * (20 + 0.0387 * items) + tm * tn / 1e5 * (31 + 1.1 * (sk - 1))
+        if not best or us < cost:
+            best, cost = form, us
+    return best
+
+
+def deep_form(M: int, N: int, K: int) -> int:
+    """gemm_xd form, K in slices, of a product of 257 .. 1024 rows without a tuned one that has long K and too few tiles for
+    the CUs, which the library takes whole: the form of least cost by a fit (us; 6 to 9 % off) of the bytes a workgroup reads, those that
+    all of them do and the slices' sums.  us, library / this: 2048 x 7168, 257 rows 28.5 / 23.0, 512 32.0 / 28.3, 640 40.2 / 35.4,
+    1024 45.9 / 42.5; 2048 x 14336, 448 rows 58.8 / 40.8; 1024 x 7168, 1024 32.4 / 27.5; 2304 x 9216 1.24 times, 5120 x 13824 1.26, 4096 x
+    11008 1.17 over thirteen row counts.  Shorter K: 2048 x 4096, 768 rows 24.1 / 26.9; three of the library's row tiles of
+    256 on wider W: 4096 x 7168, 768 rows 54.9 / 57.7, 4096 x 8192 57.9 / 61.0."""
+    if not (257 <= M <= DECODE_MAX_M and K >= 5632 and _xd_enabled and _enabled) or 640 < M <= 768 and N >= 4096 and K <= 8192:
+        return 0
+    return _deep_form(M, N, K)
 
 
 def wide_form(M: int, N: int, K: int) -> int:

@@ -424,6 +424,19 @@ def test_xd_gemm_one_tall_tile(hipk, form, M, K, epi):
     _check(out, ref)
 
 
+@pytest.mark.parametrize("M,N,K", [(257, 2048, 5632), (512, 1024, 7168), (640, 1536, 5696), (1000, 2048, 7168), (300, 2304, 9216)])
+@pytest.mark.parametrize("pad", [0, 8, 4])
+def test_linear_of_long_k(hipk, M, N, K, pad):
+    """Few tiles and long K in slices, rows apart (4: off 16 bytes, the library): fp32 sums rounded once."""
+    form = G.deep_form(M, N, K)
+    assert form and (G.route(M, N, K, K + pad) == ("xd", form)) == (pad % 8 == 0)
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x = torch.randn(M, K + pad, device="cuda", generator=g).to(torch.bfloat16)[:, :K]
+    w = (torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).to(torch.bfloat16)
+    for _ in range(2):  # the counters are armed again
+        _check(G.linear(x, w), _ref(x, w, "store", None))
+
+
 @pytest.mark.parametrize("v", range(1, 10))
 @pytest.mark.parametrize("M", [1, 2, 3, 8, 9, 16])
 @pytest.mark.parametrize("N,N2,K,relu2", [(256, 128, 512, True), (128, 384, 1536, False), (512, 256, 128, True)])

@@ -35,6 +35,20 @@ def test_tall_tiles_rule(monkeypatch, M, N, K, glu, want):
         assert not G.xd_supported(M, N, K, want - 1000, glu) and not G.xd_supported(M, N, K, want + 1, glu)
 
 
+@pytest.mark.parametrize("N,K", [(2048, 7168), (2048, 14336), (1024, 5632), (4096, 8192), (3072, 5696), (2080, 7168)])
+def test_deep_products_rule(monkeypatch, N, K):
+    monkeypatch.setattr(G, "_xd_enabled", True)
+    for M in (257, 300, 512, 640, 641, 768, 769, 1024):
+        form = G.deep_form(M, N, K)
+        if 640 < M <= 768 and N >= 4096 or N == 2080 and not form:  # the library; no whole tiles
+            assert form == 0
+            continue
+        mt, nf, sk = G.xd_form(form)
+        assert sk > 1 and G.xd_supported(M, N, K, form)
+        assert 100 <= -(-M // G.XD_ROWS[mt]) * (N // (32 * nf)) * sk <= 256  # a workgroup a CU
+    assert not G.deep_form(256, N, K) and not G.deep_form(1025, N, K) and not G.deep_form(512, N, 5568)
+
+
 @pytest.mark.parametrize("M,form,want", [
     (256, 244, 1244),   # one 256-row tile: every weight byte read once
     (128, 141, 1141),
