@@ -230,13 +230,19 @@ def _resolve(M: int, N: int, K: int, ldx: int) -> tuple[str, int]:
                 return ("lt", ent[0])
     if M > DECODE_MAX_M:
         if w4_shape_ok(M, N, K):
-            # 256 x 256 tiles for a quarter of the CUs at most: smaller ones
-            if -(-M // 256) * (N // 256) <= 64 and _xd_enabled and xd_supported(M, N, K, 141):
-                return ("xd", 141)
+            # 256 x 256 tiles for a quarter of the CUs at most, or a half: smaller ones (4096 rows, 2048 x 2048 39.1 / 31.3 us,
+            # 2048 x 7168 134 / 99)
+            tiles = -(-M // 256) * (N // 256)
+            form = 141 if tiles <= 64 else 241 if tiles <= 128 else 0
+            if form and _xd_enabled and xd_supported(M, N, K, form):
+                return ("xd", form)
             return ("w4", 0)
         a = _prefill_algo(M, N, K, ldx, 0)
         if a >= 0:
             return ("lt", a)
+        full = full_form(M, N, K)
+        if full and ldx % 8 == 0:
+            return ("xd", full)
         return ("w4", 0) if _w4_long(M, N, K) else ("torch", 0)
     if dot2_ok(M, N, K, ldx):
         return ("skinny", 1)
@@ -256,12 +262,14 @@ def _resolve(M: int, N: int, K: int, ldx: int) -> tuple[str, int]:
     if ldx % 8 == 0 and stream_ok(M, N, K) and (found is None or (found[0], N, K, ldx) not in _kept):
         return ("skinny", STREAM)
     if found is None:
-        deep = deep_form(M, N, K)
-        if deep and ldx % 8 == 0:
-            return ("xd", deep)
+        form = deep_form(M, N, K) or full_form(M, N, K)
+        if form and ldx % 8 == 0:
+            return ("xd", form)
         v = skinny_variant(M, N, K, ldx)
         return ("skinny", v) if v else ("torch", 0)
     _, (algo, sk, midm, xd, _) = found
+    if K <= 1024 and not (sk or midm or xd) and ldx % 8 == 0 and full_form(M, N, K):
+        return ("xd", full_form(M, N, K))
     if algo < 0 and not (sk or midm or xd):
         return ("torch", 0)  # measured: the library's heuristic pick beat every candidate
     if sk and M <= SKINNY_MAX_M and skinny_supports(sk, M, N, K, ldx):
@@ -372,6 +380,26 @@ def deep_form(M: int, N: int, K: int) -> int:
     if not (257 <= M <= DECODE_MAX_M and K >= 5632 and _xd_enabled and _enabled) or 640 < M <= 768 and N >= 4096 and K <= 8192:
         return 0
     return _deep_form(M, N, K)
+
+
+def full_form(M: int, N: int, K: int) -> int:
+    """gemm_xd form of a plain product of 129 .. 3072 rows without a tuned one that some tile, the smallest that makes at
+    most a workgroup a CU, cuts into one well filled round: 200 workgroups, 128 where K is short.  420 sizes of 24 widths, K 512
+    .. 5120, the library's time / this: 200 .. 256 workgroups 1.31 (K 512, 768), 1.20 (to 1536), 1.21 (2048), 1.13 (to 3072), 1.11, nine
+    of 203 below 0.97; K to 1536, 128 .. 199 1.27; longer K and fewer 1.06, a third below 0.97.  us: 6656 x 2048, 256 rows 24.7 /
+    16.9, 448 24.4 / 19.9, 1024 31.1 / 29.6; 12800 x 4096, 256 49.4 / 42.8; 3072 x 2048, 1088 23.6 / 19.1; past 3072 rows 3072 x 2048,
+    3360 37.7 / 39.9, 1024 x 3072, 4064 28.3 / 33.0.  The table's library solutions of short K as well: 4096 x 512, 256 rows 8.2 /
+    5.5, 1024 9.7 / 8.6."""
+    if not (129 <= M <= 3072 and _xd_enabled and _enabled):
+        return 0
+    for form in (121, 141, 161, 241, 261):
+        mt, nf, _ = xd_form(form)
+        items = -(-M // XD_ROWS[mt]) * (N // (32 * nf))
+        if items <= 256 and xd_supported(M, N, K, form):
+            if items < (128 if K <= 1536 else 200):
+                return 0
+            return form + 1000 if _xd_nt and xd_nt_ok(M, form) else form
+    return 0
 
 
 def wide_form(M: int, N: int, K: int) -> int:

@@ -424,6 +424,18 @@ def test_xd_gemm_one_tall_tile(hipk, form, M, K, epi):
     _check(out, ref)
 
 
+@pytest.mark.parametrize("M,N,K", [(129, 4160, 512), (200, 6656, 2048), (1057, 3072, 2048), (3072, 2048, 1024), (150, 16640, 1088)])
+@pytest.mark.parametrize("pad", [0, 8, 4])
+def test_linear_of_one_full_round(hipk, M, N, K, pad):
+    """One round of gemm_xd tiles, rows apart (4: off 16 bytes, the library): fp32 sums rounded once."""
+    form = G.full_form(M, N, K)
+    assert form and (G.route(M, N, K, K + pad) == ("xd", form)) == (pad % 8 == 0)
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x = torch.randn(M, K + pad, device="cuda", generator=g).to(torch.bfloat16)[:, :K]
+    w = (torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).to(torch.bfloat16)
+    _check(G.linear(x, w), _ref(x, w, "store", None))
+
+
 @pytest.mark.parametrize("M,N,K", [(257, 2048, 5632), (512, 1024, 7168), (640, 1536, 5696), (1000, 2048, 7168), (300, 2304, 9216)])
 @pytest.mark.parametrize("pad", [0, 8, 4])
 def test_linear_of_long_k(hipk, M, N, K, pad):

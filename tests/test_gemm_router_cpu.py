@@ -49,6 +49,20 @@ def test_deep_products_rule(monkeypatch, N, K):
     assert not G.deep_form(256, N, K) and not G.deep_form(1025, N, K) and not G.deep_form(512, N, 5568)
 
 
+@pytest.mark.parametrize("M,N,K,want", [
+    (256, 6656, 2048, 121), (448, 6656, 2048, 141), (1024, 6656, 2048, 241), (2048, 3072, 2048, 161), (300, 12800, 4096, 241),
+    (256, 25600, 4096, 1241),                   # one row tile: weights past the caches
+    (129, 4096, 512, 121), (1024, 4096, 512, 141), (192, 8192, 512, 121),
+    (640, 6656, 2048, 0), (128, 12800, 4096, 0), (3073, 3072, 2048, 0), (300, 6640, 2048, 0), (256, 4096, 256, 0),
+])
+def test_full_round_rule(monkeypatch, M, N, K, want):
+    monkeypatch.setattr(G, "_xd_nt", True)
+    monkeypatch.setattr(G, "_xd_enabled", True)
+    assert G.full_form(M, N, K) == want
+    if want:
+        assert G.xd_supported(M, N, K, want) and G.xd_form(want)[2] == 1
+
+
 @pytest.mark.parametrize("M,form,want", [
     (256, 244, 1244),   # one 256-row tile: every weight byte read once
     (128, 141, 1141),
