@@ -1121,8 +1121,7 @@ def _glu_default(M: int, I: int, K: int, act: str = "silu") -> int:
     4096, 128 rows 40.9 / 34.6, 448 62.9 / 56.5; 28672 x 8192, 24 rows 169 / 155, 96 199 / 177.
     Tiles of 128 columns a half lose to narrower ones up to 128 rows (28672 x 8192 188 / 199, narrow 179),
     with long K above them (20480 x 8192, 160 rows 179 / 203; 16384 x 4096 154 / 137) and to the library from
-    256 rows to gemm_w4's first (14336 x 4096, 320 rows 82 / 97; 7168 x 4096, 600 72 / 87, 5632 x 2048 39 / 48), but for
-    short K that fills the CUs (7168 x 2048, 560 rows 47.4 / 47.2, in one launch).
+    256 rows to gemm_w4's first (14336 x 4096, 320 rows 82 / 97; 7168 x 4096, 600 72 / 87, 5632 x 2048 39 / 48).
     Above 512 rows for the shapes that leave gemm_w4 fewer than three quarters of the CUs: 3584 x 2048, 768 rows
     90 / 29.6, 1024 49 / 30.7; 7168 x 2048, 1024 rows (224 tiles) 53.0 / 53.4.
     The clamped activation has tiles of 64 and 128 columns only: 64 in place of 32 up to 128 rows (7168 x
@@ -1131,7 +1130,7 @@ def _glu_default(M: int, I: int, K: int, act: str = "silu") -> int:
         return 0
     form = xd_default_form(M, I, K, True)
     if form // 10 % 10 == 8 and M < W4_GLU_MIN_M:
-        if M > 256 and not (M > 512 and K <= 2048 and -(-M // 256) * (I // 128) >= 160) or M > 128 and K > 4096:
+        if M > 256 or M > 128 and K > 4096:
             return 0
         if M <= 128:
             form = 141
