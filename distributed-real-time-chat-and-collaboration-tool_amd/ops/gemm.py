@@ -1107,8 +1107,16 @@ def glu_form(M: int, N2: int, K: int, ldx: int, act: str = "silu") -> int:
     found = _decode_entry(M, N2, K, ldx)
     form = found[1][4] if found is not None else 0
     if not form or act == "clamped" and form // 10 % 10 not in XD_CLAMP_NF:
-        form = _glu_default(M, N2 // 2, K, act)
+        form = _glu_default(M, N2 // 2, K, act) or _glu_prompt(M, N2 // 2, K)
     return form if form and xd_supported(M, N2 // 2, K, form, glu=True) else 0
+
+
+def _glu_prompt(M: int, I: int, K: int) -> int:
+    """gemm_xd gated form of 513 rows up to gemm_w4's first where short K fills the CUs with tiles of 256 x 256: as fast as
+    the library and a pass on the chip (7168 x 2048, 560 rows 47.2 / 47.4 us, 608 49.3 / 47.5), but prompts of these rows, which
+    no decode step is padded to, are as long as their host path, and this is one launch for two (width 2048, two prompts of 300
+    642 -> 554 us)."""
+    return 281 if 512 < M < W4_GLU_MIN_M and K <= 2048 and 160 <= -(-M // 256) * (I // 128) <= 256 else 0
 
 
 def _glu_default(M: int, I: int, K: int, act: str = "silu") -> int:

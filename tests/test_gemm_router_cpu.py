@@ -63,6 +63,15 @@ def test_full_round_rule(monkeypatch, M, N, K, want):
         assert G.xd_supported(M, N, K, want) and G.xd_form(want)[2] == 1
 
 
+@pytest.mark.parametrize("M,I,K,want", [(513, 7168, 2048, 281), (639, 7168, 2048, 281), (512, 7168, 2048, 241), (600, 5632, 2048, 0),
+                                        (600, 7168, 2112, 0), (600, 14336, 2048, 0)])
+@pytest.mark.parametrize("act", ["silu", "clamped"])
+def test_gated_prompts_of_short_k(monkeypatch, M, I, K, want, act):
+    monkeypatch.setattr(G, "_xd_enabled", True)
+    monkeypatch.setattr(G, "_activate", lambda: {})
+    assert G.glu_form(M, 2 * I, K, K, act) == want
+
+
 @pytest.mark.parametrize("M,form,want", [
     (256, 244, 1244),   # one 256-row tile: every weight byte read once
     (128, 141, 1141),
