@@ -697,6 +697,12 @@ __global__ __launch_bounds__(256) void stage_rows_kernel(unsigned* __restrict__ 
 // 204; 224 of 256 rows 627 / 612, 64 of 64 597 / 582.
 __global__ __launch_bounds__(256) void step_stage_kernel(unsigned* __restrict__ dst, const unsigned* host0, const unsigned* host1,
                                                          StageRanges r, StepTokens t, int* turn) {
+  // One wave reads the turn for its workgroup, and counts it when it has it: no read is left that the next turn could
+  // overtake.  (Read by every wave, a barrier behind the read and a count behind that do not make the other waves' reads
+  // complete: a barrier waits for no load from memory.)
+  __shared__ int whose;
+  int turn_now = 0;
+  if (threadIdx.x < 64) turn_now = __hip_atomic_load(turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   // the tokens are what a step waits for: both sets' are on their way with the turn, one trip over the bus
   unsigned ahead[6];
   const int first = blockIdx.x * 1024 + threadIdx.x;
@@ -709,9 +715,10 @@ __global__ __launch_bounds__(256) void step_stage_kernel(unsigned* __restrict__ 
       ahead[3 * k + 2] = host_word(h + t.host + first);
     }
   }
-  const int set = __hip_atomic_load(turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const unsigned* host = set & 1 ? host1 : host0;
+  if (threadIdx.x == 0) whose = turn_now;
   __syncthreads();
+  const int set = whose;
+  const unsigned* host = set & 1 ? host1 : host0;
   if (threadIdx.x == 0 &&
       __hip_atomic_fetch_add(turn + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)(gridDim.x * gridDim.y) - 1) {
     __hip_atomic_store(turn + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -1,0 +1,32 @@
+"""Decode staging: what of it can be checked without a GPU."""
+import os
+import re
+import subprocess
+
+import pytest
+
+from drtc_amd import _build
+
+
+@pytest.mark.skipif(not os.path.exists(_build.HIPCC), reason="no hipcc")
+def test_the_turn_has_arrived_before_a_workgroup_counts_itself(tmp_path):
+    """step_stage_kernel, as compiled: no read of whose turn it is (the only load at agent scope) is under way at the
+    workgroup's first barrier, behind which the workgroup counts and the last one gives the turn away.  The barrier itself
+    waits for no load."""
+    src, asm = os.path.join(_build.CSRC, "kernels", "sampling.hip"), tmp_path / "sampling.s"
+    subprocess.run([_build.HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=fast", "-Xclang", "-target-feature",
+                    "-Xclang", "-packed-fp32-ops", "--offload-device-only", "-S", src, "-o", str(asm)], check=True,
+                   capture_output=True)
+    text = asm.read_text()
+    body = text[re.search(r"^\w*step_stage_kernel\w*:", text, re.M).end():]
+    under_way, looked = False, 0
+    for line in body[:body.index("s_endpgm")].splitlines():
+        op = line.split(";")[0].strip()
+        if op.startswith("global_load") and re.search(r"\bsc1\b", op) and not re.search(r"\bsc0\b", op):
+            under_way, looked = True, looked + 1
+        elif op.startswith("s_waitcnt") and re.search(r"vmcnt\(0\)", op):
+            under_way = False
+        elif op.startswith("s_barrier"):
+            assert looked and not under_way
+            return
+    raise AssertionError("no barrier")
