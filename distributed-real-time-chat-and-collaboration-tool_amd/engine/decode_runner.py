@@ -21,6 +21,7 @@ from __future__ import annotations
 
 import bisect
 import os
+import weakref
 
 import numpy as np
 import torch
@@ -42,6 +43,23 @@ def check_tokens(ids: np.ndarray, vocab: int) -> None:
     if ids.view(f"u{ids.itemsize}").max() >= vocab if ids.dtype.kind == "i" else ids.min() < 0 or ids.max() >= vocab:
         bad = ids[(ids < 0) | (ids >= vocab)]
         raise ValueError(f"token {bad[0]} outside of the vocabulary of {vocab}")
+
+
+# pinned buffers of runners that went while a graph was being recorded, and the events of their last steps
+_retired: list[tuple[list, tuple]] = []
+
+
+def _retire(events: list, buffers: tuple) -> None:
+    """Give a runner's pinned ``buffers`` back when its last steps have gone by.  Kernels read and write them by address,
+    which the host allocator does not know of: it would hand them out while a step is still under way."""
+    _retired.append((events, buffers))
+    if torch.cuda.is_initialized() and torch.cuda.is_current_stream_capturing():
+        return  # nothing may be waited for: the next runner to go does
+    while _retired:
+        for e in _retired[-1][0]:
+            if e is not None:
+                e.synchronize()
+        _retired.pop()
 
 
 class DecodeRunner:
@@ -92,6 +110,7 @@ class DecodeRunner:
             h.fill_(-1)
         self.h_out = [torch.zeros(B, dtype=torch.int32, pin_memory=pin) for _ in range(2)]
         self.events = [torch.cuda.Event() if pin else None for _ in range(2)]
+        weakref.finalize(self, _retire, self.events, (*self.h_stage, *self.h_out)).atexit = False
         self._k = 0
         # the set that the next replay reads (ops.step_stage), on the device and as the host has it
         self.turn, self._turn = torch.zeros(2, dtype=torch.int32, device=dev), 0

@@ -1,9 +1,12 @@
 """Decode staging: what of it can be checked without a GPU."""
+import gc
 import os
 import re
 import subprocess
+import weakref
 
 import pytest
+import torch
 
 from drtc_amd import _build
 
@@ -30,3 +33,38 @@ def test_the_turn_has_arrived_before_a_workgroup_counts_itself(tmp_path):
             assert looked and not under_way
             return
     raise AssertionError("no barrier")
+
+
+@pytest.mark.parametrize("recording", [False, True])
+def test_pinned_buffers_outlive_the_steps_of_a_runner(monkeypatch, recording):
+    """A runner that goes with steps under way keeps the buffers that their kernels address until the steps' events have
+    gone by, which are not waited for while a graph is recorded."""
+    from drtc_amd.engine import decode_runner
+    from drtc_amd.models import TINY_LLAMA, TransformerLM
+
+    m = TransformerLM(TINY_LLAMA, "cpu", seed=1)
+    seen = []
+
+    class Event:
+        def synchronize(self):
+            seen.append(all(b() is not None for b in buffers))
+
+    def runner():
+        r = decode_runner.DecodeRunner(m, m.new_cache(4, 4), 4, 8)
+        r.events[:] = [Event(), Event()]
+        return r
+
+    r = runner()
+    buffers = [weakref.ref(t) for t in (*r.h_stage, *r.h_out)]
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: recording)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: recording)
+    del r
+    gc.collect()
+    if recording:
+        assert not seen and all(b() is not None for b in buffers)
+        monkeypatch.undo()
+        r = runner()
+        del r
+        gc.collect()
+    assert seen == [True] * (4 if recording else 2) and not decode_runner._retired
+    assert all(b() is None for b in buffers)
