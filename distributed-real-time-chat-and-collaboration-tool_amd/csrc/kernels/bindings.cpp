@@ -248,8 +248,11 @@ PYBIND11_MODULE(_hipk, m) {
   m.def("embed", [](u64 out, u64 ids, int wide, u64 table, int rows, int V, int H, u64 st) {
     return drtc::launch_embed(P<void>(out), P<const void>(ids), wide, P<const void>(table), rows, V, H, S(st));
   });
-  static const auto stage_ranges = [](const std::vector<std::pair<unsigned, unsigned>>& ranges) {
+  using Ranges = std::vector<std::pair<unsigned, unsigned>>;
+  using Table = std::tuple<unsigned, unsigned, unsigned, unsigned, unsigned>;  // drtc::StageTable's first five
+  static const auto stage_ranges = [](const Ranges& ranges, const Table& t) {
     drtc::StageRanges r{};
+    r.table = {std::get<0>(t), std::get<1>(t), std::get<2>(t), std::get<3>(t), std::get<4>(t), 0, 0};
     if (ranges.size() > drtc::kStageRanges) r.n = -1;
     else for (const auto& [first, words] : ranges) {
       r.first[r.n] = first;
@@ -257,13 +260,13 @@ PYBIND11_MODULE(_hipk, m) {
     }
     return r;
   };
-  m.def("stage_rows", [](u64 dst, u64 host, const std::vector<std::pair<unsigned, unsigned>>& ranges, u64 st) {
-    return drtc::launch_stage_rows(P<void>(dst), P<const void>(host), stage_ranges(ranges), S(st));
-  });
-  m.def("step_stage", [](u64 dst, u64 host0, u64 host1, const std::vector<std::pair<unsigned, unsigned>>& ranges, u64 ids,
-                         u64 sampled, unsigned src, unsigned host, int B, u64 counter, u64 position, u64 turn, u64 st) {
+  m.def("stage_rows", [](u64 dst, u64 host, const Ranges& ranges, u64 st, const Table& table) {
+    return drtc::launch_stage_rows(P<void>(dst), P<const void>(host), stage_ranges(ranges, table), S(st));
+  }, py::arg(), py::arg(), py::arg(), py::arg(), py::arg() = Table{});
+  m.def("step_stage", [](u64 dst, u64 host0, u64 host1, const Ranges& ranges, const Table& table, u64 ids, u64 sampled, unsigned src,
+                         unsigned host, int B, u64 counter, u64 position, u64 turn, u64 st) {
     const drtc::StepTokens t{P<int>(ids), P<const int>(sampled), src, host, B, P<int64_t>(counter), P<int64_t>(position)};
-    return drtc::launch_step_stage(P<void>(dst), P<const void>(host0), P<const void>(host1), stage_ranges(ranges), t,
+    return drtc::launch_step_stage(P<void>(dst), P<const void>(host0), P<const void>(host1), stage_ranges(ranges, table), t,
                                    P<int>(turn), S(st));
   });
   m.def("step_begin", [](u64 ids, u64 src, u64 sampled, u64 host, int B, u64 counter, u64 position, u64 st) {

@@ -64,13 +64,20 @@ int launch_prefill_attn(void* out, int out_stride, const void* qkv,
                         hipStream_t st);
 
 int launch_embed(void* out, const void* ids, int wide, const void* table, int rows, int V, int H, hipStream_t st);
-// ranges of words that a step's staging copies, first and count of each
-constexpr int kStageRanges = 12;
+// ranges of words that a step's staging copies, first and count of each, and of a table [rows, columns] as many of a row's
+// words as its length comes to, one to `per` of it (rows 0: none)
+constexpr int kStageRanges = 12, kStageWords = 1024, kStageChunk = 128;  // words to a workgroup, columns to a row's 16 lanes
+struct StageTable {
+  unsigned first, rows, columns, lengths, per;
+  unsigned ahead, chunks;  // (the launchers')
+};
 struct StageRanges {
   int n;
   unsigned first[kStageRanges], words[kStageRanges];
+  StageTable table;
+  unsigned rest, start[kStageRanges + 1];  // (the launchers': first workgroups of the table behind `ahead`, of each range)
 };
-int launch_stage_rows(void* dst, const void* host, const StageRanges& r, hipStream_t st);
+int launch_stage_rows(void* dst, const void* host, StageRanges r, hipStream_t st);
 // step_begin's, its src and host arrays as words of the staging sets
 struct StepTokens {
   int* ids;
@@ -79,7 +86,7 @@ struct StepTokens {
   int B;
   int64_t *counter, *position;
 };
-int launch_step_stage(void* dst, const void* host0, const void* host1, const StageRanges& r, const StepTokens& t, int* turn,
+int launch_step_stage(void* dst, const void* host0, const void* host1, StageRanges r, const StepTokens& t, int* turn,
                       hipStream_t st);
 int launch_step_begin(int* ids, const int64_t* src, const int* sampled, const int* host, int B, int64_t* counter,
                       int64_t* position, hipStream_t st);

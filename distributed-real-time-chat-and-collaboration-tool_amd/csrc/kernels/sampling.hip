@@ -677,8 +677,8 @@ __global__ __launch_bounds__(256) void step_begin_kernel(int* __restrict__ ids, 
 DRTC_DEVICE unsigned host_word(const unsigned* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-DRTC_DEVICE void stage_words(unsigned* dst, const unsigned* host, unsigned first, unsigned words) {
-  const unsigned i = blockIdx.x * 1024 + threadIdx.x;
+DRTC_DEVICE void stage_words(unsigned* dst, const unsigned* host, unsigned first, unsigned words, unsigned blk) {
+  const unsigned i = blk * kStageWords + threadIdx.x;
   unsigned v[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j)
@@ -687,8 +687,59 @@ DRTC_DEVICE void stage_words(unsigned* dst, const unsigned* host, unsigned first
   for (int j = 0; j < 4; ++j)
     if (i + 256 * j < words) dst[first + i + 256 * j] = v[j];
 }
+// The table's first `ahead` columns, of all rows, which wait for no length.
+DRTC_DEVICE void stage_ahead(unsigned* dst, const unsigned* host, const StageTable& t, unsigned blk) {
+  const unsigned e = blk * kStageWords + threadIdx.x, words = t.rows * t.ahead;
+  if (t.ahead == t.columns) {
+    stage_words(dst, host, t.first, words, blk);
+    return;
+  }
+  unsigned at[4], v[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const unsigned row = (e + 256 * j) / t.ahead;
+    at[j] = t.first + row * t.columns + (e + 256 * j - row * t.ahead);
+    if (e + 256 * j < words) v[j] = host_word(host + at[j]);
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (e + 256 * j < words) dst[at[j]] = v[j];
+}
+// The others as far as the rows' lengths say, 16 rows to a workgroup: 16 lanes a row take every chunks-th kStageChunk columns
+// from `chunk` on.  The lengths are one request of the workgroup: many workgroups ask for the same ones, and the bus
+// serves requests for a line one after the other.
+DRTC_DEVICE void stage_rest(unsigned* dst, const unsigned* host, const StageTable& t, unsigned row, unsigned chunk) {
+  __shared__ unsigned needs[16];
+  if (threadIdx.x < 16) {
+    const unsigned length = row + threadIdx.x < t.rows ? host_word(host + t.lengths + row + threadIdx.x) : 0;
+    needs[threadIdx.x] = min(length / t.per + (length % t.per != 0), t.columns);
+  }
+  __syncthreads();
+  const unsigned need = needs[threadIdx.x >> 4], at = t.first + (row + (threadIdx.x >> 4)) * t.columns;
+  for (unsigned c = t.ahead + kStageChunk * chunk + (threadIdx.x & 15); c < need; c += kStageChunk * t.chunks) {
+    unsigned v[kStageChunk / 16];
+#pragma unroll
+    for (unsigned j = 0; j < kStageChunk / 16; ++j)
+      if (c + 16 * j < need) v[j] = host_word(host + at + c + 16 * j);
+#pragma unroll
+    for (unsigned j = 0; j < kStageChunk / 16; ++j)
+      if (c + 16 * j < need) dst[at + c + 16 * j] = v[j];
+  }
+}
+DRTC_DEVICE void stage_part(unsigned* dst, const unsigned* host, const StageRanges& r, unsigned blk) {
+  if (blk < r.rest) {
+    stage_ahead(dst, host, r.table, blk);
+  } else if (blk < r.start[0]) {
+    const unsigned group = (blk - r.rest) / r.table.chunks;
+    stage_rest(dst, host, r.table, 16 * group, blk - r.rest - group * r.table.chunks);
+  } else {
+    int i = 0;
+    while (blk >= r.start[i + 1]) ++i;
+    stage_words(dst, host, r.first[i], r.words[i], blk - r.start[i]);
+  }
+}
 __global__ __launch_bounds__(256) void stage_rows_kernel(unsigned* __restrict__ dst, const unsigned* host, StageRanges r) {
-  stage_words(dst, host, r.first[blockIdx.y], r.words[blockIdx.y]);
+  stage_part(dst, host, r, blockIdx.x);
 }
 
 // The same along with the start of the step, the first node of its graph: the two staging sets take turns, and the last
@@ -703,69 +754,73 @@ __global__ __launch_bounds__(256) void step_stage_kernel(unsigned* __restrict__ 
   __shared__ int whose;
   int turn_now = 0;
   if (threadIdx.x < 64) turn_now = __hip_atomic_load(turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  // the tokens are what a step waits for: both sets' are on their way with the turn, one trip over the bus
+  // the tokens, the first workgroups', are what a step waits for: both sets' are on their way with the turn, one trip
+  const int tokens = (t.B + 255) / 256, i = blockIdx.x * 256 + threadIdx.x;
   unsigned ahead[6];
-  const int first = blockIdx.x * 1024 + threadIdx.x;
-  if ((int)blockIdx.y == r.n && first < t.B) {
+  if (i < t.B) {
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const unsigned* h = k ? host1 : host0;
-      ahead[3 * k] = host_word(h + t.src + 2 * first);
-      ahead[3 * k + 1] = host_word(h + t.src + 2 * first + 1);
-      ahead[3 * k + 2] = host_word(h + t.host + first);
+      ahead[3 * k] = host_word(h + t.src + 2 * i);
+      ahead[3 * k + 1] = host_word(h + t.src + 2 * i + 1);
+      ahead[3 * k + 2] = host_word(h + t.host + i);
     }
   }
   if (threadIdx.x == 0) whose = turn_now;
   __syncthreads();
   const int set = whose;
-  const unsigned* host = set & 1 ? host1 : host0;
   if (threadIdx.x == 0 &&
-      __hip_atomic_fetch_add(turn + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)(gridDim.x * gridDim.y) - 1) {
+      __hip_atomic_fetch_add(turn + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1) {
     __hip_atomic_store(turn + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(turn, set ^ 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  if ((int)blockIdx.y < r.n) {
-    stage_words(dst, host, r.first[blockIdx.y], r.words[blockIdx.y]);
+  if ((int)blockIdx.x >= tokens) {
+    stage_part(dst, set & 1 ? host1 : host0, r, blockIdx.x - tokens);
     return;
   }
-  for (int i = blockIdx.x * 1024 + threadIdx.x; i < min(t.B, (int)(blockIdx.x + 1) * 1024); i += 256) {
-    const int e = i - blockIdx.x * 1024 >= 256;  // (the first ones are asked for ahead)
-    unsigned lo = ahead[0], hi = ahead[1], id = ahead[2];
-    if (e) {
-      lo = host_word(host + t.src + 2 * i), hi = host_word(host + t.src + 2 * i + 1), id = host_word(host + t.host + i);
-    } else if (set & 1) {
-      lo = ahead[3], hi = ahead[4], id = ahead[5];
-    }
+  if (i < t.B) {
+    const unsigned lo = set & 1 ? ahead[3] : ahead[0], hi = set & 1 ? ahead[4] : ahead[1], id = set & 1 ? ahead[5] : ahead[2];
     const int64_t s = (int64_t)((uint64_t)hi << 32 | lo);
     t.ids[i] = s < 0 ? (int)id : s < t.B ? t.sampled[s] : -1;
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
+  if (i == 0) {
     const int64_t c = *t.counter;
     *t.position = c;
     *t.counter = c + 1;
   }
 }
 
-static bool stage_ok(const void* dst, const StageRanges& r, unsigned& most) {
-  most = 0;
-  if (r.n < 0 || r.n > kStageRanges || (uintptr_t)dst % 4) return false;
-  for (int i = 0; i < r.n; ++i) most = std::max(most, r.words[i]);
+// Cuts the ranges and the table into workgroups; false: out of what the kernels take.
+static bool stage_cut(const void* dst, StageRanges& r) {
+  StageTable& t = r.table;
+  if (r.n < 0 || r.n > kStageRanges || (uintptr_t)dst % 4 || (t.rows && (!t.per || (uint64_t)t.rows * t.columns >= 1u << 31)))
+    return false;
+  if (t.columns == 0) t.rows = 0;
+  // ahead of the lengths: 16 KB of all rows, a fraction of a trip over the bus.  Of the rest at most 512 workgroups, or eight to
+  // 16 rows, as each counts itself; more columns than they have lanes for are taken in turn.  Steps of four layers of 2048, us,
+  // tables of 512 / 5120 / 32,768 tokens: 1024 rows of contexts of 150, whole rows by the copy engines 1003 / 1009 / 1071, by this
+  // kernel's ranges 971 / 988 / 1418, this 968 / 969 / 973; 64 rows of 1500 413 / 415 (5120 / 32,768), 398 / 403, 396 / 396
+  t.ahead = t.rows ? std::min(t.columns, std::max(16u, 4096u / t.rows)) : 1;
+  const unsigned groups = t.rows && t.columns > t.ahead ? (t.rows + 15) / 16 : 0;
+  t.chunks = groups ? std::min((t.columns - t.ahead + kStageChunk - 1) / kStageChunk, std::max(8u, 512u / groups)) : 1;
+  r.rest = (t.rows * t.ahead + kStageWords - 1) / kStageWords;
+  r.start[0] = r.rest + groups * t.chunks;
+  for (int i = 0; i < r.n; ++i) r.start[i + 1] = r.start[i] + (r.words[i] + kStageWords - 1) / kStageWords;
   return true;
 }
 
-int launch_stage_rows(void* dst, const void* host, const StageRanges& r, hipStream_t st) {
-  unsigned most;
-  if (!stage_ok(dst, r, most) || (uintptr_t)host % 4) return -1;
-  if (most == 0) return 0;
-  stage_rows_kernel<<<dim3((most + 1023) / 1024, r.n), 256, 0, st>>>((unsigned*)dst, (const unsigned*)host, r);
+int launch_stage_rows(void* dst, const void* host, StageRanges r, hipStream_t st) {
+  if (!stage_cut(dst, r) || (uintptr_t)host % 4) return -1;
+  const unsigned grid = r.start[r.n];
+  if (grid == 0) return 0;
+  stage_rows_kernel<<<grid, 256, 0, st>>>((unsigned*)dst, (const unsigned*)host, r);
   return (int)hipGetLastError();
 }
 
-int launch_step_stage(void* dst, const void* host0, const void* host1, const StageRanges& r, const StepTokens& t, int* turn,
+int launch_step_stage(void* dst, const void* host0, const void* host1, StageRanges r, const StepTokens& t, int* turn,
                       hipStream_t st) {
-  unsigned most;
-  if (!stage_ok(dst, r, most) || (uintptr_t)host0 % 4 || (uintptr_t)host1 % 4 || t.B <= 0) return -1;
-  step_stage_kernel<<<dim3((std::max(most, (unsigned)t.B) + 1023) / 1024, r.n + 1), 256, 0, st>>>(
+  if (!stage_cut(dst, r) || (uintptr_t)host0 % 4 || (uintptr_t)host1 % 4 || t.B <= 0) return -1;
+  step_stage_kernel<<<(t.B + 255) / 256 + r.start[r.n], 256, 0, st>>>(
       (unsigned*)dst, (const unsigned*)host0, (const unsigned*)host1, r, t, turn);
   return (int)hipGetLastError();
 }

@@ -77,7 +77,7 @@ class DecodeRunner:
         B, MB = max_batch, max_blocks
         # ---- device buffers (persistent: graphs capture these addresses)
         n_i32 = 3 * B + B * MB + B + B
-        # one allocation, so that a step's staging is one copy
+        # one allocation, so that a step's staging is one launch
         self.stage = torch.zeros(16 * B + 4 * n_i32 + 8 * B, dtype=torch.uint8, device=dev)
         self.i64, self.i32, self.f32 = self._parts(self.stage, B)
         self.ids = self.i32[0:B]
@@ -153,9 +153,10 @@ class DecodeRunner:
             B, MB = self.max_batch, self.max_blocks
             i32, f32 = 16 * B, 16 * B + 4 * self.n_i32
             at = [(8 * B * j, 8 * Bb) for j in (0, 1)] + [(i32 + 4 * B * j, 4 * Bb) for j in range(4)]
-            at += [(i32 + 16 * B, 4 * Bb * MB), (i32 + 4 * B * (4 + MB), 4 * Bb)]
-            at += [(f32 + 4 * B * j, 4 * Bb) for j in (0, 1)]
-            r = self._stagings[Bb, k] = ops.StageRows(self.stage, self.h_stage[k], [(a, a + n) for a, n in at])
+            at += [(i32 + 4 * B * (4 + MB), 4 * Bb)] + [(f32 + 4 * B * j, 4 * Bb) for j in (0, 1)]
+            # of the block tables the blocks that the contexts have: at 1024 rows of up to 32,768 tokens whole rows are 4 MB
+            r = self._stagings[Bb, k] = ops.StageRows(self.stage, self.h_stage[k], [(a, a + n) for a, n in at],
+                                                      (i32 + 16 * B, Bb, MB, i32 + 8 * B, ops.KV_BLOCK))
         return r
 
     # ------------------------------------------------------------------

@@ -109,19 +109,26 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor | None = None,
 
 class StageRows:
     """``dst[a:b] = host[a:b]`` for the byte ranges (a, b), multiples of 4, of two uint8 buffers of one size, at every call.
+    ``table`` (at, rows, columns, lengths, per): of the 32-bit words [rows, columns] at byte ``at`` also, row r's first
+    ceil(length / per) at least, its length the r-th 32-bit word of ``host`` from byte ``lengths`` on.
     On the GPU ``host`` is pinned, and a kernel reads it: it stays unchanged until the stream is past it."""
 
-    def __init__(self, dst: torch.Tensor, host: torch.Tensor, ranges: list[tuple[int, int]]):
+    def __init__(self, dst: torch.Tensor, host: torch.Tensor, ranges: list[tuple[int, int]],
+                 table: tuple[int, int, int, int, int] | None = None):
         assert dst.shape == host.shape and dst.dtype == host.dtype == torch.uint8
         assert dst.is_contiguous() and host.is_contiguous()
-        assert all(0 <= a <= b <= dst.numel() and a % 4 == b % 4 == 0 for a, b in ranges)
-        self.dst, self.host, self.ranges = dst, host, ranges
+        at, rows, columns, lengths, per = table or (0, 0, 0, 0, 1)
+        whole, n = (at, at + 4 * rows * columns), dst.numel()
+        assert all(0 <= a <= b <= n and a % 4 == b % 4 == 0 for a, b in [*ranges, whole, (lengths, lengths + 4 * rows)])
+        assert rows >= 0 and columns >= 0 and per >= 1
+        self.dst, self.host, self.ranges = dst, host, [*ranges, whole]
         self.kernel = on_gpu(dst) and host.is_pinned()
         self.args = dst.data_ptr(), host.data_ptr(), [(a // 4, (b - a) // 4) for a, b in ranges]
+        self.table = at // 4, rows, columns, lengths // 4, per
 
     def __call__(self) -> None:
         if self.kernel:
-            check(hipk().stage_rows(*self.args, stream_ptr(self.dst)), "stage_rows")
+            check(hipk().stage_rows(*self.args, stream_ptr(self.dst), self.table), "stage_rows")
             return
         for a, b in self.ranges:
             self.dst[a:b].copy_(self.host[a:b])
@@ -133,12 +140,12 @@ def step_stage(stages: list[StageRows], ids: torch.Tensor, src: int, host: int, 
     its staging set, in one launch: the set is ``turn[0]``, which the launch gives to the other one (int32 [2], [1] 0)."""
     a, b = stages
     B, size = ids.numel(), a.dst.numel()
-    assert a.kernel and b.kernel and a.dst is b.dst and a.ranges == b.ranges and src % 8 == host % 4 == 0
-    assert 0 <= src <= size - 8 * B and 0 <= host <= size - 4 * B
+    assert a.kernel and b.kernel and a.dst is b.dst and a.ranges == b.ranges and a.table == b.table
+    assert src % 8 == host % 4 == 0 and 0 <= src <= size - 8 * B and 0 <= host <= size - 4 * B
     for t, dt, n in ((ids, torch.int32, B), (sampled, torch.int32, B), (counter, torch.int64, 1),
                      (position, torch.int64, 1), (turn, torch.int32, 2)):
         assert t.dtype == dt and t.is_contiguous() and t.numel() == n and t.is_cuda
-    check(hipk().step_stage(a.args[0], a.args[1], b.args[1], a.args[2], ids.data_ptr(), sampled.data_ptr(), src // 4,
+    check(hipk().step_stage(a.args[0], a.args[1], b.args[1], a.args[2], a.table, ids.data_ptr(), sampled.data_ptr(), src // 4,
                             host // 4, B, counter.data_ptr(), position.data_ptr(), turn.data_ptr(), stream_ptr(ids)),
           "step_stage")
 

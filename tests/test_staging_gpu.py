@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 import torch
 
+from drtc_amd import ops
 from drtc_amd.engine.decode_runner import DecodeRunner
 from drtc_amd.models import TINY_LLAMA, TransformerLM
 
@@ -38,3 +39,50 @@ def test_a_runner_that_goes_waits_for_its_steps(hipk):
     del r
     gc.collect()
     assert all(e.query() for e in events)
+
+
+@pytest.mark.parametrize("rows,columns,per", [(1, 1, 32), (1, 700, 32), (1, 40000, 1), (15, 64, 32), (17, 1100, 8), (300, 65, 32),
+                                              (1024, 16, 32), (1024, 600, 32), (1500, 130, 1), (9000, 200, 3)])
+def test_table_rows_by_their_lengths(hipk, rows, columns, per):
+    """Every word that a row's length asks for, none beyond the columns that go ahead of the lengths (4096 words of all
+    rows, 16 of each at least), nothing outside; lengths of 0, of whole blocks and past the table."""
+    rng = np.random.default_rng(rows)
+    need = rng.integers(0, columns + 1, rows)
+    need[::7] = rng.integers(0, min(columns, 20) + 1, len(need[::7]))
+    need[rows // 2] = columns
+    lengths = np.maximum(0, per * need - rng.integers(0, per, rows))
+    lengths[rows // 3] = per * columns + 5
+    need = np.minimum(-(-lengths // per), columns)
+    words = 3 + rows + 2 + rows * columns + 1  # gaps of words that stay
+    at_len, at_tab = 3, 3 + rows + 2
+    host = torch.zeros(4 * words, dtype=torch.uint8, pin_memory=True)
+    h = host.numpy().view(np.int32)
+    h[:] = rng.integers(1, 1 << 30, words)
+    h[at_len:at_len + rows] = lengths
+    dst = torch.full((4 * words,), 255, dtype=torch.uint8, device="cuda")
+    ops.StageRows(dst, host, [(0, 4), (8, 8)], (4 * at_tab, rows, columns, 4 * at_len, per))()
+    got = dst.cpu().numpy().view(np.int32)
+    table, want = got[at_tab:-1].reshape(rows, columns), h[at_tab:-1].reshape(rows, columns)
+    at, ahead = np.arange(columns), max(16, 4096 // rows)
+    assert ((table == want) | (at >= need[:, None])).all()
+    assert ((table == -1) | (at < np.maximum(need, ahead)[:, None])).all()
+    assert got[0] == h[0] and (got[1:at_tab] == -1).all() and got[-1] == -1
+    with pytest.raises(AssertionError):
+        ops.StageRows(dst, host, [], (4 * at_tab + 8, rows, columns, 4 * at_len, per))
+
+
+def test_a_step_reads_the_blocks_that_its_contexts_have(hipk):
+    """Of block tables as wide as long models' only the contexts' blocks cross the bus, with a graph and without; the tokens
+    are the narrow tables'."""
+    m = TransformerLM(TINY_LLAMA, "cuda", seed=3)
+    n = 1000
+    ids, blocks, tokens = np.arange(n) % 400, [[1 + i] for i in range(n)], []
+    for width, graphs in ((1, True), (1024, True), (1024, False)):
+        r = DecodeRunner(m, m.new_cache(n + 1, 4), 1024, width, use_graphs=graphs)
+        if graphs:
+            r.capture(r.bucket(n))
+        r.bt.fill_(7)
+        tokens.append(np.stack([r.wait(_launch(r, ids, np.full(n, at), blocks)) for at in range(3)]))
+        assert (r.bt[:n, :1].cpu().numpy() == blocks).all()
+        assert (r.bt[:, 16:] == 7).all()
+    assert all((t == tokens[0]).all() for t in tokens)
