@@ -450,6 +450,11 @@ def _aligned(x: torch.Tensor, w: torch.Tensor) -> bool:
     return x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
 
 
+def _staged(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """What kernels that load rows into LDS take: whole 16-byte pieces, 32-bit offsets of up to 256 rows."""
+    return _aligned(x, w) and x.stride(0) < 1 << 22
+
+
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """y = x @ w.T for x [M, K] (row stride ldx), w [N, K] contiguous."""
     if not _gpu_bf16(x, w):
@@ -466,8 +471,7 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         return y
     if kind == "skinny" and (arg != STREAM or _aligned(x, w)):
         return skinny_linear(x, w, arg)
-    # LDS-DMA: whole 16-byte pieces, 32-bit offsets of up to 256 rows
-    if kind in ("midm", "xd") and _aligned(x, w) and x.stride(0) < 1 << 22:
+    if kind in ("midm", "xd") and _staged(x, w):
         if kind == "xd":
             return xd_gemm(x, w, form=arg)
         return midm_gemm(x, w, "store", splits=arg % 100, nf=arg // 100 or 4)
@@ -1168,7 +1172,7 @@ def fused_glu_ok(x: torch.Tensor, w: torch.Tensor, act: str) -> bool:
     ones, or a tuned gated gemm_xd form)."""
     if w4_glu_ok(x, w, act) or _stream_glu_ok(x, w, act) and _aligned(x, w):
         return True
-    return (act in GATED and _gpu_bf16(x, w) and w.shape[1] == x.shape[1] and _aligned(x, w)
+    return (act in GATED and _gpu_bf16(x, w) and w.shape[1] == x.shape[1] and _staged(x, w)
             and glu_form(x.shape[0], w.shape[0], x.shape[1], x.shape[1], act) != 0)
 
 
@@ -1232,7 +1236,7 @@ def squared_relu(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.T
         kind, form = route(M, w.shape[0], K, x.stride(0))
         if (kind, form) == ("skinny", STREAM):
             return stream_gemm(x, w, "relu2", out=out)
-        if kind == "xd":
+        if kind == "xd" and _staged(x, w):
             return xd_gemm(x, w, "relu2", out=out, form=form)
         if kind == "skinny" and out.dtype == x.dtype:
             N = w.shape[0]

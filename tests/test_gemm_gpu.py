@@ -184,6 +184,18 @@ def test_linear_takes_rows_at_any_address(hipk, M, N, K, kind):
         assert _rel(G.linear(x, w), x.float() @ w.float().t()) < 1e-2
 
 
+@pytest.mark.parametrize("M,N,K", [(256, 25600, 4096), (257, 2048, 5632)])
+def test_squared_relu_takes_rows_far_apart(hipk, M, N, K):
+    """Rows too far apart for 32-bit offsets of 256 of them, at sizes that the rules send to gemm_xd."""
+    assert G.route(M, N, K, 1 << 22)[0] == "xd"
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+    w = (torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).to(torch.bfloat16)
+    far = torch.empty((M - 1 << 22) + K, dtype=torch.bfloat16, device="cuda").as_strided((M, K), (1 << 22, 1)).copy_(x)
+    out = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    assert _rel(G.squared_relu(far, w, out), (x.float() @ w.float().t()).relu().square()) < 1e-2
+
+
 @pytest.mark.parametrize("M,splits", [(33, 1), (200, 4)])
 def test_midm_takes_operands_at_any_address(hipk, M, splits):
     """Input and weights off 16 bytes, residual and output (also in place) off 8, and rows too far apart for 32-bit offsets."""

@@ -1,8 +1,10 @@
 """CPU checks of the decode-GEMM router's gemm_xd forms and of the in-tree tuning table
 (ops/gemm.py; no GPU work: forms are parsed and shape-checked on the host)."""
 import json
+import types
 
 import pytest
+import torch
 
 from drtc_amd.ops import gemm as G
 
@@ -145,3 +147,23 @@ def test_gemma_2048_decode_shapes_carry_a_gemm_xd_form():
             assert e.get("prefill") and e["xd"] == want
             M, N, K, _ = (int(v) for v in k.split(","))
             assert G.xd_supported(M, N, K, want)
+
+
+@pytest.mark.parametrize("op,M,N,K", [("squared_relu", 256, 25600, 4096), ("gated", 513, 14336, 2048), ("gated", 160, 25600, 2048)])
+@pytest.mark.parametrize("stride", [1 << 22, 4104])
+def test_rows_far_apart_stay_with_the_library(monkeypatch, op, M, N, K, stride):
+    """gemm_xd's tiles of 256 rows have 32-bit offsets; the products with something behind them keep ``linear``'s bound."""
+    monkeypatch.setattr(G, "on_gpu", lambda t: True)
+    monkeypatch.setattr(G, "_activate", lambda: {})
+    monkeypatch.setattr(G, "_prefill_algo", lambda *a: -1)
+    monkeypatch.setattr(G, "_routes", {})
+    monkeypatch.setattr(G, "hipk", lambda: types.SimpleNamespace(relu2=lambda *a: 0))
+    monkeypatch.setattr(G, "stream_ptr", lambda t: 0)
+    monkeypatch.setattr("drtc_amd.ops.activation.act_glu", lambda y, act, limit=0.0: y)
+    taken = []
+    monkeypatch.setattr(G, "xd_gemm", lambda *a, **k: taken.append("xd"))
+    monkeypatch.setattr(G.F, "linear", lambda x, w: taken.append("library") or torch.empty(1, dtype=x.dtype))
+    x = torch.empty((M - 1) * stride + K, dtype=torch.bfloat16).as_strided((M, K), (stride, 1))
+    w = torch.empty(N, K, dtype=torch.bfloat16)
+    G.squared_relu(x, w, torch.empty(M, N, dtype=torch.bfloat16)) if op == "squared_relu" else G.gated(x, w)
+    assert taken == ["library" if stride == 1 << 22 else "xd"]
