@@ -442,7 +442,7 @@ def route(M: int, N: int, K: int, ldx: int) -> tuple[str, int]:
 
 
 def _gpu_bf16(x: torch.Tensor, w: torch.Tensor) -> bool:
-    return (on_gpu(x) and _enabled and x.dim() == 2 and x.dtype == torch.bfloat16
+    return (on_gpu(x) and _enabled and x.dim() == w.dim() == 2 and x.dtype == torch.bfloat16
             and w.dtype == torch.bfloat16 and x.stride(1) == 1 and w.is_contiguous())
 
 
@@ -457,7 +457,7 @@ def _staged(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """y = x @ w.T for x [M, K] (row stride ldx), w [N, K] contiguous."""
-    if not _gpu_bf16(x, w):
+    if not _gpu_bf16(x, w) or w.shape[1] != x.shape[1]:  # (refuses widths that differ)
         return F.linear(x, w)
     M, K = x.shape
     N = w.shape[0]
@@ -525,7 +525,8 @@ def linear_beside(x: torch.Tensor, w: torch.Tensor, x2: torch.Tensor, w2: torch.
                   relu2: bool = False) -> tuple[torch.Tensor, torch.Tensor]:
     """``linear(x, w)``, and ``linear(x2, w2)`` or (``relu2``, into ``out2``) ``squared_relu``: in one launch where both are
     products of the same K that the skinny kernels take (gemv.hip SkinnyBeside), by the first's choice of them."""
-    if _gpu_bf16(x, w) and _gpu_bf16(x2, w2) and x.shape == x2.shape and x.shape[0] <= SKINNY_MAX_M:
+    if (_gpu_bf16(x, w) and _gpu_bf16(x2, w2) and x.shape == x2.shape and x.shape[0] <= SKINNY_MAX_M
+            and w.shape[1] == w2.shape[1] == x.shape[1]):
         (M, K), N, N2 = x.shape, w.shape[0], w2.shape[0]
         v, v2 = _choice(M, N, K, x.stride(0)), _choice(M, N2, K, x2.stride(0))
         if v in DUAL and v2 in DUAL and (v == v2 or v != 1 != v2) and skinny_supports(v, M, N2, K, x2.stride(0)) and (
@@ -1232,7 +1233,7 @@ def squared_relu(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.T
     if w4_ok(x, w) and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0:
         return mfma_gemm(x, w, "relu2", out=out, variant=_w4v(K),
                          group_m=w4_group_m(M, w.shape[0], K))
-    if _gpu_bf16(x, w) and _aligned(x, w) and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0:
+    if _gpu_bf16(x, w) and w.shape[1] == K and _aligned(x, w) and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0:
         kind, form = route(M, w.shape[0], K, x.stride(0))
         if (kind, form) == ("skinny", STREAM):
             return stream_gemm(x, w, "relu2", out=out)

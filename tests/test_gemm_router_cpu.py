@@ -167,3 +167,25 @@ def test_rows_far_apart_stay_with_the_library(monkeypatch, op, M, N, K, stride):
     w = torch.empty(N, K, dtype=torch.bfloat16)
     G.squared_relu(x, w, torch.empty(M, N, dtype=torch.bfloat16)) if op == "squared_relu" else G.gated(x, w)
     assert taken == ["library" if stride == 1 << 22 else "xd"]
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 2048, 4096), (16, 2048, 4096), (300, 2048, 5632), (256, 6656, 2048), (129, 25600, 2048)])
+@pytest.mark.parametrize("less", [64, -64])
+def test_widths_that_differ_are_refused(monkeypatch, M, N, K, less):
+    """Ahead of every kernel, which would take the rows of W for K apart and K long."""
+    monkeypatch.setattr(G, "on_gpu", lambda t: True)
+    monkeypatch.setattr(G, "_activate", lambda: {})
+    monkeypatch.setattr(G, "_prefill_algo", lambda *a: -1)
+    monkeypatch.setattr(G, "_routes", {})
+    monkeypatch.setattr(G, "hipk", lambda: pytest.fail("a kernel took it"))
+    monkeypatch.setattr(G, "stream_ptr", lambda t: 0)
+    x, w, wrong = (torch.empty(n, k, dtype=torch.bfloat16) for n, k in ((M, K), (N, K), (N, K - less)))
+    out = torch.empty(M, N, dtype=torch.bfloat16)
+    for call in (lambda: G.linear(x, wrong), lambda: G.squared_relu(x, wrong, out), lambda: G.linear_parts(x, wrong),
+                 lambda: G.linear_beside(x, wrong, x, wrong)):
+        with pytest.raises(RuntimeError, match="shapes cannot be multiplied"):
+            call()
+    if M <= 16:
+        monkeypatch.setattr(G, "hipk", lambda: types.SimpleNamespace(skinny_gemm=lambda *a: 0 if a[15] == 0 else pytest.fail("both")))
+        with pytest.raises(RuntimeError, match="shapes cannot be multiplied"):
+            G.linear_beside(x, w, x, wrong)
