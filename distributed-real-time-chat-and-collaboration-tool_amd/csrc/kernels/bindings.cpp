@@ -121,15 +121,16 @@ PYBIND11_MODULE(_hipk, m) {
                                 variant - 7, limit, S(st));
   });
   // gemm_w4 grouped persistent form (ops.gemm.mfma_gemm_grouped): per-group weights, device
-  // row offsets
+  // row offsets; aidx: as launch_gemm_w4_grouped's
   m.def("gemm_grouped", [](u64 c, u64 a, u64 b, u64 grp, int n_grp, int max_rows, int N, int K,
                            int lda, int ldb, int ldc, int64_t b_grp, int epi, int up_off,
-                           int group_m, int ksplit, int64_t c_split, float limit, u64 st) {
+                           int group_m, int ksplit, int64_t c_split, float limit, u64 st, u64 aidx, int a_rows) {
     return drtc::launch_gemm_w4_grouped(P<void>(c), P<const void>(a), P<const void>(b),
                                         P<const int>(grp), n_grp, max_rows, N, K, lda, ldb, ldc,
                                         b_grp, epi, up_off, group_m, ksplit, c_split, limit,
-                                        nullptr, 0, S(st));
-  });
+                                        P<const int>(aidx), a_rows, S(st));
+  }, py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(),
+     py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg() = 0, py::arg() = 0);
   // gemm_xd (ops.gemm.xd_gemm): decode-shaped tiles, XCD-partitioned order, split-K 1..8
   m.def("gemm_xd", [](u64 c, u64 a, u64 b, u64 r, int M, int N, int K, int lda, int ldb, int ldc,
                       int ldr, int epi, int mt, int nf, int splitk, u64 slab, int64_t slab_bytes,

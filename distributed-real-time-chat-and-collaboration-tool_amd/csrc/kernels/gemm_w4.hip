@@ -1067,8 +1067,9 @@ int launch_gemm_w4_grouped(void* c, const void* a, const void* b, const int* grp
                            int epi, int up_off, int group_m, int ksplit, int64_t c_split,
                            float limit, const int* aidx, int a_rows, hipStream_t st) {
   const bool glu = epi == W4_SILU || epi == W4_GELU || epi == W4_CLAMP;
-  // (three K tiles: the first one's wait covers the indexes, the last two's loads use them)
-  if (aidx != nullptr && (epi == W4_STORE || K < 192 || a_rows < 1 || (int64_t)a_rows * lda * 2 >= (1ll << 31)))
+  // Four K tiles: the last two's loads use the indexes, which the second one's wait is the first to cover.  (The first
+  // one's, behind a full tile, leaves that tile's stores and the indexes asked for behind them under way.)
+  if (aidx != nullptr && (epi == W4_STORE || K < 256 || a_rows < 1 || (int64_t)a_rows * lda * 2 >= (1ll << 31)))
     return -1;
   if (epi != W4_STORE && epi != W4_RELU2 && !glu) return -1;
   if (ksplit < 1 || (epi != W4_STORE && ksplit != 1)) return -1;  // an activation cannot be split

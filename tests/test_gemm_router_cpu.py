@@ -189,3 +189,13 @@ def test_widths_that_differ_are_refused(monkeypatch, M, N, K, less):
         monkeypatch.setattr(G, "hipk", lambda: types.SimpleNamespace(skinny_gemm=lambda *a: 0 if a[15] == 0 else pytest.fail("both")))
         with pytest.raises(RuntimeError, match="shapes cannot be multiplied"):
             G.linear_beside(x, w, x, wrong)
+
+
+@pytest.mark.parametrize("K", [128, 192])
+def test_rows_by_a_list_want_four_k_tiles(K):
+    """Fewer, and a tile's row indexes would be read ahead of the first wait that covers them.  (Refused on the host.)"""
+    from drtc_amd.ops._ext import hipk
+
+    N, rows, p = 512, 600, 1 << 20
+    args = (p, p, p, p, 2, rows, N, K, K, K, N, 2 * N * K, G.EPI["silu"], N, 4, 1, 0, 0.0, 0, p, rows)
+    assert hipk().gemm_grouped(*args) == -1
