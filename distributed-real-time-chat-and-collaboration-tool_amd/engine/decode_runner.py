@@ -277,7 +277,7 @@ class DecodeRunner:
         g = self._graphs.get(Bb)
         if g is None:
             self._staging(Bb, k)()
-        elif self._turn != k:  # a step without a graph came between
+        elif self._turn != k:  # this set's turn was passed over: its launch raised, or ran without a graph
             self.turn[:1].fill_(k)
         timing = nb and self.time_gpu
         if timing:

@@ -86,3 +86,25 @@ def test_a_step_reads_the_blocks_that_its_contexts_have(hipk):
         assert (r.bt[:n, :1].cpu().numpy() == blocks).all()
         assert (r.bt[:, 16:] == 7).all()
     assert all((t == tokens[0]).all() for t in tokens)
+
+
+@pytest.mark.parametrize("between", ["raised", "eager"])
+def test_a_turn_passed_over(hipk, between):
+    """Between steps of a graph a launch that raises with its set chosen, or a step without a graph: the next replay reads
+    its own set, not the other one's positions, slots and tokens."""
+    tokens = []
+    for passed in (False, True):
+        r, got = _runner(), []
+        for at in range(6):
+            if passed and at in (2, 3):
+                if between == "raised":
+                    with pytest.raises(ValueError):
+                        r.launch(1, np.array([9], np.int32), np.zeros(3, np.int32), *[None] * 6)
+                else:
+                    graphs, r._graphs, r.use_graphs = r._graphs, {}, False
+            got.append(r.wait(_launch(r, [5 + at], [at], [[1]])).tolist())
+            assert int(r.positions[0]) == at and int(r.slots[0]) == 32 + at
+            if not r.use_graphs:
+                r._graphs, r.use_graphs = graphs, True
+        tokens.append(got)
+    assert tokens[0] == tokens[1]
