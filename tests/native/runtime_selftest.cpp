@@ -1,6 +1,5 @@
 // Host-side self-test of the native CPU runtime (csrc/runtime), built with
-// -fsanitize=address,undefined by tests/test_native_sanitizers.py (SURVEY §5
-// "Race detection / sanitizers": ASan/UBSan builds for the C++ extensions).
+// -fsanitize=address,undefined by tests/test_native_sanitizers.py.
 //
 //  * bcrypt: hashes of random passwords/salts equal libxcrypt's crypt_rn()
 //    output (costs 4-5, $2a$ and $2b$, 0..80-byte passwords incl. the

@@ -284,7 +284,7 @@ def test_cli_send_checks_channel_and_history_auto_logout(cluster):
 
 def test_per_feature_llm_routing(tmp_path):
     """Each AI RPC goes to its feature's LLM service (NodeConfig.llm_smart / llm_summary /
-    llm_ask / llm_suggest): one node serving the per-feature model matrix of BASELINE.json."""
+    llm_ask / llm_suggest): one node serving a model to each feature."""
     backends = {f: ScriptedBackend() for f in ("smart", "summary", "ask", "suggest")}
     ports = {f: free_port() for f in backends}
     servers = [serve_llm(b, port=ports[f], bind="127.0.0.1") for f, b in backends.items()]

@@ -692,7 +692,7 @@ def test_splitk_watch_reports_a_fault_without_a_sync(hipk):
 
 def test_hbm_budget_too_small_for_one_sequence_is_an_error(hipk):
     """An engine group whose HBM budget cannot hold its weights plus one max_model_len sequence
-    of KV cache fails at start with the numbers, instead of starting with 2 blocks (ADVICE r5)."""
+    of KV cache fails at start with the numbers, instead of starting with 2 blocks."""
     from drtc_amd.engine import LLMEngine
     from drtc_amd.models import LLAMA3_8B, TransformerLM
 

@@ -326,7 +326,7 @@ def test_replica_pool_evicts_dead_replica_and_respawns():
 
 def test_fit_prompt_keeps_instruction_head_and_tail():
     """Over-long prompts lose their oldest conversation lines, never the
-    summarize instruction (VERDICT r1 weak #10)."""
+    summarize instruction."""
     from drtc_amd.engine import ChatTokenizer
     from drtc_amd.llm.prompts import ChatLine, fit_prompt, summarize_prompt
 
@@ -402,8 +402,8 @@ def test_pool_router_timeout_aborts_on_the_replica():
 
 
 def test_default_engine_batch_per_model():
-    """Without --max-batch the LLM server sizes the engine batch per model from the
-    BASELINE measurements that stay inside the reference's deadlines."""
+    """Without --max-batch the LLM server sizes the engine batch per model from
+    measurements that stay inside the reference's deadlines."""
     from drtc_amd.llm.server import default_max_batch
 
     assert default_max_batch("llama-3-8b") == 1024
@@ -507,7 +507,7 @@ def test_serve_placement_needs_budgets_on_shared_gpus():
 def test_serve_group_without_gpus_is_placed_where_it_is_built(monkeypatch):
     """A tp1 --serve group without @GPUS runs on GPU 0 (one replica): the placement check and
     the build use that same rule, so it does not collide with groups on the other GPUs of a
-    --gpus 8 server (ADVICE r5)."""
+    --gpus 8 server."""
     import argparse
 
     from drtc_amd.llm import server as S

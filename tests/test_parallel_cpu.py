@@ -140,7 +140,7 @@ def _tp_worker(rank, world, port, q):
 def _tp_engine_worker(rank, world, port, q):
     """TP=2 engines whose ranks see different free memory: the block count is
     agreed (MIN over the group), so the lockstep schedulers admit and preempt
-    identically and produce the same tokens (engine.py:71)."""
+    identically and produce the same tokens."""
     sys.path.insert(0, ROOT)
     os.environ.update(MASTER_ADDR="127.0.0.1", MASTER_PORT=str(port))
     dist.init_process_group("gloo", rank=rank, world_size=world)

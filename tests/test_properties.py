@@ -1,4 +1,4 @@
-"""Property-based tests (hypothesis; SURVEY.md §4.2 unit-test plan): random
+"""Property-based tests (hypothesis): random
 fault schedules against the Raft safety invariants, random command streams
 against the replicated chat state machine, and the parsers / prompt fitting /
 JWT / block allocator over arbitrary inputs.  CPU only."""

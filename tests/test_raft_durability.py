@@ -1,4 +1,4 @@
-"""Raft wire/disk interoperability and crash safety (VERDICT r1 items 3, 5, 7).
+"""Raft wire/disk interoperability and crash safety.
 
 * The exported reference-format pair (raft_log_port_*.pkl + raft_state_port_*.pkl)
   replays, with the reference's apply semantics (ref server/raft_node.py:1196-1397,

@@ -1,4 +1,4 @@
-"""Product shutdown without aborts (VERDICT r5 item 5).
+"""Product shutdown without aborts.
 
 SIGTERM to the deployed processes must end them in order and with exit code 0 within 10 s,
 with no "terminate called" abort from a thread left inside native code at interpreter exit:
