@@ -645,9 +645,10 @@ DRTC_DEVICE void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier
 
 // Four heads of 128 and sequences of some length: the scores of the next tile are computed between the exponentials and
 // the outputs of this one.  What bounds a wave above is that its matrix instructions and its softmax follow one
-// another, and the barrier of each tile keeps the two waves of a SIMD in step.  (Matrix cores busy 42.6 -> 48 %, cycles
-// 660,000 -> 588,000 at 4 x 4000 tokens of 16 heads; the clock falls from 2.2 to 2.05 GHz, power bounds the rest.)
-// us, above / this: 4 x 4000 of 16 heads over 4 281 / 274, 4 x 3000 of 32 over 8 324 / 316, one of 700 26.4 / 25.7, of 2000
+// another, and the barrier of each tile keeps the two waves of a SIMD in step.  (4 x 4000 tokens of
+// 16 heads over 4: 633,000 -> 587,000 cycles, matrix cores busy 41 -> 44 % of them, waits for an instruction to issue
+// 104 -> 77 M of 288 -> 268 M wave cycles; the clock 2.16 -> 2.10 GHz.)
+// us, above / this: 4 x 4000 of 16 heads over 4 293 / 280, 4 x 3000 of 32 over 8 324 / 316, one of 700 26.4 / 25.7, of 2000
 // 64 / 58 (above without its pinned reads).  Few tiles do not pay for the first one's scores by themselves (one of 256
 // 14.2 / 14.7, 16 x 512 90 / 94), two heads not for the registers (8 x 2000 180 / 258), persistent workgroups not for
 // theirs (8 x 1000 50.3 / 52.3, 16 x 512 of 32 82.5 / 85.4): the caller picks by the longest sequence.  Every sum is the

@@ -1315,8 +1315,8 @@ int launch_moe(void* out, const void* x, const void* router_logits, const void* 
   }
   if (variant == 4) {
     // gate_up reads the token rows through the list: a pass of copying them in expert order first took 119 us a layer of
-    // 12,160 tokens of 4096, two experts each (pass of three layers 14.59 -> 14.31 ms), 144 us of 15,000 with two
-    // of 16 (20.84 -> 20.34 ms).  Still copied, into zbuf, which gate_up has consumed before down writes Z: tokens past a
+    // 12,160 tokens of 4096, four of 16 experts each (a prompt step of four layers, three of them of all rows, 14.59 -> 14.31 ms),
+    // 144 us of 15,000, four of 20 (20.84 -> 20.34 ms).  Still copied, into zbuf, which gate_up has consumed before down writes Z: tokens past a
     // descriptor's 2 GiB or off 16 bytes.
     const bool listed = (int64_t)T * H * 2 < (1ll << 31) && (uintptr_t)x % 16 == 0;
     if (!listed)

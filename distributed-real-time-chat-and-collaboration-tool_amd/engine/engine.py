@@ -50,9 +50,9 @@ def _check_sampled(toks: np.ndarray) -> None:
 
 
 def _pad_tokens(T: int) -> int:
-    """Prefill token-count bucket.  Padding rows cost what others do, and in a mixture they all go to the same experts
-    (four layers of 16 experts of 4096 x 3584, 266 rows: as 512 2100 us, as 288 1400; 2048 x 1792, 3676 rows as 3840 2233, as
-    3712 2114), so a bucket is a sixteenth of the count wide, an eighth at most."""
+    """Prefill token-count bucket: 32 rows wide up to 1024 tokens, above at most a sixteenth of the count, 256.  Padding rows
+    cost what others do, and in a mixture they all go to the same experts (four layers of 16 experts of 4096 x 3584, 266 rows:
+    as 512 2100 us, as 288 1400; 2048 x 1792, 3676 rows as 3840 2233, as 3712 2114)."""
     step = 32 if T <= 1024 else 64 if T <= 2048 else 128 if T <= 4096 else 256
     return -(-T // step) * step
 

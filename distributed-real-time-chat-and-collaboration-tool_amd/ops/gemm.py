@@ -1157,7 +1157,7 @@ def _glu_default(M: int, I: int, K: int, act: str = "silu") -> int:
     if not form or not xd_supported(M, I, K, form, True):
         return 0
     mt, nf, _ = xd_form(form)
-    if -(-M // (128 * mt)) * (I // (16 * nf)) < (112 if K <= 2048 else 160):
+    if -(-M // XD_ROWS[mt]) * (I // (16 * nf)) < (112 if K <= 2048 else 160):
         return 0
     return form + 1000 if xd_nt_ok(M, form) else form
 
@@ -1289,8 +1289,9 @@ def xd_supported(M: int, N: int, K: int, form: int, glu: bool = False) -> bool:
     if not (M >= 1 and N % tno == 0 and K % 64 == 0 and K // 64 // sk > XD_TILES[(mt, nf)]):
         return False
     # split-K: the partial slots and tile counters fit the device workspace
-    tiles = -(-M // (128 * max(mt, 1))) * (N // tno)
-    return sk == 1 or (tiles * sk * (128 * mt) * (32 * nf) * 4 <= WS_SLAB_BYTES
+    rows = XD_ROWS[mt]
+    tiles = -(-M // rows) * (N // tno)
+    return sk == 1 or (tiles * sk * rows * (32 * nf) * 4 <= WS_SLAB_BYTES
                        and 2 * tiles + 2 <= WS_COUNTERS)  # + the fault word (last counter)
 
 
@@ -1304,11 +1305,11 @@ def xd_default_form(M: int, N: int, K: int, glu: bool = False) -> int:
         if not xd_supported(M, N, K, form, glu):
             continue
         mt, nf, sk = xd_form(form)
-        tno = 16 * nf if glu else 32 * nf
-        items = -(-M // (128 * mt)) * (N // tno) * sk
+        tno, rows = 16 * nf if glu else 32 * nf, XD_ROWS[mt]
+        items = -(-M // rows) * (N // tno) * sk
         rounds = -(-items // 256)
-        c = rounds * ((128 * mt + 32 * nf) * (K // sk) * 2 + 100_000
-                      + 5 * (sk - 1) * (128 * mt) * (32 * nf) * 4)
+        c = rounds * ((rows + 32 * nf) * (K // sk) * 2 + 100_000
+                      + 5 * (sk - 1) * rows * (32 * nf) * 4)
         if cost is None or c < cost:
             best, cost = form, c
     return best
@@ -1318,9 +1319,10 @@ def xd_gemm(x: torch.Tensor, w: torch.Tensor, epi: str = "store",
             residual: torch.Tensor | None = None, out: torch.Tensor | None = None,
             form: int = 0, ws: tuple[torch.Tensor, torch.Tensor] | None = None,
             limit: float = 0.0) -> torch.Tensor:
-    """Decode-shaped hand GEMM, csrc/kernels/gemm_xd.hip: y = epi(x @ w.T) on 128 mt x 32 nf
-    tiles, K split over 1..8 slices, with the tile order partitioned by XCD (each XCD streams
-    its own weight column panels through its L2 for every row tile); mt 0: 64 rows, plain, one slice.  epi "store";
+    """Decode-shaped hand GEMM, csrc/kernels/gemm_xd.hip: y = epi(x @ w.T) on tiles of XD_ROWS[mt] rows x 32 nf
+    columns, K split over 1..8 slices, with the tile order partitioned by XCD (each XCD streams
+    its own weight column panels through its L2 for every row tile).  mt 0 (64 rows): plain, one slice; mt 3 to 5 (160, 192
+    and 224 rows): one row tile, one slice, non-temporal weight loads.  epi "store";
     "residual" (``out`` may be ``residual``); "silu" / "gelu_tanh": w is the fused [gate; up]
     weight [2I, K] and y[:, n] = act(x . gate_n) * (x . up_n); "clamped": bounded by ``limit``
     (tiles of XD_CLAMP_NF); "relu2": relu(x @ w.T)^2.  ``form`` = mt * 100 + nf * 10 + splitk (+ 1000: non-temporal weight loads; 0: ``xd_default_form``)."""
