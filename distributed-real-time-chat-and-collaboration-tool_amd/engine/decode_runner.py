@@ -55,11 +55,14 @@ def _retire(events: list, buffers: tuple) -> None:
     _retired.append((events, buffers))
     if torch.cuda.is_initialized() and torch.cuda.is_current_stream_capturing():
         return  # nothing may be waited for: the next runner to go does
-    while _retired:
-        for e in _retired[-1][0]:
+    while True:
+        try:
+            last = _retired.pop()  # (held here until its steps are over; runners may go in several threads at once)
+        except IndexError:
+            return
+        for e in last[0]:
             if e is not None:
                 e.synchronize()
-        _retired.pop()
 
 
 class DecodeRunner:

@@ -68,3 +68,31 @@ def test_pinned_buffers_outlive_the_steps_of_a_runner(monkeypatch, recording):
         gc.collect()
     assert seen == [True] * (4 if recording else 2) and not decode_runner._retired
     assert all(b() is None for b in buffers)
+
+
+def test_runners_that_go_while_another_is_waited_for():
+    """As from another thread, or the collector during the wait: each one's buffers until its own steps are over."""
+    from drtc_amd.engine import decode_runner
+
+    class Buffer:
+        pass
+
+    order, buffers = [], [Buffer(), Buffer()]
+    alive = [weakref.ref(b) for b in buffers]
+
+    class Event:
+        def __init__(self, i, nested=None):
+            self.i, self.nested = i, nested
+
+        def synchronize(self):
+            if self.nested:
+                nested, self.nested = self.nested, None
+                decode_runner._retire(*nested)
+            order.append((self.i, alive[self.i]() is not None))
+
+    held = (buffers.pop(),)
+    decode_runner._retire([Event(0, ([Event(1)], held))], (buffers.pop(),))
+    assert order == [(1, True), (0, True)] and alive[0]() is None and not decode_runner._retired
+    del held
+    gc.collect()
+    assert alive[1]() is None
