@@ -389,14 +389,22 @@ def full_form(M: int, N: int, K: int) -> int:
     of 203 below 0.97; K to 1536, 128 .. 199 1.27; longer K and fewer 1.06, a third below 0.97.  us: 6656 x 2048, 256 rows 24.7 /
     16.9, 448 24.4 / 19.9, 1024 31.1 / 29.6; 12800 x 4096, 256 49.4 / 42.8; 3072 x 2048, 1088 23.6 / 19.1; past 3072 rows 3072 x 2048,
     3360 37.7 / 39.9, 1024 x 3072, 4064 28.3 / 33.0.  The table's library solutions of short K as well: 4096 x 512, 256 rows 8.2 /
-    5.5, 1024 9.7 / 8.6."""
+    5.5, 1024 9.7 / 8.6.
+    Longer K, over 28,000 sizes of 30 widths: 5120 .. 7168 1.09, longer 1.08; left to the library where a class of them loses:
+    K above 7168 with less than three quarters of the tiles' rows used, but in 64 columns (0.87 in tiles of 256 x 128, 0.96 of 128 x 128; 12800
+    x 12800, 261 rows 130.8 / 183.8, of 300 rows at K 7168 1.01, from 385 rows on 1.13), tiles of 256 x 192 with less than four
+    fifths (0.93 .. 1.02), 64 columns past 2048 rows (K to 5120 0.98, longer 0.95 .. 0.84)."""
     if not (129 <= M <= 3072 and _xd_enabled and _enabled):
         return 0
     for form in (121, 141, 161, 241, 261):
         mt, nf, _ = xd_form(form)
-        items = -(-M // XD_ROWS[mt]) * (N // (32 * nf))
+        rows = -(-M // XD_ROWS[mt])
+        items = rows * (N // (32 * nf))
         if items <= 256 and xd_supported(M, N, K, form):
             if items < (128 if K <= 1536 else 200):
+                return 0
+            used = M / (rows * XD_ROWS[mt])
+            if K > 7168 and nf > 2 and used < 0.75 or K > 1536 and form == 261 and used < 0.8 or K > 3072 and nf == 2 and M > 2048:
                 return 0
             return form + 1000 if _xd_nt and xd_nt_ok(M, form) else form
     return 0

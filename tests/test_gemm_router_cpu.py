@@ -56,6 +56,10 @@ def test_deep_products_rule(monkeypatch, N, K):
     (256, 25600, 4096, 1241),                   # one row tile: weights past the caches
     (129, 4096, 512, 121), (1024, 4096, 512, 141), (192, 8192, 512, 121),
     (640, 6656, 2048, 0), (128, 12800, 4096, 0), (3073, 3072, 2048, 0), (300, 6640, 2048, 0), (256, 4096, 256, 0),
+    (261, 12800, 12800, 0), (383, 12800, 7232, 0), (384, 12800, 7232, 241), (261, 12800, 7168, 241),  # rows of the tiles used
+    (160, 6656, 12288, 121), (161, 14336, 8192, 0), (192, 14336, 8192, 141),
+    (614, 13824, 4096, 0), (615, 13824, 4096, 261), (520, 13824, 1536, 261),
+    (2049, 768, 8192, 0), (2049, 768, 3072, 121), (1100, 1536, 8192, 121),  # tiles of 64 columns
 ])
 def test_full_round_rule(monkeypatch, M, N, K, want):
     monkeypatch.setattr(G, "_xd_nt", True)
