@@ -1102,14 +1102,53 @@ static double moe_xd_us(int E, double rows, int bm, int H, int I, bool glu) {
   const bool split = bm == 256 && rows < kMoeW4Rows && tiles * H <= 32768;  // down in two K slices (launch_moe)
   return up * (per * H + 3) + down * (split ? per * I / 2 + 20 : per * I + 3);
 }
+// The same of a layer as a fit of 11,990 sizes (widths 512 .. 6144 and 512 .. 14336, 4 .. 128 experts, 96 .. 800 rows in the mean,
+// half of them within 7 %): a round costs by itself and its tiles by their number, so that a last round of few tiles is not a
+// whole one; the number of tiles spreads as the choice of experts does; the weights' bytes bound all from below.  bm 128:
+// moe_half_tiles; 256: gemm_w4 from a tile per expert on, gemm_xd's 256 x 256 tiles below it.
+static double moe_fit_us(int E, double rows, int bm, int H, int I, bool glu) {
+  struct Fit {
+    double round_k, tiles_k, round, layer, tbs, pairs, spread;
+  };
+  const Fit f = rows < kMoeW4Rows ? (bm == 128 ? Fit{0.0081, 0.0044, 12.7, 3.1, 4.13, 1.82, 0.06} : Fit{0.0137, 0.0087, 19.3, -2.2, 1e6, 1.89, 0.06})
+                                  : (bm == 128 ? Fit{0.0056, 0.0068, 10.4, 9.0, 3.06, 0.80, 0.06} : Fit{0.0040, 0.0166, 14.5, 14.5, 3.71, 1.36, 0.01});
+  const auto ramp = [](double x) { return std::min(1., std::max(0., 0.5 + x / 4)); };  // of a value x spreads above a bound
+  double tiles = E, var = 0;
+  const double sd = std::max(1., sqrt(rows * (1. - 1. / E)));
+  for (int at = bm;; at += bm) {
+    const double p = ramp((rows - at) / sd);
+    if (p <= 0) break;
+    tiles += E * p;
+    var += E * p * (1 - p);
+  }
+  const int up = glu ? 2 * I : I;
+  double us = 0;
+  for (const auto& [cols, k] : {std::pair<double, double>{up, H}, {H, I}}) {
+    const double x = tiles * cols / 65536, w = sqrt(var * cols / 65536 * cols / 65536 + f.spread * f.spread);
+    double rounds = 1;
+    for (int m = 1;; ++m) {
+      const double p = ramp((x - m) / w);
+      if (p <= 0) break;
+      rounds += p;
+    }
+    us += rounds * (f.round_k * k + f.round) + x * f.tiles_k * k;
+  }
+  const double bytes = 2e-6 * E * (double)H * (up + I) / f.tbs;
+  return f.layer + f.pairs * 1e-6 * E * rows * H + sqrt(sqrt(us * us * us * us + bytes * bytes * bytes * bytes));
+}
 // Whether tiles of 128 rows are the faster ones: fewer rows of padding, or a round less.  us of a layer, 256 rows (variant
 // 3 or 4) / 128: 20 x 2048 x 1792, squared relu, 640 tokens 150 / 102, 1536 222 / 156, 896 127 / 148; 20 x 4096 x 3584, 640 tokens
-// 385 / 313, 1536 556 / 495; 16 x 4096 x 3584, gated, 640 tokens 337 / 388, 1152 572 / 550, 1536 633 / 651.  whole: gemm_xd
+// 385 / 313, 1536 556 / 495; 16 x 4096 x 3584, gated, 640 tokens 337 / 388, 1152 572 / 550, 1536 633 / 651.  Both estimates must say
+// so, the second nearly, or with a tenth to spare for many experts or long rows: of 11,015 sizes of 113 rows and more the first alone
+// takes 47 %, 1.066 times 256 rows' speed over all, with 8 % of its choices more than a tenth slower (16 x 1024 x 3584, squared relu,
+// 458 rows 151 / 208; 32 x 512 x 3584, 468 rows 191 / 250); both take 34 %, 1.071, with 1.7 %.
+// whole: gemm_xd
 // loads 16-byte pieces at 32-bit offsets of x and of an expert's matrix, which gemm_w4 behind its gather need not.
 static bool moe_half_tiles(int T, int E, int rows, int H, int I, bool glu, bool whole) {
   const int64_t most = 1 << 30;
   return whole && (int64_t)T * H < most && (int64_t)(I + 256) * H < most && (int64_t)(H + 256) * I < most && moe_xd_ok(181, I, H, glu) && moe_xd_ok(181, H, I, false) &&
-         moe_xd_us(E, rows, 128, H, I, glu) < 0.96 * moe_xd_us(E, rows, 256, H, I, glu);
+         moe_xd_us(E, rows, 128, H, I, glu) < 0.96 * moe_xd_us(E, rows, 256, H, I, glu) &&
+         moe_fit_us(E, rows, 128, H, I, glu) < (E > 24 || I > 4096 ? 0.9 : 1.03) * moe_fit_us(E, rows, 256, H, I, glu);
 }
 
 // The variant of a layer of T tokens and P pairs over E experts, bf16; whole: rows and weights start at 16 bytes.

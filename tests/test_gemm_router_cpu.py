@@ -203,3 +203,15 @@ def test_rows_by_a_list_want_four_k_tiles(K):
     N, rows, p = 512, 600, 1 << 20
     args = (p, p, p, p, 2, rows, N, K, K, K, N, 2 * N * K, G.EPI["silu"], N, 4, 1, 0, 0.0, 0, p, rows)
     assert hipk().gemm_grouped(*args) == -1
+
+
+@pytest.mark.parametrize("T,k,E,H,I,glu,want", [
+    (3664, 2, 16, 1024, 3584, False, 4), (7490, 2, 32, 512, 3584, False, 4), (7141, 1, 16, 1024, 3584, True, 4),  # 208 / 151, ... us in 128 rows
+    (2367, 3, 16, 1024, 1792, False, 4), (3200, 4, 32, 2048, 7168, True, 4),
+    (1408, 4, 20, 2048, 1792, False, 3), (1152, 4, 16, 4096, 3584, True, 3), (2048, 4, 16, 4096, 3584, True, 4), (4096, 4, 16, 4096, 3584, True, 4),
+])
+def test_rows_to_an_experts_tile(T, k, E, H, I, glu, want):
+    """128 rows (variant 3) where both estimates of a layer's time say so, 256 (4) elsewhere."""
+    from drtc_amd.ops._ext import hipk
+
+    assert hipk().moe_variant(T, T * k, E, H, I, glu, True) == want
