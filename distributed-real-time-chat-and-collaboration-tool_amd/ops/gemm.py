@@ -341,11 +341,15 @@ def tall_form(M: int, N: int, K: int, glu: bool = False, act: str = "silu") -> i
     2048, 160 33.4 / 30.3; 25600 x 4096, 224 57.2 / 54.2; 20480 x 2048 (160 tiles), 160 28.2 / 26.4, 224 30.0 / 29.2; in tiles of
     64: 14336 x 2048 gated, 132 rows 22.3 / 18.3, 160 20.4 / 19.4, 12800 x 2048 20.1 / 19.0, 16384 x 4096 gated 39.1 / 36.7.
     More than a round: 57344 x 4096 gated, 176 rows 100.6 / 109; fewer tiles: 16384 x 4096 gated, 160 rows 39.1 / 48.4, and of 64
-    8448 x 2048, 160 rows 17.6 / 17.9; 192 rows in tiles of 64 12800 x 2048 21.5 / 21.4."""
+    8448 x 2048, 160 rows 17.6 / 17.9; 192 rows in tiles of 64 12800 x 2048 21.5 / 21.4.  Tiles of 64 where the others' rows of W are
+    multiples of 4 KB apart, or long: over 3300 sizes K 2048, 4096, 6144, 8192 1.06, 1.07, 1.02, 1.18, 11008 and 14336 1.06 and 1.11, but
+    2304 .. 3584 0.96, 5120 0.91, 7168 0.98 (13312 x 5120 gated, 148 rows 40.5 / 46.3)."""
     if not (129 <= M <= 224 and K >= 2048 and _xd_enabled and _enabled and _xd_nt):
         return 0
     mt, rows = 3 if M <= 160 else 4 if M <= 192 else 5, 2 * N if glu else N
-    nf = 4 if rows % 128 == 0 and 160 <= rows // 128 <= 256 else 2 if mt == 3 and rows % 64 == 0 and 192 <= rows // 64 <= 256 else 0
+    nf = 4 if rows % 128 == 0 and 160 <= rows // 128 <= 256 else 0
+    if not nf and mt == 3 and rows % 64 == 0 and 192 <= rows // 64 <= 256 and (K % 2048 == 0 or K > 8192):
+        nf = 2
     if not nf or act == "clamped" and nf not in XD_CLAMP_NF:
         return 0
     form = 1001 + 100 * mt + 10 * nf

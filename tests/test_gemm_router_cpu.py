@@ -27,6 +27,8 @@ def test_nontemporal_forms_only_for_built_tiles():
     (224, 32000, 2048, False, 1541), (160, 7168, 2048, True, 1321), (161, 7168, 2048, True, 0), (128, 32000, 4096, False, 0),
     (225, 32000, 4096, False, 0), (160, 28672, 4096, True, 0), (160, 32000, 1024, False, 0), (160, 8448, 2048, False, 0),
     (160, 32016, 4096, False, 0),
+    (148, 6656, 5120, True, 0), (148, 6656, 4096, True, 1321), (148, 13312, 3072, False, 0), (148, 13312, 11008, False, 1321),
+    (148, 25600, 5120, False, 1341),  # tiles of 128 columns at any K
 ])
 def test_tall_tiles_rule(monkeypatch, M, N, K, glu, want):
     monkeypatch.setattr(G, "_xd_nt", True)
