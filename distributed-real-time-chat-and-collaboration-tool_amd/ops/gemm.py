@@ -1132,13 +1132,13 @@ def _glu_round(M: int, I: int, K: int) -> int:
     """gemm_xd gated form of tiles of 256 x 256 that one round takes.  From gemm_w4's first rows where 177 .. 256 of them keep the
     CUs busy, which gemm_w4 takes 2 to 11 % longer for (7168 x 2048 rows of W a half, 1024 rows 56.7 / 53.5 us; 7168 x 4096 99.3 / 89.9;
     6144 x 3072, 800 rows 73.1 / 68.8; 8192 x 4096, 640 95.1 / 86.6; fewer tiles: 5632 x 2048, 896 rows 46.4 / 47.2; more than a
-    round: 14336 x 1536 82.3 / 85.4).  From 513 rows where K is short: as fast as the library and a pass on the chip (7168 x
+    round: 14336 x 1536 82.3 / 85.4).  Over 2000 sizes K from 1792 on 1.04 .. 1.16, K 1024, 1280 and 1536 0.93, 0.96 and 0.99: gemm_w4's.  From 513 rows where K is short: as fast as the library and a pass on the chip (7168 x
     2048, 560 rows 47.4 / 47.2, 608 47.5 / 49.3), but prompts of these rows, which no decode step is padded to, are as long as their
     host path, and this is one launch for two (two prompts of 300, width 2048: 642 -> 519 a pass)."""
     tiles = -(-M // 256) * (I // 128)
     if tiles > 256 or M > DECODE_MAX_M:
         return 0
-    return 281 if M >= W4_GLU_MIN_M and tiles > 176 or 512 < M < W4_GLU_MIN_M and K <= 2048 and tiles >= 160 else 0
+    return 281 if M >= W4_GLU_MIN_M and tiles > 176 and K >= 1792 or 512 < M < W4_GLU_MIN_M and K <= 2048 and tiles >= 160 else 0
 
 
 def _glu_default(M: int, I: int, K: int, act: str = "silu") -> int:

@@ -74,7 +74,7 @@ def test_full_round_rule(monkeypatch, M, N, K, want):
 @pytest.mark.parametrize("M,I,K,want", [
     (513, 7168, 2048, 281), (639, 7168, 2048, 281), (512, 7168, 2048, 241), (600, 5632, 2048, 0), (600, 7168, 2112, 0),
     (600, 14336, 2048, 0), (769, 7168, 4096, 281), (1024, 7168, 4096, 281), (640, 8192, 4096, 281), (1024, 8320, 4096, 0),
-    (1024, 5632, 4096, 281),
+    (1024, 5632, 4096, 281), (910, 8192, 1024, 0), (910, 8192, 1728, 0), (910, 8192, 1792, 281), (560, 8192, 1024, 281),
 ])
 @pytest.mark.parametrize("act", ["silu", "clamped"])
 def test_gated_tiles_of_one_round(monkeypatch, M, I, K, want, act):
