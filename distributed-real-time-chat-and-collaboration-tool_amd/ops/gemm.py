@@ -231,9 +231,10 @@ def _resolve(M: int, N: int, K: int, ldx: int) -> tuple[str, int]:
     if M > DECODE_MAX_M:
         if w4_shape_ok(M, N, K):
             # 256 x 256 tiles for a quarter of the CUs at most, or a half: smaller ones (4096 rows, 2048 x 2048 39.1 / 31.3 us,
-            # 2048 x 7168 134 / 99)
+            # 2048 x 7168 134 / 99; 2000 sizes 1.1 .. 2.9 times, 1.5 .. 2 of them where an XCD has more tiles than another), but for
+            # 120 and 128 tiles of up to four columns, the same number to each XCD (8159 rows, 1024 x 8192 134 / 163)
             tiles = -(-M // 256) * (N // 256)
-            form = 141 if tiles <= 64 else 241 if tiles <= 128 else 0
+            form = 141 if tiles <= 64 else 241 if tiles <= 128 and (N > 1024 or tiles < 116 or tiles % 8) else 0
             if form and _xd_enabled and xd_supported(M, N, K, form):
                 return ("xd", form)
             return ("w4", 0)

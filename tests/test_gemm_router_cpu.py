@@ -155,6 +155,16 @@ def test_gemma_2048_decode_shapes_carry_a_gemm_xd_form():
             assert G.xd_supported(M, N, K, want)
 
 
+@pytest.mark.parametrize("M,N,want", [
+    (8159, 1024, ("w4", 0)), (7680, 1024, ("w4", 0)), (7424, 1024, ("xd", 241)), (7936, 1024, ("xd", 241)), (7168, 1024, ("xd", 241)),
+    (16384, 512, ("w4", 0)), (16384, 256, ("xd", 141)), (10000, 768, ("w4", 0)), (10400, 768, ("xd", 241)), (4096, 2048, ("xd", 241)),
+    (6100, 1280, ("xd", 241)), (9000, 2048, ("w4", 0)),
+])
+def test_half_a_round_of_large_tiles(monkeypatch, M, N, want):
+    monkeypatch.setattr(G, "_xd_enabled", True)
+    assert G._resolve(M, N, 4096, 4096) == want
+
+
 @pytest.mark.parametrize("op,M,N,K", [("squared_relu", 256, 25600, 4096), ("gated", 513, 14336, 2048), ("gated", 160, 25600, 2048)])
 @pytest.mark.parametrize("stride", [1 << 22, 4104])
 def test_rows_far_apart_stay_with_the_library(monkeypatch, op, M, N, K, stride):
