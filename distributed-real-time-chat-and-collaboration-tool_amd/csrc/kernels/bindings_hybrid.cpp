@@ -146,6 +146,7 @@ void bind_hybrid(py::module_& m) {
     PTR(gate); VAL(ldg);
     return drtc::launch_latent_prefill(f32, a, S(st));
   });
+  m.def("latent_up_merges", &drtc::latent_up_merges);
   m.def("latent_decode", [](int f32, const py::dict& d, u64 y, u64 w, int N, int64_t yb, int64_t yh, u64 st) {
     const Fields f{d};
     drtc::LatentDecodeArgs a{};

@@ -74,6 +74,7 @@ struct LatentDecodeArgs {
   int ldg;
 };
 int launch_latent_decode(int f32, const LatentDecodeArgs& a, hipStream_t st);
+bool latent_up_merges(int B, int R, int nsplits);
 int launch_latent_decode_up(int f32, const LatentDecodeArgs& a, void* y, const void* w, int N, int64_t yb, int64_t yh,
                             hipStream_t st);
 int launch_head_gemm(int f32, void* y, const void* x, const void* w, int B, int H, int N, int K,

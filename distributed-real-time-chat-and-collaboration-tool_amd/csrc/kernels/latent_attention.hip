@@ -1201,15 +1201,21 @@ int launch_latent_front(int f32, const LatentPrepArgs& a, const void* w, hipStre
   return (int)hipGetLastError();
 }
 
+// Whether the way up adds up the splits itself, in each of its workgroups again: where a thread has one vector of the rows,
+// B R <= 1024 (965 sizes of 4 to 64 heads, behind each other in a graph: 1.12, of more than 16 splits 1.37; two vectors 1.00, 0.83 at
+// least, three 0.92, eight 0.77: 16 rows of 16 heads, two splits of 512 dims 14.6 / 21.8 us), and up to 64 KB of them.
+// A step of one row at 3500, two such layers, 381 -> 364 us with the launch below.
+bool latent_up_merges(int B, int R, int nsplits) {
+  return B <= 16 && B * R <= 1024 && B * nsplits <= kUpParts && (int64_t)B * nsplits * R <= 16384;
+}
+
 // Decode: launch_latent_decode, and y[b, h, :] = w[h] out[b, h, :] for w [H, N, R].
 int launch_latent_decode_up(int f32, const LatentDecodeArgs& a, void* y, const void* w, int N, int64_t yb, int64_t yh,
                             hipStream_t st) {
   if (a.B == 0) return 0;
   const HeadGemm q{(bf16_t*)y, (const bf16_t*)a.out, (const bf16_t*)w, a.B, N, a.R, yb, yh, (int64_t)a.H * a.R, a.R};
-  // few rows: the product adds up the splits itself, in each of its workgroups again, up to 64 KB each (a step of one row at
-  // 3500, two such layers 381 -> 364 us with the launch below; 16 rows, 128 KB, 436 -> 439)
-  if (!lat_decode_split(f32, a) || !head_gemm_whole(N, a.R, yb, yh, q.xb, q.xh) || a.R % 128 || a.B > 16 ||
-      a.B * a.nsplits > kUpParts || (int64_t)a.B * a.nsplits * a.R > 16384) {
+  if (!lat_decode_split(f32, a) || !head_gemm_whole(N, a.R, yb, yh, q.xb, q.xh) || a.R % 128 ||
+      !latent_up_merges(a.B, a.R, a.nsplits)) {
     const int e = launch_latent_decode(f32, a, st);
     return e ? e : launch_head_gemm(f32, y, a.out, w, a.B, a.H, N, a.R, yb, yh, q.xb, q.xh, st);
   }
