@@ -1201,12 +1201,13 @@ int launch_latent_front(int f32, const LatentPrepArgs& a, const void* w, hipStre
   return (int)hipGetLastError();
 }
 
-// Whether the way up adds up the splits itself, in each of its workgroups again: where a thread has one vector of the rows,
-// B R <= 1024 (965 sizes of 4 to 64 heads, behind each other in a graph: 1.12, of more than 16 splits 1.37; two vectors 1.00, 0.83 at
-// least, three 0.92, eight 0.77: 16 rows of 16 heads, two splits of 512 dims 14.6 / 21.8 us), and up to 64 KB of them.
+// Whether the way up adds up the splits itself, in each of its workgroups again: where a thread has up to two vectors of the
+// rows, B R <= 2048 (965 sizes of 4 to 64 heads, behind each other in a graph: one vector 1.12, of more than 16 splits 1.37, two 1.00
+// and in decode steps of three and four rows 1.00 to 1.01, three 0.92, eight 0.77: 16 rows of 16 heads, two splits of 512 dims
+// 14.6 / 21.8 us), and up to 64 KB of them.
 // A step of one row at 3500, two such layers, 381 -> 364 us with the launch below.
 bool latent_up_merges(int B, int R, int nsplits) {
-  return B <= 16 && B * R <= 1024 && B * nsplits <= kUpParts && (int64_t)B * nsplits * R <= 16384;
+  return B <= 16 && B * R <= 2048 && B * nsplits <= kUpParts && (int64_t)B * nsplits * R <= 16384;
 }
 
 // Decode: launch_latent_decode, and y[b, h, :] = w[h] out[b, h, :] for w [H, N, R].

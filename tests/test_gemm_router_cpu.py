@@ -230,9 +230,9 @@ def test_rows_to_an_experts_tile(T, k, E, H, I, glu, want):
 
 
 def test_few_rows_ways_up_add_up_their_splits():
-    """One vector of the rows to a thread, 64 KB of splits."""
+    """Two vectors of the rows to a thread, 64 KB of splits."""
     from drtc_amd.ops._ext import hipk
 
     take = lambda *a: hipk().latent_up_merges(*a)
-    assert take(1, 512, 2) and take(1, 512, 32) and take(2, 512, 16) and take(4, 256, 16) and take(8, 128, 16)
-    assert not (take(3, 512, 2) or take(16, 512, 2) or take(5, 256, 4) or take(16, 256, 4) or take(1, 512, 33) or take(9, 128, 2))
+    assert take(1, 512, 2) and take(1, 512, 32) and take(4, 512, 8) and take(8, 256, 8) and take(16, 128, 8)
+    assert not (take(5, 512, 2) or take(16, 512, 2) or take(9, 256, 4) or take(16, 256, 4) or take(1, 512, 33) or take(17, 64, 2))
