@@ -210,10 +210,21 @@ struct W4Tile {
 //          256 B/clk limit beside the landing LDS-DMA (PMC: +72 % SQ_WAIT_INST_LDS against
 //          hipBLASLt's kernel of the same tile, profiles/r4j)
 //   V & 64 grouped form; V & 128 its A rows are read through an index list
+// The 64 MFMAs of a half in 2 x 2 blocks of fragments, (0,0) (0,1) (1,1) (1,0), the blocks of a pair of A fragments left
+// to right, of the next pair right to left.  Row by row (A held for 8) an MFMA draws more power, and the large products
+// run at the card's power limit: from registers alone, random operands, 2040 -> 2090 TFLOP/s (both operands new each
+// time: 1965; A held, B back and forth: 2055; 4 x 4 blocks: 2055); this kernel, 16384 x 4096 x 4096 store 1518 -> 1545,
+// gated 1501 -> 1527, 12160 x 6144 x 4096 1401 -> 1433, 16000 x 2048 x 7168 with residual 1405 -> 1430.  Zero operands,
+// below the limit, take the same time either way.
+constexpr int w4_order(int q) {
+  const int blk = q >> 2, n = q & 3, bi = blk >> 2, bj = (bi & 1) ? 3 - (blk & 3) : blk & 3;
+  return (2 * bi + (n >> 1)) * 8 + 2 * bj + (n == 1 || n == 2);
+}
+
 template <int V, bool DMA, bool NEXT, bool Z, int Q>
 DRTC_DEVICE void w4_step(f32x4 (&acc)[8][8], bf16x8 (&fa0)[8], bf16x8 (&fb0)[8],
                          bf16x8 (&fa1)[8], bf16x8 (&fb1)[8], const W4Tile& T, const W4Dma& d) {
-  constexpr int i = (Q >> 3) & 7, j = Q & 7;
+  constexpr int ij = w4_order(Q & 63), i = ij >> 3, j = ij & 7;
   if constexpr (Q < 64 && Z)  // first K tile of a persistent tile: accumulate onto 0
     acc[i][j] = mfma16(fa0[i], fb0[j], (f32x4){0.f, 0.f, 0.f, 0.f});
   else if constexpr (Q < 64)
@@ -253,7 +264,7 @@ DRTC_DEVICE void w4_step(f32x4 (&acc)[8][8], bf16x8 (&fa0)[8], bf16x8 (&fb0)[8],
     if constexpr (s < 7) asm volatile("s_add_u32 m0, m0, 0x1000" ::: "memory");
   }
   // ---- tile t + 1: its DMA (issued during tile t - 1) landed for every wave, then its
-  // half-0 fragments: fa0[0], fb0[0..7], fa0[1..7]
+  // half-0 fragments: fa0[0..1], fb0[0..7], fa0[2..7]
   constexpr bool kSpread = (V & 32) != 0;
   constexpr int qn = kSpread ? 63 : 103;
   // this step's own DMAs (tile t + 2) issued before qn: B 8 + A (1 at qn 63, 8 at 103)
@@ -275,19 +286,19 @@ DRTC_DEVICE void w4_step(f32x4 (&acc)[8][8], bf16x8 (&fa0)[8], bf16x8 (&fb0)[8],
   }
   if constexpr (NEXT && kSpread && Q > qn && ((Q - qn - 1) & 3) == 0 && (Q - qn - 1) / 4 < 16) {
     constexpr int r = (Q - qn - 1) / 4;
-    if constexpr (r == 0)
-      fa0[0] = w4_rd(T.lds, T.nxt + T.ra0);
-    else if constexpr (r <= 8)
-      fb0[r - 1] = w4_rd(T.lds, T.nxt + T.rb0 + 128 * (r - 1));
+    if constexpr (r <= 1)
+      fa0[r] = w4_rd(T.lds, T.nxt + T.ra0 + 2048 * r);
+    else if constexpr (r <= 9)
+      fb0[r - 2] = w4_rd(T.lds, T.nxt + T.rb0 + 128 * (r - 2));
     else
       fa0[r - 8] = w4_rd(T.lds, T.nxt + T.ra0 + 2048 * (r - 8));
   }
   if constexpr (NEXT && !kSpread && Q > qn && Q <= qn + 16) {
     constexpr int r = Q - qn - 1;
-    if constexpr (r == 0)
-      fa0[0] = w4_rd(T.lds, T.nxt + T.ra0);
-    else if constexpr (r <= 8)
-      fb0[r - 1] = w4_rd(T.lds, T.nxt + T.rb0 + 128 * (r - 1));
+    if constexpr (r <= 1)
+      fa0[r] = w4_rd(T.lds, T.nxt + T.ra0 + 2048 * r);
+    else if constexpr (r <= 9)
+      fb0[r - 2] = w4_rd(T.lds, T.nxt + T.rb0 + 128 * (r - 2));
     else
       fa0[r - 8] = w4_rd(T.lds, T.nxt + T.ra0 + 2048 * (r - 8));
   }
@@ -339,6 +350,13 @@ DRTC_DEVICE void w4_epilogue(const W4Params& p, bf16_t* cbase, f32x4 (&acc)[8][8
                              int mend, int tn, int wm, int wn, int l16, int g, int slice) {
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
+    if constexpr (!w4_res<EPI>() && (V & 32) != 0) {
+      // A row's accumulators leave the AGPRs when its turn comes.  Copied out ahead, all 256 spill the DMA offsets of A:
+      // their reload in the next tile's first K step waits for every store and load under way (store form, 2-3 kcycles of
+      // 168 a tile at K = 4096).  With a residual the rows loaded ahead fill these registers, and this order spills.
+#pragma unroll
+      for (int j = 0; j < 8; ++j) asm volatile("" : "+a"(acc[i][j]));
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int m = row0 + 128 * wm + 16 * i + 4 * g + r;
