@@ -3,15 +3,21 @@
 //  * temperature <= 0 : greedy argmax (ties -> lowest index), one row pass.
 //  * 0 < top_k <= 1024: exact top-k, then temperature softmax + top-p over the
 //    k candidates.  Selection without a histogram in the common case: every
-//    thread keeps the max key of the elements it streams; the k-th largest of
-//    those 1024 thread maxima is a lower bound tau0 on the k-th largest logit
-//    (the top-k thread maxima are k distinct elements >= tau0), so gathering
-//    `key >= tau0` yields all top-k plus a few extra (~k + O(1) on real logit
-//    rows), and such an element can only sit in a thread whose own max is
-//    >= tau0: only those ~k threads re-read their own elements to gather.
-//    One row pass.  If ties push the gather past 1024 slots, the row falls
-//    back to a 16-bit radix select (two histogram passes) and a ballot-
+//    thread keeps the max key of the elements it streams; a threshold tau0 that
+//    k of those 1024 thread maxima reach, and few more, is a lower bound on the
+//    k-th largest logit, so gathering `key >= tau0` yields all top-k plus a few
+//    extra, and such an element can only sit in a thread whose own max is
+//    >= tau0: only those ~k threads' elements are read again, eight lanes to a
+//    thread.  One row pass.  If ties push the gather past 1024 slots, the row
+//    falls back to a 16-bit radix select (two histogram passes) and a ballot-
 //    compacted full gather.
+//    What bounds a row is the chain of its stages, and fetching code that runs
+//    once a step: tau0 by one wave's ballots instead of the workgroup's
+//    histograms, a gather in a few instructions instead of one unrolled over 32
+//    elements, and every request of the row and its parameters at the start.
+//    V 32000, top-k 64, top-p 0.95, before / now: 1 row 11.3 / 6.9 us, 64 11.6 /
+//    7.4, 512 16.1 / 10.4, 1024 31.1 / 20.5; V 128256, 1 row 18.6 / 11.8, 1024
+//    72.0 / 62.7.
 //    Up to 128 candidates find their places by counting and are drawn from by one wave;
 //    more are bitonic-sorted.  All tokens tied with the k-th value stay.
 //  * top_k == 0       : temperature sampling with EXACT top-p over the whole
@@ -34,6 +40,8 @@
 // A NaN or -inf is never drawn; a row of nothing else gets the token -1.
 #include "common.h"
 #include "launchers.h"
+
+#include <type_traits>
 
 namespace drtc {
 
@@ -90,6 +98,35 @@ DRTC_DEVICE void for_row(const unsigned short* lr, int V, bool vec, F&& f) {
     for (int i = tid; i < V; i += kSampThreads) f(i, lr[i]);
   }
 }
+
+// A row that fits the workgroup's registers, read once: vectors of a thread in for_row's order, -inf behind the end.
+constexpr int kHeld = 4, kHeldRow = 8 * kHeld * kSampThreads;
+struct HeldRow {
+  u16x8 x[kHeld];
+  DRTC_DEVICE void load(const unsigned short* lr, int V) {
+    const u16x8 none = {0xff80, 0xff80, 0xff80, 0xff80, 0xff80, 0xff80, 0xff80, 0xff80};
+#pragma unroll
+    for (int u = 0; u < kHeld; ++u) {
+      const int v = threadIdx.x + u * kSampThreads;
+      x[u] = v < V >> 3 ? *reinterpret_cast<const u16x8*>(lr + 8 * v) : none;
+    }
+  }
+  template <class F>
+  DRTC_DEVICE void operator()(F&& f) const {
+#pragma unroll
+    for (int u = 0; u < kHeld; ++u)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f(8 * ((int)threadIdx.x + u * kSampThreads) + j, x[u][j]);
+  }
+};
+template <int U>
+struct ReadRow {
+  const unsigned short* lr;
+  int V;
+  bool vec;
+  template <class F>
+  DRTC_DEVICE void operator()(F&& f) const { for_row<U>(lr, V, vec, f); }
+};
 
 DRTC_DEVICE float wave_sum(float x) {
 #pragma unroll
@@ -293,28 +330,88 @@ DRTC_DEVICE int gather_ge(SampShared& s, const unsigned short* lr, int V, bool v
   return s.misc[2];
 }
 
+// The wave's largest in lane 63: shifts within rows of 16, then a row's last lane to the next row and the next two.
+template <int... Ctrl>
+DRTC_DEVICE unsigned last_max(unsigned x) {
+  ((x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, Ctrl, 0xf, 0xf, false))), ...);
+  return x;
+}
+
+// A threshold that at least k of 1024 keys reach, found by one wave that holds 16 to a lane: down from the largest in
+// doubled steps, then halved, until not many more than k reach it (112 where they may be so few: sample_few; all that
+// reach it are to fit the candidates) or no higher one does.
+DRTC_DEVICE unsigned few_above(const unsigned short* keys, int k) {
+  const int lane = threadIdx.x & 63, enough = k < 96 ? 112 : min(k + k / 16, max(k, 900));
+  u32x4 x[2];
+  unsigned top = 0;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    x[i] = *reinterpret_cast<const u32x4*>(keys + 512 * i + 8 * lane);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) top = max(top, max(x[i][j] >> 16, x[i][j] & 0xffffu));
+  }
+  top = last_max<0x111, 0x112, 0x114, 0x118, 0x142, 0x143>(top);
+  auto reach = [&](unsigned t) {
+    int n = 0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        n += __popcll(__ballot(x[i][j] >= t << 16)) + __popcll(__ballot((unsigned short)x[i][j] >= (unsigned short)t));
+    return n;
+  };
+  unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)top, 63) + 1, lo = hi;
+  int n = 0;
+  for (unsigned d = 32; n < k; d *= 2) {  // (0 is reached by all)
+    hi = lo;
+    lo = lo > d ? lo - d : 0;
+    n = reach(lo);
+  }
+  while (n > enough && hi - lo > 1) {
+    const unsigned mid = (lo + hi) / 2;
+    const int m = reach(mid);
+    if (m >= k) {
+      lo = mid;
+      n = m;
+    } else {
+      hi = mid;
+    }
+  }
+  return lo;
+}
+
 // The rest of sample_topk for up to 128 gathered candidates, n: each finds its place by counting those
-// ahead of it (8 threads to a candidate), then one wave does what is left, two candidates to a lane - the
-// same sums in the same order as the form below with two barriers instead of some fifty.  V 32000, top-k
-// 64, top-p 0.95: 1 row 15.0 -> 11.2 us, 1024 rows 39.7 -> 31.2; V 128256, 1024 rows 78.0 -> 71.8.
+// ahead of it (8 threads to a candidate; sort: their places' keys, of rows whose indexes have 16 bits), then one wave does what
+// is left, two candidates to a lane - the same sums in the same order as the form below with two barriers instead of some fifty.
 constexpr int kFew = 128;
+// an order of all bit patterns, zeros alike
+DRTC_DEVICE unsigned place_key(float v) { return v == 0.f ? 0x8000u : ord16((unsigned short)(__float_as_uint(v) >> 16)); }
 // against the largest: 1 for itself, at +inf too
 DRTC_DEVICE float weight(float v, float top, float inv_t) { return v == top ? 1.f : __expf((v - top) * inv_t); }
-DRTC_DEVICE void sample_few(SampShared& s, const TokenOut& out, int row, float temp, int k, int n, float pp,
-                            uint64_t seed, uint64_t st) {
+DRTC_DEVICE void sample_few(SampShared& s, const unsigned* sort, const TokenOut& out, int row, float temp, int k, int n,
+                            float pp) {
   const int tid = threadIdx.x, lane = tid & 63, own = tid >> 3;
   float* const sv = reinterpret_cast<float*>(&s.hist[8][0]);
   int* const si = reinterpret_cast<int*>(&s.hist[9][0]);
-  // an order of all bit patterns, zeros alike: every candidate gets a place of its own
-  auto order = [](float v) { return v == 0.f ? 0x8000u : ord16((unsigned short)(__float_as_uint(v) >> 16)); };
+  auto order = [](float v) { return place_key(v); };
+  // every candidate gets a place of its own
   if (own < n) {
     const float v = s.val[own];
     const int id = s.idx[own];
-    const unsigned key = order(v);
     int ahead = 0;
-    for (int j = tid & 7; j < n; j += 8) {
-      const unsigned kj = order(s.val[j]);
-      ahead += kj > key || (kj == key && s.idx[j] < id);
+    if (sort) {  // (0 behind the last)
+      const unsigned mine = sort[own];
+#pragma unroll
+      for (int i = 0; i < kFew / 32; ++i) {
+        const u32x4 q = *reinterpret_cast<const u32x4*>(sort + 32 * i + 4 * (tid & 7));
+        ahead += (q[0] > mine) + (q[1] > mine) + (q[2] > mine) + (q[3] > mine);
+      }
+    } else {
+      const unsigned key = order(v);
+      for (int j = tid & 7; j < n; j += 8) {
+        const unsigned kj = order(s.val[j]);
+        ahead += kj > key || (kj == key && s.idx[j] < id);
+      }
     }
     ahead += __shfl_xor(ahead, 1, 64);
     ahead += __shfl_xor(ahead, 2, 64);
@@ -358,7 +455,7 @@ DRTC_DEVICE void sample_few(SampShared& s, const TokenOut& out, int row, float t
     const uint64_t hit = __ballot(i < n && x[z] >= need && (i == 0 || lo[z] < need));
     if (hit) cut = 64 * z + __ffsll((unsigned long long)hit) - 1;
   }
-  const float target = uniform(seed, st, row, 0) * __shfl(cut >= 64 ? x[1] : x[0], cut & 63, 64);
+  const float target = s.wred[0][0] * __shfl(cut >= 64 ? x[1] : x[0], cut & 63, 64);  // (the draw)
   int at = 0;  // (the first, where a temperature that is no number leaves no weights)
 #pragma unroll
   for (int z = 0; z < 2; ++z) {
@@ -369,66 +466,115 @@ DRTC_DEVICE void sample_few(SampShared& s, const TokenOut& out, int row, float t
   if (lane == 0) out.put(row, si[at]);
 }
 
-template <int U>
-DRTC_DEVICE void sample_topk(SampShared& s, const TokenOut& out, const unsigned short* lr, int V,
+// each: visits the thread's elements of the row
+template <int U, class Row>
+DRTC_DEVICE void sample_topk(SampShared& s, const TokenOut& out, const Row& each, const unsigned short* lr, int V,
                              bool vec, int row, float temp, int k, float pp, uint64_t seed,
                              uint64_t st) {
-  const int tid = threadIdx.x;
-  // ---- pass 1: per-thread max key; tau0 = k-th largest of the thread maxima
+  const int tid = threadIdx.x, lane = tid & 63;
+  // ---- pass 1: per-thread max key; tau0: reached by k of the thread maxima, by few more where it can be
   float most = -INFINITY;  // (of floats: NaNs drop out, and +0 is above -0 as in the keys)
-  for_row<U>(lr, V, vec, [&](int, unsigned short b) { most = fmaxf(most, bits2f(b)); });
+  each([&](int, unsigned short b) { most = fmaxf(most, bits2f(b)); });
   const unsigned tm = ord16((unsigned short)(__float_as_uint(most) >> 16));
-  unsigned* h = &s.hist[0][0];
-  h[tid] = tm;  // hist doubles as a 1024-key buffer here
+  // hist doubles as a buffer of 1024 keys, of the threads that are looked at again, and of the candidates' sort keys
+  unsigned short* const h = reinterpret_cast<unsigned short*>(&s.hist[0][0]);
+  int* const again = reinterpret_cast<int*>(&s.hist[4][0]);
+  unsigned* const sort = V <= 0x10000 ? &s.hist[12][0] : nullptr;
+  h[tid] = (unsigned short)tm;
+  s.hist[12 + tid / 256][tid & 255] = 0;
   __syncthreads();
-  // radix select over the 1024 thread maxima (LDS only)
-  unsigned prefix = 0, mask = 0;
-  int remaining = k;
-  for (int pass = 8; pass >= 0; pass -= 8) {
-    unsigned* bins = &s.hist[4][0];  // bins after the 1024-key buffer (hist[0..3])
-    if (tid < 256) bins[tid] = 0;
-    __syncthreads();
-    const unsigned key = h[tid];
-    if ((key & mask) == prefix) atomicAdd(&bins[(key >> pass) & 255u], 1u);
-    __syncthreads();
-    select_bin(s, bins, remaining);
-    prefix |= (unsigned)s.misc[0] << pass;
-    mask |= 255u << pass;
-    remaining = s.misc[1];
-    __syncthreads();
+  if (tid < 64) {
+    const unsigned t = few_above(h, k);
+    if (tid == 0) {
+      s.misc[0] = (int)t;
+      s.misc[2] = s.misc[3] = 0;
+    }
+  } else if (tid == 64) {
+    s.wred[0][0] = uniform(seed, st, row, 0);
   }
-  prefix = max(prefix, kLowKey);
-  // ---- gather key >= tau0 (>= k elements by construction, or all numbers).  Such an element
-  // can only sit in a thread whose own max is >= tau0, so only those threads
-  // (about k of the 1024) re-read their own elements: no second row pass.
-  if (tid == 0) s.misc[2] = 0;
-  s.val[tid] = -INFINITY;
-  s.idx[tid] = 0x7fffffff;
   __syncthreads();
-  if (tm >= prefix) {
-    for_row<U>(lr, V, vec, [&](int i, unsigned short b) {
-      if (ord16(b) - prefix <= kTopKey - prefix) {  // key in [prefix, kTopKey]
-        const int slot = atomicAdd(&s.misc[2], 1);
-        if (slot < kCand) { s.val[slot] = bits2f(b); s.idx[slot] = i; }
+  const unsigned prefix = max((unsigned)s.misc[0], kLowKey);
+  // places in a list for the lanes of m, counted by one atomic for the wave
+  auto places = [&](int* count, int n) {
+    int base = 0;
+    if (lane == 0) base = atomicAdd(count, n);
+    return __builtin_amdgcn_readfirstlane(base);
+  };
+  auto below = [](uint64_t m) { return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u)); };
+  // ---- gather key >= tau0 (>= k elements by construction, or all numbers).  Such an element can only sit in a thread
+  // whose own max is >= tau0: of those threads' elements (about k of the 1024) every lane takes a few of one's, eight
+  // lanes to a thread.
+  if (const uint64_t m = __ballot(tm >= prefix)) {
+    const int at = places(&s.misc[3], __popcll(m)) + below(m);
+    if (tm >= prefix) again[at] = tid;
+  }
+  __syncthreads();
+  const int threads = s.misc[3], nv = vec ? V >> 3 : 0;
+  // N elements from index i on, those that are `in` the row
+  auto take = [&](auto count, int i, bool in) {
+    constexpr int N = decltype(count)::value;
+    typedef unsigned short Some __attribute__((ext_vector_type(N)));
+    Some x = {};
+    if (in) x = *reinterpret_cast<const Some*>(lr + i);
+    uint64_t m[N];
+    int n = 0;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      m[j] = __ballot(in && ord16(x[j]) - prefix <= kTopKey - prefix);  // key in [prefix, kTopKey]
+      n += __popcll(m[j]);
+    }
+    if (n == 0) return;
+    int base = places(&s.misc[2], n);
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const int slot = base + below(m[j]);
+      if ((m[j] >> lane & 1) && slot < kCand) {
+        const float v = bits2f(x[j]);
+        s.val[slot] = v;
+        s.idx[slot] = i + j;
+        if (sort) sort[slot] = place_key(v) << 16 | (0xffffu - (unsigned)(i + j));
       }
-    });
+      base += __popcll(m[j]);
+    }
+  };
+#pragma unroll 1
+  for (int g = 0; g < threads; g += kSampThreads / 8) {
+    const bool on = g + (tid >> 3) < threads;
+    const int t = on ? again[g + (tid >> 3)] : 0;
+#pragma unroll 1
+    for (int v = 0; v < nv; v += 4 * kSampThreads) {
+      const int at = v + t + (tid >> 1 & 3) * kSampThreads;
+      take(std::integral_constant<int, 4>{}, 8 * at + 4 * (tid & 1), on && at < nv);
+    }
+#pragma unroll 1
+    for (int e = 8 * nv; e < V; e += 8 * kSampThreads) {
+      const int at = e + t + (tid & 7) * kSampThreads;
+      take(std::integral_constant<int, 1>{}, at, on && at < V);
+    }
   }
   __syncthreads();
   int n = s.misc[2];
+  const unsigned* gathered = sort;  // (not by gather_ge)
   if (n > kCand) {  // heavy ties: exact k-th key by radix select, gather again
     const unsigned thr = radix_kth<U>(s, lr, V, vec, k);
     n = min(gather_ge<U>(s, lr, V, vec, thr), kCand);
+    gathered = nullptr;
   }
   if (n == 0) {
     if (tid == 0) out.put(row, -1);
     return;
   }
   if (n <= kFew) {
-    sample_few(s, out, row, temp, k, n, pp, seed, st);
+    sample_few(s, gathered, out, row, temp, k, n, pp);
     return;
   }
   int np2 = 1;
   while (np2 < n) np2 <<= 1;
+  if (tid >= n) {
+    s.val[tid] = -INFINITY;
+    s.idx[tid] = 0x7fffffff;
+  }
+  __syncthreads();
   // ---- bitonic sort, descending (ties -> lower index first)
   for (int size = 2; size <= np2; size <<= 1) {
     for (int stride = size >> 1; stride > 0; stride >>= 1) {
@@ -602,7 +748,7 @@ DRTC_DEVICE void sample_topp_full(SampShared& s, const TokenOut& out, const unsi
 // OCC = 1: one 1024-thread workgroup per CU (91 VGPRs, 4-deep load unroll); OCC = 2: two
 // (<= 64 VGPRs, 2-deep unroll), so one row's selection tail (scans, block reductions,
 // barriers) overlaps another row's stream on the same CU.
-template <int OCC>
+template <int OCC, bool HELD>
 __global__ __launch_bounds__(kSampThreads, 4 * OCC) void sample_kernel(
     int* __restrict__ out_tokens, const bf16_t* __restrict__ logits, int V,
     int ld, const float* __restrict__ temperature, const int* __restrict__ top_k,
@@ -614,14 +760,23 @@ __global__ __launch_bounds__(kSampThreads, 4 * OCC) void sample_kernel(
   const int lane = tid & 63, wid = tid >> 6;
   const unsigned short* lr = (const unsigned short*)(logits + (int64_t)row * ld);
   const bool vec = ((reinterpret_cast<uintptr_t>(lr) & 15) == 0);
+  // the row and everything that says what to do with it are asked for together
+  using Row = std::conditional_t<HELD, HeldRow, ReadRow<U>>;
+  Row each;
+  if constexpr (HELD) each.load(lr, V);
+  else each = {lr, V, vec};
   const float temp = temperature ? temperature[row] : 0.f;
+  const uint64_t st = step ? (uint64_t)step[0] : 0ull;
+  const float asked = top_p ? top_p[row] : 1.f, pp = asked > 0.f && asked < 1.f ? asked : 1.f;
+  int k = top_k ? top_k[row] : 0;
   const TokenOut out{out_tokens, mirror.turn ? mirror.host[~*mirror.turn & 1] : nullptr};  // (the turn is the next step's)
+  __builtin_amdgcn_sched_barrier(0);
   __shared__ SampShared s;
 
   if (temp <= 0.f) {  // ---------------------------------- greedy argmax
     float best = -INFINITY;
     int bi = 0x7fffffff;
-    for_row<U>(lr, V, vec, [&](int i, unsigned short b) {
+    each([&](int i, unsigned short b) {
       const float v = bits2f(b);
       if (v > best || (v == best && i < bi)) { best = v; bi = i; }
     });
@@ -640,12 +795,9 @@ __global__ __launch_bounds__(kSampThreads, 4 * OCC) void sample_kernel(
     }
     return;
   }
-  const uint64_t st = step ? (uint64_t)step[0] : 0ull;
-  const float pp = (top_p && top_p[row] > 0.f && top_p[row] < 1.f) ? top_p[row] : 1.f;
-  int k = top_k ? top_k[row] : 0;
   if (k >= V) k = 0;
   if (k > 0) {
-    sample_topk<U>(s, out, lr, V, vec, row, temp, min(k, kCand), pp, seed, st);
+    sample_topk<U>(s, out, each, lr, V, vec, row, temp, min(k, kCand), pp, seed, st);
   } else {
     sample_topp_full<U>(s, out, lr, V, vec, row, temp, pp, seed, st);
   }
@@ -844,12 +996,13 @@ int launch_sample(int* out_tokens, const void* logits, int B, int V, int ld,
     const char* e = getenv("DRTC_SAMPLER_OCC");
     return e && e[0] == '1' ? 1 : 2;
   }();
-  if (occ == 2)
-    hipLaunchKernelGGL(sample_kernel<2>, dim3(B), dim3(kSampThreads), 0, st, out_tokens,
-                       (const bf16_t*)logits, V, ld, temperature, top_k, top_p, seed, step, mirror);
-  else
-    hipLaunchKernelGGL(sample_kernel<1>, dim3(B), dim3(kSampThreads), 0, st, out_tokens,
-                       (const bf16_t*)logits, V, ld, temperature, top_k, top_p, seed, step, mirror);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(B), dim3(kSampThreads), 0, st, out_tokens, (const bf16_t*)logits, V, ld, temperature,
+                       top_k, top_p, seed, step, mirror);
+  };
+  const bool held = V <= kHeldRow && V % 8 == 0 && ld % 8 == 0 && (uintptr_t)logits % 16 == 0;
+  if (occ == 2) held ? go(sample_kernel<2, true>) : go(sample_kernel<2, false>);
+  else held ? go(sample_kernel<1, true>) : go(sample_kernel<1, false>);
   return (int)hipGetLastError();
 }
 

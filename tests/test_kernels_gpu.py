@@ -634,6 +634,32 @@ def test_sample_skips_nans(hipk, V, k, nans):
         assert (clean.cpu()[live, got[live].long()] > float("-inf")).all()
 
 
+@pytest.mark.parametrize("V", [8, 1024, 8192, 32760, 32768, 32776, 65536, 65544])
+@pytest.mark.parametrize("k", [1, 64, 200, 1000])
+def test_sample_row_forms(hipk, V, k):
+    """Rows held in registers (16-byte rows of up to 32,768), read in vectors and read one by one (a view that starts
+    2 bytes off) give the same tokens, with and without ties, greedy rows among them; all in the top k.  (Where more than
+    1024 tie for the k places, the sampler keeps 1024 of them, whichever: those rows are only in the top k.)"""
+    B, k = 40, min(k, V - 1)
+    g = torch.Generator().manual_seed(V + k)
+    lg = torch.randn(B, V, generator=g) * 2
+    lg[::2] = (lg[::2] * 8).round() / 8
+    lg = lg.to(torch.bfloat16).to(DEV)
+    odd = torch.empty(B, V + 8, dtype=torch.bfloat16, device=DEV)[:, 1:V + 1]
+    odd.copy_(lg)
+    temp = torch.linspace(0.3, 1.5, B, device=DEV)
+    temp[5::7] = 0
+    args = (torch.full((B,), k, dtype=torch.int32, device=DEV), torch.full((B,), 0.9, device=DEV))
+    kth = lg.float().topk(k).values[:, -1]
+    fits = (lg.float() >= kth[:, None]).sum(1) <= 1024
+    assert k == 1000 or fits[1::2].all()
+    for i in range(3):
+        step = torch.tensor([i], device=DEV)
+        got = ops.sample(lg, temp, *args, seed=9, step=step).long()
+        assert torch.equal(got[fits], ops.sample(odd, temp, *args, seed=9, step=step).long()[fits])
+        assert (lg.float().gather(1, got[:, None])[:, 0] >= kth).all()
+
+
 def test_sample_top_p_full_vocab_exact(hipk):
     """top_k = 0: every draw lies in the exact nucleus of the full 128k vocab,
     and most draws are ranked below 1024 (nothing is truncated to a candidate
