@@ -169,7 +169,11 @@ struct DecodeRope {
   const float* cos_sin;   // [max_pos][D]: cos | sin
   bf16_t* k_cache;        // the caches the kernel reads (written for the step's token)
   bf16_t* v_cache;
+  const float* parts;     // paged_decode_kernel, PARTS: the rows as n_parts 32-bit sums [B][q_stride], part_stride apart
+  int64_t part_stride;
+  int n_parts;            // 2 .. kQkvParts
 };
+constexpr int kQkvParts = 4;
 
 // rotate the lane's fragments f[0..KS) of one head (position pos), rounding as rope_kv
 template <int D>
@@ -248,7 +252,12 @@ DRTC_DEVICE float load_part(const float* p) {
 // blocks two heads two waves each, where a workgroup to a head would leave three waves or two without work and
 // four or eight at work on a CU: 1024 x 20 tokens 45.8 -> 33.6 us (persistent: 36.7), x 40 58.3 -> 47.9 (51.8), x 60
 // 64.3 -> 61.5 (66.8), 512 x 20 24.7 -> 19.9 (20.7), 256 x 40 18.3 -> 16.8 (17.4); 256 x 20 13.8 -> 13.4 (12.0).
-template <int D, bool ROPE>
+// PARTS (up to 64 rows, attention.py decode_qkv_parts): q, k and v come as the sums of the projection's K slices
+// (gemm_midm.hip), added up here, in order, and rounded as the projection rounds its rows.  A projection cut in slices fills
+// the chip: 6144 x 4096, whole / two slices, 4 rows 12.6 / 10.6 us, 16 rows 14.1 / 11.1, 64 rows 17.0 / 13.8 (four); 3072 x
+// 2048, 16 rows 6.2 / 5.4.  Every wave needs all of q: a quarter of the heads each, which meet in the LDS beside the staged
+// rows (16 x 1000 19.0 us, as from rows; each wave adding up all of them, two workgroups to a CU for the registers: 21.4).
+template <int D, bool ROPE, bool PARTS = false>
 __global__ __launch_bounds__(256, D >= 256 ? 2 : 4) void paged_decode_kernel(
     bf16_t* __restrict__ out, float* __restrict__ part_o,
     float* __restrict__ part_ml, int* __restrict__ counters, const bf16_t* __restrict__ q,
@@ -275,10 +284,26 @@ __global__ __launch_bounds__(256, D >= 256 ? 2 : 4) void paged_decode_kernel(
   const int ph_b = bt[min(blk_begin + w + 4, bt_stride - 1)];
   bf16x8 qf[KS];  // Q^T B-operand fragments (zero for padding columns col >= G)
   const bf16_t* qrow = q + (int64_t)b * q_stride + (int64_t)(h * G + col) * D;
+  // two values a lane of every fourth q head, and of the step token's k and v
+  constexpr int NP = PARTS ? kQkvParts : 1, QH = PARTS ? 4 : 1;
+  [[maybe_unused]] f32x2 qp[QH][NP], kp[NP], vp[NP];
+  if constexpr (PARTS) {
+    const float* at = rope.parts + (int64_t)b * q_stride + 2 * (lane & (D / 2 - 1));
 #pragma unroll
-  for (int s = 0; s < KS; ++s) {
-    if (col < G) qf[s] = load_bf16x8(qrow + 32 * s + 8 * g);
-    else for (int j = 0; j < 8; ++j) qf[s][j] = f2bf(0.f);
+    for (int i = 0; i < NP; ++i)
+      if (i < rope.n_parts) {
+#pragma unroll
+        for (int j = 0; j < QH; ++j)
+          if (w + 4 * j < G) qp[j][i] = *reinterpret_cast<const f32x2*>(at + i * rope.part_stride + (h * G + w + 4 * j) * D);
+        kp[i] = *reinterpret_cast<const f32x2*>(at + i * rope.part_stride + (Hq + h) * D);
+        vp[i] = *reinterpret_cast<const f32x2*>(at + i * rope.part_stride + (Hq + Hkv + h) * D);
+      }
+  } else {
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      if (col < G) qf[s] = load_bf16x8(qrow + 32 * s + 8 * g);
+      else for (int j = 0; j < 8; ++j) qf[s][j] = f2bf(0.f);
+    }
   }
   const int ctx = context_lens[b];
   const int nc = ROPE ? ctx - 1 : ctx;  // tokens read from the cache
@@ -310,7 +335,7 @@ __global__ __launch_bounds__(256, D >= 256 ? 2 : 4) void paged_decode_kernel(
     ph_a = bt[min(sub, bt_stride - 1)];
   }
   const bool alone = nblk == 1;  // one wave has it all, and nothing to merge
-  if (alone && sub != 0) return;
+  if (!PARTS && alone && sub != 0) return;
 
   const int blk_end = min(nblk, blk_begin + blocks_per_part);
 
@@ -341,7 +366,7 @@ __global__ __launch_bounds__(256, D >= 256 ? 2 : 4) void paged_decode_kernel(
     const __amdgpu_buffer_rsrc_t rc = dma_rsrc(rope.cos_sin + (int64_t)__builtin_amdgcn_readfirstlane(pos) * D);
 #pragma unroll
     for (int i = 0; i < D / 64; ++i) dma_dword_lds(dst + 512 + 256 * i, at + 256u * i, rc);
-    if (taker) {
+    if (taker && !PARTS) {
       const __amdgpu_buffer_rsrc_t rq = dma_rsrc(q + (int64_t)b * q_stride + (int64_t)(Hq + h) * D);
       const unsigned in = lane < D / 2 ? at : kNoRow;  // a row: D / 2 dwords
       dma_dword_lds(dst, in, rq);
@@ -360,6 +385,31 @@ __global__ __launch_bounds__(256, D >= 256 ? 2 : 4) void paged_decode_kernel(
     else wait_vm<0>();
     asm volatile("" ::: "memory");
     const float* cs = reinterpret_cast<const float*>(stage + 512);
+    if constexpr (PARTS) {
+      char* const ql = reinterpret_cast<char*>(smem + 128 + 64 * D) + 4096;  // [G][D] bf16
+      auto put = [&](char* to, const f32x2 (&x)[NP]) {
+        f32x2 y = x[0];
+#pragma unroll
+        for (int i = 1; i < NP; ++i)
+          if (i < rope.n_parts) y += x[i];
+        const bf16x2 v = {f2bf(y[0]), f2bf(y[1])};
+        if (lane < D / 2) *reinterpret_cast<bf16x2*>(to + 4 * lane) = v;
+      };
+#pragma unroll
+      for (int j = 0; j < QH; ++j)
+        if (w + 4 * j < G) put(ql + (w + 4 * j) * D * 2, qp[j]);
+      if (taker) {
+        put(stage, kp);
+        put(stage + 256, vp);
+      }
+      lds_barrier();
+      if (alone && sub != 0) return;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        if (col < G) qf[s] = *reinterpret_cast<const bf16x8*>(ql + (col * D + 32 * s + 8 * g) * 2);
+        else for (int j = 0; j < 8; ++j) qf[s][j] = f2bf(0.f);
+      }
+    }
     rope_frags_lds<D>(qf, cs, g);
     if (taker) {
       const bf16_t* kn = reinterpret_cast<const bf16_t*>(stage);
@@ -1174,7 +1224,8 @@ int launch_paged_decode_rope(void* out, float* part_o, float* part_ml, const voi
                              const int* block_tables, int bt_stride, const int* context_lens,
                              int B, int Hq, int Hkv, int D, float scale, int max_parts,
                              int blocks_per_part, const int* positions, const int64_t* slots,
-                             const float* cos_sin, int max_wgs, int* counters, int variant, hipStream_t st) {
+                             const float* cos_sin, int max_wgs, int* counters, int variant, const float* parts,
+                             int n_parts, hipStream_t st) {
   if (B == 0) return 0;
   if (Hkv <= 0 || Hq % Hkv != 0 || Hq / Hkv > 16 || (D != 64 && D != 128)) return -1;
   if (!positions || !slots || !cos_sin || q_stride < (Hq + 2 * Hkv) * D) return -1;
@@ -1194,12 +1245,19 @@ int launch_paged_decode_rope(void* out, float* part_o, float* part_ml, const voi
   int wgs = std::min((items + 3) / 4, 2 * n_cu);
   if (max_wgs > 0) wgs = std::min(wgs, max_wgs);
   const dim3 pgrid(std::max(1, wgs)), pblock(256);
-  const DecodeRope r{positions, slots, cos_sin, (bf16_t*)k_cache, (bf16_t*)v_cache};
+  if (parts && (variant != 1 || n_parts < 2 || n_parts > kQkvParts || q_stride % 4 || (uintptr_t)parts % 16)) return -1;
+  const DecodeRope r{positions, slots, cos_sin, (bf16_t*)k_cache, (bf16_t*)v_cache, parts, (int64_t)B * q_stride, n_parts};
   if (variant == 1) {  // a workgroup per (sequence, kv head, partition)
     if (max_parts > 1 && !counters) return -2;
     if (max_parts > kFusedMergeParts) return -1;
     const dim3 grid(B * Hkv, max_parts);
     const size_t lds = (128 + 4 * (size_t)D * 16) * sizeof(float) + 4096;  // and the staged rows
+    if (parts) {
+      (D == 64 ? paged_decode_kernel<64, true, true> : paged_decode_kernel<128, true, true>)<<<grid, pblock, lds + Hq / Hkv * D * 2, st>>>(
+          (bf16_t*)out, part_o, part_ml, counters, nullptr, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache,
+          block_tables, bt_stride, context_lens, Hq, Hkv, sl2, max_parts, blocks_per_part, 1, r);
+      return (int)hipGetLastError();
+    }
     (D == 64 ? paged_decode_kernel<64, true> : paged_decode_kernel<128, true>)<<<grid, pblock, lds, st>>>(
         (bf16_t*)out, part_o, part_ml, counters, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache,
         (const bf16_t*)v_cache, block_tables, bt_stride, context_lens, Hq, Hkv, sl2, max_parts, blocks_per_part,

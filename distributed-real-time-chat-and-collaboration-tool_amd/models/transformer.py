@@ -608,8 +608,13 @@ class TransformerLM:
         D = cfg.head_dim
         B = ids.shape[0]
 
+        # the attention adds up the sums of that many K slices of the projection
+        parts = 0
+        if meta.workspace is not None and self.device.type == "cuda":
+            parts = ops.decode_qkv_parts(B, sh.hkv, D, meta.block_tables.shape[1], meta.workspace.max_parts)
+
         def attn(i, L, x):
-            qkv = ops.norm_linear(x, L["qkv"])
+            qkv = ops.norm_linear(x, L["qkv"], parts)
             kc, vc = kv_caches[i]
             # RoPE + the step's KV write inside the attention launch (persistent kernel)
             a = ops.paged_decode_attention_rope(qkv, meta.positions, meta.slots, self.cos_sin,

@@ -12,7 +12,7 @@ is fused here.
 """
 from ._ext import on_gpu, reference_mode
 from .activation import act_glu, act_glu_ref
-from .attention import (KV_BLOCK, DecodeWorkspace, decode_partitioning, paged_decode_attention,
+from .attention import (KV_BLOCK, DecodeWorkspace, decode_partitioning, decode_qkv_parts, paged_decode_attention,
                         paged_decode_attention_rope, set_prefill_persist,
                         paged_decode_ref, prefill_attention, prefill_attention_ref, prefill_tiles)
 from .delta import DeltaWeights, Portions, delta_decode, delta_scan, short_conv
@@ -41,7 +41,7 @@ __all__ = [
     "fused_glu_ok",
     "mfma_gemm", "linear_residual", "residual_fusable", "PendingNorm", "fused_moe", "router_logits",
     "fused_moe_ref", "moe_norm_ok", "act_glu", "act_glu_ref", "KV_BLOCK", "DecodeWorkspace",
-    "decode_partitioning", "paged_decode_attention", "paged_decode_attention_rope",
+    "decode_partitioning", "decode_qkv_parts", "paged_decode_attention", "paged_decode_attention_rope",
     "paged_decode_ref", "prefill_attention", "prefill_attention_ref", "prefill_tiles",
     "set_prefill_persist", "rmsnorm", "rmsnorm_ref", "build_rope_cache", "rope_kv_",
     "rope_kv_ref", "kv_write_v", "kv_write_v_ref", "sample", "sample_ref", "StageRows", "step_begin", "step_stage", "dyt", "dyt_ref",

@@ -10,6 +10,7 @@ import os
 import torch
 
 from ._ext import check, hipk, on_gpu, ptr, stream_ptr
+from .gemm import Parts
 from .rope import v_block_tokens
 
 KV_BLOCK = 32  # tokens per cache block (fixed by the decode kernel)
@@ -309,7 +310,22 @@ def fused_rope_variant(variant: int, D: int, max_parts: int, max_blocks: int = 0
     return 1 if max_parts <= (128 if FUSED_SPLIT_MERGE else 1) else 0
 
 
-def paged_decode_attention_rope(qkv: torch.Tensor, positions: torch.Tensor, slots: torch.Tensor,
+QKV_PARTS = 4  # attention_decode.hip kQkvParts
+
+
+def decode_qkv_parts(B: int, Hkv: int, D: int, max_blocks: int, max_parts: int, max_wgs: int = 0) -> int:
+    """K slices' sums that ``paged_decode_attention_rope`` adds up itself, 0 where it wants rows: its kernel 1 does, for up to
+    64 rows.  us of a decode step of four layers, rows / sums: width 4096, 3 x 300 tokens 451 / 442, 8 x 500 465 / 453, 24 x
+    400 510 / 498, 32 x 1000 591 / 579, 48 x 300 553 / 537, 64 x 800 646 / 629; width 2048, 20 x 500 274 / 269, 48 x 1000 329 /
+    311, 64 x 300 297 / 275; beyond 64 rows the projection has filled the chip: 72 x 300 589 / 611, 96 x 300 621 / 640, 140 x
+    300 747 / 768."""
+    if B > 64 or not FUSED_ROPE:
+        return 0
+    variant = decode_variant(B, Hkv, D, max_blocks)
+    return QKV_PARTS if fused_rope_variant(variant, D, max_parts, max_blocks, max_wgs) == 1 else 0
+
+
+def paged_decode_attention_rope(qkv: torch.Tensor | Parts, positions: torch.Tensor, slots: torch.Tensor,
                                 cos_sin: torch.Tensor, Hq: int, Hkv: int, D: int,
                                 k_cache: torch.Tensor, v_cache: torch.Tensor,
                                 block_tables: torch.Tensor, context_lens: torch.Tensor,
@@ -323,25 +339,36 @@ def paged_decode_attention_rope(qkv: torch.Tensor, positions: torch.Tensor, slot
     of ``rope_kv_`` followed by ``paged_decode_attention``.  On the GPU one launch does it at
     head sizes 64 and 128 (``fused_rope_variant``); other shapes run the two ops.
     ``max_wgs`` > 0 caps the persistent grid at that many 4-wave workgroups (attention on
-    part of the chip, beside another stream's GEMMs; 0: two per CU)."""
+    part of the chip, beside another stream's GEMMs; 0: two per CU).  ``qkv`` may be the projection's ``Parts``
+    (``decode_qkv_parts``; added up ahead elsewhere)."""
     from .rope import rope_kv_
 
     B = qkv.shape[0]
-    q = qkv.as_strided((B, Hq, D), (qkv.stride(0), D, 1))
-    variant = decode_variant(B, Hkv, D, block_tables.shape[1]) if on_gpu(qkv) else 0
-    fused = 0
+    parts = None
+    if isinstance(qkv, Parts):
+        n = qkv.slab.shape[0]
+        if (on_gpu(qkv.slab) and 2 <= n <= QKV_PARTS and k_cache.data_ptr() % 16 == 0 and qkv.slab.is_contiguous()
+                and qkv.shape[1] % 4 == 0 and qkv.slab.data_ptr() % 16 == 0
+                and blocks_per_part is not None and workspace is not None
+                and n <= decode_qkv_parts(B, Hkv, D, block_tables.shape[1], workspace.max_parts, max_wgs)):
+            parts = qkv
+        else:
+            qkv = qkv.tensor()
+    fused = 1 if parts is not None else 0
     # staged into LDS: a row by whole words, K by 16-byte pieces
-    whole = qkv.data_ptr() % 4 == 0 and qkv.stride(0) % 2 == 0 and k_cache.data_ptr() % 16 == 0
-    if on_gpu(qkv) and FUSED_ROPE and whole:
+    if not fused and on_gpu(qkv) and FUSED_ROPE and qkv.data_ptr() % 4 == 0 and qkv.stride(0) % 2 == 0 and k_cache.data_ptr() % 16 == 0:
+        variant = decode_variant(B, Hkv, D, block_tables.shape[1])
         max_parts = (workspace.max_parts if blocks_per_part is not None and workspace is not None
                      else decode_partitioning(B, Hkv, block_tables.shape[1], variant=variant, D=D)[1])
         fused = fused_rope_variant(variant, D, max_parts, block_tables.shape[1], max_wgs)
     if not fused:
+        q = qkv.as_strided((B, Hq, D), (qkv.stride(0), D, 1))
         rope_kv_(qkv, positions, slots, cos_sin, Hq, Hkv, D, k_cache, v_cache, KV_BLOCK)
         return paged_decode_attention(q, k_cache, v_cache, block_tables, context_lens, scale,
                                       out=out, blocks_per_part=blocks_per_part,
                                       workspace=workspace)
-    assert qkv.dtype == torch.bfloat16 and qkv.stride(1) == 1
+    rows = qkv if parts is None else parts.slab
+    assert qkv.dtype == torch.bfloat16 and rows.stride(-1) == 1
     assert qkv.shape[1] >= (Hq + 2 * Hkv) * D
     nb, hkv, bs, D2 = k_cache.shape
     assert hkv == Hkv and bs == KV_BLOCK and D2 == D and k_cache.is_contiguous()
@@ -354,16 +381,16 @@ def paged_decode_attention_rope(qkv: torch.Tensor, positions: torch.Tensor, slot
     if blocks_per_part is None or workspace is None:
         blocks_per_part, max_parts = decode_partitioning(B, Hkv, block_tables.shape[1],
                                                          variant=variant, D=D)
-        workspace = DecodeWorkspace(B, Hq, D, max_parts, qkv.device)
+        workspace = DecodeWorkspace(B, Hq, D, max_parts, rows.device)
     if out is None:
-        out = torch.empty((B, Hq, D), dtype=qkv.dtype, device=qkv.device)
+        out = torch.empty((B, Hq, D), dtype=qkv.dtype, device=rows.device)
     assert out.is_contiguous() and out.shape == (B, Hq, D)
     check(hipk().paged_decode_rope(out.data_ptr(), ptr(workspace.part_o), ptr(workspace.part_ml),
-                                   qkv.data_ptr(), qkv.stride(0), k_cache.data_ptr(),
+                                   0 if parts else rows.data_ptr(), rows.stride(-2), k_cache.data_ptr(),
                                    v_cache.data_ptr(), block_tables.data_ptr(),
                                    block_tables.stride(0), context_lens.data_ptr(), B, Hq, Hkv, D,
                                    float(scale), workspace.max_parts, blocks_per_part,
                                    positions.data_ptr(), slots.data_ptr(), cos_sin.data_ptr(),
-                                   int(max_wgs), ptr(workspace.counters), fused,
-                                   stream_ptr(qkv)), "paged_decode_rope")
+                                   int(max_wgs), ptr(workspace.counters), fused, stream_ptr(rows),
+                                   rows.data_ptr() if parts else 0, rows.shape[0] if parts else 0), "paged_decode_rope")
     return out

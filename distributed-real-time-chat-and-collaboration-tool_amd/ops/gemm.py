@@ -635,15 +635,19 @@ def _norm_fused(p, w: torch.Tensor, act: int = -1):
     return y
 
 
-def norm_linear(p, w: torch.Tensor) -> torch.Tensor:
-    """y = rmsnorm(p.x [+ p.residual]) @ w.T for an ``ops.PendingNorm`` p.
+def norm_linear(p, w: torch.Tensor, parts: int = 0) -> torch.Tensor | Parts:
+    """y = rmsnorm(p.x [+ p.residual]) @ w.T for an ``ops.PendingNorm`` p; ``parts``: or the sums of up to that
+    many K slices (``linear_parts``).
 
     When the projection would run on the skinny dot2 kernel anyway (small decode batches,
     measured per shape) the norm is fused into it (gemv.hip ``skinny_norm_gemm_kernel``):
     one launch instead of two, and the new residual stream is written by the GEMM.
     Otherwise the norm is materialised and ``linear`` runs."""
     y = _norm_fused(p, w)
-    return linear(p.materialize(), w) if y is None else y
+    if y is not None:
+        return y
+    h = p.materialize()
+    return linear_parts(h, w, parts) if parts > 1 else linear(h, w)
 
 
 def norm_glu_row(p, w: torch.Tensor, act: str = "silu"):
@@ -1450,13 +1454,13 @@ class Parts:
 
 MAX_PARTS = 8  # common.h kMaxParts
 _parts_enabled = os.environ.get("DRTC_PARTS", "1") != "0"
-# (M, N, K) -> (16-column fragments, K slices) of ``linear_parts``, None: ``linear``
-_parts_forms: dict[tuple[int, int, int], tuple[int, int] | None] = {}
+# (M, N, K, most) -> (16-column fragments, K slices) of ``linear_parts``, None: ``linear``
+_parts_forms: dict[tuple[int, int, int, int], tuple[int, int] | None] = {}
 
 
-def parts_form(M: int, N: int, K: int) -> tuple[int, int] | None:
-    """How ``linear_parts`` cuts a product of M rows, None where ``linear`` is as fast.  us of ``linear`` as it was before
-    ``small_form`` / of the parts, to which reading them adds 0.3 - 2:
+def parts_form(M: int, N: int, K: int, most: int = MAX_PARTS) -> tuple[int, int] | None:
+    """How ``linear_parts`` cuts a product of M rows into up to ``most`` slices, None where ``linear`` is as fast.  us of
+    ``linear`` as it was before ``small_form`` / of the parts, to which reading them adds 0.3 - 2:
       K from 5120 on, 3 rows to 256: 4096 x 14336, 4 rows 22.7 / 19.8, 16 24.2 / 19.8, 64 28.3 / 22.7, 160 39.0 / 30.8, 256
         58.0 / 38.6; 2048 x 7168, 4 rows 11.0 / 7.4, 160 24.2 / 14.1; 2048 x 5632, 256 rows 20.9 / 16.0; two rows and one
         stay with the dot2 form (2048 x 7168 8.4 / 7.4, 7.5 / 7.3)
@@ -1471,14 +1475,14 @@ def parts_form(M: int, N: int, K: int) -> tuple[int, int] | None:
       and a product's rows would be rounded to 16 in between.
     The cut: the least of a workgroup's operands at 50 GB/s or its weights at 24, a quarter of a microsecond to
     a slice, and the parts read again by the whole chip or by a row's CU."""
-    key = (M, N, K)
+    key = (M, N, K, most)
     if key in _parts_forms:
         return _parts_forms[key]
     rows = (3, 256) if K >= 5120 else (3, 160) if K >= 4096 else (17, 128 if N <= 2048 else 64) if K >= 2048 else (1, 0)
     best = None
     if _parts_enabled and _midm_enabled and K % 64 == 0 and 1024 <= N <= 8192 and rows[0] <= M <= rows[1]:
         for nf in (2, 4):
-            for s in range(2, MAX_PARTS + 1):
+            for s in range(2, most + 1):
                 tiles = N // (32 * nf) * s
                 if N % (32 * nf) or tiles > 256 or K // 64 // s < 4:
                     continue
@@ -1491,13 +1495,13 @@ def parts_form(M: int, N: int, K: int) -> tuple[int, int] | None:
     return form
 
 
-def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | Parts:
-    """``linear``, or its K slices' sums (csrc/kernels/gemm_midm.hip) where ``parts_form`` says so."""
+def linear_parts(x: torch.Tensor, w: torch.Tensor, most: int = MAX_PARTS) -> torch.Tensor | Parts:
+    """``linear``, or the sums of up to ``most`` K slices (csrc/kernels/gemm_midm.hip) where ``parts_form`` says so."""
     if x.shape[0] > MIDM_MAX_M:  # (a prompt's host path is as long as its kernels up to some 600 rows)
         return linear(x, w)
     if _gpu_bf16(x, w) and w.shape[1] == x.shape[1] and _aligned(x, w):
         (M, K), N = x.shape, w.shape[0]
-        form = parts_form(M, N, K) if M * x.stride(0) < 1 << 30 else None
+        form = parts_form(M, N, K, most) if M * x.stride(0) < 1 << 30 else None
         if form is not None:
             nf, S = form
             slab = torch.empty((S, M, N), dtype=torch.float32, device=x.device)

@@ -311,6 +311,35 @@ def test_paged_decode_rope_workgroups(hipk, D, Hq, Hkv, parts, ctx_lens):
     assert parts == 1 or not ws.counters.any()
 
 
+@pytest.mark.parametrize("D,Hq,Hkv,bpp", [(128, 32, 8, 8), (64, 16, 2, 4), (128, 12, 4, 64), (64, 4, 4, 4)])
+@pytest.mark.parametrize("n", [2, 3, 4])
+def test_paged_decode_rope_of_slices(hipk, D, Hq, Hkv, bpp, n):
+    """q, k and v as the sums of the projection's K slices: the bits of the launch that takes their sum's rows, in
+    output and caches, contexts of one token to several partitions and padded rows among them."""
+    ctx_lens = [1, 2, 32, 33, 0, 65, 129, 257, 600]
+    B, N = len(ctx_lens), (Hq + 2 * Hkv) * D + 4 * n
+    _, kc, vc, bt, _ = _paged_setup(B, Hq, Hkv, D, [max(c, 1) for c in ctx_lens], seed=41)
+    cl = torch.tensor(ctx_lens, dtype=torch.int32, device=DEV)
+    slab = torch.randn(n, B, N, generator=torch.Generator().manual_seed(42)).to(DEV)
+    rows = slab[0].clone()
+    for i in range(1, n):
+        rows += slab[i]
+    pos = (cl - 1).clamp(min=0)
+    slots = torch.tensor([int(bt[b, p // 32]) * 32 + p % 32 if c else -1
+                          for b, (c, p) in enumerate(zip(ctx_lens, pos.tolist()))], device=DEV)
+    cs = ops.build_rope_cache(1024, D, 5e5, device=DEV)
+    parts = -(-bt.shape[1] // bpp)
+    assert ops.decode_qkv_parts(B, Hkv, D, bt.shape[1], parts) == 4
+    got = []
+    for qkv in (rows.to(torch.bfloat16), ops.Parts(slab, torch.bfloat16)):
+        k, v = kc.clone(), vc.clone()
+        out = ops.paged_decode_attention_rope(qkv, pos, slots, cs, Hq, Hkv, D, k, v, bt, cl, D ** -0.5, blocks_per_part=bpp,
+                                              workspace=ops.DecodeWorkspace(B, Hq, D, parts, DEV))
+        got.append((out, k, v))
+    for a, b, what in zip(*got, ("output", "k cache", "v cache")):
+        assert torch.equal(a, b), what
+
+
 @pytest.mark.parametrize("variant", [1, 2, 3])
 def test_paged_decode_strided_q_and_padding(hipk, variant):
     Hq, Hkv, D = 32, 8, 128
