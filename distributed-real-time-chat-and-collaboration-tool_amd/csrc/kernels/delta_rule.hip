@@ -750,17 +750,16 @@ __global__ __launch_bounds__(NTHR, 2) void delta_chunk_kernel(DeltaArgs a) {
 //                written as MFMA operands, 16 bytes per lane (ChainEntry)
 //   delta_chain  a workgroup per (portion, head, 16 CT value columns): its waves divide the key
 //                channels of S, kept as accumulator tiles; the partial products meet in LDS, wave ct
-//                forms R, U and O of column tile ct.  R and U of 16 tokens are one tile each, whose
-//                layout is also a B operand
+//                forms R, U and O of column tile ct (CT = 1: delta_chain_narrow).  R and U of 16
+//                tokens are one tile each, whose layout is also a B operand
 //   delta_read   output norm and gate, rings
 // The chain is bound by the fp32 MFMA (32 cycles each, 64 + 32 of them per chunk and column tile, over
 // NW waves) and by two exchanges through LDS.  Only the keys' products are ahead of the first: the queries' run while
 // the parts come back.  The operands of two chunks are under way at any time, which the compiler's waits count only
 // since nothing older than they is pending in the loop (S is waited for ahead of it, pointers are uniform): before, every
-// second chunk waited for all loads, 1.6 us per 16 tokens, now 1.0 at CT = 1 and 1.4 at CT = 2, 10.3 in delta_chunk,
-// whose five barriers also wait for the staging.  Heads of 128, 4 x 3,500 tokens, 16 heads: 640 us (prep 190,
-// chain 446 -> 387, read 64), delta_chunk 2,244; one portion of 4,000: 364 (chain 417 -> 262) against
-// 2,492.  With portions and heads enough for every CU delta_chunk keeps the fp32 units as busy without
+// second chunk waited for all loads, 1.6 us per 16 tokens, now 1.4 at CT = 2 (0.8 in delta_chain_narrow), 10.3 in
+// delta_chunk, whose five barriers also wait for the staging.  Heads of 128, 4 x 3,500 tokens, 16 heads: 615 us (prep 190,
+// chain 365, read 64), delta_chunk 2,244; one portion of 4,000: 300 (chain 205) against 2,492.  With portions and heads enough for every CU delta_chunk keeps the fp32 units as busy without
 // operands in memory (64 x 250, 32 heads: 959 against 1,249).
 // Chunks are numbered through the portions in their order: at most rows / 16 + nseg of them.
 template <int DT>
@@ -938,7 +937,7 @@ __global__ __launch_bounds__(256, 5) void delta_prep_kernel(DeltaArgs a, int h0)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float e = fast_exp2(c4[r]);
-        k4[r] *= e;
+        k4[r] *= -e;  // R = V - (E*K)^T S is a sum
         q4[r] *= e;
       }
       *(f32x4*)(w + E::ek + v * 4) = k4;
@@ -964,7 +963,7 @@ template <class T, int DT, int CT>
 __global__ __launch_bounds__(64 * chain_waves(DT), 2) void delta_chain_kernel(DeltaArgs a, int h0, int nh) {
   using E = ChainEntry<DT>;
   constexpr int NW = chain_waves(DT), TW = DT / NW;
-  static_assert(CT <= NW, "a wave to a column tile");
+  static_assert(CT > 1 && CT <= NW, "a wave to a column tile");
   __shared__ __attribute__((aligned(16))) float part[NW * 2 * CT * 256], us[CT * 256];
   const int seg = blockIdx.x / nh, hh = blockIdx.x % nh, h = h0 + hh;
   // uniform, and in scalar registers: the loads of a chunk advance a scalar pointer past fixed lane offsets
@@ -1000,10 +999,8 @@ __global__ __launch_bounds__(64 * chain_waves(DT), 2) void delta_chain_kernel(De
     for (int ct = 0; ct < CT; ++ct) asm volatile("" : "+v"(st[t][ct]));
   entry = uniform(entry);
   const float* p = a.ws + ((int64_t)entry * nh + hh) * E::N;
-  // a wave of its own for R, U and O of column tile wc
-  const int wc = (w + NW - (CT == 1 ? (blockIdx.y + blockIdx.y / NW * 2) % NW : 0)) % NW;
-  const bool lead = wc < CT;
-  const int xo = x0 + 16 * min(wc, CT - 1) + col;
+  const bool lead = w < CT;  // wave ct forms R, U and O of column tile ct
+  const int xo = x0 + 16 * min(w, CT - 1) + col;
   const T* v = (const T*)a.conv + (int64_t)row0 * a.C + 2 * a.Hk * a.dim + h * a.vdim;
   unsigned vrow[4], vlast[4];  // of a lane's rows of a chunk; of the last one, where rows behind the end are the last row
 #pragma unroll
@@ -1054,7 +1051,7 @@ __global__ __launch_bounds__(64 * chain_waves(DT), 2) void delta_chain_kernel(De
     load_u(odd, chunk(1));
   }
   float* mypart = part + w * 2 * CT * 256 + 4 * lane;
-  const float* sums = part + 256 * min(wc, CT - 1) + 4 * lane;
+  const float* sums = part + 256 * min(w, CT - 1) + 4 * lane;
   auto compute = [&](int c, Ops& x) {
     const float* ahead = chunk(c + 2);
     f32x4 rk[CT], ok[CT];
@@ -1088,10 +1085,10 @@ __global__ __launch_bounds__(64 * chain_waves(DT), 2) void delta_chain_kernel(De
       for (int i = 1; i < NW; ++i) rs[0] += rs[i];
       f32x4 u = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int r = 0; r < 4; ++r) res[r] = 16 * c + 4 * g + r < n ? to_f32(x.v[r]) - rs[0][r] : 0.f;
+      for (int r = 0; r < 4; ++r) res[r] = 16 * c + 4 * g + r < n ? to_f32(x.v[r]) + rs[0][r] : 0.f;
 #pragma unroll
       for (int r = 0; r < 4; ++r) u = mfma_f32(x.mu[r], res[r], u);
-      *(f32x4*)(us + 256 * wc + 4 * lane) = u;
+      *(f32x4*)(us + 256 * w + 4 * lane) = u;
     }
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) *(f32x4*)(mypart + 256 * (CT + ct)) = ok[ct];
@@ -1134,6 +1131,193 @@ __global__ __launch_bounds__(64 * chain_waves(DT), 2) void delta_chain_kernel(De
   if (nch & 1) compute(nch - 1, even);
   state([&](int t, int ct, int r, bool in, float* at) {
     if (in) *at = st[t][ct][r];
+  });
+}
+
+// The same with one column tile to a workgroup, for few chains: a chunk's serial path sets the time, so every wave forms R
+// and U itself (four MFMAs more, an exchange through LDS less), M_O R and the outputs are divided over the waves, a chunk's
+// outputs are summed beside the next one's products, and operands come through buffer descriptors that scalar adds move on
+// (with addresses in vector registers a chunk was 250 instructions of a wave that is alone on its SIMD, now 130).  One
+// workgroup to a CU: 16 chains of 4,000 tokens 253 -> 205 us, the MFMAs half of it, 32 156 -> 145; two and more to a CU:
+// 64 chains of 3,500 392 -> 365, 96 of 2,000 308 -> 277.  Two tiles in one workgroup, which reads the operands once: 315, 202,
+// 379, 354; operands four chunks ahead spill.
+template <class T, int DT>
+__global__ __launch_bounds__(64 * chain_waves(DT), 2) void delta_chain_narrow_kernel(DeltaArgs a, int h0, int nh) {
+  using E = ChainEntry<DT>;
+  constexpr int NW = chain_waves(DT), TW = DT / NW, RW = 4 / NW;
+  static_assert(NW * RW == 4, "the four rows of a lane to the waves");
+  // parts of the keys' and of the queries' products by chunk parity: one barrier a chunk
+  __shared__ __attribute__((aligned(16))) float part[2][2][NW * 256];
+  const int seg = blockIdx.x / nh, hh = blockIdx.x % nh, h = h0 + hh;
+  auto uniform = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+  const int slot = uniform(a.seg_state[seg]);
+  if (slot < 0) return;
+  const int n = uniform(a.seg_len[seg]), row0 = uniform(a.seg_row[seg]), pos0 = uniform(a.seg_pos[seg]);
+  const int nch = (n + 15) / 16;
+  const int w = wave_id_uniform(), lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
+  const int x0 = 16 * blockIdx.y;
+  int entry = 0;
+  for (int s = lane; s < seg; s += 64) entry += (a.seg_len[s] + 15) / 16;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) entry += __shfl_xor(entry, o, 64);
+  float* S = a.state + ((int64_t)slot * a.H + h) * a.dim * a.vdim;
+  auto state = [&](auto&& f) {
+#pragma unroll
+    for (int t = 0; t < TW; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int d = 16 * (TW * w + t) + 4 * g + r, x = x0 + col;
+        f(t, r, d < a.dim && x < a.vdim, S + (int64_t)d * a.vdim + x);
+      }
+  };
+  f32x4 st[TW];
+  state([&](int t, int r, bool in, float* at) { st[t][r] = pos0 > 0 && in ? *at : 0.f; });
+  // S is there before the loop: else its first use in there waits for all loads, those of the chunks ahead too
+#pragma unroll
+  for (int t = 0; t < TW; ++t) asm volatile("" : "+v"(st[t]));
+  entry = uniform(entry);
+  const char* ahead = (const char*)(a.ws + ((int64_t)entry * nh + hh) * E::N);  // chunk to load next, or the last one
+  const int64_t stride = (int64_t)nh * E::N * 4;
+  const unsigned vk = 1024 * TW * w + 16 * lane, vg = 64 * TW * w + 16 * g, vm = 16 * lane;
+  // Wave 0 starts the keys' sums with V: rows behind the portion's end, and all rows in the other waves, load as 0
+  const T* v = (const T*)a.conv + (int64_t)row0 * a.C + 2 * a.Hk * a.dim + h * a.vdim;
+  const unsigned vfull = uniform(w == 0 ? 16 * a.C * (int)sizeof(T) : 0);
+  const unsigned vtail = uniform(w == 0 ? (n - 16 * (nch - 1)) * a.C * (int)sizeof(T) : 0);
+  unsigned vv[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) vv[r] = ((4 * g + r) * a.C + min(x0 + col, a.vdim - 1)) * (unsigned)sizeof(T);
+  auto rsrc = [](const void* at, unsigned bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)at, (short)0, (int)bytes, 0x00020000);
+  };
+  auto ld = [](__amdgpu_buffer_rsrc_t b, unsigned off, unsigned soff) {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(b, off, soff, 0));
+  };
+  // operands of two chunks: each part is loaded again, two chunks ahead, where it has been read
+  struct Ops {
+    f32x4 ek[TW], eq[TW], kd[TW], gt[TW], mu;
+    float mo[RW];
+    unsigned v[4];  // a word each: packed in pairs, they would be waited for where they are loaded
+  };
+  auto load_k = [&](Ops& x) {
+    const auto b = rsrc(ahead, E::N * 4);
+#pragma unroll
+    for (int t = 0; t < TW; ++t) {
+      x.ek[t] = ld(b, vk + 1024 * t, 4 * E::ek);
+      x.eq[t] = ld(b, vk + 1024 * t, 4 * E::eq);
+    }
+  };
+  auto load_rest = [&](Ops& x, int c) {  // in the order of the chunks
+    const auto b = rsrc(ahead, E::N * 4);
+    x.mu = ld(b, vm, 4 * E::mu);
+#pragma unroll
+    for (int j = 0; j < RW; ++j)
+      x.mo[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(b, vm + 4 * (RW * w + j), 4 * E::mo, 0));
+    const auto bv = rsrc(v, c < nch - 1 ? vfull : c == nch - 1 ? vtail : 0);
+    v += 16 * a.C;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if constexpr (sizeof(T) == 2) x.v[r] = __builtin_amdgcn_raw_buffer_load_b16(bv, vv[r], 0, 0);
+      else x.v[r] = __builtin_amdgcn_raw_buffer_load_b32(bv, vv[r], 0, 0);
+    }
+#pragma unroll
+    for (int t = 0; t < TW; ++t) {
+      x.kd[t] = ld(b, vk + 1024 * t, 4 * E::kd);
+      x.gt[t] = ld(b, vg + 64 * t, 4 * E::gt);
+    }
+    ahead += c + 1 < nch ? stride : 0;
+  };
+  Ops even, odd;
+  if (nch > 0) {
+    load_k(even);
+    load_rest(even, 0);
+    load_k(odd);
+    load_rest(odd, 1);
+  }
+  // Outputs: rows 4 g + RW w + j are this wave's
+  const int64_t ldo = (int64_t)a.H * a.vdim16;
+  float* o = a.ws_o + (int64_t)(entry - 1) * 16 * ldo + h * a.vdim16;  // of the chunk ahead of the next one
+  const unsigned orow = 4 * ((4 * g + RW * w) * (unsigned)ldo + x0 + col);
+  auto read_out = [&](float (&ys)[RW][NW], const int par) {
+#pragma unroll
+    for (int j = 0; j < RW; ++j)
+#pragma unroll
+      for (int i = 0; i < NW; ++i) ys[j][i] = part[1][par][i * 256 + 4 * lane + RW * w + j];
+  };
+  auto write_out = [&](const float (&ys)[RW][NW], bool any) {
+    const auto b = rsrc(o, any ? 64 * (unsigned)ldo : 0);
+    o += 16 * ldo;
+#pragma unroll
+    for (int j = 0; j < RW; ++j) {
+      float y = ys[j][0];
+#pragma unroll
+      for (int i = 1; i < NW; ++i) y += ys[j][i];
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, y), b, orow, 4 * j * (unsigned)ldo, 0);
+    }
+  };
+  auto compute = [&](int c, Ops& x, const int par) {
+    f32x4 rk, ok, u;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      rk[r] = __builtin_bit_cast(float, sizeof(T) == 2 ? x.v[r] << 16 : x.v[r]);
+      ok[r] = u[r] = 0.f;
+    }
+    // the queries' products fill the waits for the keys' parts and for U
+    auto queries = [&](int lo, int hi) {
+#pragma unroll
+      for (int i = lo; i < hi; ++i) ok = mfma_f32(x.eq[i >> 2][i & 3], st[i >> 2][i & 3], ok);
+    };
+#pragma unroll
+    for (int t = 0; t < TW; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) rk = mfma_f32(x.ek[t][r], st[t][r], rk);
+    *(f32x4*)(part[0][par] + w * 256 + 4 * lane) = rk;
+    lds_barrier();
+    f32x4 rs[NW];
+#pragma unroll
+    for (int i = 0; i < NW; ++i) rs[i] = *(const f32x4*)(part[0][par] + i * 256 + 4 * lane);
+    float ys[RW][NW];
+    read_out(ys, 1 - par);  // of the chunk before; of none ahead of the first, whose store is out of range
+    __builtin_amdgcn_sched_barrier(0);
+    queries(0, 3 * TW);
+#pragma unroll
+    for (int i = 1; i < NW; ++i) rs[0] += rs[i];
+    if (16 * c + 16 > n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) rs[0][r] = 16 * c + 4 * g + r < n ? rs[0][r] : 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) u = mfma_f32(x.mu[r], rs[0][r], u);
+    queries(3 * TW, 4 * TW);
+    load_k(x);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < TW; ++t) st[t] *= x.gt[t];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int t = 0; t < TW; ++t) st[t] = mfma_f32(x.kd[t][r], u[r], st[t]);
+#pragma unroll
+    for (int j = 0; j < RW; ++j) {  // M_O R: a k-step to each wave
+      const f32x4 y = rs[0];
+      ok = mfma_f32(x.mo[j], RW == 1 ? w & 2 ? w & 1 ? y[3] : y[2] : w & 1 ? y[1] : y[0] : w ? y[2 + j] : y[j], ok);
+    }
+    *(f32x4*)(part[1][par] + w * 256 + 4 * lane) = ok;
+    load_rest(x, c + 2);
+    write_out(ys, c > 0);
+  };
+#pragma unroll 1
+  for (int c = 0; c + 1 < nch; c += 2) {
+    compute(c, even, 0);
+    compute(c + 1, odd, 1);
+  }
+  if (nch & 1) compute(nch - 1, even, 0);
+  lds_barrier();
+  if (nch > 0) {
+    float ys[RW][NW];
+    read_out(ys, (nch - 1) & 1);
+    write_out(ys, true);
+  }
+  state([&](int t, int r, bool in, float* at) {
+    if (in) *at = st[t][r];
   });
 }
 
@@ -1380,10 +1564,10 @@ static int chain_go(const DeltaArgs& a, hipStream_t st) {
       kernel<<<dim3(a.nseg * m, (a.vdim16 + columns - 1) / columns), dim3(64 * NW), 0, st>>>(a, h0, m);
     };
     // The fewest columns to a workgroup wait least between its products and overlap with a CU's other ones; more
-    // read the operands less often.  Heads of 128, us with 16 / 32 columns: 16 chains of 4,000 tokens 262 / 371, 32 of 868
-    // 64 / 86, 64 of 3,500 387 / 390, 96 of 2,000 334 / 358, 144 of 1,000 269 / 231.
+    // read the operands less often.  Heads of 128, us with 16 / 32 columns: 16 chains of 4,000 tokens 205 / 371, 32 of 868
+    // 55 / 86, 64 of 3,500 365 / 390, 96 of 2,000 277 / 358; with 16 / 64 columns 144 of 1,000 234 / 213.
     const int64_t chains = (int64_t)a.nseg * m;
-    if (chains * ((a.vdim16 + 15) / 16) <= 768) go(delta_chain_kernel<T, DT, 1>, 16);
+    if (chains * ((a.vdim16 + 15) / 16) <= 768) go(delta_chain_narrow_kernel<T, DT>, 16);
     else if (NW == 4 && chains * ((a.vdim16 + 63) / 64) >= 512) go(delta_chain_kernel<T, DT, NW>, 16 * NW);
     else go(delta_chain_kernel<T, DT, 2>, 32);
   }
