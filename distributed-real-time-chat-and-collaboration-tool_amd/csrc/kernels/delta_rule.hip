@@ -1138,7 +1138,7 @@ __global__ __launch_bounds__(64 * chain_waves(DT), 2) void delta_chain_kernel(De
 // and U itself (four MFMAs more, an exchange through LDS less), M_O R and the outputs are divided over the waves, a chunk's
 // outputs are summed beside the next one's products, and operands come through buffer descriptors that scalar adds move on
 // (with addresses in vector registers a chunk was 250 instructions of a wave that is alone on its SIMD, now 130).  One
-// workgroup to a CU: 16 chains of 4,000 tokens 253 -> 205 us, the MFMAs half of it, 32 156 -> 145; two and more to a CU:
+// workgroup to a CU: 16 chains of 4,000 tokens 253 -> 205 us, the MFMAs half of it, 32 262 -> 245; more to a CU:
 // 64 chains of 3,500 392 -> 365, 96 of 2,000 308 -> 277.  Two tiles in one workgroup, which reads the operands once: 315, 202,
 // 379, 354; operands four chunks ahead spill.
 template <class T, int DT>
@@ -1565,7 +1565,7 @@ static int chain_go(const DeltaArgs& a, hipStream_t st) {
     };
     // The fewest columns to a workgroup wait least between its products and overlap with a CU's other ones; more
     // read the operands less often.  Heads of 128, us with 16 / 32 columns: 16 chains of 4,000 tokens 205 / 371, 32 of 868
-    // 55 / 86, 64 of 3,500 365 / 390, 96 of 2,000 277 / 358; with 16 / 64 columns 144 of 1,000 234 / 213.
+    // 50 / 86, 64 of 3,500 365 / 390, 96 of 2,000 277 / 358; with 16 / 64 columns 144 of 1,000 234 / 213.
     const int64_t chains = (int64_t)a.nseg * m;
     if (chains * ((a.vdim16 + 15) / 16) <= 768) go(delta_chain_narrow_kernel<T, DT>, 16);
     else if (NW == 4 && chains * ((a.vdim16 + 63) / 64) >= 512) go(delta_chain_kernel<T, DT, NW>, 16 * NW);

@@ -706,8 +706,8 @@ __global__ __launch_bounds__(64 * NH * ND, 2) void latent_decode_kernel(LatentDe
 // straight into LDS, by loads that the waves wait for by count, while the two before them are worked on; each of a head
 // tile's ND waves takes 64 / ND of the 64 tokens' scores and hands them to the others through LDS, where the form above
 // has every wave compute them all.  Chunk c (16 bytes) of row t lies at c ^ (t / 2 % 8).  That form was bound
-// by each block's chain - the scores' LDS reads fourfold, one wave a SIMD, two barriers for 64 tokens in both: 200
-// sequences of 500 tokens, 16 heads of 512 + 64: 47 -> 33 us; 64 of 1500, 32 heads, four splits: 28.4 -> 26.6.
+// by each block's chain - the scores' LDS reads fourfold, one wave a SIMD, two barriers for 64 tokens in both: 64
+// sequences of 1500 tokens, 48 heads of 512 + 64 38.6 us alone.
 template <int RT, int NH, int ND>
 struct LatPair {
   static constexpr int KS = 2 * RT + 2, LW = 32 * KS, CPR = LW / 8, NW = NH * ND;
@@ -851,6 +851,169 @@ __global__ __launch_bounds__(64 * NH * ND, 1) void latent_decode_pair_kernel(Lat
   lat_decode_out<RT, ND>(a, b, h, sp, nparts, dw, g, R, o, m, lsum);
 }
 
+// The same for latents of 512 and up to 32 heads, a block at a time, three more on their way: what a CU takes in never waits
+// for a barrier.  A wave's scores are 16 of the block's tokens over one half of the columns; V's operands are read during the
+// softmax, K's ahead of their products, and blocks inside the context are not masked.  200 sequences of 500 tokens, 16
+// heads: 33 -> 29 us in the pass (5.1 TB/s behind 6.5 us of launch and first loads, which a context of one block takes), alone 25.6 -> 23.4,
+// 256 x 400 25.2 -> 22.7, 64 x 1500 27.3 -> 25.2; 32 heads, 200 x 30 10.7 -> 9.3, 256 x 400 29.2 -> 26.9, 200 x 500 29.6 / 29.7, window of
+// 1024 64 x 1500 29.4 / 28.8.  Slower than pairs for latents of 256 (16 heads 200 x 500 16.6 / 17.8, 32 18.8 / 22.6: two barriers for half the
+// tokens) and for more heads (64 x 1500 of 48 38.6 / 40.5: registers for fewer reads ahead), which keep them.
+template <int NH>
+struct LatRing {
+  static constexpr int RT = 8, ND = 4, KS = 2 * RT + 2, LW = 32 * KS, CPR = LW / 8, NW = NH * ND, ST = 4;
+  static constexpr int TILE = kLB * LW;                                // elements of a block
+  static constexpr size_t BYTES = (size_t)ST * TILE * 2 + 1024 * NW;   // and [NW][64] f32x4 of scores
+};
+// the largest of the lanes 16 apart
+DRTC_DEVICE float rows_max(float v) {
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+template <int NH>
+__global__ __launch_bounds__(256 * NH, 2) void latent_decode_ring_kernel(LatentDecodeArgs a) {
+  using L = LatRing<NH>;
+  constexpr int LW = L::LW, RT = L::RT, ND = L::ND, R = 64 * RT, NTW = 4 * RT / ND, ST = L::ST, KS = L::KS / 2;
+  constexpr int LOADS = 2 * L::KS, DP = LOADS / L::NW;   // loads of 1 KiB to a block, and to a wave (the first ones one more)
+  constexpr int MORE = LOADS % L::NW, DM = DP + (MORE > 0);
+  extern __shared__ __attribute__((aligned(16))) bf16_t lat_lds[];
+  f32x4* const scores = reinterpret_cast<f32x4*>(lat_lds + ST * L::TILE);
+  const int b = blockIdx.x, sp = blockIdx.z;
+  const int w = wave_id_uniform(), lane = threadIdx.x & 63;
+  const int hw = w / ND, dw = w % ND, grp = dw & 1, s0 = (dw >> 1) * KS;
+  const int col = lane & 15, g = lane >> 4;
+  const int h = (blockIdx.y * NH + hw) * 16 + col;
+  bf16x8 qf[KS];
+  const bf16_t* qp = (const bf16_t*)a.qa + ((int64_t)b * a.H + min(h, a.H - 1)) * LW;
+#pragma unroll
+  for (int s = 0; s < KS; ++s) qf[s] = load_bf16x8(qp + 32 * (s0 + s) + 8 * g);  // (rows past the heads: not stored)
+  // without a window the first blocks' table entries need not wait for the context's length (those behind it are not used)
+  const int* bt = a.block_tables + (int64_t)b * a.bt_stride;
+  int table = a.window > 0 ? 0 : bt[min(sp * a.tiles_per_split + lane, a.bt_stride - 1)];
+  const int ctx = a.context_lens[b];
+  if (ctx <= 0) {
+    if (sp == 0 && h < a.H)
+      for (int i = dw * 4 + g; i < R; i += 4 * ND)
+        ((bf16_t*)a.out)[((int64_t)b * a.H + h) * R + i] = f2bf(0.f);
+    return;
+  }
+  const int lo = a.window > 0 ? max(0, ctx - a.window) : 0;
+  const int t0 = lo / kLB, t1 = (ctx + kLB - 1) / kLB;
+  const int nparts = (t1 - t0 + a.tiles_per_split - 1) / a.tiles_per_split;
+  const int tb = t0 + sp * a.tiles_per_split, te = min(t1, tb + a.tiles_per_split);
+  if (tb >= te) return;
+  // the table, 64 entries ahead, a lane each; waited for here, not where it is read among the ring's loads
+  int table_at = tb;
+  auto next_table = [&](int t) {
+    table_at = t;
+    table = t + lane < te ? bt[t + lane] : 0;
+    asm volatile("" : "+v"(table)::"memory");
+  };
+  if (a.window > 0) next_table(tb);
+  else asm volatile("" : "+v"(table)::"memory");
+#pragma unroll
+  for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(qf[s])::"memory");
+  // load j of a block, of 1 KiB; wave w takes j = w, w + NW, ...
+  unsigned voff[DM];
+#pragma unroll
+  for (int i = 0; i < DM; ++i) {
+    const int c = 64 * (i * L::NW + w) + lane, t = c / L::CPR, p = c - t * L::CPR;
+    voff[i] = (unsigned)(t * L::CPR + (p ^ (t / 2 % 8))) * 16u;
+  }
+  const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(lds_ptr)lat_lds);
+  auto fetch = [&](int t) {
+    if (t - table_at >= 64) next_table(t);
+    const __amdgpu_buffer_rsrc_t rows =
+        dma_rsrc((const bf16_t*)a.cache + (int64_t)__builtin_amdgcn_readlane(table, t - table_at) * L::TILE);
+    const unsigned to = lds0 + (unsigned)((t - tb) % ST) * (L::TILE * 2) + 1024u * w;
+#pragma unroll
+    for (int i = 0; i < DM; ++i)
+      if (i < DP || w < MORE) dma16<true>(to + 1024u * (i * L::NW), voff[i], rows, 0u);
+  };
+#pragma unroll 1
+  for (int t = tb; t < min(tb + ST - 1, te); ++t) fetch(t);
+  f32x4 o[NTW];
+#pragma unroll
+  for (int i = 0; i < NTW; ++i) o[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  float m = kNegBig, lsum = 0.f;
+  const float sl2 = a.scale * kLog2e;
+  const int tr_row = (col >> 2) + 4 * g, tr_x = tr_row / 2 % 8, key_x = col / 2 % 8;
+  for (int t = tb; t < te; ++t) {
+    const bf16_t* kb = lat_lds + (t - tb) % ST * L::TILE;
+    const int younger = min(ST - 2, te - 1 - t);
+    if (w < MORE) wait_groups<DM, ST - 2>(younger);
+    else wait_groups<DP, ST - 2>(younger);
+    lds_barrier();  // the block has landed, and everyone is through with the block before and its scores
+    if (t + ST - 1 < te) fetch(t + ST - 1);
+    {  // tokens 16 grp .. of the block
+      f32x4 part[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+      const bf16_t* row = kb + (16 * grp + col) * LW;
+      bf16x8 kf[KS];
+#pragma unroll
+      for (int s = 0; s < KS; ++s) kf[s] = load_bf16x8(row + ((4 * (s0 + s) + g) ^ key_x) * 8);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < KS; ++s) part[s & 1] = mfma16(kf[s], qf[s], part[s & 1]);
+      scores[w * 64 + lane] = part[0] + part[1];
+    }
+    lds_barrier();
+    f32x4 sc[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) sc[q] = scores[(hw * ND + q) * 64 + lane] + scores[(hw * ND + 2 + q) * 64 + lane];
+    __builtin_amdgcn_sched_barrier(0);
+    bf16x8 vf[NTW];
+#pragma unroll
+    for (int i = 0; i < NTW; ++i) {
+      const int c = (2 * (NTW * dw + i) + ((col & 3) >> 1)) ^ tr_x;
+      const bf16_t* at = kb + tr_row * LW + c * 8 + 4 * (col & 1);
+      const bf16x4 x = lat_read_tr16(at), y = lat_read_tr16(at + 16 * LW);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) { vf[i][j] = x[j]; vf[i][4 + j] = y[j]; }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const bool whole = t * kLB >= lo && (t + 1) * kLB <= ctx;
+    float bmax = kNegBig;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      if (!whole) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int pos = t * kLB + 16 * q + 4 * g + r;
+          sc[q][r] = pos >= lo && pos < ctx ? sc[q][r] * sl2 : kNegBig;
+        }
+      } else {
+        sc[q] *= sl2;
+      }
+      bmax = fmaxf(bmax, fmaxf(fmaxf(sc[q][0], sc[q][1]), fmaxf(sc[q][2], sc[q][3])));
+    }
+    bmax = rows_max(bmax);
+    const float m_new = fmaxf(m, bmax);  // every block of a split holds a visible token
+    const float alpha = fast_exp2(m - m_new);
+    const bool moved = __any(m_new > m);
+    m = m_new;
+    bf16x8 pf;
+    float psum = 0.f;
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float p = fast_exp2(sc[q][r] - m_new);
+        psum += p;
+        pf[4 * q + r] = f2bf(p);
+      }
+    lsum = lsum * alpha + psum;
+    if (moved) {
+#pragma unroll
+      for (int i = 0; i < NTW; ++i) o[i] *= alpha;
+    }
+#pragma unroll
+    for (int i = 0; i < NTW; ++i) o[i] = mfma16(vf[i], pf, o[i]);
+  }
+  lat_decode_out<RT, ND>(a, b, h, sp, nparts, dw, g, R, o, m, lsum);
+}
+
 // Merge of the window splits (and the sink): one workgroup per (sequence, head).
 __global__ __launch_bounds__(128) void latent_merge_kernel(LatentDecodeArgs a) {
   const int b = blockIdx.x, h = blockIdx.y;
@@ -879,6 +1042,8 @@ __global__ __launch_bounds__(128) void latent_merge_kernel(LatentDecodeArgs a) {
   }
 }
 
+template <int RT, int NH>
+constexpr bool lat_ring = RT == 8 && NH <= 2;
 template <int RT, int NH, int ND>
 static void lat_decode_go(const LatentDecodeArgs& a, hipStream_t st) {
   const size_t lds = (size_t)2 * kLB * (a.LW + kLatPad) * 2;
@@ -887,7 +1052,10 @@ static void lat_decode_go(const LatentDecodeArgs& a, hipStream_t st) {
     // (into LDS by whole 16-byte pieces)
     if (a.R == 64 * RT && a.LW == 32 * (2 * RT + 2) && (uintptr_t)a.cache % 16 == 0) {
       constexpr int NP = NH == 2 ? 4 : ND;  // eight waves where the heads fill two tiles
-      latent_decode_pair_kernel<RT, NH, NP><<<grid, dim3(64 * NH * NP), LatPair<RT, NH, NP>::BYTES, st>>>(a);
+      if constexpr (lat_ring<RT, NH>)
+        latent_decode_ring_kernel<NH><<<grid, dim3(256 * NH), LatRing<NH>::BYTES, st>>>(a);
+      else
+        latent_decode_pair_kernel<RT, NH, NP><<<grid, dim3(64 * NH * NP), LatPair<RT, NH, NP>::BYTES, st>>>(a);
       return;
     }
     if (a.R == 64 * RT && a.LW == 32 * (2 * RT + 1)) {
@@ -1256,8 +1424,12 @@ static int lat_decode_attr() {
 }
 template <int RT, int NH, int ND>
 static int lat_pair_attr() {
-  return (int)hipFuncSetAttribute((const void*)latent_decode_pair_kernel<RT, NH, ND>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)LatPair<RT, NH, ND>::BYTES);
+  if constexpr (lat_ring<RT, NH>)
+    return (int)hipFuncSetAttribute((const void*)latent_decode_ring_kernel<NH>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)LatRing<NH>::BYTES);
+  else
+    return (int)hipFuncSetAttribute((const void*)latent_decode_pair_kernel<RT, NH, ND>,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)LatPair<RT, NH, ND>::BYTES);
 }
 template <int NH, int ND>
 static int lat_decode_lds() {

@@ -1029,6 +1029,33 @@ def test_latent_decode_in_pairs_of_blocks(H, R, parts):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H", [16, 17, 32])
+@pytest.mark.parametrize("parts", [1, 2])
+def test_latent_decode_a_block_at_a_time(H, parts):
+    """Latents of 512, up to 32 heads: from one block to more than the LDS holds twice, whole last blocks and ones of one
+    token; table entries behind a context, which are read, lead nowhere.  Rounding of the test above."""
+    R, rot, nb, dev = 512, 64, 10, "cuda"
+    LW = ops.latent_width(R, rot)
+    ctx = [n for blocks in range(1, 10) for n in (32 * blocks, 32 * blocks - 31)]
+    B, g = len(ctx), torch.Generator().manual_seed(H)
+    cache = torch.randn(B * nb + 1, 32, LW, generator=g).mul_(0.5).to(torch.bfloat16)
+    bt = torch.randperm(B * nb, generator=g).view(B, nb).to(torch.int32) + 1
+    far = bt.clone()
+    for b, n in enumerate(ctx):
+        far[b, -(-n // 32):] = 2 ** 30
+    qa = torch.randn(B, H, LW, generator=g).mul_(0.5).to(torch.bfloat16)
+    for window in (None, 33, 200):
+        ws = ops.LatentDecodeWorkspace(B, H, R, window, nb, dev)
+        ws.per, ws.splits = -(-nb // parts), parts
+        ws.part_o, ws.part_ml = torch.empty(B, H, parts, R, device=dev), torch.empty(B, H, parts, 2, device=dev)
+        out = ops.latent_decode_attention(qa.to(dev), cache.to(dev), R, far.to(dev),
+                                          torch.tensor(ctx, dtype=torch.int32, device=dev), window, 0.05, None, ws)
+        for b, n in enumerate(ctx):
+            rows = cache[bt[b].long()].reshape(-1, LW)[max(0, n - (window or n)):n].double()
+            close(out[b], (qa[b].double() @ rows.T * 0.05).softmax(-1) @ rows[:, :R], 2e-2)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("B", [1, 3, 16, 17, 65])
 @pytest.mark.parametrize("H,R,dim,vdim,splits,gated", [(16, 512, 128, 128, 20, True), (4, 256, 128, 40, 3, False),
                                                         (5, 128, 256, 64, 2, True), (20, 448, 128, 128, 4, True),
