@@ -758,8 +758,9 @@ __global__ __launch_bounds__(NTHR, 2) void delta_chunk_kernel(DeltaArgs a) {
 // the parts come back.  The operands of two chunks are under way at any time, which the compiler's waits count only
 // since nothing older than they is pending in the loop (S is waited for ahead of it, pointers are uniform): before, every
 // second chunk waited for all loads, 1.6 us per 16 tokens, now 1.4 at CT = 2 (0.8 in delta_chain_narrow), 10.3 in
-// delta_chunk, whose five barriers also wait for the staging.  Heads of 128, 4 x 3,500 tokens, 16 heads: 615 us (prep 190,
-// chain 365, read 64), delta_chunk 2,244; one portion of 4,000: 300 (chain 205) against 2,492.  With portions and heads enough for every CU delta_chunk keeps the fp32 units as busy without
+// delta_chunk, whose five barriers also wait for the staging.  Heads of 128, 4 x 3,500 tokens, 16 heads: 605 us (prep 173,
+// chain 365, read 64), delta_chunk 2,244; one portion of 4,000: 290 (chain 205) against 2,492.  With portions and heads enough
+// for every CU delta_chunk keeps the fp32 units as busy without
 // operands in memory (64 x 250, 32 heads: 959 against 1,249).
 // Chunks are numbered through the portions in their order: at most rows / 16 + nseg of them.
 template <int DT>
@@ -862,50 +863,76 @@ __global__ __launch_bounds__(256, 5) void delta_prep_kernel(DeltaArgs a, int h0)
     }
   }
   __syncthreads();
-  // A and B: 16 lanes to a block of 4 x 4 pairs, every lane its channels; ten blocks of the lower
-  // triangle (a pair per lane read five vectors of LDS for every product, and took 130 us of 190)
-  if (tid < 160) {
-    const int blk = tid >> 4, l16 = tid & 15;
-    const int bi = blk < 1 ? 0 : blk < 3 ? 1 : blk < 6 ? 2 : 3, bj = blk - bi * (bi + 1) / 2;
-    float A[4][4], B[4][4];
+  // A and B: 32 lanes to a block of 4 x 4 pairs, a lane four channels.  Of two blocks apart the decay is cut at the later one's
+  // first token, 2^{c_i - c_r} 2^{c_r - c_j}: 8 exponentials for 16 pairs, none of them above 1.  Waves 0 .. 2 take these, wave 3
+  // the four blocks of neighbours.  (16 lanes to a block and an exponential a pair, on two waves and a half, left the last
+  // SIMD idle.  Heads of 128, 16 heads, 4 x 3,500 tokens 194 -> 173 us, 2.2 TB/s of operands written, 4,000 61 -> 52, 868 x 2 33 -> 29;
+  // two or four heads to a workgroup, each head's rows asked for ahead of the one before, are no faster: 174, 177.)
+  {
+    const int wv = tid >> 6, half = (tid >> 5) & 1, d = 4 * (tid & 31), l16 = tid & 15;
+    auto at4 = [&](const float* m, int t) { return d < DP ? *(const f32x4*)(m + t * DS + d) : (f32x4){0.f, 0.f, 0.f, 0.f}; };
+    auto exp4 = [](f32x4 x) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+      for (int m = 0; m < 4; ++m) x[m] = fast_exp2(x[m]);
+      return x;
+    };
+    auto dot4 = [](f32x4 x, f32x4 y) { return x[0] * y[0] + x[1] * y[1] + x[2] * y[2] + x[3] * y[3]; };
+    // lanes of 16: sums of A, the next 16 lanes of B; then a pair to a lane
+    auto put = [&](const float (&A)[16], const float (&B)[16], int bi, int bj) {
+      float x = 0.f;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) A[i][j] = B[i][j] = 0.f;
-#pragma unroll 1
-    for (int d = 4 * l16; d < DP; d += 64) {
-      f32x4 xj[4], zj[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        xj[j] = *(const f32x4*)(ks + (4 * bj + j) * DS + d);
-        zj[j] = *(const f32x4*)(cs + (4 * bj + j) * DS + d);
+      for (int e = 0; e < 16; ++e) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(A[e]), __float_as_uint(B[e]), false, false);
+        const float v = sum_lanes<16>(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+        x = l16 == e ? v : x;
       }
+      (tid & 16 ? bm : am)[4 * bi + (l16 >> 2)][4 * bj + (l16 & 3)] = x;
+    };
+    float A[16], B[16];
+    if (wv < 3) {
+      const int blk = 2 * wv + half, bi = blk < 1 ? 1 : blk < 3 ? 2 : 3, bj = blk - (blk < 1 ? 0 : blk < 3 ? 1 : 3);
+      const f32x4 cr = at4(cs, 4 * bi);
+      f32x4 y[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[j] = at4(ks, 4 * bj + j) * exp4(cr - at4(cs, 4 * bj + j));
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const f32x4 k4 = *(const f32x4*)(ks + (4 * bi + i) * DS + d);
-        const f32x4 q4 = *(const f32x4*)(qs + (4 * bi + i) * DS + d);
-        const f32x4 c4 = *(const f32x4*)(cs + (4 * bi + i) * DS + d);
+        f32x4 k4 = at4(ks, 4 * bi + i), q4 = at4(qs, 4 * bi + i);
+        if (i > 0) {
+          const f32x4 e = exp4(at4(cs, 4 * bi + i) - cr);
+          k4 *= e;
+          q4 *= e;
+        }
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int m = 0; m < 4; ++m) {
-            const float y = xj[j][m] * fast_exp2(fminf(c4[m] - zj[j][m], 0.f));
-            A[i][j] += k4[m] * y;
-            B[i][j] += q4[m] * y;
-          }
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        A[i][j] = sum_lanes<16>(A[i][j]);
-        B[i][j] = sum_lanes<16>(B[i][j]);
-        if (l16 == 4 * i + j) {
-          am[4 * bi + i][4 * bj + j] = A[i][j];
-          bm[4 * bi + i][4 * bj + j] = B[i][j];
+        for (int j = 0; j < 4; ++j) {
+          A[4 * i + j] = dot4(k4, y[j]);
+          B[4 * i + j] = dot4(q4, y[j]);
         }
       }
+      put(A, B, bi, bj);
+    } else {
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        const int bi = 2 * n + half;
+        f32x4 x[4], z[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          x[j] = at4(ks, 4 * bi + j);
+          z[j] = at4(cs, 4 * bi + j);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const f32x4 q4 = at4(qs, 4 * bi + i);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const f32x4 y = j < i ? x[j] * exp4(z[i] - z[j]) : x[j];
+            A[4 * i + j] = j < i ? dot4(x[i], y) : 0.f;
+            B[4 * i + j] = j <= i ? dot4(q4, y) : 0.f;
+          }
+        }
+        put(A, B, bi, bi);
+      }
+    }
   }
   __syncthreads();
   if (tid < 64) {  // column tid & 15 of M_U by forward substitution; four rows of it of M_O = B M_U

@@ -361,6 +361,28 @@ def test_delta_decode_state_ahead(hipk, dt, H, Hk, d, dv, taps):
     assert ((sg.cpu() - state).abs() <= tol * (1 + state.abs()))[state.isfinite()].all() and sg.isfinite().all()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("shift", [-6.0, 2.0, 12.0, 90.0])
+@pytest.mark.parametrize("d", [128, 64, 24])
+def test_delta_chains_of_any_decay(shift, d):
+    """Decays of a token from hardly any to more than an exponent holds, mixed over channels, in chunks prepared ahead against
+    token by token; sums of up to 128 products of unit vectors in fp32: 5e-5 as above."""
+    H, dv, taps, n, dev = 3, 40, 3, 83, "cuda"
+    g = torch.Generator().manual_seed(d)
+    r = lambda *shape: torch.randn(*shape, generator=g).to(dev)
+    C = 2 * H * d + H * dv
+    w = ops.DeltaWeights(r(taps, C), torch.linspace(-1, 1, H).exp().to(dev), shift * torch.rand(H * d, generator=g).to(dev), 1 + 0.1 * r(dv),
+                         1e-5, H, H, d, dv)
+    proj, decay, gate, ring = r(n, C + 8), r(n, H * d), r(n, H * dv), r(1, taps, C)
+    p, pos = _portions(dev, [n], [0], [0])
+    conv = ops.short_conv(proj, w, ring, pos, p)
+    assert ops.delta._chain_ok(w, decay, gate, p)
+    got, want = (ops.delta_scan(proj, C, conv, w, ring.clone(), s, decay, gate, p, c)
+                 for s, c in ((torch.zeros(1, H, d, dv, device=dev), 0), (torch.zeros(1, H, d, dv, device=dev), 2)))
+    assert got.isfinite().all()
+    close(got, want.double().cpu(), 5e-5)
+
+
 @on
 @pytest.mark.parametrize("case", CHAIN_CASES, ids=str)
 def test_delta_chains(target, case, monkeypatch):
