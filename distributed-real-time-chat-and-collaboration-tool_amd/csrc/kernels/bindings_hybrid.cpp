@@ -151,7 +151,7 @@ void bind_hybrid(py::module_& m) {
     const Fields f{d};
     drtc::LatentDecodeArgs a{};
     PTR(out); PTR(part_o); PTR(part_ml); PTR(qa); PTR(cache); PTR(block_tables); VAL(bt_stride);
-    PTR(context_lens); VAL(B); VAL(H); VAL(R); VAL(LW); VAL(window); VAL(tiles_per_split);
+    VAL(bt_cols); PTR(context_lens); VAL(B); VAL(H); VAL(R); VAL(LW); VAL(window); VAL(tiles_per_split);
     VAL(nsplits); VAL(scale); PTR(sink); PTR(gate); VAL(ldg);
     return w ? drtc::launch_latent_decode_up(f32, a, P<void>(y), P<void>(w), N, yb, yh, S(st))
              : drtc::launch_latent_decode(f32, a, S(st));

@@ -65,7 +65,7 @@ struct LatentDecodeArgs {
   const void* qa;         // [B, H, LW]
   const void* cache;
   const int* block_tables;
-  int bt_stride;
+  int bt_stride, bt_cols;  // elements from row to row, and of a row
   const int* context_lens;
   int B, H, R, LW, window, tiles_per_split, nsplits;
   float scale;

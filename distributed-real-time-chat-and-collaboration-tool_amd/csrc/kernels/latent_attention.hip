@@ -891,7 +891,7 @@ __global__ __launch_bounds__(256 * NH, 2) void latent_decode_ring_kernel(LatentD
   for (int s = 0; s < KS; ++s) qf[s] = load_bf16x8(qp + 32 * (s0 + s) + 8 * g);  // (rows past the heads: not stored)
   // without a window the first blocks' table entries need not wait for the context's length (those behind it are not used)
   const int* bt = a.block_tables + (int64_t)b * a.bt_stride;
-  int table = a.window > 0 ? 0 : bt[min(sp * a.tiles_per_split + lane, a.bt_stride - 1)];
+  int table = a.window > 0 || a.bt_cols < 1 ? 0 : bt[min(sp * a.tiles_per_split + lane, a.bt_cols - 1)];
   const int ctx = a.context_lens[b];
   if (ctx <= 0) {
     if (sp == 0 && h < a.H)

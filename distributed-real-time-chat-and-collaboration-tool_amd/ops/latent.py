@@ -319,7 +319,7 @@ def latent_decode_attention(qa: torch.Tensor, cache: torch.Tensor, kv_rank: int,
     check(hipk().latent_decode(int(qa.dtype == torch.float32), dict(
         out=out.data_ptr(), part_o=ptr(ws.part_o), part_ml=ptr(ws.part_ml), qa=qa.data_ptr(),
         cache=cache.data_ptr(), block_tables=block_tables.data_ptr(),
-        bt_stride=block_tables.stride(0), context_lens=context_lens.data_ptr(), B=B, H=H,
+        bt_stride=block_tables.stride(0), bt_cols=block_tables.shape[1], context_lens=context_lens.data_ptr(), B=B, H=H,
         R=kv_rank, LW=LW, window=window or 0, tiles_per_split=ws.per, nsplits=ws.splits,
         scale=float(scale), sink=ptr(sink), gate=ptr(gate),
         ldg=gate.stride(0) if gate is not None else 0), ptr(y), ptr(up), 0 if up is None else up.shape[1],

@@ -1078,6 +1078,32 @@ def test_latent_decode_a_block_at_a_time(H, parts):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("shared", [True, False])
+@pytest.mark.parametrize("window", [None, 50])
+def test_latent_decode_of_tables_of_any_stride(shared, window):
+    """One table's row for all sequences, and rows of fewer entries than lie between them; rounding of the tests above."""
+    H, R, nb, ctx, dev = 16, 512, 5, [1, 33, 160, 64, 0], "cuda"
+    g = torch.Generator().manual_seed(nb)
+    cache = torch.randn(4 * nb + 1, 32, R + 64, generator=g).mul_(0.5).to(torch.bfloat16)
+    bt = torch.stack([torch.randperm(4 * nb, generator=g)[:nb + 3] + 1 for _ in ctx]).to(torch.int32)
+    bt = bt[:1, :nb].expand(len(ctx), nb) if shared else bt[:, :nb]
+    table = bt[:1].to(dev).expand(len(ctx), nb) if shared else torch.full((len(ctx), nb + 3), 2 ** 30, dtype=torch.int32, device=dev)
+    if not shared:
+        table[:, :nb] = bt.to(dev)
+        table = table[:, :nb]
+    assert table.stride(0) == (0 if shared else nb + 3)
+    qa = torch.randn(len(ctx), H, R + 64, generator=g).mul_(0.5).to(torch.bfloat16)
+    out = ops.latent_decode_attention(qa.to(dev), cache.to(dev), R, table, torch.tensor(ctx, dtype=torch.int32, device=dev),
+                                      window, 0.05, None)
+    for b, n in enumerate(ctx):
+        if n == 0:
+            assert (out[b] == 0).all()
+            continue
+        rows = cache[bt[b].long()].reshape(-1, R + 64)[max(0, n - (window or n)):n].double()
+        close(out[b], (qa[b].double() @ rows.T * 0.05).softmax(-1) @ rows[:, :R], 2e-2)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("B", [1, 3, 16, 17, 65])
 @pytest.mark.parametrize("H,R,dim,vdim,splits,gated", [(16, 512, 128, 128, 20, True), (4, 256, 128, 40, 3, False),
                                                         (5, 128, 256, 64, 2, True), (20, 448, 128, 128, 4, True),
