@@ -168,14 +168,18 @@ CHAIN_BYTES = 1 << 30  # operands of the chunks prepared ahead: as many heads at
 
 def _chain_ok(w: DeltaWeights, decay: torch.Tensor, gate: torch.Tensor, p: Portions) -> bool:
     """Whether the recurrence runs as delta_prep / chain / read: where the longest portion, and not the
-    work of all, sets the time of the one-launch form.  That form has a workgroup per (portion, head),
-    the chains need operands prepared in memory; with about one workgroup per CU they are equal (16
-    heads of 128: 16 x 1,000 tokens 603 against 681 us, 20 x 150 149 against 151, 64 x 24 124 against
-    84).  Portions of a few chunks do not repay three launches (16 heads: 8 x 16 tokens 35 against
-    26 us; 32 heads: one of 48 tokens 34 against 44)."""
+    work of all, sets the time of the one-launch form.  That form has a workgroup per (portion, head), and the chains need
+    operands prepared in memory.  Up to a workgroup per CU, by the rows of the longest portion (heads of 128, 16 of them: 8 x 60
+    tokens 58 us against 63, 10 x 700 304 / 543, 16 x 500 306 / 388; 32: 9 x 500 350 / 515); up to three where the longest has 320
+    tokens, since a second and third round of workgroups is mostly empty (16 heads: 20 x 700 498 / 750, 24 x 300 288 / 329, 30 x
+    480 507 / 527, 48 x 300 534 / 619; 32: 10 x 1400 992 / 1447, 12 x 350 324 / 358, 18 x 800 1007 / 1263, 26 x 550 987 / 1050).
+    Two full workgroups a CU have no such gaps (16 x 900 of 32 997 / 980, 32 x 450 of 16 530 / 520), short portions not the
+    time for three launches (32 x 150 of 16 206 / 181, 16 x 250 of 32 311 / 287), nor portions of a few chunks (16 heads: 8 x 16
+    tokens 35 us against 26; 32 heads: one of 48 tokens 34 against 44)."""
+    work, longest, groups = p.row_state.numel() * w.heads, 256 * p.max_len, p.seg_row.numel() * w.heads
     return (w.dim % 8 == w.vdim % 8 == 0 and w.dim <= 128 and w.vdim <= 256
-            and decay.stride(0) % 8 == gate.stride(0) % 8 == 0
-            and p.max_len > 32 and p.row_state.numel() * w.heads <= 256 * p.max_len)
+            and decay.stride(0) % 8 == gate.stride(0) % 8 == 0 and p.max_len > 32
+            and (work <= longest or p.max_len >= 320 and work <= 3 * longest and not 480 < groups <= 512))
 
 
 def _chain_workspace(w: DeltaWeights, rows: int, n: int, dev) -> tuple[torch.Tensor, torch.Tensor] | None:

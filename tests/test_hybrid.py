@@ -362,6 +362,46 @@ def test_delta_decode_state_ahead(hipk, dt, H, Hk, d, dv, taps):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,Hk,d,dv,lens", [(16, 8, 32, 48, [321, 333] * 9 + [1, 17, 320]), (16, 16, 128, 72, [340] + [271] * 20),
+                                            (48, 16, 24, 40, [325, 7, 48] * 6)])
+def test_delta_chains_past_a_workgroup_a_cu(monkeypatch, dt, H, Hk, d, dv, lens):
+    """Chunks prepared ahead where the one-launch form has up to three rounds of workgroups, against that form: sums of the same
+    products in another order; continued states, slots in another order and one portion of padding."""
+    dev, n, taps = "cuda", len(lens), 3
+    g = torch.Generator().manual_seed(d + n)
+    r = lambda *shape: torch.randn(*shape, generator=g).to(dev)
+    C, rows = 2 * Hk * d + H * dv, sum(lens)
+    w = ops.DeltaWeights(r(taps, C), torch.linspace(-1, 1, H).exp().to(dev), r(H * d) - 2, 1 + 0.1 * r(dv), 1e-5, H, Hk, d, dv)
+    proj, decay, gate = r(rows, -(-(C + H) // 8) * 8).to(dt), r(rows, H * d).to(dt), r(rows, H * dv).to(dt)
+    ring, state = r(n, taps, C).to(dt), r(n, H, d, dv)
+    p, pos = _portions(dev, lens, [3 * (i % 2) for i in range(n)], [-1 if i == 2 else n - 1 - i for i in range(n)])
+    conv = ops.short_conv(proj, w, ring, pos, p)
+    assert ops.delta._chain_ok(w, decay, gate, p) and rows * H > 256 * max(lens)
+    out = []
+    for force in (True, False):
+        monkeypatch.setattr(ops.delta, "_chain_ok", lambda *a, force=force: force)
+        s, q = state.clone(), ring.clone()
+        o = ops.delta_scan(proj, C, conv, w, q, s, decay, gate, p)
+        out.append((o[p.row_state >= 0], s, q))
+    for got, want in zip(*out):
+        close(got, want.double().cpu(), tol(dt, 5e-5, 2e-2))
+
+
+@pytest.mark.parametrize("n,tokens,heads,chain", [(8, 60, 16, True), (1, 32, 16, False), (20, 450, 16, True), (24, 600, 16, True),
+                                                  (32, 450, 16, False), (16, 900, 32, False), (16, 250, 32, False),
+                                                  (12, 900, 32, True), (24, 550, 32, True), (26, 550, 32, False)])
+def test_which_portions_take_the_chains(n, tokens, heads, chain):
+    """Equal portions: three workgroups of the one-launch form a CU are 24 portions of 32 heads."""
+    w = ops.DeltaWeights(*(None,) * 4, 1e-5, heads, heads, 128, 128)
+    rows = torch.empty(1, heads * 128)
+    row_state = torch.zeros(1, dtype=torch.int32).expand(n * tokens)
+    one = torch.zeros(n, dtype=torch.int32)
+    p = ops.Portions(one, one, one, one, row_state, row_state, tokens)
+    assert ops.delta._chain_ok(w, rows, rows, p) == chain
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("shift", [-6.0, 2.0, 12.0, 90.0])
 @pytest.mark.parametrize("d", [128, 64, 24])
 def test_delta_chains_of_any_decay(shift, d):
