@@ -1263,7 +1263,9 @@ __global__ __launch_bounds__(64 * chain_waves(DT), 2) void delta_chain_narrow_ke
   // Outputs: rows 4 g + RW w + j are this wave's
   const int64_t ldo = (int64_t)a.H * a.vdim16;
   float* o = a.ws_o + (int64_t)(entry - 1) * 16 * ldo + h * a.vdim16;  // of the chunk ahead of the next one
-  const unsigned orow = 4 * ((4 * g + RW * w) * (unsigned)ldo + x0 + col);
+  unsigned orow[RW];
+#pragma unroll
+  for (int j = 0; j < RW; ++j) orow[j] = 4 * ((4 * g + RW * w + j) * (unsigned)ldo + x0 + col);
   auto read_out = [&](float (&ys)[RW][NW], const int par) {
 #pragma unroll
     for (int j = 0; j < RW; ++j)
@@ -1278,7 +1280,8 @@ __global__ __launch_bounds__(64 * chain_waves(DT), 2) void delta_chain_narrow_ke
       float y = ys[j][0];
 #pragma unroll
       for (int i = 1; i < NW; ++i) y += ys[j][i];
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, y), b, orow, 4 * j * (unsigned)ldo, 0);
+      // (no scalar offset: it is taken off the descriptor's size, and off a size of 0 it would leave everything in range)
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, y), b, orow[j], 0, 0);
     }
   };
   auto compute = [&](int c, Ops& x, const int par) {

@@ -423,6 +423,37 @@ def test_delta_chains_of_any_decay(shift, d):
     close(got, want.double().cpu(), 5e-5)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("d", [24, 32, 64, 128])
+def test_delta_chains_write_their_own_rows(monkeypatch, dt, d):
+    """Chunks of several portions, a column tile to a workgroup, two and four waves: nothing ahead of the outputs' workspace is
+    written, and all rows, the last ones of a portion ahead of another among them, are those of the form token by token."""
+    H, dv, taps, lens, dev = 3, 40, 3, [7, 48, 16, 33], "cuda"
+    n, ldo = len(lens), H * 48
+    g = torch.Generator().manual_seed(d)
+    r = lambda *shape: torch.randn(*shape, generator=g).to(dev)
+    C, rows = 2 * H * d + H * dv, sum(lens)
+    w = ops.DeltaWeights(r(taps, C), torch.linspace(-1, 1, H).exp().to(dev), r(H * d) - 2, 1 + 0.1 * r(dv), 1e-5, H, H, d, dv)
+    proj, decay, gate, ring = r(rows, C + 8).to(dt), r(rows, H * d).to(dt), r(rows, H * dv).to(dt), r(n, taps, C).to(dt)
+    p, pos = _portions(dev, lens, [0] * n, range(n))
+    conv = ops.short_conv(proj, w, ring, pos, p)
+    assert ops.delta._chain_ok(w, decay, gate, p)
+    made, guard = ops.delta._chain_workspace, []
+
+    def behind_a_guard(*a):
+        ws, out = made(*a)
+        guard.append(torch.full((16 * ldo + out.numel(),), 7.0, device=dev))
+        return ws, guard[0][16 * ldo:]
+
+    monkeypatch.setattr(ops.delta, "_chain_workspace", behind_a_guard)
+    got, want = ((ops.delta_scan(proj, C, conv, w, ring.clone(), s, decay, gate, p, c), s)
+                 for s, c in ((torch.zeros(n, H, d, dv, device=dev), 0), (torch.zeros(n, H, d, dv, device=dev), 2)))
+    assert len(guard) == 1 and (guard[0][:16 * ldo] == 7).all()
+    for a, b in zip(got, want):
+        close(a, b.double().cpu(), tol(dt, 5e-5, 3e-2))
+
+
 @on
 @pytest.mark.parametrize("case", CHAIN_CASES, ids=str)
 def test_delta_chains(target, case, monkeypatch):
