@@ -168,18 +168,23 @@ CHAIN_BYTES = 1 << 30  # operands of the chunks prepared ahead: as many heads at
 
 def _chain_ok(w: DeltaWeights, decay: torch.Tensor, gate: torch.Tensor, p: Portions) -> bool:
     """Whether the recurrence runs as delta_prep / chain / read: where the longest portion, and not the
-    work of all, sets the time of the one-launch form.  That form has a workgroup per (portion, head), and the chains need
-    operands prepared in memory.  Up to a workgroup per CU, by the rows of the longest portion (heads of 128, 16 of them: 8 x 60
-    tokens 58 us against 63, 10 x 700 304 / 543, 16 x 500 306 / 388; 32: 9 x 500 350 / 515); up to three where the longest has 320
-    tokens, since a second and third round of workgroups is mostly empty (16 heads: 20 x 700 498 / 750, 24 x 300 288 / 329, 30 x
-    480 507 / 527, 48 x 300 534 / 619; 32: 10 x 1400 992 / 1447, 12 x 350 324 / 358, 18 x 800 1007 / 1263, 26 x 550 987 / 1050).
-    Two full workgroups a CU have no such gaps (16 x 900 of 32 997 / 980, 32 x 450 of 16 530 / 520), short portions not the
-    time for three launches (32 x 150 of 16 206 / 181, 16 x 250 of 32 311 / 287), nor portions of a few chunks (16 heads: 8 x 16
-    tokens 35 us against 26; 32 heads: one of 48 tokens 34 against 44)."""
+    work of all, sets the time of the one-launch form.  That form has a workgroup per (portion, head), two of them to a CU at a
+    time, and the chains need operands prepared in memory.  By ratio, the work of all over a CU's share of as much as the longest
+    portion (heads of 128; us chains / one launch; equal portions, or of the lengths given):
+      up to 1: 16 heads 8 x 60 tokens 58 / 63, 16 x 500 280 / 328; 32 heads 8 x 900 491 / 607; from 320 tokens on also
+      up to 1.55 (1.45 below 500 tokens) of up to 512 workgroups, the second half of which is partly empty: 32 heads 11 x 320 267 /
+        293, 12 x 600 509 / 573, 8 x 900 and 8 x 450 740 / 833, 1500 and 15 x 900 1010 / 1328, 15 of 360 to 600 514-517 / 521-571;
+        nearly full it has no such gap: 15 x 320 333 / 299, 14 x 500 490 / 468, 16 x 500 537 / 487, 15 of 192 to 320 299-305 / 283-302
+      up to 2.75 of up to 768, of which the last 256 run one to a CU: 32 heads 17 x 500 631 / 765, 20 of 360 to 600 697-701 /
+        833-917, 22 x 500 751 / 766; again not where nearly full: 23 x 500 787 / 766, 24 x 500 802 / 766
+      up to 3 of more, whose portions differ: 32 heads 600 and 60 x 150 746 / 914, 29 of 360 to 600 979-988 / 1007-1032.
+    Shorter portions have not the time for three launches (32 x 150 of 16 heads 206 / 181, 16 x 250 of 32 311 / 287), nor have
+    portions of a few chunks (16 heads: 8 x 16 tokens 35 / 26; 32 heads: one of 48 tokens 34 / 44)."""
     work, longest, groups = p.row_state.numel() * w.heads, 256 * p.max_len, p.seg_row.numel() * w.heads
+    most = (1.55 if p.max_len >= 500 else 1.45) if groups <= 512 else 2.75 if groups <= 768 else 3
     return (w.dim % 8 == w.vdim % 8 == 0 and w.dim <= 128 and w.vdim <= 256
             and decay.stride(0) % 8 == gate.stride(0) % 8 == 0 and p.max_len > 32
-            and (work <= longest or p.max_len >= 320 and work <= 3 * longest and not 480 < groups <= 512))
+            and work <= (most if p.max_len >= 320 else 1) * longest)
 
 
 def _chain_workspace(w: DeltaWeights, rows: int, n: int, dev) -> tuple[torch.Tensor, torch.Tensor] | None:

@@ -390,14 +390,28 @@ def test_delta_chains_past_a_workgroup_a_cu(monkeypatch, dt, H, Hk, d, dv, lens)
 
 @pytest.mark.parametrize("n,tokens,heads,chain", [(8, 60, 16, True), (1, 32, 16, False), (20, 450, 16, True), (24, 600, 16, True),
                                                   (32, 450, 16, False), (16, 900, 32, False), (16, 250, 32, False),
-                                                  (12, 900, 32, True), (24, 550, 32, True), (26, 550, 32, False)])
+                                                  (12, 900, 32, True), (24, 550, 32, False), (26, 550, 32, False),
+                                                  (11, 320, 32, True), (13, 320, 32, False), (13, 900, 32, False), (15, 500, 32, False),
+                                                  (17, 500, 32, True), (22, 500, 32, True), (23, 500, 32, False), (30, 500, 16, False)])
 def test_which_portions_take_the_chains(n, tokens, heads, chain):
-    """Equal portions: three workgroups of the one-launch form a CU are 24 portions of 32 heads."""
+    """Equal portions: three workgroups of the one-launch form a CU are 24 portions of 32 heads.  Those that fill their last
+    round of workgroups by more than half lose up to a tenth as chains."""
+    _takes_chains([tokens] * n, heads, chain)
+
+
+@pytest.mark.parametrize("lens,heads,chain", [([1500] + [900] * 15, 32, True), ([900] * 8 + [450] * 8, 32, True),
+                                              ([500] + [290] * 31, 16, True), ([800] * 10 + [400] * 20, 32, True),
+                                              ([600] * 20 + [300] * 20, 32, False), ([600] + [150] * 60, 32, True)])
+def test_which_uneven_portions_take_the_chains(lens, heads, chain):
+    _takes_chains(lens, heads, chain)
+
+
+def _takes_chains(lens, heads, chain):
     w = ops.DeltaWeights(*(None,) * 4, 1e-5, heads, heads, 128, 128)
     rows = torch.empty(1, heads * 128)
-    row_state = torch.zeros(1, dtype=torch.int32).expand(n * tokens)
-    one = torch.zeros(n, dtype=torch.int32)
-    p = ops.Portions(one, one, one, one, row_state, row_state, tokens)
+    row_state = torch.zeros(1, dtype=torch.int32).expand(sum(lens))
+    one = torch.zeros(len(lens), dtype=torch.int32)
+    p = ops.Portions(one, one, one, one, row_state, row_state, max(lens))
     assert ops.delta._chain_ok(w, rows, rows, p) == chain
 
 
