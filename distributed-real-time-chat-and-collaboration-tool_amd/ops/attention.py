@@ -347,7 +347,8 @@ def paged_decode_attention_rope(qkv: torch.Tensor | Parts, positions: torch.Tens
     parts = None
     if isinstance(qkv, Parts):
         n = qkv.slab.shape[0]
-        if (on_gpu(qkv.slab) and 2 <= n <= QKV_PARTS and k_cache.data_ptr() % 16 == 0 and qkv.slab.is_contiguous()
+        if (on_gpu(qkv.slab) and qkv.slab.dtype == torch.float32 and 2 <= n <= QKV_PARTS
+                and k_cache.data_ptr() % 16 == 0 and qkv.slab.is_contiguous()
                 and qkv.shape[1] % 4 == 0 and qkv.slab.data_ptr() % 16 == 0
                 and blocks_per_part is not None and workspace is not None
                 and n <= decode_qkv_parts(B, Hkv, D, block_tables.shape[1], workspace.max_parts, max_wgs)):
@@ -385,8 +386,9 @@ def paged_decode_attention_rope(qkv: torch.Tensor | Parts, positions: torch.Tens
     if out is None:
         out = torch.empty((B, Hq, D), dtype=qkv.dtype, device=rows.device)
     assert out.is_contiguous() and out.shape == (B, Hq, D)
+    # (a slab of one row is contiguous whatever that row's stride says)
     check(hipk().paged_decode_rope(out.data_ptr(), ptr(workspace.part_o), ptr(workspace.part_ml),
-                                   0 if parts else rows.data_ptr(), rows.stride(-2), k_cache.data_ptr(),
+                                   0 if parts else rows.data_ptr(), qkv.shape[1] if parts else qkv.stride(0), k_cache.data_ptr(),
                                    v_cache.data_ptr(), block_tables.data_ptr(),
                                    block_tables.stride(0), context_lens.data_ptr(), B, Hq, Hkv, D,
                                    float(scale), workspace.max_parts, blocks_per_part,

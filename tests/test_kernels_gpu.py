@@ -340,6 +340,29 @@ def test_paged_decode_rope_of_slices(hipk, D, Hq, Hkv, bpp, n):
         assert torch.equal(a, b), what
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_paged_decode_rope_of_one_row_of_slices(hipk, dtype):
+    """One sequence's slices, whose row has a stride that nothing uses, and slices of another type than the projection's:
+    the bits of their sum's row."""
+    D, Hq, Hkv, n = 128, 32, 8, 3
+    N = (Hq + 2 * Hkv) * D
+    _, kc, vc, bt, cl = _paged_setup(1, Hq, Hkv, D, [77], seed=43)
+    slab = torch.randn(1, n, N, generator=torch.Generator().manual_seed(44)).to(DEV, dtype).transpose(0, 1)
+    assert slab.is_contiguous() and slab.stride(1) == n * N
+    rows = ((slab[0] + slab[1]) + slab[2]).to(torch.bfloat16)
+    pos, slots = cl - 1, torch.tensor([int(bt[0, 2]) * 32 + 76 % 32], device=DEV)
+    cs, parts = ops.build_rope_cache(1024, D, 5e5, device=DEV), -(-bt.shape[1] // 8)
+    assert ops.decode_qkv_parts(1, Hkv, D, bt.shape[1], parts) == 4
+    got = []
+    for qkv in (rows, ops.Parts(slab, torch.bfloat16)):
+        k, v = kc.clone(), vc.clone()
+        out = ops.paged_decode_attention_rope(qkv, pos, slots, cs, Hq, Hkv, D, k, v, bt, cl, D ** -0.5, blocks_per_part=8,
+                                              workspace=ops.DecodeWorkspace(1, Hq, D, parts, DEV))
+        got.append((out, k, v))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("variant", [1, 2, 3])
 def test_paged_decode_strided_q_and_padding(hipk, variant):
     Hq, Hkv, D = 32, 8, 128
