@@ -388,6 +388,22 @@ def test_parts_forms():
                                               (65, 4096, 2048), (64, 4096, 1984), (64, 8256, 4096), (64, 4096, 4104)])
 
 
+@pytest.mark.parametrize("limits", [(4, G.MAX_PARTS), (G.MAX_PARTS, 4)])
+def test_parts_forms_of_up_to_four_slices(monkeypatch, limits):
+    """A reader of up to four slices gets no more, whichever limit was asked first; 3 rows on from K = 4096, 17 from 2048."""
+    monkeypatch.setattr(G, "_parts_forms", {})
+    seen = {most: set() for most in limits}
+    for M in (2, 3, 16, 17, 33, 64):
+        for N, K in ((6144, 4096), (3072, 2048), (2304, 2048), (4096, 5120), (5120, 4096)):
+            for most in limits:
+                form = G.parts_form(M, N, K, most)
+                assert (form is not None) == (M >= (3 if K >= 4096 else 17)), (M, N, K, most)
+                if form:
+                    assert 2 <= form[1] <= most and N % (32 * form[0]) == 0 and K // 64 // form[1] >= 4
+                    seen[most].add(form)
+    assert max(s for _, s in seen[4]) == 4 and max(s for _, s in seen[G.MAX_PARTS]) > 4
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,form", [(1, 1024, 256, (2, 1)), (17, 1088, 320, (2, 5)), (33, 2048, 4096, (2, 8)),
                                        (64, 4096, 704, (4, 8)), (96, 1024, 2112, (4, 3)), (150, 4096, 5632, (2, 4)),

@@ -363,6 +363,33 @@ def test_paged_decode_rope_of_one_row_of_slices(hipk, dtype):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("B,W,Hq,Hkv", [(3, 4096, 32, 8), (16, 4096, 32, 8), (64, 4096, 32, 8), (17, 2048, 16, 4), (64, 2048, 16, 4)])
+def test_projection_slices_reach_the_attention(hipk, monkeypatch, B, W, Hq, Hkv):
+    """The projection's slices, no more of them than decode attention adds up, go into it as they are; against the product of
+    the same normalised rows in 64 bits, rotated and attended in fp32 (tolerance of the tests above)."""
+    D, ctx_lens = 128, [1 + 37 * i % 300 for i in range(B)]
+    _, kc, vc, bt, cl = _paged_setup(B, Hq, Hkv, D, ctx_lens, seed=B)
+    g = torch.Generator().manual_seed(W + B)
+    x, res = (torch.randn(B, W, generator=g).to(torch.bfloat16).to(DEV) for _ in range(2))
+    w = (torch.randn((Hq + 2 * Hkv) * D, W, generator=g) * W ** -0.5).to(torch.bfloat16).to(DEV)
+    parts = -(-bt.shape[1] // 4)
+    most = ops.decode_qkv_parts(B, Hkv, D, bt.shape[1], parts)
+    p = ops.PendingNorm(x, res, torch.ones(W, dtype=torch.bfloat16, device=DEV), 1e-5, False)
+    qkv = ops.norm_linear(p, w, most)
+    assert most == 4 and isinstance(qkv, ops.Parts) and 2 <= qkv.slab.shape[0] <= most
+    monkeypatch.setattr(ops.Parts, "tensor", lambda self: pytest.fail("added up ahead"))
+    slots = torch.tensor([int(bt[b, (c - 1) // 32]) * 32 + (c - 1) % 32 for b, c in enumerate(ctx_lens)], device=DEV)
+    cs = ops.build_rope_cache(512, D, 5e5, device=DEV)
+    rows, k, v = (p.materialize().double() @ w.double().T).float(), kc.float(), vc.float()
+    ops.rope_kv_ref(rows, cl - 1, slots, cs, Hq, Hkv, D, k, v, ops.KV_BLOCK)
+    want = ops.paged_decode_ref(rows[:, :Hq * D].view(B, Hq, D), k, v, bt, cl, D ** -0.5)
+    out = ops.paged_decode_attention_rope(qkv, cl - 1, slots, cs, Hq, Hkv, D, kc, vc, bt, cl, D ** -0.5, blocks_per_part=4,
+                                          workspace=ops.DecodeWorkspace(B, Hq, D, parts, DEV))
+    _close(out, want, 2e-2, 2e-2, "output")
+    _close(kc, k, 1e-2, 1e-2, "k cache")
+    _close(vc, v, 1e-2, 1e-2, "v cache")
+
+
 @pytest.mark.parametrize("variant", [1, 2, 3])
 def test_paged_decode_strided_q_and_padding(hipk, variant):
     Hq, Hkv, D = 32, 8, 128
