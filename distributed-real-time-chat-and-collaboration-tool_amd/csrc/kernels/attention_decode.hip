@@ -254,9 +254,11 @@ DRTC_DEVICE float load_part(const float* p) {
 // 64.3 -> 61.5 (66.8), 512 x 20 24.7 -> 19.9 (20.7), 256 x 40 18.3 -> 16.8 (17.4); 256 x 20 13.8 -> 13.4 (12.0).
 // PARTS (up to 64 rows, attention.py decode_qkv_parts): q, k and v come as the sums of the projection's K slices
 // (gemm_midm.hip), added up here, in order, and rounded as the projection rounds its rows.  A projection cut in slices fills
-// the chip: 6144 x 4096, whole / two slices, 4 rows 12.6 / 10.6 us, 16 rows 14.1 / 11.1, 64 rows 17.0 / 13.8 (four); 3072 x
-// 2048, 16 rows 6.2 / 5.4.  Every wave needs all of q: a quarter of the heads each, which meet in the LDS beside the staged
-// rows (16 x 1000 19.0 us, as from rows; each wave adding up all of them, two workgroups to a CU for the registers: 21.4).
+// the chip: 6144 x 4096, whole / two slices, 3 rows 12.3 / 10.6 us, 16 rows 14.1 / 11.0, 64 rows 16.7 / 13.9; 3072 x 2048, cut
+// in four from 17 rows on, 17 rows 7.0 / 5.4, 64 rows 7.1 / 6.6.  Every wave needs all of q: a quarter of the heads each, which
+// meet in the LDS beside the staged rows (16 x 1000 19.0 us, as from rows; each wave adding up all of them, two workgroups to
+// a CU for the registers: 21.4).  From 15 heads of 128 to a kv head on that LDS makes four workgroups a CU three, which
+// costs less than the slices give (decode_qkv_parts).
 template <int D, bool ROPE, bool PARTS = false>
 __global__ __launch_bounds__(256, D >= 256 ? 2 : 4) void paged_decode_kernel(
     bf16_t* __restrict__ out, float* __restrict__ part_o,

@@ -317,8 +317,11 @@ def decode_qkv_parts(B: int, Hkv: int, D: int, max_blocks: int, max_parts: int, 
     """K slices' sums that ``paged_decode_attention_rope`` adds up itself, 0 where it wants rows: its kernel 1 does, for up to
     64 rows.  us of a decode step of four layers, rows / sums: width 4096, 3 x 300 tokens 451 / 442, 8 x 500 465 / 453, 24 x
     400 510 / 498, 32 x 1000 591 / 579, 48 x 300 553 / 537, 64 x 800 646 / 629; width 2048, 20 x 500 274 / 269, 48 x 1000 329 /
-    311, 64 x 300 297 / 275; beyond 64 rows the projection has filled the chip: 72 x 300 589 / 611, 96 x 300 621 / 640, 140 x
-    300 747 / 768."""
+    311, 64 x 300 297 / 275.  Every partition of a context reads the slices, which costs less than they give at any
+    length: width 4096, 4 x 2000 463 / 458, 8 x 4000 545 / 538, 64 x 2000 830 / 819, 16 x 4000 653 / 642, 3 x 16000 597 / 592, 8 x
+    12000 739 / 731; width 2048, 64 x 2000 435 / 416, 20 x 8000 494 / 491; 16 heads to a kv head, 4096 16 x 1000 486.6 /
+    487.2, 16 x 4000 535.5 / 536.3, 64 x 2000 622 / 620, 3 x 16000 573 / 550, 2048 64 x 2000 349 / 335.  Beyond 64 rows the projection
+    has filled the chip: 72 x 300 589 / 611, 96 x 300 621 / 640, 140 x 300 747 / 768."""
     if B > 64 or not FUSED_ROPE:
         return 0
     variant = decode_variant(B, Hkv, D, max_blocks)
