@@ -13,11 +13,12 @@
 //    compacted full gather.
 //    What bounds a row is the chain of its stages, and fetching code that runs
 //    once a step: tau0 by one wave's ballots instead of the workgroup's
-//    histograms, a gather in a few instructions instead of one unrolled over 32
-//    elements, and every request of the row and its parameters at the start.
-//    V 32000, top-k 64, top-p 0.95, before / now: 1 row 11.3 / 6.9 us, 64 11.6 /
-//    7.4, 512 16.1 / 10.4, 1024 31.1 / 20.5; V 128256, 1 row 18.6 / 11.8, 1024
-//    72.0 / 62.7.
+//    histograms, and a gather in a few instructions instead of one unrolled over
+//    32 elements.  A row of up to 32,768 is held in registers, asked for when it
+//    is known to need them: the other modes read as ever (greedy, exact top-p).
+//    V 32000, top-k 64, top-p 0.95, before / now: 1 row 11.4 / 6.9 us, 256 12.0 /
+//    8.2, 1024 31.4 / 22.2; V 128256, 1 row 19.7 / 13.0, 256 26.2 / 21.4, 1024
+//    72.2 / 63.5.
 //    Up to 128 candidates find their places by counting and are drawn from by one wave;
 //    more are bitonic-sorted.  All tokens tied with the k-th value stay.
 //  * top_k == 0       : temperature sampling with EXACT top-p over the whole
@@ -393,7 +394,6 @@ DRTC_DEVICE void sample_few(SampShared& s, const unsigned* sort, const TokenOut&
   const int tid = threadIdx.x, lane = tid & 63, own = tid >> 3;
   float* const sv = reinterpret_cast<float*>(&s.hist[8][0]);
   int* const si = reinterpret_cast<int*>(&s.hist[9][0]);
-  auto order = [](float v) { return place_key(v); };
   // every candidate gets a place of its own
   if (own < n) {
     const float v = s.val[own];
@@ -407,9 +407,9 @@ DRTC_DEVICE void sample_few(SampShared& s, const unsigned* sort, const TokenOut&
         ahead += (q[0] > mine) + (q[1] > mine) + (q[2] > mine) + (q[3] > mine);
       }
     } else {
-      const unsigned key = order(v);
+      const unsigned key = place_key(v);
       for (int j = tid & 7; j < n; j += 8) {
-        const unsigned kj = order(s.val[j]);
+        const unsigned kj = place_key(s.val[j]);
         ahead += kj > key || (kj == key && s.idx[j] < id);
       }
     }
@@ -423,12 +423,12 @@ DRTC_DEVICE void sample_few(SampShared& s, const unsigned* sort, const TokenOut&
   }
   __syncthreads();
   if (tid >= 64) return;
-  const unsigned kth = order(sv[min(k, n) - 1]);
+  const unsigned kth = place_key(sv[min(k, n) - 1]);
   float x[2], lo[2];
   int total_n = 0;
 #pragma unroll
   for (int z = 0; z < 2; ++z)  // ties with the k-th value stay
-    total_n += __popcll(__ballot(lane + 64 * z < n && order(sv[min(lane + 64 * z, n - 1)]) >= kth));
+    total_n += __popcll(__ballot(lane + 64 * z < n && place_key(sv[min(lane + 64 * z, n - 1)]) >= kth));
   n = total_n;
   const float top = sv[0], inv_t = 1.f / temp;
 #pragma unroll
@@ -760,23 +760,14 @@ __global__ __launch_bounds__(kSampThreads, 4 * OCC) void sample_kernel(
   const int lane = tid & 63, wid = tid >> 6;
   const unsigned short* lr = (const unsigned short*)(logits + (int64_t)row * ld);
   const bool vec = ((reinterpret_cast<uintptr_t>(lr) & 15) == 0);
-  // the row and everything that says what to do with it are asked for together
-  using Row = std::conditional_t<HELD, HeldRow, ReadRow<U>>;
-  Row each;
-  if constexpr (HELD) each.load(lr, V);
-  else each = {lr, V, vec};
   const float temp = temperature ? temperature[row] : 0.f;
-  const uint64_t st = step ? (uint64_t)step[0] : 0ull;
-  const float asked = top_p ? top_p[row] : 1.f, pp = asked > 0.f && asked < 1.f ? asked : 1.f;
-  int k = top_k ? top_k[row] : 0;
   const TokenOut out{out_tokens, mirror.turn ? mirror.host[~*mirror.turn & 1] : nullptr};  // (the turn is the next step's)
-  __builtin_amdgcn_sched_barrier(0);
   __shared__ SampShared s;
 
   if (temp <= 0.f) {  // ---------------------------------- greedy argmax
     float best = -INFINITY;
     int bi = 0x7fffffff;
-    each([&](int i, unsigned short b) {
+    for_row<U>(lr, V, vec, [&](int i, unsigned short b) {
       const float v = bits2f(b);
       if (v > best || (v == best && i < bi)) { best = v; bi = i; }
     });
@@ -795,8 +786,18 @@ __global__ __launch_bounds__(kSampThreads, 4 * OCC) void sample_kernel(
     }
     return;
   }
+  // Nothing of a row is asked for ahead of these two: held for a row that turned out greedy or of exact top-p, 64 registers
+  // spilled (1024 rows of 32,000 with top-p alone 62 -> 77 us, of 512 22 -> 33, greedy 8.4 -> 15.7), and the round trip that
+  // it saves is 0.4 us of a row.  k behind the greedy rows, which would wait for it (1024 x 32000 18.6 / 19.0).
+  int k = top_k ? top_k[row] : 0;
   if (k >= V) k = 0;
+  const uint64_t st = step ? (uint64_t)step[0] : 0ull;
+  const float asked = top_p ? top_p[row] : 1.f, pp = asked > 0.f && asked < 1.f ? asked : 1.f;
   if (k > 0) {
+    using Row = std::conditional_t<HELD, HeldRow, ReadRow<U>>;
+    Row each;
+    if constexpr (HELD) each.load(lr, V);
+    else each = {lr, V, vec};
     sample_topk<U>(s, out, each, lr, V, vec, row, temp, min(k, kCand), pp, seed, st);
   } else {
     sample_topp_full<U>(s, out, lr, V, vec, row, temp, pp, seed, st);

@@ -739,6 +739,27 @@ def test_sample_row_forms(hipk, V, k):
         assert (lg.float().gather(1, got[:, None])[:, 0] >= kth).all()
 
 
+@pytest.mark.parametrize("V", [8, 512, 8192, 32768, 32776])
+def test_sample_modes_in_one_batch(hipk, V):
+    """Greedy rows, rows of top-p alone and of top-k beside one another: the tokens of the same rows from a view that starts
+    2 bytes off, whose form holds no row; greedy ones the first largest."""
+    B, g = 60, torch.Generator().manual_seed(V)
+    lg = (torch.randn(B, V, generator=g) * 2).to(torch.bfloat16).to(DEV)
+    odd = torch.empty(B, V + 8, dtype=torch.bfloat16, device=DEV)[:, 1:V + 1]
+    odd.copy_(lg)
+    temp = torch.linspace(0.3, 1.5, B, device=DEV)
+    temp[::3] = 0
+    k = torch.full((B,), min(64, V - 1), dtype=torch.int32, device=DEV)
+    k[1::3] = 0
+    top_p = torch.linspace(0.5, 1.2, B, device=DEV)
+    for i in range(3):
+        step = torch.tensor([i], device=DEV)
+        got = ops.sample(lg, temp, k, top_p, seed=3, step=step).long()
+        assert torch.equal(got, ops.sample(odd, temp, k, top_p, seed=3, step=step).long())
+        best = lg[::3].float().max(1).values[:, None]
+        assert torch.equal(got[::3], (lg[::3].float() == best).int().argmax(1))
+
+
 def test_sample_top_p_full_vocab_exact(hipk):
     """top_k = 0: every draw lies in the exact nucleus of the full 128k vocab,
     and most draws are ranked below 1024 (nothing is truncated to a candidate
