@@ -741,8 +741,9 @@ def test_sample_row_forms(hipk, V, k):
 
 @pytest.mark.parametrize("V", [8, 512, 8192, 32768, 32776])
 def test_sample_modes_in_one_batch(hipk, V):
-    """Greedy rows, rows of top-p alone and of top-k beside one another: the tokens of the same rows from a view that starts
-    2 bytes off, whose form holds no row; greedy ones the first largest."""
+    """Greedy rows, rows of top-p alone and of top-k beside one another, and the same rows from a view that starts 2 bytes off,
+    whose form holds no row: top-k gives the same tokens, greedy the first largest; top-p alone, whose draw goes through the
+    threads' elements in their order, in both a token that less than top-p of the mass is ahead of."""
     B, g = 60, torch.Generator().manual_seed(V)
     lg = (torch.randn(B, V, generator=g) * 2).to(torch.bfloat16).to(DEV)
     odd = torch.empty(B, V + 8, dtype=torch.bfloat16, device=DEV)[:, 1:V + 1]
@@ -752,12 +753,17 @@ def test_sample_modes_in_one_batch(hipk, V):
     k = torch.full((B,), min(64, V - 1), dtype=torch.int32, device=DEV)
     k[1::3] = 0
     top_p = torch.linspace(0.5, 1.2, B, device=DEV)
+    x = lg[1::3].double()
+    p = torch.softmax(x / temp[1::3, None].double(), 1)
     for i in range(3):
         step = torch.tensor([i], device=DEV)
-        got = ops.sample(lg, temp, k, top_p, seed=3, step=step).long()
-        assert torch.equal(got, ops.sample(odd, temp, k, top_p, seed=3, step=step).long())
+        got, other = (ops.sample(z, temp, k, top_p, seed=3, step=step).long() for z in (lg, odd))
+        assert torch.equal(got[2::3], other[2::3]) and torch.equal(got[::3], other[::3])
         best = lg[::3].float().max(1).values[:, None]
         assert torch.equal(got[::3], (lg[::3].float() == best).int().argmax(1))
+        for t in (got[1::3], other[1::3]):
+            ahead = (p * (x > x.gather(1, t[:, None]))).sum(1)
+            assert (ahead < top_p[1::3].double() + 1e-4).all()  # (sums of 32 bits there)
 
 
 def test_sample_top_p_full_vocab_exact(hipk):
