@@ -8,9 +8,9 @@
 //    k-th largest logit, so gathering `key >= tau0` yields all top-k plus a few
 //    extra, and such an element can only sit in a thread whose own max is
 //    >= tau0: only those ~k threads' elements are read again, eight lanes to a
-//    thread.  One row pass.  If ties push the gather past 1024 slots, the row
-//    falls back to a 16-bit radix select (two histogram passes) and a ballot-
-//    compacted full gather.
+//    thread (many threads: each its own).  One row pass.  If ties push the gather
+//    past 1024 slots, the row falls back to a 16-bit radix select (two histogram
+//    passes) and a ballot-compacted full gather.
 //    What bounds a row is the chain of its stages, and fetching code that runs
 //    once a step: tau0 by one wave's ballots instead of the workgroup's
 //    histograms, and a gather in a few instructions instead of one unrolled over
@@ -339,10 +339,9 @@ DRTC_DEVICE unsigned last_max(unsigned x) {
 }
 
 // A threshold that at least k of 1024 keys reach, found by one wave that holds 16 to a lane: down from the largest in
-// doubled steps, then halved, until not many more than k reach it (112 where they may be so few: sample_few; all that
-// reach it are to fit the candidates) or no higher one does.
-DRTC_DEVICE unsigned few_above(const unsigned short* keys, int k) {
-  const int lane = threadIdx.x & 63, enough = k < 96 ? 112 : min(k + k / 16, max(k, 900));
+// doubled steps, then halved, until no more than `enough` reach it or no higher one does.
+DRTC_DEVICE unsigned few_above(const unsigned short* keys, int k, int enough) {
+  const int lane = threadIdx.x & 63;
   u32x4 x[2];
   unsigned top = 0;
 #pragma unroll
@@ -466,6 +465,7 @@ DRTC_DEVICE void sample_few(SampShared& s, const unsigned* sort, const TokenOut&
   if (lane == 0) out.put(row, si[at]);
 }
 
+constexpr int kAlike = 112;  // thresholds of any k up to this one let as many threads through
 // each: visits the thread's elements of the row
 template <int U, class Row>
 DRTC_DEVICE void sample_topk(SampShared& s, const TokenOut& out, const Row& each, const unsigned short* lr, int V,
@@ -477,20 +477,26 @@ DRTC_DEVICE void sample_topk(SampShared& s, const TokenOut& out, const Row& each
   each([&](int, unsigned short b) { most = fmaxf(most, bits2f(b)); });
   const unsigned tm = ord16((unsigned short)(__float_as_uint(most) >> 16));
   // hist doubles as a buffer of 1024 keys, of the threads that are looked at again, and of the candidates' sort keys
-  unsigned short* const h = reinterpret_cast<unsigned short*>(&s.hist[0][0]);
   int* const again = reinterpret_cast<int*>(&s.hist[4][0]);
   unsigned* const sort = V <= 0x10000 ? &s.hist[12][0] : nullptr;
-  h[tid] = (unsigned short)tm;
   s.hist[12 + tid / 256][tid & 255] = 0;
+  if (tid == 64) s.wred[0][0] = uniform(seed, st, row, 0);
+  if (tid == 0) s.misc[2] = s.misc[3] = 0;
+  const bool many = k > kAlike && (k > 224 || V <= 16384);
+  if (many) {
+    s.val[tid] = -INFINITY;
+    s.idx[tid] = 0x7fffffff;
+  }
+  unsigned short* const h = reinterpret_cast<unsigned short*>(&s.hist[0][0]);
+  h[tid] = (unsigned short)tm;
   __syncthreads();
   if (tid < 64) {
-    const unsigned t = few_above(h, k);
-    if (tid == 0) {
-      s.misc[0] = (int)t;
-      s.misc[2] = s.misc[3] = 0;
-    }
-  } else if (tid == 64) {
-    s.wred[0][0] = uniform(seed, st, row, 0);
+    // c of 1024 threads reach a threshold by about -1024 log(1 - c / 1024) elements: as many as are likely to fit 128 candidates
+    // (sample_few), 256 or 512 (powers of two, the sort).  No more than k threads with elements: all of them are looked at.
+    const int full = vec ? V >> 3 : V;
+    const int enough = full < 768 ? k : k <= kAlike ? kAlike : k <= 214 ? 214 : k <= 384 ? 384 : k;
+    const unsigned t = full <= k ? 0 : few_above(h, k, enough);
+    if (tid == 0) s.misc[0] = (int)t;
   }
   __syncthreads();
   const unsigned prefix = max((unsigned)s.misc[0], kLowKey);
@@ -502,59 +508,71 @@ DRTC_DEVICE void sample_topk(SampShared& s, const TokenOut& out, const Row& each
   };
   auto below = [](uint64_t m) { return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u)); };
   // ---- gather key >= tau0 (>= k elements by construction, or all numbers).  Such an element can only sit in a thread
-  // whose own max is >= tau0: of those threads' elements (about k of the 1024) every lane takes a few of one's, eight
-  // lanes to a thread.
-  if (const uint64_t m = __ballot(tm >= prefix)) {
-    const int at = places(&s.misc[3], __popcll(m)) + below(m);
-    if (tm >= prefix) again[at] = tid;
-  }
-  __syncthreads();
-  const int threads = s.misc[3], nv = vec ? V >> 3 : 0;
-  // N elements from index i on, those that are `in` the row
-  auto take = [&](auto count, int i, bool in) {
-    constexpr int N = decltype(count)::value;
-    typedef unsigned short Some __attribute__((ext_vector_type(N)));
-    Some x = {};
-    if (in) x = *reinterpret_cast<const Some*>(lr + i);
-    uint64_t m[N];
-    int n = 0;
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-      m[j] = __ballot(in && ord16(x[j]) - prefix <= kTopKey - prefix);  // key in [prefix, kTopKey]
-      n += __popcll(m[j]);
-    }
-    if (n == 0) return;
-    int base = places(&s.misc[2], n);
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-      const int slot = base + below(m[j]);
-      if ((m[j] >> lane & 1) && slot < kCand) {
-        const float v = bits2f(x[j]);
-        s.val[slot] = v;
-        s.idx[slot] = i + j;
-        if (sort) sort[slot] = place_key(v) << 16 | (0xffffu - (unsigned)(i + j));
+  // whose own max is >= tau0.  Few threads: of their elements (about k of the 1024) every lane takes a few of one's, eight
+  // lanes to a thread, 128 threads at a time.  Many: each looks through its own, which is one turn, where the lanes would
+  // wait for the memory several times, or be idle where a thread has a vector or two.  256 rows, us by lanes / by threads: V
+  // 8000, k 200 15.5 / 14.8, k 300 19.2 / 17.1; V 16000, k 250 19.2 / 18.0; V 32000, k 200 16.2 / 18.8, k 1000 53.7 / 51.7; V
+  // 50304, k 250 23.2 / 22.3; V 128256, k 200 29.2 / 33.0, k 500 46.7 / 42.3, k 1000 139 / 130.
+  if (many) {
+    if (tm >= prefix) for_row<U>(lr, V, vec, [&](int i, unsigned short b) {
+      if (ord16(b) - prefix <= kTopKey - prefix) {  // key in [prefix, kTopKey]
+        const int slot = atomicAdd(&s.misc[2], 1);
+        if (slot < kCand) { s.val[slot] = bits2f(b); s.idx[slot] = i; }
       }
-      base += __popcll(m[j]);
+    });
+  } else {
+    if (const uint64_t m = __ballot(tm >= prefix)) {
+      const int at = places(&s.misc[3], __popcll(m)) + below(m);
+      if (tm >= prefix) again[at] = tid;
     }
-  };
+    __syncthreads();
+    const int threads = s.misc[3], nv = vec ? V >> 3 : 0;
+    // N elements from index i on, those that are `in` the row
+    auto take = [&](auto count, int i, bool in) {
+      constexpr int N = decltype(count)::value;
+      typedef unsigned short Some __attribute__((ext_vector_type(N)));
+      Some x = {};
+      if (in) x = *reinterpret_cast<const Some*>(lr + i);
+      uint64_t m[N];
+      int n = 0;
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        m[j] = __ballot(in && ord16(x[j]) - prefix <= kTopKey - prefix);  // key in [prefix, kTopKey]
+        n += __popcll(m[j]);
+      }
+      if (n == 0) return;
+      int base = places(&s.misc[2], n);
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        const int slot = base + below(m[j]);
+        if ((m[j] >> lane & 1) && slot < kCand) {
+          const float v = bits2f(x[j]);
+          s.val[slot] = v;
+          s.idx[slot] = i + j;
+          if (sort) sort[slot] = place_key(v) << 16 | (0xffffu - (unsigned)(i + j));
+        }
+        base += __popcll(m[j]);
+      }
+    };
 #pragma unroll 1
-  for (int g = 0; g < threads; g += kSampThreads / 8) {
-    const bool on = g + (tid >> 3) < threads;
-    const int t = on ? again[g + (tid >> 3)] : 0;
+    for (int g = 0; g < threads; g += kSampThreads / 8) {
+      const bool on = g + (tid >> 3) < threads;
+      const int t = on ? again[g + (tid >> 3)] : 0;
 #pragma unroll 1
-    for (int v = 0; v < nv; v += 4 * kSampThreads) {
-      const int at = v + t + (tid >> 1 & 3) * kSampThreads;
-      take(std::integral_constant<int, 4>{}, 8 * at + 4 * (tid & 1), on && at < nv);
-    }
+      for (int v = 0; v < nv; v += 4 * kSampThreads) {
+        const int at = v + t + (tid >> 1 & 3) * kSampThreads;
+        take(std::integral_constant<int, 4>{}, 8 * at + 4 * (tid & 1), on && at < nv);
+      }
 #pragma unroll 1
-    for (int e = 8 * nv; e < V; e += 8 * kSampThreads) {
-      const int at = e + t + (tid & 7) * kSampThreads;
-      take(std::integral_constant<int, 1>{}, at, on && at < V);
+      for (int e = 8 * nv; e < V; e += 8 * kSampThreads) {
+        const int at = e + t + (tid & 7) * kSampThreads;
+        take(std::integral_constant<int, 1>{}, at, on && at < V);
+      }
     }
   }
   __syncthreads();
   int n = s.misc[2];
-  const unsigned* gathered = sort;  // (not by gather_ge)
+  const unsigned* gathered = many ? nullptr : sort;  // (nor by gather_ge)
   if (n > kCand) {  // heavy ties: exact k-th key by radix select, gather again
     const unsigned thr = radix_kth<U>(s, lr, V, vec, k);
     n = min(gather_ge<U>(s, lr, V, vec, thr), kCand);
@@ -570,11 +588,13 @@ DRTC_DEVICE void sample_topk(SampShared& s, const TokenOut& out, const Row& each
   }
   int np2 = 1;
   while (np2 < n) np2 <<= 1;
-  if (tid >= n) {
-    s.val[tid] = -INFINITY;
-    s.idx[tid] = 0x7fffffff;
+  if (!many) {
+    if (tid >= n) {
+      s.val[tid] = -INFINITY;
+      s.idx[tid] = 0x7fffffff;
+    }
+    __syncthreads();
   }
-  __syncthreads();
   // ---- bitonic sort, descending (ties -> lower index first)
   for (int size = 2; size <= np2; size <<= 1) {
     for (int stride = size >> 1; stride > 0; stride >>= 1) {

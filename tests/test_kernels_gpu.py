@@ -739,6 +739,14 @@ def test_sample_row_forms(hipk, V, k):
         assert (lg.float().gather(1, got[:, None])[:, 0] >= kth).all()
 
 
+@pytest.mark.parametrize("V", [520, 1024, 6136, 6144, 16384, 16392])
+@pytest.mark.parametrize("k", [65, 112, 113, 214, 215, 224, 225, 384, 385])
+def test_sample_row_forms_of_many(hipk, V, k):
+    """The same at the sizes where the threshold lets more threads through, and where a thread looks through its own
+    elements instead of eight lanes (of rows of up to 16384 from 113 on, of all from 225 on)."""
+    test_sample_row_forms(hipk, V, k)
+
+
 @pytest.mark.parametrize("V", [8, 512, 8192, 32768, 32776])
 def test_sample_modes_in_one_batch(hipk, V):
     """Greedy rows, rows of top-p alone and of top-k beside one another, and the same rows from a view that starts 2 bytes off,
