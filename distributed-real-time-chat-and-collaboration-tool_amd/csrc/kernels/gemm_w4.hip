@@ -215,7 +215,8 @@ struct W4Tile {
 // run at the card's power limit: from registers alone, random operands, 2040 -> 2090 TFLOP/s (both operands new each
 // time: 1965; A held, B back and forth: 2055; 4 x 4 blocks: 2055); this kernel, 16384 x 4096 x 4096 store 1518 -> 1545,
 // gated 1501 -> 1527, 12160 x 6144 x 4096 1401 -> 1433, 16000 x 2048 x 7168 with residual 1405 -> 1430.  Zero operands,
-// below the limit, take the same time either way.
+// below the limit, take the same time either way.  Only the forms whose reads are spread (V & 32): with the burst of reads, the
+// per-tile form takes 41 us row by row and 57 in blocks at 4096 x 2048 x 2048, 95 and 117 at 4096 x 4096 x 4096.
 constexpr int w4_order(int q) {
   const int blk = q >> 2, n = q & 3, bi = blk >> 2, bj = (bi & 1) ? 3 - (blk & 3) : blk & 3;
   return (2 * bi + (n >> 1)) * 8 + 2 * bj + (n == 1 || n == 2);
@@ -224,7 +225,8 @@ constexpr int w4_order(int q) {
 template <int V, bool DMA, bool NEXT, bool Z, int Q>
 DRTC_DEVICE void w4_step(f32x4 (&acc)[8][8], bf16x8 (&fa0)[8], bf16x8 (&fb0)[8],
                          bf16x8 (&fa1)[8], bf16x8 (&fb1)[8], const W4Tile& T, const W4Dma& d) {
-  constexpr int ij = w4_order(Q & 63), i = ij >> 3, j = ij & 7;
+  constexpr bool kSpread = (V & 32) != 0;
+  constexpr int ij = kSpread ? w4_order(Q & 63) : Q & 63, i = ij >> 3, j = ij & 7;
   if constexpr (Q < 64 && Z)  // first K tile of a persistent tile: accumulate onto 0
     acc[i][j] = mfma16(fa0[i], fb0[j], (f32x4){0.f, 0.f, 0.f, 0.f});
   else if constexpr (Q < 64)
@@ -264,8 +266,7 @@ DRTC_DEVICE void w4_step(f32x4 (&acc)[8][8], bf16x8 (&fa0)[8], bf16x8 (&fb0)[8],
     if constexpr (s < 7) asm volatile("s_add_u32 m0, m0, 0x1000" ::: "memory");
   }
   // ---- tile t + 1: its DMA (issued during tile t - 1) landed for every wave, then its
-  // half-0 fragments: fa0[0..1], fb0[0..7], fa0[2..7]
-  constexpr bool kSpread = (V & 32) != 0;
+  // half-0 fragments: fa0[0..1], fb0[0..7], fa0[2..7]; in a burst fa0[0], fb0[0..7], fa0[1..7]
   constexpr int qn = kSpread ? 63 : 103;
   // this step's own DMAs (tile t + 2) issued before qn: B 8 + A (1 at qn 63, 8 at 103)
   constexpr int kYoung = kSpread ? 9 : 16;
@@ -295,10 +296,10 @@ DRTC_DEVICE void w4_step(f32x4 (&acc)[8][8], bf16x8 (&fa0)[8], bf16x8 (&fb0)[8],
   }
   if constexpr (NEXT && !kSpread && Q > qn && Q <= qn + 16) {
     constexpr int r = Q - qn - 1;
-    if constexpr (r <= 1)
-      fa0[r] = w4_rd(T.lds, T.nxt + T.ra0 + 2048 * r);
-    else if constexpr (r <= 9)
-      fb0[r - 2] = w4_rd(T.lds, T.nxt + T.rb0 + 128 * (r - 2));
+    if constexpr (r == 0)
+      fa0[0] = w4_rd(T.lds, T.nxt + T.ra0);
+    else if constexpr (r <= 8)
+      fb0[r - 1] = w4_rd(T.lds, T.nxt + T.rb0 + 128 * (r - 1));
     else
       fa0[r - 8] = w4_rd(T.lds, T.nxt + T.ra0 + 2048 * (r - 8));
   }
