@@ -707,7 +707,7 @@ __global__ __launch_bounds__(64 * NH * ND, 2) void latent_decode_kernel(LatentDe
 // tile's ND waves takes 64 / ND of the 64 tokens' scores and hands them to the others through LDS, where the form above
 // has every wave compute them all.  Chunk c (16 bytes) of row t lies at c ^ (t / 2 % 8).  That form was bound
 // by each block's chain - the scores' LDS reads fourfold, one wave a SIMD, two barriers for 64 tokens in both: 64
-// sequences of 1500 tokens, 48 heads of 512 + 64 38.6 us alone.
+// sequences of 1500 tokens, 32 heads of 512 + 64, four splits: 28.4 -> 26.6 us.
 template <int RT, int NH, int ND>
 struct LatPair {
   static constexpr int KS = 2 * RT + 2, LW = 32 * KS, CPR = LW / 8, NW = NH * ND;
@@ -851,13 +851,13 @@ __global__ __launch_bounds__(64 * NH * ND, 1) void latent_decode_pair_kernel(Lat
   lat_decode_out<RT, ND>(a, b, h, sp, nparts, dw, g, R, o, m, lsum);
 }
 
-// The same for latents of 512 and up to 32 heads, a block at a time, three more on their way: what a CU takes in never waits
-// for a barrier.  A wave's scores are 16 of the block's tokens over one half of the columns; V's operands are read during the
-// softmax, K's ahead of their products, and blocks inside the context are not masked.  200 sequences of 500 tokens, 16
-// heads: 33 -> 29 us in the pass (5.1 TB/s behind 6.5 us of launch and first loads, which a context of one block takes), alone 25.6 -> 23.4,
-// 256 x 400 25.2 -> 22.7, 64 x 1500 27.3 -> 25.2; 32 heads, 200 x 30 10.7 -> 9.3, 256 x 400 29.2 -> 26.9, 200 x 500 29.6 / 29.7, window of
-// 1024 64 x 1500 29.4 / 28.8.  Slower than pairs for latents of 256 (16 heads 200 x 500 16.6 / 17.8, 32 18.8 / 22.6: two barriers for half the
-// tokens) and for more heads (64 x 1500 of 48 38.6 / 40.5: registers for fewer reads ahead), which keep them.
+// The same for latents of 512 and up to 16 heads, and for up to 32 where a split has few blocks (lat_ring_takes): a block at a
+// time, three more on their way, so that what a CU takes in never waits for a barrier.  A wave's scores are 16 of the block's
+// tokens over one half of the columns; V's operands are read during the softmax, K's ahead of their products, and blocks inside
+// the context are not masked.  16 heads, pairs -> this: 200 sequences of 500 tokens 33 -> 29 us in the pass (5.1 TB/s behind 6.5
+// us of launch and first loads, which a context of one block takes), alone 25.6 -> 23.4, 256 x 400 25.2 -> 22.7, 64 x 1500 27.3 ->
+// 25.2.  Slower than pairs for latents of 256 (16 heads 200 x 500 16.6 / 17.8, 32 18.8 / 22.6: two barriers for half the tokens) and
+// for more heads (64 x 1500 of 48 38.6 / 40.5: registers for fewer reads ahead), which keep them.
 template <int NH>
 struct LatRing {
   static constexpr int RT = 8, ND = 4, KS = 2 * RT + 2, LW = 32 * KS, CPR = LW / 8, NW = NH * ND, ST = 4;
@@ -1044,6 +1044,23 @@ __global__ __launch_bounds__(128) void latent_merge_kernel(LatentDecodeArgs a) {
 
 template <int RT, int NH>
 constexpr bool lat_ring = RT == 8 && NH <= 2;
+template <int RT, int NH>
+constexpr bool lat_pair = RT != 8 || NH != 1;  // (up to 16 heads of 512 all go by single blocks)
+// Whether 17 to 32 heads go by single blocks, by the blocks of a split (a table wider than the contexts counts as long ones).  The
+// ring starts 1 - 2 us sooner and reads no lone last block twice; pairs have one barrier a block less, and few heads beyond the
+// first 16 need little of what the ring gives.  us, pairs / ring, of rows of 576 that no cache holds:
+//   odd, up to 11: 17 heads 0.99 - 1.04 times as fast, 24 1.00 - 1.06, 32 1.01 - 1.08 (64 x 1500 of 32, a window of 1024, splits of
+//     nine: 29.8 / 29.2)
+//   even, more than 24 heads: up to 12 without a window 0.98 - 1.28 (64 x 400 of 32 21.1 / 20.1, 200 x 200 20.2 / 19.7), with
+//     one, whose start waits for the context anyway, four (0.98 - 1.04; six: 40 x 1500 24.0 / 24.5)
+//   even, 20 to 24 heads: four without a window 0.99 - 1.26, with one 0.95 - 1.02; eight 0.98 - 1.00
+//   even, 17 to 19: 0.92 - 0.98 (40 x 1500 24.6 / 25.8), but for contexts of a block
+//   more: 32 heads 64 x 1000 in one split of 40 55.0 / 58.5, 40 x 3000 in splits of 20 40.0 / 41.7; short contexts in such a table
+//     give up what the ring's start saves (64 x 20 12.0 / 9.9, 100 x 100 15.7 / 14.8).
+static bool lat_ring_takes(const LatentDecodeArgs& a) {
+  const int n = a.tiles_per_split, even = a.H > 24 ? (a.window > 0 ? 4 : 12) : a.H >= 20 && a.window <= 0 ? 4 : 0;
+  return a.H <= 16 || n <= (n % 2 ? 11 : even);
+}
 template <int RT, int NH, int ND>
 static void lat_decode_go(const LatentDecodeArgs& a, hipStream_t st) {
   const size_t lds = (size_t)2 * kLB * (a.LW + kLatPad) * 2;
@@ -1053,10 +1070,14 @@ static void lat_decode_go(const LatentDecodeArgs& a, hipStream_t st) {
     if (a.R == 64 * RT && a.LW == 32 * (2 * RT + 2) && (uintptr_t)a.cache % 16 == 0) {
       constexpr int NP = NH == 2 ? 4 : ND;  // eight waves where the heads fill two tiles
       if constexpr (lat_ring<RT, NH>)
-        latent_decode_ring_kernel<NH><<<grid, dim3(256 * NH), LatRing<NH>::BYTES, st>>>(a);
-      else
+        if (lat_ring_takes(a)) {
+          latent_decode_ring_kernel<NH><<<grid, dim3(256 * NH), LatRing<NH>::BYTES, st>>>(a);
+          return;
+        }
+      if constexpr (lat_pair<RT, NH>) {
         latent_decode_pair_kernel<RT, NH, NP><<<grid, dim3(64 * NH * NP), LatPair<RT, NH, NP>::BYTES, st>>>(a);
-      return;
+        return;
+      }
     }
     if (a.R == 64 * RT && a.LW == 32 * (2 * RT + 1)) {
       latent_decode_kernel<RT, NH, ND, 2 * RT + 1><<<grid, block, lds, st>>>(a);
@@ -1424,12 +1445,15 @@ static int lat_decode_attr() {
 }
 template <int RT, int NH, int ND>
 static int lat_pair_attr() {
+  int e = 0;
   if constexpr (lat_ring<RT, NH>)
-    return (int)hipFuncSetAttribute((const void*)latent_decode_ring_kernel<NH>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)LatRing<NH>::BYTES);
-  else
-    return (int)hipFuncSetAttribute((const void*)latent_decode_pair_kernel<RT, NH, ND>,
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)LatPair<RT, NH, ND>::BYTES);
+    e = (int)hipFuncSetAttribute((const void*)latent_decode_ring_kernel<NH>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 (int)LatRing<NH>::BYTES);
+  if constexpr (lat_pair<RT, NH>)
+    if (!e)
+      e = (int)hipFuncSetAttribute((const void*)latent_decode_pair_kernel<RT, NH, ND>,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)LatPair<RT, NH, ND>::BYTES);
+  return e;
 }
 template <int NH, int ND>
 static int lat_decode_lds() {

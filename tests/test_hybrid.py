@@ -1163,6 +1163,29 @@ def test_latent_decode_a_block_at_a_time(H, parts):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H", [17, 24, 25, 32])
+@pytest.mark.parametrize("per", [4, 6, 11, 12, 13, 14])
+def test_latent_decode_by_the_blocks_of_a_split(H, per):
+    """17 to 32 heads, by single blocks or in pairs: around the lengths where the one takes over from the other, with lone last
+    blocks and splits that a context does not reach.  Rounding of the test above."""
+    R, nb, dev = 512, 2 * per, "cuda"
+    ctx = [1, 32 * per - 31, 32 * per, 32 * per + 1, 32 * (2 * per - 1), 32 * 2 * per]
+    B, g = len(ctx), torch.Generator().manual_seed(H + per)
+    cache = torch.randn(B * nb + 1, 32, R + 64, generator=g).mul_(0.5).to(torch.bfloat16)
+    bt = torch.randperm(B * nb, generator=g).view(B, nb).to(torch.int32) + 1
+    qa = torch.randn(B, H, R + 64, generator=g).mul_(0.5).to(torch.bfloat16)
+    for window in (None, 150):
+        ws = ops.LatentDecodeWorkspace(B, H, R, window, nb, dev)
+        ws.per, ws.splits = per, 2
+        ws.part_o, ws.part_ml = torch.empty(B, H, 2, R, device=dev), torch.empty(B, H, 2, 2, device=dev)
+        out = ops.latent_decode_attention(qa.to(dev), cache.to(dev), R, bt.to(dev),
+                                          torch.tensor(ctx, dtype=torch.int32, device=dev), window, 0.05, None, ws)
+        for b, n in enumerate(ctx):
+            rows = cache[bt[b].long()].reshape(-1, R + 64)[max(0, n - (window or n)):n].double()
+            close(out[b], (qa[b].double() @ rows.T * 0.05).softmax(-1) @ rows[:, :R], 2e-2)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("shared", [True, False])
 @pytest.mark.parametrize("window", [None, 50])
 def test_latent_decode_of_tables_of_any_stride(shared, window):
